@@ -263,6 +263,46 @@ int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch
     return 0;
 }
 
+int cached_split_weight(State *st, const float *host, size_t n, size_t channels, size_t taps, const float4 **out, char *error, size_t capacity) {
+    if (host == nullptr || n == 0 || n % 32 != 0 || channels == 0 || channels % 64 != 0 || (taps != 1 && taps != 3) || n > SIZE_MAX / channels / taps / sizeof(float) / 2) {
+        set_error(error, capacity, "invalid product weight");
+        return -1;
+    }
+    const size_t count = n * channels * taps;
+    const WeightKey key{host, count * sizeof(float), -(int)taps};
+    std::lock_guard<std::mutex> lock(st->mu);
+    auto it = st->weights.find(key);
+    if (it != st->weights.end()) {
+        *out = static_cast<const float4 *>(it->second.data);
+        return 0;
+    }
+    if (st->pack_staging_floats < count) {
+        if (st->pack_staging != nullptr) {
+            MYNAH_TRY(hipStreamSynchronize(st->stream));   // the packing of an earlier weight may still read it
+            (void)hipFree(st->pack_staging);
+            st->pack_staging = nullptr;
+            st->pack_staging_floats = 0;
+        }
+        MYNAH_TRY(hipMalloc(reinterpret_cast<void **>(&st->pack_staging), count * sizeof(float)));
+        st->pack_staging_floats = count;
+    }
+    CachedWeight cw;
+    cw.n = n;
+    cw.k = channels * taps;
+    cw.bytes = count * sizeof(float) + kSplitWeightOverrun;
+    MYNAH_TRY(hipMalloc(&cw.data, cw.bytes));
+    // one stream, in order: upload, rearrange (the next weight's upload waits for it); pageable source, taken when the call returns
+    if (hip_check(hipMemcpyAsync(st->pack_staging, host, count * sizeof(float), hipMemcpyHostToDevice, st->stream), "weight upload", error, capacity) != 0 ||
+        launch_split_pack(st, st->pack_staging, static_cast<float4 *>(cw.data), n, channels, taps, error, capacity) != 0) {
+        (void)hipFree(cw.data);
+        return -1;
+    }
+    st->weight_bytes += cw.bytes;
+    st->weights.emplace(key, cw);
+    *out = static_cast<const float4 *>(cw.data);
+    return 0;
+}
+
 int cached_vector(State *st, const float *host, size_t n, const float **dev, char *error, size_t capacity) {
     if (host == nullptr || n == 0) {
         *dev = nullptr;
@@ -432,6 +472,7 @@ static void hip_close(void *opaque) {
     if (st->pinned != nullptr) (void)hipHostFree(st->pinned);
     if (st->flush != nullptr) (void)hipFree(st->flush);
     if (st->cross_norm != nullptr) (void)hipFree(st->cross_norm);
+    if (st->pack_staging != nullptr) (void)hipFree(st->pack_staging);
     if (st->attn_partial != nullptr) (void)hipFree(st->attn_partial);
     if (st->attn_counters != nullptr) (void)hipFree(st->attn_counters);
     if (st->seam_slots != nullptr) (void)hipFree(st->seam_slots);
@@ -1166,32 +1207,49 @@ extern "C" int mynah_hip_cross_kv_dev(void *opaque, const float *dev_memory, siz
         return -1;
     }
     if (memory_length == 0 || layers == 0) return 0;
+    for (size_t l = 0; l < layers; ++l)
+        if (norm_gain[l] == nullptr || kv_w[l] == nullptr) {
+            set_error(error, capacity, "cross K/V: missing layer weight");
+            return -1;
+        }
+    // More rows than the quantised products take, at the matrix-core kernel's granularity: every layer in two launches, LayerNorm and
+    // product.  One layer's product is 36 tiles of work on 256 CUs and its LayerNorm a launch as long: 12 layers of 180 rows
+    // took 36 launches and 630 us one after the other.
+    const bool grouped = memory_length > kQuantMaxRows && width % 64 == 0 && xattn_width % 32 == 0 && memory_length <= 0x10000 && width <= 0x10000 && xattn_width <= 0x10000;
+    const size_t group = grouped ? (layers < kSplitMaxLayers ? layers : kSplitMaxLayers) : 1;
     // The normalised rows live in a buffer the backend keeps and grows: one allocation per call would add up between
     // synchronisations when a caller prepares many utterances in a row.  An outgrown buffer may still be read by earlier
     // launches: it waits in the list that the next idle stream frees (bounded like mynah_hip_dev_free's).
-    if (st->cross_norm_floats < memory_length * width) {
+    const size_t norm_floats = group * memory_length * width + kSplitOverrun;
+    if (st->cross_norm_floats < norm_floats) {
         if (st->cross_norm != nullptr) {
             st->pending_free.push_back(st->cross_norm);
             st->cross_norm = nullptr;
             st->cross_norm_floats = 0;
             if (st->pending_free.size() >= kMaxPendingFrees && hipStreamSynchronize(st->stream) == hipSuccess) free_pending(st);
         }
-        MYNAH_TRY(hipMalloc(reinterpret_cast<void **>(&st->cross_norm), memory_length * width * sizeof(float)));
-        st->cross_norm_floats = memory_length * width;
+        MYNAH_TRY(hipMalloc(reinterpret_cast<void **>(&st->cross_norm), norm_floats * sizeof(float)));
+        st->cross_norm_floats = norm_floats;
     }
     float *const normed = st->cross_norm;
     const size_t per_layer = memory_length * xattn_width;
-    for (size_t l = 0; l < layers; ++l) {
-        if (norm_gain[l] == nullptr || kv_w[l] == nullptr) {
-            set_error(error, capacity, "cross K/V: missing layer weight");
-            return -1;
+    for (size_t l0 = 0; l0 < layers; l0 += group) {
+        const size_t count = layers - l0 < group ? layers - l0 : group;
+        SplitLayers table{};
+        for (size_t i = 0; i < count; ++i) {
+            if (cached_vector(st, norm_gain[l0 + i], width, &table.gain[i], error, capacity) != 0) return -1;
+            if (norm_bias != nullptr && cached_vector(st, norm_bias[l0 + i], width, &table.bias[i], error, capacity) != 0) return -1;
+            if (grouped && cached_split_weight(st, kv_w[l0 + i], 2 * xattn_width, width, 1, &table.w[i], error, capacity) != 0) return -1;
         }
-        const float *dgain = nullptr, *dbias = nullptr;
-        if (cached_vector(st, norm_gain[l], width, &dgain, error, capacity) != 0) return -1;
-        if (norm_bias != nullptr && cached_vector(st, norm_bias[l], width, &dbias, error, capacity) != 0) return -1;
-        if (launch_layernorm(st, dev_memory, normed, dgain, dbias, memory_length, width, error, capacity) != 0) return -1;
-        if (matmul_device(st, normed, dev_cross_k + l * per_layer, memory_length, width, xattn_width, kv_w[l], nullptr, error, capacity) != 0) return -1;
-        if (matmul_device(st, normed, dev_cross_v + l * per_layer, memory_length, width, xattn_width, kv_w[l] + xattn_width * width, nullptr, error,
+        if (grouped) {
+            if (launch_split_cross_kv(st, dev_memory, memory_length, width, table, count, xattn_width, normed, dev_cross_k + l0 * per_layer,
+                                      dev_cross_v + l0 * per_layer, error, capacity) != 0)
+                return -1;
+            continue;
+        }
+        if (launch_layernorm(st, dev_memory, normed, table.gain[0], table.bias[0], memory_length, width, error, capacity) != 0) return -1;
+        if (matmul_device(st, normed, dev_cross_k + l0 * per_layer, memory_length, width, xattn_width, kv_w[l0], nullptr, error, capacity) != 0) return -1;
+        if (matmul_device(st, normed, dev_cross_v + l0 * per_layer, memory_length, width, xattn_width, kv_w[l0] + xattn_width * width, nullptr, error,
                           capacity) != 0)
             return -1;
     }

@@ -78,7 +78,7 @@ struct PackedWeight {
 struct WeightKey {
     const void *host;
     size_t bytes;
-    int kind;   // 0 plain f32 vector/matrix, 1 + qtype*2 + arith for converted matrices, 64 + kernel + 32 * in_ch for conv1d chunks
+    int kind;   // 0 plain f32 vector/matrix, 1 + qtype*2 + arith for converted matrices, 64 + kernel + 32 * in_ch for conv1d chunks, -taps for split products
     bool operator==(const WeightKey &o) const { return host == o.host && bytes == o.bytes && kind == o.kind; }
 };
 struct WeightKeyHash {
@@ -176,6 +176,9 @@ struct State {
     size_t scratch_bytes = 0;
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
+    // f32 weights on their way into the order of the split products' kernels (grown on demand)
+    float *pack_staging = nullptr;
+    size_t pack_staging_floats = 0;
     // normalised encoder memory of mynah_hip_cross_kv_dev (grown on demand; an outgrown one waits in pending_free)
     float *cross_norm = nullptr;
     size_t cross_norm_floats = 0;
@@ -235,6 +238,8 @@ struct ConvBlocks {
 constexpr int kConvChannels = 8;      // input channels per chunk: the convolution kernels' step along the inner dimension
 inline size_t conv_chunk_floats(size_t kernel) { return 32u * (kConvChannels * kernel + 4u); }
 int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch, size_t kernel, ConvBlocks *out, char *error, size_t capacity);
+// An f32 weight [n, channels, taps] in the order in which split_product.hip's kernels take it; n a multiple of 32, channels of 64.
+int cached_split_weight(State *st, const float *host, size_t n, size_t channels, size_t taps, const float4 **out, char *error, size_t capacity);
 int ensure_attention_workspace(State *st, size_t batch, size_t heads, size_t head_width, size_t max_valid,
                                char *error, size_t capacity, size_t chunk_rows = kAttnChunk);
 int ensure_pinned(State *st, size_t bytes, char *error, size_t capacity);

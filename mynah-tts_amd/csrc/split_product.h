@@ -1,0 +1,64 @@
+// f32 products on the bf16 matrix cores: every operand value is taken apart into three bf16 pieces whose sum IS the value, and
+// a product is put together from the six pairs of pieces that reach f32.
+//
+// v_mfma_f32_32x32x2_f32 does 64 multiply-adds per lane in 64 cycles, v_mfma_f32_32x32x16_bf16 does 512 in 32: six of the
+// latter for eight of the former make 192 cycles against 512, and both accumulate in f32.
+//   x = h + m + l:  h = bf16(x), m = bf16(x - h), l = x - h - m.  Both differences are exact (a value has 24 significant bits, a
+//   piece holds 8, and a rounding leaves at most half a place of the piece before it), so nothing of the operand is lost
+//   down to |x| = 2^-110.
+//   x y = hh' + (hm' + mh') + (mm' + hl' + lh') + (ml' + lm' + ll'); the last three are left out: |m| <= 2^-8 |h| and
+//   |l| <= 2^-16 |h| make them 2^-23 of the product at most and 2^-26 on average, of either sign, where one f32 addition rounds
+//   2^-24 of the running sum -- and a step of 16 along the inner dimension has six such additions here and eight there.
+// Against double precision sums (192 x 3072 outputs, inner length 2304, relative error of the 2-norm): 4e-7 here, 8e-7 with
+// the f32 matrix instruction.  An infinite operand gives NaN where a plain product may give infinity; NaN stays NaN.
+#pragma once
+
+#include "device_common.h"
+
+namespace mynah {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {   // one instruction (v_cvt_pk_bf16_f32, round to nearest even)
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+}
+__device__ __forceinline__ float bf16_low(unsigned p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float bf16_high(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
+
+// The three pieces of four neighbouring values, 8 bytes each (22 vector instructions).
+struct SplitFour {
+    uint2 piece[3];
+    __device__ __forceinline__ explicit SplitFour(const float4 v) {
+        const unsigned h0 = bf16_pair(v.x, v.y), h1 = bf16_pair(v.z, v.w);
+        const float x = v.x - bf16_low(h0), y = v.y - bf16_high(h0), z = v.z - bf16_low(h1), w = v.w - bf16_high(h1);
+        const unsigned m0 = bf16_pair(x, y), m1 = bf16_pair(z, w);
+        piece[0] = make_uint2(h0, h1);
+        piece[1] = make_uint2(m0, m1);
+        piece[2] = make_uint2(bf16_pair(x - bf16_low(m0), y - bf16_high(m0)), bf16_pair(z - bf16_low(m1), w - bf16_high(m1)));
+    }
+};
+// ... of eight: one operand of a matrix instruction per piece.
+__device__ __forceinline__ void split_eight(const float4 a, const float4 b, bf16x8 (&out)[3]) {
+    const SplitFour x(a), y(b);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) out[p] = __builtin_bit_cast(bf16x8, make_uint4(x.piece[p].x, x.piece[p].y, y.piece[p].x, y.piece[p].y));
+}
+
+// One 16-deep step: acc += a * w over the six pairs, the smallest first.
+__device__ __forceinline__ f32x16 split_multiply(const bf16x8 (&a)[3], const bf16x8 (&w)[3], f32x16 acc) {
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], w[0], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], w[2], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], w[1], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], w[0], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], w[1], acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], w[0], acc, 0, 0, 0);
+}
+
+// Row of C held in accumulator register r of lane l for a 32x32 tile; the column is l % 32.
+__device__ __forceinline__ int split_acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+
+}  // namespace mynah
