@@ -64,14 +64,13 @@ struct mynah_hip_encoder {
     std::unordered_map<int, hipGraphExec_t> graphs;   // by padded length
     std::unordered_map<int, int> eager_runs;          // a padded length runs eagerly once before it is captured
     size_t max_lds = 0;
-    // f32 operands (the reference's own arithmetic, src/graph.c:634-711: every product an f32 GEMM): f32 copies of the tables
-    // and weights (conv weights tap-major, owned here), and f32 workspaces for exactly max_positions rows
+    // f32 operands (the reference's own arithmetic, src/graph.c:634-711: every product an f32 GEMM): f32 tables, weights in the
+    // order of split_product.hip, f32 rows padded like the f16 form's
     bool f32 = false;
     const CachedWeight *tok32 = nullptr, *pos32 = nullptr;
-    std::vector<const float *> qkv32, o32, up32, down32;
-    std::vector<float *> conv32;   // owned tap-major copies behind up32 / down32 when taps == 3
-    float *f_nrm = nullptr, *f_qkv = nullptr, *f_scores = nullptr, *f_ctx = nullptr, *f_hid = nullptr, *f_col = nullptr, *f_tmp = nullptr;
-    int *f_ids = nullptr;
+    std::vector<const float4 *> qkv32, o32, up32, down32;
+    float *f_nrm = nullptr, *f_qkv = nullptr, *f_ctx = nullptr, *f_hid = nullptr;
+    float *f_nrm_alloc = nullptr, *f_hid_alloc = nullptr;   // f_nrm and f_hid begin kLeadRows rows into these
 };
 
 namespace {
@@ -272,6 +271,20 @@ k_enc_gemm(const _Float16 *const a_arg, const _Float16 *const w_arg, const int M
     }
 }
 
+// Token gather + position add (src/graph.c:729-737, :649-651), f32 tables.  Rows [tokens, tpad) are zeroed.
+__global__ void __launch_bounds__(kThreads) k_enc_embed_f32(const int *ids, const EncParams *params, const float *tok, const float *pos, float *x, int width) {
+    const int t = blockIdx.x;
+    const int tokens = params->tokens;
+    for (int c = threadIdx.x * 4; c < width; c += kThreads * 4) {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (t < tokens) {
+            const float4 a = *reinterpret_cast<const float4 *>(tok + (size_t)ids[t] * width + c), b = *reinterpret_cast<const float4 *>(pos + (size_t)t * width + c);
+            v = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+        }
+        *reinterpret_cast<float4 *>(x + (size_t)t * width + c) = v;
+    }
+}
+
 // Token gather + position add (src/graph.c:729-737, :649-651).  Rows [tokens, tpad) are zeroed.
 __global__ void __launch_bounds__(kThreads) k_enc_embed(const int *ids, const EncParams *params, const _Float16 *tok, const _Float16 *pos,
                                                         float *x, int width) {
@@ -306,13 +319,14 @@ __global__ void __launch_bounds__(kThreads) k_enc_embed(const int *ids, const En
 // (256 rows: 64 workgroups) -- a row per workgroup spreads them over the chip.
 // No request stands under a condition (a place beyond the row, or a partial plane the product did not write, asks for a
 // place that exists and is set to zero afterwards): the waits then name exactly the requests they need.
-template <bool F16_OUT, int NV, int RPW>
+enum { ROWS_RESULT = 0, ROWS_F16 = 1, ROWS_F32 = 2 };   // params->out (real rows only), f16 operand rows, f32 operand rows
+template <int OUT, int NV, int RPW>
 __global__ void __launch_bounds__(64 * RPW) k_enc_rows(float *x, const float *part, const EncParams *params, int rows, int width, int splits,
-                                                        size_t split_stride, const float *gain, const float *bias, _Float16 *out_f16) {
+                                                        size_t split_stride, const float *gain, const float *bias, void *out_rows) {
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * RPW + (threadIdx.x >> 6);
     if (row >= rows) return;
-    if constexpr (!F16_OUT) {
+    if constexpr (OUT == ROWS_RESULT) {
         if (row >= params->tokens) return;
     }
     float4 *xr = reinterpret_cast<float4 *>(x + (size_t)row * width);
@@ -329,32 +343,40 @@ __global__ void __launch_bounds__(64 * RPW) k_enc_rows(float *x, const float *pa
         bb[u] = bias4[at];
     }
     if (part != nullptr) {
-        // all splits are requested at once and added in split order: the sum does not depend on how the splits were scheduled
-        constexpr int kSplits = 4;   // kMaxSplits of the products
-        float4 p[kSplits][NV];
+        // the splits are requested kSplits at a time and added in split order: the sum does not depend on how the splits were
+        // scheduled.  (The f16 products make at most four planes; the f32 form, whose products have more K to split, up to kMaxSplitsF32.)
+        constexpr int kSplits = OUT == ROWS_F16 ? 4 : 6;
+        float4 t[NV];
 #pragma unroll
-        for (int z = 0; z < kSplits; ++z) {
-            const float4 *const plane = reinterpret_cast<const float4 *>(part + (z < splits ? z : splits - 1) * split_stride + (size_t)row * width);
+        for (int u = 0; u < NV; ++u) t[u] = zero4;
+        for (int z0 = 0; z0 < (OUT == ROWS_F16 ? 1 : splits); z0 += kSplits) {
+            float4 p[kSplits][NV];
+#pragma unroll
+            for (int z = 0; z < kSplits; ++z) {
+                const float4 *const plane = reinterpret_cast<const float4 *>(part + (z0 + z < splits ? z0 + z : splits - 1) * split_stride + (size_t)row * width);
+#pragma unroll
+                for (int u = 0; u < NV; ++u) {
+                    const int i = lane + 64 * u;
+                    p[z][u] = plane[i < n4 ? i : n4 - 1];
+                }
+            }
 #pragma unroll
             for (int u = 0; u < NV; ++u) {
-                const int i = lane + 64 * u;
-                p[z][u] = plane[i < n4 ? i : n4 - 1];
+#pragma unroll
+                for (int z = 0; z < kSplits; ++z)
+                    if (z0 + z >= splits || lane + 64 * u >= n4) p[z][u] = zero4;
+            }
+#pragma unroll
+            for (int u = 0; u < NV; ++u) {
+#pragma unroll
+                for (int z = 0; z < kSplits; ++z) { t[u].x += p[z][u].x; t[u].y += p[z][u].y; t[u].z += p[z][u].z; t[u].w += p[z][u].w; }
             }
         }
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
-            if (lane + 64 * u >= n4) v[u] = zero4;
-#pragma unroll
-            for (int z = 0; z < kSplits; ++z)
-                if (z >= splits || lane + 64 * u >= n4) p[z][u] = zero4;
-        }
-#pragma unroll
-        for (int u = 0; u < NV; ++u) {
             const int i = lane + 64 * u;
-            float4 t = p[0][u];
-#pragma unroll
-            for (int z = 1; z < kSplits; ++z) { t.x += p[z][u].x; t.y += p[z][u].y; t.z += p[z][u].z; t.w += p[z][u].w; }
-            v[u].x += t.x; v[u].y += t.y; v[u].z += t.z; v[u].w += t.w;
+            if (i >= n4) v[u] = zero4;
+            v[u].x += t[u].x; v[u].y += t[u].y; v[u].z += t[u].z; v[u].w += t[u].w;
             if (i < n4) xr[i] = v[u];
         }
     }
@@ -366,7 +388,7 @@ __global__ void __launch_bounds__(64 * RPW) k_enc_rows(float *x, const float *pa
         if (!in || bias == nullptr) bb[u] = zero4;
     }
     if (gain == nullptr) {
-        if constexpr (!F16_OUT) {
+        if constexpr (OUT == ROWS_RESULT) {
 #pragma unroll
             for (int u = 0; u < NV; ++u)
                 if (lane + 64 * u < n4) reinterpret_cast<float4 *>(params->out + (size_t)row * width)[lane + 64 * u] = v[u];
@@ -392,9 +414,11 @@ __global__ void __launch_bounds__(64 * RPW) k_enc_rows(float *x, const float *pa
         if (i < n4) {
             const float y0 = (v[u].x - mean) * rstd * gg[u].x + bb[u].x, y1 = (v[u].y - mean) * rstd * gg[u].y + bb[u].y;
             const float y2 = (v[u].z - mean) * rstd * gg[u].z + bb[u].z, y3 = (v[u].w - mean) * rstd * gg[u].w + bb[u].w;
-            if constexpr (F16_OUT) {
+            if constexpr (OUT == ROWS_F16) {
                 half4 h = {(_Float16)y0, (_Float16)y1, (_Float16)y2, (_Float16)y3};
-                reinterpret_cast<half4 *>(out_f16 + (size_t)row * width)[i] = h;
+                reinterpret_cast<half4 *>(static_cast<_Float16 *>(out_rows) + (size_t)row * width)[i] = h;
+            } else if constexpr (OUT == ROWS_F32) {
+                reinterpret_cast<float4 *>(static_cast<float *>(out_rows) + (size_t)row * width)[i] = make_float4(y0, y1, y2, y3);
             } else {
                 reinterpret_cast<float4 *>(params->out + (size_t)row * width)[i] = make_float4(y0, y1, y2, y3);
             }
@@ -402,18 +426,17 @@ __global__ void __launch_bounds__(64 * RPW) k_enc_rows(float *x, const float *pa
     }
 }
 
-template <bool F16_OUT>
-void launch_rows(State *st, int width, dim3 grid, float *x, const float *part, int splits, size_t split_stride, const float *gain,
-                 const float *bias, _Float16 *out_f16, const EncParams *params, int rows) {
-    (void)grid;
+template <int OUT>
+void launch_rows(State *st, int width, float *x, const float *part, int splits, size_t split_stride, const float *gain, const float *bias, void *out_rows,
+                 const EncParams *params, int rows) {
     constexpr int kRowsPerWg = 1;
     const dim3 rows_grid((unsigned)((rows + kRowsPerWg - 1) / kRowsPerWg));
     if (width <= 1024)
-        hipLaunchKernelGGL((k_enc_rows<F16_OUT, 4, kRowsPerWg>), rows_grid, dim3(64 * kRowsPerWg), 0, st->stream, x, part, params, rows, width, splits, split_stride,
-                           gain, bias, out_f16);
+        hipLaunchKernelGGL((k_enc_rows<OUT, 4, kRowsPerWg>), rows_grid, dim3(64 * kRowsPerWg), 0, st->stream, x, part, params, rows, width, splits, split_stride,
+                           gain, bias, out_rows);
     else
-        hipLaunchKernelGGL((k_enc_rows<F16_OUT, 16, kRowsPerWg>), rows_grid, dim3(64 * kRowsPerWg), 0, st->stream, x, part, params, rows, width, splits, split_stride,
-                           gain, bias, out_f16);
+        hipLaunchKernelGGL((k_enc_rows<OUT, 16, kRowsPerWg>), rows_grid, dim3(64 * kRowsPerWg), 0, st->stream, x, part, params, rows, width, splits, split_stride,
+                           gain, bias, out_rows);
 }
 
 // One (32-query tile, head): S = scale * Q K^T over all keys (f32, in LDS) -> row softmax numerators
@@ -632,7 +655,6 @@ int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size
     const int w = (int)e->width, f = (int)e->ffn;
     hipLaunchKernelGGL(k_enc_embed, dim3(tpad), dim3(kThreads), 0, st->stream, e->ids, e->params, static_cast<const _Float16 *>(e->tok->data),
                        static_cast<const _Float16 *>(e->pos->data), e->x, w);
-    const dim3 row_grid((tpad + 3) / 4);
     const float scale = 1.0f / sqrtf((float)e->head_width);
     const size_t lds = attention_lds_bytes((size_t)tpad);
     const size_t split_stride = (size_t)tpad * w;
@@ -642,7 +664,7 @@ int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size
     const float *pending = nullptr;   // partials of the last product, not yet added to x
     int pending_splits = 0;
     for (size_t l = 0; l < e->layers; ++l) {
-        launch_rows<true>(st, w, row_grid, e->x, pending, pending_splits, split_stride, e->n1g[l], e->n1b[l], e->nrm, e->params, tpad);
+        launch_rows<ROWS_F16>(st, w, e->x, pending, pending_splits, split_stride, e->n1g[l], e->n1b[l], e->nrm, e->params, tpad);
         GemmArgs g{};
         g.a = e->nrm; g.w = static_cast<const _Float16 *>(e->qkv[l]->data); g.M = tpad; g.N = 3 * w; g.K = w;
         g.out = e->qk; g.vt = e->vt; g.width = w;
@@ -657,7 +679,7 @@ int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size
         g = GemmArgs{};
         g.a = e->ctx; g.w = static_cast<const _Float16 *>(e->o[l]->data); g.M = tpad; g.N = w; g.K = w; g.part = e->part;
         if (launch_gemm<ENC_PARTIAL>(st, g, o_splits, error, capacity) != 0) return -1;
-        launch_rows<true>(st, w, row_grid, e->x, e->part, o_splits, split_stride, e->n2g[l], e->n2b[l], e->nrm, e->params, tpad);
+        launch_rows<ROWS_F16>(st, w, e->x, e->part, o_splits, split_stride, e->n2g[l], e->n2b[l], e->nrm, e->params, tpad);
         g = GemmArgs{};
         g.a = e->nrm; g.M = tpad; g.N = f; g.K = w * taps; g.out = e->hid; g.taps = taps; g.cin = w;
         g.w = taps > 1 ? e->conv_up[l] : static_cast<const _Float16 *>(e->up[l]->data);
@@ -672,118 +694,169 @@ int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size
         pending_splits = down_splits;
     }
     // last residual update, then the final norm (src/graph.c:696-701) or a plain copy when the stack has none
-    launch_rows<false>(st, w, row_grid, e->x, pending, pending_splits, split_stride, e->nog, e->nob, nullptr, e->params, tpad);
+    launch_rows<ROWS_RESULT>(st, w, e->x, pending, pending_splits, split_stride, e->nog, e->nob, nullptr, e->params, tpad);
     return hip_check(hipGetLastError(), "encoder prefill launch", error, capacity);
 }
 
 // ---- f32 operands: the stack as the reference computes it ---------------------------------------------------------------
-// transformer_stack (src/graph.c:634-711) is LayerNorm -> QKV linear -> per head sgemm(Q K^T, alpha = scale) -> masked row
-// softmax -> sgemm(P V) -> O linear -> residual -> LayerNorm -> causal_conv_ffn -> residual, all f32.  This form runs exactly
-// that sequence on the library's f32 operators (LayerNorm rows, the f32 matrix-core product, GELU with tanhf, residual add),
-// so that only the order of additions inside a product differs from the CPU: 1e-5 instead of the 2e-3 of f16 operands.
-// It is the accuracy form, not the fast one: some forty launches per layer, no graph.
+// transformer_stack (src/graph.c:634-711) is LayerNorm -> QKV linear -> per head scaled Q K^T -> masked row softmax -> P V -> O linear
+// -> residual -> LayerNorm -> causal_conv_ffn -> residual, all f32.  This form keeps every value f32 -- only the order of additions
+// inside a product differs from the CPU: 1e-5 instead of the 2e-3 of f16 operands.  The products run on the bf16 matrix cores in
+// three-piece form (split_product.h: f32 operands, f32 sums), scores and P V on the f32 ones, in eight kernels a layer, captured like
+// the f16 form's.  192 tokens, causal, three taps: 3.5 ms as the library's f32 operators one after the other (some forty launches
+// a layer, most of them a fraction of the chip).
 
-// Row r = h * T + t of the scores [heads, T, T]: softmax over the keys the query may see (src/graph.c:446-449 masks key > query;
-// softmax_row_inplace, src/graph.c:245-257: max, exp, sum, divide), zeros behind them.
-__global__ void __launch_bounds__(256) k_enc_softmax_rows(float *scores, int T, int causal) {
-    __shared__ float s4[4];
-    const int t = (int)(blockIdx.x % (unsigned)T);
-    float *row = scores + (size_t)blockIdx.x * T;
-    const int valid = causal ? t + 1 : T;
-    float m = -3.0e38f;
-    for (int i = threadIdx.x; i < valid; i += 256) m = fmaxf(m, row[i]);
-    m = block_max(m, s4);
-    float sum = 0.0f;
-    for (int i = threadIdx.x; i < valid; i += 256) {
-        const float e = expf(row[i] - m);
-        row[i] = e;
-        sum += e;
+// One (32-query tile, head), f32 throughout: S = scale * Q K^T (in LDS) -> softmax numerators and 1 / sum -> P V.
+// Wavefront w scores key tiles w, w + 4, ..; for P V it takes columns 32 * (w % 2) .. over keys half w / 2.  A matrix instruction
+// (v_mfma_f32_32x32x2_f32) takes one value per lane and operand, of inner index l / 32: the scores give lanes below 32 columns 0..31
+// of the head and the rest 32..63, P V gives them keys 0..3 and 4..7 of eight, so that both come in 16-byte reads (any pairing of
+// inner indices is the same sum).  qkv rows are read as they lie: a lane's 128 bytes of its own row cost 64 line visits a
+// request, a quarter of the time the tile's matrix instructions take.
+__global__ void __launch_bounds__(kThreads) k_enc_attention_f32(const float *qkv, float *ctx, const EncParams *params, int tpad, int width, float scale,
+                                                                int causal) {
+    const int tokens = params->tokens;
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ float s_inv[kQTile];
+    __shared__ __align__(16) float s_half[2][16][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hi = lane >> 5;
+    const int q0 = blockIdx.x * kQTile, head = blockIdx.y;
+    const int keys = causal ? q0 + kQTile : tpad;            // what lies behind is masked for every query here; a multiple of 32
+    const int sstride = tpad + kScorePad;
+    float *S = reinterpret_cast<float *>(smem);
+    const size_t stride = 3 * (size_t)width;
+    const float *const base = qkv + head * 64;
+    float fq[32], fk[32];
+    const auto fetch = [&](float (&f)[32], const float *row) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float4 v = *reinterpret_cast<const float4 *>(row + 32 * hi + 4 * i);
+            f[4 * i] = v.x; f[4 * i + 1] = v.y; f[4 * i + 2] = v.z; f[4 * i + 3] = v.w;
+        }
+    };
+    fetch(fq, base + (size_t)(q0 + (lane & 31)) * stride);
+    for (int tile = wave; tile < keys / 32; tile += 4) {
+        fetch(fk, base + width + (size_t)(tile * 32 + (lane & 31)) * stride);
+        floatx16 acc = {0};
+#pragma unroll
+        for (int i = 0; i < 32; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fq[i], fk[i], acc, 0, 0, 0);
+        const int key = tile * 32 + (lane & 31);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const bool seen = key < tokens && (!causal || key <= q0 + acc_row(r, lane));   // src/graph.c:446-449
+            S[acc_row(r, lane) * sstride + key] = seen ? acc[r] * scale : -3.0e38f;
+        }
     }
-    sum = block_sum(sum, s4);
-    for (int i = threadIdx.x; i < T; i += 256) row[i] = i < valid ? row[i] / sum : 0.0f;
+    __syncthreads();
+    {   // softmax_row_inplace (src/graph.c:245-257) of row tid / 8 by eight lanes; the division by the sum is left to the end
+        const int row = tid >> 3, part = tid & 7;
+        float4 *srow = reinterpret_cast<float4 *>(S + row * sstride);
+        const int npieces = keys / 4;
+        float m = -3.0e38f;
+        for (int c = part; c < npieces; c += 8) {
+            const float4 v = srow[c];
+            m = fmaxf(fmaxf(m, fmaxf(v.x, v.y)), fmaxf(v.z, v.w));
+        }
+        m = fmaxf(m, __shfl_xor(m, 1));
+        m = fmaxf(m, __shfl_xor(m, 2));
+        m = fmaxf(m, __shfl_xor(m, 4));
+        float l = 0.0f;
+        for (int c = part; c < npieces; c += 8) {
+            float4 v = srow[c];
+            v.x = expf(v.x - m); v.y = expf(v.y - m); v.z = expf(v.z - m); v.w = expf(v.w - m);
+            l += (v.x + v.y) + (v.z + v.w);
+            srow[c] = v;
+        }
+        l += __shfl_xor(l, 1);
+        l += __shfl_xor(l, 2);
+        l += __shfl_xor(l, 4);
+        if (part == 0) s_inv[row] = 1.0f / l;
+    }
+    __syncthreads();
+    {
+        const int wn = wave & 1, kh = wave >> 1, span = keys / 2;   // a multiple of 16
+        const float *prow = S + (lane & 31) * sstride + kh * span + 4 * hi;
+        const float *vcol = base + 2 * width + (size_t)(kh * span + 4 * hi) * stride + wn * 32 + (lane & 31);
+        floatx16 acc = {0};
+        float fv[2][8];   // sixteen keys of this wavefront's columns, requested a step ahead
+        const auto request = [&](float (&f)[8], int k) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] = vcol[(size_t)(k + 8 * (i >> 2) + (i & 3)) * stride];
+        };
+        const auto multiply = [&](const float (&f)[8], int k) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float4 p = *reinterpret_cast<const float4 *>(prow + k + 8 * j);
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p.x, f[4 * j], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p.y, f[4 * j + 1], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p.z, f[4 * j + 2], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p.w, f[4 * j + 3], acc, 0, 0, 0);
+            }
+        };
+        request(fv[0], 0);
+        for (int k = 0; k < span; k += 32) {
+            request(fv[1], min(k + 16, span - 16));
+            multiply(fv[0], k);
+            request(fv[0], min(k + 32, span - 16));
+            if (k + 16 < span) multiply(fv[1], k + 16);
+        }
+        if (kh == 1) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s_half[wn][r][lane] = acc[r];
+        }
+        __syncthreads();
+        if (kh == 0) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = acc_row(r, lane);
+                ctx[(size_t)(q0 + row) * width + head * 64 + wn * 32 + (lane & 31)] = (acc[r] + s_half[wn][r][lane]) * s_inv[row];
+            }
+        }
+    }
 }
 
-// unfold_causal (src/graph.c:271-286) in the tap-major order of the conv weights here: col[t][j * C + i] = in[t - (taps - 1) + j][i],
-// zero for rows before the first.
-__global__ void __launch_bounds__(256) k_enc_unfold(const float *in, float *col, int T, int C, int taps) {
-    const size_t n = (size_t)T * taps * C;
-    for (size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x; idx < n; idx += (size_t)gridDim.x * 256) {
-        const int i = (int)(idx % (size_t)C);
-        const size_t tj = idx / (size_t)C;
-        const int j = (int)(tj % (size_t)taps);
-        const int t = (int)(tj / (size_t)taps);
-        const int src = t - (taps - 1) + j;
-        col[idx] = src >= 0 ? in[(size_t)src * C + i] : 0.0f;
+// hid = GELU(sum of the up product's splits, in split order); a float4 per thread.
+__global__ void __launch_bounds__(256) k_enc_sum_gelu(const float4 *part, float4 *hid, int pieces, int splits) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= pieces) return;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int z0 = 0; z0 < splits; z0 += 4) {
+        float4 p[4];
+#pragma unroll
+        for (int z = 0; z < 4; ++z) p[z] = part[(size_t)min(z0 + z, splits - 1) * pieces + i];
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+            if (z0 + z < splits) { s.x += p[z].x; s.y += p[z].y; s.z += p[z].z; s.w += p[z].w; }
     }
+    hid[i] = make_float4(gelu_tanh(s.x), gelu_tanh(s.y), gelu_tanh(s.z), gelu_tanh(s.w));
 }
 
-// Conv weight [n][cin][taps] as f32 [n][taps][cin] in device memory (the caller owns it).
-int tap_major_f32(const float *host, size_t n, size_t cin, size_t taps, float **out, char *error, size_t capacity) {
-    *out = nullptr;
-    std::vector<float> packed;
-    try {
-        packed.resize(n * cin * taps);
-    } catch (...) {
-        set_error(error, capacity, "out of memory converting an encoder conv weight");
-        return -1;
-    }
-    for (size_t o = 0; o < n; ++o)
-        for (size_t i = 0; i < cin; ++i)
-            for (size_t j = 0; j < taps; ++j) packed[(o * taps + j) * cin + i] = host[(o * cin + i) * taps + j];
-    void *dev = nullptr;
-    if (hip_check(hipMalloc(&dev, packed.size() * sizeof(float)), "encoder conv weight", error, capacity) != 0) return -1;
-    if (hip_check(hipMemcpy(dev, packed.data(), packed.size() * sizeof(float), hipMemcpyHostToDevice), "encoder conv weight upload", error, capacity) != 0) {
-        (void)hipFree(dev);
-        return -1;
-    }
-    *out = static_cast<float *>(dev);
-    return 0;
-}
+constexpr size_t kMaxSplitsF32 = 12;   // planes of partial sums; the next pass reads them all
 
-int f32_matrix(State *st, const float *host, size_t n, size_t k, const CachedWeight **out, char *error, size_t capacity) {
-    return cached_matrix(st, host, n, k, MYNAH_HIP_F32, out, error, capacity);
-}
-
-int prefill_f32(State *st, mynah_hip_encoder *e, int T, float *dev_out, char *error, size_t capacity) {
-    const size_t w = e->width, f = e->ffn, taps = e->taps, heads = e->heads, hw = e->head_width;
-    const float scale = 1.0f / sqrtf((float)hw);
-    const float *tables[1] = {static_cast<const float *>(e->tok32->data)};
-    if (launch_gather(st, tables, 1, e->f_ids, (size_t)T, w, 1.0f, static_cast<const float *>(e->pos32->data), e->x, error, capacity) != 0) return -1;
+int enqueue_prefill_f32(State *st, mynah_hip_encoder *e, int tpad, char *error, size_t capacity) {
+    const size_t w = e->width, f = e->ffn, taps = e->taps, rows = (size_t)tpad;
+    const float scale = 1.0f / sqrtf((float)e->head_width);
+    hipLaunchKernelGGL(k_enc_embed_f32, dim3(tpad), dim3(kThreads), 0, st->stream, e->ids, e->params, static_cast<const float *>(e->tok32->data),
+                       static_cast<const float *>(e->pos32->data), e->x, (int)w);
+    const int o_splits = split_product_splits(st, rows, w, w, kMaxSplitsF32), up_splits = split_product_splits(st, rows, w, f, kMaxSplitsF32),
+              down_splits = split_product_splits(st, rows, f, w, kMaxSplitsF32);
+    const float *pending = nullptr;   // partial sums of the last product, not yet added to x
     for (size_t l = 0; l < e->layers; ++l) {
-        if (launch_layernorm(st, e->x, e->f_nrm, e->n1g[l], e->n1b[l], (size_t)T, w, error, capacity) != 0) return -1;
-        if (launch_gemm_f32(st, e->f_nrm, e->f_qkv, (size_t)T, w, 3 * w, e->qkv32[l], nullptr, error, capacity) != 0) return -1;
-        for (size_t h = 0; h < heads; ++h)   // scores_h = scale * Q_h K_h^T (src/graph.c:428-445)
-            if (launch_sgemm(st, 0, 1, (size_t)T, (size_t)T, hw, scale, e->f_qkv + h * hw, 3 * w, e->f_qkv + w + h * hw, 3 * w, 0.0f,
-                             e->f_scores + h * (size_t)T * T, (size_t)T, error, capacity) != 0)
-                return -1;
-        hipLaunchKernelGGL(k_enc_softmax_rows, dim3((unsigned)(heads * (size_t)T)), dim3(256), 0, st->stream, e->f_scores, T, e->causal);
-        MYNAH_TRY(hipGetLastError());
-        for (size_t h = 0; h < heads; ++h)   // ctx_h = P_h V_h (src/graph.c:451-462)
-            if (launch_sgemm(st, 0, 0, (size_t)T, hw, (size_t)T, 1.0f, e->f_scores + h * (size_t)T * T, (size_t)T, e->f_qkv + 2 * w + h * hw, 3 * w, 0.0f,
-                             e->f_ctx + h * hw, w, error, capacity) != 0)
-                return -1;
-        if (launch_gemm_f32(st, e->f_ctx, e->f_tmp, (size_t)T, w, w, e->o32[l], nullptr, error, capacity) != 0) return -1;
-        if (launch_residual(st, e->x, e->f_tmp, (size_t)T * w, error, capacity) != 0) return -1;
-        if (launch_layernorm(st, e->x, e->f_nrm, e->n2g[l], e->n2b[l], (size_t)T, w, error, capacity) != 0) return -1;
-        const float *up_in = e->f_nrm;
-        if (taps > 1) {
-            hipLaunchKernelGGL(k_enc_unfold, dim3(1024), dim3(256), 0, st->stream, e->f_nrm, e->f_col, T, (int)w, (int)taps);
-            MYNAH_TRY(hipGetLastError());
-            up_in = e->f_col;
-        }
-        if (launch_gemm_f32(st, up_in, e->f_hid, (size_t)T, w * taps, f, e->up32[l], nullptr, error, capacity) != 0) return -1;
-        if (launch_gelu(st, e->f_hid, (size_t)T * f, error, capacity) != 0) return -1;
-        const float *down_in = e->f_hid;
-        if (taps > 1) {
-            hipLaunchKernelGGL(k_enc_unfold, dim3(1024), dim3(256), 0, st->stream, e->f_hid, e->f_col, T, (int)f, (int)taps);
-            MYNAH_TRY(hipGetLastError());
-            down_in = e->f_col;
-        }
-        if (launch_gemm_f32(st, down_in, e->f_tmp, (size_t)T, f * taps, w, e->down32[l], nullptr, error, capacity) != 0) return -1;
-        if (launch_residual(st, e->x, e->f_tmp, (size_t)T * w, error, capacity) != 0) return -1;
+        launch_rows<ROWS_F32>(st, (int)w, e->x, pending, down_splits, rows * w, e->n1g[l], e->n1b[l], e->f_nrm, e->params, tpad);
+        // (not split: the attention kernel reads every row several times and would add the planes up as often)
+        if (launch_split_product(st, e->f_nrm, e->qkv32[l], rows, w, 1, 3 * w, 1, e->f_qkv, error, capacity) != 0) return -1;
+        hipLaunchKernelGGL(k_enc_attention_f32, dim3(tpad / kQTile, (unsigned)e->heads), dim3(kThreads), attention_lds_bytes(rows), st->stream, e->f_qkv, e->f_ctx,
+                           e->params, tpad, (int)w, scale, e->causal);
+        if (launch_split_product(st, e->f_ctx, e->o32[l], rows, w, 1, w, o_splits, e->part, error, capacity) != 0) return -1;
+        launch_rows<ROWS_F32>(st, (int)w, e->x, e->part, o_splits, rows * w, e->n2g[l], e->n2b[l], e->f_nrm, e->params, tpad);
+        if (launch_split_product(st, e->f_nrm, e->up32[l], rows, w, taps, f, up_splits, e->part, error, capacity) != 0) return -1;
+        const int pieces = (int)(rows * f / 4);
+        hipLaunchKernelGGL(k_enc_sum_gelu, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st->stream, reinterpret_cast<const float4 *>(e->part),
+                           reinterpret_cast<float4 *>(e->f_hid), pieces, up_splits);
+        if (launch_split_product(st, e->f_hid, e->down32[l], rows, f, taps, w, down_splits, e->part, error, capacity) != 0) return -1;
+        pending = e->part;
     }
-    if (e->nog != nullptr) return launch_layernorm(st, e->x, dev_out, e->nog, e->nob, (size_t)T, w, error, capacity);
-    return launch_copy(st, dev_out, e->x, (size_t)T * w, error, capacity);
+    launch_rows<ROWS_RESULT>(st, (int)w, e->x, pending, down_splits, rows * w, e->nog, e->nob, nullptr, e->params, tpad);
+    return hip_check(hipGetLastError(), "encoder prefill launch", error, capacity);
 }
 
 }  // namespace
@@ -826,8 +899,8 @@ extern "C" int mynah_hip_encoder_create(void *state, const mynah_hip_encoder_des
     }
     e->f32 = d->operands_f32 != 0;
     if (e->f32) {
-        if (f32_matrix(st, d->tok_table, d->vocab, d->width, &e->tok32, error, capacity) != 0) return fail();
-        if (f32_matrix(st, d->pos_table, d->max_positions, d->width, &e->pos32, error, capacity) != 0) return fail();
+        if (cached_matrix(st, d->tok_table, d->vocab, d->width, MYNAH_HIP_F32, &e->tok32, error, capacity) != 0) return fail();
+        if (cached_matrix(st, d->pos_table, d->max_positions, d->width, MYNAH_HIP_F32, &e->pos32, error, capacity) != 0) return fail();
     } else {
         if (f16_matrix(st, d->tok_table, d->vocab, d->width, &e->tok, error, capacity) != 0) return fail();
         if (f16_matrix(st, d->pos_table, d->max_positions, d->width, &e->pos, error, capacity) != 0) return fail();
@@ -841,24 +914,15 @@ extern "C" int mynah_hip_encoder_create(void *state, const mynah_hip_encoder_des
             return fail();
         }
         if (e->f32) {
-            if (f32_matrix(st, d->qkv_w[l], 3 * d->width, d->width, &cw, error, capacity) != 0) return fail();
-            e->qkv32.push_back(static_cast<const float *>(cw->data));
-            if (f32_matrix(st, d->o_w[l], d->width, d->width, &cw, error, capacity) != 0) return fail();
-            e->o32.push_back(static_cast<const float *>(cw->data));
-            if (e->taps == 1) {
-                if (f32_matrix(st, d->up_w[l], d->ffn_width, d->width, &cw, error, capacity) != 0) return fail();
-                e->up32.push_back(static_cast<const float *>(cw->data));
-                if (f32_matrix(st, d->down_w[l], d->width, d->ffn_width, &cw, error, capacity) != 0) return fail();
-                e->down32.push_back(static_cast<const float *>(cw->data));
-            } else {
-                float *dev = nullptr;
-                if (tap_major_f32(d->up_w[l], d->ffn_width, d->width, e->taps, &dev, error, capacity) != 0) return fail();
-                e->conv32.push_back(dev);
-                e->up32.push_back(dev);
-                if (tap_major_f32(d->down_w[l], d->width, d->ffn_width, e->taps, &dev, error, capacity) != 0) return fail();
-                e->conv32.push_back(dev);
-                e->down32.push_back(dev);
-            }
+            const float4 *packed = nullptr;
+            if (cached_split_weight(st, d->qkv_w[l], 3 * d->width, d->width, 1, &packed, error, capacity) != 0) return fail();
+            e->qkv32.push_back(packed);
+            if (cached_split_weight(st, d->o_w[l], d->width, d->width, 1, &packed, error, capacity) != 0) return fail();
+            e->o32.push_back(packed);
+            if (cached_split_weight(st, d->up_w[l], d->ffn_width, d->width, e->taps, &packed, error, capacity) != 0) return fail();
+            e->up32.push_back(packed);
+            if (cached_split_weight(st, d->down_w[l], d->width, d->ffn_width, e->taps, &packed, error, capacity) != 0) return fail();
+            e->down32.push_back(packed);
         } else {
         if (f16_matrix(st, d->qkv_w[l], 3 * d->width, d->width, &cw, error, capacity) != 0) return fail();
         e->qkv.push_back(cw);
@@ -896,37 +960,36 @@ extern "C" int mynah_hip_encoder_create(void *state, const mynah_hip_encoder_des
         return hip_check(hipMemsetAsync(*p, 0, bytes, st->stream), "encoder workspace clear", error, capacity);
     };
     if (e->f32) {
-        const size_t T = d->max_positions, wide = (w > f ? w : f) * e->taps;
-        if (alloc(reinterpret_cast<void **>(&e->x), T * w * sizeof(float)) != 0 || alloc(reinterpret_cast<void **>(&e->f_nrm), T * w * sizeof(float)) != 0 ||
-            alloc(reinterpret_cast<void **>(&e->f_qkv), T * 3 * w * sizeof(float)) != 0 ||
-            alloc(reinterpret_cast<void **>(&e->f_scores), e->heads * T * T * sizeof(float)) != 0 ||
-            alloc(reinterpret_cast<void **>(&e->f_ctx), T * w * sizeof(float)) != 0 || alloc(reinterpret_cast<void **>(&e->f_hid), T * f * sizeof(float)) != 0 ||
-            alloc(reinterpret_cast<void **>(&e->f_col), T * wide * sizeof(float)) != 0 || alloc(reinterpret_cast<void **>(&e->f_tmp), T * w * sizeof(float)) != 0 ||
-            alloc(reinterpret_cast<void **>(&e->f_ids), T * sizeof(int)) != 0)
+        const size_t pad = kSplitOverrun, wide = (w > f ? w : f) * kMaxSplitsF32;
+        if (alloc(reinterpret_cast<void **>(&e->x), tp * w * sizeof(float)) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->f_nrm_alloc), ((kLeadRows + tp) * w + pad) * sizeof(float)) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->f_qkv), tp * 3 * w * sizeof(float)) != 0 || alloc(reinterpret_cast<void **>(&e->f_ctx), (tp * w + pad) * sizeof(float)) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->f_hid_alloc), ((kLeadRows + tp) * f + pad) * sizeof(float)) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->part), tp * wide * sizeof(float)) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->ids), tp * sizeof(int) + sizeof(EncParams)) != 0)
             return fail();
-        if (hip_check(hipHostMalloc(reinterpret_cast<void **>(&e->ids_host), T * sizeof(int), hipHostMallocDefault), "encoder ids staging", error, capacity) != 0)
+        e->f_nrm = e->f_nrm_alloc + kLeadRows * w;   // rows -2 and -1 stay zero
+        e->f_hid = e->f_hid_alloc + kLeadRows * f;
+    } else {
+        if (alloc(reinterpret_cast<void **>(&e->x), tp * w * sizeof(float)) != 0 || alloc(reinterpret_cast<void **>(&e->nrm_alloc), (kLeadRows + tp) * w * 2) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->qk), tp * 2 * w * 2) != 0 || alloc(reinterpret_cast<void **>(&e->vt), w * tp * 2) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->ctx), tp * w * 2) != 0 || alloc(reinterpret_cast<void **>(&e->hid_alloc), (kLeadRows + tp) * f * 2) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->ids), tp * sizeof(int) + sizeof(EncParams)) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->part), kMaxSplits * tp * w * sizeof(float)) != 0)
             return fail();
-        if (hip_check(hipStreamSynchronize(st->stream), "encoder create", error, capacity) != 0) return fail();
-        *out = e;
-        return 0;
+        e->nrm = e->nrm_alloc + kLeadRows * w;   // rows -2 and -1 stay zero; widths are multiples of 64, so both stay 16-byte aligned
+        e->hid = e->hid_alloc + kLeadRows * f;
     }
-    if (alloc(reinterpret_cast<void **>(&e->x), tp * w * sizeof(float)) != 0 || alloc(reinterpret_cast<void **>(&e->nrm_alloc), (kLeadRows + tp) * w * 2) != 0 ||
-        alloc(reinterpret_cast<void **>(&e->qk), tp * 2 * w * 2) != 0 || alloc(reinterpret_cast<void **>(&e->vt), w * tp * 2) != 0 ||
-        alloc(reinterpret_cast<void **>(&e->ctx), tp * w * 2) != 0 || alloc(reinterpret_cast<void **>(&e->hid_alloc), (kLeadRows + tp) * f * 2) != 0 ||
-        alloc(reinterpret_cast<void **>(&e->ids), tp * sizeof(int) + sizeof(EncParams)) != 0 ||
-        alloc(reinterpret_cast<void **>(&e->part), kMaxSplits * tp * w * sizeof(float)) != 0)
-        return fail();
     if (hip_check(hipHostMalloc(reinterpret_cast<void **>(&e->ids_host), tp * sizeof(int) + sizeof(EncParams), hipHostMallocDefault),
                   "encoder ids staging", error, capacity) != 0)
         return fail();
     e->params = reinterpret_cast<EncParams *>(e->ids + tp);   // tp is a multiple of 64: 8-byte aligned
-    e->nrm = e->nrm_alloc + kLeadRows * w;   // rows -2 and -1 stay zero; widths are multiples of 64, so both stay 16-byte aligned
-    e->hid = e->hid_alloc + kLeadRows * f;
     if (attention_lds_bytes(e->tpad_max) > 48 * 1024) {
         const int bytes = (int)attention_lds_bytes(e->tpad_max);
         if (hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<1, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
             hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
-            hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<4, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0)
+            hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<4, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
+            hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention_f32), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0)
             return fail();
     }
     if (hip_check(hipStreamSynchronize(st->stream), "encoder create", error, capacity) != 0) return fail();
@@ -944,8 +1007,7 @@ extern "C" void mynah_hip_encoder_destroy(void *state, mynah_hip_encoder *e) {
         if (p != nullptr) (void)hipFree(p);
     for (_Float16 *p : e->conv_up) (void)hipFree(p);
     for (_Float16 *p : e->conv_down) (void)hipFree(p);
-    for (float *p : e->conv32) (void)hipFree(p);
-    for (void *p : {(void *)e->f_nrm, (void *)e->f_qkv, (void *)e->f_scores, (void *)e->f_ctx, (void *)e->f_hid, (void *)e->f_col, (void *)e->f_tmp, (void *)e->f_ids})
+    for (void *p : {(void *)e->f_nrm_alloc, (void *)e->f_qkv, (void *)e->f_ctx, (void *)e->f_hid_alloc})
         if (p != nullptr) (void)hipFree(p);
     if (e->ids_host != nullptr) (void)hipHostFree(e->ids_host);
     delete e;
@@ -968,17 +1030,12 @@ extern "C" int mynah_hip_encoder_prefill(void *state, mynah_hip_encoder *e, cons
             return -1;
         }
     }
+    if (e->f32 && dev_embed_f16 != nullptr) {
+        set_error(error, capacity, "encoder_prefill: with f32 operands there are no f16 token rows to return");
+        return -1;
+    }
     // the staging buffer of the previous call may still be in flight
     MYNAH_TRY(hipStreamSynchronize(st->stream));
-    if (e->f32) {
-        if (dev_embed_f16 != nullptr) {
-            set_error(error, capacity, "encoder_prefill: with f32 operands there are no f16 token rows to return");
-            return -1;
-        }
-        for (size_t t = 0; t < tokens; ++t) e->ids_host[t] = ids[t];
-        MYNAH_TRY(hipMemcpyAsync(e->f_ids, e->ids_host, tokens * sizeof(int), hipMemcpyHostToDevice, st->stream));
-        return prefill_f32(st, e, (int)tokens, dev_out, error, capacity);
-    }
     const size_t tp = e->tpad_max;
     for (size_t t = 0; t < tokens; ++t) e->ids_host[t] = ids[t];
     EncParams *hp = reinterpret_cast<EncParams *>(e->ids_host + tp);
@@ -989,16 +1046,17 @@ extern "C" int mynah_hip_encoder_prefill(void *state, mynah_hip_encoder *e, cons
     MYNAH_TRY(hipMemcpyAsync(e->ids, e->ids_host, tokens * sizeof(int), hipMemcpyHostToDevice, st->stream));
     MYNAH_TRY(hipMemcpyAsync(e->params, hp, sizeof(EncParams), hipMemcpyHostToDevice, st->stream));
 
-    const int tpad = ((int)tokens + kTile - 1) / kTile * kTile;
+    const int granule = e->f32 ? kQTile : kTile, tpad = ((int)tokens + granule - 1) / granule * granule;
+    const auto enqueue = e->f32 ? enqueue_prefill_f32 : enqueue_prefill;
     if (!st->graph_mode || e->eager_runs[tpad] == 0) {
         e->eager_runs[tpad] = 1;
-        return enqueue_prefill(st, e, tpad, error, capacity);
+        return enqueue(st, e, tpad, error, capacity);
     }
     hipGraphExec_t &exec = e->graphs[tpad];
     if (exec == nullptr) {
         hipGraph_t graph = nullptr;
         MYNAH_TRY(hipStreamBeginCapture(st->stream, hipStreamCaptureModeThreadLocal));
-        const int rc = enqueue_prefill(st, e, tpad, error, capacity);
+        const int rc = enqueue(st, e, tpad, error, capacity);
         const hipError_t end = hipStreamEndCapture(st->stream, &graph);
         if (rc != 0 || end != hipSuccess) {
             if (graph != nullptr) (void)hipGraphDestroy(graph);
