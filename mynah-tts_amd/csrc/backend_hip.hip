@@ -224,42 +224,54 @@ int cached_matrix(State *st, const float *host, size_t n, size_t k, int want_qty
     return 0;
 }
 
+// A weight's f32 values on the device, for a kernel on the backend's stream to rearrange (the next weight waits for it there).
+static int stage_weight(State *st, const float *host, size_t count, char *error, size_t capacity) {
+    if (st->pack_staging_floats < count) {
+        if (st->pack_staging != nullptr) {
+            MYNAH_TRY(hipStreamSynchronize(st->stream));   // an earlier weight's kernel may still read it
+            (void)hipFree(st->pack_staging);
+            st->pack_staging = nullptr;
+            st->pack_staging_floats = 0;
+        }
+        MYNAH_TRY(hipMalloc(reinterpret_cast<void **>(&st->pack_staging), count * sizeof(float)));
+        st->pack_staging_floats = count;
+    }
+    return copy_to_device(st, st->pack_staging, host, count * sizeof(float), error, capacity);
+}
+
 int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch, size_t kernel, ConvBlocks *out, char *error, size_t capacity) {
     if (host == nullptr || out_ch == 0 || in_ch == 0 || kernel == 0 || kernel > 64 || in_ch > (size_t)(INT_MAX / 64) ||
         out_ch > SIZE_MAX / in_ch / kernel / sizeof(float)) {
         set_error(error, capacity, "invalid convolution weight");
         return -1;
     }
-    const size_t tiles = ((out_ch + 31) / 32 + 1) & ~(size_t)1, blocks = ((in_ch + kConvChannels - 1) / kConvChannels + 3) & ~(size_t)3;
-    const size_t row = kConvChannels * kernel + 4, chunk = conv_chunk_floats(kernel);
+    const size_t tiles = (out_ch + 31) / 32, blocks = (in_ch + 15) / 16;
     out->tiles = (int)tiles;
     out->blocks = (int)blocks;
     const WeightKey key{host, out_ch * in_ch * kernel * sizeof(float), (int)(64 + kernel + 32 * in_ch)};
     std::lock_guard<std::mutex> lock(st->mu);
     auto it = st->weights.find(key);
     if (it != st->weights.end()) {
-        out->data = static_cast<const float *>(it->second.data);
+        out->data = static_cast<const uint4 *>(it->second.data);
         return 0;
     }
-    if (tiles > (size_t)INT_MAX || tiles * blocks > SIZE_MAX / sizeof(float) / chunk / 2) {
+    if (tiles > (size_t)INT_MAX || tiles * blocks > SIZE_MAX / (kernel * 3072) / 2) {
         set_error(error, capacity, "convolution weight too large");
         return -1;
     }
-    std::vector<float> packed(tiles * blocks * chunk + 1024, 0.0f);
-    for (size_t o = 0; o < out_ch; ++o)
-        for (size_t i = 0; i < in_ch; ++i) {
-            float *dst = packed.data() + ((i / kConvChannels) * tiles + o / 32) * chunk + (o % 32) * row + (i % kConvChannels) * kernel;
-            const float *src = host + (o * in_ch + i) * kernel;
-            for (size_t k = 0; k < kernel; ++k) dst[k] = src[k];
-        }
     CachedWeight cw;
     cw.n = out_ch;
     cw.k = in_ch * kernel;
-    cw.bytes = packed.size() * sizeof(float);
-    if (device_copy_of(packed.data(), cw.bytes, &cw.data, error, capacity) != 0) return -1;
+    cw.bytes = (tiles * blocks + 5) * kernel * 3072 + kSplitWeightOverrun;   // (the kernels request up to five blocks past the end)
+    if (stage_weight(st, host, out_ch * in_ch * kernel, error, capacity) != 0) return -1;
+    MYNAH_TRY(hipMalloc(&cw.data, cw.bytes));
+    if (launch_conv_pack(st, st->pack_staging, static_cast<uint4 *>(cw.data), out_ch, in_ch, kernel, error, capacity) != 0) {
+        (void)hipFree(cw.data);
+        return -1;
+    }
     st->weight_bytes += cw.bytes;
     st->weights.emplace(key, cw);
-    out->data = static_cast<const float *>(cw.data);
+    out->data = static_cast<const uint4 *>(cw.data);
     return 0;
 }
 
@@ -276,24 +288,13 @@ int cached_split_weight(State *st, const float *host, size_t n, size_t channels,
         *out = static_cast<const float4 *>(it->second.data);
         return 0;
     }
-    if (st->pack_staging_floats < count) {
-        if (st->pack_staging != nullptr) {
-            MYNAH_TRY(hipStreamSynchronize(st->stream));   // the packing of an earlier weight may still read it
-            (void)hipFree(st->pack_staging);
-            st->pack_staging = nullptr;
-            st->pack_staging_floats = 0;
-        }
-        MYNAH_TRY(hipMalloc(reinterpret_cast<void **>(&st->pack_staging), count * sizeof(float)));
-        st->pack_staging_floats = count;
-    }
+    if (stage_weight(st, host, count, error, capacity) != 0) return -1;
     CachedWeight cw;
     cw.n = n;
     cw.k = channels * taps;
     cw.bytes = count * sizeof(float) + kSplitWeightOverrun;
     MYNAH_TRY(hipMalloc(&cw.data, cw.bytes));
-    // one stream, in order: upload, rearrange (the next weight's upload waits for it); pageable source, taken when the call returns
-    if (hip_check(hipMemcpyAsync(st->pack_staging, host, count * sizeof(float), hipMemcpyHostToDevice, st->stream), "weight upload", error, capacity) != 0 ||
-        launch_split_pack(st, st->pack_staging, static_cast<float4 *>(cw.data), n, channels, taps, error, capacity) != 0) {
+    if (launch_split_pack(st, st->pack_staging, static_cast<float4 *>(cw.data), n, channels, taps, error, capacity) != 0) {
         (void)hipFree(cw.data);
         return -1;
     }

@@ -5,10 +5,10 @@
 //
 //   conv1d          out[o][t] = bias[o] + sum_i sum_k w[(o*in + i)*K + k] * in[i][t - (K-1-k)*dilation]   (conv1d_causal,
 //                   src/graph.c:2010-2160).  The reference builds an im2col matrix and calls sgemm; here the same GEMM
-//                   (M = out channels, N = length, inner = in channels x taps) runs on the f32 matrix cores with the
-//                   im2col done by addressing: a workgroup stages the input rows of eight channels once, with a halo of
-//                   (K-1)*dilation positions, and every tap reads the same rows at its own offset.  f32 operands,
-//                   f32 accumulation (v_mfma_f32_32x32x2_f32); only the order of the additions differs from the CPU's.
+//                   (M = out channels, N = length, inner = in channels x taps) runs on the bf16 matrix cores in three-piece
+//                   form (split_product.h: f32 operands, f32 accumulation, the accuracy of an f32 product) with the im2col
+//                   done by addressing: a workgroup stages the input rows of sixteen channels once, with a halo of
+//                   (K-1)*dilation positions, and every tap reads the same rows at its own offset.
 //   conv_transpose  grouped, trimmed to output_length (conv_transpose_causal / convt_channel, src/graph.c:2179-2231):
 //                   one thread per output element, contributions added in the reference's order (input channel, then
 //                   input position), so the result is bit-identical to the scalar CPU loop.
@@ -18,14 +18,13 @@
 
 #include <type_traits>
 
-#include "kernels.h"
+#include "split_product.h"
 
 using namespace mynah;
 
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef f32x16 floatx16;
 
 constexpr int kConvMaxKernel = 16;
 constexpr int kConvMaxHalo = 128;     // (kernel - 1) * dilation
@@ -102,174 +101,203 @@ __device__ __forceinline__ void conv_emit(const ConvArgs &a, int m, size_t index
     }
 }
 
-// The products of one staged block of eight input channels for a wavefront's 32 x 64 tile.  The two inner indices one
-// matrix instruction consumes are the same tap of two neighbouring channels (lanes 0-31: the even channel, lanes 32-63:
-// the odd one), so a lane walks its channel's taps with plain increments.  wrow: this lane's output row at its first
-// channel; irow: its first channel's staged row at its output position.
-// With the tap count known at compile time the operands are requested TWO products ahead and the scheduler is fenced
-// around every product: left to itself the compiler reads a product's input operand into one and the same register right
-// before it, and with one wavefront on a SIMD every product then waits out an LDS read (some 120 cycles against the 64
-// of the instruction itself).  Past the last product the requests stay inside the staging area and are not used.
-// pairs: channel pairs of the block that exist (the tensor's last block may hold fewer than four; the rest is zeros in
-// both operands and is left out -- the same for every lane of the wavefront).
-template <int KF, int NT = 2>
-__device__ __forceinline__ void conv_products(const float *wrow, const float *irow, const int kernel_arg, const int dilation, const int win,
-                                              floatx16 &acc0, floatx16 &acc1, const int pairs = kConvChannels / 2) {
-    if constexpr (KF != 0) {
-        constexpr int kSteps = (kConvChannels / 2) * KF;
-        float wv[3], x0[3], x1[3];
-        int tap = 0;
-        const auto request = [&](int slot) {
-            wv[slot] = wrow[0];
-            x0[slot] = irow[0];
-            x1[slot] = NT > 1 ? irow[32] : 0.0f;
-            const bool wrap = tap + 1 == KF;   // then: the first tap of the next channel pair
-            wrow += wrap ? KF + 1 : 1;
-            irow += wrap ? 2 * win - (KF - 1) * dilation : dilation;
-            tap = wrap ? 0 : tap + 1;
-        };
-        request(0);
-        request(1);
+// The convolution's inner dimension goes in steps of one tap of sixteen input channels: one 16-deep matrix instruction per pair of
+// pieces.  Weights: taken apart once, when they are cached, in the order of the steps (ConvBlocks), so that a wavefront's three
+// pieces of a step are three requests of 1 KiB straight to its registers -- a weight serves length / 64 wavefronts, and taking it
+// apart there would cost each of them 44 vector instructions a step.  Inputs: a staged (position, eight channels) is 16 bytes
+// of LDS per piece, so a tap's operand is 512 consecutive bytes for 32 positions, whatever the tap's offset.
+// (108 channels x 16384, taps 3 / 7 / 11 in one launch: 70 us with f32 instructions, which have the matrix cores busy for 59 us; the six
+// bf16 instructions of a step are busy for 24.)
+struct ConvWeights {   // the weight pieces of one row tile, requested kAhead steps before they are multiplied
+    static constexpr int kAhead = 3;
+    const uint4 *next;
+    size_t skip;       // from the end of a block to the next one this wavefront multiplies
+    int tap = 0;       // of the next request (a constant wherever the tap count is one)
+    uint4 ring[kAhead][3];
+    __device__ __forceinline__ void request(int slot, int taps) {
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            if (s % KF == 0 && s != 0 && s / KF >= pairs) break;   // (looked at where a pair begins)
-            request((s + 2) % 3);
-            __builtin_amdgcn_sched_barrier(0x77);
-            acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[s % 3], x0[s % 3], acc0, 0, 0, 0);
-            if constexpr (NT > 1) acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[s % 3], x1[s % 3], acc1, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0x77);
+        for (int q = 0; q < 3; ++q) ring[slot][q] = next[64 * q];
+        next += 192;
+        if (++tap == taps) {
+            tap = 0;
+            next += skip;
         }
-        return;
     }
-    const int kernel = kernel_arg;
-    float wv = wrow[0], x0 = irow[0], x1 = NT > 1 ? irow[32] : 0.0f;
+    // (what runs past the last step is requested and not used: the cache pads its copies)
+    __device__ __forceinline__ ConvWeights(const uint4 *first, size_t skip_arg, int taps) : next(first), skip(skip_arg) {
 #pragma unroll
-    for (int pair = 0; pair < kConvChannels / 2; ++pair) {
-        for (int k = 0; k < kernel; ++k) {
-            // the product after this one: the next tap, or the first tap of the next channel pair
-            const bool wrap = k + 1 == kernel;
-            wrow += wrap ? kernel + 1 : 1;
-            irow += wrap ? 2 * win - (kernel - 1) * dilation : dilation;
-            const float nw = wrow[0], n0 = irow[0], n1 = NT > 1 ? irow[32] : 0.0f;
-            acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(wv, x0, acc0, 0, 0, 0);
-            if constexpr (NT > 1) acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(wv, x1, acc1, 0, 0, 0);
-            wv = nw; x0 = n0; x1 = n1;
+        for (int i = 0; i < kAhead; ++i) request(i, taps);
+    }
+};
+
+// The products of the blocks of sixteen channels a wavefront multiplies, for its 32 rows x (32 * NT) positions.
+// stage(block): makes the block's inputs readable and returns where this lane's first operand lies: element [piece * piece_stride +
+// position], lanes 32.. eight channels on.  With the tap count known (KF) the loop over a block's steps is unrolled, and three blocks at
+// a time, after which the weights' registers repeat.  (A step's fragments are read right before it: two or three wavefronts share a
+// SIMD, and a second set of fragment registers, read a step ahead, spilled: 1884 against 1754 us for a 64-frame decode.)
+template <int KF, int NT, class Stage>
+__device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, const int dilation, const int piece_stride, const int blocks, const Stage stage,
+                                              floatx16 (&acc)[NT]) {
+    bf16x8 x[NT][3];
+    const auto read = [&](const uint4 *at) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) x[n][q] = __builtin_bit_cast(bf16x8, at[q * piece_stride + 32 * n]);
+    };
+    const auto multiply = [&](int slot) {
+        bf16x8 fw[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) fw[q] = __builtin_bit_cast(bf16x8, w.ring[slot][q]);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = split_multiply(fw, x[n], acc[n]);
+    };
+    if constexpr (KF != 0) {
+        for (int block = 0;;) {
+#pragma unroll
+            for (int u = 0; u < ConvWeights::kAhead; ++u) {
+                const uint4 *at = stage(block);
+#pragma unroll
+                for (int tap = 0; tap < KF; ++tap) {
+                    const int s = u * KF + tap;
+                    read(at + tap * dilation);
+                    multiply(s % ConvWeights::kAhead);
+                    w.request(s % ConvWeights::kAhead, KF);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (++block == blocks) return;
+            }
+        }
+    } else {
+        for (int block = 0; block < blocks; ++block) {
+            const uint4 *at = stage(block);
+            for (int tap = 0; tap < taps; ++tap) {
+                read(at + tap * dilation);
+                multiply(0);
+#pragma unroll
+                for (int i = 0; i + 1 < ConvWeights::kAhead; ++i)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) w.ring[i][q] = w.ring[i + 1][q];
+                w.request(ConvWeights::kAhead - 1, taps);
+            }
         }
     }
 }
 
+// One (position, eight channels) on its way to LDS: eight requests, then the pieces of the eight values.
+struct ConvColumn {
+    float v[8];
+    // rows channel .. channel + 7 of the input at position t (channel is the same for every lane); a channel the input does not
+    // have repeats its last one -- its weights are zeros
+    __device__ __forceinline__ void request(const ConvArgs &a, int channel, int t) {
+        const float *const at = a.in + t;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = at[(size_t)min(channel + e, a.in_ch - 1) * a.length];
+    }
+    __device__ __forceinline__ void store(uint4 *at, int piece_stride, bool inside) const {
+        bf16x8 p[3];
+        float u[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) u[e] = inside ? v[e] : 0.0f;   // (in front of the row)
+        split_eight(make_float4(u[0], u[1], u[2], u[3]), make_float4(u[4], u[5], u[6], u[7]), p);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) at[q * piece_stride] = __builtin_bit_cast(uint4, p[q]);
+    }
+};
+
 // Workgroup tile: (32 * WM) output channels x (64 * WN) positions; a wavefront owns 32 x 64 (two 32 x 32 accumulators).
-// KF: number of taps known at compile time (0 = from the arguments): the staging loops then have exactly as many slots as
-// the block has 16-byte pieces and the product loop is straight-line code.  The codec's 3, 7 and 11 taps get such builds.
-// The weights arrive cut into chunks (ConvBlocks): the tile's block of a step is WM whole chunks in a row, already in the
-// layout LDS keeps, so staging it is a plain copy -- no index arithmetic, no bounds.
+// KF: number of taps known at compile time (0 = from the arguments); the codec's 3, 7 and 11 taps get such builds.
 // FUSED: the build that mynah_hip_conv1d_fused launches (residuals, scale, activation after the products); the seam's
 // conv1d keeps a build without any of it.
+// Two stages of one block of channels: a block is stored while the one before it is multiplied (by other wavefronts: three
+// to a SIMD), its requests leave a block earlier.
 // (the tile's work as a function: the kernel of one convolution and the kernel of several side by side both run it)
-// LEAN: the residual values are requested in the epilogue instead of before the last block's products (64 registers less:
-// the build that runs several convolutions side by side wants three workgroups on a CU).
-template <int WM, int WN, int KF, bool FUSED, bool LEAN = false>
-__device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const float *const chunks_arg, const int tiles_arg, float *const lds) {
+template <int WM, int WN, int KF, bool FUSED>
+__device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, uint4 *const lds) {
     constexpr int TM = 32 * WM, TN = 64 * WN;
     ConvArgs a = a_arg;
     if constexpr (KF != 0) a.kernel = KF;
-    const int kb = kConvChannels * a.kernel;   // inner elements per step
-    const int a_stride = kb + 4;               // the chunks' row stride: rows stay 16-byte aligned, and a stride of 4 mod 8 words
-                                               // spreads the 32 rows a wavefront reads for a product over eight banks
     const int halo = (a.kernel - 1) * a.dilation;
-    const int win = TN + halo;                 // staged positions per input channel
-    // 16-byte pieces of the tile's weight block, and the slots (one piece per thread) that cover them; the last slot may
-    // reach past the block, into the next chunk or the zeros after the last one, and lands in LDS the products never read
-    constexpr int kSlots = (WM * 8 * (kConvChannels * (KF != 0 ? KF : kConvMaxKernel) + 4) + 255) / 256;
-    const int pieces = WM * 8 * a_stride;
-    const int slots = KF != 0 ? kSlots : (pieces + 255) / 256;
-    // (the input rows first: their LDS addresses are then the staged positions themselves, with nothing to add per request)
-    float *s_in = lds;                         // [kConvChannels][win]
-    float *s_w = lds + kConvChannels * win;    // [TM][a_stride], then the last slot's excess; 16-byte aligned
+    const int win = TN + halo;                 // staged positions
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
     const int m0 = blockIdx.y * TM, t0 = blockIdx.x * TN;
+    const int half = lane >> 5, col = lane & 31;
 
-    // Staging slots of a thread: weights -- piece tid + 256 * c of the block; input rows -- channel ch, position
-    // tid + 256 * x of the window (its place in the row is the same for every block: kept, -1 outside the row).
-    constexpr int kWinParts = (TN + kConvMaxHalo + 255) / 256;
-    floatx4 stage_w[kSlots];
-    float stage_in[kConvChannels][kWinParts];
-    int in_pos[kWinParts];
+    // Staging: a thread takes one position of the first eight channels and one of the second, half a workgroup apart (a window of
+    // 128 + halo positions then leaves every wavefront the same work); windows beyond 256 positions a third, the first
+    // half of the workgroup for the first eight channels.
+    constexpr int kColumns = TN + kConvMaxHalo > 256 ? 3 : 2;
+    static_assert(TN + kConvMaxHalo <= 384, "three columns a thread cover the window");
+    int place[kColumns];      // window position, or -1
+    int from[kColumns];       // position in the row, clamped into it
+    bool inside[kColumns];
 #pragma unroll
-    for (int x = 0; x < kWinParts; ++x) {
-        const int xx = tid + 256 * x, t = t0 - halo + xx;
-        in_pos[x] = (xx < win && t >= 0 && t < a.length) ? t : -1;
+    for (int x = 0; x < kColumns; ++x) {
+        const int p = x == 0 ? tid : x == 1 ? (tid + 128) & 255 : 256 + (tid & 127);
+        const int t = t0 - halo + p;
+        place[x] = p < win ? p : -1;
+        inside[x] = t >= 0;
+        from[x] = min(max(t, 0), a.length - 1);
     }
-    const floatx4 *w_next = reinterpret_cast<const floatx4 *>(chunks_arg) + (size_t)(WM * blockIdx.y) * (8 * a_stride) + tid;   // this thread's first piece
-    const size_t w_step = (size_t)tiles_arg * (8 * a_stride);   // pieces from a block to the next
-    const auto fetch = [&](int i0) {   // global -> registers: the weight block and input rows of channels [i0, i0 + 8); nothing waits here
+    const auto group_of = [&](int x) { return x < 2 ? x : __builtin_amdgcn_readfirstlane(tid >> 7); };
+    ConvColumn column[kColumns];
+    const auto fetch = [&](int block) {
 #pragma unroll
-        for (int c = 0; c < kSlots; ++c)
-            if (KF != 0 || c < slots) stage_w[c] = w_next[256 * c];
-        w_next += w_step;
-#pragma unroll
-        for (int ch = 0; ch < kConvChannels; ++ch) {
-            const bool row_exists = i0 + ch < a.in_ch;
-            const float *row = a.in + (row_exists ? (size_t)(i0 + ch) * a.length : 0);
-#pragma unroll
-            for (int x = 0; x < kWinParts; ++x) stage_in[ch][x] = row[in_pos[x] >= 0 ? in_pos[x] : 0];   // always a legal address
-        }
+        for (int x = 0; x < kColumns; ++x) column[x].request(a, 16 * block + 8 * group_of(x), from[x]);
     };
-    const auto publish = [&](int i0) {   // registers -> LDS (zeros where the input has no such channel or position)
+    uint4 *stage_now = lds, *stage_next = lds + 6 * win;   // [piece][eight channels][position]
+    const auto publish = [&](uint4 *stage) {
 #pragma unroll
-        for (int c = 0; c < kSlots; ++c)
-            if (KF != 0 || c < slots) reinterpret_cast<floatx4 *>(s_w)[tid + 256 * c] = stage_w[c];
-#pragma unroll
-        for (int ch = 0; ch < kConvChannels; ++ch) {
-            const bool row_exists = i0 + ch < a.in_ch;
-#pragma unroll
-            for (int x = 0; x < kWinParts; ++x) {
-                const int xx = tid + 256 * x;
-                if (xx < win) s_in[ch * win + xx] = (row_exists && in_pos[x] >= 0) ? stage_in[ch][x] : 0.0f;
-            }
-        }
+        for (int x = 0; x < kColumns; ++x)
+            if (place[x] >= 0) column[x].store(stage + group_of(x) * win + place[x], 2 * win, inside[x]);
     };
+    const int tile = min((int)blockIdx.y * WM + wm, w_arg.tiles - 1);
 
     // The accumulators start from the rows' biases (requested here, beside the first block: at the end each would be a
     // round trip of its own in front of the stores), so a value is bias + products in the products' order.
-    const int half = lane >> 5, col = lane & 31;
-    floatx16 acc0, acc1;
+    floatx16 acc[2];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-        acc0[r] = (a.bias != nullptr && m < a.out_ch) ? a.bias[m] : 0.0f;
+        acc[0][r] = (a.bias != nullptr && m < a.out_ch) ? a.bias[m] : 0.0f;
     }
-    acc1 = acc0;
-    // The fused build's residual values are requested before the last block's products instead of behind them (a round
-    // trip in front of the stores otherwise); a residual may be the output itself -- every workgroup reads and writes its
-    // own tile only.
-    float res_first[FUSED ? 32 : 1], res_second[FUSED ? 32 : 1];
-    const auto request_residuals = [&]() {
-        if constexpr (FUSED) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-                const int t = t0 + wn * 64 + col;
-                const bool in0 = m < a.out_ch && t < a.length, in1 = m < a.out_ch && t + 32 < a.length;
-                const size_t i0 = in0 ? (size_t)m * a.length + t : 0, i1 = in1 ? (size_t)m * a.length + t + 32 : 0;
-                if (a.residual != nullptr) { res_first[r] = a.residual[i0]; res_first[16 + r] = a.residual[i1]; }
-                if (a.residual2 != nullptr) { res_second[r] = a.residual2[i0]; res_second[16 + r] = a.residual2[i1]; }
-            }
-        }
-    };
+    acc[1] = acc[0];
     fetch(0);
-    for (int i0 = 0; i0 < a.in_ch; i0 += kConvChannels) {
-        publish(i0);
-        __syncthreads();
-        if (i0 + kConvChannels < a.in_ch) fetch(i0 + kConvChannels);   // in flight during the products below
-        else if constexpr (!LEAN) request_residuals();
-        conv_products<KF>(s_w + (wm * 32 + col) * a_stride + half * a.kernel, s_in + half * win + wn * 64 + col, a.kernel, a.dilation,
-                          win, acc0, acc1, min(kConvChannels / 2, (a.in_ch - i0 + 1) / 2));
-        __syncthreads();
+    ConvWeights w(w_arg.data + (size_t)tile * w_arg.blocks * a.kernel * 192 + lane, 0, a.kernel);
+    publish(stage_now);
+    fetch(min(1, w_arg.blocks - 1));
+    const auto stage = [&](int block) {
+        __syncthreads();   // this block is stored, and nobody multiplies the one whose place the next one takes
+        const uint4 *at = stage_now + half * win + wn * 64 + col;
+        if (block + 1 < w_arg.blocks) {
+            publish(stage_next);
+            fetch(min(block + 2, w_arg.blocks - 1));
+        }
+        uint4 *t = stage_now;
+        stage_now = stage_next;
+        stage_next = t;
+        return at;
+    };
+    conv_products<KF, 2>(w, a.kernel, a.dilation, 2 * win, w_arg.blocks, stage, acc);
+    __syncthreads();   // the epilogue's pieces of LDS overwrite the stages
+    floatx16 &acc0 = acc[0], &acc1 = acc[1];
+    // The fused build's residual values, requested side by side; a residual may be the output itself -- every workgroup reads and
+    // writes its own tile only.
+    float res_first[FUSED ? 32 : 1], res_second[FUSED ? 32 : 1];
+    if constexpr (FUSED) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+            const int t = t0 + wn * 64 + col;
+            const bool in0 = m < a.out_ch && t < a.length, in1 = m < a.out_ch && t + 32 < a.length;
+            const size_t i0 = in0 ? (size_t)m * a.length + t : 0, i1 = in1 ? (size_t)m * a.length + t + 32 : 0;
+            if (a.residual != nullptr) { res_first[r] = a.residual[i0]; res_first[16 + r] = a.residual[i1]; }
+            if (a.residual2 != nullptr) { res_second[r] = a.residual2[i0]; res_second[16 + r] = a.residual2[i1]; }
+        }
     }
     // accumulator element r of a lane: row 8 * (r / 4) + 4 * (lane / 32) + r % 4, column lane % 32
-    // conv + bias, then the residuals (requested before the last products, to a legal address whatever the value's place)
+    // conv + bias, then the residuals (requested to a legal address whatever the value's place)
     // and the scale, in conv_combine's order, without a branch per value: an addition that is not wanted at all is left out
     // by the build of this loop that runs.
     // A finished tile on its way to memory: from the accumulators' layout (a store instruction there covers 32 positions of
@@ -277,7 +305,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const float *co
     // wavefront's own piece of LDS (free after the last products' barrier) to whole rows of 64 consecutive positions, whose
     // validity is the same for every lane -- a loop over the rows that exist, the positions' own check once around it.
     const auto store_tile = [&](float *dst, const floatx16 &first, const floatx16 &second) {
-        float *s_tile = lds + wave * (32 * kTileStride);
+        float *s_tile = reinterpret_cast<float *>(lds) + wave * (32 * kTileStride);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row = 8 * (r >> 2) + 4 * half + (r & 3);
@@ -292,7 +320,6 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const float *co
             for (int row = 0; row < rows; ++row, p += a.length) *p = s_tile[row * kTileStride + lane];
         }
     };
-    if constexpr (LEAN) request_residuals();
     const auto combine = [&](auto has_first, auto has_second) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -317,7 +344,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const float *co
     else combine(std::false_type{}, std::false_type{});
     if (!a.activate) return;
     // The rows' alphas and 1 / (alpha + 1e-9) through the wavefront's own piece of LDS (free after the last products' barrier)
-    float *s_alpha = lds + 4 * (32 * kTileStride) + wave * 64;
+    float *s_alpha = reinterpret_cast<float *>(lds) + 4 * (32 * kTileStride) + wave * 64;
     if (lane < 32) {
         const int m = m0 + wm * 32 + lane;
         const float al = m < a.snake_channels ? a.alpha[m] : 0.0f;
@@ -354,7 +381,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const float *co
     }
     // Some argument needs the library's sine: the wavefront's 32 x 64 tile goes through LDS and a rolled loop finishes it
     // a row at a time, with one copy of that long routine.
-    float *s_tile = lds + wave * (32 * kTileStride);
+    float *s_tile = reinterpret_cast<float *>(lds) + wave * (32 * kTileStride);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int row = 8 * (r >> 2) + 4 * half + (r & 3);
@@ -370,105 +397,80 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const float *co
         conv_emit(a, m0 + wm * 32 + row, index, s_tile[row * kTileStride + lane], s_alpha[row], s_alpha[32 + row]);
 }
 
+// (the rows, the weights and the shape lead the arguments and repeat fields of a_arg: leading scalar arguments are in registers
+// when a wavefront starts, a structure passed by value is fetched from memory where its fields are first used)
 template <int WM, int WN, int KF, bool FUSED>
-__global__ void __launch_bounds__(256) k_conv1d(const float *const in_arg, float *const out_arg, const float *const chunks_arg, const float *const bias_arg, const int in_ch_arg,
-                                                const int out_ch_arg, const int length_arg, const int kernel_arg, const int dilation_arg, const int tiles_arg,
-                                                const ConvArgs a_arg) {
-    extern __shared__ __align__(16) float lds[];
-    // (the rows, the weights and the shape lead the arguments and repeat fields of a_arg: leading scalar arguments are in
-    // registers when a wavefront starts, a structure passed by value is fetched from memory where its fields are first used)
+__global__ void __launch_bounds__(256, 3) k_conv1d(const float *const in_arg, float *const out_arg, const uint4 *const weights_arg, const float *const bias_arg, const int in_ch_arg,
+                                                   const int out_ch_arg, const int length_arg, const int kernel_arg, const int dilation_arg, const int tiles_arg,
+                                                   const ConvArgs a_arg) {
+    extern __shared__ __align__(16) uint4 lds[];
     ConvArgs a = a_arg;
     a.in = in_arg; a.out = out_arg; a.bias = bias_arg; a.in_ch = in_ch_arg; a.out_ch = out_ch_arg; a.length = length_arg;
     a.kernel = kernel_arg; a.dilation = dilation_arg;
-    conv_tile<WM, WN, KF, FUSED>(a, chunks_arg, tiles_arg, lds);
+    conv_tile<WM, WN, KF, FUSED>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, lds);
 }
 
 // The same product for short rows (few positions, many channels: the codec's first stages), where 64 x 128 tiles would
 // leave most of the chip idle: a workgroup owns a 32 x 64 tile and its four wavefronts split the input channels between
-// them (wavefront w takes channel blocks w, w + 4, ...: one weight chunk each), each staging its own blocks in its own
+// them (wavefront w takes blocks w, w + 4, ... of sixteen channels), each staging its own blocks in its own
 // part of LDS; the four partial tiles are added in wavefront order at the end, so the result does not depend on timing.
 // NT: 32-position halves per tile (2, or 1 for the very shortest rows: twice the workgroups).
-template <int KF, int NT>
-__device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const float *const chunks_arg, const int tiles_arg, float *const lds) {
+// PARTS: positions of the window a lane stages (2 while the window is no longer than 128: the third costs 16 registers).
+template <int KF, int NT, int PARTS>
+__device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, uint4 *const lds) {
     constexpr int TM = 32, TN = 32 * NT;
     ConvArgs a = a_arg;
     if constexpr (KF != 0) a.kernel = KF;
-    const int kb = kConvChannels * a.kernel;
-    const int a_stride = kb + 4;   // the chunks' row stride (see k_conv1d)
     const int halo = (a.kernel - 1) * a.dilation;
     const int win = TN + halo;
-    // a chunk is 8 * a_stride 16-byte pieces; a lane's slots (one piece each) cover it, the last one possibly reaching past
-    // it (into the next chunk or the zeros after the last one: LDS the products never read)
-    constexpr int kSlots = (8 * (kConvChannels * (KF != 0 ? KF : kConvMaxKernel) + 4) + 63) / 64;
-    const int slots = KF != 0 ? kSlots : (8 * a_stride + 63) / 64;
-    const int per_wave = slots * 256 + kConvChannels * win;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float *s_in = lds + wave * per_wave;       // [kConvChannels][win] of this wavefront
-    float *s_w = s_in + kConvChannels * win;   // [TM][a_stride], then the last slot's excess; 16-byte aligned
+    uint4 *s_in = lds + wave * (6 * win);      // [piece][eight channels][position] of this wavefront
     const int m0 = blockIdx.y * TM, t0 = blockIdx.x * TN;
-    constexpr int kWinParts = (TN + kConvMaxHalo + 63) / 64;
-
-    floatx16 acc0, acc1;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) { acc0[r] = 0.0f; acc1[r] = 0.0f; }
     const int half = lane >> 5, col = lane & 31;
-    const int blocks = (a.in_ch + kConvChannels - 1) / kConvChannels;
-    const int rounds = (blocks + 3) / 4;   // the same count for every wavefront (a block past the end is a chunk of zeros)
-    floatx4 stage_w[kSlots];
-    float stage_in[kConvChannels][kWinParts];
-    int in_pos[kWinParts];    // input: position in the row, the same in every round (-1: outside the row or the window)
+
+    floatx16 acc[NT];
 #pragma unroll
-    for (int x = 0; x < kWinParts; ++x) {
-        const int xx = lane + 64 * x, t = t0 - halo + xx;
-        in_pos[x] = (xx < win && t >= 0 && t < a.length) ? t : -1;
-    }
-    // this lane's first piece of the wavefront's first chunk; four blocks on from round to round
-    const floatx4 *w_next = reinterpret_cast<const floatx4 *>(chunks_arg) + ((size_t)wave * tiles_arg + blockIdx.y) * (8 * a_stride) + lane;
-    const size_t w_step = (size_t)4 * tiles_arg * (8 * a_stride);
-    const auto fetch = [&](int round) {   // global -> registers: this wavefront's channel block of the round; nothing waits here
-        const int i0 = (4 * round + wave) * kConvChannels;
+    for (int n = 0; n < NT; ++n) acc[n] = floatx16{0};
+    const int mine = (w_arg.blocks - wave + 3) / 4;   // this wavefront's blocks
+    if (mine > 0) {
+        ConvColumn column[2][PARTS];
+        const auto fetch = [&](int i) {
 #pragma unroll
-        for (int c = 0; c < kSlots; ++c)
-            if (KF != 0 || c < slots) stage_w[c] = w_next[64 * c];
-        w_next += w_step;
+            for (int x = 0; x < PARTS; ++x)
+                if (64 * x < win) {   // (the same for every lane)
 #pragma unroll
-        for (int ch = 0; ch < kConvChannels; ++ch) {
-            const bool row_exists = i0 + ch < a.in_ch;
-            const float *row = a.in + (row_exists ? (size_t)(i0 + ch) * a.length : 0);
-#pragma unroll
-            for (int x = 0; x < kWinParts; ++x) stage_in[ch][x] = row[in_pos[x] >= 0 ? in_pos[x] : 0];   // always a legal address
-        }
-    };
-    fetch(0);
-    for (int round = 0; round < rounds; ++round) {
-        const int i0 = (4 * round + wave) * kConvChannels;
-#pragma unroll
-        for (int c = 0; c < kSlots; ++c)
-            if (KF != 0 || c < slots) reinterpret_cast<floatx4 *>(s_w)[lane + 64 * c] = stage_w[c];
-#pragma unroll
-        for (int ch = 0; ch < kConvChannels; ++ch) {
-            const bool row_exists = i0 + ch < a.in_ch;
-#pragma unroll
-            for (int x = 0; x < kWinParts; ++x) {
-                const int xx = lane + 64 * x;
-                if (xx < win) s_in[ch * win + xx] = (row_exists && in_pos[x] >= 0) ? stage_in[ch][x] : 0.0f;
-            }
-        }
+                    for (int g = 0; g < 2; ++g)
+                        column[g][x].request(a, 16 * (4 * i + wave) + 8 * g, min(max(t0 - halo + lane + 64 * x, 0), a.length - 1));
+                }
+        };
+        fetch(0);
+        const size_t per_block = (size_t)a.kernel * 192;
+        ConvWeights w(w_arg.data + ((size_t)blockIdx.y * w_arg.blocks + wave) * per_block + lane, 3 * per_block, a.kernel);
         // (no workgroup barrier in the loop: a wavefront stages into its own part of LDS and reads nothing else, and its own
         // LDS accesses complete in the order it issued them -- the four wavefronts walk their channel blocks independently)
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        if (round + 1 < rounds) fetch(round + 1);   // in flight during the products below
-        conv_products<KF, NT>(s_w + col * a_stride + half * a.kernel, s_in + half * win + col, a.kernel, a.dilation, win, acc0, acc1);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const auto stage = [&](int i) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int x = 0; x < PARTS; ++x) {
+                const int p = lane + 64 * x;
+                if (p < win) {
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) column[g][x].store(s_in + g * win + p, 2 * win, t0 - halo + p >= 0);
+                }
+            }
+            fetch(min(i + 1, mine - 1));   // in flight during this block's products
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            return const_cast<const uint4 *>(s_in + half * win + col);
+        };
+        conv_products<KF, NT>(w, a.kernel, a.dilation, 2 * win, mine, stage, acc);
     }
     __syncthreads();   // the partial tiles below overwrite every wavefront's staging area
     // partial tiles through LDS: [wavefront][element r][lane], then ((p0 + p1) + p2) + p3 + bias
-    float *s_part = lds;
+    float *s_part = reinterpret_cast<float *>(lds);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        s_part[(wave * 32 + r) * 64 + lane] = acc0[r];
-        s_part[(wave * 32 + 16 + r) * 64 + lane] = acc1[r];
-    }
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s_part[(wave * 32 + 16 * n + r) * 64 + lane] = acc[n][r];
     __syncthreads();
     // A thread finishes the tile's values at (row (tid / 64) + 4 j, position tid % 64): a store instruction then covers one
     // row's 64 consecutive positions and whether the row exists is the same for all its lanes (in the accumulators' order an
@@ -495,7 +497,7 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const flo
     }
     // with an activation: the values go back through LDS (a thread reads what it wrote) so that one copy of the
     // activation's code serves the eight of them
-    float *s_alpha = lds + 4 * 32 * 64;   // [32] alpha, [32] 1 / (alpha + 1e-9) of the tile's rows
+    float *s_alpha = reinterpret_cast<float *>(lds) + 4 * 32 * 64;   // [32] alpha, [32] 1 / (alpha + 1e-9) of the tile's rows
     if (tid < 32) {
         const float al = m0 + tid < a.snake_channels ? a.alpha[m0 + tid] : 0.0f;
         s_alpha[tid] = al;
@@ -511,16 +513,16 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const flo
     }
 }
 
-template <int KF, int NT>
-__global__ void __launch_bounds__(256) k_conv1d_split(const float *const in_arg, float *const out_arg, const float *const chunks_arg, const float *const bias_arg, const int in_ch_arg,
-                                                      const int out_ch_arg, const int length_arg, const int kernel_arg, const int dilation_arg, const int tiles_arg,
-                                                      const ConvArgs a_arg) {
-    extern __shared__ __align__(16) float lds[];
+template <int KF, int NT, int PARTS>
+__global__ void __launch_bounds__(256, 2) k_conv1d_split(const float *const in_arg, float *const out_arg, const uint4 *const weights_arg, const float *const bias_arg, const int in_ch_arg,
+                                                         const int out_ch_arg, const int length_arg, const int kernel_arg, const int dilation_arg, const int tiles_arg,
+                                                         const ConvArgs a_arg) {
+    extern __shared__ __align__(16) uint4 lds[];
     // (leading scalar arguments: see k_conv1d)
     ConvArgs a = a_arg;
     a.in = in_arg; a.out = out_arg; a.bias = bias_arg; a.in_ch = in_ch_arg; a.out_ch = out_ch_arg; a.length = length_arg;
     a.kernel = kernel_arg; a.dilation = dilation_arg;
-    conv_split_tile<KF, NT>(a, chunks_arg, tiles_arg, lds);
+    conv_split_tile<KF, NT, PARTS>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, lds);
 }
 
 // Several convolutions of one shape side by side in one launch (the three branches of a residual layer: same rows in and
@@ -532,31 +534,47 @@ __global__ void __launch_bounds__(256) k_conv1d_split(const float *const in_arg,
 constexpr int kConvBatchMax = 4;
 struct ConvBatchArgs {
     ConvArgs item[kConvBatchMax];
-    const float *chunks[kConvBatchMax];
-    int tiles;
+    ConvBlocks weights[kConvBatchMax];
+    int order[kConvBatchMax];   // blockIdx.z -> member: the ones with the most taps first, so that a long workgroup is not started last
 };
 
-// (three wavefronts per SIMD asked of the compiler: alone, a 256-thread workgroup is given every register of the CU)
 template <int WM, int WN>
 __global__ void __launch_bounds__(256, 3) k_conv1d_batch(const ConvBatchArgs b) {
-    extern __shared__ __align__(16) float lds[];
-    const int z = blockIdx.z;
+    extern __shared__ __align__(16) uint4 lds[];
+    const int z = b.order[blockIdx.z];
     switch (b.item[z].kernel) {
-        case 3: conv_tile<WM, WN, 3, true, true>(b.item[z], b.chunks[z], b.tiles, lds); break;
-        case 7: conv_tile<WM, WN, 7, true, true>(b.item[z], b.chunks[z], b.tiles, lds); break;
-        default: conv_tile<WM, WN, 11, true, true>(b.item[z], b.chunks[z], b.tiles, lds); break;
+        case 3: conv_tile<WM, WN, 3, true>(b.item[z], b.weights[z], lds); break;
+        case 7: conv_tile<WM, WN, 7, true>(b.item[z], b.weights[z], lds); break;
+        default: conv_tile<WM, WN, 11, true>(b.item[z], b.weights[z], lds); break;
     }
 }
 
-template <int NT>
+template <int NT, int PARTS>
 __global__ void __launch_bounds__(256, 2) k_conv1d_split_batch(const ConvBatchArgs b) {
-    extern __shared__ __align__(16) float lds[];
-    const int z = blockIdx.z;
+    extern __shared__ __align__(16) uint4 lds[];
+    const int z = b.order[blockIdx.z];
     switch (b.item[z].kernel) {
-        case 3: conv_split_tile<3, NT>(b.item[z], b.chunks[z], b.tiles, lds); break;
-        case 7: conv_split_tile<7, NT>(b.item[z], b.chunks[z], b.tiles, lds); break;
-        default: conv_split_tile<11, NT>(b.item[z], b.chunks[z], b.tiles, lds); break;
+        case 3: conv_split_tile<3, NT, PARTS>(b.item[z], b.weights[z], lds); break;
+        case 7: conv_split_tile<7, NT, PARTS>(b.item[z], b.weights[z], lds); break;
+        default: conv_split_tile<11, NT, PARTS>(b.item[z], b.weights[z], lds); break;
     }
+}
+
+__global__ void __launch_bounds__(256) k_conv_pack(const float *src, uint4 *dst, size_t count, int out_ch, int in_ch, int kernel, int blocks) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count) return;
+    const int lane = (int)(i & 63);
+    const size_t step = i >> 6, tile = step / ((size_t)blocks * kernel);
+    const int tap = (int)(step % (size_t)kernel), block = (int)(step / (size_t)kernel % (size_t)blocks);
+    const size_t o = tile * 32 + (lane & 31);
+    const int c0 = block * 16 + (lane >> 5) * 8;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = o < (size_t)out_ch && c0 + e < in_ch ? src[(o * in_ch + c0 + e) * kernel + tap] : 0.0f;
+    bf16x8 p[3];
+    split_eight(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]), p);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) dst[step * 192 + q * 64 + lane] = __builtin_bit_cast(uint4, p[q]);
 }
 
 struct ConvTransposeArgs {
@@ -632,87 +650,94 @@ __global__ void __launch_bounds__(256) k_rows_combine(const RowsCombineArgs a) {
     }
 }
 
+// LDS of a launch: two stages of one block of channels (the channel-split kernel: one per wavefront), or what the epilogue keeps there.
+template <int WM, int WN>
+size_t conv_lds(const ConvArgs &a) {
+    const size_t stages = (size_t)2 * 6 * (64 * WN + (a.kernel - 1) * a.dilation) * 16, epilogue = (4 * 32 * kTileStride + 4 * 64) * sizeof(float);
+    return stages > epilogue ? stages : epilogue;
+}
+template <int NT>
+size_t conv_split_lds(const ConvArgs &a) {
+    const size_t stages = (size_t)4 * 6 * (32 * NT + (a.kernel - 1) * a.dilation) * 16, epilogue = (4 * 32 * 64 + 64) * sizeof(float);
+    return stages > epilogue ? stages : epilogue;
+}
+constexpr int kConvMaxLds = 2 * 6 * (256 + kConvMaxHalo) * 16;   // the largest of them
+
 template <int WM, int WN, int KF, bool FUSED>
-int launch_conv_f(State *st, const ConvArgs &a, const ConvBlocks &chunks, char *error, size_t capacity) {
+int launch_conv_f(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
     constexpr int TM = 32 * WM, TN = 64 * WN;
-    const int slots = (WM * 8 * (kConvChannels * a.kernel + 4) + 255) / 256;
-    // two more staged rows than are filled: the product loop requests the operands of two products past its last one
-    size_t lds = ((size_t)slots * 1024 + (size_t)(kConvChannels + 2) * (TN + (a.kernel - 1) * a.dilation) + 64) * sizeof(float);
-    if (lds < (4 * 32 * kTileStride + 4 * 64) * sizeof(float)) lds = (4 * 32 * kTileStride + 4 * 64) * sizeof(float);   // the fused epilogue's tiles and alphas
     static bool raised = false;   // per instantiation
-    if (lds > 48 * 1024 && !raised) {
-        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d<WM, WN, KF, FUSED>), hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
+    if (!raised) {
+        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d<WM, WN, KF, FUSED>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
         raised = true;
     }
     const dim3 grid((unsigned)((a.length + TN - 1) / TN), (unsigned)((a.out_ch + TM - 1) / TM));
-    hipLaunchKernelGGL((k_conv1d<WM, WN, KF, FUSED>), grid, dim3(256), lds, st->stream, a.in, a.out, chunks.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel, a.dilation,
-                       chunks.tiles, a);
+    hipLaunchKernelGGL((k_conv1d<WM, WN, KF, FUSED>), grid, dim3(256), (conv_lds<WM, WN>(a)), st->stream, a.in, a.out, weights.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel,
+                       a.dilation, weights.tiles, a);
     return hip_check(hipGetLastError(), "conv1d launch", error, capacity);
 }
 
 template <int WM, int WN, int KF>
-int launch_conv_k(State *st, const ConvArgs &a, const ConvBlocks &chunks, char *error, size_t capacity) {
-    if (a.residual != nullptr || a.residual2 != nullptr || a.scaled || a.activate) return launch_conv_f<WM, WN, KF, true>(st, a, chunks, error, capacity);
-    return launch_conv_f<WM, WN, KF, false>(st, a, chunks, error, capacity);
+int launch_conv_k(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
+    if (a.residual != nullptr || a.residual2 != nullptr || a.scaled || a.activate) return launch_conv_f<WM, WN, KF, true>(st, a, weights, error, capacity);
+    return launch_conv_f<WM, WN, KF, false>(st, a, weights, error, capacity);
 }
 
 template <int WM, int WN>
-int launch_conv(State *st, const ConvArgs &a, const ConvBlocks &chunks, char *error, size_t capacity) {
+int launch_conv(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
     switch (a.kernel) {
-        case 3: return launch_conv_k<WM, WN, 3>(st, a, chunks, error, capacity);
-        case 7: return launch_conv_k<WM, WN, 7>(st, a, chunks, error, capacity);
-        case 11: return launch_conv_k<WM, WN, 11>(st, a, chunks, error, capacity);
-        default: return launch_conv_k<WM, WN, 0>(st, a, chunks, error, capacity);
+        case 3: return launch_conv_k<WM, WN, 3>(st, a, weights, error, capacity);
+        case 7: return launch_conv_k<WM, WN, 7>(st, a, weights, error, capacity);
+        case 11: return launch_conv_k<WM, WN, 11>(st, a, weights, error, capacity);
+        default: return launch_conv_k<WM, WN, 0>(st, a, weights, error, capacity);
     }
 }
 
-template <int KF, int NT>
-int launch_conv_split_k(State *st, const ConvArgs &a, const ConvBlocks &chunks, char *error, size_t capacity) {
-    const int slots = (8 * (kConvChannels * a.kernel + 4) + 63) / 64;
-    const size_t per_wave = (size_t)slots * 256 + (size_t)kConvChannels * (32 * NT + (a.kernel - 1) * a.dilation);
-    size_t lds = (4 * per_wave + 2 * (32 * NT + (a.kernel - 1) * a.dilation) + 64) * sizeof(float);   // see launch_conv_f about the two extra rows
-    if (lds < (4 * 32 * 64 + 64) * sizeof(float)) lds = (4 * 32 * 64 + 64) * sizeof(float);   // the partial tiles, and the rows' alphas behind them
+inline int conv_split_parts(const ConvArgs &a, int tn) { return tn + (a.kernel - 1) * a.dilation <= 128 ? 2 : 3; }
+
+template <int KF, int NT, int PARTS>
+int launch_conv_split_p(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
     static bool raised = false;
     if (!raised) {
-        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_split<KF, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));
+        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_split<KF, NT, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
         raised = true;
     }
     const dim3 grid((unsigned)((a.length + 32 * NT - 1) / (32 * NT)), (unsigned)((a.out_ch + 31) / 32));
-    hipLaunchKernelGGL((k_conv1d_split<KF, NT>), grid, dim3(256), lds, st->stream, a.in, a.out, chunks.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel, a.dilation,
-                       chunks.tiles, a);
+    hipLaunchKernelGGL((k_conv1d_split<KF, NT, PARTS>), grid, dim3(256), conv_split_lds<NT>(a), st->stream, a.in, a.out, weights.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel,
+                       a.dilation, weights.tiles, a);
     return hip_check(hipGetLastError(), "conv1d launch", error, capacity);
 }
 
+template <int KF, int NT>
+int launch_conv_split_k(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
+    return conv_split_parts(a, 32 * NT) == 2 ? launch_conv_split_p<KF, NT, 2>(st, a, weights, error, capacity) : launch_conv_split_p<KF, NT, 3>(st, a, weights, error, capacity);
+}
+
 template <int NT>
-int launch_conv_split_n(State *st, const ConvArgs &a, const ConvBlocks &chunks, char *error, size_t capacity) {
+int launch_conv_split_n(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
     switch (a.kernel) {
-        case 3: return launch_conv_split_k<3, NT>(st, a, chunks, error, capacity);
-        case 7: return launch_conv_split_k<7, NT>(st, a, chunks, error, capacity);
-        case 11: return launch_conv_split_k<11, NT>(st, a, chunks, error, capacity);
-        default: return launch_conv_split_k<0, NT>(st, a, chunks, error, capacity);
+        case 3: return launch_conv_split_k<3, NT>(st, a, weights, error, capacity);
+        case 7: return launch_conv_split_k<7, NT>(st, a, weights, error, capacity);
+        case 11: return launch_conv_split_k<11, NT>(st, a, weights, error, capacity);
+        default: return launch_conv_split_k<0, NT>(st, a, weights, error, capacity);
     }
 }
 
-int launch_conv_split(State *st, const ConvArgs &a, const ConvBlocks &chunks, char *error, size_t capacity) {
+int launch_conv_split(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
     const long tiles = (long)((a.out_ch + 31) / 32) * ((a.length + 63) / 64);
-    if (tiles < st->cu_count) return launch_conv_split_n<1>(st, a, chunks, error, capacity);
-    return launch_conv_split_n<2>(st, a, chunks, error, capacity);
+    if (tiles < st->cu_count) return launch_conv_split_n<1>(st, a, weights, error, capacity);
+    return launch_conv_split_n<2>(st, a, weights, error, capacity);
 }
 
-// LDS of the largest member, as the single launches size it
+// LDS of the largest member
 template <int WM, int WN>
 int launch_conv_batch(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
     constexpr int TM = 32 * WM, TN = 64 * WN;
-    size_t lds = (4 * 32 * kTileStride + 4 * 64) * sizeof(float);
-    for (int i = 0; i < count; ++i) {
-        const ConvArgs &a = b.item[i];
-        const int slots = (WM * 8 * (kConvChannels * a.kernel + 4) + 255) / 256;
-        const size_t need = ((size_t)slots * 1024 + (size_t)(kConvChannels + 2) * (TN + (a.kernel - 1) * a.dilation) + 64) * sizeof(float);
-        lds = need > lds ? need : lds;
-    }
+    size_t lds = 0;
+    for (int i = 0; i < count; ++i) lds = conv_lds<WM, WN>(b.item[i]) > lds ? conv_lds<WM, WN>(b.item[i]) : lds;
     static bool raised = false;   // per instantiation
     if (!raised) {
-        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_batch<WM, WN>), hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
+        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_batch<WM, WN>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
         raised = true;
     }
     const ConvArgs &a = b.item[0];
@@ -721,33 +746,40 @@ int launch_conv_batch(State *st, const ConvBatchArgs &b, int count, char *error,
     return hip_check(hipGetLastError(), "conv1d batch launch", error, capacity);
 }
 
-template <int NT>
-int launch_conv_split_batch(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
-    size_t lds = (4 * 32 * 64 + 64) * sizeof(float);
-    for (int i = 0; i < count; ++i) {
-        const ConvArgs &a = b.item[i];
-        const int slots = (8 * (kConvChannels * a.kernel + 4) + 63) / 64;
-        const size_t per_wave = (size_t)slots * 256 + (size_t)kConvChannels * (32 * NT + (a.kernel - 1) * a.dilation);
-        const size_t need = (4 * per_wave + 2 * (32 * NT + (a.kernel - 1) * a.dilation) + 64) * sizeof(float);
-        lds = need > lds ? need : lds;
-    }
+template <int NT, int PARTS>
+int launch_conv_split_batch_p(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
+    size_t lds = 0;
+    for (int i = 0; i < count; ++i) lds = conv_split_lds<NT>(b.item[i]) > lds ? conv_split_lds<NT>(b.item[i]) : lds;
     static bool raised = false;
     if (!raised) {
-        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_split_batch<NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));
+        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_split_batch<NT, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
         raised = true;
     }
     const ConvArgs &a = b.item[0];
     const dim3 grid((unsigned)((a.length + 32 * NT - 1) / (32 * NT)), (unsigned)((a.out_ch + 31) / 32), (unsigned)count);
-    hipLaunchKernelGGL((k_conv1d_split_batch<NT>), grid, dim3(256), lds, st->stream, b);
+    hipLaunchKernelGGL((k_conv1d_split_batch<NT, PARTS>), grid, dim3(256), lds, st->stream, b);
     return hip_check(hipGetLastError(), "conv1d batch launch", error, capacity);
+}
+
+template <int NT>
+int launch_conv_split_batch(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
+    bool two = true;
+    for (int i = 0; i < count; ++i) two = two && conv_split_parts(b.item[i], 32 * NT) == 2;
+    return two ? launch_conv_split_batch_p<NT, 2>(st, b, count, error, capacity) : launch_conv_split_batch_p<NT, 3>(st, b, count, error, capacity);
 }
 
 }  // namespace
 
+int mynah::launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_ch, size_t in_ch, size_t kernel, char *error, size_t capacity) {
+    const size_t blocks = (in_ch + 15) / 16, count = (out_ch + 31) / 32 * blocks * kernel * 64;
+    hipLaunchKernelGGL(k_conv_pack, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st->stream, src, dst, count, (int)out_ch, (int)in_ch, (int)kernel, (int)blocks);
+    return hip_check(hipGetLastError(), "weight packing launch", error, capacity);
+}
+
 // Checks one convolution's arguments, caches its weights and fills the kernels' argument block.
 static int conv1d_prepare(State *st, const float *dev_input, float *dev_output, int in_channels, int out_channels, int length,
                           int kernel, int dilation, const float *weight, const float *bias, const mynah_hip_conv1d_extra *extra,
-                          ConvArgs *out_args, ConvBlocks *out_chunks, char *error, size_t capacity) {
+                          ConvArgs *out_args, ConvBlocks *out_weights, char *error, size_t capacity) {
     if (st == nullptr || dev_input == nullptr || dev_output == nullptr || weight == nullptr || in_channels <= 0 || out_channels <= 0 ||
         length <= 0 || kernel <= 0 || dilation <= 0) {
         set_error(error, capacity, "invalid conv1d arguments");   // the checks of metal_ops_conv1d, gpu/metal/backend_metal_ops.m:371-372
@@ -758,8 +790,8 @@ static int conv1d_prepare(State *st, const float *dev_input, float *dev_output, 
         set_error(error, capacity, "conv1d: kernel above 16 taps, reach above 128 positions or tensor too large");
         return -1;
     }
-    ConvBlocks chunks;
-    if (cached_conv_blocks(st, weight, (size_t)out_channels, (size_t)in_channels, (size_t)kernel, &chunks, error, capacity) != 0) return -1;
+    ConvBlocks weights;
+    if (cached_conv_blocks(st, weight, (size_t)out_channels, (size_t)in_channels, (size_t)kernel, &weights, error, capacity) != 0) return -1;
     const float *dev_bias = nullptr;
     if (cached_vector(st, bias, (size_t)out_channels, &dev_bias, error, capacity) != 0) return -1;
     ConvArgs a{dev_input, dev_output, dev_bias, in_channels, out_channels, length, kernel, dilation};
@@ -781,7 +813,7 @@ static int conv1d_prepare(State *st, const float *dev_input, float *dev_output, 
         if (a.activate && a.snake_channels != 0 && cached_vector(st, extra->snake_alpha, extra->snake_channels, &a.alpha, error, capacity) != 0) return -1;
     }
     *out_args = a;
-    *out_chunks = chunks;
+    *out_weights = weights;
     return 0;
 }
 
@@ -789,13 +821,13 @@ static int conv1d_prepare(State *st, const float *dev_input, float *dev_output, 
 // channels to share out): small tiles with the channels split over the wavefronts
 static bool conv_takes_split(const State *st, int in_channels, int out_channels, int length) {
     const long tiles = out_channels <= 32 ? (long)((length + 255) / 256) : (long)((out_channels + 63) / 64) * ((length + 127) / 128);
-    return tiles < st->cu_count && in_channels >= 4 * kConvChannels;
+    return tiles < st->cu_count && in_channels >= 32;
 }
 
-static int conv1d_launch(State *st, const ConvArgs &a, const ConvBlocks &chunks, char *error, size_t capacity) {
-    if (conv_takes_split(st, a.in_ch, a.out_ch, a.length)) return launch_conv_split(st, a, chunks, error, capacity);
-    if (a.out_ch <= 32) return launch_conv<1, 4>(st, a, chunks, error, capacity);
-    return launch_conv<2, 2>(st, a, chunks, error, capacity);
+static int conv1d_launch(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
+    if (conv_takes_split(st, a.in_ch, a.out_ch, a.length)) return launch_conv_split(st, a, weights, error, capacity);
+    if (a.out_ch <= 32) return launch_conv<1, 4>(st, a, weights, error, capacity);
+    return launch_conv<2, 2>(st, a, weights, error, capacity);
 }
 
 static int conv1d_entry(void *state, const float *dev_input, float *dev_output, int in_channels, int out_channels, int length,
@@ -803,10 +835,10 @@ static int conv1d_entry(void *state, const float *dev_input, float *dev_output, 
                         char *error, size_t capacity) {
     State *st = enter_state(state);
     ConvArgs a;
-    ConvBlocks chunks;
-    if (conv1d_prepare(st, dev_input, dev_output, in_channels, out_channels, length, kernel, dilation, weight, bias, extra, &a, &chunks, error, capacity) != 0)
+    ConvBlocks weights;
+    if (conv1d_prepare(st, dev_input, dev_output, in_channels, out_channels, length, kernel, dilation, weight, bias, extra, &a, &weights, error, capacity) != 0)
         return -1;
-    return conv1d_launch(st, a, chunks, error, capacity);
+    return conv1d_launch(st, a, weights, error, capacity);
 }
 
 extern "C" int mynah_hip_conv1d(void *state, const float *dev_input, float *dev_output, int in_channels, int out_channels, int length,
@@ -832,15 +864,16 @@ extern "C" int mynah_hip_conv1d_fused_batch(void *state, const mynah_hip_conv1d_
         return -1;
     }
     ConvBatchArgs b{};
-    ConvBlocks chunks[kConvBatchMax];
     bool side_by_side = true;
     for (size_t i = 0; i < count; ++i) {
         const mynah_hip_conv1d_item &it = items[i];
         if (conv1d_prepare(st, it.dev_input, it.dev_output, in_channels, out_channels, length, it.kernel, it.dilation, it.weight, it.bias, &it.extra,
-                           &b.item[i], &chunks[i], error, capacity) != 0)
+                           &b.item[i], &b.weights[i], error, capacity) != 0)
             return -1;
-        b.chunks[i] = chunks[i].data;
-        side_by_side = side_by_side && (it.kernel == 3 || it.kernel == 7 || it.kernel == 11) && chunks[i].tiles == chunks[0].tiles;
+        side_by_side = side_by_side && (it.kernel == 3 || it.kernel == 7 || it.kernel == 11);
+        size_t at = i;   // most taps first
+        for (; at > 0 && items[b.order[at - 1]].kernel < it.kernel; --at) b.order[at] = b.order[at - 1];
+        b.order[at] = (int)i;
         // the members run at the same time: what one writes, no other may read or write
         for (size_t j = 0; j < count; ++j) {
             if (j == i) continue;
@@ -855,10 +888,9 @@ extern "C" int mynah_hip_conv1d_fused_batch(void *state, const mynah_hip_conv1d_
             }
         }
     }
-    b.tiles = chunks[0].tiles;
     if (!side_by_side || count == 1) {   // other tap counts: one after the other (the same values)
         for (size_t i = 0; i < count; ++i)
-            if (conv1d_launch(st, b.item[i], chunks[i], error, capacity) != 0) return -1;
+            if (conv1d_launch(st, b.item[i], b.weights[i], error, capacity) != 0) return -1;
         return 0;
     }
     if (conv_takes_split(st, in_channels, out_channels, length)) {

@@ -225,18 +225,13 @@ State *enter_state(void *opaque, bool enqueues = true);
 int cached_matrix(State *st, const float *host, size_t n, size_t k, int want_qtype, const CachedWeight **out,
                   char *error, size_t capacity);
 int cached_vector(State *st, const float *host, size_t n, const float **dev, char *error, size_t capacity);
-// A conv1d weight [out_ch, in_ch, kernel] in the form the convolution kernels stage it (codec_ops.hip): cut into chunks of
-// 32 output channels x 8 input channels, each chunk 32 rows of 8 * kernel + 4 floats (a row holds the taps of its eight
-// channels one after the other, then four floats of padding: the row stride the kernels keep in LDS), zeros where the
-// tensor has no row or channel.  Chunk (block b of input channels, tile t of output channels) starts at float
-// (b * tiles + t) * conv_chunk_floats(kernel); `tiles` is even and `blocks` a multiple of four (whole chunks of zeros
-// past the tensor), and four kilobytes of zeros follow the last chunk, so a kernel copies whole chunks without a bounds check.
+// A conv1d weight [out_ch, in_ch, kernel] in the form the convolution kernels multiply it (codec_ops.hip): three bf16 pieces per value
+// (split_product.h), per tile of 32 output channels, block of 16 input channels and tap three runs of 64 uint4s, one per piece, lane
+// l's being output channel l % 32, input channels 8 * (l / 32) .. + 7 of the block; zeros where the tensor has no row or channel.
 struct ConvBlocks {
-    const float *data = nullptr;
+    const uint4 *data = nullptr;
     int tiles = 0, blocks = 0;
 };
-constexpr int kConvChannels = 8;      // input channels per chunk: the convolution kernels' step along the inner dimension
-inline size_t conv_chunk_floats(size_t kernel) { return 32u * (kConvChannels * kernel + 4u); }
 int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch, size_t kernel, ConvBlocks *out, char *error, size_t capacity);
 // An f32 weight [n, channels, taps] in the order in which split_product.hip's kernels take it; n a multiple of 32, channels of 64.
 int cached_split_weight(State *st, const float *host, size_t n, size_t channels, size_t taps, const float4 **out, char *error, size_t capacity);

@@ -58,6 +58,7 @@ struct SplitLayers {
     const float4 *w[kSplitMaxLayers];
     const float *gain[kSplitMaxLayers], *bias[kSplitMaxLayers];   // bias entries may be null
 };
+int launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_ch, size_t in_ch, size_t kernel, char *error, size_t capacity);
 int launch_split_pack(State *st, const float *src, float4 *dst, size_t n, size_t channels, size_t taps, char *error, size_t capacity);
 int split_product_splits(const State *st, size_t rows, size_t channels, size_t n, size_t most);
 // part[z][rows][n] = split z's share of in[rows][channels] * W (taps == 3: causal convolution, two rows in front of `in` are zeros).
