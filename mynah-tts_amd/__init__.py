@@ -141,6 +141,7 @@ def load_library(path=LIB_PATH):
     lib.mynah_hip_decoder_destroy.restype = None
     lib.mynah_hip_decoder_step.argtypes = [_vp, _vp, C.POINTER(DecoderSlot), _sz, *_err]
     lib.mynah_hip_output_head.argtypes = [_vp, _vp, _sz, _sz, _vp, _vp, _sz, _sz, _vp, _vp, *_err]
+    lib.mynah_hip_decoder_step_head.argtypes = [_vp, _vp, C.POINTER(DecoderSlot), _sz, _vp, _vp, _sz, _sz, _vp, _vp, *_err]
     lib.mynah_hip_decoder_stage_enqueue.argtypes = [_vp, _vp, _sz, C.c_int, *_err]
     lib.mynah_hip_decoder_step_probe.argtypes = [_vp, _vp, C.POINTER(DecoderSlot), _sz, _vp, _vp, *_err]
     lib.mynah_hip_local_create.argtypes = [_vp, C.POINTER(DecoderDesc), C.POINTER(LocalDesc), C.POINTER(_vp), *_err]
@@ -178,7 +179,7 @@ class BackendError(RuntimeError):
 
 
 def _np_ptr(a):
-    return None if a is None else a.ctypes.data_as(_vp)
+    return None if a is None else a.__array_interface__["data"][0]
 
 
 class DeviceBuffer:
@@ -226,12 +227,14 @@ class Backend:
         if rc != 0:
             raise BackendError("mynah_backend_hip_open failed: " + err.value.decode())
         self._keep = []   # host arrays whose addresses key the device weight cache
+        self._kept = {}   # id -> (array, address) of those that were handed in as they are kept
+        self._error = C.create_string_buffer(512)   # one thread at a time uses a backend
         if quant is not None or arith is not None:
             self.set_quant(F32 if quant is None else quant, ARITH_STRICT if arith is None else arith)
 
     # -- plumbing
     def _call(self, name, *args):
-        err = C.create_string_buffer(512)
+        err = self._error
         rc = getattr(self.lib, name)(self.state, *args, err, 512)
         if rc != 0:
             raise BackendError("%s: %s" % (name, err.value.decode()))
@@ -239,9 +242,23 @@ class Backend:
 
     def keep(self, array):
         """Pin a host tensor for the life of the backend (the cache keys on its address)."""
+        known = self._kept.get(id(array))
+        if known is not None and known[0] is array:
+            return array
         a = np.ascontiguousarray(array, np.float32)
         self._keep.append(a)
+        if a is array:
+            self._kept[id(a)] = (a, _np_ptr(a))
         return a
+
+    def address(self, array):
+        """Address of a host tensor pinned by `keep` (None for None): what the C ABI takes as a weight."""
+        if array is None:
+            return None
+        known = self._kept.get(id(array))
+        if known is not None and known[0] is array:
+            return known[1]
+        return _np_ptr(self.keep(array))
 
     def close(self):
         if self.state:
@@ -355,28 +372,26 @@ class Backend:
         self._call("mynah_hip_clip_dev", _vp(d), _sz(n))
 
     def conv1d(self, din, dout, in_ch, out_ch, length, kernel, dilation, weight, bias=None):
-        self._call("mynah_hip_conv1d", din, dout, in_ch, out_ch, length, kernel, dilation, _np_ptr(self.keep(weight)),
-                   None if bias is None else _np_ptr(self.keep(bias)))
+        self._call("mynah_hip_conv1d", din, dout, in_ch, out_ch, length, kernel, dilation, self.address(weight), self.address(bias))
 
     def conv_transpose_dev(self, din, dout, in_ch, out_ch, length, output_length, kernel, stride, groups, weight, bias=None):
-        self._call("mynah_hip_conv_transpose_dev", din, dout, in_ch, out_ch, length, output_length, kernel, stride, groups,
-                   _np_ptr(self.keep(weight)), None if bias is None else _np_ptr(self.keep(bias)))
+        self._call("mynah_hip_conv_transpose_dev", din, dout, in_ch, out_ch, length, output_length, kernel, stride, groups, self.address(weight), self.address(bias))
 
     def snake_dev(self, d, alpha, channels, length, snake_channels):
-        self._call("mynah_hip_snake_dev", d, _np_ptr(self.keep(alpha)), _sz(channels), _sz(length), _sz(snake_channels))
+        self._call("mynah_hip_snake_dev", d, self.address(alpha), _sz(channels), _sz(length), _sz(snake_channels))
 
     def snake_copy_dev(self, din, dout, alpha, channels, length, snake_channels):
-        self._call("mynah_hip_snake_copy_dev", din, dout, _np_ptr(self.keep(alpha)), _sz(channels), _sz(length), _sz(snake_channels))
+        self._call("mynah_hip_snake_copy_dev", din, dout, self.address(alpha), _sz(channels), _sz(length), _sz(snake_channels))
 
     def conv1d_fused(self, din, dout, in_ch, out_ch, length, kernel, dilation, weight, bias=None, residual=None, residual2=None,
                      scale=1.0, alpha=None, snake_channels=None, activated=None):
         """conv1d, then per value: + residual, + residual2, * scale, and (alpha given) the half-snake, written to dout or,
         with `activated`, beside the plain value."""
         extra = Conv1dExtra(residual, residual2, scale, 0 if alpha is None else 1,
-                            None if alpha is None else _np_ptr(self.keep(alpha)),
+                            self.address(alpha),
                             0 if alpha is None else (out_ch // 2 if snake_channels is None else snake_channels), activated)
-        self._call("mynah_hip_conv1d_fused", din, dout, in_ch, out_ch, length, kernel, dilation, _np_ptr(self.keep(weight)),
-                   None if bias is None else _np_ptr(self.keep(bias)), C.byref(extra))
+        self._call("mynah_hip_conv1d_fused", din, dout, in_ch, out_ch, length, kernel, dilation, self.address(weight), self.address(bias),
+                   C.byref(extra))
 
     def conv1d_fused_batch(self, items, in_ch, out_ch, length):
         """Up to four conv1d_fused calls of one shape in one launch.  items: dicts with din, dout, kernel, dilation, weight and,
@@ -386,16 +401,15 @@ class Backend:
             alpha = it.get("alpha")
             snake = 0 if alpha is None else (out_ch // 2 if it.get("snake_channels") is None else it["snake_channels"])
             slot.dev_input, slot.dev_output, slot.kernel, slot.dilation = it["din"], it["dout"], it["kernel"], it["dilation"]
-            slot.weight = _np_ptr(self.keep(it["weight"]))
-            slot.bias = None if it.get("bias") is None else _np_ptr(self.keep(it["bias"]))
+            slot.weight, slot.bias = self.address(it["weight"]), self.address(it.get("bias"))
             slot.extra = Conv1dExtra(it.get("residual"), it.get("residual2"), it.get("scale", 1.0), 0 if alpha is None else 1,
-                                     None if alpha is None else _np_ptr(self.keep(alpha)), snake, it.get("activated"))
+                                     self.address(alpha), snake, it.get("activated"))
         self._call("mynah_hip_conv1d_fused_batch", arr, _sz(len(items)), in_ch, out_ch, length)
 
     def rows_combine_dev(self, dins, scale, douts, alphas, channels, length, snake_channels=None):
         """((in0 + in1) + ...) * scale into every output, through the half-snake of alphas[j] where that is not None."""
         arr_in, arr_out = (_vp * len(dins))(*dins), (_vp * len(douts))(*douts)
-        arr_al = (_vp * len(douts))(*[None if a is None else _np_ptr(self.keep(a)) for a in alphas])
+        arr_al = (_vp * len(douts))(*[self.address(a) for a in alphas])
         self._call("mynah_hip_rows_combine_dev", arr_in, _sz(len(dins)), C.c_float(scale), arr_out, arr_al, _sz(len(douts)), _sz(channels),
                    _sz(length), _sz(channels // 2 if snake_channels is None else snake_channels))
 
