@@ -232,6 +232,22 @@ int mynah_hip_rows_combine_dev(void *state, const float *const *dev_inputs, size
                                const float *const *alphas, size_t outputs, size_t channels, size_t length, size_t snake_channels,
                                char *error, size_t error_capacity);
 
+/* A whole residual layer (res_layer_device, src/graph.c:2423-2498) as one call: `branches` (one to four) chains of `positions` blocks
+ *   x = x + conv(half_snake(conv(half_snake(x; alpha_in); weight_in, bias_in, dilation); alpha_skip); weight_skip, bias_skip, 1)
+ * all from dev_input, then ((b0 + b1) + ...) * (1 / branches), through the half-snake of then_alpha when that is not null, to
+ * dev_output.  blocks[branch * positions + position]; every half-snake has channels / 2 snake rows; weights, biases (may be null)
+ * and alphas are host pointers, cached like every weight.  dev_work: 3 * branches row sets [channels, length] of the caller's,
+ * overwritten.  The values are those of the operator sequence above, bit for bit; up to 128 channels with 3, 7 or 11 taps a
+ * position of all branches is one launch.  No counterpart in the reference's seam. */
+typedef struct mynah_hip_res_block {
+    const float *alpha_in, *weight_in, *bias_in;
+    const float *alpha_skip, *weight_skip, *bias_skip;
+    int kernel_in, kernel_skip, dilation;
+} mynah_hip_res_block;
+int mynah_hip_res_layer_dev(void *state, const mynah_hip_res_block *blocks, size_t branches, size_t positions, const float *dev_input,
+                            float *dev_output, size_t channels, size_t length, const float *then_alpha, float *const *dev_work,
+                            char *error, size_t error_capacity);
+
 /* ------------------------------------------------------------------------------------------
  * Section 2 -- what the single-stream seam lacks
  * ------------------------------------------------------------------------------------------ */

@@ -9,6 +9,7 @@ There is no CPU fallback: if the library is missing or no MI355X is present, loa
 fails loudly.
 """
 import ctypes as C
+import operator
 import os
 
 import numpy as np
@@ -55,6 +56,11 @@ class Conv1dExtra(C.Structure):
 class Conv1dItem(C.Structure):
     _fields_ = [("dev_input", _vp), ("dev_output", _vp), ("kernel", C.c_int), ("dilation", C.c_int), ("weight", _vp), ("bias", _vp),
                 ("extra", Conv1dExtra)]
+
+
+class ResBlock(C.Structure):
+    _fields_ = [("alpha_in", _vp), ("weight_in", _vp), ("bias_in", _vp), ("alpha_skip", _vp), ("weight_skip", _vp), ("bias_skip", _vp),
+                ("kernel_in", C.c_int), ("kernel_skip", C.c_int), ("dilation", C.c_int)]
 
 
 class EncoderDesc(C.Structure):
@@ -119,6 +125,7 @@ def load_library(path=LIB_PATH):
     lib.mynah_hip_snake_copy_dev.argtypes = [_vp, _vp, _vp, _vp, _sz, _sz, _sz, *_err]
     lib.mynah_hip_rows_combine_dev.argtypes = [_vp, C.POINTER(_vp), _sz, C.c_float, C.POINTER(_vp), C.POINTER(_vp), _sz, _sz, _sz, _sz, *_err]
     lib.mynah_hip_conv1d_fused_batch.argtypes = [_vp, C.POINTER(Conv1dItem), _sz, C.c_int, C.c_int, C.c_int, *_err]
+    lib.mynah_hip_res_layer_dev.argtypes = [_vp, C.POINTER(ResBlock), _sz, _sz, _vp, _vp, _sz, _sz, _vp, _vp, *_err]
     lib.mynah_hip_conv1d_fused.argtypes = [_vp, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _vp, _vp,
                                            C.POINTER(Conv1dExtra), *_err]
     lib.mynah_hip_set_quant.argtypes = [_vp, C.c_int, C.c_int, *_err]
@@ -228,6 +235,7 @@ class Backend:
             raise BackendError("mynah_backend_hip_open failed: " + err.value.decode())
         self._keep = []   # host arrays whose addresses key the device weight cache
         self._kept = {}   # id -> (array, address) of those that were handed in as they are kept
+        self._res_layers = {}   # id of a residual layer's blocks -> (blocks, what they hold, descriptor)
         self._error = C.create_string_buffer(512)   # one thread at a time uses a backend
         if quant is not None or arith is not None:
             self.set_quant(F32 if quant is None else quant, ARITH_STRICT if arith is None else arith)
@@ -412,6 +420,24 @@ class Backend:
         arr_al = (_vp * len(douts))(*[self.address(a) for a in alphas])
         self._call("mynah_hip_rows_combine_dev", arr_in, _sz(len(dins)), C.c_float(scale), arr_out, arr_al, _sz(len(douts)), _sz(channels),
                    _sz(length), _sz(channels // 2 if snake_channels is None else snake_channels))
+
+    def res_layer_dev(self, blocks, din, dout, channels, length, work, then_alpha=None):
+        """A residual layer as one call.  blocks[branch][position] = (alpha_in, (w_in, b_in), alpha_skip, (w_skip, b_skip),
+        dilation); work: three row sets per branch."""
+        desc = self._res_layers.get(id(blocks))
+        parts = [a for branch in blocks for b in branch for a in (b[0], b[1][0], b[1][1], b[2], b[3][0], b[3][1], b[4])]
+        if desc is None or len(desc[1]) != len(parts) or not all(map(operator.is_, desc[1], parts)):
+            arr = (ResBlock * (len(blocks) * len(blocks[0])))()
+            slots = iter(arr)
+            for branch in blocks:
+                for a_in, (w_in, b_in), a_skip, (w_skip, b_skip), dilation in branch:
+                    s = next(slots)
+                    s.alpha_in, s.weight_in, s.bias_in = self.address(a_in), self.address(w_in), self.address(b_in)
+                    s.alpha_skip, s.weight_skip, s.bias_skip = self.address(a_skip), self.address(w_skip), self.address(b_skip)
+                    s.kernel_in, s.kernel_skip, s.dilation = w_in.shape[2], w_skip.shape[2], dilation
+            desc = self._res_layers[id(blocks)] = (blocks, parts, arr)   # (held: an id stays one object's)
+        self._call("mynah_hip_res_layer_dev", desc[2], len(blocks), len(blocks[0]), din, dout, channels, length, self.address(then_alpha),
+                   (_vp * len(work))(*work))
 
     def argmax_dev(self, dlogits, vocab, codebook_size, eos_id, allow_eos):
         out = C.c_uint(0)

@@ -332,6 +332,32 @@ int cached_vector(State *st, const float *host, size_t n, const float **dev, cha
     return 0;
 }
 
+int cached_snake_pairs(State *st, const float *host, size_t n, const float **dev, char *error, size_t capacity) {
+    if (host == nullptr || n == 0 || n > SIZE_MAX / (4 * sizeof(float))) {
+        set_error(error, capacity, "invalid snake alphas");
+        return -1;
+    }
+    const WeightKey key{host, n * sizeof(float), -100};
+    std::lock_guard<std::mutex> lock(st->mu);
+    auto it = st->weights.find(key);
+    if (it == st->weights.end()) {
+        std::vector<float> pairs(2 * n);
+        for (size_t i = 0; i < n; ++i) {
+            pairs[2 * i] = host[i];
+            pairs[2 * i + 1] = 1.0f / (host[i] + 1e-9f);
+        }
+        CachedWeight cw;
+        cw.n = 2;
+        cw.k = n;
+        cw.bytes = pairs.size() * sizeof(float);
+        if (device_copy_of(pairs.data(), cw.bytes, &cw.data, error, capacity) != 0) return -1;
+        st->weight_bytes += cw.bytes;
+        it = st->weights.emplace(key, cw).first;
+    }
+    *dev = static_cast<const float *>(it->second.data);
+    return 0;
+}
+
 // out[b] = W in[b] (+bias) for `batch` device rows: fused matvec tiles, or the generic f32 GEMM.
 // ln_gain (device vector) non-null: the rows are normalised first (LayerNorm prologue of the product; one weight pass only), and
 // with ln_out_slots every stream's normalised row is also stored at that device table's output[stream].

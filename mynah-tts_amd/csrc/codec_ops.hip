@@ -135,33 +135,35 @@ struct ConvWeights {   // the weight pieces of one row tile, requested kAhead st
 // position], lanes 32.. eight channels on.  With the tap count known (KF) the loop over a block's steps is unrolled, and three blocks at
 // a time, after which the weights' registers repeat.  (A step's fragments are read right before it: two or three wavefronts share a
 // SIMD, and a second set of fragment registers, read a step ahead, spilled: 1884 against 1754 us for a 64-frame decode.)
-template <int KF, int NT, class Stage>
+template <int KF, int NT, bool AHEAD = false, class Stage>
 __device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, const int dilation, const int piece_stride, const int blocks, const Stage stage,
                                               floatx16 (&acc)[NT]) {
-    bf16x8 x[NT][3];
-    const auto read = [&](const uint4 *at) {
+    bf16x8 x[AHEAD ? 2 : 1][NT][3];
+    const auto read = [&](int set, const uint4 *at) {
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int q = 0; q < 3; ++q) x[n][q] = __builtin_bit_cast(bf16x8, at[q * piece_stride + 32 * n]);
+            for (int q = 0; q < 3; ++q) x[set][n][q] = __builtin_bit_cast(bf16x8, at[q * piece_stride + 32 * n]);
     };
-    const auto multiply = [&](int slot) {
+    const auto multiply = [&](int set, int slot) {
         bf16x8 fw[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) fw[q] = __builtin_bit_cast(bf16x8, w.ring[slot][q]);
 #pragma unroll
-        for (int n = 0; n < NT; ++n) acc[n] = split_multiply(fw, x[n], acc[n]);
+        for (int n = 0; n < NT; ++n) acc[n] = split_multiply(fw, x[set][n], acc[n]);
     };
     if constexpr (KF != 0) {
         for (int block = 0;;) {
 #pragma unroll
             for (int u = 0; u < ConvWeights::kAhead; ++u) {
                 const uint4 *at = stage(block);
+                if constexpr (AHEAD) read((u * KF) & 1, at);
 #pragma unroll
                 for (int tap = 0; tap < KF; ++tap) {
                     const int s = u * KF + tap;
-                    read(at + tap * dilation);
-                    multiply(s % ConvWeights::kAhead);
+                    if constexpr (!AHEAD) read(0, at + tap * dilation);
+                    else if (tap + 1 < KF) read((s + 1) & 1, at + (tap + 1) * dilation);
+                    multiply(AHEAD ? s & 1 : 0, s % ConvWeights::kAhead);
                     w.request(s % ConvWeights::kAhead, KF);
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -172,8 +174,8 @@ __device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, co
         for (int block = 0; block < blocks; ++block) {
             const uint4 *at = stage(block);
             for (int tap = 0; tap < taps; ++tap) {
-                read(at + tap * dilation);
-                multiply(0);
+                read(0, at + tap * dilation);
+                multiply(0, 0);
 #pragma unroll
                 for (int i = 0; i + 1 < ConvWeights::kAhead; ++i)
 #pragma unroll
@@ -219,7 +221,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
     if constexpr (KF != 0) a.kernel = KF;
     const int halo = (a.kernel - 1) * a.dilation;
     const int win = TN + halo;                 // staged positions
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN;
     const int m0 = blockIdx.y * TM, t0 = blockIdx.x * TN;
     const int half = lane >> 5, col = lane & 31;
@@ -366,10 +368,14 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
             const int row = 8 * (r >> 2) + 4 * half + (r & 3), m = m0 + wm * 32 + row;
             const float al = s_alpha[row], inv_a = s_alpha[32 + row];
             const float v0 = acc0[r], v1 = acc1[r];
-            const float s0 = short_sine(al * v0), s1 = short_sine(al * v1);
-            const bool snake_row = m < a.snake_channels;
-            act0[r] = snake_row ? v0 + s0 * s0 * inv_a : (v0 < 0.0f ? v0 * 0.01f : v0);
-            act1[r] = snake_row ? v1 + s1 * s1 * inv_a : (v1 < 0.0f ? v1 * 0.01f : v1);
+            act0[r] = v0 < 0.0f ? v0 * 0.01f : v0;
+            act1[r] = v1 < 0.0f ? v1 * 0.01f : v1;
+            if (m0 + wm * 32 + 8 * (r >> 2) < a.snake_channels) {   // (else no lane's row of these registers is a snake row: half of all)
+                const float s0 = short_sine(al * v0), s1 = short_sine(al * v1);
+                const bool snake_row = m < a.snake_channels;
+                act0[r] = snake_row ? v0 + s0 * s0 * inv_a : act0[r];
+                act1[r] = snake_row ? v1 + s1 * s1 * inv_a : act1[r];
+            }
         }
         if (a.act_out != nullptr) {
             store_tile(a.out, acc0, acc1);
@@ -423,7 +429,7 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
     if constexpr (KF != 0) a.kernel = KF;
     const int halo = (a.kernel - 1) * a.dilation;
     const int win = TN + halo;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint4 *s_in = lds + wave * (6 * win);      // [piece][eight channels][position] of this wavefront
     const int m0 = blockIdx.y * TM, t0 = blockIdx.x * TN;
     const int half = lane >> 5, col = lane & 31;
@@ -558,6 +564,257 @@ __global__ void __launch_bounds__(256, 2) k_conv1d_split_batch(const ConvBatchAr
         case 7: conv_split_tile<7, NT, PARTS>(b.item[z], b.weights[z], lds); break;
         default: conv_split_tile<11, NT, PARTS>(b.item[z], b.weights[z], lds); break;
     }
+}
+
+// ---- a residual block in one launch ---------------------------------------------------------------------------------------
+// out = x + conv_skip(snake(conv_in(snake(x)))) for up to four branches of a residual layer side by side, up to 128 channels: what
+// would be two launches and, between them and around them, three row sets written and read again.  A workgroup takes all rows of a
+// window of 64 * WN positions of the inner rows r = snake(conv_in(snake(x))), (taps - 1) more than the positions it finishes:
+// it stages snake(x) (a position and its halo are activated once, since every row is here), multiplies, activates, leaves the
+// pieces of r in LDS over the stages, and multiplies again from there.  Every value is the separate calls' arithmetic in their
+// order: the same bits.
+// (27 channels x 65536, taps 3 / 7 / 11: 63 us against 2 x 39 us as two launches; 54 x 2560: 27 us against 2 x 22.)
+struct ResMember {
+    const float *in;                      // [channels, length]
+    float *out;
+    const float2 *snake_in, *snake_skip;  // (alpha, 1 / (alpha + 1e-9)) of the first snake_channels rows
+    const uint4 *w_in, *w_skip;           // ConvBlocks data
+    const float *b_in, *b_skip;           // or null
+    int kernel, dilation;
+};
+constexpr int kResMaxChannels = 128, kResMaxReach = 64;
+struct ResArgs {
+    ResMember member[kConvBatchMax];
+    int order[kConvBatchMax];
+    int channels, length, snake_channels, blocks, tiles;
+};
+
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+
+template <int WM, int WN, int NT, int KF>
+__device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember &m, uint4 *const lds, float2 *const s_pairs) {
+    constexpr int WP = 32 * NT, RN = WP * WN, T = 64 * WM * WN, TN = RN - (KF - 1);
+    const int t0 = blockIdx.x * TN;
+    if (t0 >= a.length) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, col = lane & 31;
+    const int wm = wave / WN, wn = wave % WN;
+    const int halo = (KF - 1) * m.dilation, win = RN + halo;
+    const int first = t0 - (KF - 1) - halo;   // position of the window's first column
+
+    // staging: columns (a position, eight channels) of a thread; a wavefront's columns are of one half of a block's channels.  Up to
+    // T / 2 positions: a thread takes one column, the workgroup's halves the two halves of the channels; else one of each half, the
+    // second half a workgroup apart, and (windows of more than T positions) the first 128 threads a third.
+    constexpr int kReach = RN + kResMaxReach, kColumns = kReach <= T / 2 ? 1 : kReach <= T ? 2 : 3;
+    static_assert(kReach <= T + 64 && (kColumns == 1 || T == 256), "columns cover the window");
+    int place[kColumns];
+    const auto group_of = [&](int x) { return kColumns == 1 ? wave / (T / 128) : x < 2 ? x : wave & 1; };
+#pragma unroll
+    for (int x = 0; x < kColumns; ++x) {
+        const int p = kColumns == 1 ? tid & (T / 2 - 1) : x == 0 ? tid : x == 1 ? (kColumns == 2 ? (tid + 128) & 255 : tid) : tid < 128 ? 256 + (tid & 63) : win;
+        place[x] = p < win ? p : -1;
+    }
+    f32x8 column[kColumns];
+    const auto fetch = [&](int block) {
+#pragma unroll
+        for (int x = 0; x < kColumns; ++x) {
+            const int channel = 16 * block + 8 * group_of(x);
+            const float *const at = m.in + min(max(first + place[x], 0), a.length - 1);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) column[x][e] = at[(size_t)min(channel + e, a.channels - 1) * a.length];
+        }
+    };
+    const auto publish = [&](int block, uint4 *stage) {
+#pragma unroll
+        for (int x = 0; x < kColumns; ++x) {
+            if (place[x] < 0) continue;
+            const int channel = 16 * block + 8 * group_of(x);
+            f32x8 v = column[x];
+            bool large = false;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (channel + e < a.snake_channels) large = large || !(fabsf(m.snake_in[channel + e].x * v[e]) < kShortSineLimit);
+            if (!__any(large)) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    if (channel + e < a.snake_channels) {   // (the same for every lane)
+                        const float2 pair = m.snake_in[channel + e];
+                        const float sn = short_sine(pair.x * v[e]);
+                        v[e] = v[e] + sn * sn * pair.y;
+                    } else {
+                        v[e] = v[e] < 0.0f ? v[e] * 0.01f : v[e];
+                    }
+                }
+            } else {
+#pragma unroll 1
+                for (int e = 0; e < 8; ++e) {
+                    const bool snake_row = channel + e < a.snake_channels;
+                    const float2 pair = snake_row ? m.snake_in[channel + e] : make_float2(0.0f, 0.0f);
+                    v[e] = half_snake(v[e], snake_row, pair.x, pair.y);
+                }
+            }
+            if (first + place[x] < 0) v = f32x8{0};   // in front of the rows
+            bf16x8 p[3];
+            split_eight(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]), p);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) stage[(q * 2 + group_of(x)) * win + place[x]] = __builtin_bit_cast(uint4, p[q]);
+        }
+    };
+    if (tid < kResMaxChannels) s_pairs[tid] = tid < a.snake_channels ? m.snake_skip[tid] : make_float2(0.0f, 0.0f);
+
+    // the rows' biases, which the sums start from: both convolutions' requested here, none under a condition
+    float bias_in[16], bias_skip[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = min(wm * 32 + split_acc_row(r, lane), a.channels - 1);
+        bias_in[r] = m.b_in != nullptr ? m.b_in[row] : 0.0f;
+        bias_skip[r] = m.b_skip != nullptr ? m.b_skip[row] : 0.0f;
+    }
+    const auto start = [&](const float (&bias)[16], f32x16 (&acc)[NT]) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][r] = wm * 32 + split_acc_row(r, lane) < a.channels ? bias[r] : 0.0f;
+#pragma unroll
+        for (int n = 1; n < NT; ++n) acc[n] = acc[0];
+    };
+    const size_t w_at = (size_t)min(wm, a.tiles - 1) * a.blocks * KF * 192 + lane;
+    fetch(0);
+    ConvWeights w(m.w_in + w_at, 0, KF);
+    uint4 *stage_now = lds, *stage_next = lds + 6 * win;
+    f32x16 acc[NT];
+    start(bias_in, acc);
+    publish(0, stage_now);
+    fetch(min(1, a.blocks - 1));
+    conv_products<KF, NT, true>(w, KF, m.dilation, 2 * win, a.blocks, [&](int block) {
+        __syncthreads();
+        const uint4 *at = stage_now + half * win + wn * WP + col;
+        if (block + 1 < a.blocks) {
+            publish(block + 1, stage_next);
+            fetch(min(block + 2, a.blocks - 1));
+        }
+        uint4 *t = stage_now;
+        stage_now = stage_next;
+        stage_next = t;
+        return at;
+    }, acc);
+
+    // the finished rows' residual (x itself), on its way during the rest: whole rows of consecutive positions, as it is stored
+    const int rows = min(32, a.channels - wm * 32);
+    constexpr int kRowsAtOnce = 64 / WP;                 // rows a wavefront stores with one instruction
+    const int row0 = lane / WP, p_out = wn * WP + lane % WP, t_out = t0 + p_out;
+    const size_t at_out = (size_t)(rows > 0 ? wm * 32 : 0) * a.length + min(t_out, a.length - 1);
+    float x[32 / kRowsAtOnce];
+#pragma unroll
+    for (int i = 0; i < 32 / kRowsAtOnce; ++i) x[i] = m.in[at_out + (size_t)max(min(row0 + kRowsAtOnce * i, rows - 1), 0) * a.length];
+    // the inner rows: activated, zero in front of the first position, in pieces to LDS where the second convolution reads them
+    ConvWeights w2(m.w_skip + w_at, 0, KF);
+    bool large = false;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const float al = s_pairs[wm * 32 + split_acc_row(r, lane)].x;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) large = large || !(fabsf(al * acc[n][r]) < kShortSineLimit);
+    }
+    if (!__any(large)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = wm * 32 + split_acc_row(r, lane);
+            const float2 pair = s_pairs[row];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const float v = acc[n][r];
+                float y = v < 0.0f ? v * 0.01f : v;
+                if (wm * 32 + 8 * (r >> 2) < a.snake_channels) {   // (else no lane's row of these registers is a snake row)
+                    const float sn = short_sine(pair.x * v);
+                    y = row < a.snake_channels ? v + sn * sn * pair.y : y;
+                }
+                acc[n][r] = y;
+            }
+        }
+    } else {
+#pragma unroll 1
+        for (int r = 0; r < 16; ++r) {
+            const int row = wm * 32 + split_acc_row(r, lane);
+            const float2 pair = s_pairs[row];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n][r] = half_snake(acc[n][r], row < a.snake_channels, pair.x, pair.y);
+        }
+    }
+    __syncthreads();   // the stages have been read
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int p = wn * WP + 32 * n + col;
+        const bool in_front = t0 - (KF - 1) + p < 0;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {   // rows 8 g + 4 half .. + 3 of the tile: half of the eight channels of one place
+            const int block = wm * 2 + (g >> 1);
+            if (block >= a.blocks) continue;
+            const float4 v = make_float4(acc[n][4 * g], acc[n][4 * g + 1], acc[n][4 * g + 2], acc[n][4 * g + 3]);
+            const SplitFour s(in_front ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : v);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) reinterpret_cast<uint2 *>(&lds[(block * 6 + q * 2 + (g & 1)) * RN + p])[half] = s.piece[q];
+        }
+    }
+    start(bias_skip, acc);
+    __syncthreads();
+    conv_products<KF, NT, true>(w2, KF, 1, 2 * RN, a.blocks, [&](int block) { return const_cast<const uint4 *>(lds + (block * 6 + half) * RN + wn * WP + col); }, acc);
+
+    // + x, and out, in whole rows (see store_tile of conv_tile)
+    __syncthreads();   // the inner rows have been read
+    constexpr int kPitch = WP + 1;
+    float *const s_tile = reinterpret_cast<float *>(lds) + wave * (32 * kPitch);
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s_tile[split_acc_row(r, lane) * kPitch + 32 * n + col] = acc[n][r];
+    if (rows <= 0 || p_out >= TN || t_out >= a.length) return;
+#pragma unroll
+    for (int i = 0; i < 32 / kRowsAtOnce; ++i) {
+        const int row = row0 + kRowsAtOnce * i;
+        if (row < rows) m.out[at_out + (size_t)row * a.length] = x[i] + s_tile[row * kPitch + lane % WP];
+    }
+}
+
+template <int WM, int WN, int NT>
+__global__ void __launch_bounds__(64 * WM * WN, 2) k_res_block(const ResArgs a) {
+    extern __shared__ __align__(16) uint4 lds[];
+    __shared__ float2 s_pairs[kResMaxChannels];
+    const int z = a.order[blockIdx.y];
+    switch (a.member[z].kernel) {
+        case 3: res_block_tile<WM, WN, NT, 3>(a, a.member[z], lds, s_pairs); break;
+        case 7: res_block_tile<WM, WN, NT, 7>(a, a.member[z], lds, s_pairs); break;
+        default: res_block_tile<WM, WN, NT, 11>(a, a.member[z], lds, s_pairs); break;
+    }
+}
+
+template <int WM, int WN, int NT>
+int launch_res_block_n(State *st, const ResArgs &a, int count, char *error, size_t capacity) {
+    constexpr int RN = 32 * NT * WN;
+    int taps = 0, reach = 0;
+    for (int i = 0; i < count; ++i) {
+        taps = a.member[i].kernel > taps ? a.member[i].kernel : taps;
+        const int halo = (a.member[i].kernel - 1) * a.member[i].dilation;
+        reach = halo > reach ? halo : reach;
+    }
+    size_t lds = (size_t)2 * 6 * (RN + reach) * 16;                                   // two stages, or
+    const size_t inner = ((size_t)a.blocks * 6 * RN + 16) * 16;                        // the inner rows (a tap past the last place is read, not used), or
+    const size_t tiles = (size_t)WM * WN * 32 * (32 * NT + 1) * sizeof(float);        // the finished tiles
+    lds = inner > lds ? inner : lds;
+    lds = tiles > lds ? tiles : lds;
+    static bool raised = false;
+    if (!raised) {
+        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_res_block<WM, WN, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 112 * 1024));
+        raised = true;
+    }
+    const int finished = RN - (taps - 1);
+    hipLaunchKernelGGL((k_res_block<WM, WN, NT>), dim3((unsigned)((a.length + finished - 1) / finished), (unsigned)count), dim3(64 * WM * WN), lds, st->stream, a);
+    return hip_check(hipGetLastError(), "residual block launch", error, capacity);
+}
+
+// 64 positions to a wavefront, or 32 where that many workgroups still find a CU each: a wavefront's chain of products is then half as
+// long, which is all that counts there.  (A position's values do not depend on the tile it is in.)
+template <int WM, int WN>
+int launch_res_block(State *st, const ResArgs &a, int count, char *error, size_t capacity) {
+    const long narrow = (long)(a.length + 32 * WN - 11) / (32 * WN - 10) * count;
+    return narrow <= st->cu_count * 4 / 4 ? launch_res_block_n<WM, WN, 1>(st, a, count, error, capacity) : launch_res_block_n<WM, WN, 2>(st, a, count, error, capacity);
 }
 
 __global__ void __launch_bounds__(256) k_conv_pack(const float *src, uint4 *dst, size_t count, int out_ch, int in_ch, int kernel, int blocks) {
@@ -817,11 +1074,14 @@ static int conv1d_prepare(State *st, const float *dev_input, float *dev_output, 
     return 0;
 }
 
-// few output channels: one row of wavefronts, wider in time; too few large tiles to fill the chip (and enough input
-// channels to share out): small tiles with the channels split over the wavefronts
+// few output channels: one row of wavefronts, wider in time; too few large tiles to fill the chip and enough input channels to
+// share out (more than one block for each of four wavefronts): small tiles with the channels split over the wavefronts.  The two
+// add in different orders, so the choice is the shape's alone, for single, batched and fused launches alike.  216 channels: the two
+// meet at 4096 positions (three members, 72 us either way), and the large tiles' launch has no more wavefronts than it needs;
+// 108 channels: the small tiles' three members at 1280 positions take 14 us, a fused block of large tiles 41.
 static bool conv_takes_split(const State *st, int in_channels, int out_channels, int length) {
     const long tiles = out_channels <= 32 ? (long)((length + 255) / 256) : (long)((out_channels + 63) / 64) * ((length + 127) / 128);
-    return tiles < st->cu_count && in_channels >= 32;
+    return in_channels > 64 && tiles < (in_channels > kResMaxChannels ? (long)st->cu_count / 4 : (long)st->cu_count * 3 / 8);
 }
 
 static int conv1d_launch(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
@@ -992,6 +1252,138 @@ extern "C" int mynah_hip_rows_combine_dev(void *state, const float *const *dev_i
     }
     hipLaunchKernelGGL(k_rows_combine, dim3((unsigned)((a.count + 255) / 256)), dim3(256), 0, st->stream, a);
     return hip_check(hipGetLastError(), "rows_combine launch", error, capacity);
+}
+
+// One position (block) of every branch in one launch, where the fused kernel takes it; *done tells.
+static int res_position(State *st, const mynah_hip_res_block *blocks, size_t branches, size_t stride, const float *const *in, float *const *out, size_t channels,
+                        size_t length, bool *done, char *error, size_t capacity) {
+    *done = false;
+    ResArgs a{};
+    // Above 32 channels only while the launch does not fill the chip: with enough tiles the two launches overlap their phases
+    // better (108 channels x 16384: 138 us a position fused, 124 as two launches; 54 x 32768: 94 and 77; 27 x 65536: 63 and 78).
+    if (conv_takes_split(st, (int)channels, (int)channels, (int)length)) return 0;
+    if (channels > 32 && (length + 53) / 54 * branches > (size_t)st->cu_count) return 0;
+    for (size_t i = 0; i < branches; ++i) {
+        const mynah_hip_res_block &b = blocks[i * stride];
+        const int k = b.kernel_in;
+        if (channels > (size_t)kResMaxChannels || k != b.kernel_skip || (k != 3 && k != 7 && k != 11) || (k - 1) * (long)b.dilation > kResMaxReach) return 0;
+    }
+    a.channels = (int)channels;
+    a.length = (int)length;
+    a.snake_channels = (int)(channels / 2);
+    for (size_t i = 0; i < branches; ++i) {
+        const mynah_hip_res_block &b = blocks[i * stride];
+        ResMember &m = a.member[i];
+        ConvBlocks w_in, w_skip;
+        if (cached_conv_blocks(st, b.weight_in, channels, channels, (size_t)b.kernel_in, &w_in, error, capacity) != 0 ||
+            cached_conv_blocks(st, b.weight_skip, channels, channels, (size_t)b.kernel_skip, &w_skip, error, capacity) != 0 ||
+            cached_vector(st, b.bias_in, channels, &m.b_in, error, capacity) != 0 || cached_vector(st, b.bias_skip, channels, &m.b_skip, error, capacity) != 0)
+            return -1;
+        if (a.snake_channels > 0) {
+            const float *in_pairs = nullptr, *skip_pairs = nullptr;
+            if (cached_snake_pairs(st, b.alpha_in, channels / 2, &in_pairs, error, capacity) != 0 ||
+                cached_snake_pairs(st, b.alpha_skip, channels / 2, &skip_pairs, error, capacity) != 0)
+                return -1;
+            m.snake_in = reinterpret_cast<const float2 *>(in_pairs);
+            m.snake_skip = reinterpret_cast<const float2 *>(skip_pairs);
+        }
+        m.in = in[i];
+        m.out = out[i];
+        m.w_in = w_in.data;
+        m.w_skip = w_skip.data;
+        m.kernel = b.kernel_in;
+        m.dilation = b.dilation;
+        a.blocks = w_in.blocks;
+        a.tiles = w_in.tiles;
+        size_t at = i;   // most taps first
+        for (; at > 0 && a.member[a.order[at - 1]].kernel < m.kernel; --at) a.order[at] = a.order[at - 1];
+        a.order[at] = (int)i;
+    }
+    *done = true;
+    if (channels <= 32) return launch_res_block<1, 4>(st, a, (int)branches, error, capacity);
+    if (channels <= 64) return launch_res_block<2, 2>(st, a, (int)branches, error, capacity);
+    return launch_res_block<4, 2>(st, a, (int)branches, error, capacity);
+}
+
+extern "C" int mynah_hip_res_layer_dev(void *state, const mynah_hip_res_block *blocks, size_t branches, size_t positions, const float *dev_input,
+                                       float *dev_output, size_t channels, size_t length, const float *then_alpha, float *const *dev_work, char *error,
+                                       size_t capacity) {
+    State *st = enter_state(state);
+    if (st == nullptr || blocks == nullptr || branches == 0 || branches > (size_t)kConvBatchMax || positions == 0 || dev_input == nullptr || dev_output == nullptr ||
+        dev_input == dev_output || dev_work == nullptr || channels == 0 || channels > (size_t)INT_MAX || length == 0 || length > (size_t)INT_MAX) {
+        set_error(error, capacity, "invalid residual layer arguments (one to four branches)");
+        return -1;
+    }
+    for (size_t i = 0; i < 3 * branches; ++i) {
+        bool distinct = dev_work[i] != nullptr && dev_work[i] != dev_input && dev_work[i] != dev_output;
+        for (size_t j = 0; j < i; ++j) distinct = distinct && dev_work[i] != dev_work[j];
+        if (!distinct) {
+            set_error(error, capacity, "residual layer: work rows must be buffers of their own");
+            return -1;
+        }
+    }
+    for (size_t i = 0; i < branches * positions; ++i) {
+        const mynah_hip_res_block &b = blocks[i];
+        if (b.weight_in == nullptr || b.weight_skip == nullptr || b.kernel_in <= 0 || b.kernel_skip <= 0 || b.dilation <= 0 ||
+            (channels >= 2 && (b.alpha_in == nullptr || b.alpha_skip == nullptr))) {
+            set_error(error, capacity, "residual layer: missing weight or alpha");
+            return -1;
+        }
+    }
+    const size_t snake = channels / 2;
+    float *const *const currents = dev_work, *const *const activated = dev_work + branches, *const *const residuals = dev_work + 2 * branches;
+    const float *source[kConvBatchMax];   // each branch's rows so far
+    float *target[kConvBatchMax];
+    for (size_t i = 0; i < branches; ++i) source[i] = dev_input;
+    bool have_activated = false;          // `activated` holds the source rows through the next block's first half-snake
+    for (size_t p = 0; p < positions; ++p) {
+        bool done = false;
+        // (the fused block reads its neighbours' rows: never in place)
+        for (size_t i = 0; i < branches; ++i) target[i] = source[i] == currents[i] ? residuals[i] : currents[i];
+        if (res_position(st, blocks + p, branches, positions, source, target, channels, length, &done, error, capacity) != 0) return -1;
+        if (!done) {
+            const float *alphas[kConvBatchMax];
+            if (!have_activated)
+                for (size_t i = 0; i < branches; ++i) {
+                    // (one launch when all branches start from the same rows)
+                    if (source[i] == dev_input && i > 0) continue;
+                    const size_t outs = source[i] == dev_input ? branches : 1;
+                    for (size_t j = 0; j < outs; ++j) alphas[j] = snake != 0 ? blocks[(i + j) * positions + p].alpha_in : dev_input;
+                    const float *in[1] = {source[i]};
+                    if (mynah_hip_rows_combine_dev(state, in, 1, 1.0f, activated + i, alphas, outs, channels, length, snake, error, capacity) != 0) return -1;
+                }
+            mynah_hip_conv1d_item items[kConvBatchMax] = {};
+            float *const *const inner = target[0] == residuals[0] ? currents : residuals;   // the buffers neither read nor finished by this position
+            for (size_t i = 0; i < branches; ++i) {
+                const mynah_hip_res_block &b = blocks[i * positions + p];
+                items[i] = mynah_hip_conv1d_item{activated[i], inner[i], b.kernel_in, b.dilation, b.weight_in, b.bias_in, {nullptr, nullptr, 1.0f, 1, b.alpha_skip, snake, nullptr}};
+            }
+            bool in_place = source[0] == inner[0];   // the source rows are still needed: they move on in place below
+            if (in_place) {
+                for (size_t i = 0; i < branches; ++i) {
+                    items[i].dev_output = target[i];
+                    target[i] = const_cast<float *>(source[i]);
+                }
+            }
+            if (mynah_hip_conv1d_fused_batch(state, items, branches, (int)channels, (int)channels, (int)length, error, capacity) != 0) return -1;
+            const bool more = p + 1 < positions;
+            for (size_t i = 0; i < branches; ++i) {
+                const mynah_hip_res_block &b = blocks[i * positions + p];
+                const float *inner_rows = items[i].dev_output;
+                items[i] = mynah_hip_conv1d_item{inner_rows, target[i], b.kernel_skip, 1, b.weight_skip, b.bias_skip,
+                                                 {source[i], nullptr, 1.0f, more ? 1 : 0, more ? blocks[i * positions + p + 1].alpha_in : nullptr, more ? snake : 0,
+                                                  more ? activated[i] : nullptr}};
+            }
+            if (mynah_hip_conv1d_fused_batch(state, items, branches, (int)channels, (int)channels, (int)length, error, capacity) != 0) return -1;
+            have_activated = more;
+        } else {
+            have_activated = false;
+        }
+        for (size_t i = 0; i < branches; ++i) source[i] = target[i];
+    }
+    float *outs[1] = {dev_output};
+    const float *alphas[1] = {then_alpha};
+    return mynah_hip_rows_combine_dev(state, source, branches, (float)(1.0 / (double)branches), outs, alphas, 1, channels, length, snake, error, capacity);
 }
 
 extern "C" int mynah_hip_snake_dev(void *state, float *dev_data, const float *alpha, size_t channels, size_t length, size_t snake_channels,

@@ -78,7 +78,7 @@ struct PackedWeight {
 struct WeightKey {
     const void *host;
     size_t bytes;
-    int kind;   // 0 plain f32 vector/matrix, 1 + qtype*2 + arith for converted matrices, 64 + kernel + 32 * in_ch for conv1d chunks, -taps for split products
+    int kind;   // 0 plain f32 vector/matrix, 1 + qtype*2 + arith for converted matrices, 64 + kernel + 32 * in_ch for conv1d chunks, -taps for split products, -100 for snake pairs
     bool operator==(const WeightKey &o) const { return host == o.host && bytes == o.bytes && kind == o.kind; }
 };
 struct WeightKeyHash {
@@ -232,6 +232,8 @@ struct ConvBlocks {
     const uint4 *data = nullptr;
     int tiles = 0, blocks = 0;
 };
+// (alpha, 1 / (alpha + 1e-9f)) of a half-snake's rows, as the kernels would form the second
+int cached_snake_pairs(State *st, const float *host, size_t n, const float **dev, char *error, size_t capacity);
 int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch, size_t kernel, ConvBlocks *out, char *error, size_t capacity);
 // An f32 weight [n, channels, taps] in the order in which split_product.hip's kernels take it; n a multiple of 32, channels of 64.
 int cached_split_weight(State *st, const float *host, size_t n, size_t channels, size_t taps, const float4 **out, char *error, size_t capacity);
