@@ -814,7 +814,7 @@ int launch_res_block_n(State *st, const ResArgs &a, int count, char *error, size
 template <int WM, int WN>
 int launch_res_block(State *st, const ResArgs &a, int count, char *error, size_t capacity) {
     const long narrow = (long)(a.length + 32 * WN - 11) / (32 * WN - 10) * count;
-    return narrow <= st->cu_count * 4 / 4 ? launch_res_block_n<WM, WN, 1>(st, a, count, error, capacity) : launch_res_block_n<WM, WN, 2>(st, a, count, error, capacity);
+    return narrow <= st->cu_count ? launch_res_block_n<WM, WN, 1>(st, a, count, error, capacity) : launch_res_block_n<WM, WN, 2>(st, a, count, error, capacity);
 }
 
 __global__ void __launch_bounds__(256) k_conv_pack(const float *src, uint4 *dst, size_t count, int out_ch, int in_ch, int kernel, int blocks) {

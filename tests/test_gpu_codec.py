@@ -158,6 +158,45 @@ def test_fused_res_layer_is_the_operator_sequence(pkg, backend, orc, nerr, C, L)
         d.free()
 
 
+# a block as one launch: every tile shape (at most 32, 64, 128 channels), rows and channels one off a tile's, a chip full of tiles
+@pytest.mark.parametrize("C,L", [(16, 1), (27, 54), (32, 55), (33, 53), (64, 109), (65, 107), (108, 641), (128, 54), (128, 700), (27, 20000)])
+def test_res_layer_call(pkg, backend, orc, nerr, C, L):
+    """mynah_hip_res_layer_dev is the operator sequence bit for bit, whatever follows (a half-snake or none), and refuses work rows
+    that are the layer's own or each other's."""
+    import importlib
+    codec = importlib.import_module(pkg.__name__ + ".codec")
+    _announce("residual layer call %d x %d" % (C, L))
+    x, blocks = _res_layer_inputs(C, L, 90 + C)
+    blocks[1][1][0][0] = blocks[2][2][2][-1] = np.float32(9000.0)   # a half-snake's argument beyond the fast range of its sine
+    then = np.full(C // 2, 0.7, np.float32)
+    n = C * L
+    din = backend.alloc(n).write(x)
+    bufs = [backend.alloc(n) for _ in range(11)]
+    at = [b.ptr for b in bufs]
+    codec.res_layer(backend, blocks, din.ptr, at[0], C, L, *at[1:5])
+    want = bufs[0].read()
+    codec.res_layer_batched(backend, blocks, din.ptr, at[1], C, L, at[2:5], at[5:8], at[8:11])
+    assert np.array_equal(want.view(np.uint32), bufs[1].read().view(np.uint32))
+    assert np.array_equal(din.read().reshape(C, L), x), "the layer's input was written"
+    backend.snake_dev(at[0], then, C, L, C // 2)
+    want = bufs[0].read()
+    codec.res_layer_batched(backend, blocks, din.ptr, at[1], C, L, at[2:5], at[5:8], at[8:11], then_alpha=then)
+    assert np.array_equal(want.view(np.uint32), bufs[1].read().view(np.uint32))
+    if n < 8000:
+        total = np.zeros_like(x)
+        for branch in blocks:
+            cur = x.copy()
+            for a_in, (w_in, b_in), a_skip, (w_skip, b_skip), d in branch:
+                cur = cur + orc.conv1d_causal(orc.snake(orc.conv1d_causal(orc.snake(cur, a_in, C // 2), w_in, b_in, d), a_skip, C // 2), w_skip, b_skip, 1)
+            total += cur
+        assert nerr(bufs[1].read().reshape(C, L), orc.snake(total * np.float32(1.0 / 3.0), then, C // 2)) < 1e-5
+    for work in ([din.ptr] + at[3:11], at[2:10] + [at[2]], [at[1]] + at[3:11]):
+        with pytest.raises(pkg.BackendError):
+            codec.res_layer_batched(backend, blocks, din.ptr, at[1], C, L, work[0:3], work[3:6], work[6:9])
+    for d in bufs + [din]:
+        d.free()
+
+
 def test_conv_batch_members_and_refusals(pkg, backend):
     """conv1d_fused_batch, two to four members: with tap counts outside 3 / 7 / 11 (run one after the other) and with them
     (one launch) every member gets its own conv1d_fused result bit for bit; a member that writes what another reads is refused."""
