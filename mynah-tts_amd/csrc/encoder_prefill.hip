@@ -31,6 +31,7 @@
 // All products are "NT": C[m][n] = sum_k A[m][k] * W[n][k], both operands K-contiguous, which is how
 // the 32x32x16 MFMA wants them: lane l supplies row (l % 32) of A (or of W) and the eight consecutive
 // k values 8*(l / 32) .. +7 of the 16-deep step.
+#include <algorithm>
 #include <new>
 
 #include "device_common.h"
@@ -58,8 +59,6 @@ struct mynah_hip_encoder {
     float *x = nullptr, *part = nullptr;   // part: [splits, Tpad, w] partial products of the O and FFN-down products
     _Float16 *nrm = nullptr, *qk = nullptr, *vt = nullptr, *ctx = nullptr, *hid = nullptr;
     _Float16 *nrm_alloc = nullptr, *hid_alloc = nullptr;   // nrm and hid begin kLeadRows rows into these
-    int *ids = nullptr;        // [tpad_max] token ids, followed by one EncParams
-    int *ids_host = nullptr;   // pinned twin of ids
     EncParams *params = nullptr;
     std::unordered_map<int, hipGraphExec_t> graphs;   // by padded length
     std::unordered_map<int, int> eager_runs;          // a padded length runs eagerly once before it is captured
@@ -271,45 +270,44 @@ k_enc_gemm(const _Float16 *const a_arg, const _Float16 *const w_arg, const int M
     }
 }
 
-// Token gather + position add (src/graph.c:729-737, :649-651), f32 tables.  Rows [tokens, tpad) are zeroed.
-__global__ void __launch_bounds__(kThreads) k_enc_embed_f32(const int *ids, const EncParams *params, const float *tok, const float *pos, float *x, int width) {
-    const int t = blockIdx.x;
-    const int tokens = params->tokens;
-    for (int c = threadIdx.x * 4; c < width; c += kThreads * 4) {
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t < tokens) {
-            const float4 a = *reinterpret_cast<const float4 *>(tok + (size_t)ids[t] * width + c), b = *reinterpret_cast<const float4 *>(pos + (size_t)t * width + c);
-            v = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+// A lane's part of a row pass from here on: the LayerNorm of the row it holds in v (pieces past the row are zero), written as f16
+// (operand of the next product) or f32.  Two-pass statistics (src/kernels.c:186-244, eps 1e-5).
+enum { ROWS_RESULT = 0, ROWS_F16 = 1, ROWS_F32 = 2 };   // params->out (real rows only), f16 operand rows, f32 operand rows
+template <int OUT, int NV>
+__device__ __forceinline__ void norm_row(const float4 (&v)[NV], const float4 (&gg)[NV], const float4 (&bb)[NV], int lane, int row, int width, void *out_rows) {
+    const int n4 = width / 4;
+    float s = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) s += (v[u].x + v[u].y) + (v[u].z + v[u].w);   // pieces past the row are zero
+    const float mean = wave_sum(s) / (float)width;
+    float q = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        if (lane + 64 * u < n4) {
+            const float a = v[u].x - mean, b = v[u].y - mean, c = v[u].z - mean, d = v[u].w - mean;
+            q += (a * a + b * b) + (c * c + d * d);
         }
-        *reinterpret_cast<float4 *>(x + (size_t)t * width + c) = v;
     }
-}
-
-// Token gather + position add (src/graph.c:729-737, :649-651).  Rows [tokens, tpad) are zeroed.
-__global__ void __launch_bounds__(kThreads) k_enc_embed(const int *ids, const EncParams *params, const _Float16 *tok, const _Float16 *pos,
-                                                        float *x, int width) {
-    const int t = blockIdx.x;
-    const int tokens = params->tokens;
-    uint16_t *embed_out = params->embed_out;
-    for (int c = threadIdx.x * 8; c < width; c += kThreads * 8) {
-        float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
-        if (t < tokens) {
-            const uint4 traw = *reinterpret_cast<const uint4 *>(tok + (size_t)ids[t] * width + c);
-            const half8 tv = *reinterpret_cast<const half8 *>(&traw);
-            const half8 pv = *reinterpret_cast<const half8 *>(pos + (size_t)t * width + c);
-            if (embed_out != nullptr) *reinterpret_cast<uint4 *>(embed_out + (size_t)t * width + c) = traw;
-            lo = make_float4((float)tv[0] + (float)pv[0], (float)tv[1] + (float)pv[1], (float)tv[2] + (float)pv[2], (float)tv[3] + (float)pv[3]);
-            hi = make_float4((float)tv[4] + (float)pv[4], (float)tv[5] + (float)pv[5], (float)tv[6] + (float)pv[6], (float)tv[7] + (float)pv[7]);
+    const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)width + 1.0e-5f);
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int i = lane + 64 * u;
+        if (i < n4) {
+            const float y0 = (v[u].x - mean) * rstd * gg[u].x + bb[u].x, y1 = (v[u].y - mean) * rstd * gg[u].y + bb[u].y;
+            const float y2 = (v[u].z - mean) * rstd * gg[u].z + bb[u].z, y3 = (v[u].w - mean) * rstd * gg[u].w + bb[u].w;
+            if constexpr (OUT == ROWS_F16) {
+                half4 h = {(_Float16)y0, (_Float16)y1, (_Float16)y2, (_Float16)y3};
+                reinterpret_cast<half4 *>(static_cast<_Float16 *>(out_rows) + (size_t)row * width)[i] = h;
+            } else {
+                reinterpret_cast<float4 *>(static_cast<float *>(out_rows) + (size_t)row * width)[i] = make_float4(y0, y1, y2, y3);
+            }
         }
-        *reinterpret_cast<float4 *>(x + (size_t)t * width + c) = lo;
-        *reinterpret_cast<float4 *>(x + (size_t)t * width + c + 4) = hi;
     }
 }
 
 // Row pass between two products, one wavefront per row: first the residual update
-// x += sum over K splits of the previous product's partials (src/graph.c:470, :316), then LayerNorm with
-// two-pass statistics (src/kernels.c:186-244, eps 1e-5) written as f16 (operand of the next product) or
-// f32 (the encoder's output, to params->out, rows below params->tokens only).  gain == nullptr: no
+// x += sum over K splits of the previous product's partials (src/graph.c:470, :316), then LayerNorm (norm_row), the
+// encoder's output going to params->out, rows below params->tokens only.  gain == nullptr: no
 // LayerNorm, the updated row is copied out as f32.  A lane keeps its NV float4 pieces of the row in
 // registers (width <= 256 * NV; the widest supported row, 4096, takes NV = 16).
 // (Argument order: what the row's first requests are formed from stands among the first fourteen dwords, which are in registers
@@ -319,7 +317,6 @@ __global__ void __launch_bounds__(kThreads) k_enc_embed(const int *ids, const En
 // (256 rows: 64 workgroups) -- a row per workgroup spreads them over the chip.
 // No request stands under a condition (a place beyond the row, or a partial plane the product did not write, asks for a
 // place that exists and is set to zero afterwards): the waits then name exactly the requests they need.
-enum { ROWS_RESULT = 0, ROWS_F16 = 1, ROWS_F32 = 2 };   // params->out (real rows only), f16 operand rows, f32 operand rows
 template <int OUT, int NV, int RPW>
 __global__ void __launch_bounds__(64 * RPW) k_enc_rows(float *x, const float *part, const EncParams *params, int rows, int width, int splits,
                                                         size_t split_stride, const float *gain, const float *bias, void *out_rows) {
@@ -395,35 +392,7 @@ __global__ void __launch_bounds__(64 * RPW) k_enc_rows(float *x, const float *pa
         }
         return;
     }
-    float s = 0.0f;
-#pragma unroll
-    for (int u = 0; u < NV; ++u) s += (v[u].x + v[u].y) + (v[u].z + v[u].w);   // pieces past the row are zero
-    const float mean = wave_sum(s) / (float)width;
-    float q = 0.0f;
-#pragma unroll
-    for (int u = 0; u < NV; ++u) {
-        if (lane + 64 * u < n4) {
-            const float a = v[u].x - mean, b = v[u].y - mean, c = v[u].z - mean, d = v[u].w - mean;
-            q += (a * a + b * b) + (c * c + d * d);
-        }
-    }
-    const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)width + 1.0e-5f);
-#pragma unroll
-    for (int u = 0; u < NV; ++u) {
-        const int i = lane + 64 * u;
-        if (i < n4) {
-            const float y0 = (v[u].x - mean) * rstd * gg[u].x + bb[u].x, y1 = (v[u].y - mean) * rstd * gg[u].y + bb[u].y;
-            const float y2 = (v[u].z - mean) * rstd * gg[u].z + bb[u].z, y3 = (v[u].w - mean) * rstd * gg[u].w + bb[u].w;
-            if constexpr (OUT == ROWS_F16) {
-                half4 h = {(_Float16)y0, (_Float16)y1, (_Float16)y2, (_Float16)y3};
-                reinterpret_cast<half4 *>(static_cast<_Float16 *>(out_rows) + (size_t)row * width)[i] = h;
-            } else if constexpr (OUT == ROWS_F32) {
-                reinterpret_cast<float4 *>(static_cast<float *>(out_rows) + (size_t)row * width)[i] = make_float4(y0, y1, y2, y3);
-            } else {
-                reinterpret_cast<float4 *>(params->out + (size_t)row * width)[i] = make_float4(y0, y1, y2, y3);
-            }
-        }
-    }
+    norm_row<OUT, NV>(v, gg, bb, lane, row, width, OUT == ROWS_RESULT ? static_cast<void *>(params->out) : out_rows);
 }
 
 template <int OUT>
@@ -437,6 +406,69 @@ void launch_rows(State *st, int width, float *x, const float *part, int splits, 
     else
         hipLaunchKernelGGL((k_enc_rows<OUT, 16, kRowsPerWg>), rows_grid, dim3(64 * kRowsPerWg), 0, st->stream, x, part, params, rows, width, splits, split_stride,
                            gain, bias, out_rows);
+}
+
+// The pass in front of the first product: token gather + position add (src/graph.c:729-737, :649-651), then the first layer's
+// LayerNorm; a wavefront per row, rows [tokens, rows) zero.  All that changes from call to call arrives with this launch: the
+// ids are kernel arguments, and the first workgroup leaves the rest (EncParams) in device memory for the graph that follows.
+// So a call neither copies nor waits for the previous one's copies, and calls queue up behind each other: with two copies of
+// 6 us and a wait in front of them, and the gather and the norm launches of their own, 256 rows took 254 us, 192 rows of the f32
+// form 560; now 234 and 532.
+constexpr int kIdsPerLaunch = 512;   // kernel arguments end at 4 KiB; longer inputs take a second launch
+struct EncFirst {
+    const void *tok, *pos;     // f16 or f32, as the operands
+    float *x;
+    const float *gain, *bias;
+    void *out_rows;
+    EncParams *params;
+    EncParams call;
+    int first, rows, width;
+    int ids[kIdsPerLaunch];
+};
+template <int OUT, int NV>
+__global__ void __launch_bounds__(64) k_enc_first(const EncFirst a) {
+    const int lane = threadIdx.x, at_row = blockIdx.x, row = a.first + at_row, n4 = a.width / 4;
+    const bool real = row < a.call.tokens;
+    const size_t id = real ? (size_t)a.ids[at_row] : 0, pos = real ? (size_t)row : 0;
+    if (row == 0 && lane == 0) *a.params = a.call;
+    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 v[NV], gg[NV], bb[NV];
+    const float4 *const gain4 = reinterpret_cast<const float4 *>(a.gain), *const bias4 = reinterpret_cast<const float4 *>(a.bias != nullptr ? a.bias : a.gain);
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int i = lane + 64 * u, at = i < n4 ? i : n4 - 1;
+        gg[u] = gain4[at];
+        bb[u] = bias4[at];
+        if constexpr (OUT == ROWS_F16) {
+            const half4 t = reinterpret_cast<const half4 *>(static_cast<const _Float16 *>(a.tok) + id * a.width)[at];
+            const half4 p = reinterpret_cast<const half4 *>(static_cast<const _Float16 *>(a.pos) + pos * a.width)[at];
+            if (a.call.embed_out != nullptr && real && i < n4) reinterpret_cast<half4 *>(a.call.embed_out + (size_t)row * a.width)[i] = t;
+            v[u] = make_float4((float)t[0] + (float)p[0], (float)t[1] + (float)p[1], (float)t[2] + (float)p[2], (float)t[3] + (float)p[3]);
+        } else {
+            const float4 t = reinterpret_cast<const float4 *>(static_cast<const float *>(a.tok) + id * a.width)[at];
+            const float4 p = reinterpret_cast<const float4 *>(static_cast<const float *>(a.pos) + pos * a.width)[at];
+            v[u] = make_float4(t.x + p.x, t.y + p.y, t.z + p.z, t.w + p.w);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int i = lane + 64 * u;
+        if (!real || i >= n4) v[u] = zero4;
+        if (a.bias == nullptr) bb[u] = zero4;
+        if (i < n4) reinterpret_cast<float4 *>(a.x + (size_t)row * a.width)[i] = v[u];
+    }
+    norm_row<OUT, NV>(v, gg, bb, lane, row, a.width, a.out_rows);
+}
+
+template <int OUT>
+int launch_first(State *st, EncFirst &a, const int32_t *ids, char *error, size_t capacity) {
+    for (a.first = 0; a.first < a.rows; a.first += kIdsPerLaunch) {
+        const int rows = std::min(kIdsPerLaunch, a.rows - a.first), real = std::clamp(a.call.tokens - a.first, 0, kIdsPerLaunch);
+        std::copy(ids + a.first, ids + a.first + real, a.ids);
+        if (a.width <= 1024) hipLaunchKernelGGL((k_enc_first<OUT, 4>), dim3((unsigned)rows), dim3(64), 0, st->stream, a);
+        else hipLaunchKernelGGL((k_enc_first<OUT, 16>), dim3((unsigned)rows), dim3(64), 0, st->stream, a);
+    }
+    return hip_check(hipGetLastError(), "encoder embedding launch", error, capacity);
 }
 
 // One (32-query tile, head): S = scale * Q K^T over all keys (f32, in LDS) -> row softmax numerators
@@ -649,12 +681,10 @@ int pick_splits(int k) {
     return 1;
 }
 
-// Every kernel of one prefill over `tpad` padded rows, in stream order.  Everything that changes from call to
+// Every kernel of one prefill over `tpad` padded rows behind k_enc_first, in stream order.  Everything that changes from call to
 // call (token count, output pointers) is read from e->params on the device, so the sequence can be captured once.
 int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size_t capacity) {
     const int w = (int)e->width, f = (int)e->ffn;
-    hipLaunchKernelGGL(k_enc_embed, dim3(tpad), dim3(kThreads), 0, st->stream, e->ids, e->params, static_cast<const _Float16 *>(e->tok->data),
-                       static_cast<const _Float16 *>(e->pos->data), e->x, w);
     const float scale = 1.0f / sqrtf((float)e->head_width);
     const size_t lds = attention_lds_bytes((size_t)tpad);
     const size_t split_stride = (size_t)tpad * w;
@@ -664,7 +694,7 @@ int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size
     const float *pending = nullptr;   // partials of the last product, not yet added to x
     int pending_splits = 0;
     for (size_t l = 0; l < e->layers; ++l) {
-        launch_rows<ROWS_F16>(st, w, e->x, pending, pending_splits, split_stride, e->n1g[l], e->n1b[l], e->nrm, e->params, tpad);
+        if (l > 0) launch_rows<ROWS_F16>(st, w, e->x, pending, pending_splits, split_stride, e->n1g[l], e->n1b[l], e->nrm, e->params, tpad);
         GemmArgs g{};
         g.a = e->nrm; g.w = static_cast<const _Float16 *>(e->qkv[l]->data); g.M = tpad; g.N = 3 * w; g.K = w;
         g.out = e->qk; g.vt = e->vt; g.width = w;
@@ -835,13 +865,11 @@ constexpr size_t kMaxSplitsF32 = 12;   // planes of partial sums; the next pass 
 int enqueue_prefill_f32(State *st, mynah_hip_encoder *e, int tpad, char *error, size_t capacity) {
     const size_t w = e->width, f = e->ffn, taps = e->taps, rows = (size_t)tpad;
     const float scale = 1.0f / sqrtf((float)e->head_width);
-    hipLaunchKernelGGL(k_enc_embed_f32, dim3(tpad), dim3(kThreads), 0, st->stream, e->ids, e->params, static_cast<const float *>(e->tok32->data),
-                       static_cast<const float *>(e->pos32->data), e->x, (int)w);
     const int o_splits = split_product_splits(st, rows, w, w, kMaxSplitsF32), up_splits = split_product_splits(st, rows, w, f, kMaxSplitsF32),
               down_splits = split_product_splits(st, rows, f, w, kMaxSplitsF32);
     const float *pending = nullptr;   // partial sums of the last product, not yet added to x
     for (size_t l = 0; l < e->layers; ++l) {
-        launch_rows<ROWS_F32>(st, (int)w, e->x, pending, down_splits, rows * w, e->n1g[l], e->n1b[l], e->f_nrm, e->params, tpad);
+        if (l > 0) launch_rows<ROWS_F32>(st, (int)w, e->x, pending, down_splits, rows * w, e->n1g[l], e->n1b[l], e->f_nrm, e->params, tpad);
         // (not split: the attention kernel reads every row several times and would add the planes up as often)
         if (launch_split_product(st, e->f_nrm, e->qkv32[l], rows, w, 1, 3 * w, 1, e->f_qkv, error, capacity) != 0) return -1;
         hipLaunchKernelGGL(k_enc_attention_f32, dim3(tpad / kQTile, (unsigned)e->heads), dim3(kThreads), attention_lds_bytes(rows), st->stream, e->f_qkv, e->f_ctx,
@@ -966,7 +994,7 @@ extern "C" int mynah_hip_encoder_create(void *state, const mynah_hip_encoder_des
             alloc(reinterpret_cast<void **>(&e->f_qkv), tp * 3 * w * sizeof(float)) != 0 || alloc(reinterpret_cast<void **>(&e->f_ctx), (tp * w + pad) * sizeof(float)) != 0 ||
             alloc(reinterpret_cast<void **>(&e->f_hid_alloc), ((kLeadRows + tp) * f + pad) * sizeof(float)) != 0 ||
             alloc(reinterpret_cast<void **>(&e->part), tp * wide * sizeof(float)) != 0 ||
-            alloc(reinterpret_cast<void **>(&e->ids), tp * sizeof(int) + sizeof(EncParams)) != 0)
+            alloc(reinterpret_cast<void **>(&e->params), sizeof(EncParams)) != 0)
             return fail();
         e->f_nrm = e->f_nrm_alloc + kLeadRows * w;   // rows -2 and -1 stay zero
         e->f_hid = e->f_hid_alloc + kLeadRows * f;
@@ -974,16 +1002,12 @@ extern "C" int mynah_hip_encoder_create(void *state, const mynah_hip_encoder_des
         if (alloc(reinterpret_cast<void **>(&e->x), tp * w * sizeof(float)) != 0 || alloc(reinterpret_cast<void **>(&e->nrm_alloc), (kLeadRows + tp) * w * 2) != 0 ||
             alloc(reinterpret_cast<void **>(&e->qk), tp * 2 * w * 2) != 0 || alloc(reinterpret_cast<void **>(&e->vt), w * tp * 2) != 0 ||
             alloc(reinterpret_cast<void **>(&e->ctx), tp * w * 2) != 0 || alloc(reinterpret_cast<void **>(&e->hid_alloc), (kLeadRows + tp) * f * 2) != 0 ||
-            alloc(reinterpret_cast<void **>(&e->ids), tp * sizeof(int) + sizeof(EncParams)) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->params), sizeof(EncParams)) != 0 ||
             alloc(reinterpret_cast<void **>(&e->part), kMaxSplits * tp * w * sizeof(float)) != 0)
             return fail();
         e->nrm = e->nrm_alloc + kLeadRows * w;   // rows -2 and -1 stay zero; widths are multiples of 64, so both stay 16-byte aligned
         e->hid = e->hid_alloc + kLeadRows * f;
     }
-    if (hip_check(hipHostMalloc(reinterpret_cast<void **>(&e->ids_host), tp * sizeof(int) + sizeof(EncParams), hipHostMallocDefault),
-                  "encoder ids staging", error, capacity) != 0)
-        return fail();
-    e->params = reinterpret_cast<EncParams *>(e->ids + tp);   // tp is a multiple of 64: 8-byte aligned
     if (attention_lds_bytes(e->tpad_max) > 48 * 1024) {
         const int bytes = (int)attention_lds_bytes(e->tpad_max);
         if (hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<1, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
@@ -1003,13 +1027,12 @@ extern "C" void mynah_hip_encoder_destroy(void *state, mynah_hip_encoder *e) {
     if (st != nullptr) (void)hipStreamSynchronize(st->stream);
     for (auto &g : e->graphs)
         if (g.second != nullptr) (void)hipGraphExecDestroy(g.second);
-    for (void *p : {(void *)e->x, (void *)e->nrm_alloc, (void *)e->qk, (void *)e->vt, (void *)e->ctx, (void *)e->hid_alloc, (void *)e->ids, (void *)e->part})
+    for (void *p : {(void *)e->x, (void *)e->nrm_alloc, (void *)e->qk, (void *)e->vt, (void *)e->ctx, (void *)e->hid_alloc, (void *)e->params, (void *)e->part})
         if (p != nullptr) (void)hipFree(p);
     for (_Float16 *p : e->conv_up) (void)hipFree(p);
     for (_Float16 *p : e->conv_down) (void)hipFree(p);
     for (void *p : {(void *)e->f_nrm_alloc, (void *)e->f_qkv, (void *)e->f_ctx, (void *)e->f_hid_alloc})
         if (p != nullptr) (void)hipFree(p);
-    if (e->ids_host != nullptr) (void)hipHostFree(e->ids_host);
     delete e;
 }
 
@@ -1034,19 +1057,19 @@ extern "C" int mynah_hip_encoder_prefill(void *state, mynah_hip_encoder *e, cons
         set_error(error, capacity, "encoder_prefill: with f32 operands there are no f16 token rows to return");
         return -1;
     }
-    // the staging buffer of the previous call may still be in flight
-    MYNAH_TRY(hipStreamSynchronize(st->stream));
-    const size_t tp = e->tpad_max;
-    for (size_t t = 0; t < tokens; ++t) e->ids_host[t] = ids[t];
-    EncParams *hp = reinterpret_cast<EncParams *>(e->ids_host + tp);
-    hp->tokens = (int)tokens;
-    hp->reserved = 0;
-    hp->embed_out = dev_embed_f16;
-    hp->out = dev_out;
-    MYNAH_TRY(hipMemcpyAsync(e->ids, e->ids_host, tokens * sizeof(int), hipMemcpyHostToDevice, st->stream));
-    MYNAH_TRY(hipMemcpyAsync(e->params, hp, sizeof(EncParams), hipMemcpyHostToDevice, st->stream));
-
     const int granule = e->f32 ? kQTile : kTile, tpad = ((int)tokens + granule - 1) / granule * granule;
+    EncFirst first;
+    first.tok = e->f32 ? e->tok32->data : e->tok->data;
+    first.pos = e->f32 ? e->pos32->data : e->pos->data;
+    first.x = e->x;
+    first.gain = e->n1g[0];
+    first.bias = e->n1b[0];
+    first.out_rows = e->f32 ? static_cast<void *>(e->f_nrm) : e->nrm;
+    first.params = e->params;
+    first.call = EncParams{(int)tokens, 0, dev_embed_f16, dev_out};
+    first.rows = tpad;
+    first.width = (int)e->width;
+    if ((e->f32 ? launch_first<ROWS_F32>(st, first, ids, error, capacity) : launch_first<ROWS_F16>(st, first, ids, error, capacity)) != 0) return -1;
     const auto enqueue = e->f32 ? enqueue_prefill_f32 : enqueue_prefill;
     if (!st->graph_mode || e->eager_runs[tpad] == 0) {
         e->eager_runs[tpad] = 1;

@@ -229,3 +229,30 @@ def test_encoder_f32_operands_return_no_f16_rows(pkg, backend, synth):
     with pytest.raises(pkg.BackendError, match="f32 operands"):
         enc.prefill(np.zeros(4, np.int32), dembed.ptr, dout.ptr)
     enc.destroy()
+
+
+@pytest.mark.parametrize("operands_f32", [False, True])
+def test_encoder_calls_queue_up(pkg, backend, orc, synth, nerr, operands_f32):
+    """Calls issued behind each other without a wait keep their own ids, token counts and outputs, to both sides of one launch's
+    worth of ids (512) and up to the longest input; the longest also against the oracle."""
+    _announce("encoder calls behind each other f32=%s" % operands_f32)
+    cfg = dict(synth.encoder_config(layers=1, width=64, heads=1, ffn=128, vocab=300, max_positions=1024), causal=True, ffn_kernel=1, operands_f32=operands_f32)
+    w = synth.encoder_weights_f16(cfg, seed=85, kernel=1)
+    rng = np.random.default_rng(86)
+    calls = [rng.integers(0, 300, size=n).astype(np.int32) for n in (1, 512, 513, 31, 512, 1024, 33)]
+    enc = pkg.Encoder(backend, cfg, w)
+    outs = [backend.alloc(ids.size * 64) for ids in calls]
+    alone = []
+    for ids, out in zip(calls, outs):
+        enc.prefill(ids, 0, out.ptr)
+        alone.append(out.read())
+    for _ in range(3):
+        for ids, out in zip(calls, outs):
+            enc.prefill(ids.copy(), 0, out.ptr)
+    for out, want in zip(outs, alone):
+        assert np.array_equal(out.read().view(np.uint32), want.view(np.uint32))
+    enc.destroy()
+    _, want = orc.encoder_prefill(cfg, _f16_bits(w), calls[5])
+    assert nerr(alone[5].reshape(-1, 64), want) < (1e-5 if operands_f32 else 2e-3)
+    for out in outs:
+        out.free()
