@@ -499,6 +499,7 @@ static void hip_close(void *opaque) {
     if (st->pinned != nullptr) (void)hipHostFree(st->pinned);
     if (st->flush != nullptr) (void)hipFree(st->flush);
     if (st->cross_norm != nullptr) (void)hipFree(st->cross_norm);
+    if (st->conv_parts != nullptr) (void)hipFree(st->conv_parts);
     if (st->pack_staging != nullptr) (void)hipFree(st->pack_staging);
     if (st->attn_partial != nullptr) (void)hipFree(st->attn_partial);
     if (st->attn_counters != nullptr) (void)hipFree(st->attn_counters);

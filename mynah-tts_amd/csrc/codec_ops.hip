@@ -44,6 +44,9 @@ struct ConvArgs {
     const float *alpha = nullptr;       // [snake_channels]
     int snake_channels = 0;
     float *act_out = nullptr;           // null: `out` gets the activated value; else `out` keeps the value before it and this gets the activated one
+    // channel-split tiles only: workgroups that share a tile's channels, and where each leaves its sums ([splits][out_ch][length])
+    int splits = 1;
+    float *parts = nullptr;
 };
 
 // sin(x) in some twenty instructions for |x| < kShortSineLimit (the library routine, which also serves arguments of any
@@ -112,6 +115,7 @@ struct ConvWeights {   // the weight pieces of one row tile, requested kAhead st
     static constexpr int kAhead = 3;
     const uint4 *next;
     size_t skip;       // from the end of a block to the next one this wavefront multiplies
+    int blocks;        // it multiplies
     int tap = 0;       // of the next request (a constant wherever the tap count is one)
     uint4 ring[kAhead][3];
     __device__ __forceinline__ void request(int slot, int taps) {
@@ -120,11 +124,11 @@ struct ConvWeights {   // the weight pieces of one row tile, requested kAhead st
         next += 192;
         if (++tap == taps) {
             tap = 0;
-            next += skip;
+            if (--blocks > 0) next += skip;
         }
     }
-    // (what runs past the last step is requested and not used: the cache pads its copies)
-    __device__ __forceinline__ ConvWeights(const uint4 *first, size_t skip_arg, int taps) : next(first), skip(skip_arg) {
+    // (what runs past the last step is requested and not used: it is what follows the last block, and the cache pads its copies)
+    __device__ __forceinline__ ConvWeights(const uint4 *first, size_t skip_arg, int blocks_arg, int taps) : next(first), skip(skip_arg), blocks(blocks_arg) {
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) request(i, taps);
     }
@@ -266,7 +270,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
     }
     acc[1] = acc[0];
     fetch(0);
-    ConvWeights w(w_arg.data + (size_t)tile * w_arg.blocks * a.kernel * 192 + lane, 0, a.kernel);
+    ConvWeights w(w_arg.data + (size_t)tile * w_arg.blocks * a.kernel * 192 + lane, 0, 1, a.kernel);
     publish(stage_now);
     fetch(min(1, w_arg.blocks - 1));
     const auto stage = [&](int block) {
@@ -422,6 +426,8 @@ __global__ void __launch_bounds__(256, 3) k_conv1d(const float *const in_arg, fl
 // part of LDS; the four partial tiles are added in wavefront order at the end, so the result does not depend on timing.
 // NT: 32-position halves per tile (2, or 1 for the very shortest rows: twice the workgroups).
 // PARTS: positions of the window a lane stages (2 while the window is no longer than 128: the third costs 16 registers).
+// a.splits > 1: that many workgroups share the tile's channels (wavefront w of workgroup s is wavefront 4 s + w of them all), each
+// leaves its sum in a.parts, and k_conv_finish adds them in order and does what is left.
 template <int KF, int NT, int PARTS>
 __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, uint4 *const lds) {
     constexpr int TM = 32, TN = 32 * NT;
@@ -431,13 +437,14 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
     const int win = TN + halo;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint4 *s_in = lds + wave * (6 * win);      // [piece][eight channels][position] of this wavefront
-    const int m0 = blockIdx.y * TM, t0 = blockIdx.x * TN;
+    const int split = (int)blockIdx.x % a.splits, sharing = 4 * a.splits, rank = 4 * split + wave;   // this wavefront among those that share the channels
+    const int m0 = blockIdx.y * TM, t0 = (int)blockIdx.x / a.splits * TN;
     const int half = lane >> 5, col = lane & 31;
 
     floatx16 acc[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[n] = floatx16{0};
-    const int mine = (w_arg.blocks - wave + 3) / 4;   // this wavefront's blocks
+    const int mine = (w_arg.blocks - rank + sharing - 1) / sharing;   // this wavefront's blocks
     if (mine > 0) {
         ConvColumn column[2][PARTS];
         const auto fetch = [&](int i) {
@@ -446,12 +453,12 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
                 if (64 * x < win) {   // (the same for every lane)
 #pragma unroll
                     for (int g = 0; g < 2; ++g)
-                        column[g][x].request(a, 16 * (4 * i + wave) + 8 * g, min(max(t0 - halo + lane + 64 * x, 0), a.length - 1));
+                        column[g][x].request(a, 16 * (sharing * i + rank) + 8 * g, min(max(t0 - halo + lane + 64 * x, 0), a.length - 1));
                 }
         };
         fetch(0);
         const size_t per_block = (size_t)a.kernel * 192;
-        ConvWeights w(w_arg.data + ((size_t)blockIdx.y * w_arg.blocks + wave) * per_block + lane, 3 * per_block, a.kernel);
+        ConvWeights w(w_arg.data + ((size_t)blockIdx.y * w_arg.blocks + rank) * per_block + lane, (size_t)(sharing - 1) * per_block, mine, a.kernel);
         // (no workgroup barrier in the loop: a wavefront stages into its own part of LDS and reads nothing else, and its own
         // LDS accesses complete in the order it issued them -- the four wavefronts walk their channel blocks independently)
         const auto stage = [&](int i) {
@@ -491,8 +498,13 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
         const int e = ((((row >> 3) << 2) | (row & 3)) + 16 * (pos >> 5)) * 64 + ((row >> 2) & 1) * 32 + (pos & 31);
         const float sum = ((s_part[e] + s_part[2048 + e]) + s_part[4096 + e]) + s_part[6144 + e];
         value[j] = 0.0f;
+        if (a.splits > 1) {
+            if (t_ok && m < a.out_ch) a.parts[((size_t)split * a.out_ch + m) * a.length + t] = sum;
+            continue;
+        }
         if (t_ok && m < a.out_ch) value[j] = conv_combine(a, (size_t)m * a.length + t, sum + (a.bias != nullptr ? a.bias[m] : 0.0f));
     }
+    if (a.splits > 1) return;
     if (!a.activate) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -538,6 +550,7 @@ __global__ void __launch_bounds__(256, 2) k_conv1d_split(const float *const in_a
 // different convolutions whose staging and products overlap.  Tap counts 3, 7 and 11 only (the builds with straight-line
 // products); always the build with the fused epilogue (with nothing to add it leaves the product's own bits).
 constexpr int kConvBatchMax = 4;
+constexpr int kConvMaxSplits = 8;
 struct ConvBatchArgs {
     ConvArgs item[kConvBatchMax];
     ConvBlocks weights[kConvBatchMax];
@@ -564,6 +577,24 @@ __global__ void __launch_bounds__(256, 2) k_conv1d_split_batch(const ConvBatchAr
         case 7: conv_split_tile<7, NT, PARTS>(b.item[z], b.weights[z], lds); break;
         default: conv_split_tile<11, NT, PARTS>(b.item[z], b.weights[z], lds); break;
     }
+}
+
+// What is left of convolutions whose channels several workgroups shared: their sums in order, the bias, and the epilogue.
+__global__ void __launch_bounds__(256) k_conv_finish(const ConvBatchArgs b) {
+    const ConvArgs &a = b.item[blockIdx.z];
+    const int t = (int)blockIdx.x * 256 + (int)threadIdx.x, m = (int)blockIdx.y;
+    if (t >= a.length) return;
+    const size_t index = (size_t)m * a.length + t, set = (size_t)a.out_ch * a.length;
+    float part[kConvMaxSplits];
+#pragma unroll
+    for (int s = 0; s < kConvMaxSplits; ++s) part[s] = a.parts[index + (size_t)min(s, a.splits - 1) * set];   // (side by side, under no condition)
+    const bool snake_row = a.activate && m < a.snake_channels;
+    const float al = snake_row ? a.alpha[m] : 0.0f, bias = a.bias != nullptr ? a.bias[m] : 0.0f;
+    float sum = part[0];
+#pragma unroll
+    for (int s = 1; s < kConvMaxSplits; ++s)
+        if (s < a.splits) sum += part[s];
+    conv_emit(a, m, index, conv_combine(a, index, sum + bias), al, 1.0f / (al + 1e-9f));
 }
 
 // ---- a residual block in one launch ---------------------------------------------------------------------------------------
@@ -677,7 +708,7 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
     };
     const size_t w_at = (size_t)min(wm, a.tiles - 1) * a.blocks * KF * 192 + lane;
     fetch(0);
-    ConvWeights w(m.w_in + w_at, 0, KF);
+    ConvWeights w(m.w_in + w_at, 0, 1, KF);
     uint4 *stage_now = lds, *stage_next = lds + 6 * win;
     f32x16 acc[NT];
     start(bias_in, acc);
@@ -705,7 +736,7 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
 #pragma unroll
     for (int i = 0; i < 32 / kRowsAtOnce; ++i) x[i] = m.in[at_out + (size_t)max(min(row0 + kRowsAtOnce * i, rows - 1), 0) * a.length];
     // the inner rows: activated, zero in front of the first position, in pieces to LDS where the second convolution reads them
-    ConvWeights w2(m.w_skip + w_at, 0, KF);
+    ConvWeights w2(m.w_skip + w_at, 0, 1, KF);
     bool large = false;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -959,7 +990,7 @@ int launch_conv_split_p(State *st, const ConvArgs &a, const ConvBlocks &weights,
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_split<KF, NT, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
         raised = true;
     }
-    const dim3 grid((unsigned)((a.length + 32 * NT - 1) / (32 * NT)), (unsigned)((a.out_ch + 31) / 32));
+    const dim3 grid((unsigned)((a.length + 32 * NT - 1) / (32 * NT) * a.splits), (unsigned)((a.out_ch + 31) / 32));
     hipLaunchKernelGGL((k_conv1d_split<KF, NT, PARTS>), grid, dim3(256), conv_split_lds<NT>(a), st->stream, a.in, a.out, weights.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel,
                        a.dilation, weights.tiles, a);
     return hip_check(hipGetLastError(), "conv1d launch", error, capacity);
@@ -980,7 +1011,19 @@ int launch_conv_split_n(State *st, const ConvArgs &a, const ConvBlocks &weights,
     }
 }
 
+int launch_conv_finish(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
+    const ConvArgs &a = b.item[0];
+    hipLaunchKernelGGL(k_conv_finish, dim3((unsigned)((a.length + 255) / 256), (unsigned)a.out_ch, (unsigned)count), dim3(256), 0, st->stream, b);
+    return hip_check(hipGetLastError(), "conv1d finish launch", error, capacity);
+}
+
 int launch_conv_split(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
+    if (a.splits > 1) {
+        ConvBatchArgs b{};
+        b.item[0] = a;
+        const int rc = a.length <= 32 ? launch_conv_split_n<1>(st, a, weights, error, capacity) : launch_conv_split_n<2>(st, a, weights, error, capacity);
+        return rc != 0 ? rc : launch_conv_finish(st, b, 1, error, capacity);
+    }
     const long tiles = (long)((a.out_ch + 31) / 32) * ((a.length + 63) / 64);
     if (tiles < st->cu_count) return launch_conv_split_n<1>(st, a, weights, error, capacity);
     return launch_conv_split_n<2>(st, a, weights, error, capacity);
@@ -1013,7 +1056,7 @@ int launch_conv_split_batch_p(State *st, const ConvBatchArgs &b, int count, char
         raised = true;
     }
     const ConvArgs &a = b.item[0];
-    const dim3 grid((unsigned)((a.length + 32 * NT - 1) / (32 * NT)), (unsigned)((a.out_ch + 31) / 32), (unsigned)count);
+    const dim3 grid((unsigned)((a.length + 32 * NT - 1) / (32 * NT) * a.splits), (unsigned)((a.out_ch + 31) / 32), (unsigned)count);
     hipLaunchKernelGGL((k_conv1d_split_batch<NT, PARTS>), grid, dim3(256), lds, st->stream, b);
     return hip_check(hipGetLastError(), "conv1d batch launch", error, capacity);
 }
@@ -1033,8 +1076,34 @@ int mynah::launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_
     return hip_check(hipGetLastError(), "weight packing launch", error, capacity);
 }
 
+// few output channels: one row of wavefronts, wider in time; too few large tiles to fill the chip and enough input channels to
+// share out (more than one block for each of four wavefronts): small tiles with the channels split over the wavefronts.  The two
+// add in different orders, so the choice is the shape's alone, for single, batched and fused launches alike.  216 channels: the two
+// meet at 4096 positions (three members, 72 us either way), and the large tiles' launch has no more wavefronts than it needs;
+// 108 channels: the small tiles' three members at 1280 positions take 14 us, a fused block of large tiles 41.
+static bool conv_takes_split(const State *st, int in_channels, int out_channels, int length) {
+    const long tiles = out_channels <= 32 ? (long)((length + 255) / 256) : (long)((out_channels + 63) / 64) * ((length + 127) / 128);
+    return in_channels > 64 && tiles < (in_channels > kResMaxChannels ? (long)st->cu_count / 4 : (long)st->cu_count * 3 / 8);
+}
+
+// How many workgroups share a channel-split tile.  A few short rows leave most of the chip idle while each tile's workgroup pulls the
+// weights of all channels through one CU (some 40 GB/s: 0.9 MB with 432 channels and eleven taps); so as many as bring a wavefront's
+// blocks of channels down while three members' workgroups are two to a CU at most.  The sums' order follows, so this is the shape's
+// alone, too.  Taps 3 / 7 / 11 side by side: 432 channels x 40 24.6 -> 11.2 us, 216 x 320 18.9 -> 12.4, and 4.0 for k_conv_finish; 108 x 1280
+// stays with one (14.2 us, 12.4 + 4.2 shared), its seven blocks are few enough.  Twice kConvSharedTiles: nothing measurable.
+constexpr int kConvSharedTiles = 160;
+static int conv_splits(int in_channels, int out_channels, int length) {
+    const long tiles = (long)((out_channels + 31) / 32) * ((length + 63) / 64), blocks = (in_channels + 15) / 16;
+    if (in_channels <= kResMaxChannels) return 1;
+    for (long each = 1; 4 * each < blocks; ++each) {
+        const long splits = (blocks + 4 * each - 1) / (4 * each);
+        if (splits <= kConvMaxSplits && tiles * splits <= kConvSharedTiles) return (int)splits;
+    }
+    return 1;
+}
+
 // Checks one convolution's arguments, caches its weights and fills the kernels' argument block.
-static int conv1d_prepare(State *st, const float *dev_input, float *dev_output, int in_channels, int out_channels, int length,
+static int conv1d_prepare(State *st, int member, const float *dev_input, float *dev_output, int in_channels, int out_channels, int length,
                           int kernel, int dilation, const float *weight, const float *bias, const mynah_hip_conv1d_extra *extra,
                           ConvArgs *out_args, ConvBlocks *out_weights, char *error, size_t capacity) {
     if (st == nullptr || dev_input == nullptr || dev_output == nullptr || weight == nullptr || in_channels <= 0 || out_channels <= 0 ||
@@ -1069,19 +1138,19 @@ static int conv1d_prepare(State *st, const float *dev_input, float *dev_output, 
         a.act_out = extra->dev_activated;
         if (a.activate && a.snake_channels != 0 && cached_vector(st, extra->snake_alpha, extra->snake_channels, &a.alpha, error, capacity) != 0) return -1;
     }
+    if (in_channels > kResMaxChannels) {   // (whatever the length: a call that is captured then finds the memory that an earlier one with its weights allocated)
+        constexpr size_t floats = (size_t)kConvSharedTiles * 32 * 64;   // of one convolution
+        if (st->conv_parts == nullptr &&
+            hip_check(hipMalloc(reinterpret_cast<void **>(&st->conv_parts), kConvBatchMax * floats * sizeof(float)), "conv1d workspace", error, capacity) != 0)
+            return -1;
+        if (conv_takes_split(st, in_channels, out_channels, length)) {
+            a.splits = conv_splits(in_channels, out_channels, length);
+            a.parts = st->conv_parts + (size_t)member * floats;
+        }
+    }
     *out_args = a;
     *out_weights = weights;
     return 0;
-}
-
-// few output channels: one row of wavefronts, wider in time; too few large tiles to fill the chip and enough input channels to
-// share out (more than one block for each of four wavefronts): small tiles with the channels split over the wavefronts.  The two
-// add in different orders, so the choice is the shape's alone, for single, batched and fused launches alike.  216 channels: the two
-// meet at 4096 positions (three members, 72 us either way), and the large tiles' launch has no more wavefronts than it needs;
-// 108 channels: the small tiles' three members at 1280 positions take 14 us, a fused block of large tiles 41.
-static bool conv_takes_split(const State *st, int in_channels, int out_channels, int length) {
-    const long tiles = out_channels <= 32 ? (long)((length + 255) / 256) : (long)((out_channels + 63) / 64) * ((length + 127) / 128);
-    return in_channels > 64 && tiles < (in_channels > kResMaxChannels ? (long)st->cu_count / 4 : (long)st->cu_count * 3 / 8);
 }
 
 static int conv1d_launch(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
@@ -1096,7 +1165,7 @@ static int conv1d_entry(void *state, const float *dev_input, float *dev_output, 
     State *st = enter_state(state);
     ConvArgs a;
     ConvBlocks weights;
-    if (conv1d_prepare(st, dev_input, dev_output, in_channels, out_channels, length, kernel, dilation, weight, bias, extra, &a, &weights, error, capacity) != 0)
+    if (conv1d_prepare(st, 0, dev_input, dev_output, in_channels, out_channels, length, kernel, dilation, weight, bias, extra, &a, &weights, error, capacity) != 0)
         return -1;
     return conv1d_launch(st, a, weights, error, capacity);
 }
@@ -1127,7 +1196,7 @@ extern "C" int mynah_hip_conv1d_fused_batch(void *state, const mynah_hip_conv1d_
     bool side_by_side = true;
     for (size_t i = 0; i < count; ++i) {
         const mynah_hip_conv1d_item &it = items[i];
-        if (conv1d_prepare(st, it.dev_input, it.dev_output, in_channels, out_channels, length, it.kernel, it.dilation, it.weight, it.bias, &it.extra,
+        if (conv1d_prepare(st, (int)i, it.dev_input, it.dev_output, in_channels, out_channels, length, it.kernel, it.dilation, it.weight, it.bias, &it.extra,
                            &b.item[i], &b.weights[i], error, capacity) != 0)
             return -1;
         side_by_side = side_by_side && (it.kernel == 3 || it.kernel == 7 || it.kernel == 11);
@@ -1156,6 +1225,10 @@ extern "C" int mynah_hip_conv1d_fused_batch(void *state, const mynah_hip_conv1d_
     if (conv_takes_split(st, in_channels, out_channels, length)) {
         // (the tile's width does not enter a value's arithmetic -- same channel blocks per wavefront, same order -- so the
         // members may take the wider tile, half the weight traffic per product, as soon as all of them together fill the chip)
+        if (b.item[0].splits > 1) {
+            const int rc = length <= 32 ? launch_conv_split_batch<1>(st, b, (int)count, error, capacity) : launch_conv_split_batch<2>(st, b, (int)count, error, capacity);
+            return rc != 0 ? rc : launch_conv_finish(st, b, (int)count, error, capacity);
+        }
         const long tiles = (long)((out_channels + 31) / 32) * ((length + 63) / 64);
         if (tiles * (long)count < st->cu_count) return launch_conv_split_batch<1>(st, b, (int)count, error, capacity);
         return launch_conv_split_batch<2>(st, b, (int)count, error, capacity);

@@ -182,6 +182,8 @@ struct State {
     // normalised encoder memory of mynah_hip_cross_kv_dev (grown on demand; an outgrown one waits in pending_free)
     float *cross_norm = nullptr;
     size_t cross_norm_floats = 0;
+    // sums of the workgroups that share a convolution's channels (codec_ops.hip)
+    float *conv_parts = nullptr;
     // cache-flush buffer
     void *flush = nullptr;
     size_t flush_bytes = 0;

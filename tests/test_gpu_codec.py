@@ -236,6 +236,35 @@ def test_conv_batch_members_and_refusals(pkg, backend):
         d.free()
 
 
+# channels shared between workgroups (more than 128, few short rows): one position, either side of the narrow and the wide tile, the last
+# shape that shares and the first that does not, a last workgroup without a block of its own, any tap count
+@pytest.mark.parametrize("C,O,L", [(432, 432, 1), (432, 400, 32), (432, 432, 33), (129, 70, 64), (216, 216, 1408), (216, 216, 1409), (600, 30, 65), (144, 31, 130)])
+def test_channels_shared_between_workgroups(backend, orc, nerr, C, O, L):
+    """Against the oracle, single calls and members side by side (the same bits), with everything the epilogue can do."""
+    _announce("shared channels %d -> %d x %d" % (C, O, L))
+    rng = np.random.default_rng(C + O + L)
+    x, r = rng.standard_normal((C, L)).astype(np.float32), rng.standard_normal((O, L)).astype(np.float32)
+    alpha = (np.abs(rng.standard_normal(O // 2)) + 0.1).astype(np.float32)
+    din, dres = backend.alloc(C * L).write(x), backend.alloc(O * L).write(r)
+    taps = (3, 7, 11, 5)
+    ws = [(rng.standard_normal((O, C, k)) / np.sqrt(C * k)).astype(np.float32) for k in taps]
+    bs = [rng.standard_normal(O).astype(np.float32) for _ in taps]
+    bufs = [backend.alloc(O * L) for _ in range(8)]
+    extras = [dict(residual=dres.ptr, scale=0.5), dict(alpha=alpha, activated=bufs[7].ptr), dict(alpha=alpha), dict()]
+    plain = [orc.conv1d_causal(x, w, b, 1 + 2 * i) for i, (w, b) in enumerate(zip(ws, bs))]
+    want = [(plain[0] + r) * np.float32(0.5), plain[1], orc.snake(plain[2], alpha, O // 2), plain[3]]
+    for i, k in enumerate(taps):
+        backend.conv1d_fused(din.ptr, bufs[i].ptr, C, O, L, k, 1 + 2 * i, ws[i], bs[i], **extras[i])
+        assert nerr(bufs[i].read().reshape(O, L), want[i]) < 1e-5, k
+    assert nerr(bufs[7].read().reshape(O, L), orc.snake(plain[1], alpha, O // 2)) < 1e-5
+    backend.conv1d_fused_batch([dict(din=din.ptr, dout=bufs[4 + i].ptr, kernel=taps[i], dilation=1 + 2 * i, weight=ws[i], bias=bs[i], **extras[i])
+                                for i in range(3)], C, O, L)
+    for a, b in zip(bufs[:3], bufs[4:7]):
+        assert np.array_equal(a.read().view(np.uint32), b.read().view(np.uint32))
+    for d in bufs + [din, dres]:
+        d.free()
+
+
 def test_conv_batch_on_the_wider_split_tiles(backend):
     """432 channels x 512 positions: alone a convolution takes the channel-split kernel's 32 x 32 tiles, three side by side
     its 32 x 64 tiles.  The tile's width is not part of a value's arithmetic: every member keeps its single call's bits."""
