@@ -757,7 +757,7 @@ __device__ __forceinline__ void finish_activations(const PrologueParams &p, cons
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// One wavefront stages one stream (matvec builds for more than two streams with int8 / int4 weights).  Lane l holds, for
+// One wavefront stages one stream (matvec builds for more than two streams).  Lane l holds, for
 // each of the four "virtual wavefronts" v of the 256-thread scheme above and each i < NVT, the float4 f = 64 v + l + 256 i:
 // what thread 64 v + l of that scheme holds, at xr[v * NVT + i].  Every sum is formed per virtual wavefront in that
 // thread's order, reduced over the lanes by the same butterfly and combined ((a0 + a1) + a2) + a3 as block_reduce does, so
@@ -789,12 +789,11 @@ __device__ __forceinline__ void load_stream_row(const PrologueParams &p, const f
     (void)live;
 }
 
-// Second half for one wavefront and its stream: LayerNorm (optional) -> quantisation -> the stream's bytes in LDS.  The caller
+// Second half for one wavefront and its stream: LayerNorm (optional) -> quantisation (int8 / int4 weights) -> the stream's bytes in LDS.  The caller
 // puts one workgroup barrier behind it.  live == false (a place of the batch tile without a stream): zeros are staged.
 template <int QT, int NVT>
 __device__ __forceinline__ void finish_stream_row(const PrologueParams &p, const int stream, const bool live, const int lane, float4 (&xr)[4 * NVT],
                                                   const float4 (&gv)[4 * NVT], const float4 (&bv)[4 * NVT], unsigned char *smem, float *s_sx) {
-    static_assert(kQuantised<QT>, "only the quantising builds stage a stream per wavefront");
     const int nf4 = p.k >> 2;
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -855,6 +854,16 @@ __device__ __forceinline__ void finish_stream_row(const PrologueParams &p, const
                 if (p.ln_out != nullptr && first && f < nf4) reinterpret_cast<float4 *>(p.ln_out)[f] = y;
                 if (p.ln_out_slots != nullptr && blockIdx.x == 0 && live && f < nf4) reinterpret_cast<float4 *>(p.ln_out_slots->output[stream])[f] = y;
             }
+    }
+    if constexpr (!kQuantised<QT>) {
+        float4 *const rows = reinterpret_cast<float4 *>(smem) + (size_t)stream * nf4;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int i = 0; i < NVT; ++i)
+                if (64 * v + lane + kThreads * i < nf4) rows[64 * v + lane + kThreads * i] = xr[v * NVT + i];
+        if (lane == 0) s_sx[stream] = 1.0f;
+        return;
     }
     float amax = 0.0f;
 #pragma unroll

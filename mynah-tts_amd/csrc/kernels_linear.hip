@@ -53,24 +53,26 @@ __device__ __forceinline__ float *stream_out(const LinearArgs &a, int b) {
 // GELU epilogue (the step's FFN-up projection).
 enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2 };
 
-// More than two streams with int8 / int4 weights: one wavefront stages one stream (load_stream_row / finish_stream_row,
+// More than two streams: one wavefront stages one stream (load_stream_row / finish_stream_row,
 // device_common.h) -- staging every stream's activations is what such a launch spends most of its time on, every workgroup
 // has to do all of it, and a wavefront that owns a whole row needs no barrier and no exchange to normalise and quantise it.
 // The workgroup has as many wavefronts as the batch tile has streams (at least four); the products then go to sets of four
 // wavefronts, each set doing the matvec as the four wavefronts of a small-batch workgroup would for four of the streams.
-// For f16 / f32 weights staging is a LayerNorm or a copy by the 256 threads together.
-template <int BT, int QT>
-constexpr bool kWaveStaging = BT > kConsumerFoldMaxBatch && kQuantised<QT>;
-template <int BT, int QT>
-constexpr int kLinearThreads = kWaveStaging<BT, QT> ? 64 * (BT > 4 ? BT : 4) : kThreads;
+// (f16 / f32 weights: the same without the quantisation, same bits as by the 256 threads together; as one tile of eight staged by those,
+// output projection / up / down 5.2 / 8.2 / 7.6 us, now 5.1 / 5.7 / 7.0 beside a second lane; sixteen f16 streams 880 -> 807 us a step, four
+// 504 -> 460.)
+template <int BT>
+constexpr bool kWaveStaging = BT > kConsumerFoldMaxBatch;
+template <int BT>
+constexpr int kLinearThreads = kWaveStaging<BT> ? 64 * (BT > 4 ? BT : 4) : kThreads;
 
 // The builds whose leading arguments are repacked (see the kernel): specialised ones, one or two streams.
 template <int BT, int SPEC>
 constexpr bool kPackedLead = BT <= 2 && SPEC != SPEC_ANY;
 // The same for more streams, when the rows of a launch lie at a fixed stride (the step's workspaces do): the specialised
 // builds that stage a stream per wavefront take two row pointers and two strides instead of sixteen row pointers.
-template <int BT, int QT, int SPEC>
-constexpr bool kStridedLead = kWaveStaging<BT, QT> && SPEC != SPEC_ANY;
+template <int BT, int SPEC>
+constexpr bool kStridedLead = kWaveStaging<BT> && SPEC != SPEC_ANY;
 
 // n:20 | rows per workgroup:12 | streams:4 | input stride / 4:14 | output stride / 4:14 (strides in floats)
 struct StridedShape {
@@ -125,7 +127,7 @@ __device__ __forceinline__ LeadShape unpack_lead(const unsigned long long v) {
 }
 
 template <int QT, int BT, int NVT, int KFIX, int SPEC>
-__global__ void __launch_bounds__((kLinearThreads<BT, QT>))
+__global__ void __launch_bounds__(kLinearThreads<BT>)
 k_linear(const float *const in0, const float *const fold_partial, const float *const fold_partial_ml, const StepSlots *const fold_slots,
          const void *const w, const float *const scales, float *const out0, const int n, const int batch, const LinearArgs a_arg,
          const int rows_per_wg_arg, const int lg_arg) {
@@ -135,7 +137,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
     // (Only for one or two streams: with more, the rows of a.in and a.out are picked by a run-time index, and a structure that
     // has been written to is then kept in scratch memory -- the eight-stream matvecs took 20 us instead of 4.5.)
     static_assert(64 + sizeof(LinearArgs) > 0x100 + 4, "the warmed lines lie inside the kernel arguments");
-    constexpr bool kStrided = kStridedLead<BT, QT, SPEC>;
+    constexpr bool kStrided = kStridedLead<BT, SPEC>;
     WarmArguments warm{0u, 0u, 0u, 0u};
     if constexpr (BT <= 2 || kStrided) warm = warm_kernel_arguments<4>();
     LinearArgs a = a_arg;
@@ -191,7 +193,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
     // a one-stream build is launched for exactly one stream (launch_linear_b): its first request then depends on no argument
     // that comes out of memory (n and batch are the fifteenth and sixteenth dword, one past what is in registers at start)
     if constexpr (BT == 1) a.batch = 1;
-    constexpr bool kWaves = kWaveStaging<BT, QT>;   // a wavefront per stream (see above); otherwise the 256 threads stage every stream together
+    constexpr bool kWaves = kWaveStaging<BT>;   // a wavefront per stream (see above); otherwise the 256 threads stage every stream together
     // The kernel arguments that the first requests are formed from, fetched here in one go: left to the compiler each is
     // fetched where it is first used, with a wait of its own, and three such round trips stood in a row in front of the
     // first request for an activation row.
@@ -209,7 +211,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
     // second four take the same rows for the upper half of the streams: PB streams per wavefront, from stream_base on.  Every
     // wavefront works, so no request stands under a condition.
     constexpr int PB = (kWaves && BT > 4) ? BT / 2 : BT;
-    static_assert(!kWaves || kLinearThreads<BT, QT> == kThreads * (BT / PB), "one set of four wavefronts per PB streams");
+    static_assert(!kWaves || kLinearThreads<BT> == kThreads * (BT / PB), "one set of four wavefronts per PB streams");
     // the arguments a specialised build does not look at
     const float *const arg_bias = SPEC != SPEC_ANY ? nullptr : a.bias;
     int8_t *const arg_probe_qx = SPEC != SPEC_ANY ? nullptr : a.probe_qx;
@@ -615,7 +617,7 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
     if (passes < 1) passes = 1;
     // strided builds take more streams than their tile holds as groups of BT side by side (the grid's second dimension);
     // with twice the rows per workgroup when the groups together would otherwise be more workgroups than the chip has CUs
-    const int groups = kStridedLead<BT, QT, SPEC> ? (a.batch + BT - 1) / BT : 1;
+    const int groups = kStridedLead<BT, SPEC> ? (a.batch + BT - 1) / BT : 1;
     if (groups > 1 && (long)((a.n + rows_per_wg_pass * passes - 1) / (rows_per_wg_pass * passes)) * groups > st->cu_count) passes *= 2;
     const int rows_per_wg = rows_per_wg_pass * passes;
     const int grid = (a.n + rows_per_wg - 1) / rows_per_wg;
@@ -626,7 +628,7 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
                                       hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));
         raised = true;
     }
-    if constexpr (kStridedLead<BT, QT, SPEC>) {
+    if constexpr (kStridedLead<BT, SPEC>) {
         StridedShape shape{};
         shape.n = a.n; shape.rows_per_wg = rows_per_wg; shape.batch = a.batch;
         if (!rows_strided(a, &shape.in_stride, &shape.out_stride) || !strided_fits(shape)) {   // launch_linear_q sends such launches to the general build; this is the backstop
@@ -634,7 +636,7 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
             return -1;
         }
         const StepSlots *const packed = reinterpret_cast<const StepSlots *>(pack_strided(shape));
-        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, SPEC>), dim3(grid, groups), dim3(kLinearThreads<BT, QT>), lds, st->stream, a.in[0],
+        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, SPEC>), dim3(grid, groups), dim3(kLinearThreads<BT>), lds, st->stream, a.in[0],
                            SPEC == SPEC_UP ? a.ln_gain : nullptr, SPEC == SPEC_UP ? a.ln_bias : nullptr, packed, a.w, a.scales, a.out[0], a.n, a.batch, a,
                            rows_per_wg, lg);
     } else if constexpr (kPackedLead<BT, SPEC>) {
@@ -654,10 +656,10 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
         const float *lead0 = a.in[0], *lead1 = nullptr, *lead2 = nullptr;
         if (SPEC == SPEC_UP) { lead1 = a.ln_gain; lead2 = a.ln_bias; }
         else if (folding) { lead0 = reinterpret_cast<const float *>(a.fold_slots); lead1 = a.fold_partial; lead2 = a.fold_partial_ml; }
-        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, SPEC>), dim3(grid), dim3(kLinearThreads<BT, QT>), lds, st->stream, lead0, lead1, lead2, packed,
+        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, SPEC>), dim3(grid), dim3(kLinearThreads<BT>), lds, st->stream, lead0, lead1, lead2, packed,
                            a.w, a.scales, a.out[0], a.n, a.batch, a, rows_per_wg, lg);
     } else {
-        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, SPEC>), dim3(grid), dim3(kLinearThreads<BT, QT>), lds, st->stream, a.in[0], a.fold_partial,
+        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, SPEC>), dim3(grid), dim3(kLinearThreads<BT>), lds, st->stream, a.in[0], a.fold_partial,
                            a.fold_partial_ml, a.fold_slots, a.w, a.scales, a.out[0], a.n, a.batch, a, rows_per_wg, lg);
     }
     return hip_check(hipGetLastError(), "linear launch", error, capacity);
@@ -668,13 +670,13 @@ int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity
     if (a.batch <= 1) return launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
     if (a.batch == 2) return launch_linear_t<QT, 2, NVT, KFIX, SPEC>(st, a, error, capacity);
     if (a.batch <= 4) return launch_linear_t<QT, 4, NVT, KFIX, SPEC>(st, a, error, capacity);
-    // five to eight streams, rows at a fixed stride, int8 / int4 weights, residual epilogue (the output projections and the
+    // five to eight streams, rows at a fixed stride, residual epilogue (the output projections and the
     // FFN-down product): two groups of four in one launch -- what a workgroup stages, every stream of its tile, halves, and a
     // stream's bits do not depend on the tile it runs in.  (Measured with eight ragged streams: step 497 -> 483 us; the FFN-up
     // product the same way, whose LayerNorm prologue each group then runs for its four rows, 497 us with twice the rows per
     // workgroup and 486 us with twice the workgroups; with the second pass's operands requested ahead as below, 476 against 477 us:
     // it keeps the tile of eight.)
-    if (kStridedLead<4, QT, SPEC> && SPEC == SPEC_RESIDUAL && stream_groups_enabled()) return launch_linear_t<QT, 4, NVT, KFIX, SPEC>(st, a, error, capacity);
+    if (kStridedLead<4, SPEC> && SPEC == SPEC_RESIDUAL && stream_groups_enabled()) return launch_linear_t<QT, 4, NVT, KFIX, SPEC>(st, a, error, capacity);
     return launch_linear_t<QT, 8, NVT, KFIX, SPEC>(st, a, error, capacity);
 }
 
@@ -691,10 +693,10 @@ int launch_linear_q(State *st, const LinearArgs &a, char *error, size_t capacity
         fit.is_self = a.fold_is_self; fit.stream0 = a.fold_stream0; fit.heads = a.fold_heads; fit.max_units = a.fold_max_units; fit.head_width = a.fold_head_width;
     }
     bool packs = lead_fits(fit);
-    if (a.batch > 2) {   // more streams: the specialised builds of quantised weights take rows at a fixed stride
+    if (a.batch > 2) {   // more streams: the specialised builds take rows at a fixed stride
         StridedShape strided{};
         strided.n = a.n; strided.batch = a.batch; strided.rows_per_wg = 2048;
-        packs = !kQuantised<QT> || (rows_strided(a, &strided.in_stride, &strided.out_stride) && strided_fits(strided));
+        packs = rows_strided(a, &strided.in_stride, &strided.out_stride) && strided_fits(strided);
     }
     const bool residual = plain && packs && a.epilogue == EPI_RESIDUAL && a.ln_gain == nullptr;
     const bool up = plain && packs && a.epilogue == EPI_GELU && a.ln_gain != nullptr && a.fold_partial == nullptr;

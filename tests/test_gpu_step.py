@@ -99,6 +99,29 @@ def test_one_block_batch1_kv256(pkg, backend, orc, synth, nerr, qtype_name):
     backend.set_quant(0)
 
 
+@pytest.mark.parametrize("qtype_name", ["f32", "f16"])
+@pytest.mark.parametrize("batch", [3, 5, 7])
+def test_unquantised_tiles_with_empty_places(pkg, backend, orc, synth, nerr, qtype_name, batch):
+    """f16 / f32 weights, stream counts that leave a place of a tile or of its second group empty: against the oracle, and every stream
+    bit-identical to the same stream run alone (one stream is staged by the whole workgroup, more by a wavefront each)."""
+    _announce("empty places b=%d %s" % (batch, qtype_name))
+    lengths, mems = [5, 64, 0, 129, 63, 2, 190][:batch], [7, 64, 3, 32, 65, 1, 27][:batch]
+    cfg = synth.decoder_config(layers=1, capacity=200)
+    weights = synth.decoder_weights(cfg, seed=4)
+    streams = synth.decoder_streams(cfg, lengths, mems, seed=5)
+    backend.set_quant(QT[qtype_name])
+    h = Harness(pkg, backend, cfg, weights, streams)
+    want, _, _ = _oracle_step(orc, cfg, weights, streams, QT[qtype_name])
+    got = h.step()
+    h.close()
+    for b in range(batch):
+        assert nerr(got[b], want[b]) < TOL[qtype_name], "stream %d" % b
+        solo = Harness(pkg, backend, cfg, weights, [streams[b]])
+        assert np.array_equal(solo.step()[0].view(np.uint32), got[b].view(np.uint32)), "stream %d" % b
+        solo.close()
+    backend.set_quant(0)
+
+
 @pytest.mark.parametrize("qtype_name", ["f32", "int8", "int4", "f16"])
 def test_two_layers_ragged_batch8_and_bit_identity(pkg, backend, orc, synth, nerr, qtype_name):
     """Ragged B=8 (incl. an empty cache and chunk-edge lengths) against the oracle, eager and graph replay,
