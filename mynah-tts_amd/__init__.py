@@ -236,13 +236,12 @@ class Backend:
         self._keep = []   # host arrays whose addresses key the device weight cache
         self._kept = {}   # id -> (array, address) of those that were handed in as they are kept
         self._res_layers = {}   # id of a residual layer's blocks -> (blocks, what they hold, descriptor)
-        self._error = C.create_string_buffer(512)   # one thread at a time uses a backend
         if quant is not None or arith is not None:
             self.set_quant(F32 if quant is None else quant, ARITH_STRICT if arith is None else arith)
 
     # -- plumbing
     def _call(self, name, *args):
-        err = self._error
+        err = C.create_string_buffer(512)   # each call's own: threads may share a backend
         rc = getattr(self.lib, name)(self.state, *args, err, 512)
         if rc != 0:
             raise BackendError("%s: %s" % (name, err.value.decode()))
@@ -435,6 +434,8 @@ class Backend:
                     s.alpha_in, s.weight_in, s.bias_in = self.address(a_in), self.address(w_in), self.address(b_in)
                     s.alpha_skip, s.weight_skip, s.bias_skip = self.address(a_skip), self.address(w_skip), self.address(b_skip)
                     s.kernel_in, s.kernel_skip, s.dilation = w_in.shape[2], w_skip.shape[2], dilation
+            if len(self._res_layers) >= 64:   # a codec has five; lists made anew for each call are not collected
+                self._res_layers.clear()
             desc = self._res_layers[id(blocks)] = (blocks, parts, arr)   # (held: an id stays one object's)
         self._call("mynah_hip_res_layer_dev", desc[2], len(blocks), len(blocks[0]), din, dout, channels, length, self.address(then_alpha),
                    (_vp * len(work))(*work))
