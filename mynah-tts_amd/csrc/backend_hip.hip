@@ -128,7 +128,7 @@ int ensure_attention_workspace(State *st, size_t batch, size_t heads, size_t hea
 }
 
 // ------------------------------------------------------------------------------------------ weight cache
-// Keyed by (host address, byte size, conversion), on the contract that the host memory is an
+// Keyed by (host address, byte size, conversion, and the row length where the converted form depends on it), on the contract that the host memory is an
 // immutable model tensor that outlives the backend (gpu/cuda/backend_cuda.cu:193-219).
 int cached_matrix(State *st, const float *host, size_t n, size_t k, int want_qtype, const CachedWeight **out,
                   char *error, size_t capacity) {
@@ -140,7 +140,8 @@ int cached_matrix(State *st, const float *host, size_t n, size_t k, int want_qty
     if (qtype == MYNAH_HIP_INT4 && (k % 32u) != 0) qtype = MYNAH_HIP_F32;   // src/qmat.c:630
     if (qtype != MYNAH_HIP_F32 && k > kQuantMaxK) qtype = MYNAH_HIP_F32;    // src/qmat.c:33,774
     if (qtype != MYNAH_HIP_F32 && !linear_fast_supported(qtype, n, k)) qtype = MYNAH_HIP_F32;
-    const WeightKey key{host, n * k * sizeof(float), 1 + qtype * 2 + (qtype == MYNAH_HIP_INT8 || qtype == MYNAH_HIP_INT4 ? st->arith : 0)};
+    const WeightKey key{host, n * k * sizeof(float), 1 + qtype * 2 + (qtype == MYNAH_HIP_INT8 || qtype == MYNAH_HIP_INT4 ? st->arith : 0),
+                        qtype == MYNAH_HIP_INT8 ? k : 0};
     std::lock_guard<std::mutex> lock(st->mu);
     auto it = st->weights.find(key);
     if (it != st->weights.end()) {
@@ -248,7 +249,7 @@ int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch
     const size_t tiles = (out_ch + 31) / 32, blocks = (in_ch + 15) / 16;
     out->tiles = (int)tiles;
     out->blocks = (int)blocks;
-    const WeightKey key{host, out_ch * in_ch * kernel * sizeof(float), (int)(64 + kernel + 32 * in_ch)};
+    const WeightKey key{host, out_ch * in_ch * kernel * sizeof(float), (int)(64 + kernel), in_ch};
     std::lock_guard<std::mutex> lock(st->mu);
     auto it = st->weights.find(key);
     if (it != st->weights.end()) {
@@ -281,7 +282,7 @@ int cached_split_weight(State *st, const float *host, size_t n, size_t channels,
         return -1;
     }
     const size_t count = n * channels * taps;
-    const WeightKey key{host, count * sizeof(float), -(int)taps};
+    const WeightKey key{host, count * sizeof(float), -(int)taps, channels};
     std::lock_guard<std::mutex> lock(st->mu);
     auto it = st->weights.find(key);
     if (it != st->weights.end()) {
@@ -314,7 +315,7 @@ int cached_vector(State *st, const float *host, size_t n, const float **dev, cha
         set_error(error, capacity, "invalid vector size");
         return -1;
     }
-    const WeightKey key{host, bytes, 0};
+    const WeightKey key{host, bytes, 0, 0};
     std::lock_guard<std::mutex> lock(st->mu);
     auto it = st->weights.find(key);
     if (it != st->weights.end()) {
@@ -337,7 +338,7 @@ int cached_snake_pairs(State *st, const float *host, size_t n, const float **dev
         set_error(error, capacity, "invalid snake alphas");
         return -1;
     }
-    const WeightKey key{host, n * sizeof(float), -100};
+    const WeightKey key{host, n * sizeof(float), -100, 0};
     std::lock_guard<std::mutex> lock(st->mu);
     auto it = st->weights.find(key);
     if (it == st->weights.end()) {

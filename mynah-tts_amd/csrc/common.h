@@ -78,12 +78,14 @@ struct PackedWeight {
 struct WeightKey {
     const void *host;
     size_t bytes;
-    int kind;   // 0 plain f32 vector/matrix, 1 + qtype*2 + arith for converted matrices, 64 + kernel + 32 * in_ch for conv1d chunks, -taps for split products, -100 for snake pairs
-    bool operator==(const WeightKey &o) const { return host == o.host && bytes == o.bytes && kind == o.kind; }
+    int kind;   // 0 plain f32 vector/matrix, 1 + qtype*2 + arith for converted matrices, 64 + kernel for conv1d blocks, -taps for split products, -100 for snake pairs
+    size_t row; // what else the stored form depends on: the row length of an int8 matrix (a scale per row), the input channels of conv1d blocks and
+                // split products (their order); 0 for the forms that are a tensor's values one after the other whatever its shape
+    bool operator==(const WeightKey &o) const { return host == o.host && bytes == o.bytes && kind == o.kind && row == o.row; }
 };
 struct WeightKeyHash {
     size_t operator()(const WeightKey &k) const {
-        return std::hash<const void *>()(k.host) ^ (k.bytes * 0x9e3779b97f4a7c15ull) ^ ((size_t)k.kind << 56);
+        return std::hash<const void *>()(k.host) ^ ((k.bytes + (k.row << 20)) * 0x9e3779b97f4a7c15ull) ^ ((size_t)k.kind << 56);
     }
 };
 

@@ -49,3 +49,38 @@ def test_encoder_f32_tiles(backend, pkg, orc, synth, nerr, kernel, tokens):
     packed.update({k: w.get(k) for k in ("norm1_g", "norm1_b", "norm2_g", "norm2_b", "norm_out_g", "norm_out_b")})
     _, want = orc.encoder_prefill(cfg, packed, ids)
     assert nerr(got, want) < 1e-5
+
+
+def test_one_buffer_under_two_shapes(backend, pkg, orc):
+    """A weight's stored form may depend on its shape (the order of a split product's blocks and of a convolution's, the scales of int8
+    rows): the same memory used under two shapes of equal size gives each its own products."""
+    print("[gpu-case] one weight buffer, two shapes", flush=True)
+    rng = np.random.default_rng(5)
+    shared = backend.keep(rng.standard_normal(128 * 64).astype(np.float32))
+    rows = 40
+    backend.set_quant(pkg.F32)
+    for width, xw in ((128, 32), (64, 64)):
+        gain = backend.keep(np.ones(width, np.float32))
+        memory = rng.standard_normal((rows, width)).astype(np.float32)
+        dmem, dk, dv = backend.alloc(rows * width).write(memory), backend.alloc(rows * xw), backend.alloc(rows * xw)
+        backend.cross_kv_dev(dmem.ptr, rows, width, [gain], None, [shared], xw, dk.ptr, dv.ptr)
+        got = np.concatenate([dk.read().reshape(rows, xw), dv.read().reshape(rows, xw)], axis=1)
+        want = np.stack([orc.layernorm(r, gain, None) for r in memory]).astype(np.float64) @ shared.reshape(2 * xw, width).astype(np.float64).T
+        assert np.linalg.norm(got - want) < 2e-6 * np.linalg.norm(want), (width, xw)
+        for d in (dmem, dk, dv):
+            d.free()
+    for out_ch, in_ch in ((64, 128), (128, 64)):
+        x, w = rng.standard_normal((in_ch, 70)).astype(np.float32), shared.reshape(out_ch, in_ch, 1)
+        dx, dy = backend.alloc(x.size).write(x), backend.alloc(out_ch * 70)
+        backend.conv1d(dx.ptr, dy.ptr, in_ch, out_ch, 70, 1, 1, w, None)
+        want = w[:, :, 0].astype(np.float64) @ x.astype(np.float64)
+        assert np.linalg.norm(dy.read().reshape(want.shape) - want) < 2e-6 * np.linalg.norm(want), (out_ch, in_ch)
+        dx.free()
+        dy.free()
+    backend.set_quant(pkg.INT8)
+    for n, k in ((64, 128), (128, 64)):
+        w, x = shared.reshape(n, k), rng.standard_normal((1, k)).astype(np.float32)
+        want = x.astype(np.float64) @ w.astype(np.float64).T
+        # both factors rounded to int8: a step of 1 / 127 of the largest value, uniform, over k terms -- about 1e-2 of the product's norm
+        assert np.linalg.norm(backend.matmul(x, w) - want) < 3e-2 * np.linalg.norm(want), (n, k)
+    backend.set_quant(pkg.F32)
