@@ -237,7 +237,8 @@ int mynah_hip_rows_combine_dev(void *state, const float *const *dev_inputs, size
  * all from dev_input, then ((b0 + b1) + ...) * (1 / branches), through the half-snake of then_alpha when that is not null, to
  * dev_output.  blocks[branch * positions + position]; every half-snake has channels / 2 snake rows; weights, biases (may be null)
  * and alphas are host pointers, cached like every weight.  dev_work: 3 * branches row sets [channels, length] of the caller's,
- * overwritten.  The values are those of the operator sequence above, bit for bit; up to 128 channels with 3, 7 or 11 taps a
+ * overwritten, none of them another one or dev_input (a single branch's first may be dev_input); dev_output may be dev_input or
+ * any of them.  The values are those of the operator sequence above, bit for bit; up to 128 channels with 3, 7 or 11 taps a
  * position of all branches is one launch.  No counterpart in the reference's seam. */
 typedef struct mynah_hip_res_block {
     const float *alpha_in, *weight_in, *bias_in;

@@ -423,21 +423,22 @@ class Backend:
     def res_layer_dev(self, blocks, din, dout, channels, length, work, then_alpha=None):
         """A residual layer as one call.  blocks[branch][position] = (alpha_in, (w_in, b_in), alpha_skip, (w_skip, b_skip),
         dilation); work: three row sets per branch."""
+        positions = len(blocks[0])   # every branch has that many blocks (more are not looked at)
+        if len(work) != 3 * len(blocks):
+            raise ValueError("res_layer_dev: three row sets per branch, not %d for %d branches" % (len(work), len(blocks)))
+        layer = [branch[p] for branch in blocks for p in range(positions)]
         desc = self._res_layers.get(id(blocks))
-        parts = [a for branch in blocks for b in branch for a in (b[0], b[1][0], b[1][1], b[2], b[3][0], b[3][1], b[4])]
+        parts = [a for b in layer for a in (b[0], b[1][0], b[1][1], b[2], b[3][0], b[3][1], b[4])]
         if desc is None or len(desc[1]) != len(parts) or not all(map(operator.is_, desc[1], parts)):
-            arr = (ResBlock * (len(blocks) * len(blocks[0])))()
-            slots = iter(arr)
-            for branch in blocks:
-                for a_in, (w_in, b_in), a_skip, (w_skip, b_skip), dilation in branch:
-                    s = next(slots)
-                    s.alpha_in, s.weight_in, s.bias_in = self.address(a_in), self.address(w_in), self.address(b_in)
-                    s.alpha_skip, s.weight_skip, s.bias_skip = self.address(a_skip), self.address(w_skip), self.address(b_skip)
-                    s.kernel_in, s.kernel_skip, s.dilation = w_in.shape[2], w_skip.shape[2], dilation
+            arr = (ResBlock * len(layer))()
+            for s, (a_in, (w_in, b_in), a_skip, (w_skip, b_skip), dilation) in zip(arr, layer):
+                s.alpha_in, s.weight_in, s.bias_in = self.address(a_in), self.address(w_in), self.address(b_in)
+                s.alpha_skip, s.weight_skip, s.bias_skip = self.address(a_skip), self.address(w_skip), self.address(b_skip)
+                s.kernel_in, s.kernel_skip, s.dilation = w_in.shape[2], w_skip.shape[2], dilation
             if len(self._res_layers) >= 64:   # a codec has five; lists made anew for each call are not collected
                 self._res_layers.clear()
             desc = self._res_layers[id(blocks)] = (blocks, parts, arr)   # (held: an id stays one object's)
-        self._call("mynah_hip_res_layer_dev", desc[2], len(blocks), len(blocks[0]), din, dout, channels, length, self.address(then_alpha),
+        self._call("mynah_hip_res_layer_dev", desc[2], len(blocks), positions, din, dout, channels, length, self.address(then_alpha),
                    (_vp * len(work))(*work))
 
     def argmax_dev(self, dlogits, vocab, codebook_size, eos_id, allow_eos):

@@ -55,5 +55,6 @@ def res_layer_fused(backend, blocks, din, dout, channels, length, current, activ
 
 
 def res_layer_batched(backend, blocks, din, dout, channels, length, currents, activateds, residuals, then_alpha=None):
-    """currents, activateds, residuals: one buffer per branch each (the branches run side by side)."""
-    backend.res_layer_dev(blocks, din, dout, channels, length, [*currents, *activateds, *residuals], then_alpha)
+    """currents, activateds, residuals: one buffer per branch each (the branches run side by side).  dout may be din or any of them."""
+    n = len(blocks)
+    backend.res_layer_dev(blocks, din, dout, channels, length, [*currents[:n], *activateds[:n], *residuals[:n]], then_alpha)

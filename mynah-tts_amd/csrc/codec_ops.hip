@@ -1383,12 +1383,14 @@ extern "C" int mynah_hip_res_layer_dev(void *state, const mynah_hip_res_block *b
                                        size_t capacity) {
     State *st = enter_state(state);
     if (st == nullptr || blocks == nullptr || branches == 0 || branches > (size_t)kConvBatchMax || positions == 0 || dev_input == nullptr || dev_output == nullptr ||
-        dev_input == dev_output || dev_work == nullptr || channels == 0 || channels > (size_t)INT_MAX || length == 0 || length > (size_t)INT_MAX) {
+        dev_work == nullptr || channels == 0 || channels > (size_t)INT_MAX || length == 0 || length > (size_t)INT_MAX) {
         set_error(error, capacity, "invalid residual layer arguments (one to four branches)");
         return -1;
     }
+    // (the output is written by the last launch alone, value by value from the branches' rows: it may be the input or any of the work rows;
+    // a single branch may also grow in its input)
     for (size_t i = 0; i < 3 * branches; ++i) {
-        bool distinct = dev_work[i] != nullptr && dev_work[i] != dev_input && dev_work[i] != dev_output;
+        bool distinct = dev_work[i] != nullptr && (dev_work[i] != dev_input || (i == 0 && branches == 1));
         for (size_t j = 0; j < i; ++j) distinct = distinct && dev_work[i] != dev_work[j];
         if (!distinct) {
             set_error(error, capacity, "residual layer: work rows must be buffers of their own");

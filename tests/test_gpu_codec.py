@@ -162,7 +162,7 @@ def test_fused_res_layer_is_the_operator_sequence(pkg, backend, orc, nerr, C, L)
 @pytest.mark.parametrize("C,L", [(16, 1), (27, 54), (32, 55), (33, 53), (64, 109), (65, 107), (108, 641), (128, 54), (128, 700), (27, 20000)])
 def test_res_layer_call(pkg, backend, orc, nerr, C, L):
     """mynah_hip_res_layer_dev is the operator sequence bit for bit, whatever follows (a half-snake or none), and refuses work rows
-    that are the layer's own or each other's."""
+    that are the layer's input or each other's."""
     import importlib
     codec = importlib.import_module(pkg.__name__ + ".codec")
     _announce("residual layer call %d x %d" % (C, L))
@@ -190,10 +190,41 @@ def test_res_layer_call(pkg, backend, orc, nerr, C, L):
                 cur = cur + orc.conv1d_causal(orc.snake(orc.conv1d_causal(orc.snake(cur, a_in, C // 2), w_in, b_in, d), a_skip, C // 2), w_skip, b_skip, 1)
             total += cur
         assert nerr(bufs[1].read().reshape(C, L), orc.snake(total * np.float32(1.0 / 3.0), then, C // 2)) < 1e-5
-    for work in ([din.ptr] + at[3:11], at[2:10] + [at[2]], [at[1]] + at[3:11]):
+    for work in ([din.ptr] + at[3:11], at[2:10] + [at[2]]):
         with pytest.raises(pkg.BackendError):
             codec.res_layer_batched(backend, blocks, din.ptr, at[1], C, L, work[0:3], work[3:6], work[6:9])
     for d in bufs + [din]:
+        d.free()
+
+
+@pytest.mark.parametrize("C,L", [(27, 130), (108, 200), (216, 90)])
+def test_res_layer_output_and_branch_forms(pkg, backend, C, L):
+    """The layer's output may be its input or any of the work rows, in one launch a block or several; a single branch may grow in its
+    input; blocks that the first branch does not have are not looked at, and a branch with fewer, or too few work rows, is an error."""
+    import importlib
+    codec = importlib.import_module(pkg.__name__ + ".codec")
+    _announce("residual layer output forms %d x %d" % (C, L))
+    x, blocks = _res_layer_inputs(C, L, 140 + C)
+    n = C * L
+    bufs = [backend.alloc(n) for _ in range(11)]
+    at = [b.ptr for b in bufs]
+
+    def layer(blocks, dout, work):
+        bufs[0].write(x.ravel())
+        codec.res_layer_batched(backend, blocks, at[0], dout, C, L, work[0:3], work[3:6], work[6:9])
+        return next(b for b in bufs if b.ptr == dout).read().view(np.uint32)
+
+    want = layer(blocks, at[1], at[2:11])
+    for dout in (at[0], at[2], at[6], at[10]):
+        assert np.array_equal(layer(blocks, dout, at[2:11]), want), at.index(dout)
+    assert np.array_equal(layer([blocks[0], blocks[1] + blocks[2], blocks[2]], at[1], at[2:11]), want)
+    with pytest.raises(IndexError):
+        layer([blocks[0], blocks[1][:2], blocks[2]], at[1], at[2:11])
+    with pytest.raises(ValueError):
+        backend.res_layer_dev(blocks, at[0], at[1], C, L, at[2:10])
+    one = layer(blocks[2:], at[1], at[2:11])
+    assert np.array_equal(layer(blocks[2:], at[1], [at[0]] + at[3:11]), one)
+    for d in bufs:
         d.free()
 
 
