@@ -1,12 +1,12 @@
 """The codec's residual layer as two sequences of backend calls.
 
 `res_layer` issues what res_layer_device issues (src/graph.c:2423-2498): per branch a copy of the input, per block
-copy, snake, conv, snake, conv, residual add, then the branch added to the output, and the sum scaled by a third at the
-end.  `res_layer_fused` computes the same values, bit for bit, from a third of the launches: the element-wise operators
+copy, snake, conv, snake, conv, residual add, then the branch added to the output, and the sum scaled by 1 / branches (the model's
+three: a third) at the end.  `res_layer_fused` computes the same values, bit for bit, from a third of the launches: the element-wise operators
 travel in the epilogue of the convolution before them (mynah_hip_conv1d_fused), and only a branch's first activation is a
 pass of its own (snake_copy_dev).  `res_layer_batched` is the whole layer as one call (mynah_hip_res_layer_dev), the three branches
-side by side -- they do not depend on each other until their sum -- and, up to 128 channels, a block of all branches in one
-launch.  Same values again, bit for bit.
+side by side -- they do not depend on each other until their sum -- and a block of all branches in one launch up to 32 channels, and
+up to 64 for the middle range of lengths (three branches: some 2700 to 20000 positions).  Same values again, bit for bit.
 
 blocks[branch][block] = (alpha_in, (w_in, b_in), alpha_skip, (w_skip, b_skip), dilation); the branch's kernel size is the
 weights' last dimension.  Buffers are device allocations of channels * length floats.
@@ -29,7 +29,7 @@ def res_layer(backend, blocks, din, dout, channels, length, current, activated, 
             backend.copy_dev(dout, current, n)          # the reference adds to uploaded zeros (src/graph.c:2441,2492)
         else:
             backend.residual_inplace(dout, current, n)
-    backend.scale_dev(dout, n, 1.0 / 3.0)
+    backend.scale_dev(dout, n, 1.0 / len(blocks))
 
 
 def res_layer_fused(backend, blocks, din, dout, channels, length, current, activated, residual, then_alpha=None):
@@ -50,7 +50,7 @@ def res_layer_fused(backend, blocks, din, dout, channels, length, current, activ
                 # the branch's last block adds the branch to the output, and the last branch scales the sum
                 backend.conv1d_fused(residual, dout, channels, channels, length, kernel, 1, w_skip, b_skip, residual=before,
                                      residual2=None if index == 0 else dout,
-                                     scale=1.0 / 3.0 if index + 1 == len(blocks) else 1.0,
+                                     scale=1.0 / len(blocks) if index + 1 == len(blocks) else 1.0,
                                      alpha=then_alpha if index + 1 == len(blocks) else None)
 
 

@@ -603,8 +603,8 @@ __global__ void __launch_bounds__(256) k_conv_finish(const ConvBatchArgs b) {
 // window of 64 * WN positions of the inner rows r = snake(conv_in(snake(x))), (taps - 1) more than the positions it finishes:
 // it stages snake(x) (a position and its halo are activated once, since every row is here), multiplies, activates, leaves the
 // pieces of r in LDS over the stages, and multiplies again from there.  Every value is the separate calls' arithmetic in their
-// order: the same bits.
-// (27 channels x 65536, taps 3 / 7 / 11: 63 us against 2 x 39 us as two launches; 54 x 2560: 27 us against 2 x 22.)
+// order: the same bits.  SPLIT: the order of the channel-split tiles, whose four wavefronts take a block of channels each up to
+// 64 channels -- a block's sums from zero, added block after block, then the bias; else that of the large tiles, one chain from the bias.
 struct ResMember {
     const float *in;                      // [channels, length]
     float *out;
@@ -622,7 +622,7 @@ struct ResArgs {
 
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 
-template <int WM, int WN, int NT, int KF>
+template <int WM, int WN, int NT, bool SPLIT, int KF>
 __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember &m, uint4 *const lds, float2 *const s_pairs) {
     constexpr int WP = 32 * NT, RN = WP * WN, T = 64 * WM * WN, TN = RN - (KF - 1);
     const int t0 = blockIdx.x * TN;
@@ -700,21 +700,45 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
         bias_in[r] = m.b_in != nullptr ? m.b_in[row] : 0.0f;
         bias_skip[r] = m.b_skip != nullptr ? m.b_skip[row] : 0.0f;
     }
-    const auto start = [&](const float (&bias)[16], f32x16 (&acc)[NT]) {
+    f32x16 acc[NT], sum[SPLIT ? NT : 1];
+    const auto start = [&](const float (&bias)[16]) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[0][r] = wm * 32 + split_acc_row(r, lane) < a.channels ? bias[r] : 0.0f;
+        for (int r = 0; r < 16; ++r) acc[0][r] = !SPLIT && wm * 32 + split_acc_row(r, lane) < a.channels ? bias[r] : 0.0f;
 #pragma unroll
         for (int n = 1; n < NT; ++n) acc[n] = acc[0];
+        if constexpr (SPLIT) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n) sum[n] = f32x16{0};
+        }
+    };
+    // (SPLIT) a block's sums to those of the blocks before it; in the end, the bias
+    const auto add_block = [&]() {
+        if constexpr (SPLIT) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                sum[n] += acc[n];
+                acc[n] = f32x16{0};
+            }
+        }
+    };
+    const auto finish = [&](const float (&bias)[16]) {
+        add_block();
+        if constexpr (SPLIT) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[n][r] = sum[n][r] + bias[r];
+        }
     };
     const size_t w_at = (size_t)min(wm, a.tiles - 1) * a.blocks * KF * 192 + lane;
     fetch(0);
     ConvWeights w(m.w_in + w_at, 0, 1, KF);
     uint4 *stage_now = lds, *stage_next = lds + 6 * win;
-    f32x16 acc[NT];
-    start(bias_in, acc);
+    start(bias_in);
     publish(0, stage_now);
     fetch(min(1, a.blocks - 1));
     conv_products<KF, NT, true>(w, KF, m.dilation, 2 * win, a.blocks, [&](int block) {
+        if (block > 0) add_block();
         __syncthreads();
         const uint4 *at = stage_now + half * win + wn * WP + col;
         if (block + 1 < a.blocks) {
@@ -726,6 +750,7 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
         stage_next = t;
         return at;
     }, acc);
+    finish(bias_in);
 
     // the finished rows' residual (x itself), on its way during the rest: whole rows of consecutive positions, as it is stored
     const int rows = min(32, a.channels - wm * 32);
@@ -784,9 +809,13 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
             for (int q = 0; q < 3; ++q) reinterpret_cast<uint2 *>(&lds[(block * 6 + q * 2 + (g & 1)) * RN + p])[half] = s.piece[q];
         }
     }
-    start(bias_skip, acc);
+    start(bias_skip);
     __syncthreads();
-    conv_products<KF, NT, true>(w2, KF, 1, 2 * RN, a.blocks, [&](int block) { return const_cast<const uint4 *>(lds + (block * 6 + half) * RN + wn * WP + col); }, acc);
+    conv_products<KF, NT, true>(w2, KF, 1, 2 * RN, a.blocks, [&](int block) {
+        if (block > 0) add_block();
+        return const_cast<const uint4 *>(lds + (block * 6 + half) * RN + wn * WP + col);
+    }, acc);
+    finish(bias_skip);
 
     // + x, and out, in whole rows (see store_tile of conv_tile)
     __syncthreads();   // the inner rows have been read
@@ -804,20 +833,20 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
     }
 }
 
-template <int WM, int WN, int NT>
+template <int WM, int WN, int NT, bool SPLIT>
 __global__ void __launch_bounds__(64 * WM * WN, 2) k_res_block(const ResArgs a) {
     extern __shared__ __align__(16) uint4 lds[];
     __shared__ float2 s_pairs[kResMaxChannels];
     const int z = a.order[blockIdx.y];
     switch (a.member[z].kernel) {
-        case 3: res_block_tile<WM, WN, NT, 3>(a, a.member[z], lds, s_pairs); break;
-        case 7: res_block_tile<WM, WN, NT, 7>(a, a.member[z], lds, s_pairs); break;
-        default: res_block_tile<WM, WN, NT, 11>(a, a.member[z], lds, s_pairs); break;
+        case 3: res_block_tile<WM, WN, NT, SPLIT, 3>(a, a.member[z], lds, s_pairs); break;
+        case 7: res_block_tile<WM, WN, NT, SPLIT, 7>(a, a.member[z], lds, s_pairs); break;
+        default: res_block_tile<WM, WN, NT, SPLIT, 11>(a, a.member[z], lds, s_pairs); break;
     }
 }
 
-template <int WM, int WN, int NT>
-int launch_res_block_n(State *st, const ResArgs &a, int count, char *error, size_t capacity) {
+template <int WM, int WN, int NT, bool SPLIT = false>
+int launch_res_block(State *st, const ResArgs &a, int count, char *error, size_t capacity) {
     constexpr int RN = 32 * NT * WN;
     int taps = 0, reach = 0;
     for (int i = 0; i < count; ++i) {
@@ -832,20 +861,12 @@ int launch_res_block_n(State *st, const ResArgs &a, int count, char *error, size
     lds = tiles > lds ? tiles : lds;
     static bool raised = false;
     if (!raised) {
-        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_res_block<WM, WN, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 112 * 1024));
+        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_res_block<WM, WN, NT, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, 112 * 1024));
         raised = true;
     }
     const int finished = RN - (taps - 1);
-    hipLaunchKernelGGL((k_res_block<WM, WN, NT>), dim3((unsigned)((a.length + finished - 1) / finished), (unsigned)count), dim3(64 * WM * WN), lds, st->stream, a);
+    hipLaunchKernelGGL((k_res_block<WM, WN, NT, SPLIT>), dim3((unsigned)((a.length + finished - 1) / finished), (unsigned)count), dim3(64 * WM * WN), lds, st->stream, a);
     return hip_check(hipGetLastError(), "residual block launch", error, capacity);
-}
-
-// 64 positions to a wavefront, or 32 where that many workgroups still find a CU each: a wavefront's chain of products is then half as
-// long, which is all that counts there.  (A position's values do not depend on the tile it is in.)
-template <int WM, int WN>
-int launch_res_block(State *st, const ResArgs &a, int count, char *error, size_t capacity) {
-    const long narrow = (long)(a.length + 32 * WN - 11) / (32 * WN - 10) * count;
-    return narrow <= st->cu_count ? launch_res_block_n<WM, WN, 1>(st, a, count, error, capacity) : launch_res_block_n<WM, WN, 2>(st, a, count, error, capacity);
 }
 
 __global__ void __launch_bounds__(256) k_conv_pack(const float *src, uint4 *dst, size_t count, int out_ch, int in_ch, int kernel, int blocks) {
@@ -1017,6 +1038,12 @@ int launch_conv_finish(State *st, const ConvBatchArgs &b, int count, char *error
     return hip_check(hipGetLastError(), "conv1d finish launch", error, capacity);
 }
 
+// The channel-split tiles of `count` convolutions side by side: 32 positions wide while 64 would leave CUs without one.  (The width does
+// not enter a value's arithmetic -- same channel blocks per wavefront, same order.)
+bool conv_split_narrow(const State *st, int out_channels, int length, long count) {
+    return (long)((out_channels + 31) / 32) * ((length + 63) / 64) * count < st->cu_count;
+}
+
 int launch_conv_split(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
     if (a.splits > 1) {
         ConvBatchArgs b{};
@@ -1024,8 +1051,7 @@ int launch_conv_split(State *st, const ConvArgs &a, const ConvBlocks &weights, c
         const int rc = a.length <= 32 ? launch_conv_split_n<1>(st, a, weights, error, capacity) : launch_conv_split_n<2>(st, a, weights, error, capacity);
         return rc != 0 ? rc : launch_conv_finish(st, b, 1, error, capacity);
     }
-    const long tiles = (long)((a.out_ch + 31) / 32) * ((a.length + 63) / 64);
-    if (tiles < st->cu_count) return launch_conv_split_n<1>(st, a, weights, error, capacity);
+    if (conv_split_narrow(st, a.out_ch, a.length, 1)) return launch_conv_split_n<1>(st, a, weights, error, capacity);
     return launch_conv_split_n<2>(st, a, weights, error, capacity);
 }
 
@@ -1076,14 +1102,19 @@ int mynah::launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_
     return hip_check(hipGetLastError(), "weight packing launch", error, capacity);
 }
 
-// few output channels: one row of wavefronts, wider in time; too few large tiles to fill the chip and enough input channels to
-// share out (more than one block for each of four wavefronts): small tiles with the channels split over the wavefronts.  The two
-// add in different orders, so the choice is the shape's alone, for single, batched and fused launches alike.  216 channels: the two
-// meet at 4096 positions (three members, 72 us either way), and the large tiles' launch has no more wavefronts than it needs;
-// 108 channels: the small tiles' three members at 1280 positions take 14 us, a fused block of large tiles 41.
+// Too few large tiles to fill the chip and more than one block of channels to share out: small tiles with the channels split over the
+// wavefronts.  (Few output channels: the large tiles are one row of wavefronts, wider in time.)  The two add in different orders, so
+// the choice is the shape's alone, for single, batched and fused launches alike, and the line lies where a residual layer's
+// three members meet; one convolution alone would change over later.  us, small tiles / large:
+//   three members of taps 3, 7, 11, six launches:  216 channels x 3072 327 / 383, x 3584 388 / 393, x 4096 429 / 401;
+//     108 x 4096 184 / 204, x 5120 209 / 212, x 6144 251 / 230
+//   alone, 3 / 11 taps:  216 x 3072 18.7 33 / 26 54;  108 x 5120 12.2 19 / 17.8 29.5;  54 x 12000 9.9 (11.8 with 7 taps) / 13 17;
+//     64 -> 864 x 640 9.6 (13.4) / 13.3 17.8, x 1280 16.3 (19) / 14 17.5;  32 -> 864 x 5, 7 taps: 8.8 / 11.6, x 128 7.9 / 12
+// A layer of at most 32 channels has two blocks at most and runs as one launch a block, in the large tiles' order.
 static bool conv_takes_split(const State *st, int in_channels, int out_channels, int length) {
     const long tiles = out_channels <= 32 ? (long)((length + 255) / 256) : (long)((out_channels + 63) / 64) * ((length + 127) / 128);
-    return in_channels > 64 && tiles < (in_channels > kResMaxChannels ? (long)st->cu_count / 4 : (long)st->cu_count * 3 / 8);
+    if (in_channels < 32 || (in_channels == 32 && out_channels <= 32)) return false;
+    return tiles < (in_channels > kResMaxChannels ? (long)st->cu_count * 7 / 16 : (long)st->cu_count * 3 / 8);
 }
 
 // How many workgroups share a channel-split tile.  A few short rows leave most of the chip idle while each tile's workgroup pulls the
@@ -1223,14 +1254,12 @@ extern "C" int mynah_hip_conv1d_fused_batch(void *state, const mynah_hip_conv1d_
         return 0;
     }
     if (conv_takes_split(st, in_channels, out_channels, length)) {
-        // (the tile's width does not enter a value's arithmetic -- same channel blocks per wavefront, same order -- so the
-        // members may take the wider tile, half the weight traffic per product, as soon as all of them together fill the chip)
+        // (the wider tile, half the weight traffic per product, as soon as all members together fill the chip)
         if (b.item[0].splits > 1) {
             const int rc = length <= 32 ? launch_conv_split_batch<1>(st, b, (int)count, error, capacity) : launch_conv_split_batch<2>(st, b, (int)count, error, capacity);
             return rc != 0 ? rc : launch_conv_finish(st, b, (int)count, error, capacity);
         }
-        const long tiles = (long)((out_channels + 31) / 32) * ((length + 63) / 64);
-        if (tiles * (long)count < st->cu_count) return launch_conv_split_batch<1>(st, b, (int)count, error, capacity);
+        if (conv_split_narrow(st, out_channels, length, (long)count)) return launch_conv_split_batch<1>(st, b, (int)count, error, capacity);
         return launch_conv_split_batch<2>(st, b, (int)count, error, capacity);
     }
     if (out_channels <= 32) return launch_conv_batch<1, 4>(st, b, (int)count, error, capacity);
@@ -1327,20 +1356,40 @@ extern "C" int mynah_hip_rows_combine_dev(void *state, const float *const *dev_i
     return hip_check(hipGetLastError(), "rows_combine launch", error, capacity);
 }
 
-// One position (block) of every branch in one launch, where the fused kernel takes it; *done tells.
+// The one-launch build for a position of a layer, or none.  Which are there follows the order in which the layer's convolutions add
+// (conv_takes_split) and whether all workgroups find a place at once: two to a CU (512 threads: one), 32 positions to a wavefront,
+// whose chain of products is then half as long, before 64.  Measured per layer of three positions, branches of 3 / 7 / 11 taps, us:
+//   27 channels: x 12288 67 narrow, 86 wide, 106 as two launches a position; x 20480 75, 90, 116; x 24576 (more than fit) 112, 100, 117
+//   54, split order: x 2560 81 narrow, 75 as two launches of narrow split tiles; x 3072 80, 82; x 8192 97, 141; x 10240 134, 157
+//   54, large order: x 16384 163 wide, 174 as two launches; x 20480 177, 203; x 20992 (more than fit) 229, 201
+//   108, large order, 3 and 11 taps: x 6144 173 narrow, 202; x 8192 186, 204; x 12288 (more than fit) 276, 240
+// (three branches of 65 to 128 channels are never in the large order and few enough)
+enum ResBuild { RES_NONE, RES_32_NARROW, RES_32_WIDE, RES_64_SPLIT, RES_64_WIDE, RES_128 };
+static ResBuild res_build(const State *st, const mynah_hip_res_block *blocks, size_t branches, size_t stride, size_t channels, size_t length) {
+    if (channels > (size_t)kResMaxChannels) return RES_NONE;
+    for (size_t i = 0; i < branches; ++i) {
+        const int k = blocks[i * stride].kernel_in;
+        if (k != blocks[i * stride].kernel_skip || (k != 3 && k != 7 && k != 11) || (k - 1) * (long)blocks[i * stride].dilation > kResMaxReach) return RES_NONE;
+    }
+    const auto fit = [&](long columns, int each) {   // workgroups of that many columns, the taps' reach of them only read
+        long n = 0;
+        for (size_t i = 0; i < branches; ++i) n += ((long)length + columns - blocks[i * stride].kernel_in) / (columns - (blocks[i * stride].kernel_in - 1));
+        return n <= (long)st->cu_count * each;
+    };
+    if (channels <= 32) return fit(128, 2) ? RES_32_NARROW : RES_32_WIDE;
+    const bool split = conv_takes_split(st, (int)channels, (int)channels, (int)length);
+    if (channels > 64) return !split && fit(64, 1) ? RES_128 : RES_NONE;
+    if (split) return conv_split_narrow(st, (int)channels, (int)length, (long)branches) ? RES_NONE : RES_64_SPLIT;
+    return fit(128, 2) ? RES_64_WIDE : RES_NONE;
+}
+
+// One position (block) of every branch in one launch, where there is a build for it; *done tells.
 static int res_position(State *st, const mynah_hip_res_block *blocks, size_t branches, size_t stride, const float *const *in, float *const *out, size_t channels,
                         size_t length, bool *done, char *error, size_t capacity) {
-    *done = false;
+    const ResBuild build = res_build(st, blocks, branches, stride, channels, length);
+    *done = build != RES_NONE;
+    if (!*done) return 0;
     ResArgs a{};
-    // Above 32 channels only while the launch does not fill the chip: with enough tiles the two launches overlap their phases
-    // better (108 channels x 16384: 138 us a position fused, 124 as two launches; 54 x 32768: 94 and 77; 27 x 65536: 63 and 78).
-    if (conv_takes_split(st, (int)channels, (int)channels, (int)length)) return 0;
-    if (channels > 32 && (length + 53) / 54 * branches > (size_t)st->cu_count) return 0;
-    for (size_t i = 0; i < branches; ++i) {
-        const mynah_hip_res_block &b = blocks[i * stride];
-        const int k = b.kernel_in;
-        if (channels > (size_t)kResMaxChannels || k != b.kernel_skip || (k != 3 && k != 7 && k != 11) || (k - 1) * (long)b.dilation > kResMaxReach) return 0;
-    }
     a.channels = (int)channels;
     a.length = (int)length;
     a.snake_channels = (int)(channels / 2);
@@ -1372,10 +1421,13 @@ static int res_position(State *st, const mynah_hip_res_block *blocks, size_t bra
         for (; at > 0 && a.member[a.order[at - 1]].kernel < m.kernel; --at) a.order[at] = a.order[at - 1];
         a.order[at] = (int)i;
     }
-    *done = true;
-    if (channels <= 32) return launch_res_block<1, 4>(st, a, (int)branches, error, capacity);
-    if (channels <= 64) return launch_res_block<2, 2>(st, a, (int)branches, error, capacity);
-    return launch_res_block<4, 2>(st, a, (int)branches, error, capacity);
+    switch (build) {
+        case RES_32_NARROW: return launch_res_block<1, 4, 1>(st, a, (int)branches, error, capacity);
+        case RES_32_WIDE: return launch_res_block<1, 4, 2>(st, a, (int)branches, error, capacity);
+        case RES_64_SPLIT: return launch_res_block<2, 2, 1, true>(st, a, (int)branches, error, capacity);
+        case RES_64_WIDE: return launch_res_block<2, 2, 2>(st, a, (int)branches, error, capacity);
+        default: return launch_res_block<4, 2, 1>(st, a, (int)branches, error, capacity);
+    }
 }
 
 extern "C" int mynah_hip_res_layer_dev(void *state, const mynah_hip_res_block *blocks, size_t branches, size_t positions, const float *dev_input,

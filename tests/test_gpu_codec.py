@@ -34,7 +34,9 @@ def test_known_answer(backend):
 # 1/3/5), the post-conv, and shapes that end inside a tile or are shorter than a tap's reach
 SHAPES = [(32, 864, 75, 7, 1), (432, 432, 600, 3, 1), (216, 216, 700, 7, 3), (108, 108, 1000, 11, 5), (54, 54, 3000, 11, 1),
           (27, 27, 5000, 7, 5), (27, 1, 9000, 3, 1), (5, 70, 33, 1, 1), (9, 33, 20, 11, 5), (8, 64, 128, 2, 1),
-          (40, 48, 300, 16, 8), (64, 40, 257, 5, 2), (33, 65, 129, 4, 1), (128, 96, 64, 1, 1)]   # generic tap counts, the largest reach, odd edges
+          (40, 48, 300, 16, 8), (64, 40, 257, 5, 2), (33, 65, 129, 4, 1), (128, 96, 64, 1, 1),
+          # channels split over the wavefronts from 32 on: a few positions, the last row count that splits and the first that does not
+          (32, 864, 1, 7, 1), (32, 32, 200, 7, 1), (31, 864, 40, 7, 1), (33, 300, 2432, 3, 1), (33, 300, 2433, 3, 1)]   # generic tap counts, the largest reach, odd edges
 
 
 @pytest.mark.parametrize("shape", SHAPES)
@@ -110,11 +112,11 @@ def test_res_block_chain(backend, orc, nerr):
         d.free()
 
 
-def _res_layer_inputs(C, L, seed):
+def _res_layer_inputs(C, L, seed, taps=(3, 7, 11)):
     rng = np.random.default_rng(seed)
     alpha = lambda: (np.abs(rng.standard_normal(C // 2)) + 0.1).astype(np.float32)
     conv = lambda k: ((rng.standard_normal((C, C, k)) / np.sqrt(C * k)).astype(np.float32), rng.standard_normal(C).astype(np.float32) * np.float32(0.1))
-    blocks = [[(alpha(), conv(k), alpha(), conv(k), d) for d in (1, 3, 5)] for k in (3, 7, 11)]
+    blocks = [[(alpha(), conv(k), alpha(), conv(k), d) for d in (1, 3, 5)] for k in taps]
     return rng.standard_normal((C, L)).astype(np.float32), blocks
 
 
@@ -158,7 +160,7 @@ def test_fused_res_layer_is_the_operator_sequence(pkg, backend, orc, nerr, C, L)
         d.free()
 
 
-# a block as one launch: every tile shape (at most 32, 64, 128 channels), rows and channels one off a tile's, a chip full of tiles
+# a block as one launch up to 32 channels, two launches for the short rows above: rows and channels one off a tile's
 @pytest.mark.parametrize("C,L", [(16, 1), (27, 54), (32, 55), (33, 53), (64, 109), (65, 107), (108, 641), (128, 54), (128, 700), (27, 20000)])
 def test_res_layer_call(pkg, backend, orc, nerr, C, L):
     """mynah_hip_res_layer_dev is the operator sequence bit for bit, whatever follows (a half-snake or none), and refuses work rows
@@ -193,6 +195,31 @@ def test_res_layer_call(pkg, backend, orc, nerr, C, L):
     for work in ([din.ptr] + at[3:11], at[2:10] + [at[2]]):
         with pytest.raises(pkg.BackendError):
             codec.res_layer_batched(backend, blocks, din.ptr, at[1], C, L, work[0:3], work[3:6], work[6:9])
+    for d in bufs + [din]:
+        d.free()
+
+
+# (branches by their taps) each build of the one-launch block and the edges between it and its neighbours, on 256 CUs: at most 32 channels
+# narrow and wide; to 64 two launches / split order / wide in the large order / two launches; to 128 (fewer branches) split tiles / one launch
+@pytest.mark.parametrize("C,L,taps", [(27, 20780, (3, 7, 11)), (27, 20786, (3, 7, 11)), (32, 30300, (3, 11)), (64, 2688, (3, 7, 11)), (64, 2689, (3, 7, 11)),
+                                      (33, 4609, (3, 7, 11)), (50, 8193, (7,)), (54, 12160, (11, 3, 3, 7)), (54, 12161, (3, 7, 11)), (64, 20741, (3, 7, 11)),
+                                      (54, 20800, (3, 7, 11)), (108, 6016, (11,)), (108, 6017, (11,)), (65, 6017, (3, 11)), (128, 6090, (7, 3)),
+                                      (113, 13824, (11,)), (113, 13825, (11,)), (216, 3456, (3, 7)), (216, 3585, (3, 7))])
+def test_res_layer_builds(pkg, backend, C, L, taps):
+    """mynah_hip_res_layer_dev is the operator sequence bit for bit whichever way its blocks are launched."""
+    import importlib
+    codec = importlib.import_module(pkg.__name__ + ".codec")
+    _announce("residual layer builds %d x %d taps %s" % (C, L, taps))
+    x, blocks = _res_layer_inputs(C, L, 200 + C, taps)
+    n, b = C * L, len(taps)
+    din = backend.alloc(n).write(x)
+    bufs = [backend.alloc(n) for _ in range(2 + max(4, 3 * b))]
+    at = [d.ptr for d in bufs]
+    codec.res_layer(backend, blocks, din.ptr, at[0], C, L, *at[2:6])
+    codec.res_layer_batched(backend, blocks, din.ptr, at[1], C, L, at[2:2 + b], at[2 + b:2 + 2 * b], at[2 + 2 * b:2 + 3 * b])
+    want, got = bufs[0].read(), bufs[1].read()
+    assert np.isfinite(want).all()
+    assert np.array_equal(want.view(np.uint32), got.view(np.uint32))
     for d in bufs + [din]:
         d.free()
 
