@@ -773,7 +773,7 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention_f32(const float *qkv
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const bool seen = key < tokens && (!causal || key <= q0 + acc_row(r, lane));   // src/graph.c:446-449
-            S[acc_row(r, lane) * sstride + key] = seen ? acc[r] * scale : -3.0e38f;
+            S[acc_row(r, lane) * sstride + key] = seen ? acc[r] * scale : -__builtin_inff();
         }
     }
     __syncthreads();
@@ -781,7 +781,7 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention_f32(const float *qkv
         const int row = tid >> 3, part = tid & 7;
         float4 *srow = reinterpret_cast<float4 *>(S + row * sstride);
         const int npieces = keys / 4;
-        float m = -3.0e38f;
+        float m = -__builtin_inff();   // (every row sees a key: m is one of its scores in the end)
         for (int c = part; c < npieces; c += 8) {
             const float4 v = srow[c];
             m = fmaxf(fmaxf(m, fmaxf(v.x, v.y)), fmaxf(v.z, v.w));

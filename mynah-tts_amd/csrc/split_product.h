@@ -10,7 +10,10 @@
 //   |l| <= 2^-16 |h| make them 2^-23 of the product at most and 2^-26 on average, of either sign, where one f32 addition rounds
 //   2^-24 of the running sum -- and a step of 16 along the inner dimension has six such additions here and eight there.
 // Against double precision sums (192 x 3072 outputs, inner length 2304, relative error of the 2-norm): 4e-7 here, 8e-7 with
-// the f32 matrix instruction.  An infinite operand gives NaN where a plain product may give infinity; NaN stays NaN.
+// the f32 matrix instruction.
+// Operands without three finite pieces -- infinite, NaN, or so large that the first piece rounds to infinity (kSplitLimit) -- make every
+// sum they enter infinite or NaN.  Such a sum is looked for once, when it is finished (split_all_finite), and put in its place comes the
+// chain of f32 multiply-adds it stands for, from the operands themselves: an infinity stays one, and a large value is a value.
 #pragma once
 
 #include "device_common.h"
@@ -46,6 +49,31 @@ __device__ __forceinline__ void split_eight(const float4 a, const float4 b, bf16
     const SplitFour x(a), y(b);
 #pragma unroll
     for (int p = 0; p < 3; ++p) out[p] = __builtin_bit_cast(bf16x8, make_uint4(x.piece[p].x, x.piece[p].y, y.piece[p].x, y.piece[p].y));
+}
+
+constexpr float kSplitLimit = 0x1.ffp127f;   // bf16 rounds what is not below it to infinity
+__device__ __forceinline__ bool split_finite(float x) { return fabsf(x) < __builtin_inff(); }
+// Whether all sums of the wavefront are finite (one instruction a value: 0 * x is 0 or NaN).
+template <int N>
+__device__ __forceinline__ bool split_all_finite(const f32x16 (&acc)[N]) {
+    float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zero[r & 3] = __builtin_fmaf(acc[n][r], 0.0f, zero[r & 3]);
+    return !__any((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.0f);
+}
+// Where pieces are all that is kept of an operand, one from kSplitLimit on is kept as (infinity, upper half, lower half of its bits): it
+// makes its products infinite or NaN as it must, and can be had again.  piece: 16 bits each, as they lie in memory.
+__device__ __forceinline__ void split_keep_bits(float x, unsigned short &h, unsigned short &m, unsigned short &l) {
+    if (fabsf(x) < kSplitLimit) return;
+    h = 0x7f80;
+    m = (unsigned short)(__float_as_uint(x) >> 16);
+    l = (unsigned short)__float_as_uint(x);
+}
+__device__ __forceinline__ float split_value(unsigned short h, unsigned short m, unsigned short l) {
+    if (h == 0x7f80) return __uint_as_float((unsigned)m << 16 | l);
+    return __uint_as_float((unsigned)h << 16) + (__uint_as_float((unsigned)m << 16) + __uint_as_float((unsigned)l << 16));   // exact
 }
 
 // One 16-deep step: acc += a * w over the six pairs, the smallest first.

@@ -163,6 +163,44 @@ __device__ __forceinline__ void split_tile(const float *const a, const int lda, 
     }
 }
 
+// A finished tile to memory, a lane's column at `out`.  A sum that is no finite number is stored again as the chain of f32 multiply-adds
+// over the same blocks (split_product.h): looked for behind the stores, where it is cheapest (before them: 0.4 us a launch).
+template <int MT, int TAPS>
+__device__ __forceinline__ void split_store(const float *const a, const int lda, const int row0, const int rows, const float4 *const w, const int blocks,
+                                            const f32x16 (&acc)[MT], float *const out, const int pitch) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = row0 + 32 * t + split_acc_row(r, lane);
+            if (m < rows) out[(size_t)m * pitch] = acc[t][r];
+        }
+    if (split_all_finite(acc)) return;
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll 1
+        for (int r = 0; r < 16; ++r) {
+            const int m = row0 + 32 * t + split_acc_row(r, lane);
+            if (m >= rows || split_finite(acc[t][r])) continue;
+            float s = 0.0f;
+#pragma unroll 1
+            for (int c = 0; c < 32 * blocks && s == s; c += 4)
+#pragma unroll
+                for (int tap = 0; tap < TAPS; ++tap) {
+                    const int row = m - (TAPS - 1) + tap;
+                    if (row < 0) continue;
+                    const float4 x = *reinterpret_cast<const float4 *>(a + (size_t)row * lda + c);
+                    const float4 v = w[((c >> 4) * TAPS + tap) * 128 + ((c >> 2) & 1) * 64 + ((c >> 3) & 1) * 32 + (lane & 31)];
+                    s = __builtin_fmaf(x.x, v.x, s);
+                    s = __builtin_fmaf(x.y, v.y, s);
+                    s = __builtin_fmaf(x.z, v.z, s);
+                    s = __builtin_fmaf(x.w, v.w, s);
+                }
+            out[(size_t)m * pitch] = s;
+        }
+}
+
 // Workgroup -> (row tile, column tile and split): the row tiles of one piece of the weight run on one XCD (workgroup i runs on
 // XCD i % 8), which then fetches that piece once.
 struct SplitWork {
@@ -186,14 +224,7 @@ __global__ void __launch_bounds__(512) k_split_rows(const float *const a, const 
     const float4 *tile = w + ((size_t)(min(col0, N - 32) / 32) * (channels / 32) + z * blocks) * (2 * TAPS * 128);
     split_tile<MT, TAPS>(a + z * blocks * 32, channels, m0, M, tile, blocks, lds, acc);
     if (threadIdx.x >= 256 || col0 >= N) return;
-    float *const out = part + (size_t)z * M * N + col0 + (lane & 31);
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = m0 + 32 * t + split_acc_row(r, lane);
-            if (m < M) out[(size_t)m * N] = acc[t][r];
-        }
+    split_store<MT, TAPS>(a + z * blocks * 32, channels, m0, M, tile, blocks, acc, part + (size_t)z * M * N + col0 + (lane & 31), N);
 }
 
 // The K and V halves of every layer's kv_net on that layer's normalised memory, one launch: blockIdx.y names the layer.
@@ -210,13 +241,7 @@ __global__ void __launch_bounds__(512) k_split_cross_kv(const float *const norme
     split_tile<2, 1>(normed + (size_t)layer * M * width, width, m0, M, tile, width / 32, lds, acc);
     if (threadIdx.x >= 256 || col0 >= N) return;
     float *const out = (col0 < xw ? k_out + col0 : v_out + col0 - xw) + (size_t)layer * M * xw + (lane & 31);
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = m0 + 32 * t + split_acc_row(r, lane);
-            if (m < M) out[(size_t)m * xw] = acc[t][r];
-        }
+    split_store<2, 1>(normed + (size_t)layer * M * width, width, m0, M, tile, width / 32, acc, out, xw);
 }
 
 // The memory's rows under every layer's LayerNorm (gain, optional bias), one workgroup per row and layer: normed[layer][row].

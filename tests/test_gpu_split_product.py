@@ -84,3 +84,102 @@ def test_one_buffer_under_two_shapes(backend, pkg, orc):
         # both factors rounded to int8: a step of 1 / 127 of the largest value, uniform, over k terms -- about 1e-2 of the product's norm
         assert np.linalg.norm(backend.matmul(x, w) - want) < 3e-2 * np.linalg.norm(want), (n, k)
     backend.set_quant(pkg.F32)
+
+
+def test_cross_kv_extremes(backend, pkg, orc):
+    """Operands without three finite bf16 pieces: infinities, NaN, values from 2^128 - 2^119 on.  What f32 multiply-adds give, and only in
+    the outputs that they enter."""
+    print("[gpu-case] cross K/V extremes", flush=True)
+    rng = np.random.default_rng(8)
+    backend.set_quant(pkg.F32)
+    rows, width, xw = 70, 128, 96
+    gain = backend.keep(np.full(width, 0.2, np.float32))
+    memory = rng.standard_normal((rows, width)).astype(np.float32)
+    memory[5, 3] = np.inf                                   # a row of NaN behind the LayerNorm: the other rows do not change
+    w = rng.standard_normal((2 * xw, width)).astype(np.float32)
+    w[7, 11], w[8, 12], w[9, 13] = np.inf, -np.inf, np.nan
+    w[100, 20:22] = np.inf, -np.inf
+    w[40, 2], w[41, 127] = 3.4028235e38, -3.3962e38          # finite sums: |normed| < 1 there nearly everywhere
+    w[42, 60] = 3.396e38                                     # just below the limit
+    w = backend.keep(w)
+    dmem, dk, dv = backend.alloc(rows * width).write(memory), backend.alloc(rows * xw), backend.alloc(rows * xw)
+    backend.cross_kv_dev(dmem.ptr, rows, width, [gain], None, [w], xw, dk.ptr, dv.ptr)
+    got = np.concatenate([dk.read().reshape(rows, xw), dv.read().reshape(rows, xw)], axis=1).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        normed = np.stack([orc.layernorm(r, gain, None) for r in memory]).astype(np.float64)
+        want = normed @ w.astype(np.float64).T               # beyond f32's range: an infinity of that sign
+        want = np.where(np.abs(want) > 3.4028235e38, np.sign(want) * np.inf, want)
+    assert np.isnan(got[5]).all()
+    keep = np.arange(rows) != 5
+    got, want = got[keep], want[keep]
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isinf(want[:, [7, 8]]).all() and np.isnan(want[:, 9]).all()
+    assert np.isnan(want[:, 100]).any() and np.isinf(want[:, 100]).any()   # (as the two factors' signs differ or agree)
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    finite = np.isfinite(want)
+    assert finite[:, [40, 41, 42]].mean() > 0.9
+    # (a normalised value near zero carries the rounding of its row's mean, up to 2^-23, whatever its own size)
+    size = np.nan_to_num(np.abs(w.astype(np.float64)), posinf=0)
+    allowed = 2e-6 * np.abs(normed[keep]) @ size.T + 2.0 ** -23 * size.sum(axis=1)
+    assert (np.abs(got[finite] - want[finite]) < allowed[finite]).all()
+    for d in (dmem, dk, dv):
+        d.free()
+
+
+@pytest.mark.parametrize("taps", [1, 3])
+def test_encoder_f32_large_weights(backend, pkg, synth, nerr, taps):
+    """A value row and an FFN row that fill f32's range, their products scaled back by the weights behind them: the same stack as with both
+    in the ordinary range (powers of two throughout; the FFN row's GELU is saturated in both)."""
+    print("[gpu-case] encoder f32, weights at the range's end, taps=%d" % taps, flush=True)
+    cfg = dict(synth.encoder_config(layers=1, width=128, heads=2, ffn=192, vocab=32, max_positions=64), causal=True, ffn_kernel=taps, operands_f32=True)
+    rng = np.random.default_rng(taps)
+    normal = lambda *shape: (0.02 * rng.standard_normal(shape)).astype(np.float32)
+    base = {"tok_table": normal(32, 128), "pos_table": normal(64, 128), "qkv": normal(1, 384, 128), "o": normal(1, 128, 128),
+            "up": normal(1, 192, 128 * taps), "down": normal(1, 128, 192 * taps), "norm_out_g": np.ones(128, np.float32), "norm_out_b": None}
+    for name in ("norm1", "norm2"):
+        base[name + "_g"], base[name + "_b"] = np.full((1, 128), 1e-3, np.float32), None
+    top = np.float32(3.4e38 * 2.0 ** -128)                   # at 2^128 times its size above the first piece's range
+    base["qkv"][0, 256 + 70, 9] = base["up"][0, 33, 5 * taps] = top
+    base["o"][0, :, 70] = rng.standard_normal(128) * 2.0 ** 30    # (scaled back: 2^-98, above the range in which an operand loses bits)
+    base["up"][0, 33] *= np.float32(2.0 ** 44)               # (GELU differs from max(x, 0) by 0.17 at most: 1e-11 of such values)
+    base["down"].reshape(1, 128, 192, taps)[0, :, 33] *= np.float32(2.0 ** -10)
+    large = {k: None if v is None else v.copy() for k, v in base.items()}
+    large["qkv"][0, 256 + 70] *= np.float32(2.0 ** 64)
+    large["qkv"][0, 256 + 70] *= np.float32(2.0 ** 64)
+    large["o"][0, :, 70] *= np.float32(2.0 ** -64)
+    large["o"][0, :, 70] *= np.float32(2.0 ** -64)
+    large["up"][0, 33] *= np.float32(2.0 ** 84)
+    large["down"].reshape(1, 128, 192, taps)[0, :, 33] *= np.float32(2.0 ** -84)
+    ids = rng.integers(0, 32, size=41).astype(np.int32)
+    out = []
+    for w in (base, large):
+        enc = pkg.Encoder(backend, cfg, w)
+        dout = backend.alloc(41 * 128)
+        enc.prefill(ids, 0, dout.ptr)
+        out.append(dout.read())
+        enc.destroy()
+        dout.free()
+    assert np.isfinite(out[1]).all()
+    assert nerr(out[1], out[0]) < 1e-5
+
+
+def test_cross_kv_tiny_weights(backend, pkg, orc):
+    """Below 2^-110 an operand keeps fewer than its 24 bits: its third piece ends at bf16's smallest subnormal, 2^-133, so that at most half
+    of that is lost."""
+    print("[gpu-case] cross K/V, tiny weights", flush=True)
+    rng = np.random.default_rng(9)
+    backend.set_quant(pkg.F32)
+    rows, width, xw = 33, 64, 64
+    gain = backend.keep(np.ones(width, np.float32))
+    memory = rng.standard_normal((rows, width)).astype(np.float32)
+    w = backend.keep((rng.standard_normal((2 * xw, width)) * np.exp2(rng.integers(-126, -105, size=(2 * xw, 1)))).astype(np.float32))
+    dmem, dk, dv = backend.alloc(rows * width).write(memory), backend.alloc(rows * xw), backend.alloc(rows * xw)
+    backend.cross_kv_dev(dmem.ptr, rows, width, [gain], None, [w], xw, dk.ptr, dv.ptr)
+    got = np.concatenate([dk.read().reshape(rows, xw), dv.read().reshape(rows, xw)], axis=1).astype(np.float64)
+    normed = np.stack([orc.layernorm(r, gain, None) for r in memory]).astype(np.float64)
+    want, lost = normed @ w.astype(np.float64).T, np.abs(normed).sum(axis=1, keepdims=True) * 2.0 ** -134
+    rounding = 2e-6 * np.abs(normed) @ np.abs(w.astype(np.float64)).T + width * 2.0 ** -150
+    over = (np.abs(got - want) - rounding) / lost
+    print("largest loss, of half a smallest subnormal a term: %g" % over.max(), flush=True)
+    assert over.max() < 1.0
+    for d in (dmem, dk, dv):
+        d.free()
