@@ -15,6 +15,7 @@
 //   snake           x + sin(a x)^2 * (1 / (a + 1e-9)) on the first snake_channels rows, leaky ReLU (0.01) on the rest
 //                   (snake_row, src/backend.c:643-658).
 #include <limits.h>
+#include <stddef.h>
 
 #include <type_traits>
 
@@ -25,6 +26,8 @@ using namespace mynah;
 namespace {
 
 typedef f32x16 floatx16;
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short ushort8 __attribute__((ext_vector_type(8)));
 
 constexpr int kConvMaxKernel = 16;
 constexpr int kConvMaxHalo = 128;     // (kernel - 1) * dilation
@@ -47,6 +50,7 @@ struct ConvArgs {
     // channel-split tiles only: workgroups that share a tile's channels, and where each leaves its sums ([splits][out_ch][length])
     int splits = 1;
     float *parts = nullptr;
+    const uint4 *weights = nullptr;   // ConvBlocks data
 };
 
 // sin(x) in some twenty instructions for |x| < kShortSineLimit (the library routine, which also serves arguments of any
@@ -190,6 +194,39 @@ __device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, co
     }
 }
 
+// What a sum of pieces that is no finite number stands for (split_product.h): the chain of f32 multiply-adds, from `s`, over the channels
+// (eight, then the taps, then the next eight) of every block that mine(block) names.  w: the output row's first piece of the first block and
+// tap; inside(tap): whether the tap's position lies in the row; fetch(channel, tap, x): its eight inputs from that channel on.
+template <class Mine, class Inside, class Fetch>
+__device__ __forceinline__ float conv_chain(const uint4 *const w, const int channels, const int taps, const Mine mine, const Inside inside, const Fetch fetch, float s) {
+#pragma unroll 1
+    for (int c = 0; c < channels && s == s; c += 8) {
+        if (!mine(c >> 4)) continue;
+#pragma unroll 1
+        for (int tap = 0; tap < taps; ++tap) {
+            if (!inside(tap)) continue;
+            const uint4 *const at = w + (size_t)((c >> 4) * taps + tap) * 192 + ((c >> 3) & 1) * 32;
+            const ushort8 h = __builtin_bit_cast(ushort8, at[0]), m = __builtin_bit_cast(ushort8, at[64]), l = __builtin_bit_cast(ushort8, at[128]);
+            float x[8];
+            fetch(c, tap, x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (c + e < channels) s = __builtin_fmaf(split_value(h[e], m[e], l[e]), x[e], s);
+        }
+    }
+    return s;
+}
+// ... of a convolution's own input rows, at output position t of row `row` of a tile.
+template <class Mine>
+__device__ __forceinline__ float conv_chain_rows(const ConvArgs &a, const uint4 *const tile, const int row, const int t, const Mine mine, const float s) {
+    const int back = (a.kernel - 1) * a.dilation;
+    return conv_chain(tile + (row & 31), a.in_ch, a.kernel, mine, [&](int tap) { return t - back + tap * a.dilation >= 0; },
+                      [&](int c, int tap, float (&x)[8]) {
+#pragma unroll
+                          for (int e = 0; e < 8; ++e) x[e] = a.in[(size_t)min(c + e, a.in_ch - 1) * a.length + t - back + tap * a.dilation];
+                      }, s);
+}
+
 // One (position, eight channels) on its way to LDS: eight requests, then the pieces of the eight values.
 struct ConvColumn {
     float v[8];
@@ -211,15 +248,47 @@ struct ConvColumn {
     }
 };
 
+// What is hardly ever run of the tiles below, as calls of their own with the arguments read from memory once more: inline, their
+// registers came on top of the products' (11 taps: 4 to 11 % of a call, some of it spilled; 0.6 us of every call for the arguments).
+//
+// conv_tile's values of one position through the loop over its rows: conv_chain for a sum that is no finite number, and the library's sine.
+__device__ __noinline__ void conv_tile_rest(const ConvArgs *const args, const float *s_tile, const float *const s_alpha, const int m_first, const int rows, const int t) {
+    const ConvArgs a = *args;
+#pragma unroll 1
+    for (int row = 0; row < rows; ++row, s_tile += kTileStride) {
+        const int m = m_first + row;
+        const size_t index = (size_t)m * a.length + t;
+        float v = *s_tile;
+        if (!split_finite(v))
+            v = conv_combine(a, index, conv_chain_rows(a, a.weights + (size_t)(m >> 5) * ((a.in_ch + 15) / 16) * a.kernel * 192, m & 31, t, [](int) { return true; },
+                                                       a.bias != nullptr ? a.bias[m] : 0.0f));
+        conv_emit(a, m, index, v, s_alpha[row], s_alpha[32 + row]);
+    }
+}
+// conv_split_tile's partial sums of a thread's eight values (see there), the first taking the whole where it is no finite number.
+__device__ __noinline__ void conv_split_rest(const ConvArgs *const args, float *const s_part, const int split, const int m0, const int t) {
+    const ConvArgs a = *args;
+    const int tid = threadIdx.x, pos = tid & 63;
+#pragma unroll 1
+    for (int j = 0; j < 8; ++j) {
+        const int row = (tid >> 6) + 4 * j, m = m0 + row;
+        float *const at = s_part + ((((row >> 3) << 2) | (row & 3)) + 16 * (pos >> 5)) * 64 + ((row >> 2) & 1) * 32 + (pos & 31);
+        if (m >= a.out_ch || split_finite(((at[0] + at[2048]) + at[4096]) + at[6144])) continue;
+        at[0] = conv_chain_rows(a, a.weights + (size_t)(m >> 5) * ((a.in_ch + 15) / 16) * a.kernel * 192, row, t, [&](int block) { return block % (4 * a.splits) / 4 == split; }, 0.0f);
+        at[2048] = at[4096] = at[6144] = 0.0f;
+    }
+}
+
 // Workgroup tile: (32 * WM) output channels x (64 * WN) positions; a wavefront owns 32 x 64 (two 32 x 32 accumulators).
 // KF: number of taps known at compile time (0 = from the arguments); the codec's 3, 7 and 11 taps get such builds.
 // FUSED: the build that mynah_hip_conv1d_fused launches (residuals, scale, activation after the products); the seam's
 // conv1d keeps a build without any of it.
 // Two stages of one block of channels: a block is stored while the one before it is multiplied (by other wavefronts: three
 // to a SIMD), its requests leave a block earlier.
-// (the tile's work as a function: the kernel of one convolution and the kernel of several side by side both run it)
+// (the tile's work as a function: the kernel of one convolution and the kernel of several side by side both run it; `again`: the
+// arguments as they lie in memory, for conv_tile_rest)
 template <int WM, int WN, int KF, bool FUSED>
-__device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, uint4 *const lds) {
+__device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, const ConvArgs *const again, uint4 *const lds) {
     constexpr int TM = 32 * WM, TN = 64 * WN;
     ConvArgs a = a_arg;
     if constexpr (KF != 0) a.kernel = KF;
@@ -339,58 +408,66 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
             acc0[r] = v0;
             acc1[r] = v1;
         }
-        if (!FUSED || !a.activate) store_tile(a.out, acc0, acc1);
     };
-    if constexpr (!FUSED) {   // the seam's conv1d
-        combine(std::false_type{}, std::false_type{});
+    const bool finite = FUSED && (a.activate || split_all_finite(acc));   // (here, while the residual's values are on their way)
+    if constexpr (FUSED) {
+        if (a.residual2 != nullptr) combine(std::true_type{}, std::true_type{});    // the launch refuses a second residual without a first
+        else if (a.residual != nullptr) combine(std::true_type{}, std::false_type{});
+        else combine(std::false_type{}, std::false_type{});
+    }
+    if constexpr (!FUSED) {   // the seam's conv1d; what is no finite number is stored once more below
+        store_tile(a.out, acc0, acc1);
+        if (split_all_finite(acc)) return;
+    } else if (!a.activate && finite) {
+        store_tile(a.out, acc0, acc1);
         return;
     }
-    if (a.residual2 != nullptr) combine(std::true_type{}, std::true_type{});    // the launch refuses a second residual without a first
-    else if (a.residual != nullptr) combine(std::true_type{}, std::false_type{});
-    else combine(std::false_type{}, std::false_type{});
-    if (!a.activate) return;
     // The rows' alphas and 1 / (alpha + 1e-9) through the wavefront's own piece of LDS (free after the last products' barrier)
     float *s_alpha = reinterpret_cast<float *>(lds) + 4 * (32 * kTileStride) + wave * 64;
-    if (lane < 32) {
-        const int m = m0 + wm * 32 + lane;
-        const float al = m < a.snake_channels ? a.alpha[m] : 0.0f;
-        s_alpha[lane] = al;
-        s_alpha[32 + lane] = 1.0f / (al + 1e-9f);
-    }
-    // Common case, every sine argument below the short routine's limit: the activation on the values where they are, in
-    // registers, the short sine inlined 32 times and no branch among them.
-    bool large = false;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const float al = s_alpha[8 * (r >> 2) + 4 * half + (r & 3)];
-        large = large || !(fabsf(al * acc0[r]) < kShortSineLimit) || !(fabsf(al * acc1[r]) < kShortSineLimit);
-    }
-    if (!__any(large)) {
-        floatx16 act0, act1;
+    if (FUSED && a.activate) {
+        if (lane < 32) {
+            const int m = m0 + wm * 32 + lane;
+            const float al = m < a.snake_channels ? a.alpha[m] : 0.0f;
+            s_alpha[lane] = al;
+            s_alpha[32 + lane] = 1.0f / (al + 1e-9f);
+        }
+        // Common case, every sine argument below the short routine's limit: the activation on the values where they are, in
+        // registers, the short sine inlined 32 times and no branch among them.  (A sum that is no finite number is not below it
+        // either, whatever the alpha.)
+        bool large = false;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int row = 8 * (r >> 2) + 4 * half + (r & 3), m = m0 + wm * 32 + row;
-            const float al = s_alpha[row], inv_a = s_alpha[32 + row];
-            const float v0 = acc0[r], v1 = acc1[r];
-            act0[r] = v0 < 0.0f ? v0 * 0.01f : v0;
-            act1[r] = v1 < 0.0f ? v1 * 0.01f : v1;
-            if (m0 + wm * 32 + 8 * (r >> 2) < a.snake_channels) {   // (else no lane's row of these registers is a snake row: half of all)
-                const float s0 = short_sine(al * v0), s1 = short_sine(al * v1);
-                const bool snake_row = m < a.snake_channels;
-                act0[r] = snake_row ? v0 + s0 * s0 * inv_a : act0[r];
-                act1[r] = snake_row ? v1 + s1 * s1 * inv_a : act1[r];
+            const float al = s_alpha[8 * (r >> 2) + 4 * half + (r & 3)];
+            large = large || !(fabsf(al * acc0[r]) < kShortSineLimit) || !(fabsf(al * acc1[r]) < kShortSineLimit);
+        }
+        if (!__any(large)) {
+            floatx16 act0, act1;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = 8 * (r >> 2) + 4 * half + (r & 3), m = m0 + wm * 32 + row;
+                const float al = s_alpha[row], inv_a = s_alpha[32 + row];
+                const float v0 = acc0[r], v1 = acc1[r];
+                act0[r] = v0 < 0.0f ? v0 * 0.01f : v0;
+                act1[r] = v1 < 0.0f ? v1 * 0.01f : v1;
+                if (m0 + wm * 32 + 8 * (r >> 2) < a.snake_channels) {   // (else no lane's row of these registers is a snake row: half of all)
+                    const float s0 = short_sine(al * v0), s1 = short_sine(al * v1);
+                    const bool snake_row = m < a.snake_channels;
+                    act0[r] = snake_row ? v0 + s0 * s0 * inv_a : act0[r];
+                    act1[r] = snake_row ? v1 + s1 * s1 * inv_a : act1[r];
+                }
             }
+            if (a.act_out != nullptr) {
+                store_tile(a.out, acc0, acc1);
+                store_tile(a.act_out, act0, act1);
+            } else {
+                store_tile(a.out, act0, act1);
+            }
+            return;
         }
-        if (a.act_out != nullptr) {
-            store_tile(a.out, acc0, acc1);
-            store_tile(a.act_out, act0, act1);
-        } else {
-            store_tile(a.out, act0, act1);
-        }
-        return;
     }
-    // Some argument needs the library's sine: the wavefront's 32 x 64 tile goes through LDS and a rolled loop finishes it
-    // a row at a time, with one copy of that long routine.
+    // Some argument needs the library's sine, or some sum is no finite number: the wavefront's 32 x 64 tile goes through LDS and a rolled
+    // loop finishes it a row at a time, with one copy of that long routine.  (Nothing of a fused tile has been stored: a residual that is
+    // the output is still there to be added again.)
     float *s_tile = reinterpret_cast<float *>(lds) + wave * (32 * kTileStride);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -401,14 +478,24 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
     const int t = t0 + wn * 64 + lane;
     if (t >= a.length) return;
     const int rows = min(32, a.out_ch - (m0 + wm * 32));   // the same for the whole wavefront
-    size_t index = (size_t)(m0 + wm * 32) * a.length + t;
-#pragma unroll 1
-    for (int row = 0; row < rows; ++row, index += a.length)
-        conv_emit(a, m0 + wm * 32 + row, index, s_tile[row * kTileStride + lane], s_alpha[row], s_alpha[32 + row]);
+    conv_tile_rest(again, s_tile + lane, s_alpha, m0 + wm * 32, rows, t);
 }
 
 // (the rows, the weights and the shape lead the arguments and repeat fields of a_arg: leading scalar arguments are in registers
 // when a wavefront starts, a structure passed by value is fetched from memory where its fields are first used)
+struct ConvKernarg {
+    const float *in;
+    float *out;
+    const uint4 *weights;
+    const float *bias;
+    int in_ch, out_ch, length, kernel, dilation, tiles;
+    ConvArgs a;
+};
+static_assert(offsetof(ConvKernarg, a) == 56 && alignof(ConvArgs) == 8, "the kernels' argument lists");
+// A kernel's arguments where they lie (one structure of them, or the arguments of k_conv1d and k_conv1d_split in order).
+template <class T>
+__device__ __forceinline__ const T *conv_kernarg() { return (const T *)__builtin_amdgcn_kernarg_segment_ptr(); }
+
 template <int WM, int WN, int KF, bool FUSED>
 __global__ void __launch_bounds__(256, 3) k_conv1d(const float *const in_arg, float *const out_arg, const uint4 *const weights_arg, const float *const bias_arg, const int in_ch_arg,
                                                    const int out_ch_arg, const int length_arg, const int kernel_arg, const int dilation_arg, const int tiles_arg,
@@ -417,7 +504,7 @@ __global__ void __launch_bounds__(256, 3) k_conv1d(const float *const in_arg, fl
     ConvArgs a = a_arg;
     a.in = in_arg; a.out = out_arg; a.bias = bias_arg; a.in_ch = in_ch_arg; a.out_ch = out_ch_arg; a.length = length_arg;
     a.kernel = kernel_arg; a.dilation = dilation_arg;
-    conv_tile<WM, WN, KF, FUSED>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, lds);
+    conv_tile<WM, WN, KF, FUSED>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, &conv_kernarg<ConvKernarg>()->a, lds);
 }
 
 // The same product for short rows (few positions, many channels: the codec's first stages), where 64 x 128 tiles would
@@ -429,7 +516,7 @@ __global__ void __launch_bounds__(256, 3) k_conv1d(const float *const in_arg, fl
 // a.splits > 1: that many workgroups share the tile's channels (wavefront w of workgroup s is wavefront 4 s + w of them all), each
 // leaves its sum in a.parts, and k_conv_finish adds them in order and does what is left.
 template <int KF, int NT, int PARTS>
-__device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, uint4 *const lds) {
+__device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, const ConvArgs *const again, uint4 *const lds) {
     constexpr int TM = 32, TN = 32 * NT;
     ConvArgs a = a_arg;
     if constexpr (KF != 0) a.kernel = KF;
@@ -491,18 +578,31 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
     const int pos = tid & 63;
     const int t = t0 + pos;
     const bool t_ok = (NT > 1 || pos < 32) && t < a.length;
+    float sum[8], zero = 0.0f;
+    const auto add_parts = [&]() {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int row = (tid >> 6) + 4 * j;
+            const int e = ((((row >> 3) << 2) | (row & 3)) + 16 * (pos >> 5)) * 64 + ((row >> 2) & 1) * 32 + (pos & 31);
+            sum[j] = ((s_part[e] + s_part[2048 + e]) + s_part[4096 + e]) + s_part[6144 + e];
+            zero = __builtin_fmaf(sum[j], 0.0f, zero);
+        }
+    };
+    add_parts();
+    if (__any(t_ok && zero != 0.0f)) {   // (see split_all_finite)
+        if (t_ok) conv_split_rest(again, s_part, split, m0, t);
+        add_parts();
+    }
     float value[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int row = (tid >> 6) + 4 * j, m = m0 + row;
-        const int e = ((((row >> 3) << 2) | (row & 3)) + 16 * (pos >> 5)) * 64 + ((row >> 2) & 1) * 32 + (pos & 31);
-        const float sum = ((s_part[e] + s_part[2048 + e]) + s_part[4096 + e]) + s_part[6144 + e];
         value[j] = 0.0f;
         if (a.splits > 1) {
-            if (t_ok && m < a.out_ch) a.parts[((size_t)split * a.out_ch + m) * a.length + t] = sum;
+            if (t_ok && m < a.out_ch) a.parts[((size_t)split * a.out_ch + m) * a.length + t] = sum[j];
             continue;
         }
-        if (t_ok && m < a.out_ch) value[j] = conv_combine(a, (size_t)m * a.length + t, sum + (a.bias != nullptr ? a.bias[m] : 0.0f));
+        if (t_ok && m < a.out_ch) value[j] = conv_combine(a, (size_t)m * a.length + t, sum[j] + (a.bias != nullptr ? a.bias[m] : 0.0f));
     }
     if (a.splits > 1) return;
     if (!a.activate) {
@@ -540,7 +640,7 @@ __global__ void __launch_bounds__(256, 2) k_conv1d_split(const float *const in_a
     ConvArgs a = a_arg;
     a.in = in_arg; a.out = out_arg; a.bias = bias_arg; a.in_ch = in_ch_arg; a.out_ch = out_ch_arg; a.length = length_arg;
     a.kernel = kernel_arg; a.dilation = dilation_arg;
-    conv_split_tile<KF, NT, PARTS>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, lds);
+    conv_split_tile<KF, NT, PARTS>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, &conv_kernarg<ConvKernarg>()->a, lds);
 }
 
 // Several convolutions of one shape side by side in one launch (the three branches of a residual layer: same rows in and
@@ -562,9 +662,9 @@ __global__ void __launch_bounds__(256, 3) k_conv1d_batch(const ConvBatchArgs b) 
     extern __shared__ __align__(16) uint4 lds[];
     const int z = b.order[blockIdx.z];
     switch (b.item[z].kernel) {
-        case 3: conv_tile<WM, WN, 3, true>(b.item[z], b.weights[z], lds); break;
-        case 7: conv_tile<WM, WN, 7, true>(b.item[z], b.weights[z], lds); break;
-        default: conv_tile<WM, WN, 11, true>(b.item[z], b.weights[z], lds); break;
+        case 3: conv_tile<WM, WN, 3, true>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        case 7: conv_tile<WM, WN, 7, true>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        default: conv_tile<WM, WN, 11, true>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
     }
 }
 
@@ -573,9 +673,9 @@ __global__ void __launch_bounds__(256, 2) k_conv1d_split_batch(const ConvBatchAr
     extern __shared__ __align__(16) uint4 lds[];
     const int z = b.order[blockIdx.z];
     switch (b.item[z].kernel) {
-        case 3: conv_split_tile<3, NT, PARTS>(b.item[z], b.weights[z], lds); break;
-        case 7: conv_split_tile<7, NT, PARTS>(b.item[z], b.weights[z], lds); break;
-        default: conv_split_tile<11, NT, PARTS>(b.item[z], b.weights[z], lds); break;
+        case 3: conv_split_tile<3, NT, PARTS>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        case 7: conv_split_tile<7, NT, PARTS>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        default: conv_split_tile<11, NT, PARTS>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
     }
 }
 
@@ -620,10 +720,8 @@ struct ResArgs {
     int channels, length, snake_channels, blocks, tiles;
 };
 
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-
 template <int WM, int WN, int NT, bool SPLIT, int KF>
-__device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember &m, uint4 *const lds, float2 *const s_pairs) {
+__device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember &m, uint4 *const lds, float4 *const s_pairs) {
     constexpr int WP = 32 * NT, RN = WP * WN, T = 64 * WM * WN, TN = RN - (KF - 1);
     const int t0 = blockIdx.x * TN;
     if (t0 >= a.length) return;
@@ -690,7 +788,12 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
             for (int q = 0; q < 3; ++q) stage[(q * 2 + group_of(x)) * win + place[x]] = __builtin_bit_cast(uint4, p[q]);
         }
     };
-    if (tid < kResMaxChannels) s_pairs[tid] = tid < a.snake_channels ? m.snake_skip[tid] : make_float2(0.0f, 0.0f);
+    // the inner rows' alphas, 1 / (alpha + 1e-9), and what a value is multiplied by to be told from those that need the long way: the
+    // library's sine, or (no finite number, or none that three pieces add up to) more than that
+    if (tid < kResMaxChannels) {
+        const float2 pair = tid < a.snake_channels ? m.snake_skip[tid] : make_float2(0.0f, 0.0f);
+        s_pairs[tid] = make_float4(pair.x, pair.y, fmaxf(fabsf(pair.x), 1.01f * (kShortSineLimit / kSplitLimit)), 0.0f);
+    }
 
     // the rows' biases, which the sums start from: both convolutions' requested here, none under a condition
     float bias_in[16], bias_skip[16];
@@ -762,18 +865,18 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
     for (int i = 0; i < 32 / kRowsAtOnce; ++i) x[i] = m.in[at_out + (size_t)max(min(row0 + kRowsAtOnce * i, rows - 1), 0) * a.length];
     // the inner rows: activated, zero in front of the first position, in pieces to LDS where the second convolution reads them
     ConvWeights w2(m.w_skip + w_at, 0, 1, KF);
-    bool large = false;
+    bool large = false, kept = false;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-        const float al = s_pairs[wm * 32 + split_acc_row(r, lane)].x;
+        const float bound = s_pairs[wm * 32 + split_acc_row(r, lane)].z;
 #pragma unroll
-        for (int n = 0; n < NT; ++n) large = large || !(fabsf(al * acc[n][r]) < kShortSineLimit);
+        for (int n = 0; n < NT; ++n) large = large || !(fabsf(bound * acc[n][r]) < kShortSineLimit);
     }
     if (!__any(large)) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row = wm * 32 + split_acc_row(r, lane);
-            const float2 pair = s_pairs[row];
+            const float4 pair = s_pairs[row];
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
                 const float v = acc[n][r];
@@ -789,10 +892,30 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
 #pragma unroll 1
         for (int r = 0; r < 16; ++r) {
             const int row = wm * 32 + split_acc_row(r, lane);
-            const float2 pair = s_pairs[row];
+            const float4 pair = s_pairs[row];
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n][r] = half_snake(acc[n][r], row < a.snake_channels, pair.x, pair.y);
+            for (int n = 0; n < NT; ++n) {
+                const int t = t0 - (KF - 1) + wn * WP + 32 * n + col;
+                float v = acc[n][r];
+                if (row < a.channels && t >= 0 && t < a.length && !split_finite(SPLIT ? sum[SPLIT ? n : 0][r] : v)) {
+                    const float bias = m.b_in != nullptr ? m.b_in[row] : 0.0f;
+                    v = conv_chain(m.w_in + (w_at - lane) + (row & 31), a.channels, KF, [](int) { return true; }, [&](int tap) { return t - halo + tap * m.dilation >= 0; },
+                                   [&](int c, int tap, float (&x)[8]) {
+#pragma unroll 1
+                                       for (int e = 0; e < 8; ++e) {
+                                           const int channel = min(c + e, a.channels - 1);
+                                           const float2 in_pair = channel < a.snake_channels ? m.snake_in[channel] : make_float2(0.0f, 0.0f);
+                                           x[e] = half_snake(m.in[(size_t)channel * a.length + t - halo + tap * m.dilation], channel < a.snake_channels, in_pair.x, in_pair.y);
+                                       }
+                                   }, SPLIT ? 0.0f : bias);
+                    if (SPLIT) v = v + bias;
+                }
+                v = row < a.channels ? half_snake(v, row < a.snake_channels, pair.x, pair.y) : 0.0f;
+                kept = kept || !(fabsf(v) < kSplitLimit);
+                acc[n][r] = v;
+            }
         }
+        kept = __any(kept);
     }
     __syncthreads();   // the stages have been read
 #pragma unroll
@@ -804,7 +927,8 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
             const int block = wm * 2 + (g >> 1);
             if (block >= a.blocks) continue;
             const float4 v = make_float4(acc[n][4 * g], acc[n][4 * g + 1], acc[n][4 * g + 2], acc[n][4 * g + 3]);
-            const SplitFour s(in_front ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : v);
+            SplitFour s(in_front ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : v);
+            if (kept && !in_front) s.keep_bits(v);   // (the rows themselves are nowhere else)
 #pragma unroll
             for (int q = 0; q < 3; ++q) reinterpret_cast<uint2 *>(&lds[(block * 6 + q * 2 + (g & 1)) * RN + p])[half] = s.piece[q];
         }
@@ -816,6 +940,31 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
         return const_cast<const uint4 *>(lds + (block * 6 + half) * RN + wn * WP + col);
     }, acc);
     finish(bias_skip);
+    bool finite;
+    if constexpr (SPLIT) finite = split_all_finite(sum);
+    else finite = split_all_finite(acc);
+    if (!finite) {
+#pragma unroll 1
+        for (int r = 0; r < 16; ++r) {
+            const int row = wm * 32 + split_acc_row(r, lane);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const int p = wn * WP + 32 * n + col, t = t0 + p;
+                if (row >= a.channels || p >= TN || t >= a.length || split_finite(SPLIT ? sum[SPLIT ? n : 0][r] : acc[n][r])) continue;
+                const float bias = m.b_skip != nullptr ? m.b_skip[row] : 0.0f;
+                const float v = conv_chain(m.w_skip + (w_at - lane) + (row & 31), a.channels, KF, [](int) { return true; },
+                                           [&](int tap) { return t - (KF - 1) + tap >= 0; },
+                                           [&](int c, int tap, float (&x)[8]) {
+                                               const uint4 *const at = lds + ((c >> 4) * 6 + ((c >> 3) & 1)) * RN + p + tap;
+                                               const ushort8 xh = __builtin_bit_cast(ushort8, at[0]), xm = __builtin_bit_cast(ushort8, at[2 * RN]),
+                                                             xl = __builtin_bit_cast(ushort8, at[4 * RN]);
+#pragma unroll
+                                               for (int e = 0; e < 8; ++e) x[e] = split_value(xh[e], xm[e], xl[e]);
+                                           }, SPLIT ? 0.0f : bias);
+                acc[n][r] = SPLIT ? v + bias : v;
+            }
+        }
+    }
 
     // + x, and out, in whole rows (see store_tile of conv_tile)
     __syncthreads();   // the inner rows have been read
@@ -836,7 +985,7 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
 template <int WM, int WN, int NT, bool SPLIT>
 __global__ void __launch_bounds__(64 * WM * WN, 2) k_res_block(const ResArgs a) {
     extern __shared__ __align__(16) uint4 lds[];
-    __shared__ float2 s_pairs[kResMaxChannels];
+    __shared__ float4 s_pairs[kResMaxChannels];
     const int z = a.order[blockIdx.y];
     switch (a.member[z].kernel) {
         case 3: res_block_tile<WM, WN, NT, SPLIT, 3>(a, a.member[z], lds, s_pairs); break;
@@ -882,8 +1031,19 @@ __global__ void __launch_bounds__(256) k_conv_pack(const float *src, uint4 *dst,
     for (int e = 0; e < 8; ++e) v[e] = o < (size_t)out_ch && c0 + e < in_ch ? src[(o * in_ch + c0 + e) * kernel + tap] : 0.0f;
     bf16x8 p[3];
     split_eight(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]), p);
+    ushort8 at[3];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) dst[step * 192 + q * 64 + lane] = __builtin_bit_cast(uint4, p[q]);
+    for (int q = 0; q < 3; ++q) at[q] = __builtin_bit_cast(ushort8, p[q]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {   // (the kernels have no other copy of a weight)
+        unsigned short h = at[0][e], m = at[1][e], l = at[2][e];
+        split_keep_bits(v[e], h, m, l);
+        at[0][e] = h;
+        at[1][e] = m;
+        at[2][e] = l;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) dst[step * 192 + q * 64 + lane] = __builtin_bit_cast(uint4, at[q]);
 }
 
 struct ConvTransposeArgs {
@@ -1179,6 +1339,7 @@ static int conv1d_prepare(State *st, int member, const float *dev_input, float *
             a.parts = st->conv_parts + (size_t)member * floats;
         }
     }
+    a.weights = weights.data;
     *out_args = a;
     *out_weights = weights;
     return 0;

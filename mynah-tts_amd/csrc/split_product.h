@@ -32,37 +32,7 @@ __device__ __forceinline__ unsigned bf16_pair(float a, float b) {   // one instr
 __device__ __forceinline__ float bf16_low(unsigned p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float bf16_high(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
 
-// The three pieces of four neighbouring values, 8 bytes each (22 vector instructions).
-struct SplitFour {
-    uint2 piece[3];
-    __device__ __forceinline__ explicit SplitFour(const float4 v) {
-        const unsigned h0 = bf16_pair(v.x, v.y), h1 = bf16_pair(v.z, v.w);
-        const float x = v.x - bf16_low(h0), y = v.y - bf16_high(h0), z = v.z - bf16_low(h1), w = v.w - bf16_high(h1);
-        const unsigned m0 = bf16_pair(x, y), m1 = bf16_pair(z, w);
-        piece[0] = make_uint2(h0, h1);
-        piece[1] = make_uint2(m0, m1);
-        piece[2] = make_uint2(bf16_pair(x - bf16_low(m0), y - bf16_high(m0)), bf16_pair(z - bf16_low(m1), w - bf16_high(m1)));
-    }
-};
-// ... of eight: one operand of a matrix instruction per piece.
-__device__ __forceinline__ void split_eight(const float4 a, const float4 b, bf16x8 (&out)[3]) {
-    const SplitFour x(a), y(b);
-#pragma unroll
-    for (int p = 0; p < 3; ++p) out[p] = __builtin_bit_cast(bf16x8, make_uint4(x.piece[p].x, x.piece[p].y, y.piece[p].x, y.piece[p].y));
-}
-
 constexpr float kSplitLimit = 0x1.ffp127f;   // bf16 rounds what is not below it to infinity
-__device__ __forceinline__ bool split_finite(float x) { return fabsf(x) < __builtin_inff(); }
-// Whether all sums of the wavefront are finite (one instruction a value: 0 * x is 0 or NaN).
-template <int N>
-__device__ __forceinline__ bool split_all_finite(const f32x16 (&acc)[N]) {
-    float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int n = 0; n < N; ++n)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) zero[r & 3] = __builtin_fmaf(acc[n][r], 0.0f, zero[r & 3]);
-    return !__any((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.0f);
-}
 // Where pieces are all that is kept of an operand, one from kSplitLimit on is kept as (infinity, upper half, lower half of its bits): it
 // makes its products infinite or NaN as it must, and can be had again.  piece: 16 bits each, as they lie in memory.
 __device__ __forceinline__ void split_keep_bits(float x, unsigned short &h, unsigned short &m, unsigned short &l) {
@@ -76,6 +46,53 @@ __device__ __forceinline__ float split_value(unsigned short h, unsigned short m,
     return __uint_as_float((unsigned)h << 16) + (__uint_as_float((unsigned)m << 16) + __uint_as_float((unsigned)l << 16));   // exact
 }
 
+// The three pieces of four neighbouring values, 8 bytes each (22 vector instructions).
+struct SplitFour {
+    uint2 piece[3];
+    __device__ __forceinline__ explicit SplitFour(const float4 v) {
+        const unsigned h0 = bf16_pair(v.x, v.y), h1 = bf16_pair(v.z, v.w);
+        const float x = v.x - bf16_low(h0), y = v.y - bf16_high(h0), z = v.z - bf16_low(h1), w = v.w - bf16_high(h1);
+        const unsigned m0 = bf16_pair(x, y), m1 = bf16_pair(z, w);
+        piece[0] = make_uint2(h0, h1);
+        piece[1] = make_uint2(m0, m1);
+        piece[2] = make_uint2(bf16_pair(x - bf16_low(m0), y - bf16_high(m0)), bf16_pair(z - bf16_low(m1), w - bf16_high(m1)));
+    }
+    __device__ __forceinline__ void keep_bits(const float4 v) {
+        typedef unsigned short ushort4_t __attribute__((ext_vector_type(4)));
+        const float x[4] = {v.x, v.y, v.z, v.w};
+        ushort4_t at[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) at[q] = __builtin_bit_cast(ushort4_t, piece[q]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            unsigned short h = at[0][e], m = at[1][e], l = at[2][e];
+            split_keep_bits(x[e], h, m, l);
+            at[0][e] = h;
+            at[1][e] = m;
+            at[2][e] = l;
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) piece[q] = __builtin_bit_cast(uint2, at[q]);
+    }
+};
+// ... of eight: one operand of a matrix instruction per piece.
+__device__ __forceinline__ void split_eight(const float4 a, const float4 b, bf16x8 (&out)[3]) {
+    const SplitFour x(a), y(b);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) out[p] = __builtin_bit_cast(bf16x8, make_uint4(x.piece[p].x, x.piece[p].y, y.piece[p].x, y.piece[p].y));
+}
+
+__device__ __forceinline__ bool split_finite(float x) { return fabsf(x) < __builtin_inff(); }
+// Whether all sums of the wavefront are finite (one instruction a value: 0 * x is 0 or NaN).
+template <int N>
+__device__ __forceinline__ bool split_all_finite(const f32x16 (&acc)[N]) {
+    float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zero[r & 3] = __builtin_fmaf(acc[n][r], 0.0f, zero[r & 3]);
+    return !__any((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.0f);
+}
 // One 16-deep step: acc += a * w over the six pairs, the smallest first.
 __device__ __forceinline__ f32x16 split_multiply(const bf16x8 (&a)[3], const bf16x8 (&w)[3], f32x16 acc) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], w[0], acc, 0, 0, 0);

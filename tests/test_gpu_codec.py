@@ -450,3 +450,87 @@ def test_error_paths(pkg, backend):
         backend.conv1d_fused(d.ptr, e.ptr, 1, 1, 8, 3, 1, w3, alpha=np.ones(2, np.float32), snake_channels=2)
     e.free()
     d.free()
+
+
+def _conv_multiply_adds(x, w, b, dilation):
+    """The convolution as f32 multiply-adds (eight channels, the taps, the next eight), taps in front of the row left out."""
+    out_ch, in_ch, kernel = w.shape
+    length = x.shape[1]
+    want = np.zeros((out_ch, length), np.float32) + b[:, None]
+    for c0 in range(0, in_ch, 8):
+        for k in range(kernel):
+            back = min((kernel - 1 - k) * dilation, length)
+            for c in range(c0, min(c0 + 8, in_ch)):
+                want[:, back:] = want[:, back:].astype(np.float64) + w[:, c, k].astype(np.float64)[:, None] * x[c, :length - back].astype(np.float64)[None]
+    return want
+
+
+# large tiles (two shapes), channels split over the wavefronts, and over workgroups, each with straight-line taps and any
+@pytest.mark.parametrize("C,O,L,K,D", [(20, 70, 300, 7, 3), (27, 27, 500, 11, 1), (27, 30, 90, 4, 2), (40, 48, 300, 3, 5), (33, 65, 129, 4, 1), (432, 100, 32, 3, 1),
+                                       (150, 70, 70, 5, 2)])
+def test_conv1d_extremes(backend, C, O, L, K, D):
+    """Infinite, NaN and largest operands, in the rows and in the weights: what f32 multiply-adds give, and only in the outputs they enter.
+    (An input channel that the last block of sixteen repeats, the first and the last position and output channel are among them.)"""
+    _announce("conv1d extremes %d -> %d x %d, %d taps" % (C, O, L, K))
+    rng = np.random.default_rng(C + L)
+    x = rng.standard_normal((C, L)).astype(np.float32)
+    w = (rng.standard_normal((O, C, K)) / np.sqrt(C * K)).astype(np.float32)
+    b = rng.standard_normal(O).astype(np.float32)
+    x[C - 1, 3], x[2, L // 2], x[0, L // 2 + 5], x[1, L - 1] = np.inf, -np.inf, np.nan, 3.4e38
+    x[C - 1, 0], x[3, L // 3] = 3.4e38, -3.4028235e38
+    w[4, 5, K - 1], w[5, C - 1, 0], w[O - 1, 7, K // 2], b[6] = np.inf, np.nan, 3.4e38, -np.inf
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = _conv_multiply_adds(x, w, b, D).astype(np.float64)
+        size = _conv_multiply_adds(np.abs(np.nan_to_num(x, posinf=0, neginf=0)), np.abs(np.nan_to_num(w, posinf=0)), np.abs(np.nan_to_num(b, neginf=0)), D).astype(np.float64)
+    got = _run_conv1d(backend, x, w, b, D).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    finite = np.isfinite(want)
+    assert finite.mean() > 0.5 and (np.abs(want[finite]) > 1e36).any()
+    assert (np.abs(got[finite] - want[finite]) <= 1e-5 * np.minimum(size[finite], 3.4e38)).all()
+    # with an epilogue: the separate operators on the same values, the residual in place
+    n = O * L
+    r, alpha = rng.standard_normal((O, L)).astype(np.float32), (np.abs(rng.standard_normal(O // 2)) + 0.1).astype(np.float32)
+    din, plain, fused, act = backend.alloc(x.size).write(x), backend.alloc(n), backend.alloc(n).write(r), backend.alloc(n)
+    backend.conv1d(din.ptr, plain.ptr, C, O, L, K, D, w, b)
+    dres = backend.alloc(n).write(r)
+    backend.residual_inplace(dres.ptr, plain.ptr, n)
+    backend.conv1d_fused(din.ptr, fused.ptr, C, O, L, K, D, w, b, residual=fused.ptr, alpha=alpha, snake_channels=O // 2, activated=act.ptr)
+    assert np.array_equal(fused.read(), dres.read(), equal_nan=True)
+    fused.write(r)
+    backend.conv1d_fused(din.ptr, fused.ptr, C, O, L, K, D, w, b, residual=fused.ptr)
+    assert np.array_equal(fused.read(), dres.read(), equal_nan=True)
+    backend.snake_dev(dres.ptr, alpha, O, L, O // 2)
+    assert np.array_equal(act.read(), dres.read(), equal_nan=True)
+    for d in (din, plain, fused, act, dres):
+        d.free()
+
+
+# each build of the one-launch block, and a layer of two launches a position
+@pytest.mark.parametrize("C,L,taps", [(27, 700, (3, 7, 11)), (27, 20786, (3, 7, 11)), (64, 2689, (3, 7, 11)), (54, 12161, (3, 7, 11)), (108, 6017, (11,)), (108, 500, (3, 7, 11))])
+def test_res_layer_extremes(pkg, backend, C, L, taps):
+    """Infinite, NaN and largest values in a layer's input, weights and (by a weight of one) in its inner rows, which the one-launch block
+    keeps in three pieces alone: the operator sequence's values still."""
+    import importlib
+    codec = importlib.import_module(pkg.__name__ + ".codec")
+    _announce("residual layer extremes %d x %d taps %s" % (C, L, taps))
+    x, blocks = _res_layer_inputs(C, L, 300 + C, taps)
+    leaky = C - 2                                            # a channel without a sine
+    x[leaky, 40], x[1, 90], x[C - 1, 200], x[leaky, L - 1], x[leaky, 0] = 3.4e38, np.inf, np.nan, 3.4028235e38, -np.inf
+    for branch in blocks:
+        branch[0][1][0][leaky, leaky, :] = 1.0               # inner rows as large as the input's
+    blocks[0][2][3][0][2, 3, 0], blocks[-1][2][3][0][C - 1, 0, 1] = 3.399e38, np.inf
+    n, b = C * L, len(taps)
+    din = backend.alloc(n).write(x)
+    bufs = [backend.alloc(n) for _ in range(2 + max(4, 3 * b))]
+    at = [d.ptr for d in bufs]
+    for part in ([branch[:1] for branch in blocks], blocks):
+        codec.res_layer(backend, part, din.ptr, at[0], C, L, *at[2:6])
+        codec.res_layer_batched(backend, part, din.ptr, at[1], C, L, at[2:2 + b], at[2 + b:2 + 2 * b], at[2 + 2 * b:2 + 3 * b])
+        want, got = bufs[0].read().reshape(C, L), bufs[1].read().reshape(C, L)
+        assert np.array_equal(got, want, equal_nan=True)
+        assert np.isfinite(want).any() and not np.isfinite(want).all()
+    one = codec.res_layer(backend, [blocks[0][:1]], din.ptr, at[0], C, L, *at[2:6]) or bufs[0].read().reshape(C, L)
+    assert np.isfinite(one[:, 40:60]).any() and np.abs(one[:, 40:60][np.isfinite(one[:, 40:60])]).max() > 1e36   # (the large values are values)
+    for d in bufs + [din]:
+        d.free()
