@@ -263,7 +263,7 @@ int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch
     CachedWeight cw;
     cw.n = out_ch;
     cw.k = in_ch * kernel;
-    cw.bytes = (tiles * blocks + 5) * kernel * 3072 + kSplitWeightOverrun;   // (the kernels request up to five blocks past the end)
+    cw.bytes = (tiles * blocks * kernel + kConvStepsAhead) * 3072;   // (the kernels request that many steps past the last)
     if (stage_weight(st, host, out_ch * in_ch * kernel, error, capacity) != 0) return -1;
     MYNAH_TRY(hipMalloc(&cw.data, cw.bytes));
     if (launch_conv_pack(st, st->pack_staging, static_cast<uint4 *>(cw.data), out_ch, in_ch, kernel, error, capacity) != 0) {

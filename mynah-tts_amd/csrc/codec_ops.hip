@@ -116,7 +116,7 @@ __device__ __forceinline__ void conv_emit(const ConvArgs &a, int m, size_t index
 // (108 channels x 16384, taps 3 / 7 / 11 in one launch: 70 us with f32 instructions, which have the matrix cores busy for 59 us; the six
 // bf16 instructions of a step are busy for 24.)
 struct ConvWeights {   // the weight pieces of one row tile, requested kAhead steps before they are multiplied
-    static constexpr int kAhead = 3;
+    static constexpr int kAhead = kConvStepsAhead;
     const uint4 *next;
     size_t skip;       // from the end of a block to the next one this wavefront multiplies
     int blocks;        // it multiplies

@@ -862,11 +862,25 @@ __global__ void __launch_bounds__(256) k_enc_sum_gelu(const float4 *part, float4
 
 constexpr size_t kMaxSplitsF32 = 12;   // planes of partial sums; the next pass reads them all
 
+// The splits of a padded length's products, and the floats that their partial sums take.
+struct SplitsF32 {
+    int o, up, down;
+    size_t floats;
+    SplitsF32(const State *st, const mynah_hip_encoder *e, size_t rows) {
+        const size_t w = e->width, f = e->ffn;
+        o = split_product_splits(st, rows, w, w, kMaxSplitsF32);
+        up = split_product_splits(st, rows, w, f, kMaxSplitsF32);
+        down = split_product_splits(st, rows, f, w, kMaxSplitsF32);
+        const size_t narrow = (size_t)(o > down ? o : down) * w, wide = (size_t)up * f;
+        floats = rows * (narrow > wide ? narrow : wide);
+    }
+};
+
 int enqueue_prefill_f32(State *st, mynah_hip_encoder *e, int tpad, char *error, size_t capacity) {
     const size_t w = e->width, f = e->ffn, taps = e->taps, rows = (size_t)tpad;
     const float scale = 1.0f / sqrtf((float)e->head_width);
-    const int o_splits = split_product_splits(st, rows, w, w, kMaxSplitsF32), up_splits = split_product_splits(st, rows, w, f, kMaxSplitsF32),
-              down_splits = split_product_splits(st, rows, f, w, kMaxSplitsF32);
+    const SplitsF32 splits(st, e, rows);
+    const int o_splits = splits.o, up_splits = splits.up, down_splits = splits.down;
     const float *pending = nullptr;   // partial sums of the last product, not yet added to x
     for (size_t l = 0; l < e->layers; ++l) {
         if (l > 0) launch_rows<ROWS_F32>(st, (int)w, e->x, pending, down_splits, rows * w, e->n1g[l], e->n1b[l], e->f_nrm, e->params, tpad);
@@ -988,12 +1002,17 @@ extern "C" int mynah_hip_encoder_create(void *state, const mynah_hip_encoder_des
         return hip_check(hipMemsetAsync(*p, 0, bytes, st->stream), "encoder workspace clear", error, capacity);
     };
     if (e->f32) {
-        const size_t pad = kSplitOverrun, wide = (w > f ? w : f) * kMaxSplitsF32;
+        const size_t pad = kSplitOverrun;
+        size_t part = 0;   // (a product is split only as far as its tiles leave CUs idle: the most are not the longest rows')
+        for (size_t rows = kQTile; rows <= tp; rows += kQTile) {
+            const size_t floats = SplitsF32(st, e, rows).floats;
+            part = floats > part ? floats : part;
+        }
         if (alloc(reinterpret_cast<void **>(&e->x), tp * w * sizeof(float)) != 0 ||
             alloc(reinterpret_cast<void **>(&e->f_nrm_alloc), ((kLeadRows + tp) * w + pad) * sizeof(float)) != 0 ||
             alloc(reinterpret_cast<void **>(&e->f_qkv), tp * 3 * w * sizeof(float)) != 0 || alloc(reinterpret_cast<void **>(&e->f_ctx), (tp * w + pad) * sizeof(float)) != 0 ||
             alloc(reinterpret_cast<void **>(&e->f_hid_alloc), ((kLeadRows + tp) * f + pad) * sizeof(float)) != 0 ||
-            alloc(reinterpret_cast<void **>(&e->part), tp * wide * sizeof(float)) != 0 ||
+            alloc(reinterpret_cast<void **>(&e->part), part * sizeof(float)) != 0 ||
             alloc(reinterpret_cast<void **>(&e->params), sizeof(EncParams)) != 0)
             return fail();
         e->f_nrm = e->f_nrm_alloc + kLeadRows * w;   // rows -2 and -1 stay zero

@@ -183,3 +183,34 @@ def test_cross_kv_tiny_weights(backend, pkg, orc):
     assert over.max() < 1.0
     for d in (dmem, dk, dv):
         d.free()
+
+
+def test_workspace_and_weight_memory(backend, pkg, synth):
+    """What the encoder with f32 operands allocates follows the partial sums that its products can leave (tiles times splits are at most the
+    chip's CUs), and a packed convolution weight is its steps and the three that are requested ahead."""
+    import ctypes
+
+    def free():
+        values = ctypes.c_size_t(), ctypes.c_size_t()
+        assert backend.lib.hipMemGetInfo(ctypes.byref(values[0]), ctypes.byref(values[1])) == 0   # (the runtime that the library is linked to)
+        return values[0].value
+
+    print("[gpu-case] memory of the f32 encoder and of a convolution weight", flush=True)
+    cfg = dict(synth.encoder_config(layers=1, width=768, heads=12, ffn=3072, vocab=32, max_positions=1024), causal=True, ffn_kernel=1, operands_f32=True)
+    w = synth.encoder_weights_f16(cfg, seed=4, kernel=1)
+    backend.sync()
+    before, kept = free(), backend.cached_weight_bytes()
+    enc = pkg.Encoder(backend, cfg, w)
+    used = before - free() - (backend.cached_weight_bytes() - kept)
+    enc.destroy()
+    rows = 1024 * 4 * (4 * 768 + 2 * 768 + 3072)                             # x, normalised, context, q/k/v, hidden
+    partial = 4 * max(256 * 64 * 128, 1024 * 3072)
+    staging = 4 * 768 * 3072                                                 # the backend's own, for the largest weight
+    assert used < rows + partial + staging + (16 << 20), used                # (allocations are rounded up to 2 MiB)
+    kept = backend.cached_weight_bytes()
+    conv = np.ones((40, 33, 7), np.float32)
+    x, y = backend.alloc(33 * 10), backend.alloc(40 * 10)
+    backend.conv1d(x.ptr, y.ptr, 33, 40, 10, 7, 1, conv, None)
+    assert backend.cached_weight_bytes() - kept == (2 * 3 * 7 + 3) * 3072
+    x.free()
+    y.free()
