@@ -221,7 +221,8 @@ class DeviceBuffer:
 
 class Backend:
     """mynah_backend_open(MYNAH_TTS_DEVICE_HIP) as the reference's backend.c would wire it
-    (src/backend.c:367-475): one opaque state plus the function pointers handed back by open."""
+    (src/backend.c:367-475): one opaque state plus the function pointers handed back by open.  One thread at a time uses it:
+    its stream and workspaces serve one call after the other (only the weight cache is behind a lock)."""
 
     def __init__(self, quant=None, arith=None):
         self.lib = load_library()
@@ -241,7 +242,7 @@ class Backend:
 
     # -- plumbing
     def _call(self, name, *args):
-        err = C.create_string_buffer(512)   # each call's own: threads may share a backend
+        err = C.create_string_buffer(512)
         rc = getattr(self.lib, name)(self.state, *args, err, 512)
         if rc != 0:
             raise BackendError("%s: %s" % (name, err.value.decode()))

@@ -184,7 +184,8 @@ struct State {
     // normalised encoder memory of mynah_hip_cross_kv_dev (grown on demand; an outgrown one waits in pending_free)
     float *cross_norm = nullptr;
     size_t cross_norm_floats = 0;
-    // sums of the workgroups that share a convolution's channels (codec_ops.hip)
+    // sums of the workgroups that share a convolution's channels (codec_ops.hip): every call's between its two launches, one call after the
+    // other like all of a state's workspaces (one thread at a time, one stream)
     float *conv_parts = nullptr;
     // cache-flush buffer
     void *flush = nullptr;
