@@ -224,6 +224,35 @@ def test_res_layer_builds(pkg, backend, C, L, taps):
         d.free()
 
 
+# which of three positions leave the one launch, by a reach above 64 positions or by five taps in one branch
+@pytest.mark.parametrize("leave", [(0,), (1,), (2,), (0, 1), (0, 2), (1, 2)])
+@pytest.mark.parametrize("C,L,five", [(27, 700, False), (32, 130, True), (54, 3000, True)])
+def test_res_layer_mixed_positions(pkg, backend, C, L, five, leave):
+    """A layer some of whose positions are one launch and some two (the row sets change places between them): the operator sequence bit for bit."""
+    import importlib
+    codec = importlib.import_module(pkg.__name__ + ".codec")
+    _announce("residual layer mixed positions %d x %d %s %s" % (C, L, leave, five))
+    x, blocks = _res_layer_inputs(C, L, 400 + C)
+    rng = np.random.default_rng(C)
+    for p in leave:
+        a_in, (w_in, b_in), a_skip, (w_skip, b_skip), d = blocks[0 if five else 2][p]
+        if five:
+            w_in, w_skip = ((rng.standard_normal((C, C, 5)) / np.sqrt(5 * C)).astype(np.float32) for _ in range(2))
+        blocks[0 if five else 2][p] = (a_in, (w_in, b_in), a_skip, (w_skip, b_skip), d if five else 7)
+    n = C * L
+    din = backend.alloc(n).write(x)
+    bufs = [backend.alloc(n) for _ in range(11)]
+    at = [d.ptr for d in bufs]
+    codec.res_layer(backend, blocks, din.ptr, at[0], C, L, *at[1:5])
+    want = bufs[0].read()
+    codec.res_layer_batched(backend, blocks, din.ptr, at[1], C, L, at[2:5], at[5:8], at[8:11])
+    assert np.isfinite(want).all()
+    assert np.array_equal(want.view(np.uint32), bufs[1].read().view(np.uint32))
+    assert np.array_equal(din.read().reshape(C, L), x), "the layer's input was written"
+    for d in bufs + [din]:
+        d.free()
+
+
 @pytest.mark.parametrize("C,L", [(27, 130), (108, 200), (216, 90)])
 def test_res_layer_output_and_branch_forms(pkg, backend, C, L):
     """The layer's output may be its input or any of the work rows, in one launch a block or several; a single branch may grow in its
@@ -294,9 +323,11 @@ def test_conv_batch_members_and_refusals(pkg, backend):
         d.free()
 
 
-# channels shared between workgroups (more than 128, few short rows): one position, either side of the narrow and the wide tile, the last
-# shape that shares and the first that does not, a last workgroup without a block of its own, any tap count
-@pytest.mark.parametrize("C,O,L", [(432, 432, 1), (432, 400, 32), (432, 432, 33), (129, 70, 64), (216, 216, 1408), (216, 216, 1409), (600, 30, 65), (144, 31, 130)])
+# channels shared between workgroups (more than 128, few short rows): one position, either side of the narrow and the wide tile, either side of
+# each line between fewer workgroups (216 channels: 4 to 320 positions, 2 to 704, then one; 432: 7 to 64, 4 to 128, 3 to 192, 2 to 320), a last
+# workgroup without a block of its own, any tap count; and two rows that one workgroup a tile takes
+@pytest.mark.parametrize("C,O,L", [(432, 432, 1), (432, 400, 32), (432, 432, 33), (129, 70, 64), (216, 216, 320), (216, 216, 321), (216, 216, 704), (216, 216, 705),
+                                   (432, 432, 129), (432, 432, 192), (432, 432, 193), (216, 216, 1408), (216, 216, 1409), (600, 30, 65), (144, 31, 130)])
 def test_channels_shared_between_workgroups(backend, orc, nerr, C, O, L):
     """Against the oracle, single calls and members side by side (the same bits), with everything the epilogue can do."""
     _announce("shared channels %d -> %d x %d" % (C, O, L))
