@@ -248,12 +248,16 @@ struct ConvColumn {
     }
 };
 
-// What is hardly ever run of the tiles below, as calls of their own with the arguments read from memory once more: inline, their
-// registers came on top of the products' (11 taps: 4 to 11 % of a call, some of it spilled; 0.6 us of every call for the arguments).
-//
+// What is hardly ever run of the tiles below, with the arguments read from memory once more, behind an empty asm statement that keeps the
+// reads there (at the kernel's start they were 0.6 us of every call).
+__device__ __forceinline__ ConvArgs conv_again(const ConvArgs *args) {
+    asm volatile("" : "+s"(args));
+    return *args;
+}
 // conv_tile's values of one position through the loop over its rows: conv_chain for a sum that is no finite number, and the library's sine.
-__device__ __noinline__ void conv_tile_rest(const ConvArgs *const args, const float *s_tile, const float *const s_alpha, const int m_first, const int rows, const int t) {
-    const ConvArgs a = *args;
+// A call of its own for the fused builds: inline its registers came on top of the products' (11 taps: 4 to 11 % of a call, some of it
+// spilled).  A kernel with a call has a stack, half a microsecond of the launch behind it: not for the others.
+__device__ __forceinline__ void conv_tile_rest(const ConvArgs &a, const float *s_tile, const float *const s_alpha, const int m_first, const int rows, const int t) {
 #pragma unroll 1
     for (int row = 0; row < rows; ++row, s_tile += kTileStride) {
         const int m = m_first + row;
@@ -265,9 +269,12 @@ __device__ __noinline__ void conv_tile_rest(const ConvArgs *const args, const fl
         conv_emit(a, m, index, v, s_alpha[row], s_alpha[32 + row]);
     }
 }
+__device__ __noinline__ void conv_tile_rest_call(const ConvArgs *const args, const float *const s_tile, const float *const s_alpha, const int m_first, const int rows, const int t) {
+    conv_tile_rest(*args, s_tile, s_alpha, m_first, rows, t);
+}
 // conv_split_tile's partial sums of a thread's eight values (see there), the first taking the whole where it is no finite number.
-__device__ __noinline__ void conv_split_rest(const ConvArgs *const args, float *const s_part, const int split, const int m0, const int t) {
-    const ConvArgs a = *args;
+__device__ __forceinline__ void conv_split_rest(const ConvArgs *const args, float *const s_part, const int split, const int m0, const int t) {
+    const ConvArgs a = conv_again(args);
     const int tid = threadIdx.x, pos = tid & 63;
 #pragma unroll 1
     for (int j = 0; j < 8; ++j) {
@@ -417,8 +424,8 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
     }
     if constexpr (!FUSED) {   // the seam's conv1d; what is no finite number is stored once more below
         store_tile(a.out, acc0, acc1);
-        if (split_all_finite(acc)) return;
-    } else if (!a.activate && finite) {
+        if (__builtin_expect(split_all_finite(acc), 1)) return;
+    } else if (!a.activate && __builtin_expect(finite, 1)) {
         store_tile(a.out, acc0, acc1);
         return;
     }
@@ -440,7 +447,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
             const float al = s_alpha[8 * (r >> 2) + 4 * half + (r & 3)];
             large = large || !(fabsf(al * acc0[r]) < kShortSineLimit) || !(fabsf(al * acc1[r]) < kShortSineLimit);
         }
-        if (!__any(large)) {
+        if (__builtin_expect(!__any(large), 1)) {
             floatx16 act0, act1;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -478,7 +485,8 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
     const int t = t0 + wn * 64 + lane;
     if (t >= a.length) return;
     const int rows = min(32, a.out_ch - (m0 + wm * 32));   // the same for the whole wavefront
-    conv_tile_rest(again, s_tile + lane, s_alpha, m0 + wm * 32, rows, t);
+    if constexpr (FUSED) conv_tile_rest_call(again, s_tile + lane, s_alpha, m0 + wm * 32, rows, t);
+    else conv_tile_rest(conv_again(again), s_tile + lane, s_alpha, m0 + wm * 32, rows, t);
 }
 
 // (the rows, the weights and the shape lead the arguments and repeat fields of a_arg: leading scalar arguments are in registers
@@ -589,7 +597,7 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
         }
     };
     add_parts();
-    if (__any(t_ok && zero != 0.0f)) {   // (see split_all_finite)
+    if (__builtin_expect(__any(t_ok && zero != 0.0f), 0)) {   // (see split_all_finite)
         if (t_ok) conv_split_rest(again, s_part, split, m0, t);
         add_parts();
     }
@@ -653,18 +661,19 @@ constexpr int kConvBatchMax = 4;
 constexpr int kConvMaxSplits = 8;
 struct ConvBatchArgs {
     ConvArgs item[kConvBatchMax];
-    ConvBlocks weights[kConvBatchMax];
     int order[kConvBatchMax];   // blockIdx.z -> member: the ones with the most taps first, so that a long workgroup is not started last
 };
+
+__device__ __forceinline__ ConvBlocks conv_blocks(const ConvArgs &a) { return ConvBlocks{a.weights, (a.out_ch + 31) / 32, (a.in_ch + 15) / 16}; }
 
 template <int WM, int WN>
 __global__ void __launch_bounds__(256, 3) k_conv1d_batch(const ConvBatchArgs b) {
     extern __shared__ __align__(16) uint4 lds[];
     const int z = b.order[blockIdx.z];
     switch (b.item[z].kernel) {
-        case 3: conv_tile<WM, WN, 3, true>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
-        case 7: conv_tile<WM, WN, 7, true>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
-        default: conv_tile<WM, WN, 11, true>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        case 3: conv_tile<WM, WN, 3, true>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        case 7: conv_tile<WM, WN, 7, true>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        default: conv_tile<WM, WN, 11, true>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
     }
 }
 
@@ -673,9 +682,9 @@ __global__ void __launch_bounds__(256, 2) k_conv1d_split_batch(const ConvBatchAr
     extern __shared__ __align__(16) uint4 lds[];
     const int z = b.order[blockIdx.z];
     switch (b.item[z].kernel) {
-        case 3: conv_split_tile<3, NT, PARTS>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
-        case 7: conv_split_tile<7, NT, PARTS>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
-        default: conv_split_tile<11, NT, PARTS>(b.item[z], b.weights[z], &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        case 3: conv_split_tile<3, NT, PARTS>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        case 7: conv_split_tile<7, NT, PARTS>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        default: conv_split_tile<11, NT, PARTS>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
     }
 }
 
@@ -762,7 +771,7 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
 #pragma unroll
             for (int e = 0; e < 8; ++e)
                 if (channel + e < a.snake_channels) large = large || !(fabsf(m.snake_in[channel + e].x * v[e]) < kShortSineLimit);
-            if (!__any(large)) {
+            if (__builtin_expect(!__any(large), 1)) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     if (channel + e < a.snake_channels) {   // (the same for every lane)
@@ -872,7 +881,7 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
 #pragma unroll
         for (int n = 0; n < NT; ++n) large = large || !(fabsf(bound * acc[n][r]) < kShortSineLimit);
     }
-    if (!__any(large)) {
+    if (__builtin_expect(!__any(large), 1)) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row = wm * 32 + split_acc_row(r, lane);
@@ -928,7 +937,7 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
             if (block >= a.blocks) continue;
             const float4 v = make_float4(acc[n][4 * g], acc[n][4 * g + 1], acc[n][4 * g + 2], acc[n][4 * g + 3]);
             SplitFour s(in_front ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : v);
-            if (kept && !in_front) s.keep_bits(v);   // (the rows themselves are nowhere else)
+            if (__builtin_expect(kept, 0) && !in_front) s.keep_bits(v);   // (the rows themselves are nowhere else)
 #pragma unroll
             for (int q = 0; q < 3; ++q) reinterpret_cast<uint2 *>(&lds[(block * 6 + q * 2 + (g & 1)) * RN + p])[half] = s.piece[q];
         }
@@ -943,7 +952,7 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
     bool finite;
     if constexpr (SPLIT) finite = split_all_finite(sum);
     else finite = split_all_finite(acc);
-    if (!finite) {
+    if (__builtin_expect(!finite, 0)) {
 #pragma unroll 1
         for (int r = 0; r < 16; ++r) {
             const int row = wm * 32 + split_acc_row(r, lane);
@@ -1281,7 +1290,8 @@ static bool conv_takes_split(const State *st, int in_channels, int out_channels,
 // weights of all channels through one CU (some 40 GB/s: 0.9 MB with 432 channels and eleven taps); so as many as bring a wavefront's
 // blocks of channels down while three members' workgroups are two to a CU at most.  The sums' order follows, so this is the shape's
 // alone, too.  Taps 3 / 7 / 11 side by side: 432 channels x 40 24.6 -> 11.2 us, 216 x 320 18.9 -> 12.4, and 4.0 for k_conv_finish; 108 x 1280
-// stays with one (14.2 us, 12.4 + 4.2 shared), its seven blocks are few enough.  Twice kConvSharedTiles: nothing measurable.
+// stays with one (14.2 us, 12.4 + 4.2 shared), its seven blocks are few enough.  Half or twice kConvSharedTiles, a 432-channel layer of three positions: 64
+// positions 98 / 87 / 87 us, 128 143 / 116 / 123, 192 192 / 147 / 156, 256 230 / 175 / 168, 320 238 / 196 / 198.
 constexpr int kConvSharedTiles = 160;
 static int conv_splits(int in_channels, int out_channels, int length) {
     const long tiles = (long)((out_channels + 31) / 32) * ((length + 63) / 64), blocks = (in_channels + 15) / 16;
@@ -1385,11 +1395,12 @@ extern "C" int mynah_hip_conv1d_fused_batch(void *state, const mynah_hip_conv1d_
         return -1;
     }
     ConvBatchArgs b{};
+    ConvBlocks weights[kConvBatchMax];
     bool side_by_side = true;
     for (size_t i = 0; i < count; ++i) {
         const mynah_hip_conv1d_item &it = items[i];
         if (conv1d_prepare(st, (int)i, it.dev_input, it.dev_output, in_channels, out_channels, length, it.kernel, it.dilation, it.weight, it.bias, &it.extra,
-                           &b.item[i], &b.weights[i], error, capacity) != 0)
+                           &b.item[i], &weights[i], error, capacity) != 0)
             return -1;
         side_by_side = side_by_side && (it.kernel == 3 || it.kernel == 7 || it.kernel == 11);
         size_t at = i;   // most taps first
@@ -1411,7 +1422,7 @@ extern "C" int mynah_hip_conv1d_fused_batch(void *state, const mynah_hip_conv1d_
     }
     if (!side_by_side || count == 1) {   // other tap counts: one after the other (the same values)
         for (size_t i = 0; i < count; ++i)
-            if (conv1d_launch(st, b.item[i], b.weights[i], error, capacity) != 0) return -1;
+            if (conv1d_launch(st, b.item[i], weights[i], error, capacity) != 0) return -1;
         return 0;
     }
     if (conv_takes_split(st, in_channels, out_channels, length)) {
