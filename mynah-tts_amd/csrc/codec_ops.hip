@@ -256,7 +256,7 @@ __device__ __forceinline__ ConvArgs conv_again(const ConvArgs *args) {
 }
 // conv_tile's values of one position through the loop over its rows: conv_chain for a sum that is no finite number, and the library's sine.
 // A call of its own for the fused builds: inline its registers came on top of the products' (11 taps: 4 to 11 % of a call, some of it
-// spilled).  A kernel with a call has a stack, half a microsecond of the launch behind it: not for the others.
+// spilled).  The other builds have room for it.
 __device__ __forceinline__ void conv_tile_rest(const ConvArgs &a, const float *s_tile, const float *const s_alpha, const int m_first, const int rows, const int t) {
 #pragma unroll 1
     for (int row = 0; row < rows; ++row, s_tile += kTileStride) {
