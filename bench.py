@@ -218,8 +218,8 @@ def time_codec(pkg, backend, frames=64, runs=4, warmup=2):
     codec = importlib.import_module(pkg.__name__ + ".codec")
 
     def decode(fused):
-        """fused: the element-wise operators inside the convolutions' epilogues (mynah_hip_conv1d_fused), with "batched" also a
-        residual layer's three branches side by side in one launch per block and position (mynah_hip_conv1d_fused_batch);
+        """fused: the element-wise operators inside the convolutions' epilogues (mynah_hip_conv1d_fused), with "batched" a residual
+        layer as one call, its three branches side by side (mynah_hip_res_layer_dev: one or two launches per block and position);
         else the operator sequence decode_codec_resident issues through the seam.  All give the same samples, bit for bit."""
         nonlocal cur, up, out
         C, L = 864, frames
@@ -281,11 +281,11 @@ STAGES = [("self-attention", "k_step_attention<self>", "LayerNorm + int8 act-qua
 # then WRITE_SIZE), each scaled by what the same counter reads for the library's plain 256 MiB read+write kernel.  A figure
 # belongs to the kernel sources it was measured on: it is reported only while their hash is the one recorded here.
 MEASURED_TRAFFIC = {
-    1: {"kernel": "k_linear<k=768, residual>", "bytes": 937937, "profile": "profiles/decode_step_int8_hbm_counters.md",
-        "sources": ("kernels_linear.hip", "device_common.h", "kernels.h", "common.h"), "csrc_sha256": "1eb6ca405ed4bd2a"},
-    8: {"kernel": "k_step_attention<self>", "bytes": 54460167, "profile": "profiles/decode_step_int8_hbm_counters.md",
+    1: {"kernel": "k_linear<k=768, residual>", "bytes": 937921, "profile": "profiles/decode_step_int8_hbm_counters.md",
+        "sources": ("kernels_linear.hip", "device_common.h", "kernels.h", "common.h"), "csrc_sha256": "b6b32950dc471077"},
+    8: {"kernel": "k_step_attention<self>", "bytes": 54462396, "profile": "profiles/decode_step_int8_hbm_counters.md",
         "sources": ("kernels_step_attention.hip", "step_attention_core.h", "step_items.h", "tagged_exchange.h", "device_common.h",
-                    "kernels.h", "common.h"), "csrc_sha256": "9115d93638a9dc57"},
+                    "kernels.h", "common.h"), "csrc_sha256": "253321a9df05890c"},
 }
 
 
@@ -506,9 +506,9 @@ def main():
                                        % (codec["frames"], codec["samples"]),
                            "ms": round(codec["ms"], 3), "flops": codec["flops"], "tflops": round(codec["tflops"], 2), "bound": "mfma",
                            "peak_tflops": 416.7, "frac": round(codec["tflops"] / 416.7, 4),   # six bf16 piece products per f32 one: a sixth of 2500
-                           "form": "element-wise operators in the convolutions' epilogues and a residual layer's three branches side by side, "
-                                   "one launch per block and position (mynah_hip_conv1d_fused_batch); samples bit-identical to the seam's "
-                                   "operator sequence",
+                           "form": "a residual layer as one call (mynah_hip_res_layer_dev): element-wise operators in the convolutions' epilogues, the three "
+                                   "branches side by side, one launch per block and position at 27 channels and two elsewhere; samples bit-identical "
+                                   "to the seam's operator sequence",
                            "ms_one_launch_per_convolution": round(codec["ms_one_launch_per_convolution"], 3),
                            "ms_seam_operator_sequence": round(codec["ms_seam_operator_sequence"], 3)}
     if not args.no_cpu:
