@@ -1532,8 +1532,8 @@ extern "C" int mynah_hip_rows_combine_dev(void *state, const float *const *dev_i
 // (conv_takes_split) and whether all workgroups find a place at once: two to a CU (512 threads: one), 32 positions to a wavefront,
 // whose chain of products is then half as long, before 64.  Measured per layer of three positions, branches of 3 / 7 / 11 taps, us:
 //   27 channels: x 12288 67 narrow, 86 wide, 106 as two launches a position; x 20480 75, 90, 116; x 24576 (more than fit) 112, 100, 117
-//   54, split order: x 2560 81 narrow, 75 as two launches of narrow split tiles; x 3072 80, 82; x 8192 97, 141; x 10240 134, 157
-//   54, large order: x 16384 163 wide, 174 as two launches; x 20480 177, 203; x 20992 (more than fit) 229, 201
+//   54, split order: x 2560 84 narrow, 72 as two launches of split tiles; x 3072 85, 82; x 3584 86, 86; x 4608 86, 91; x 8192 98, 137; x 10240 137, 152
+//   54, large order: x 12288 140 wide, 164 as two launches; x 16384 161, 173; x 20480 173, 199; x 20992 (more than fit) 229, 201
 //   108, large order, 3 and 11 taps: x 6144 173 narrow, 202; x 8192 186, 204; x 12288 (more than fit) 276, 240
 // (three branches of 65 to 128 channels are never in the large order and few enough)
 enum ResBuild { RES_NONE, RES_32_NARROW, RES_32_WIDE, RES_64_SPLIT, RES_64_WIDE, RES_128 };
@@ -1551,7 +1551,7 @@ static ResBuild res_build(const State *st, const mynah_hip_res_block *blocks, si
     if (channels <= 32) return fit(128, 2) ? RES_32_NARROW : RES_32_WIDE;
     const bool split = conv_takes_split(st, (int)channels, (int)channels, (int)length);
     if (channels > 64) return !split && fit(64, 1) ? RES_128 : RES_NONE;
-    if (split) return conv_split_narrow(st, (int)channels, (int)length, (long)branches) ? RES_NONE : RES_64_SPLIT;
+    if (split) return 2 * (long)((length + 63) / 64) * (long)branches * 4 < (long)st->cu_count * 5 ? RES_NONE : RES_64_SPLIT;
     return fit(128, 2) ? RES_64_WIDE : RES_NONE;
 }
 
