@@ -183,8 +183,8 @@ def time_codec(pkg, backend, frames=64, runs=4, warmup=2):
     """The resident NanoCodec decode's operator sequence (decode_codec_resident / res_layer_device, src/graph.c:2423-2638)
     on synthetic weights: 32 -> 864 pre-conv, five stages of half-snake, grouped transposed conv (rates 8 8 4 2 2, channels
     halving) and a residual layer of 3 branches x 3 x (snake, conv k, snake, conv k) with k = 3 / 7 / 11 and dilations
-    1 / 3 / 5, then snake, the 1-channel post-conv and the clip.  f32 throughout; the convolutions run on the f32 matrix
-    cores.  Timed with HIP events on the backend's stream over whole decodes of `frames` raw frames."""
+    1 / 3 / 5, then snake, the 1-channel post-conv and the clip.  f32 operands and sums throughout; the convolutions run
+    on the bf16 matrix cores in three-piece form.  Timed with HIP events on the backend's stream over whole decodes of `frames` raw frames."""
     rng = np.random.default_rng(11)
 
     def conv_w(out_ch, in_ch, k):

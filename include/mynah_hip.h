@@ -151,7 +151,9 @@ int mynah_hip_argmax_dev(void *state, const float *dev_logits, size_t vocab, siz
  * that registers attention is also given the codec (src/graph.c:2514-2518), which fails hard without these
  * (:2552-2555): with them MYNAH_METAL_CPU_CODEC is not needed.
  * conv1d: causal, dilated; weight [out, in, kernel]; bias may be NULL (conv1d_causal, src/graph.c:2010-2160); runs
- *   on the f32 matrix cores; kernel <= 16, (kernel - 1) * dilation <= 128.
+ *   on the bf16 matrix cores with f32 operands in three bf16 pieces and f32 sums (no less precise than f32 multiply-adds;
+ *   infinite, NaN and largest operands give what those give; below 2^-110 an operand keeps fewer than 24 bits, at most 2^-134 of it is
+ *   lost); kernel <= 16, (kernel - 1) * dilation <= 128.  The products of cross_kv_dev and of the f32 encoder are made the same way.
  * conv_transpose_dev: grouped, weight [in, out / groups, kernel], output trimmed to output_length; bit-identical to
  *   the reference's scalar loop (convt_channel, src/graph.c:2179-2198).
  * snake_dev: in place; rows below snake_channels get x + sin(a x)^2 / (a + 1e-9), the rest a leaky ReLU of slope 0.01
@@ -211,7 +213,8 @@ int mynah_hip_snake_copy_dev(void *state, const float *dev_input, float *dev_out
  * residual layer (res_layer_device, src/graph.c:2423-2498, walks them one after the other) at the same block and position.
  * Each member has its own rows, weights, taps, dilation and epilogue and gets the values its own conv1d_fused call would
  * give, bit for bit; the members run at the same time, so no member may write rows that another reads or writes (refused).
- * With 3, 7 or 11 taps in every member the launch is shared; other tap counts run the members one after the other.
+ * With 3, 7 or 11 taps in every member the launch is shared (and a second one, where workgroups share a tile's channels, that
+ * adds their sums); other tap counts run the members one after the other.
  * No counterpart in the reference's seam. */
 typedef struct mynah_hip_conv1d_item {
     const float *dev_input;
@@ -493,8 +496,7 @@ typedef struct {
                                    * (src/graph.c:302-352), up_w [ffn, width, 3], down_w [width, ffn, 3] */
     int operands_f32;             /* nonzero: tables, weights and every product operand stay f32 -- transformer_stack's own
                                    * arithmetic (src/graph.c:634-711: f32 sgemm per head, f32 linears), to 1e-5 of the CPU.  The
-                                   * accuracy form: the library's f32 operators one after the other, no graph, several times the
-                                   * time of the f16 form.  0: f16 operands, f32 accumulation (2e-3) */
+                                   * accuracy form: about twice the time of the f16 form.  0: f16 operands, f32 accumulation (2e-3) */
 } mynah_hip_encoder_desc;
 typedef struct mynah_hip_encoder mynah_hip_encoder;
 

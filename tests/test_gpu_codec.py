@@ -1,5 +1,5 @@
 """GPU parity of the codec operators (mynah_hip_conv1d / _conv_transpose_dev / _snake_dev) against the oracle, through the
-C ABI.  conv1d runs on the f32 matrix cores and adds in a different order than the CPU: 1e-5 normalised.  The transposed
+C ABI.  conv1d runs in three-piece form on the bf16 matrix cores and adds in a different order than the CPU: 1e-5 normalised.  The transposed
 conv adds in the reference's order: bit-exact.  snake: the device sine against libm's, 1e-6 normalised."""
 import numpy as np
 import pytest
