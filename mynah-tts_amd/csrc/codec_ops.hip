@@ -5,8 +5,8 @@
 //
 //   conv1d          out[o][t] = bias[o] + sum_i sum_k w[(o*in + i)*K + k] * in[i][t - (K-1-k)*dilation]   (conv1d_causal,
 //                   src/graph.c:2010-2160).  The reference builds an im2col matrix and calls sgemm; here the same GEMM
-//                   (M = out channels, N = length, inner = in channels x taps) runs on the bf16 matrix cores in three-piece
-//                   form (split_product.h: f32 operands, f32 accumulation, the accuracy of an f32 product) with the im2col
+//                   (M = out channels, N = length, inner = in channels x taps) runs on the f16 matrix cores, two pieces a
+//                   value (half_product.h: f32 operands, f32 accumulation, the accuracy of an f32 product) with the im2col
 //                   done by addressing: a workgroup stages the input rows of sixteen channels once, with a halo of
 //                   (K-1)*dilation positions, and every tap reads the same rows at its own offset.
 //   conv_transpose  grouped, trimmed to output_length (conv_transpose_causal / convt_channel, src/graph.c:2179-2231):
@@ -19,6 +19,7 @@
 
 #include <type_traits>
 
+#include "half_product.h"
 #include "split_product.h"
 
 using namespace mynah;
@@ -26,8 +27,6 @@ using namespace mynah;
 namespace {
 
 typedef f32x16 floatx16;
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-typedef unsigned short ushort8 __attribute__((ext_vector_type(8)));
 
 constexpr int kConvMaxKernel = 16;
 constexpr int kConvMaxHalo = 128;     // (kernel - 1) * dilation
@@ -109,56 +108,75 @@ __device__ __forceinline__ void conv_emit(const ConvArgs &a, int m, size_t index
 }
 
 // The convolution's inner dimension goes in steps of one tap of sixteen input channels: one 16-deep matrix instruction per pair of
-// pieces.  Weights: taken apart once, when they are cached, in the order of the steps (ConvBlocks), so that a wavefront's three
-// pieces of a step are three requests of 1 KiB straight to its registers -- a weight serves length / 64 wavefronts, and taking it
-// apart there would cost each of them 44 vector instructions a step.  Inputs: a staged (position, eight channels) is 16 bytes
+// pieces.  Weights: taken apart once, when they are cached, in the order of the steps (ConvBlocks), so that a wavefront's two
+// pieces of a step are two requests of 1 KiB straight to its registers.  Inputs: a staged (position, eight channels) is 16 bytes
 // of LDS per piece, so a tap's operand is 512 consecutive bytes for 32 positions, whatever the tap's offset.
-// (108 channels x 16384, taps 3 / 7 / 11 in one launch: 70 us with f32 instructions, which have the matrix cores busy for 59 us; the six
-// bf16 instructions of a step are busy for 24.)
+// 108 channels x 16384, taps 3 / 7 / 11 in one launch, cycles of a workgroup (three to a CU, one of each): until its first product 5,000,
+// products 44,000 (its matrix instructions alone 28,000; without the weights' requests 31,500, without the LDS reads 38,000), residual
+// and stores 15,000, all workgroups at the same time.  As three bf16 pieces, with 64-bit addresses a lane and request that spilled, the
+// first product came after 35,000 and the launch took 55 us (now 41).
+// A value at `bytes` behind an address that is the same for every lane: one instruction with the address in scalar registers, where
+// pointer arithmetic by lanes takes 64-bit addresses in vector registers.
+// (opaque: what stays the same from request to request is otherwise added up ahead of all loops, 64 bits a lane and request)
+template <class T>
+__device__ __forceinline__ T load_behind(const T *base, unsigned bytes) { return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes); }
+__device__ __forceinline__ unsigned opaque(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ int opaque_scalar(int v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
 struct ConvWeights {   // the weight pieces of one row tile, requested kAhead steps before they are multiplied
     static constexpr int kAhead = kConvStepsAhead;
-    const uint4 *next;
+    const uint4 *next;   // the same for every lane, like the inputs' rows below: an address is then a pair of scalar registers and the lane's offset, where
+                         // one of 64 bits per lane and request had taken the products' registers (and spilled)
+    unsigned bytes;   // a lane's 16
     size_t skip;       // from the end of a block to the next one this wavefront multiplies
     int blocks;        // it multiplies
     int tap = 0;       // of the next request (a constant wherever the tap count is one)
-    uint4 ring[kAhead][3];
+    uint4 ring[kAhead][2];
     __device__ __forceinline__ void request(int slot, int taps) {
+        bytes = opaque(bytes);
 #pragma unroll
-        for (int q = 0; q < 3; ++q) ring[slot][q] = next[64 * q];
-        next += 192;
+        for (int q = 0; q < 2; ++q) ring[slot][q] = load_behind(next + 64 * q, bytes);
+        next += 128;
         if (++tap == taps) {
             tap = 0;
             if (--blocks > 0) next += skip;
         }
     }
     // (what runs past the last step is requested and not used: it is what follows the last block, and the cache pads its copies)
-    __device__ __forceinline__ ConvWeights(const uint4 *first, size_t skip_arg, int blocks_arg, int taps) : next(first), skip(skip_arg), blocks(blocks_arg) {
+    __device__ __forceinline__ ConvWeights(const uint4 *first, unsigned lane, size_t skip_arg, int blocks_arg, int taps)
+        : next(first), bytes(lane * 16), skip(skip_arg), blocks(blocks_arg) {
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) request(i, taps);
     }
 };
 
 // The products of the blocks of sixteen channels a wavefront multiplies, for its 32 rows x (32 * NT) positions.
-// stage(block): makes the block's inputs readable and returns where this lane's first operand lies: element [piece * piece_stride +
-// position], lanes 32.. eight channels on.  With the tap count known (KF) the loop over a block's steps is unrolled, and three blocks at
+// stage(block): makes the block's inputs readable and returns where this lane's first operand lies: element [piece * PIECE + position]
+// (a constant: one address register serves a tap's reads), lanes 32.. eight channels on.  With the tap count known (KF) the loop over a block's steps is unrolled, and three blocks at
 // a time, after which the weights' registers repeat.  (A step's fragments are read right before it: two or three wavefronts share a
 // SIMD, and a second set of fragment registers, read a step ahead, spilled: 1884 against 1754 us for a 64-frame decode.)
-template <int KF, int NT, bool AHEAD = false, class Stage>
-__device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, const int dilation, const int piece_stride, const int blocks, const Stage stage,
-                                              floatx16 (&acc)[NT]) {
-    bf16x8 x[AHEAD ? 2 : 1][NT][3];
+template <int KF, int NT, int PIECE, bool AHEAD = false, class Stage>
+__device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, const int dilation, const int blocks, const Stage stage,
+                                              HalfSums (&acc)[NT]) {
+    half8_t x[AHEAD ? 2 : 1][NT][2];
     const auto read = [&](int set, const uint4 *at) {
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int q = 0; q < 3; ++q) x[set][n][q] = __builtin_bit_cast(bf16x8, at[q * piece_stride + 32 * n]);
+            for (int q = 0; q < 2; ++q) x[set][n][q] = __builtin_bit_cast(half8_t, at[q * PIECE + 32 * n]);
     };
     const auto multiply = [&](int set, int slot) {
-        bf16x8 fw[3];
+        half8_t fw[2];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) fw[q] = __builtin_bit_cast(bf16x8, w.ring[slot][q]);
+        for (int q = 0; q < 2; ++q) fw[q] = __builtin_bit_cast(half8_t, w.ring[slot][q]);
 #pragma unroll
-        for (int n = 0; n < NT; ++n) acc[n] = split_multiply(fw, x[set][n], acc[n]);
+        for (int n = 0; n < NT; ++n) acc[n].multiply(fw, x[set][n]);
     };
     if constexpr (KF != 0) {
         for (int block = 0;;) {
@@ -187,64 +205,83 @@ __device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, co
 #pragma unroll
                 for (int i = 0; i + 1 < ConvWeights::kAhead; ++i)
 #pragma unroll
-                    for (int q = 0; q < 3; ++q) w.ring[i][q] = w.ring[i + 1][q];
+                    for (int q = 0; q < 2; ++q) w.ring[i][q] = w.ring[i + 1][q];
                 w.request(ConvWeights::kAhead - 1, taps);
             }
         }
     }
 }
 
-// What a sum of pieces that is no finite number stands for (split_product.h): the chain of f32 multiply-adds, from `s`, over the channels
-// (eight, then the taps, then the next eight) of every block that mine(block) names.  w: the output row's first piece of the first block and
-// tap; inside(tap): whether the tap's position lies in the row; fetch(channel, tap, x): its eight inputs from that channel on.
+// The rows' inverse scales, behind a packed weight's steps (see ConvBlocks).
+__device__ __forceinline__ const float *conv_inverses(const uint4 *data, size_t steps) { return reinterpret_cast<const float *>(data + steps * 192); }
+
+// What a sum of pieces that is no finite number stands for (half_product.h): the chain of f32 multiply-adds, from `s`, over the channels
+// (eight, then the taps, then the next eight) of every block that mine(block) names.  inside(tap): whether the tap's position lies in the
+// row; fetch(channel, tap, x): its eight inputs from that channel on.
+struct ConvRow {   // an output row's weights
+    const uint4 *pieces, *third;
+    float inverse;
+    __device__ __forceinline__ ConvRow(const uint4 *data, int tiles, int blocks, int taps, int row) {
+        const size_t tile = (size_t)blocks * taps, steps = tile * tiles;
+        pieces = data + (row >> 5) * tile * 128 + (row & 31);
+        third = data + steps * 128 + (row >> 5) * tile * 64 + (row & 31);
+        inverse = conv_inverses(data, steps)[row];
+    }
+};
 template <class Mine, class Inside, class Fetch>
-__device__ __forceinline__ float conv_chain(const uint4 *const w, const int channels, const int taps, const Mine mine, const Inside inside, const Fetch fetch, float s) {
+__device__ __forceinline__ float conv_chain(const ConvRow w, const int channels, const int taps, const Mine mine, const Inside inside, const Fetch fetch, float s) {
 #pragma unroll 1
     for (int c = 0; c < channels && s == s; c += 8) {
         if (!mine(c >> 4)) continue;
 #pragma unroll 1
         for (int tap = 0; tap < taps; ++tap) {
             if (!inside(tap)) continue;
-            const uint4 *const at = w + (size_t)((c >> 4) * taps + tap) * 192 + ((c >> 3) & 1) * 32;
-            const ushort8 h = __builtin_bit_cast(ushort8, at[0]), m = __builtin_bit_cast(ushort8, at[64]), l = __builtin_bit_cast(ushort8, at[128]);
+            const size_t step = (size_t)((c >> 4) * taps + tap);
+            const uint4 *const at = w.pieces + step * 128 + ((c >> 3) & 1) * 32;
+            const ushort8_t h = __builtin_bit_cast(ushort8_t, at[0]), m = __builtin_bit_cast(ushort8_t, at[64]),
+                            l = __builtin_bit_cast(ushort8_t, w.third[step * 64 + ((c >> 3) & 1) * 32]);
             float x[8];
             fetch(c, tap, x);
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                if (c + e < channels) s = __builtin_fmaf(split_value(h[e], m[e], l[e]), x[e], s);
+                if (c + e < channels) s = __builtin_fmaf(half_value(h[e], m[e], l[e], w.inverse), x[e], s);
         }
     }
     return s;
 }
-// ... of a convolution's own input rows, at output position t of row `row` of a tile.
+// ... of a convolution's own input rows, at output position t of row m.
 template <class Mine>
-__device__ __forceinline__ float conv_chain_rows(const ConvArgs &a, const uint4 *const tile, const int row, const int t, const Mine mine, const float s) {
+__device__ __forceinline__ float conv_chain_rows(const ConvArgs &a, const int m, const int t, const Mine mine, const float s) {
     const int back = (a.kernel - 1) * a.dilation;
-    return conv_chain(tile + (row & 31), a.in_ch, a.kernel, mine, [&](int tap) { return t - back + tap * a.dilation >= 0; },
+    return conv_chain(ConvRow(a.weights, (a.out_ch + 31) / 32, (a.in_ch + 15) / 16, a.kernel, m), a.in_ch, a.kernel, mine, [&](int tap) { return t - back + tap * a.dilation >= 0; },
                       [&](int c, int tap, float (&x)[8]) {
 #pragma unroll
                           for (int e = 0; e < 8; ++e) x[e] = a.in[(size_t)min(c + e, a.in_ch - 1) * a.length + t - back + tap * a.dilation];
                       }, s);
 }
 
+// Eight rows' values at one position: row channel + e, the last one for what there is not.
+__device__ __forceinline__ void request_rows(float (&v)[8], const float *first, int channel, int channels, int length, unsigned bytes) {
+    const float *row = first + (size_t)min(channel, channels - 1) * length;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        v[e] = load_behind(row, bytes);
+        row += channel + e + 1 < channels ? length : 0;
+    }
+}
 // One (position, eight channels) on its way to LDS: eight requests, then the pieces of the eight values.
 struct ConvColumn {
     float v[8];
-    // rows channel .. channel + 7 of the input at position t (channel is the same for every lane); a channel the input does not
-    // have repeats its last one -- its weights are zeros
-    __device__ __forceinline__ void request(const ConvArgs &a, int channel, int t) {
-        const float *const at = a.in + t;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = at[(size_t)min(channel + e, a.in_ch - 1) * a.length];
+    // rows channel .. channel + 7 of the input, `bytes` behind `origin` of the first row (channel and origin are the same for
+    // every lane); a channel the input does not have repeats its last one -- its weights are zeros
+    __device__ __forceinline__ void request(const float *origin, int channel, int channels, int length, unsigned &bytes) {
+        bytes = opaque(bytes);
+        channel = opaque_scalar(channel);
+        request_rows(v, origin, channel, channels, length, bytes);
     }
-    __device__ __forceinline__ void store(uint4 *at, int piece_stride, bool inside) const {
-        bf16x8 p[3];
-        float u[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) u[e] = inside ? v[e] : 0.0f;   // (in front of the row)
-        split_eight(make_float4(u[0], u[1], u[2], u[3]), make_float4(u[4], u[5], u[6], u[7]), p);
-#pragma unroll
-        for (int q = 0; q < 3; ++q) at[q * piece_stride] = __builtin_bit_cast(uint4, p[q]);
+    __device__ __forceinline__ void store(uint4 *at, int piece_stride, bool inside, float scale, float &largest) const {
+        // (in front of the row: nothing, or no number where the row's first value is none -- then the sums are looked for as such)
+        half_eight(v, inside ? scale : 0.0f, largest, at[0], at[piece_stride]);
     }
 };
 
@@ -264,8 +301,7 @@ __device__ __forceinline__ void conv_tile_rest(const ConvArgs &a, const float *s
         const size_t index = (size_t)m * a.length + t;
         float v = *s_tile;
         if (!split_finite(v))
-            v = conv_combine(a, index, conv_chain_rows(a, a.weights + (size_t)(m >> 5) * ((a.in_ch + 15) / 16) * a.kernel * 192, m & 31, t, [](int) { return true; },
-                                                       a.bias != nullptr ? a.bias[m] : 0.0f));
+            v = conv_combine(a, index, conv_chain_rows(a, m, t, [](int) { return true; }, a.bias != nullptr ? a.bias[m] : 0.0f));
         conv_emit(a, m, index, v, s_alpha[row], s_alpha[32 + row]);
     }
 }
@@ -281,12 +317,19 @@ __device__ __forceinline__ void conv_split_rest(const ConvArgs *const args, floa
         const int row = (tid >> 6) + 4 * j, m = m0 + row;
         float *const at = s_part + ((((row >> 3) << 2) | (row & 3)) + 16 * (pos >> 5)) * 64 + ((row >> 2) & 1) * 32 + (pos & 31);
         if (m >= a.out_ch || split_finite(((at[0] + at[2048]) + at[4096]) + at[6144])) continue;
-        at[0] = conv_chain_rows(a, a.weights + (size_t)(m >> 5) * ((a.in_ch + 15) / 16) * a.kernel * 192, row, t, [&](int block) { return block % (4 * a.splits) / 4 == split; }, 0.0f);
+        at[0] = conv_chain_rows(a, m, t, [&](int block) { return block % (4 * a.splits) / 4 == split; }, 0.0f);
         at[2048] = at[4096] = at[6144] = 0.0f;
     }
 }
 
-// Workgroup tile: (32 * WM) output channels x (64 * WN) positions; a wavefront owns 32 x 64 (two 32 x 32 accumulators).
+// A tile's output rows: what their sums are multiplied by, and their biases; and the largest input that each wavefront has staged.
+constexpr int conv_pitch(int positions) { return positions + kConvMaxHalo; }
+struct ConvTileRows {
+    alignas(16) float inverse[64], bias[64];
+    float largest[4];
+};
+
+// Workgroup tile: (32 * WM) output channels x (64 * WN) positions; a wavefront owns 32 x 64 (two 32 x 32 tiles of sums).
 // KF: number of taps known at compile time (0 = from the arguments); the codec's 3, 7 and 11 taps get such builds.
 // FUSED: the build that mynah_hip_conv1d_fused launches (residuals, scale, activation after the products); the seam's
 // conv1d keeps a build without any of it.
@@ -295,7 +338,7 @@ __device__ __forceinline__ void conv_split_rest(const ConvArgs *const args, floa
 // (the tile's work as a function: the kernel of one convolution and the kernel of several side by side both run it; `again`: the
 // arguments as they lie in memory, for conv_tile_rest)
 template <int WM, int WN, int KF, bool FUSED>
-__device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, const ConvArgs *const again, uint4 *const lds) {
+__device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, const ConvArgs *const again, uint4 *const lds, ConvTileRows &s_rows) {
     constexpr int TM = 32 * WM, TN = 64 * WN;
     ConvArgs a = a_arg;
     if constexpr (KF != 0) a.kernel = KF;
@@ -312,46 +355,40 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
     constexpr int kColumns = TN + kConvMaxHalo > 256 ? 3 : 2;
     static_assert(TN + kConvMaxHalo <= 384, "three columns a thread cover the window");
     int place[kColumns];      // window position, or -1
-    int from[kColumns];       // position in the row, clamped into it
+    unsigned from[kColumns];  // bytes from the window's first position (in the row) to this one, clamped into the row
     bool inside[kColumns];
+    const int first = max(t0 - halo, 0);
 #pragma unroll
     for (int x = 0; x < kColumns; ++x) {
         const int p = x == 0 ? tid : x == 1 ? (tid + 128) & 255 : 256 + (tid & 127);
         const int t = t0 - halo + p;
         place[x] = p < win ? p : -1;
         inside[x] = t >= 0;
-        from[x] = min(max(t, 0), a.length - 1);
+        from[x] = (unsigned)(min(max(t, 0), a.length - 1) - first) * 4;
     }
     const auto group_of = [&](int x) { return x < 2 ? x : __builtin_amdgcn_readfirstlane(tid >> 7); };
     ConvColumn column[kColumns];
     const auto fetch = [&](int block) {
 #pragma unroll
-        for (int x = 0; x < kColumns; ++x) column[x].request(a, 16 * block + 8 * group_of(x), from[x]);
+        for (int x = 0; x < kColumns; ++x) column[x].request(a.in + first, 16 * block + 8 * group_of(x), a.in_ch, a.length, from[x]);
     };
-    uint4 *stage_now = lds, *stage_next = lds + 6 * win;   // [piece][eight channels][position]
+    constexpr int kPitch = conv_pitch(TN);
+    uint4 *stage_now = lds, *stage_next = lds + 4 * kPitch;   // [piece][eight channels][position]
+    float scale = 1.0f, unscale = 1.0f, largest = 0.0f;
     const auto publish = [&](uint4 *stage) {
 #pragma unroll
         for (int x = 0; x < kColumns; ++x)
-            if (place[x] >= 0) column[x].store(stage + group_of(x) * win + place[x], 2 * win, inside[x]);
+            if (place[x] >= 0) column[x].store(stage + group_of(x) * kPitch + place[x], 2 * kPitch, inside[x], scale, largest);
     };
     const int tile = min((int)blockIdx.y * WM + wm, w_arg.tiles - 1);
-
-    // The accumulators start from the rows' biases (requested here, beside the first block: at the end each would be a
-    // round trip of its own in front of the stores), so a value is bias + products in the products' order.
-    floatx16 acc[2];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-        acc[0][r] = (a.bias != nullptr && m < a.out_ch) ? a.bias[m] : 0.0f;
+    // (requested here, beside the first block: at the end they would be a round trip in front of the stores)
+    if (tid < TM) {
+        s_rows.inverse[tid] = conv_inverses(w_arg.data, (size_t)w_arg.tiles * w_arg.blocks * a.kernel)[min(m0 + tid, 32 * w_arg.tiles - 1)];
+        s_rows.bias[tid] = a.bias != nullptr && m0 + tid < a.out_ch ? a.bias[m0 + tid] : 0.0f;
     }
-    acc[1] = acc[0];
-    fetch(0);
-    ConvWeights w(w_arg.data + (size_t)tile * w_arg.blocks * a.kernel * 192 + lane, 0, 1, a.kernel);
-    publish(stage_now);
-    fetch(min(1, w_arg.blocks - 1));
     const auto stage = [&](int block) {
         __syncthreads();   // this block is stored, and nobody multiplies the one whose place the next one takes
-        const uint4 *at = stage_now + half * win + wn * 64 + col;
+        const uint4 *at = stage_now + half * kPitch + wn * 64 + col;
         if (block + 1 < w_arg.blocks) {
             publish(stage_next);
             fetch(min(block + 2, w_arg.blocks - 1));
@@ -361,9 +398,38 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
         stage_next = t;
         return at;
     };
-    conv_products<KF, 2>(w, a.kernel, a.dilation, 2 * win, w_arg.blocks, stage, acc);
-    __syncthreads();   // the epilogue's pieces of LDS overwrite the stages
+    HalfSums sums[2];
+    for (bool once_more = false;; once_more = true) {
+        sums[0].clear();
+        sums[1].clear();
+        fetch(0);
+        ConvWeights w(w_arg.data + (size_t)tile * w_arg.blocks * a.kernel * 128, lane, 0, 1, a.kernel);
+        publish(stage_now);
+        fetch(min(1, w_arg.blocks - 1));
+        conv_products<KF, 2, 2 * kPitch>(w, a.kernel, a.dilation, w_arg.blocks, stage, sums);
+        largest = wave_max(largest);
+        if (lane == 0) s_rows.largest[wave] = largest;
+        __syncthreads();   // (and the epilogue's pieces of LDS overwrite the stages)
+        if (once_more) break;
+        const int e = __builtin_amdgcn_readfirstlane(half_rescale(fmaxf(fmaxf(s_rows.largest[0], s_rows.largest[1]), fmaxf(s_rows.largest[2], s_rows.largest[3]))));
+        if (__builtin_expect(e == 0, 1)) break;
+        scale = power_of_two(e);
+        unscale = power_of_two(-e);
+    }
+    // What follows starts from the thread's number anew: what the compiler may take from above it forms ahead of the products and keeps in
+    // scratch memory meanwhile (35 values of a thread, 27 MB a launch written before the first product and read behind the last).
+    const int tid_after = (int)opaque(threadIdx.x), lane_after = tid_after & 63, wave_after = __builtin_amdgcn_readfirstlane(tid_after >> 6);
+    const auto finish = [&](const int lane, const int wave) {
+    const int wm = wave / WN, wn = wave % WN, half = lane >> 5, col = lane & 31;
+    floatx16 acc[2];
     floatx16 &acc0 = acc[0], &acc1 = acc[1];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = wm * 32 + split_acc_row(r, lane);
+        const float inverse = s_rows.inverse[row], bias = s_rows.bias[row];
+        acc0[r] = sums[0].sum(r) * unscale * inverse + bias;
+        acc1[r] = sums[1].sum(r) * unscale * inverse + bias;
+    }
     // The fused build's residual values, requested side by side; a residual may be the output itself -- every workgroup reads and
     // writes its own tile only.
     float res_first[FUSED ? 32 : 1], res_second[FUSED ? 32 : 1];
@@ -487,6 +553,8 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
     const int rows = min(32, a.out_ch - (m0 + wm * 32));   // the same for the whole wavefront
     if constexpr (FUSED) conv_tile_rest_call(again, s_tile + lane, s_alpha, m0 + wm * 32, rows, t);
     else conv_tile_rest(conv_again(again), s_tile + lane, s_alpha, m0 + wm * 32, rows, t);
+    };
+    finish(lane_after, wave_after);
 }
 
 // (the rows, the weights and the shape lead the arguments and repeat fields of a_arg: leading scalar arguments are in registers
@@ -509,10 +577,11 @@ __global__ void __launch_bounds__(256, 3) k_conv1d(const float *const in_arg, fl
                                                    const int out_ch_arg, const int length_arg, const int kernel_arg, const int dilation_arg, const int tiles_arg,
                                                    const ConvArgs a_arg) {
     extern __shared__ __align__(16) uint4 lds[];
+    __shared__ ConvTileRows s_rows;
     ConvArgs a = a_arg;
     a.in = in_arg; a.out = out_arg; a.bias = bias_arg; a.in_ch = in_ch_arg; a.out_ch = out_ch_arg; a.length = length_arg;
     a.kernel = kernel_arg; a.dilation = dilation_arg;
-    conv_tile<WM, WN, KF, FUSED>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, &conv_kernarg<ConvKernarg>()->a, lds);
+    conv_tile<WM, WN, KF, FUSED>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, &conv_kernarg<ConvKernarg>()->a, lds, s_rows);
 }
 
 // The same product for short rows (few positions, many channels: the codec's first stages), where 64 x 128 tiles would
@@ -524,36 +593,42 @@ __global__ void __launch_bounds__(256, 3) k_conv1d(const float *const in_arg, fl
 // a.splits > 1: that many workgroups share the tile's channels (wavefront w of workgroup s is wavefront 4 s + w of them all), each
 // leaves its sum in a.parts, and k_conv_finish adds them in order and does what is left.
 template <int KF, int NT, int PARTS>
-__device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, const ConvArgs *const again, uint4 *const lds) {
+__device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const ConvBlocks &w_arg, const ConvArgs *const again, uint4 *const lds, ConvTileRows &s_rows) {
     constexpr int TM = 32, TN = 32 * NT;
     ConvArgs a = a_arg;
     if constexpr (KF != 0) a.kernel = KF;
     const int halo = (a.kernel - 1) * a.dilation;
     const int win = TN + halo;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    uint4 *s_in = lds + wave * (6 * win);      // [piece][eight channels][position] of this wavefront
+    constexpr int kPitch = conv_pitch(TN);
+    uint4 *s_in = lds + wave * (4 * kPitch);   // [piece][eight channels][position] of this wavefront
     const int split = (int)blockIdx.x % a.splits, sharing = 4 * a.splits, rank = 4 * split + wave;   // this wavefront among those that share the channels
     const int m0 = blockIdx.y * TM, t0 = (int)blockIdx.x / a.splits * TN;
     const int half = lane >> 5, col = lane & 31;
 
-    floatx16 acc[NT];
+    HalfSums acc[NT];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) acc[n] = floatx16{0};
+    for (int n = 0; n < NT; ++n) acc[n].clear();
+    float scale = 1.0f, unscale = 1.0f;   // (this wavefront's: its sums are its own)
+    if (tid < TM) s_rows.inverse[tid] = conv_inverses(w_arg.data, (size_t)w_arg.tiles * w_arg.blocks * a.kernel)[m0 + tid];
     const int mine = (w_arg.blocks - rank + sharing - 1) / sharing;   // this wavefront's blocks
     if (mine > 0) {
         ConvColumn column[2][PARTS];
+        const int first = max(t0 - halo, 0);
+        unsigned from[PARTS];   // see conv_tile
+#pragma unroll
+        for (int x = 0; x < PARTS; ++x) from[x] = (unsigned)(min(max(t0 - halo + lane + 64 * x, 0), a.length - 1) - first) * 4;
         const auto fetch = [&](int i) {
 #pragma unroll
             for (int x = 0; x < PARTS; ++x)
                 if (64 * x < win) {   // (the same for every lane)
 #pragma unroll
                     for (int g = 0; g < 2; ++g)
-                        column[g][x].request(a, 16 * (sharing * i + rank) + 8 * g, min(max(t0 - halo + lane + 64 * x, 0), a.length - 1));
+                        column[g][x].request(a.in + first, 16 * (sharing * i + rank) + 8 * g, a.in_ch, a.length, from[x]);
                 }
         };
-        fetch(0);
-        const size_t per_block = (size_t)a.kernel * 192;
-        ConvWeights w(w_arg.data + ((size_t)blockIdx.y * w_arg.blocks + rank) * per_block + lane, (size_t)(sharing - 1) * per_block, mine, a.kernel);
+        const size_t per_block = (size_t)a.kernel * 128;
+        float largest = 0.0f;
         // (no workgroup barrier in the loop: a wavefront stages into its own part of LDS and reads nothing else, and its own
         // LDS accesses complete in the order it issued them -- the four wavefronts walk their channel blocks independently)
         const auto stage = [&](int i) {
@@ -563,14 +638,24 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
                 const int p = lane + 64 * x;
                 if (p < win) {
 #pragma unroll
-                    for (int g = 0; g < 2; ++g) column[g][x].store(s_in + g * win + p, 2 * win, t0 - halo + p >= 0);
+                    for (int g = 0; g < 2; ++g) column[g][x].store(s_in + g * kPitch + p, 2 * kPitch, t0 - halo + p >= 0, scale, largest);
                 }
             }
             fetch(min(i + 1, mine - 1));   // in flight during this block's products
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            return const_cast<const uint4 *>(s_in + half * win + col);
+            return const_cast<const uint4 *>(s_in + half * kPitch + col);
         };
-        conv_products<KF, NT>(w, a.kernel, a.dilation, 2 * win, mine, stage, acc);
+        for (bool once_more = false;; once_more = true) {
+            fetch(0);
+            ConvWeights w(w_arg.data + ((size_t)blockIdx.y * w_arg.blocks + rank) * per_block, lane, (size_t)(sharing - 1) * per_block, mine, a.kernel);
+            conv_products<KF, NT, 2 * kPitch>(w, a.kernel, a.dilation, mine, stage, acc);
+            const int e = once_more ? 0 : half_rescale(wave_max(largest));
+            if (__builtin_expect(e == 0, 1)) break;
+            scale = power_of_two(e);
+            unscale = power_of_two(-e);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n].clear();
+        }
     }
     __syncthreads();   // the partial tiles below overwrite every wavefront's staging area
     // partial tiles through LDS: [wavefront][element r][lane], then ((p0 + p1) + p2) + p3 + bias
@@ -578,7 +663,7 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s_part[(wave * 32 + 16 * n + r) * 64 + lane] = acc[n][r];
+        for (int r = 0; r < 16; ++r) s_part[(wave * 32 + 16 * n + r) * 64 + lane] = acc[n].sum(r) * unscale * s_rows.inverse[split_acc_row(r, lane)];
     __syncthreads();
     // A thread finishes the tile's values at (row (tid / 64) + 4 j, position tid % 64): a store instruction then covers one
     // row's 64 consecutive positions and whether the row exists is the same for all its lanes (in the accumulators' order an
@@ -644,11 +729,12 @@ __global__ void __launch_bounds__(256, 2) k_conv1d_split(const float *const in_a
                                                          const int out_ch_arg, const int length_arg, const int kernel_arg, const int dilation_arg, const int tiles_arg,
                                                          const ConvArgs a_arg) {
     extern __shared__ __align__(16) uint4 lds[];
+    __shared__ ConvTileRows s_rows;
     // (leading scalar arguments: see k_conv1d)
     ConvArgs a = a_arg;
     a.in = in_arg; a.out = out_arg; a.bias = bias_arg; a.in_ch = in_ch_arg; a.out_ch = out_ch_arg; a.length = length_arg;
     a.kernel = kernel_arg; a.dilation = dilation_arg;
-    conv_split_tile<KF, NT, PARTS>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, &conv_kernarg<ConvKernarg>()->a, lds);
+    conv_split_tile<KF, NT, PARTS>(a, ConvBlocks{weights_arg, tiles_arg, (a.in_ch + 15) / 16}, &conv_kernarg<ConvKernarg>()->a, lds, s_rows);
 }
 
 // Several convolutions of one shape side by side in one launch (the three branches of a residual layer: same rows in and
@@ -669,22 +755,24 @@ __device__ __forceinline__ ConvBlocks conv_blocks(const ConvArgs &a) { return Co
 template <int WM, int WN>
 __global__ void __launch_bounds__(256, 3) k_conv1d_batch(const ConvBatchArgs b) {
     extern __shared__ __align__(16) uint4 lds[];
+    __shared__ ConvTileRows s_rows;
     const int z = b.order[blockIdx.z];
     switch (b.item[z].kernel) {
-        case 3: conv_tile<WM, WN, 3, true>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
-        case 7: conv_tile<WM, WN, 7, true>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
-        default: conv_tile<WM, WN, 11, true>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        case 3: conv_tile<WM, WN, 3, true>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds, s_rows); break;
+        case 7: conv_tile<WM, WN, 7, true>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds, s_rows); break;
+        default: conv_tile<WM, WN, 11, true>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds, s_rows); break;
     }
 }
 
 template <int NT, int PARTS>
 __global__ void __launch_bounds__(256, 2) k_conv1d_split_batch(const ConvBatchArgs b) {
     extern __shared__ __align__(16) uint4 lds[];
+    __shared__ ConvTileRows s_rows;
     const int z = b.order[blockIdx.z];
     switch (b.item[z].kernel) {
-        case 3: conv_split_tile<3, NT, PARTS>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
-        case 7: conv_split_tile<7, NT, PARTS>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
-        default: conv_split_tile<11, NT, PARTS>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds); break;
+        case 3: conv_split_tile<3, NT, PARTS>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds, s_rows); break;
+        case 7: conv_split_tile<7, NT, PARTS>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds, s_rows); break;
+        default: conv_split_tile<11, NT, PARTS>(b.item[z], conv_blocks(b.item[z]), &conv_kernarg<ConvBatchArgs>()->item[z], lds, s_rows); break;
     }
 }
 
@@ -723,15 +811,24 @@ struct ResMember {
     int kernel, dilation;
 };
 constexpr int kResMaxChannels = 128, kResMaxReach = 64;
+constexpr float kLargest = 0x1.ffp127f;   // no finite value of use in a sum is above it
 struct ResArgs {
     ResMember member[kConvBatchMax];
     int order[kConvBatchMax];
     int channels, length, snake_channels, blocks, tiles;
 };
 
+// The block's channels: (alpha, 1 / (alpha + 1e-9), a bound, -) of the inner rows' half-snake, (inverse scale, bias) of both convolutions;
+// and the largest input and inner value of each wavefront.
+struct ResRows {
+    float4 pair[kResMaxChannels];
+    float2 in[kResMaxChannels], skip[kResMaxChannels];
+    float largest[8], largest_inner[8];
+};
+
 template <int WM, int WN, int NT, bool SPLIT, int KF>
-__device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember &m, uint4 *const lds, float4 *const s_pairs) {
-    constexpr int WP = 32 * NT, RN = WP * WN, T = 64 * WM * WN, TN = RN - (KF - 1);
+__device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember &m, uint4 *const lds, ResRows &s_rows) {
+    constexpr int WP = 32 * NT, RN = WP * WN, T = 64 * WM * WN, TN = RN - (KF - 1), kPitch = RN + kResMaxReach;
     const int t0 = blockIdx.x * TN;
     if (t0 >= a.length) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, col = lane & 31;
@@ -751,14 +848,15 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
         const int p = kColumns == 1 ? tid & (T / 2 - 1) : x == 0 ? tid : x == 1 ? (kColumns == 2 ? (tid + 128) & 255 : tid) : tid < 128 ? 256 + (tid & 63) : win;
         place[x] = p < win ? p : -1;
     }
-    f32x8 column[kColumns];
+    float column[kColumns][8];
+    float scale = 1.0f, unscale = 1.0f, largest = 0.0f;
     const auto fetch = [&](int block) {
 #pragma unroll
         for (int x = 0; x < kColumns; ++x) {
-            const int channel = 16 * block + 8 * group_of(x);
-            const float *const at = m.in + min(max(first + place[x], 0), a.length - 1);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) column[x][e] = at[(size_t)min(channel + e, a.channels - 1) * a.length];
+            const int channel = opaque_scalar(16 * block + 8 * group_of(x));
+            const int origin = max(first, 0);
+            const unsigned bytes = opaque((unsigned)(min(max(first + max(place[x], 0), 0), a.length - 1) - origin) * 4);   // (never in front of origin)
+            request_rows(column[x], m.in + origin, channel, a.channels, a.length, bytes);
         }
     };
     const auto publish = [&](int block, uint4 *stage) {
@@ -766,103 +864,191 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
         for (int x = 0; x < kColumns; ++x) {
             if (place[x] < 0) continue;
             const int channel = 16 * block + 8 * group_of(x);
-            f32x8 v = column[x];
-            bool large = false;
+            float v[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (channel + e < a.snake_channels) large = large || !(fabsf(m.snake_in[channel + e].x * v[e]) < kShortSineLimit);
-            if (__builtin_expect(!__any(large), 1)) {
+            for (int e = 0; e < 8; ++e) v[e] = column[x][e];
+            // (one branch for the eight channels, which are the same for every lane: their alphas come in one request, their sines side by side)
+            if (channel < a.snake_channels) {
+                float2 pair[8];
+                float argument[8], most = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) pair[e] = m.snake_in[channel + e < a.snake_channels ? channel + e : channel];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    if (channel + e < a.snake_channels) {   // (the same for every lane)
-                        const float2 pair = m.snake_in[channel + e];
-                        const float sn = short_sine(pair.x * v[e]);
-                        v[e] = v[e] + sn * sn * pair.y;
-                    } else {
-                        v[e] = v[e] < 0.0f ? v[e] * 0.01f : v[e];
+                    argument[e] = pair[e].x * v[e];
+                    most = fmaxf(most, fabsf(argument[e]));   // (of a row without a sine, too: the long way gives its value as well)
+                }
+                if (__builtin_expect(!__any(most >= kShortSineLimit), 1)) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float sn = short_sine(argument[e]), y = v[e] + sn * sn * pair[e].y;
+                        v[e] = channel + e < a.snake_channels ? y : v[e] < 0.0f ? v[e] * 0.01f : v[e];
+                    }
+                } else {
+#pragma unroll 1
+                    for (int e = 0; e < 8; ++e) {
+                        const bool snake_row = channel + e < a.snake_channels;
+                        const float2 p = snake_row ? m.snake_in[channel + e] : make_float2(0.0f, 0.0f);
+                        v[e] = half_snake(v[e], snake_row, p.x, p.y);
                     }
                 }
             } else {
-#pragma unroll 1
-                for (int e = 0; e < 8; ++e) {
-                    const bool snake_row = channel + e < a.snake_channels;
-                    const float2 pair = snake_row ? m.snake_in[channel + e] : make_float2(0.0f, 0.0f);
-                    v[e] = half_snake(v[e], snake_row, pair.x, pair.y);
-                }
-            }
-            if (first + place[x] < 0) v = f32x8{0};   // in front of the rows
-            bf16x8 p[3];
-            split_eight(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]), p);
 #pragma unroll
-            for (int q = 0; q < 3; ++q) stage[(q * 2 + group_of(x)) * win + place[x]] = __builtin_bit_cast(uint4, p[q]);
+                for (int e = 0; e < 8; ++e) v[e] = v[e] < 0.0f ? v[e] * 0.01f : v[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = first + place[x] < 0 ? 0.0f : v[e];   // in front of the rows
+            uint4 *const at = stage + group_of(x) * kPitch + place[x];
+            half_eight(v, scale, largest, at[0], at[2 * kPitch]);
         }
     };
     // the inner rows' alphas, 1 / (alpha + 1e-9), and what a value is multiplied by to be told from those that need the long way: the
-    // library's sine, or (no finite number, or none that three pieces add up to) more than that
-    if (tid < kResMaxChannels) {
-        const float2 pair = tid < a.snake_channels ? m.snake_skip[tid] : make_float2(0.0f, 0.0f);
-        s_pairs[tid] = make_float4(pair.x, pair.y, fmaxf(fabsf(pair.x), 1.01f * (kShortSineLimit / kSplitLimit)), 0.0f);
+    // library's sine, or (no finite number, or none to speak of) more than that
+    for (int c = tid; c < kResMaxChannels; c += T) {
+        const float2 pair = c < a.snake_channels ? m.snake_skip[c] : make_float2(0.0f, 0.0f);
+        s_rows.pair[c] = make_float4(pair.x, pair.y, fmaxf(fabsf(pair.x), 1.01f * (kShortSineLimit / kLargest)), 0.0f);
+        const bool there = c < a.channels;   // (else zero: a wavefront without a row tile of its own multiplies the last one's weights)
+        const size_t steps = (size_t)a.tiles * a.blocks * KF;
+        s_rows.in[c] = make_float2(there ? conv_inverses(m.w_in, steps)[c] : 0.0f, there && m.b_in != nullptr ? m.b_in[c] : 0.0f);
+        s_rows.skip[c] = make_float2(there ? conv_inverses(m.w_skip, steps)[c] : 0.0f, there && m.b_skip != nullptr ? m.b_skip[c] : 0.0f);
     }
 
-    // the rows' biases, which the sums start from: both convolutions' requested here, none under a condition
-    float bias_in[16], bias_skip[16];
+    HalfSums sums[NT];
+    f32x16 acc[NT];   // (SPLIT: the blocks before, then) the finished sums
+    const auto start = [&]() {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = min(wm * 32 + split_acc_row(r, lane), a.channels - 1);
-        bias_in[r] = m.b_in != nullptr ? m.b_in[row] : 0.0f;
-        bias_skip[r] = m.b_skip != nullptr ? m.b_skip[row] : 0.0f;
-    }
-    f32x16 acc[NT], sum[SPLIT ? NT : 1];
-    const auto start = [&](const float (&bias)[16]) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[0][r] = !SPLIT && wm * 32 + split_acc_row(r, lane) < a.channels ? bias[r] : 0.0f;
-#pragma unroll
-        for (int n = 1; n < NT; ++n) acc[n] = acc[0];
-        if constexpr (SPLIT) {
-#pragma unroll
-            for (int n = 0; n < NT; ++n) sum[n] = f32x16{0};
+        for (int n = 0; n < NT; ++n) {
+            sums[n].clear();
+            if constexpr (SPLIT) acc[n] = f32x16{0};
         }
     };
-    // (SPLIT) a block's sums to those of the blocks before it; in the end, the bias
+    // (SPLIT) a block's sums to those of the blocks before it
     const auto add_block = [&]() {
         if constexpr (SPLIT) {
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
-                sum[n] += acc[n];
-                acc[n] = f32x16{0};
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[n][r] += sums[n].sum(r);
+                sums[n].clear();
             }
         }
     };
-    const auto finish = [&](const float (&bias)[16]) {
+    // the scales divided out, and the bias
+    const auto finish = [&](const float2 (&rows)[kResMaxChannels], float unscaled) {
         add_block();
-        if constexpr (SPLIT) {
 #pragma unroll
-            for (int n = 0; n < NT; ++n)
+        for (int n = 0; n < NT; ++n)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[n][r] = sum[n][r] + bias[r];
-        }
+            for (int r = 0; r < 16; ++r) {
+                const float2 row = rows[wm * 32 + split_acc_row(r, lane)];
+                acc[n][r] = (SPLIT ? acc[n][r] : sums[n].sum(r)) * unscaled * row.x + row.y;
+            }
     };
-    const size_t w_at = (size_t)min(wm, a.tiles - 1) * a.blocks * KF * 192 + lane;
-    fetch(0);
-    ConvWeights w(m.w_in + w_at, 0, 1, KF);
-    uint4 *stage_now = lds, *stage_next = lds + 6 * win;
-    start(bias_in);
-    publish(0, stage_now);
-    fetch(min(1, a.blocks - 1));
-    conv_products<KF, NT, true>(w, KF, m.dilation, 2 * win, a.blocks, [&](int block) {
-        if (block > 0) add_block();
-        __syncthreads();
-        const uint4 *at = stage_now + half * win + wn * WP + col;
-        if (block + 1 < a.blocks) {
-            publish(block + 1, stage_next);
-            fetch(min(block + 2, a.blocks - 1));
+    const size_t w_at = (size_t)min(wm, a.tiles - 1) * a.blocks * KF * 128;
+    uint4 *stage_now = lds, *stage_next = lds + 4 * kPitch;
+    float inner_largest;
+    for (bool once_more = false;; once_more = true) {
+        fetch(0);
+        ConvWeights w(m.w_in + w_at, lane, 0, 1, KF);
+        start();
+        publish(0, stage_now);
+        fetch(min(1, a.blocks - 1));
+        conv_products<KF, NT, 2 * kPitch, true>(w, KF, m.dilation, a.blocks, [&](int block) {
+            if (block > 0) add_block();
+            __syncthreads();
+            const uint4 *at = stage_now + half * kPitch + wn * WP + col;
+            if (block + 1 < a.blocks) {
+                publish(block + 1, stage_next);
+                fetch(min(block + 2, a.blocks - 1));
+            }
+            uint4 *t = stage_now;
+            stage_now = stage_next;
+            stage_next = t;
+            return at;
+        }, sums);
+        finish(s_rows.in, unscale);
+        bool large = false;
+    #pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float bound = s_rows.pair[wm * 32 + split_acc_row(r, lane)].z;
+    #pragma unroll
+            for (int n = 0; n < NT; ++n) large = large || !(fabsf(bound * acc[n][r]) < kShortSineLimit);
         }
-        uint4 *t = stage_now;
-        stage_now = stage_next;
-        stage_next = t;
-        return at;
-    }, acc);
-    finish(bias_in);
+        if (__builtin_expect(!__any(large), 1)) {
+    #pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = wm * 32 + split_acc_row(r, lane);
+                const float4 pair = s_rows.pair[row];
+    #pragma unroll
+                for (int n = 0; n < NT; ++n) {
+                    const float v = acc[n][r];
+                    float y = v < 0.0f ? v * 0.01f : v;
+                    if (wm * 32 + 8 * (r >> 2) < a.snake_channels) {   // (else no lane's row of these registers is a snake row)
+                        const float sn = short_sine(pair.x * v);
+                        y = row < a.snake_channels ? v + sn * sn * pair.y : y;
+                    }
+                    acc[n][r] = y;
+                }
+            }
+        } else {
+    #pragma unroll 1
+            for (int r = 0; r < 16; ++r) {
+                const int row = wm * 32 + split_acc_row(r, lane);
+                const float4 pair = s_rows.pair[row];
+    #pragma unroll
+                for (int n = 0; n < NT; ++n) {
+                    const int t = t0 - (KF - 1) + wn * WP + 32 * n + col;
+                    float v = acc[n][r];
+                    if (row < a.channels && t >= 0 && t < a.length && !split_finite(v)) {
+                        const float bias = s_rows.in[row].y;
+                        v = conv_chain(ConvRow(m.w_in, a.tiles, a.blocks, KF, row), a.channels, KF, [](int) { return true; }, [&](int tap) { return t - halo + tap * m.dilation >= 0; },
+                                       [&](int c, int tap, float (&x)[8]) {
+    #pragma unroll 1
+                                           for (int e = 0; e < 8; ++e) {
+                                               const int channel = min(c + e, a.channels - 1);
+                                               const float2 in_pair = channel < a.snake_channels ? m.snake_in[channel] : make_float2(0.0f, 0.0f);
+                                               x[e] = half_snake(m.in[(size_t)channel * a.length + t - halo + tap * m.dilation], channel < a.snake_channels, in_pair.x, in_pair.y);
+                                           }
+                                       }, SPLIT ? 0.0f : bias);
+                        if (SPLIT) v = v + bias;
+                    }
+                    v = row < a.channels ? half_snake(v, row < a.snake_channels, pair.x, pair.y) : 0.0f;
+                    acc[n][r] = v;
+                }
+            }
+        }
+        // the largest values of the workgroup, for the scales under which they are taken apart
+        largest = wave_max(largest);
+        float largest_inner = 0.0f;
+    #pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const bool in_front = t0 - (KF - 1) + wn * WP + 32 * n + col < 0;
+    #pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if (in_front) acc[n][r] = 0.0f;
+                largest_inner = fmaxf(largest_inner, fabsf(acc[n][r]));
+            }
+        }
+        largest_inner = wave_max(largest_inner);
+        if (lane == 0) {
+            s_rows.largest[wave] = largest;
+            s_rows.largest_inner[wave] = largest_inner;
+        }
+        __syncthreads();   // (and the stages have been read)
+        const auto of_all = [&](const float (&each)[8]) {
+            float v = each[0];
+    #pragma unroll
+            for (int i = 1; i < WM * WN; ++i) v = fmaxf(v, each[i]);
+            return v;
+        };
+        const int e = once_more ? 0 : __builtin_amdgcn_readfirstlane(half_rescale(of_all(s_rows.largest)));
+        if (__builtin_expect(e == 0, 1)) {
+            inner_largest = of_all(s_rows.largest_inner);
+            break;
+        }
+        scale = power_of_two(e);
+        unscale = power_of_two(-e);
+    }
 
     // the finished rows' residual (x itself), on its way during the rest: whole rows of consecutive positions, as it is stored
     const int rows = min(32, a.channels - wm * 32);
@@ -873,102 +1059,69 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
 #pragma unroll
     for (int i = 0; i < 32 / kRowsAtOnce; ++i) x[i] = m.in[at_out + (size_t)max(min(row0 + kRowsAtOnce * i, rows - 1), 0) * a.length];
     // the inner rows: activated, zero in front of the first position, in pieces to LDS where the second convolution reads them
-    ConvWeights w2(m.w_skip + w_at, 0, 1, KF);
-    bool large = false, kept = false;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const float bound = s_pairs[wm * 32 + split_acc_row(r, lane)].z;
-#pragma unroll
-        for (int n = 0; n < NT; ++n) large = large || !(fabsf(bound * acc[n][r]) < kShortSineLimit);
-    }
-    if (__builtin_expect(!__any(large), 1)) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = wm * 32 + split_acc_row(r, lane);
-            const float4 pair = s_pairs[row];
-#pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                const float v = acc[n][r];
-                float y = v < 0.0f ? v * 0.01f : v;
-                if (wm * 32 + 8 * (r >> 2) < a.snake_channels) {   // (else no lane's row of these registers is a snake row)
-                    const float sn = short_sine(pair.x * v);
-                    y = row < a.snake_channels ? v + sn * sn * pair.y : y;
-                }
-                acc[n][r] = y;
-            }
-        }
-    } else {
-#pragma unroll 1
-        for (int r = 0; r < 16; ++r) {
-            const int row = wm * 32 + split_acc_row(r, lane);
-            const float4 pair = s_pairs[row];
-#pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                const int t = t0 - (KF - 1) + wn * WP + 32 * n + col;
-                float v = acc[n][r];
-                if (row < a.channels && t >= 0 && t < a.length && !split_finite(SPLIT ? sum[SPLIT ? n : 0][r] : v)) {
-                    const float bias = m.b_in != nullptr ? m.b_in[row] : 0.0f;
-                    v = conv_chain(m.w_in + (w_at - lane) + (row & 31), a.channels, KF, [](int) { return true; }, [&](int tap) { return t - halo + tap * m.dilation >= 0; },
-                                   [&](int c, int tap, float (&x)[8]) {
-#pragma unroll 1
-                                       for (int e = 0; e < 8; ++e) {
-                                           const int channel = min(c + e, a.channels - 1);
-                                           const float2 in_pair = channel < a.snake_channels ? m.snake_in[channel] : make_float2(0.0f, 0.0f);
-                                           x[e] = half_snake(m.in[(size_t)channel * a.length + t - halo + tap * m.dilation], channel < a.snake_channels, in_pair.x, in_pair.y);
-                                       }
-                                   }, SPLIT ? 0.0f : bias);
-                    if (SPLIT) v = v + bias;
-                }
-                v = row < a.channels ? half_snake(v, row < a.snake_channels, pair.x, pair.y) : 0.0f;
-                kept = kept || !(fabsf(v) < kSplitLimit);
-                acc[n][r] = v;
-            }
-        }
-        kept = __any(kept);
-    }
-    __syncthreads();   // the stages have been read
+    ConvWeights w2(m.w_skip + w_at, lane, 0, 1, KF);
+    const int inner_e = __builtin_amdgcn_readfirstlane(half_rescale(inner_largest));
+    scale = power_of_two(inner_e);
+    unscale = power_of_two(-inner_e);
+    const bool kept = !(__uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(inner_largest))) * scale < kHalfLimit);
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const int p = wn * WP + 32 * n + col;
-        const bool in_front = t0 - (KF - 1) + p < 0;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {   // rows 8 g + 4 half .. + 3 of the tile: half of the eight channels of one place
             const int block = wm * 2 + (g >> 1);
             if (block >= a.blocks) continue;
-            const float4 v = make_float4(acc[n][4 * g], acc[n][4 * g + 1], acc[n][4 * g + 2], acc[n][4 * g + 3]);
-            SplitFour s(in_front ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : v);
-            if (__builtin_expect(kept, 0) && !in_front) s.keep_bits(v);   // (the rows themselves are nowhere else)
+            unsigned h[2], mid[2], low[2];
 #pragma unroll
-            for (int q = 0; q < 3; ++q) reinterpret_cast<uint2 *>(&lds[(block * 6 + q * 2 + (g & 1)) * RN + p])[half] = s.piece[q];
+            for (int i = 0; i < 2; ++i) {
+                float rest[2];
+                half_pieces(acc[n][4 * g + 2 * i], acc[n][4 * g + 2 * i + 1], scale, h[i], mid[i], rest);
+                low[i] = half_third(mid[i], rest);
+            }
+            uint2 piece[3] = {make_uint2(h[0], h[1]), make_uint2(mid[0], mid[1]), make_uint2(low[0], low[1])};
+            if (__builtin_expect(kept, 0)) {   // (the rows themselves are nowhere else)
+                ushort4_t at[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) at[q] = __builtin_bit_cast(ushort4_t, piece[q]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    unsigned short ph = at[0][i], pm = at[1][i], pl = at[2][i];
+                    half_keep_bits(acc[n][4 * g + i], scale, ph, pm, pl);
+                    at[0][i] = ph;
+                    at[1][i] = pm;
+                    at[2][i] = pl;
+                }
+#pragma unroll
+                for (int q = 0; q < 3; ++q) piece[q] = __builtin_bit_cast(uint2, at[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < 3; ++q) reinterpret_cast<uint2 *>(&lds[(block * 6 + q * 2 + (g & 1)) * RN + p])[half] = piece[q];
         }
     }
-    start(bias_skip);
+    start();
     __syncthreads();
-    conv_products<KF, NT, true>(w2, KF, 1, 2 * RN, a.blocks, [&](int block) {
+    conv_products<KF, NT, 2 * RN, true>(w2, KF, 1, a.blocks, [&](int block) {
         if (block > 0) add_block();
         return const_cast<const uint4 *>(lds + (block * 6 + half) * RN + wn * WP + col);
-    }, acc);
-    finish(bias_skip);
-    bool finite;
-    if constexpr (SPLIT) finite = split_all_finite(sum);
-    else finite = split_all_finite(acc);
-    if (__builtin_expect(!finite, 0)) {
+    }, sums);
+    finish(s_rows.skip, unscale);
+    if (__builtin_expect(!split_all_finite(acc), 0)) {
 #pragma unroll 1
         for (int r = 0; r < 16; ++r) {
             const int row = wm * 32 + split_acc_row(r, lane);
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
                 const int p = wn * WP + 32 * n + col, t = t0 + p;
-                if (row >= a.channels || p >= TN || t >= a.length || split_finite(SPLIT ? sum[SPLIT ? n : 0][r] : acc[n][r])) continue;
-                const float bias = m.b_skip != nullptr ? m.b_skip[row] : 0.0f;
-                const float v = conv_chain(m.w_skip + (w_at - lane) + (row & 31), a.channels, KF, [](int) { return true; },
+                if (row >= a.channels || p >= TN || t >= a.length || split_finite(acc[n][r])) continue;
+                const float bias = s_rows.skip[row].y;
+                const float v = conv_chain(ConvRow(m.w_skip, a.tiles, a.blocks, KF, row), a.channels, KF, [](int) { return true; },
                                            [&](int tap) { return t - (KF - 1) + tap >= 0; },
                                            [&](int c, int tap, float (&x)[8]) {
                                                const uint4 *const at = lds + ((c >> 4) * 6 + ((c >> 3) & 1)) * RN + p + tap;
-                                               const ushort8 xh = __builtin_bit_cast(ushort8, at[0]), xm = __builtin_bit_cast(ushort8, at[2 * RN]),
-                                                             xl = __builtin_bit_cast(ushort8, at[4 * RN]);
+                                               const ushort8_t xh = __builtin_bit_cast(ushort8_t, at[0]), xm = __builtin_bit_cast(ushort8_t, at[2 * RN]),
+                                                               xl = __builtin_bit_cast(ushort8_t, at[4 * RN]);
 #pragma unroll
-                                               for (int e = 0; e < 8; ++e) x[e] = split_value(xh[e], xm[e], xl[e]);
+                                               for (int e = 0; e < 8; ++e) x[e] = half_value(xh[e], xm[e], xl[e], unscale);
                                            }, SPLIT ? 0.0f : bias);
                 acc[n][r] = SPLIT ? v + bias : v;
             }
@@ -977,42 +1130,38 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
 
     // + x, and out, in whole rows (see store_tile of conv_tile)
     __syncthreads();   // the inner rows have been read
-    constexpr int kPitch = WP + 1;
-    float *const s_tile = reinterpret_cast<float *>(lds) + wave * (32 * kPitch);
+    constexpr int kRowPitch = WP + 1;
+    float *const s_tile = reinterpret_cast<float *>(lds) + wave * (32 * kRowPitch);
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s_tile[split_acc_row(r, lane) * kPitch + 32 * n + col] = acc[n][r];
+        for (int r = 0; r < 16; ++r) s_tile[split_acc_row(r, lane) * kRowPitch + 32 * n + col] = acc[n][r];
     if (rows <= 0 || p_out >= TN || t_out >= a.length) return;
 #pragma unroll
     for (int i = 0; i < 32 / kRowsAtOnce; ++i) {
         const int row = row0 + kRowsAtOnce * i;
-        if (row < rows) m.out[at_out + (size_t)row * a.length] = x[i] + s_tile[row * kPitch + lane % WP];
+        if (row < rows) m.out[at_out + (size_t)row * a.length] = x[i] + s_tile[row * kRowPitch + lane % WP];
     }
 }
 
 template <int WM, int WN, int NT, bool SPLIT>
 __global__ void __launch_bounds__(64 * WM * WN, 2) k_res_block(const ResArgs a) {
     extern __shared__ __align__(16) uint4 lds[];
-    __shared__ float4 s_pairs[kResMaxChannels];
+    __shared__ ResRows s_rows;
     const int z = a.order[blockIdx.y];
     switch (a.member[z].kernel) {
-        case 3: res_block_tile<WM, WN, NT, SPLIT, 3>(a, a.member[z], lds, s_pairs); break;
-        case 7: res_block_tile<WM, WN, NT, SPLIT, 7>(a, a.member[z], lds, s_pairs); break;
-        default: res_block_tile<WM, WN, NT, SPLIT, 11>(a, a.member[z], lds, s_pairs); break;
+        case 3: res_block_tile<WM, WN, NT, SPLIT, 3>(a, a.member[z], lds, s_rows); break;
+        case 7: res_block_tile<WM, WN, NT, SPLIT, 7>(a, a.member[z], lds, s_rows); break;
+        default: res_block_tile<WM, WN, NT, SPLIT, 11>(a, a.member[z], lds, s_rows); break;
     }
 }
 
 template <int WM, int WN, int NT, bool SPLIT = false>
 int launch_res_block(State *st, const ResArgs &a, int count, char *error, size_t capacity) {
     constexpr int RN = 32 * NT * WN;
-    int taps = 0, reach = 0;
-    for (int i = 0; i < count; ++i) {
-        taps = a.member[i].kernel > taps ? a.member[i].kernel : taps;
-        const int halo = (a.member[i].kernel - 1) * a.member[i].dilation;
-        reach = halo > reach ? halo : reach;
-    }
-    size_t lds = (size_t)2 * 6 * (RN + reach) * 16;                                   // two stages, or
+    int taps = 0;
+    for (int i = 0; i < count; ++i) taps = a.member[i].kernel > taps ? a.member[i].kernel : taps;
+    size_t lds = (size_t)2 * 4 * (RN + kResMaxReach) * 16;                                   // two stages, or
     const size_t inner = ((size_t)a.blocks * 6 * RN + 16) * 16;                        // the inner rows (a tap past the last place is read, not used), or
     const size_t tiles = (size_t)WM * WN * 32 * (32 * NT + 1) * sizeof(float);        // the finished tiles
     lds = inner > lds ? inner : lds;
@@ -1027,32 +1176,57 @@ int launch_res_block(State *st, const ResArgs &a, int count, char *error, size_t
     return hip_check(hipGetLastError(), "residual block launch", error, capacity);
 }
 
+// A weight's rows get a scale each: the largest value under it lies in [2^13, 2^14), unless it is 2^20 times the row's usual size and
+// more -- then what is 2^20 times that lies there, and what does not fit above it is kept as its bits (half_product.h).  A wavefront a row.
+__global__ void __launch_bounds__(64) k_conv_row_scales(const float *src, float *inverses, int out_ch, size_t per_row) {
+    const int row = (int)blockIdx.x, lane = (int)threadIdx.x;
+    float sum = 0.0f, count = 0.0f, most = -127.0f;
+    if (row < out_ch)
+        for (size_t i = lane; i < per_row; i += 64) {
+            const float v = src[(size_t)row * per_row + i];
+            const int e = exponent_of(v);
+            if (v == 0.0f || e == 128) continue;   // (nothing, or no finite number)
+            sum += (float)e;
+            count += 1.0f;
+            most = fmaxf(most, (float)e);
+        }
+    sum = wave_sum(sum);
+    count = wave_sum(count);
+    most = wave_max(most);
+    const int top = count == 0.0f ? 13 : (int)fminf(most, floorf(sum / count) + 20.0f);
+    if (lane == 0) inverses[row] = power_of_two(max(top - 13, -126));
+}
+
 __global__ void __launch_bounds__(256) k_conv_pack(const float *src, uint4 *dst, size_t count, int out_ch, int in_ch, int kernel, int blocks) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= count) return;
     const int lane = (int)(i & 63);
-    const size_t step = i >> 6, tile = step / ((size_t)blocks * kernel);
+    const size_t step = i >> 6, tile = step / ((size_t)blocks * kernel), steps = count >> 6;
     const int tap = (int)(step % (size_t)kernel), block = (int)(step / (size_t)kernel % (size_t)blocks);
     const size_t o = tile * 32 + (lane & 31);
     const int c0 = block * 16 + (lane >> 5) * 8;
-    float v[8];
+    const float scale = 1.0f / conv_inverses(dst, steps)[o];
+    ushort8_t at[3];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = o < (size_t)out_ch && c0 + e < in_ch ? src[(o * in_ch + c0 + e) * kernel + tap] : 0.0f;
-    bf16x8 p[3];
-    split_eight(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]), p);
-    ushort8 at[3];
+    for (int e = 0; e < 8; e += 2) {
+        float v[2], rest[2];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) at[q] = __builtin_bit_cast(ushort8, p[q]);
+        for (int k = 0; k < 2; ++k) v[k] = o < (size_t)out_ch && c0 + e + k < in_ch ? src[(o * in_ch + c0 + e + k) * kernel + tap] : 0.0f;
+        unsigned h, m;
+        half_pieces(v[0], v[1], scale, h, m, rest);
+        const unsigned l = half_third(m, rest);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {   // (the kernels have no other copy of a weight)
-        unsigned short h = at[0][e], m = at[1][e], l = at[2][e];
-        split_keep_bits(v[e], h, m, l);
-        at[0][e] = h;
-        at[1][e] = m;
-        at[2][e] = l;
+        for (int k = 0; k < 2; ++k) {   // (the kernels have no other copy of a weight)
+            unsigned short ph = (unsigned short)(h >> 16 * k), pm = (unsigned short)(m >> 16 * k), pl = (unsigned short)(l >> 16 * k);
+            half_keep_bits(v[k], scale, ph, pm, pl);
+            at[0][e + k] = ph;
+            at[1][e + k] = pm;
+            at[2][e + k] = pl;
+        }
     }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) dst[step * 192 + q * 64 + lane] = __builtin_bit_cast(uint4, at[q]);
+    dst[step * 128 + lane] = __builtin_bit_cast(uint4, at[0]);
+    dst[step * 128 + 64 + lane] = __builtin_bit_cast(uint4, at[1]);
+    dst[steps * 128 + step * 64 + lane] = __builtin_bit_cast(uint4, at[2]);
 }
 
 struct ConvTransposeArgs {
@@ -1130,16 +1304,16 @@ __global__ void __launch_bounds__(256) k_rows_combine(const RowsCombineArgs a) {
 
 // LDS of a launch: two stages of one block of channels (the channel-split kernel: one per wavefront), or what the epilogue keeps there.
 template <int WM, int WN>
-size_t conv_lds(const ConvArgs &a) {
-    const size_t stages = (size_t)2 * 6 * (64 * WN + (a.kernel - 1) * a.dilation) * 16, epilogue = (4 * 32 * kTileStride + 4 * 64) * sizeof(float);
+constexpr size_t conv_lds() {
+    constexpr size_t stages = (size_t)2 * 4 * conv_pitch(64 * WN) * 16, epilogue = (4 * 32 * kTileStride + 4 * 64) * sizeof(float);
     return stages > epilogue ? stages : epilogue;
 }
 template <int NT>
-size_t conv_split_lds(const ConvArgs &a) {
-    const size_t stages = (size_t)4 * 6 * (32 * NT + (a.kernel - 1) * a.dilation) * 16, epilogue = (4 * 32 * 64 + 64) * sizeof(float);
+constexpr size_t conv_split_lds() {
+    constexpr size_t stages = (size_t)4 * 4 * conv_pitch(32 * NT) * 16, epilogue = (4 * 32 * 64 + 64) * sizeof(float);
     return stages > epilogue ? stages : epilogue;
 }
-constexpr int kConvMaxLds = 2 * 6 * (256 + kConvMaxHalo) * 16;   // the largest of them
+constexpr int kConvMaxLds = 2 * 4 * (256 + kConvMaxHalo) * 16;   // the largest of them
 
 template <int WM, int WN, int KF, bool FUSED>
 int launch_conv_f(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
@@ -1150,7 +1324,7 @@ int launch_conv_f(State *st, const ConvArgs &a, const ConvBlocks &weights, char 
         raised = true;
     }
     const dim3 grid((unsigned)((a.length + TN - 1) / TN), (unsigned)((a.out_ch + TM - 1) / TM));
-    hipLaunchKernelGGL((k_conv1d<WM, WN, KF, FUSED>), grid, dim3(256), (conv_lds<WM, WN>(a)), st->stream, a.in, a.out, weights.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel,
+    hipLaunchKernelGGL((k_conv1d<WM, WN, KF, FUSED>), grid, dim3(256), (conv_lds<WM, WN>()), st->stream, a.in, a.out, weights.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel,
                        a.dilation, weights.tiles, a);
     return hip_check(hipGetLastError(), "conv1d launch", error, capacity);
 }
@@ -1181,7 +1355,7 @@ int launch_conv_split_p(State *st, const ConvArgs &a, const ConvBlocks &weights,
         raised = true;
     }
     const dim3 grid((unsigned)((a.length + 32 * NT - 1) / (32 * NT) * a.splits), (unsigned)((a.out_ch + 31) / 32));
-    hipLaunchKernelGGL((k_conv1d_split<KF, NT, PARTS>), grid, dim3(256), conv_split_lds<NT>(a), st->stream, a.in, a.out, weights.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel,
+    hipLaunchKernelGGL((k_conv1d_split<KF, NT, PARTS>), grid, dim3(256), conv_split_lds<NT>(), st->stream, a.in, a.out, weights.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel,
                        a.dilation, weights.tiles, a);
     return hip_check(hipGetLastError(), "conv1d launch", error, capacity);
 }
@@ -1224,12 +1398,10 @@ int launch_conv_split(State *st, const ConvArgs &a, const ConvBlocks &weights, c
     return launch_conv_split_n<2>(st, a, weights, error, capacity);
 }
 
-// LDS of the largest member
 template <int WM, int WN>
 int launch_conv_batch(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
     constexpr int TM = 32 * WM, TN = 64 * WN;
-    size_t lds = 0;
-    for (int i = 0; i < count; ++i) lds = conv_lds<WM, WN>(b.item[i]) > lds ? conv_lds<WM, WN>(b.item[i]) : lds;
+    constexpr size_t lds = conv_lds<WM, WN>();
     static bool raised = false;   // per instantiation
     if (!raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_batch<WM, WN>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
@@ -1243,8 +1415,7 @@ int launch_conv_batch(State *st, const ConvBatchArgs &b, int count, char *error,
 
 template <int NT, int PARTS>
 int launch_conv_split_batch_p(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
-    size_t lds = 0;
-    for (int i = 0; i < count; ++i) lds = conv_split_lds<NT>(b.item[i]) > lds ? conv_split_lds<NT>(b.item[i]) : lds;
+    constexpr size_t lds = conv_split_lds<NT>();
     static bool raised = false;
     if (!raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_split_batch<NT, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
@@ -1267,6 +1438,9 @@ int launch_conv_split_batch(State *st, const ConvBatchArgs &b, int count, char *
 
 int mynah::launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_ch, size_t in_ch, size_t kernel, char *error, size_t capacity) {
     const size_t blocks = (in_ch + 15) / 16, count = (out_ch + 31) / 32 * blocks * kernel * 64;
+    const size_t rows = (out_ch + 31) / 32 * 32;
+    float *const inverses = reinterpret_cast<float *>(dst + (count / 64) * 192);
+    hipLaunchKernelGGL(k_conv_row_scales, dim3((unsigned)rows), dim3(64), 0, st->stream, src, inverses, (int)out_ch, in_ch * kernel);
     hipLaunchKernelGGL(k_conv_pack, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st->stream, src, dst, count, (int)out_ch, (int)in_ch, (int)kernel, (int)blocks);
     return hip_check(hipGetLastError(), "weight packing launch", error, capacity);
 }

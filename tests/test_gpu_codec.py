@@ -1,5 +1,5 @@
 """GPU parity of the codec operators (mynah_hip_conv1d / _conv_transpose_dev / _snake_dev) against the oracle, through the
-C ABI.  conv1d runs in three-piece form on the bf16 matrix cores and adds in a different order than the CPU: 1e-5 normalised.  The transposed
+C ABI.  conv1d runs in two-piece form on the f16 matrix cores and adds in a different order than the CPU: 1e-5 normalised.  The transposed
 conv adds in the reference's order: bit-exact.  snake: the device sine against libm's, 1e-6 normalised."""
 import numpy as np
 import pytest
@@ -565,3 +565,25 @@ def test_res_layer_extremes(pkg, backend, C, L, taps):
     assert np.isfinite(one[:, 40:60]).any() and np.abs(one[:, 40:60][np.isfinite(one[:, 40:60])]).max() > 1e36   # (the large values are values)
     for d in bufs + [din]:
         d.free()
+
+
+def test_conv1d_input_sizes(backend):
+    """Inputs whose largest value lies on either side of the lines at which a tile is multiplied once more under a scale of its own (2^-10,
+    65520, 2^28), far from them, and rows of very different size side by side, in each kind of tile: f32's accuracy against float64."""
+    rng = np.random.default_rng(77)
+    for C, O, L, K, D in ((20, 70, 300, 7, 3), (27, 27, 500, 3, 1), (432, 64, 33, 3, 1), (216, 216, 320, 11, 1), (40, 48, 300, 5, 5)):
+        w = (rng.standard_normal((O, C, K)) / np.sqrt(C * K)).astype(np.float32)
+        w *= np.exp2(rng.integers(-60, 60, size=(O, 1, 1))).astype(np.float32)      # each output channel has a scale of its own
+        base = rng.uniform(-1, 1, size=(C, L)).astype(np.float32)
+        base[0, 0] = 1.0
+        for size in (2.0 ** -60, 2.0 ** -30, 2.0 ** -10 * (1 - 2.0 ** -20), 2.0 ** -10, 1.0, 65519.0, 65521.0, 2.0 ** 20, 2.0 ** 28 * (1 - 2.0 ** -20), 0.0):
+            _announce("conv1d input size %g, %d -> %d x %d, %d taps" % (size, C, O, L, K))
+            x = base * np.float32(size)
+            got = _run_conv1d(backend, x, w, np.zeros(O, np.float32), D).astype(np.float64)
+            want = np.zeros((O, L))
+            for k in range(K):
+                back = min((K - 1 - k) * D, L)
+                want[:, back:] += w[:, :, k].astype(np.float64) @ x[:, :L - back].astype(np.float64)
+            norm = np.linalg.norm(want, axis=1)
+            # every product's operands keep 22 bits, the sums f32's: 2^-22 a term and 2^-24 an addition of at most 150, of either sign
+            assert (np.linalg.norm(got - want, axis=1) <= 1e-6 * norm).all(), size
