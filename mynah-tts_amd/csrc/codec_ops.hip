@@ -20,7 +20,6 @@
 #include <type_traits>
 
 #include "half_product.h"
-#include "split_product.h"
 
 using namespace mynah;
 
@@ -1176,27 +1175,6 @@ int launch_res_block(State *st, const ResArgs &a, int count, char *error, size_t
     return hip_check(hipGetLastError(), "residual block launch", error, capacity);
 }
 
-// A weight's rows get a scale each: the largest value under it lies in [2^13, 2^14), unless it is 2^20 times the row's usual size and
-// more -- then what is 2^20 times that lies there, and what does not fit above it is kept as its bits (half_product.h).  A wavefront a row.
-__global__ void __launch_bounds__(64) k_conv_row_scales(const float *src, float *inverses, int out_ch, size_t per_row) {
-    const int row = (int)blockIdx.x, lane = (int)threadIdx.x;
-    float sum = 0.0f, count = 0.0f, most = -127.0f;
-    if (row < out_ch)
-        for (size_t i = lane; i < per_row; i += 64) {
-            const float v = src[(size_t)row * per_row + i];
-            const int e = exponent_of(v);
-            if (v == 0.0f || e == 128) continue;   // (nothing, or no finite number)
-            sum += (float)e;
-            count += 1.0f;
-            most = fmaxf(most, (float)e);
-        }
-    sum = wave_sum(sum);
-    count = wave_sum(count);
-    most = wave_max(most);
-    const int top = count == 0.0f ? 13 : (int)fminf(most, floorf(sum / count) + 20.0f);
-    if (lane == 0) inverses[row] = power_of_two(max(top - 13, -126));
-}
-
 __global__ void __launch_bounds__(256) k_conv_pack(const float *src, uint4 *dst, size_t count, int out_ch, int in_ch, int kernel, int blocks) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= count) return;
@@ -1206,27 +1184,14 @@ __global__ void __launch_bounds__(256) k_conv_pack(const float *src, uint4 *dst,
     const size_t o = tile * 32 + (lane & 31);
     const int c0 = block * 16 + (lane >> 5) * 8;
     const float scale = 1.0f / conv_inverses(dst, steps)[o];
-    ushort8_t at[3];
+    float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-        float v[2], rest[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) v[k] = o < (size_t)out_ch && c0 + e + k < in_ch ? src[(o * in_ch + c0 + e + k) * kernel + tap] : 0.0f;
-        unsigned h, m;
-        half_pieces(v[0], v[1], scale, h, m, rest);
-        const unsigned l = half_third(m, rest);
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {   // (the kernels have no other copy of a weight)
-            unsigned short ph = (unsigned short)(h >> 16 * k), pm = (unsigned short)(m >> 16 * k), pl = (unsigned short)(l >> 16 * k);
-            half_keep_bits(v[k], scale, ph, pm, pl);
-            at[0][e + k] = ph;
-            at[1][e + k] = pm;
-            at[2][e + k] = pl;
-        }
-    }
-    dst[step * 128 + lane] = __builtin_bit_cast(uint4, at[0]);
-    dst[step * 128 + 64 + lane] = __builtin_bit_cast(uint4, at[1]);
-    dst[steps * 128 + step * 64 + lane] = __builtin_bit_cast(uint4, at[2]);
+    for (int e = 0; e < 8; ++e) v[e] = o < (size_t)out_ch && c0 + e < in_ch ? src[(o * in_ch + c0 + e) * kernel + tap] : 0.0f;
+    uint4 piece[3];
+    half_keep_eight(v, scale, piece);   // (the kernels have no other copy of a weight)
+    dst[step * 128 + lane] = piece[0];
+    dst[step * 128 + 64 + lane] = piece[1];
+    dst[steps * 128 + step * 64 + lane] = piece[2];
 }
 
 struct ConvTransposeArgs {
@@ -1440,7 +1405,7 @@ int mynah::launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_
     const size_t blocks = (in_ch + 15) / 16, count = (out_ch + 31) / 32 * blocks * kernel * 64;
     const size_t rows = (out_ch + 31) / 32 * 32;
     float *const inverses = reinterpret_cast<float *>(dst + (count / 64) * 192);
-    hipLaunchKernelGGL(k_conv_row_scales, dim3((unsigned)rows), dim3(64), 0, st->stream, src, inverses, (int)out_ch, in_ch * kernel);
+    if (launch_half_row_scales(st, src, inverses, out_ch, rows, in_ch * kernel, error, capacity) != 0) return -1;
     hipLaunchKernelGGL(k_conv_pack, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st->stream, src, dst, count, (int)out_ch, (int)in_ch, (int)kernel, (int)blocks);
     return hip_check(hipGetLastError(), "weight packing launch", error, capacity);
 }

@@ -26,6 +26,7 @@ namespace mynah {
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned short ushort4_t __attribute__((ext_vector_type(4)));
 typedef unsigned short ushort8_t __attribute__((ext_vector_type(8)));
 
@@ -54,8 +55,16 @@ __device__ __forceinline__ unsigned half_third(unsigned m, const float (&rest)[2
     return half_pair((rest[0] * kHalfStep - (float)mm[0]) * kHalfStep, (rest[1] * kHalfStep - (float)mm[1]) * kHalfStep);
 }
 // Where pieces are all that is kept of an operand, one without a finite first piece is kept as (infinity, upper half, lower half of its
-// bits): it makes its products infinite or NaN as it must, and can be had again.
+// bits): it makes its products infinite or NaN as it must, and can be had again.  One so far below the scale that its first two pieces are
+// zero is kept as (-0, 0, its upper half, rounded).
+constexpr float kHalfNothing = 0x1p-37f;
 __device__ __forceinline__ void half_keep_bits(float x, float scale, unsigned short &h, unsigned short &m, unsigned short &l) {
+    if (x != 0.0f && fabsf(x * scale) < kHalfNothing) {
+        h = 0x8000;
+        m = 0;
+        l = (unsigned short)((__float_as_uint(x) + 0x8000u) >> 16);
+        return;
+    }
     if (fabsf(x * scale) < kHalfLimit) return;
     h = kHalfMarked;
     m = (unsigned short)(__float_as_uint(x) >> 16);
@@ -63,6 +72,7 @@ __device__ __forceinline__ void half_keep_bits(float x, float scale, unsigned sh
 }
 __device__ __forceinline__ float half_value(unsigned short h, unsigned short m, unsigned short l, float inverse) {
     if (h == kHalfMarked) return __uint_as_float((unsigned)m << 16 | l);
+    if (h == 0x8000 && m == 0) return __uint_as_float((unsigned)l << 16);
     const auto f = [](unsigned short b) { return (float)__builtin_bit_cast(_Float16, b); };
     return (f(h) + (f(m) + f(l) * (1.0f / kHalfStep)) * (1.0f / kHalfStep)) * inverse;   // exact
 }
@@ -88,8 +98,43 @@ __device__ __forceinline__ int half_rescale(float largest) {
     return quiet || loud ? min(13 - exponent_of(largest), 100) : 0;
 }
 
+// The three pieces of eight values, or their bits: where they are all that is kept of an operand.
+__device__ __forceinline__ void half_keep_eight(const float (&v)[8], float scale, uint4 (&piece)[3]) {
+    ushort8_t at[3];
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        unsigned h, m;
+        float rest[2];
+        half_pieces(v[e], v[e + 1], scale, h, m, rest);
+        const unsigned l = half_third(m, rest);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            unsigned short ph = (unsigned short)(h >> 16 * k), pm = (unsigned short)(m >> 16 * k), pl = (unsigned short)(l >> 16 * k);
+            half_keep_bits(v[e + k], scale, ph, pm, pl);
+            at[0][e + k] = ph;
+            at[1][e + k] = pm;
+            at[2][e + k] = pl;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) piece[q] = __builtin_bit_cast(uint4, at[q]);
+}
+
+__device__ __forceinline__ bool split_finite(float x) { return fabsf(x) < __builtin_inff(); }
+// Whether all sums of the wavefront are finite (one instruction a value: 0 * x is 0 or NaN).
+template <int N>
+__device__ __forceinline__ bool split_all_finite(const f32x16 (&acc)[N]) {
+    float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zero[r & 3] = __builtin_fmaf(acc[n][r], 0.0f, zero[r & 3]);
+    return !__any((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.0f);
+}
+// Row of C held in accumulator register r of lane l for a 32x32 tile; the column is l % 32.
+__device__ __forceinline__ int split_acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+
 struct HalfSums {   // a 32 x 32 tile: the products of the first pieces, and the small ones in units of 2^-11
-    typedef float f32x16 __attribute__((ext_vector_type(16)));
     f32x16 large, small;
     __device__ __forceinline__ void clear() { large = small = f32x16{0}; }
     // One 16-deep step.
