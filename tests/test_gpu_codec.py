@@ -587,3 +587,37 @@ def test_conv1d_input_sizes(backend):
             norm = np.linalg.norm(want, axis=1)
             # every product's operands keep 22 bits, the sums f32's: 2^-22 a term and 2^-24 an addition of at most 150, of either sign
             assert (np.linalg.norm(got - want, axis=1) <= 1e-6 * norm).all(), size
+
+
+@pytest.mark.parametrize("stride,kernel", [(2, 4), (4, 8), (8, 16), (2, 2), (2, 3), (4, 5), (8, 11), (4, 9), (8, 5), (3, 6), (1, 2)])
+def test_conv_transpose_forms(backend, stride, kernel):
+    """Strides and kernels on both sides of the vector form's rule, outputs that end before, at and behind the inputs' reach, rows at any
+    alignment: bit for bit the sums in the reference's order (input channel, then input position), guard values around the output."""
+    rng = np.random.default_rng(10 * stride + kernel)
+    for in_ch, out_ch, groups in ((4, 2, 2), (3, 1, 1), (6, 4, 2)):
+        for length in (1, 2, 37, 300):
+            for output in sorted({1, max(1, length * stride - 1), length * stride, (length - 1) * stride + kernel, length * stride + stride + 1}):
+                _announce("conv_transpose stride=%d kernel=%d %d -> %d in %d groups, %d -> %d" % (stride, kernel, in_ch, out_ch, groups, length, output))
+                ipg, opg = in_ch // groups, out_ch // groups
+                x = rng.standard_normal((in_ch, length)).astype(np.float32)
+                w, b = rng.standard_normal((in_ch, opg, kernel)).astype(np.float32), rng.standard_normal(out_ch).astype(np.float32)
+                want = np.zeros((out_ch, output), np.float32) + b[:, None]
+                position = np.arange(output)
+                for o in range(out_ch):
+                    for i in range((o // opg) * ipg, (o // opg + 1) * ipg):
+                        for back in range(-(-kernel // stride) - 1, -1, -1):         # earlier inputs first
+                            t = position // stride - back
+                            k = position - t * stride
+                            ok = (t >= 0) & (t < length) & (k < kernel)
+                            want[o, ok] = want[o, ok] + x[i, t[ok]] * w[i, o % opg, k[ok]]
+                        reach = (position // stride > length - 1)                   # (behind the last input: counted from the last)
+                        assert not (reach & (position - (length - 1) * stride < kernel) & (position // stride - (length - 1) >= -(-kernel // stride))).any()
+                for lead in (0, 1):
+                    din = backend.alloc(x.size).write(x)
+                    dout = backend.alloc(out_ch * output + 3).write(np.full(out_ch * output + 3, 7.0, np.float32))
+                    backend.conv_transpose_dev(din.ptr, dout.ptr + 4 * lead, in_ch, out_ch, length, output, kernel, stride, groups, w, b)
+                    got = dout.read()
+                    assert np.array_equal(got[lead:lead + want.size].reshape(want.shape), want)
+                    assert (got[:lead] == 7.0).all() and (got[lead + want.size:] == 7.0).all()
+                    din.free()
+                    dout.free()
