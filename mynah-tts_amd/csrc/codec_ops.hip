@@ -1742,14 +1742,18 @@ extern "C" int mynah_hip_rows_combine_dev(void *state, const float *const *dev_i
 }
 
 // The one-launch build for a position of a layer, or none.  Which are there follows the order in which the layer's convolutions add
-// (conv_takes_split) and whether all workgroups find a place at once: two to a CU (512 threads: one), 32 positions to a wavefront,
-// whose chain of products is then half as long, before 64.  Measured per layer of three positions, branches of 3 / 7 / 11 taps, us:
-//   27 channels: x 12288 67 narrow, 86 wide, 106 as two launches a position; x 20480 75, 90, 116; x 24576 (more than fit) 112, 100, 117
-//   54, split order: x 2560 84 narrow, 72 as two launches of split tiles; x 3072 85, 82; x 3584 86, 86; x 4608 86, 91; x 8192 98, 137; x 10240 137, 152
-//   54, large order: x 12288 140 wide, 164 as two launches; x 16384 161, 173; x 20480 173, 199; x 20992 (more than fit) 229, 201
-//   108, large order, 3 and 11 taps: x 6144 173 narrow, 202; x 8192 186, 204; x 12288 (more than fit) 276, 240
+// (conv_takes_split) and how many workgroups find a place at once: three to a CU with 32 positions to a wavefront (narrow), whose chain of
+// products is half as long, two with 64 (wide), one of 512 threads.  Narrow while all find a place; else wide while all of those do; else whichever
+// needs less time for its rounds.  Measured per layer of three positions, branches of 3 / 7 / 11 taps, us:
+//   27 channels: x 5120 47 narrow, 65 wide, 84 as two launches a position; x 28672 74, 84, 105; x 32768 (more than three to a CU) 98, 85, 111;
+//     x 40960 107, 89; x 43008 (more wide than two to a CU) 108, 129; x 65536 145, 150, 160
+//   54, split order: x 64 54 narrow, 56 as two launches; x 1024 57, 59; x 5120 71, 82; x 10240 82, 137
+//   54, large order: x 13824 92 narrow, 104 wide, 127 as two launches; x 16384 133, 113, 133; x 20480 141, 120, 154; x 22528 152, 164, 163; x 28672
+//     160, 179, 175; x 32768 193, 201, 202; x 40960 229, 200, 268
+//   108, large order, 3 and 11 taps: x 6144 173 narrow, 202; x 8192 186, 204; x 12288 (more than fit) 276, 240; three branches: x 6144 155, 160;
+//     x 7168 175, 165
 // (three branches of 65 to 128 channels are never in the large order and few enough)
-enum ResBuild { RES_NONE, RES_32_NARROW, RES_32_WIDE, RES_64_SPLIT, RES_64_WIDE, RES_128 };
+enum ResBuild { RES_NONE, RES_32_NARROW, RES_32_WIDE, RES_64_SPLIT, RES_64_NARROW, RES_64_WIDE, RES_128 };
 static ResBuild res_build(const State *st, const mynah_hip_res_block *blocks, size_t branches, size_t stride, size_t channels, size_t length) {
     if (channels > (size_t)kResMaxChannels) return RES_NONE;
     for (size_t i = 0; i < branches; ++i) {
@@ -1761,11 +1765,11 @@ static ResBuild res_build(const State *st, const mynah_hip_res_block *blocks, si
         for (size_t i = 0; i < branches; ++i) n += ((long)length + columns - blocks[i * stride].kernel_in) / (columns - (blocks[i * stride].kernel_in - 1));
         return n <= (long)st->cu_count * each;
     };
-    if (channels <= 32) return fit(128, 2) ? RES_32_NARROW : RES_32_WIDE;
+    if (channels <= 32) return fit(128, 3) || !fit(256, 2) ? RES_32_NARROW : RES_32_WIDE;
     const bool split = conv_takes_split(st, (int)channels, (int)channels, (int)length);
     if (channels > 64) return !split && fit(64, 1) ? RES_128 : RES_NONE;
-    if (split) return 2 * (long)((length + 63) / 64) * (long)branches * 4 < (long)st->cu_count * 5 ? RES_NONE : RES_64_SPLIT;
-    return fit(128, 2) ? RES_64_WIDE : RES_NONE;
+    if (split) return RES_64_SPLIT;
+    return fit(64, 3) || (!fit(128, 2) && fit(64, 7)) ? RES_64_NARROW : RES_64_WIDE;
 }
 
 // One position (block) of every branch in one launch, where there is a build for it; *done tells.
@@ -1810,6 +1814,7 @@ static int res_position(State *st, const mynah_hip_res_block *blocks, size_t bra
         case RES_32_NARROW: return launch_res_block<1, 4, 1>(st, a, (int)branches, error, capacity);
         case RES_32_WIDE: return launch_res_block<1, 4, 2>(st, a, (int)branches, error, capacity);
         case RES_64_SPLIT: return launch_res_block<2, 2, 1, true>(st, a, (int)branches, error, capacity);
+        case RES_64_NARROW: return launch_res_block<2, 2, 1>(st, a, (int)branches, error, capacity);
         case RES_64_WIDE: return launch_res_block<2, 2, 2>(st, a, (int)branches, error, capacity);
         default: return launch_res_block<4, 2, 1>(st, a, (int)branches, error, capacity);
     }
