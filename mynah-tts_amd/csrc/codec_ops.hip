@@ -114,20 +114,6 @@ __device__ __forceinline__ void conv_emit(const ConvArgs &a, int m, size_t index
 // products 44,000 (its matrix instructions alone 28,000; without the weights' requests 31,500, without the LDS reads 38,000), residual
 // and stores 15,000, all workgroups at the same time.  As three bf16 pieces, with 64-bit addresses a lane and request that spilled, the
 // first product came after 35,000 and the launch took 55 us (now 41).
-// A value at `bytes` behind an address that is the same for every lane: one instruction with the address in scalar registers, where
-// pointer arithmetic by lanes takes 64-bit addresses in vector registers.
-// (opaque: what stays the same from request to request is otherwise added up ahead of all loops, 64 bits a lane and request)
-template <class T>
-__device__ __forceinline__ T load_behind(const T *base, unsigned bytes) { return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes); }
-__device__ __forceinline__ unsigned opaque(unsigned v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-__device__ __forceinline__ int opaque_scalar(int v) {
-    asm volatile("" : "+s"(v));
-    return v;
-}
-
 struct ConvWeights {   // the weight pieces of one row tile, requested kAhead steps before they are multiplied
     static constexpr int kAhead = kConvStepsAhead;
     const uint4 *next;   // the same for every lane, like the inputs' rows below: an address is then a pair of scalar registers and the lane's offset, where

@@ -98,6 +98,20 @@ __device__ __forceinline__ int half_rescale(float largest) {
     return quiet || loud ? min(13 - exponent_of(largest), 100) : 0;
 }
 
+// A value at `bytes` behind an address that is the same for every lane: one instruction with the address in scalar registers, where
+// pointer arithmetic by lanes takes 64-bit addresses in vector registers.
+// (opaque: what stays the same from request to request is otherwise added up ahead of all loops, 64 bits a lane and request)
+template <class T>
+__device__ __forceinline__ T load_behind(const T *base, unsigned bytes) { return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes); }
+__device__ __forceinline__ unsigned opaque(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ int opaque_scalar(int v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
 // The three pieces of eight values, or their bits: where they are all that is kept of an operand.
 __device__ __forceinline__ void half_keep_eight(const float (&v)[8], float scale, uint4 (&piece)[3]) {
     ushort8_t at[3];

@@ -1,6 +1,8 @@
 // Products of many f32 rows with a weight, in f32, on the f16 matrix cores (half_product.h): the encoder prefill with f32
 // operands and the cross-attention K/V.  out[m][n] = sum over taps j and channels c of in[m - (taps - 1) + j][c] * W[n][c][j]; one tap is
 // a plain product, three are the causal convolution of the encoder's FFN (causal_conv_ffn, src/graph.c:302-352).
+#include <type_traits>
+
 #include "half_product.h"
 
 namespace mynah {
@@ -285,6 +287,161 @@ __global__ void __launch_bounds__(512) k_split_cross_kv(const float *const norme
     split_store<2, 1>(normed + (size_t)layer * M * width, width, m0, M, weight.values() + step * 128, width / 32, acc, out, xw);
 }
 
+// The same for more than 64 rows: a workgroup takes 64 * MT rows and 128 columns of a layer, wavefront w rows 32 MT (w / 4) .. and columns
+// 32 (w % 4) .. over all channels.  What a CU has to fetch bounds these products -- 64 rows a workgroup are 24 KB for 384 cycles of its matrix cores, 42 us
+// at 180 rows x 12 layers, 35 % of what it fetches the weight's third reading -- so the rows go as far as the registers do.  The rows come
+// normalised once, without any layer's gain and bias, which are applied as they are staged (the same operations in the same order as a
+// LayerNorm of each layer's own, which wrote and read twelve times the rows).
+template <int MT>
+struct WideTile {
+    static constexpr int kRows = 64 * MT, kPitch = kRows + 4;
+    uint4 a[2][2][2][2][kPitch];   // [stage][16-deep half][piece][8-deep quarter][row]
+    float largest[8];
+};
+template <int MT, bool BIAS>
+__global__ void __launch_bounds__(512) k_wide_cross_kv(const float *const rows_in, const SplitLayers layers, const int M, const int width, const int xw,
+                                                       const int mtiles, float *const k_out, float *const v_out) {
+    using Tile = WideTile<MT>;
+    extern __shared__ __align__(16) unsigned char smem[];
+    Tile &lds = *reinterpret_cast<Tile *>(smem);
+    const int N = 2 * xw, ntiles = (N + 127) / 128;
+    const SplitWork work((int)blockIdx.x, mtiles);
+    if (work.nz >= ntiles) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 2, wn = wave & 3, layer = (int)blockIdx.y;
+    const int srow = tid >> 3, sc = tid & 7, blocks = width / 32;
+    const int col0 = work.nz * 128 + wn * 32, m0 = work.m * Tile::kRows;
+    const float *const gain = layers.gain[layer], *const bias = layers.bias[layer];
+    const SplitWeight weight(layers.w[layer], (size_t)N, (size_t)width, 1);
+    const size_t step0 = (size_t)(min(col0, N - 32) / 32) * blocks * 2;
+    const float inverse = weight.inverses()[min(col0, N - 32) + (lane & 31)];
+    constexpr int kStage = 2 * 2 * 2 * Tile::kPitch;
+    uint4 *const stages = &lds.a[0][0][0][0][0];
+    float scale = 1.0f, unscale = 1.0f, largest = 0.0f;
+    HalfSums sums[MT];
+    for (bool once_more = false;; once_more = true) {
+        // (an address the same for every lane and 32 bits of a lane's own: less registers than a pointer a row)
+        const float *const rows0 = rows_in + (size_t)m0 * width;
+        unsigned at[MT], own = 16u * sc, lane_bytes = 16u * lane;
+#pragma unroll
+        for (int i = 0; i < MT; ++i) at[i] = ((unsigned)(min(m0 + srow + 64 * i, M - 1) - m0) * (unsigned)width + 4u * sc) * 4u;
+        float4 ra[2][MT], rg[2], rb[BIAS ? 2 : 1];
+        const auto request_a = [&](int set, int block) {   // (past the last block: the last one again)
+            const size_t channel = (size_t)min(block, blocks - 1) * 32;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                at[i] = opaque(at[i]);
+                ra[set][i] = load_behind(reinterpret_cast<const float4 *>(rows0 + channel), at[i]);
+            }
+            own = opaque(own);
+            rg[set] = load_behind(reinterpret_cast<const float4 *>(gain + channel), own);
+            if constexpr (BIAS) rb[set] = load_behind(reinterpret_cast<const float4 *>(bias + channel), own);
+        };
+        const auto store_a = [&](int set, uint4 *stage) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                float4 v = ra[set][i];
+                v.x *= rg[set].x; v.y *= rg[set].y; v.z *= rg[set].z; v.w *= rg[set].w;
+                if constexpr (BIAS) { v.x += rb[set].x; v.y += rb[set].y; v.z += rb[set].z; v.w += rb[set].w; }
+                uint2 piece[2];
+                float rest[2];
+                half_pieces(v.x, v.y, scale, piece[0].x, piece[1].x, rest);
+                half_pieces(v.z, v.w, scale, piece[0].y, piece[1].y, rest);
+                largest = fmaxf(largest, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    reinterpret_cast<uint2 *>(&stage[(((sc >> 2) * 2 + q) * 2 + ((sc >> 1) & 1)) * Tile::kPitch + srow + 64 * i])[sc & 1] = piece[q];
+            }
+        };
+        const uint4 *wp = layers.w[layer] + step0 * 128;
+        uint4 rw[4][2];
+        const auto request_w = [&](int slot, int step) {
+            lane_bytes = opaque(lane_bytes);
+            rw[slot][0] = load_behind(wp + step * 128, lane_bytes);
+            rw[slot][1] = load_behind(wp + step * 128 + 64, lane_bytes);
+        };
+#pragma unroll
+        for (int t = 0; t < MT; ++t) sums[t].clear();
+        request_a(0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) request_w(i, i);
+        request_a(1, 1);
+        store_a(0, stages);
+        request_a(0, 2);
+        __syncthreads();
+        for (int block = 0; block < blocks; block += 2) {   // (an even number of blocks)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const uint4 *const now = stages + u * kStage;
+                store_a((u + 1) & 1, stages + (1 - u) * kStage);
+                request_a((u + 1) & 1, block + u + 3);
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    const int s = 2 * u + half;
+                    half8_t fw[2], fa[MT][2];
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q)
+                            fa[t][q] = __builtin_bit_cast(half8_t, now[((half * 2 + q) * 2 + (lane >> 5)) * Tile::kPitch + wm * 32 * MT + 32 * t + (lane & 31)]);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) fw[q] = __builtin_bit_cast(half8_t, rw[s][q]);
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) sums[t].multiply(fa[t], fw);
+                    request_w(s, s + 4);   // into the registers multiplied here
+                }
+                __syncthreads();   // the block stored here may be read, and the one read here overwritten
+            }
+            wp += 4 * 128;
+        }
+        largest = wave_max(largest);
+        if (lane == 0) lds.largest[wave] = largest;
+        __syncthreads();
+        float of_all = lds.largest[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) of_all = fmaxf(of_all, lds.largest[i]);
+        const int e = once_more ? 0 : __builtin_amdgcn_readfirstlane(half_rescale(of_all));
+        if (__builtin_expect(e == 0, 1)) break;
+        scale = power_of_two(e);
+        unscale = power_of_two(-e);
+    }
+    if (col0 >= N) return;
+    f32x16 acc[MT];
+    float *const out = (col0 < xw ? k_out + col0 : v_out + col0 - xw) + (size_t)layer * M * xw + (lane & 31);
+    const int row0 = m0 + wm * 32 * MT;
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            acc[t][r] = sums[t].sum(r) * unscale * inverse;
+            const int m = row0 + 32 * t + split_acc_row(r, lane);
+            if (m < M) out[(size_t)m * xw] = acc[t][r];
+        }
+    if (split_all_finite(acc)) return;
+    // (see split_store)
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll 1
+        for (int r = 0; r < 16; ++r) {
+            const int m = row0 + 32 * t + split_acc_row(r, lane);
+            if (m >= M || split_finite(acc[t][r])) continue;
+            const float *const x = rows_in + (size_t)m * width;
+            const float4 *const values = weight.values() + step0 * 128 + (lane & 31);
+            float s = 0.0f;
+#pragma unroll 1
+            for (int c = 0; c < width && s == s; c += 4) {
+                const float4 v = values[(size_t)(c >> 4) * 128 + ((c >> 2) & 1) * 64 + ((c >> 3) & 1) * 32];
+                const float w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float n = x[c + e] * gain[c + e];
+                    if constexpr (BIAS) n += bias[c + e];
+                    s = __builtin_fmaf(n, w4[e], s);
+                }
+            }
+            out[(size_t)m * xw] = s;
+        }
+}
+
 // The memory's rows under every layer's LayerNorm (gain, optional bias), one workgroup per row and layer: normed[layer][row].
 __global__ void __launch_bounds__(256) k_layernorm_layers(const float *in, float *normed, const SplitLayers layers, int rows, int width) {
     __shared__ float s4[4];
@@ -366,8 +523,42 @@ int launch_split_product(State *st, const float *in, const uint4 *w, size_t rows
     return hip_check(hipGetLastError(), "f32 product launch", error, capacity);
 }
 
+template <int MT, bool BIAS>
+static int launch_wide(State *st, size_t rows, size_t width, const SplitLayers &layers, size_t count, size_t xw, const float *normed, float *k_out, float *v_out,
+                       char *error, size_t capacity) {
+    static bool raised = false;
+    if (!raised) {
+        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_wide_cross_kv<MT, BIAS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(WideTile<MT>)));
+        raised = true;
+    }
+    const size_t mtiles = (rows + 64 * MT - 1) / (64 * MT);
+    hipLaunchKernelGGL((k_wide_cross_kv<MT, BIAS>), dim3((unsigned)(((2 * xw + 127) / 128 + 7) / 8 * 8 * mtiles), (unsigned)count), dim3(512), sizeof(WideTile<MT>),
+                       st->stream, normed, layers, (int)rows, (int)width, (int)xw, (int)mtiles, k_out, v_out);
+    return hip_check(hipGetLastError(), "cross K/V launch", error, capacity);
+}
+
 int launch_split_cross_kv(State *st, const float *memory, size_t rows, size_t width, const SplitLayers &layers, size_t count, size_t xw, float *normed,
                           float *k_out, float *v_out, char *error, size_t capacity) {
+    bool biased = false, plain = false;
+    for (size_t l = 0; l < count; ++l) (layers.bias[l] != nullptr ? biased : plain) = true;
+    // Above 64 rows (all layers with a bias or all without: a launch is one build or the other).  us with the LayerNorm, 12 layers of 768,
+    // the wide product / 64 rows a workgroup: 48 rows 21.7 / 20.9, 64 22.1 / 22.0, 65 27.6 / 32.6, 128 28.6 / 34.4, 180 38 / 50
+    if (rows > 64 && !(biased && plain)) {
+        SplitLayers none{};   // (null gain: ones)
+        hipLaunchKernelGGL(k_layernorm_layers, dim3((unsigned)rows, 1), dim3(256), 0, st->stream, memory, normed, none, (int)rows, (int)width);
+        const size_t tiles = (rows + 255) / 256, mt = ((rows + tiles - 1) / tiles + 63) / 64;   // as few row tiles as there must be, and those small
+        const auto launch = [&](auto mt_constant) {
+            constexpr int MT = decltype(mt_constant)::value;
+            return biased ? launch_wide<MT, true>(st, rows, width, layers, count, xw, normed, k_out, v_out, error, capacity)
+                          : launch_wide<MT, false>(st, rows, width, layers, count, xw, normed, k_out, v_out, error, capacity);
+        };
+        switch (mt) {
+            case 1: return launch(std::integral_constant<int, 1>{});
+            case 2: return launch(std::integral_constant<int, 2>{});
+            case 3: return launch(std::integral_constant<int, 3>{});
+            default: return launch(std::integral_constant<int, 4>{});
+        }
+    }
     hipLaunchKernelGGL(k_layernorm_layers, dim3((unsigned)rows, (unsigned)count), dim3(256), 0, st->stream, memory, normed, layers, (int)rows, (int)width);
     const int mtiles = (int)((rows + 63) / 64), ntiles = (int)((2 * xw + 127) / 128);
     hipLaunchKernelGGL(k_split_cross_kv, dim3((unsigned)((ntiles + 7) / 8 * 8 * mtiles), (unsigned)count), dim3(512), 0, st->stream, normed, layers, (int)rows,

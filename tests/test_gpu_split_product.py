@@ -214,3 +214,34 @@ def test_workspace_and_weight_memory(backend, pkg, synth):
     assert backend.cached_weight_bytes() - kept == (2 * 3 * 7 + 3) * 3072
     x.free()
     y.free()
+
+
+@pytest.mark.parametrize("bias", ["none", "all", "some"])
+@pytest.mark.parametrize("rows", [65, 128, 129, 193, 256, 257, 300])
+def test_cross_kv_wide_tiles(backend, pkg, orc, rows, bias):
+    """More rows than one 64-row tile, in workgroups of 64 to 256: the last row of a tile and the first of the next, widths that end inside a
+    128-column tile, with and without LayerNorm biases (and in only some of the layers: the narrow tiles), an infinity in one row."""
+    print("[gpu-case] cross K/V wide rows=%d bias=%s" % (rows, bias), flush=True)
+    rng = np.random.default_rng(rows)
+    backend.set_quant(pkg.F32)
+    width, xw, layers = 128, 96, 3
+    gains = [backend.keep((1.0 + 0.1 * rng.standard_normal(width)).astype(np.float32)) for _ in range(layers)]
+    biases = [backend.keep(rng.standard_normal(width).astype(np.float32)) if bias == "all" or (bias == "some" and l == 1) else None for l in range(layers)]
+    kvw = [backend.keep(rng.standard_normal((2 * xw, width)).astype(np.float32)) for _ in range(layers)]
+    memory = rng.standard_normal((rows, width)).astype(np.float32)
+    memory[rows - 2, 5] = np.inf
+    dmem = backend.alloc(rows * width).write(memory)
+    guard = np.full(xw, 7.0, np.float32)
+    dk, dv = (backend.alloc(layers * rows * xw + xw).write(guard, layers * rows * xw) for _ in range(2))
+    backend.cross_kv_dev(dmem.ptr, rows, width, gains, None if bias == "none" else biases, kvw, xw, dk.ptr, dv.ptr)
+    gk, gv = dk.read(), dv.read()
+    assert np.array_equal(gk[-xw:], guard) and np.array_equal(gv[-xw:], guard)
+    got = np.concatenate([gk[:-xw].reshape(layers, rows, xw), gv[:-xw].reshape(layers, rows, xw)], axis=2).astype(np.float64)
+    keep = np.arange(rows) != rows - 2
+    assert np.isnan(got[:, rows - 2]).all()
+    for l in range(layers):
+        normed = np.stack([orc.layernorm(r, gains[l], biases[l]) for r in memory[keep]]).astype(np.float64)
+        want = normed @ kvw[l].astype(np.float64).T
+        assert np.linalg.norm(got[l][keep] - want) < 1e-6 * np.linalg.norm(want), l       # (22 bits an operand, f32 sums of 128 terms)
+    for d in (dmem, dk, dv):
+        d.free()
