@@ -18,6 +18,7 @@
 #include <stddef.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "half_product.h"
 
@@ -312,6 +313,7 @@ constexpr int conv_pitch(int positions) { return positions + kConvMaxHalo; }
 struct ConvTileRows {
     alignas(16) float inverse[64], bias[64];
     float largest[4];
+    float alpha[32], inverse_alpha[32];   // (channel-split tiles) of the rows' half-snake, and 1 / (alpha + 1e-9)
 };
 
 // Workgroup tile: (32 * WM) output channels x (64 * WN) positions; a wavefront owns 32 x 64 (two 32 x 32 tiles of sums).
@@ -595,7 +597,15 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[n].clear();
     float scale = 1.0f, unscale = 1.0f;   // (this wavefront's: its sums are its own)
-    if (tid < TM) s_rows.inverse[tid] = conv_inverses(w_arg.data, (size_t)w_arg.tiles * w_arg.blocks * a.kernel)[m0 + tid];
+    // what the finished rows need (behind the products each request would be a round trip of its own)
+    if (tid < TM) {
+        const int m = m0 + tid;
+        const float al = a.activate && m < a.snake_channels ? a.alpha[m] : 0.0f;
+        s_rows.inverse[tid] = conv_inverses(w_arg.data, (size_t)w_arg.tiles * w_arg.blocks * a.kernel)[m];
+        s_rows.bias[tid] = a.bias != nullptr && m < a.out_ch ? a.bias[m] : 0.0f;
+        s_rows.alpha[tid] = al;
+        s_rows.inverse_alpha[tid] = 1.0f / (al + 1e-9f);
+    }
     const int mine = (w_arg.blocks - rank + sharing - 1) / sharing;   // this wavefront's blocks
     if (mine > 0) {
         ConvColumn column[2][PARTS];
@@ -642,6 +652,23 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
             for (int n = 0; n < NT; ++n) acc[n].clear();
         }
     }
+    // A thread finishes the tile's values at (row wave + 4 j, position lane): a store instruction then covers one row's 64
+    // consecutive positions and whether the row exists is the same for all its lanes (in the accumulators' order an
+    // instruction covers halves of two rows, four apart).  e: where that value sits in a partial tile (element r of lane l).
+    // Residuals are requested here, side by side, before the wavefronts meet, and the activation is straight-line code for all eight values: in
+    // a loop a value at a time, with the requests where they are used, the finish was 7,000 to 9,000 of 18,000 cycles (108 channels x 1280).
+    const int pos = lane, t = t0 + pos;
+    const bool t_ok = (NT > 1 || pos < 32) && t < a.length;
+    float first[8], second[8];
+    const auto at = [&](int j) { return (size_t)min(m0 + wave + 4 * j, a.out_ch - 1) * a.length + min(t, a.length - 1); };
+    if (a.residual != nullptr && a.splits == 1) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) first[j] = a.residual[at(j)];
+        if (a.residual2 != nullptr) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) second[j] = a.residual2[at(j)];
+        }
+    }
     __syncthreads();   // the partial tiles below overwrite every wavefront's staging area
     // partial tiles through LDS: [wavefront][element r][lane], then ((p0 + p1) + p2) + p3 + bias
     float *s_part = reinterpret_cast<float *>(lds);
@@ -650,17 +677,11 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
 #pragma unroll
         for (int r = 0; r < 16; ++r) s_part[(wave * 32 + 16 * n + r) * 64 + lane] = acc[n].sum(r) * unscale * s_rows.inverse[split_acc_row(r, lane)];
     __syncthreads();
-    // A thread finishes the tile's values at (row (tid / 64) + 4 j, position tid % 64): a store instruction then covers one
-    // row's 64 consecutive positions and whether the row exists is the same for all its lanes (in the accumulators' order an
-    // instruction covers halves of two rows, four apart).  e: where that value sits in a partial tile (element r of lane l).
-    const int pos = tid & 63;
-    const int t = t0 + pos;
-    const bool t_ok = (NT > 1 || pos < 32) && t < a.length;
     float sum[8], zero = 0.0f;
     const auto add_parts = [&]() {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const int row = (tid >> 6) + 4 * j;
+            const int row = wave + 4 * j;
             const int e = ((((row >> 3) << 2) | (row & 3)) + 16 * (pos >> 5)) * 64 + ((row >> 2) & 1) * 32 + (pos & 31);
             sum[j] = ((s_part[e] + s_part[2048 + e]) + s_part[4096 + e]) + s_part[6144 + e];
             zero = __builtin_fmaf(sum[j], 0.0f, zero);
@@ -671,41 +692,74 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
         if (t_ok) conv_split_rest(again, s_part, split, m0, t);
         add_parts();
     }
+    const int rows = min(TM, a.out_ch - m0);   // rows wave + 4 j below it exist
+    if (a.splits > 1) {
+        if (!t_ok) return;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (wave + 4 * j < rows) a.parts[((size_t)split * a.out_ch + m0 + wave + 4 * j) * a.length + t] = sum[j];
+        return;
+    }
+    // conv_combine's operations
     float value[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int row = (tid >> 6) + 4 * j, m = m0 + row;
-        value[j] = 0.0f;
-        if (a.splits > 1) {
-            if (t_ok && m < a.out_ch) a.parts[((size_t)split * a.out_ch + m) * a.length + t] = sum[j];
-            continue;
-        }
-        if (t_ok && m < a.out_ch) value[j] = conv_combine(a, (size_t)m * a.length + t, sum[j] + (a.bias != nullptr ? a.bias[m] : 0.0f));
-    }
-    if (a.splits > 1) return;
-    if (!a.activate) {
+    for (int j = 0; j < 8; ++j) value[j] = sum[j] + s_rows.bias[wave + 4 * j];
+    if (a.residual != nullptr) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int m = m0 + (tid >> 6) + 4 * j;
-            if (t_ok && m < a.out_ch) a.out[(size_t)m * a.length + t] = value[j];
+        for (int j = 0; j < 8; ++j) value[j] = first[j] + value[j];
+        if (a.residual2 != nullptr) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) value[j] = second[j] + value[j];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) value[j] = value[j] * a.scale;
+    float *const out = a.out + (size_t)(m0 + wave) * a.length + t;
+    const size_t step = (size_t)4 * a.length;
+    if (!a.activate) {
+        if (t_ok) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (wave + 4 * j < rows) out[j * step] = value[j];
         }
         return;
     }
-    // with an activation: the values go back through LDS (a thread reads what it wrote) so that one copy of the
-    // activation's code serves the eight of them
-    float *s_alpha = reinterpret_cast<float *>(lds) + 4 * 32 * 64;   // [32] alpha, [32] 1 / (alpha + 1e-9) of the tile's rows
-    if (tid < 32) {
-        const float al = m0 + tid < a.snake_channels ? a.alpha[m0 + tid] : 0.0f;
-        s_alpha[tid] = al;
-        s_alpha[32 + tid] = 1.0f / (al + 1e-9f);
+    float al[8], act[8];
+    bool large = false;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        al[j] = s_rows.alpha[wave + 4 * j];
+        act[j] = value[j] < 0.0f ? value[j] * 0.01f : value[j];
+        large = large || !(fabsf(al[j] * value[j]) < kShortSineLimit);
     }
-    __syncthreads();   // every sum has been read
+    if (__builtin_expect(!__any(t_ok && large), 1)) {
+        if (m0 < a.snake_channels) {   // (else no row of the tile is a snake row)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float sn = short_sine(al[j] * value[j]), y = value[j] + sn * sn * s_rows.inverse_alpha[wave + 4 * j];
+                act[j] = m0 + wave + 4 * j < a.snake_channels ? y : act[j];
+            }
+        }
+        if (t_ok) {
+            float *const act_out = a.act_out != nullptr ? a.act_out + (size_t)(m0 + wave) * a.length + t : out;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (wave + 4 * j < rows) {
+                    if (a.act_out != nullptr) out[j * step] = value[j];
+                    act_out[j * step] = act[j];
+                }
+        }
+        return;
+    }
+    // some argument needs the library's sine: the values go through LDS (a thread reads what it wrote, behind the partial tiles, which other
+    // wavefronts may still read) so that one copy of that routine serves the eight of them
+    s_part += 4 * 2048;
 #pragma unroll
     for (int j = 0; j < 8; ++j) s_part[tid + 256 * j] = value[j];
-#pragma unroll 2
+#pragma unroll 1
     for (int j = 0; j < 8; ++j) {
-        const int row = (tid >> 6) + 4 * j, m = m0 + row;
-        if (t_ok && m < a.out_ch) conv_emit(a, m, (size_t)m * a.length + t, s_part[tid + 256 * j], s_alpha[row], s_alpha[32 + row]);
+        const int row = wave + 4 * j, m = m0 + row;
+        if (t_ok && row < rows) conv_emit(a, m, (size_t)m * a.length + t, s_part[tid + 256 * j], s_rows.alpha[row], s_rows.inverse_alpha[row]);
     }
 }
 
@@ -732,7 +786,7 @@ constexpr int kConvBatchMax = 4;
 constexpr int kConvMaxSplits = 8;
 struct ConvBatchArgs {
     ConvArgs item[kConvBatchMax];
-    int order[kConvBatchMax];   // blockIdx.z -> member: the ones with the most taps first, so that a long workgroup is not started last
+    int order[kConvBatchMax];   // blockIdx.z -> member (order_members)
 };
 
 __device__ __forceinline__ ConvBlocks conv_blocks(const ConvArgs &a) { return ConvBlocks{a.weights, (a.out_ch + 31) / 32, (a.in_ch + 15) / 16}; }
@@ -1141,8 +1195,58 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_res_block(const ResArgs a) 
     }
 }
 
+// The order in which a launch's members start, `each` workgroups apiece.  Workgroups are dealt to the CUs in turn, so member p of the order
+// covers CUs p * each .. on, round and round: the order whose most loaded CU has the fewest taps, and of equal ones the one that starts the most
+// taps first (a long workgroup is not started last).  Taps 3 / 7 / 11, us a layer of three positions, most taps first / this order: 432
+// channels x 512 (112 workgroups each) 192 / 183, 216 x 3584 (112) 258 / 249, 216 x 4096 (128) 266 / 257; where nothing is gained it is the same
+// order, and another is slower: 108 x 12288 (192) 221 / 230, 432 x 320 (140) 144 / 151.  With one or two workgroups of each member for every CU, and
+// more members than two, the second one by its taps goes first: 216 x 3072 258 / 238, 108 x 5120 173 / 165, x 4096 128 / 124, x 16384 260 / 258.
+void order_members(const State *st, const int *taps, int count, long each, int *order) {
+    int by_taps[kConvBatchMax], at[kConvBatchMax], best = INT_MAX;
+    for (int i = 0; i < count; ++i) {
+        int j = i;
+        for (; j > 0 && taps[by_taps[j - 1]] < taps[i]; --j) by_taps[j] = by_taps[j - 1];
+        by_taps[j] = i;
+    }
+    const long cus = st->cu_count, rest = each % cus;
+    if (each >= cus && each < 2 * cus && count > 2) {
+        std::swap(by_taps[0], by_taps[1]);
+        for (int i = 0; i < count; ++i) order[i] = by_taps[i];
+        return;
+    }
+    int permutations = 1;
+    for (int i = 2; i <= count; ++i) permutations *= i;
+    for (int p = 0; p < permutations; ++p) {   // (the first one is by_taps itself)
+        bool used[kConvBatchMax] = {};
+        for (int i = 0, code = p, base = permutations; i < count; ++i) {
+            base /= count - i;
+            int skip = code / base, k = 0;
+            code %= base;
+            for (; used[k] || skip > 0; ++k) skip -= used[k] ? 0 : 1;
+            used[k] = true;
+            at[i] = by_taps[k];
+        }
+        int most = 0;   // a CU's taps beyond those that every CU has: highest where some member's last round begins
+        for (int i = 0; i < count; ++i) {
+            const long cu = i * each % cus;
+            int load = 0;
+            for (int j = 0; j < count; ++j) load += (cu - j * each % cus + cus) % cus < rest ? taps[at[j]] : 0;
+            most = load > most ? load : most;
+        }
+        if (most < best) {
+            best = most;
+            for (int i = 0; i < count; ++i) order[i] = at[i];
+        }
+    }
+}
+void order_members(const State *st, ConvBatchArgs &b, int count, long each) {
+    int taps[kConvBatchMax];
+    for (int i = 0; i < count; ++i) taps[i] = b.item[i].kernel;
+    order_members(st, taps, count, each, b.order);
+}
+
 template <int WM, int WN, int NT, bool SPLIT = false>
-int launch_res_block(State *st, const ResArgs &a, int count, char *error, size_t capacity) {
+int launch_res_block(State *st, ResArgs &a, int count, char *error, size_t capacity) {
     constexpr int RN = 32 * NT * WN;
     int taps = 0;
     for (int i = 0; i < count; ++i) taps = a.member[i].kernel > taps ? a.member[i].kernel : taps;
@@ -1156,8 +1260,11 @@ int launch_res_block(State *st, const ResArgs &a, int count, char *error, size_t
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_res_block<WM, WN, NT, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, 112 * 1024));
         raised = true;
     }
-    const int finished = RN - (taps - 1);
-    hipLaunchKernelGGL((k_res_block<WM, WN, NT, SPLIT>), dim3((unsigned)((a.length + finished - 1) / finished), (unsigned)count), dim3(64 * WM * WN), lds, st->stream, a);
+    const int finished = RN - (taps - 1), each = (a.length + finished - 1) / finished;
+    int kernels[kConvBatchMax];
+    for (int i = 0; i < count; ++i) kernels[i] = a.member[i].kernel;
+    order_members(st, kernels, count, each, a.order);
+    hipLaunchKernelGGL((k_res_block<WM, WN, NT, SPLIT>), dim3((unsigned)each, (unsigned)count), dim3(64 * WM * WN), lds, st->stream, a);
     return hip_check(hipGetLastError(), "residual block launch", error, capacity);
 }
 
@@ -1326,7 +1433,7 @@ constexpr size_t conv_lds() {
 }
 template <int NT>
 constexpr size_t conv_split_lds() {
-    constexpr size_t stages = (size_t)4 * 4 * conv_pitch(32 * NT) * 16, epilogue = (4 * 32 * 64 + 64) * sizeof(float);
+    constexpr size_t stages = (size_t)4 * 4 * conv_pitch(32 * NT) * 16, epilogue = 5 * 2048 * sizeof(float);
     return stages > epilogue ? stages : epilogue;
 }
 constexpr int kConvMaxLds = 2 * 4 * (256 + kConvMaxHalo) * 16;   // the largest of them
@@ -1415,7 +1522,7 @@ int launch_conv_split(State *st, const ConvArgs &a, const ConvBlocks &weights, c
 }
 
 template <int WM, int WN>
-int launch_conv_batch(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
+int launch_conv_batch(State *st, ConvBatchArgs &b, int count, char *error, size_t capacity) {
     constexpr int TM = 32 * WM, TN = 64 * WN;
     constexpr size_t lds = conv_lds<WM, WN>();
     static bool raised = false;   // per instantiation
@@ -1425,12 +1532,13 @@ int launch_conv_batch(State *st, const ConvBatchArgs &b, int count, char *error,
     }
     const ConvArgs &a = b.item[0];
     const dim3 grid((unsigned)((a.length + TN - 1) / TN), (unsigned)((a.out_ch + TM - 1) / TM), (unsigned)count);
+    order_members(st, b, count, (long)grid.x * grid.y);
     hipLaunchKernelGGL((k_conv1d_batch<WM, WN>), grid, dim3(256), lds, st->stream, b);
     return hip_check(hipGetLastError(), "conv1d batch launch", error, capacity);
 }
 
 template <int NT, int PARTS>
-int launch_conv_split_batch_p(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
+int launch_conv_split_batch_p(State *st, ConvBatchArgs &b, int count, char *error, size_t capacity) {
     constexpr size_t lds = conv_split_lds<NT>();
     static bool raised = false;
     if (!raised) {
@@ -1439,12 +1547,13 @@ int launch_conv_split_batch_p(State *st, const ConvBatchArgs &b, int count, char
     }
     const ConvArgs &a = b.item[0];
     const dim3 grid((unsigned)((a.length + 32 * NT - 1) / (32 * NT) * a.splits), (unsigned)((a.out_ch + 31) / 32), (unsigned)count);
+    order_members(st, b, count, (long)grid.x * grid.y);
     hipLaunchKernelGGL((k_conv1d_split_batch<NT, PARTS>), grid, dim3(256), lds, st->stream, b);
     return hip_check(hipGetLastError(), "conv1d batch launch", error, capacity);
 }
 
 template <int NT>
-int launch_conv_split_batch(State *st, const ConvBatchArgs &b, int count, char *error, size_t capacity) {
+int launch_conv_split_batch(State *st, ConvBatchArgs &b, int count, char *error, size_t capacity) {
     bool two = true;
     for (int i = 0; i < count; ++i) two = two && conv_split_parts(b.item[i], 32 * NT) == 2;
     return two ? launch_conv_split_batch_p<NT, 2>(st, b, count, error, capacity) : launch_conv_split_batch_p<NT, 3>(st, b, count, error, capacity);
@@ -1593,9 +1702,6 @@ extern "C" int mynah_hip_conv1d_fused_batch(void *state, const mynah_hip_conv1d_
                            &b.item[i], &weights[i], error, capacity) != 0)
             return -1;
         side_by_side = side_by_side && (it.kernel == 3 || it.kernel == 7 || it.kernel == 11);
-        size_t at = i;   // most taps first
-        for (; at > 0 && items[b.order[at - 1]].kernel < it.kernel; --at) b.order[at] = b.order[at - 1];
-        b.order[at] = (int)i;
         // the members run at the same time: what one writes, no other may read or write
         for (size_t j = 0; j < count; ++j) {
             if (j == i) continue;
@@ -1792,9 +1898,6 @@ static int res_position(State *st, const mynah_hip_res_block *blocks, size_t bra
         m.dilation = b.dilation;
         a.blocks = w_in.blocks;
         a.tiles = w_in.tiles;
-        size_t at = i;   // most taps first
-        for (; at > 0 && a.member[a.order[at - 1]].kernel < m.kernel; --at) a.order[at] = a.order[at - 1];
-        a.order[at] = (int)i;
     }
     switch (build) {
         case RES_32_NARROW: return launch_res_block<1, 4, 1>(st, a, (int)branches, error, capacity);
