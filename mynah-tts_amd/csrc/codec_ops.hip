@@ -1574,30 +1574,30 @@ int mynah::launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_
 // wavefronts.  (Few output channels: the large tiles are one row of wavefronts, wider in time.)  The two add in different orders, so
 // the choice is the shape's alone, for single, batched and fused launches alike, and the line lies where a residual layer's
 // three members meet; one convolution alone would change over later.  us, small tiles / large:
-//   three members of taps 3, 7, 11, six launches:  216 channels x 3072 327 / 383, x 3584 388 / 393, x 4096 429 / 401;
-//     108 x 4096 184 / 204, x 5120 209 / 212, x 6144 251 / 230
-//   alone, 3 / 11 taps:  216 x 3072 18.7 33 / 26 54;  108 x 5120 12.2 19 / 17.8 29.5;  54 x 12000 9.9 (11.8 with 7 taps) / 13 17;
+//   three members of taps 3, 7, 11, six launches:  216 channels x 3584 248 / 259, x 4096 274 / 272, x 4608 289 / 311, x 5120 334 / 327;
+//     160 x 4096 173 / 195, x 6144 232 / 246;  108 x 5120 141 / 157, x 6144 156 / 159, x 7168 180 / 165
+//   alone (as three bf16 pieces), 3 / 11 taps:  216 x 3072 18.7 33 / 26 54;  108 x 5120 12.2 19 / 17.8 29.5;  54 x 12000 9.9 (11.8 with 7 taps) / 13 17;
 //     64 -> 864 x 640 9.6 (13.4) / 13.3 17.8, x 1280 16.3 (19) / 14 17.5;  32 -> 864 x 5, 7 taps: 8.8 / 11.6, x 128 7.9 / 12
 // A layer of at most 32 channels has two blocks at most and runs as one launch a block, in the large tiles' order.
 static bool conv_takes_split(const State *st, int in_channels, int out_channels, int length) {
     const long tiles = out_channels <= 32 ? (long)((length + 255) / 256) : (long)((out_channels + 63) / 64) * ((length + 127) / 128);
     if (in_channels < 32 || (in_channels == 32 && out_channels <= 32)) return false;
-    return tiles < (in_channels > kResMaxChannels ? (long)st->cu_count * 7 / 16 : (long)st->cu_count * 3 / 8);
+    return in_channels > kResMaxChannels ? tiles <= (long)st->cu_count * 9 / 16 : tiles < (long)st->cu_count * 3 / 8;
 }
 
 // How many workgroups share a channel-split tile.  A few short rows leave most of the chip idle while each tile's workgroup pulls the
 // weights of all channels through one CU (some 40 GB/s: 0.9 MB with 432 channels and eleven taps); so as many as bring a wavefront's
 // blocks of channels down while three members' workgroups are two to a CU at most.  The sums' order follows, so this is the shape's
-// alone, too.  Taps 3 / 7 / 11 side by side: 432 channels x 40 24.6 -> 11.2 us, 216 x 320 18.9 -> 12.4, and 4.0 for k_conv_finish; 108 x 1280
-// stays with one (14.2 us, 12.4 + 4.2 shared), its seven blocks are few enough.  Half or twice kConvSharedTiles, a 432-channel layer of three positions: 64
-// positions 98 / 87 / 87 us, 128 143 / 116 / 123, 192 192 / 147 / 156, 256 230 / 175 / 168, 320 238 / 196 / 198.
+// alone, too.  k_conv_finish is 3.4 us of a launch, so a wavefront must be spared three blocks at least.  us a layer of three positions, taps 3 / 7 /
+// 11, unshared / shared by so many: 432 channels (27 blocks) x 40 121 / 72 by 7, x 128 125 / 89 by 4, x 320 167 / 141 by 2; 216 (14) x 320 88 / 79 by 4,
+// x 640 92 / 99 by 2, which spares two.
 constexpr int kConvSharedTiles = 160;
 static int conv_splits(int in_channels, int out_channels, int length) {
     const long tiles = (long)((out_channels + 31) / 32) * ((length + 63) / 64), blocks = (in_channels + 15) / 16;
     if (in_channels <= kResMaxChannels) return 1;
     for (long each = 1; 4 * each < blocks; ++each) {
         const long splits = (blocks + 4 * each - 1) / (4 * each);
-        if (splits <= kConvMaxSplits && tiles * splits <= kConvSharedTiles) return (int)splits;
+        if (splits <= kConvMaxSplits && tiles * splits <= kConvSharedTiles) return (blocks + 3) / 4 - each >= 3 ? (int)splits : 1;
     }
     return 1;
 }
@@ -1839,7 +1839,7 @@ extern "C" int mynah_hip_rows_combine_dev(void *state, const float *const *dev_i
 // needs less time for its rounds.  Measured per layer of three positions, branches of 3 / 7 / 11 taps, us:
 //   27 channels: x 5120 47 narrow, 65 wide, 84 as two launches a position; x 28672 74, 84, 105; x 32768 (more than three to a CU) 98, 85, 111;
 //     x 40960 107, 89; x 43008 (more wide than two to a CU) 108, 129; x 65536 145, 150, 160
-//   54, split order: x 64 54 narrow, 56 as two launches; x 1024 57, 59; x 5120 71, 82; x 10240 82, 137
+//   54, split order: x 1024 57 narrow, 47 as two launches of split tiles; x 2560 66, 57; x 5120 70.5, 69; x 10240 86, 111
 //   54, large order: x 13824 92 narrow, 104 wide, 127 as two launches; x 16384 133, 113, 133; x 20480 141, 120, 154; x 22528 152, 164, 163; x 28672
 //     160, 179, 175; x 32768 193, 201, 202; x 40960 229, 200, 268
 //   108, large order, 3 and 11 taps: x 6144 173 narrow, 202; x 8192 186, 204; x 12288 (more than fit) 276, 240; three branches: x 6144 155, 160;
@@ -1860,7 +1860,7 @@ static ResBuild res_build(const State *st, const mynah_hip_res_block *blocks, si
     if (channels <= 32) return fit(128, 3) || !fit(256, 2) ? RES_32_NARROW : RES_32_WIDE;
     const bool split = conv_takes_split(st, (int)channels, (int)channels, (int)length);
     if (channels > 64) return !split && fit(64, 1) ? RES_128 : RES_NONE;
-    if (split) return RES_64_SPLIT;
+    if (split) return 2 * (long)((length + 63) / 64) * (long)branches < 2 * (long)st->cu_count ? RES_NONE : RES_64_SPLIT;
     return fit(64, 3) || (!fit(128, 2) && fit(64, 7)) ? RES_64_NARROW : RES_64_WIDE;
 }
 

@@ -624,8 +624,8 @@ def test_conv_transpose_forms(backend, stride, kernel):
 
 
 # (branches of 3, 7 and 11 taps, 256 CUs) the last and the first length of each one-launch build: at most 32 channels narrow / wide / narrow again; to 64
-# the shortest rows, the two orders, narrow / wide / narrow / wide
-@pytest.mark.parametrize("C,L", [(27, 31152), (27, 31153), (27, 42558), (27, 42559), (40, 1), (64, 65), (54, 12160), (54, 12161), (54, 14790), (54, 14791), (64, 20768), (64, 20769),
-                                 (33, 34510), (33, 34511)])
+# two launches / one, the two orders, narrow / wide / narrow / wide; more channels: split and large tiles
+@pytest.mark.parametrize("C,L", [(27, 31152), (27, 31153), (27, 42558), (27, 42559), (40, 1), (50, 5440), (50, 5441), (54, 12160), (54, 12161), (54, 14790), (54, 14791), (64, 20768), (64, 20769),
+                                 (33, 34510), (33, 34511), (216, 4608), (216, 4609)])
 def test_res_layer_build_lines(pkg, backend, C, L):
     test_res_layer_builds(pkg, backend, C, L, (3, 7, 11))
