@@ -134,6 +134,21 @@ struct ConvWeights {   // the weight pieces of one row tile, requested kAhead st
             if (--blocks > 0) next += skip;
         }
     }
+    // The request that is multiplied next, in slot BY, to slot 0 (and so on).
+    template <int BY>
+    __device__ __forceinline__ void turn() {
+        if constexpr (BY != 0) {
+            uint4 was[kAhead][2];
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) was[i][q] = ring[i][q];
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) ring[i][q] = was[(i + BY) % kAhead][q];
+        }
+    }
     // (what runs past the last step is requested and not used: it is what follows the last block, and the cache pads its copies)
     __device__ __forceinline__ ConvWeights(const uint4 *first, unsigned lane, size_t skip_arg, int blocks_arg, int taps)
         : next(first), bytes(lane * 16), skip(skip_arg), blocks(blocks_arg) {
@@ -164,18 +179,31 @@ __device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, co
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[n].multiply(fw, x[set][n]);
     };
-    if constexpr (KF != 0) {
+    if constexpr (KF != 0 && AHEAD) {
+        // (the one-launch block: its few blocks run once, and code that is run once is waited for, instruction by instruction; so one copy of a
+        // block's steps, the weights' registers turned back in place at its end -- three copies: 27 channels x 65536 144 us a layer, 140 with one; 54 x 32768 190, 186)
+        for (int block = 0; block < blocks; ++block) {
+            const uint4 *at = stage(block);
+            read(0, at);
+#pragma unroll
+            for (int tap = 0; tap < KF; ++tap) {
+                if (tap + 1 < KF) read((tap + 1) & 1, at + (tap + 1) * dilation);
+                multiply(tap & 1, tap % ConvWeights::kAhead);
+                w.request(tap % ConvWeights::kAhead, KF);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            w.template turn<KF % ConvWeights::kAhead>();
+        }
+    } else if constexpr (KF != 0) {
         for (int block = 0;;) {
 #pragma unroll
             for (int u = 0; u < ConvWeights::kAhead; ++u) {
                 const uint4 *at = stage(block);
-                if constexpr (AHEAD) read((u * KF) & 1, at);
 #pragma unroll
                 for (int tap = 0; tap < KF; ++tap) {
                     const int s = u * KF + tap;
-                    if constexpr (!AHEAD) read(0, at + tap * dilation);
-                    else if (tap + 1 < KF) read((s + 1) & 1, at + (tap + 1) * dilation);
-                    multiply(AHEAD ? s & 1 : 0, s % ConvWeights::kAhead);
+                    read(0, at + tap * dilation);
+                    multiply(0, s % ConvWeights::kAhead);
                     w.request(s % ConvWeights::kAhead, KF);
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -942,15 +970,29 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
         }
     };
     // the inner rows' alphas, 1 / (alpha + 1e-9), and what a value is multiplied by to be told from those that need the long way: the
-    // library's sine, or (no finite number, or none to speak of) more than that
-    for (int c = tid; c < kResMaxChannels; c += T) {
-        const float2 pair = c < a.snake_channels ? m.snake_skip[c] : make_float2(0.0f, 0.0f);
-        s_rows.pair[c] = make_float4(pair.x, pair.y, fmaxf(fabsf(pair.x), 1.01f * (kShortSineLimit / kLargest)), 0.0f);
+    // library's sine, or (no finite number, or none to speak of) more than that.  (Requested here, looked at behind the first block's requests.)
+    constexpr int kRowsEach = (kResMaxChannels + T - 1) / T;
+    float2 row_pair[kRowsEach], row_in[kRowsEach], row_skip[kRowsEach];
+#pragma unroll
+    for (int i = 0; i < kRowsEach; ++i) {
+        const int c = tid + T * i;
         const bool there = c < a.channels;   // (else zero: a wavefront without a row tile of its own multiplies the last one's weights)
         const size_t steps = (size_t)a.tiles * a.blocks * KF;
-        s_rows.in[c] = make_float2(there ? conv_inverses(m.w_in, steps)[c] : 0.0f, there && m.b_in != nullptr ? m.b_in[c] : 0.0f);
-        s_rows.skip[c] = make_float2(there ? conv_inverses(m.w_skip, steps)[c] : 0.0f, there && m.b_skip != nullptr ? m.b_skip[c] : 0.0f);
+        row_pair[i] = c < a.snake_channels ? m.snake_skip[c] : make_float2(0.0f, 0.0f);
+        row_in[i] = make_float2(there ? conv_inverses(m.w_in, steps)[c] : 0.0f, there && m.b_in != nullptr ? m.b_in[c] : 0.0f);
+        row_skip[i] = make_float2(there ? conv_inverses(m.w_skip, steps)[c] : 0.0f, there && m.b_skip != nullptr ? m.b_skip[c] : 0.0f);
     }
+    const auto keep_rows = [&]() {
+#pragma unroll
+        for (int i = 0; i < kRowsEach; ++i) {
+            const int c = tid + T * i;
+            if (c >= kResMaxChannels) break;
+            const float2 pair = row_pair[i];
+            s_rows.pair[c] = make_float4(pair.x, pair.y, fmaxf(fabsf(pair.x), 1.01f * (kShortSineLimit / kLargest)), 0.0f);
+            s_rows.in[c] = row_in[i];
+            s_rows.skip[c] = row_skip[i];
+        }
+    };
 
     HalfSums sums[NT];
     f32x16 acc[NT];   // (SPLIT: the blocks before, then) the finished sums
@@ -990,6 +1032,7 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
         fetch(0);
         ConvWeights w(m.w_in + w_at, lane, 0, 1, KF);
         start();
+        if (!once_more) keep_rows();
         publish(0, stage_now);
         fetch(min(1, a.blocks - 1));
         conv_products<KF, NT, 2 * kPitch, true>(w, KF, m.dilation, a.blocks, [&](int block) {
