@@ -12,8 +12,9 @@
 // f16 holds s x in full from 2^-14 to 2^16: that is what the scales are for.
 //   A weight has one per output row, so that the row's largest value lies in [2^13, 2^14) (half_row_scale); it is divided out of the finished sum.
 //   An input has 1, as long as the largest that a tile reads of it is in [2^-10, 65520): then what the two pieces miss is 2^-37 at most, or
-//   2^-27 of that largest.  A tile whose largest input is smaller, or larger up to 2^28, is multiplied once more with a scale of its own
-//   (half_rescale): twice the time, in tiles that hold nothing but near silence or values that no trained network has.
+//   2^-27 of that largest.  A tile whose largest input is smaller, or larger up to 2^24, is multiplied once more with a scale of its own
+//   (half_rescale): twice the time, in tiles that hold nothing but near silence or values that no trained network has.  (What stands beside a value
+//   just below 2^24 loses 2^-26 at most, which is half of f32's last place of 1/2.)
 // Operands without two finite pieces (infinite, NaN, or out of those ranges upwards) make every sum they enter infinite or NaN.  Such a sum
 // is looked for once, when it is finished, and put in its place comes the chain of f32 multiply-adds it stands for, from the operands
 // themselves, which a weight's three pieces are: an infinity stays one, and a large value is a value.
@@ -94,7 +95,7 @@ __device__ __forceinline__ float power_of_two(int e) { return __uint_as_float((u
 __device__ __forceinline__ int exponent_of(float x) { return (int)(__float_as_uint(x) >> 23 & 255) - 127; }     // (-127: zero and the subnormal values)
 // The power of two under which a tile's inputs are taken apart again, or 0 where its products hold.
 __device__ __forceinline__ int half_rescale(float largest) {
-    const bool quiet = largest < 0x1p-10f && largest > 0.0f, loud = largest >= kHalfLimit && largest < 0x1p28f;
+    const bool quiet = largest < 0x1p-10f && largest > 0.0f, loud = largest >= kHalfLimit && largest < 0x1p24f;
     return quiet || loud ? min(13 - exponent_of(largest), 100) : 0;
 }
 

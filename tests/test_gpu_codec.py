@@ -569,14 +569,14 @@ def test_res_layer_extremes(pkg, backend, C, L, taps):
 
 def test_conv1d_input_sizes(backend):
     """Inputs whose largest value lies on either side of the lines at which a tile is multiplied once more under a scale of its own (2^-10,
-    65520, 2^28), far from them, and rows of very different size side by side, in each kind of tile: f32's accuracy against float64."""
+    65520, 2^24), far from them, and rows of very different size side by side, in each kind of tile: f32's accuracy against float64."""
     rng = np.random.default_rng(77)
     for C, O, L, K, D in ((20, 70, 300, 7, 3), (27, 27, 500, 3, 1), (432, 64, 33, 3, 1), (216, 216, 320, 11, 1), (40, 48, 300, 5, 5)):
         w = (rng.standard_normal((O, C, K)) / np.sqrt(C * K)).astype(np.float32)
         w *= np.exp2(rng.integers(-60, 60, size=(O, 1, 1))).astype(np.float32)      # each output channel has a scale of its own
         base = rng.uniform(-1, 1, size=(C, L)).astype(np.float32)
         base[0, 0] = 1.0
-        for size in (2.0 ** -60, 2.0 ** -30, 2.0 ** -10 * (1 - 2.0 ** -20), 2.0 ** -10, 1.0, 65519.0, 65521.0, 2.0 ** 20, 2.0 ** 28 * (1 - 2.0 ** -20), 0.0):
+        for size in (2.0 ** -60, 2.0 ** -30, 2.0 ** -10 * (1 - 2.0 ** -20), 2.0 ** -10, 1.0, 65519.0, 65521.0, 2.0 ** 20, 2.0 ** 24 * (1 - 2.0 ** -20), 2.0 ** 24, 0.0):
             _announce("conv1d input size %g, %d -> %d x %d, %d taps" % (size, C, O, L, K))
             x = base * np.float32(size)
             got = _run_conv1d(backend, x, w, np.zeros(O, np.float32), D).astype(np.float64)

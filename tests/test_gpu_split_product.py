@@ -1,4 +1,4 @@
-"""The f32 products on the bf16 matrix cores (three bf16 pieces per operand) through the entry points that use them, at the edges of
+"""The f32 products on the f16 matrix cores (two f16 pieces per operand) through the entry points that use them, at the edges of
 their tiles: rows around 32 / 64 / a second tile, output widths that end inside a 128-column tile, more layers than one launch
 takes, both FFN forms.  Against float64 (cross K/V, weights with all 24 bits and rows of very different size) and the oracle."""
 import numpy as np
@@ -87,7 +87,7 @@ def test_one_buffer_under_two_shapes(backend, pkg, orc):
 
 
 def test_cross_kv_extremes(backend, pkg, orc):
-    """Operands without three finite bf16 pieces: infinities, NaN, values from 2^128 - 2^119 on.  What f32 multiply-adds give, and only in
+    """Operands without two finite f16 pieces: infinities, NaN, values up to f32's largest.  What f32 multiply-adds give, and only in
     the outputs that they enter."""
     print("[gpu-case] cross K/V extremes", flush=True)
     rng = np.random.default_rng(8)
@@ -163,8 +163,8 @@ def test_encoder_f32_large_weights(backend, pkg, synth, nerr, taps):
 
 
 def test_cross_kv_tiny_weights(backend, pkg, orc):
-    """Below 2^-110 an operand keeps fewer than its 24 bits: its third piece ends at bf16's smallest subnormal, 2^-133, so that at most half
-    of that is lost."""
+    """Rows of weights down to 2^-126, each under a scale of its own, which ends at 2^126: what is lost of a term is no more than half of
+    2^-133."""
     print("[gpu-case] cross K/V, tiny weights", flush=True)
     rng = np.random.default_rng(9)
     backend.set_quant(pkg.F32)
