@@ -46,58 +46,59 @@ __global__ void __launch_bounds__(256) k_split_pack(const float *src, uint4 *dst
     values[64] = make_float4(v[4], v[5], v[6], v[7]);
 }
 
-// LDS of a tile: three stages of one block of 32 channels (32 * MT + taps - 1 rows), operand-major per 16-deep half, piece and
-// 8-deep quarter, and afterwards the second group's sums; and the largest input of each wavefront.  The row pitch puts the four (half, quarter) places of a row 64 bytes
-// apart modulo 256, so that a staged row's eight threads and its three neighbours' never meet in a bank; fragment reads are
-// 512 consecutive bytes.
-template <int MT, int TAPS>
+// LDS of a tile: three stages of one block of 16 G channels (32 * MT + taps - 1 rows), operand-major per 16-deep part, piece and
+// 8-deep half, and afterwards the later groups' sums; and the largest input of each wavefront.  The row pitch puts the two halves of a row 64 bytes
+// apart modulo 256; fragment reads are 512 consecutive bytes.  (Bank conflicts are 2 % of a launch's cycles; a pitch of kRows + 2 with the pieces
+// innermost has as many.)
+template <int MT, int TAPS, int G>
 struct SplitTile {
     static constexpr int kRows = 32 * MT + (TAPS - 1), kPitch = (kRows + 11) / 16 * 16 + 4;
-    static_assert(kPitch >= kRows && kPitch % 16 == 4, "bank layout");
+    static_assert(kPitch >= kRows && kPitch % 16 == 4 && (G == 2 || G == 4), "bank layout");
     union {
-        uint4 a[3][2][2][2][kPitch];
-        float sums[4][MT][16][64];
+        uint4 a[3][G][2][2][kPitch];
+        float sums[8 - 8 / G][MT][16][64];
     };
     float largest[8];
 };
 
 constexpr int kBlocksAhead = 2;   // blocks per round of the loop below: a split's block count is a multiple of it
 
-// acc[t] = the tile's sums over `blocks` blocks of 32 channels, for rows 32 t .. of the tile and the wavefront's 32 columns;
-// valid in the first four of the eight wavefronts.
-// Wavefront w multiplies columns 32 * (w % 4) .. over the 16-deep half w / 4 of every block: two wavefronts to a SIMD, because
+// acc[t] = the tile's sums over `blocks` blocks of 16 G channels, for rows 32 t .. of the tile and the wavefront's 32 columns;
+// valid in the first 8 / G of the eight wavefronts.
+// Wavefront w multiplies columns 32 * (w % (8 / G)) .. over the 16-deep part w / (8 / G) of every block: two wavefronts to a SIMD, because
 // one alone cannot issue its vector instructions beside its own matrix instructions.
 // A wavefront's weight pieces come from memory R steps ahead and are multiplied where they arrive; the rows are staged by all eight
 // wavefronts, taken apart on the way to LDS, and serve every tap from there.  A block is stored into a stage two blocks after it was last
 // read, its requests leave two blocks before that; what runs past the last block is requested (the buffers are padded) and not
 // used, so that no request stands under a condition.  One tap: four blocks are unrolled (left after two where there are no more), so
 // that four steps of weights are in flight: a step is 192 cycles of matrix instructions, a round trip to L2 some 2,000.
-template <int MT, int TAPS>
+template <int MT, int TAPS, int G>
 __device__ __forceinline__ void split_tile(const float *const a, const int lda, const int row0, const int rows, const uint4 *const w, const float inverse,
-                                           const int blocks, SplitTile<MT, TAPS> &lds, f32x16 (&acc)[MT]) {
-    using Tile = SplitTile<MT, TAPS>;
+                                           const int blocks, SplitTile<MT, TAPS, G> &lds, f32x16 (&acc)[MT]) {
+    using Tile = SplitTile<MT, TAPS, G>;
     constexpr int UB = TAPS == 1 ? 2 * kBlocksAhead : kBlocksAhead, R = TAPS == 1 ? 4 : 2 * TAPS;   // blocks per round; steps of weights in flight
     static_assert((UB * TAPS) % R == 0 && UB % 2 == 0 && kBlocksAhead == 2, "register stages must repeat with the round");
-    const int tid = threadIdx.x, lane = tid & 63, group = tid >> 8;
-    const int srow = tid >> 3, sc = tid & 7;
-    constexpr int kRows = Tile::kRows, NP = (kRows + 63) / 64;
-    constexpr int kStage = 2 * 2 * 2 * Tile::kPitch;
+    const int tid = threadIdx.x, lane = tid & 63, group = tid / (512 / G);
+    constexpr int kPass = 512 / (4 * G);   // rows staged at once
+    const int srow = tid / (4 * G), sc = tid % (4 * G);
+    constexpr int kRows = Tile::kRows, NP = (kRows + kPass - 1) / kPass;
+    constexpr int kStage = G * 2 * 2 * Tile::kPitch;
     uint4 *const stages = &lds.a[0][0][0][0][0];
     float scale = 1.0f, unscale = 1.0f, largest = 0.0f;
     HalfSums sums[MT];
     for (bool once_more = false;; once_more = true) {
         const float *ap[NP];
 #pragma unroll
-        for (int i = 0; i < NP; ++i) ap[i] = a + (ptrdiff_t)min(row0 - (TAPS - 1) + min(srow + 64 * i, kRows - 1), rows - 1) * lda + 4 * sc;
+        for (int i = 0; i < NP; ++i) ap[i] = a + (ptrdiff_t)min(row0 - (TAPS - 1) + min(srow + kPass * i, kRows - 1), rows - 1) * lda + 4 * sc;
         float4 ra[2][NP];
         const auto request_a = [&](int set, int block) {
 #pragma unroll
-            for (int i = 0; i < NP; ++i) ra[set][i] = *reinterpret_cast<const float4 *>(ap[i] + block * 32);
+            for (int i = 0; i < NP; ++i) ra[set][i] = *reinterpret_cast<const float4 *>(ap[i] + block * (16 * G));
         };
         const auto store_a = [&](int set, uint4 *stage, bool counts) {   // (counts: not past the last block, where anything may lie)
 #pragma unroll
             for (int i = 0; i < NP; ++i)
-                if (64 * i + 64 <= kRows || srow + 64 * i < kRows) {
+                if (kPass * i + kPass <= kRows || srow + kPass * i < kRows) {
                     const float4 v = ra[set][i];
                     uint2 piece[2];
                     float rest[2];
@@ -107,13 +108,13 @@ __device__ __forceinline__ void split_tile(const float *const a, const int lda, 
                     largest = fmaxf(largest, counts ? most : 0.0f);
 #pragma unroll
                     for (int q = 0; q < 2; ++q)
-                        reinterpret_cast<uint2 *>(&stage[(((sc >> 2) * 2 + q) * 2 + ((sc >> 1) & 1)) * Tile::kPitch + srow + 64 * i])[sc & 1] = piece[q];
+                        reinterpret_cast<uint2 *>(&stage[(((sc >> 2) * 2 + q) * 2 + ((sc >> 1) & 1)) * Tile::kPitch + srow + kPass * i])[sc & 1] = piece[q];
                 }
         };
         const uint4 *wp = w + (size_t)group * (TAPS * 128) + lane;
         uint4 rw[R][2];
         const auto request_w = [&](int slot, int step) {   // step counted from wp: block step / TAPS, tap step % TAPS
-            const uint4 *p = wp + ((step / TAPS) * 2 * TAPS + step % TAPS) * 128;
+            const uint4 *p = wp + ((step / TAPS) * G * TAPS + step % TAPS) * 128;
             rw[slot][0] = p[0];
             rw[slot][1] = p[64];
         };
@@ -168,9 +169,9 @@ __device__ __forceinline__ void split_tile(const float *const a, const int lda, 
                 next = after;
                 after = t;
             }
-            wp += UB * 2 * TAPS * 128;
+            wp += UB * G * TAPS * 128;
 #pragma unroll
-            for (int i = 0; i < NP; ++i) ap[i] += UB * 32;
+            for (int i = 0; i < NP; ++i) ap[i] += UB * 16 * G;
         }
         largest = wave_max(largest);
         if (lane == 0) lds.largest[tid >> 6] = largest;
@@ -183,18 +184,23 @@ __device__ __forceinline__ void split_tile(const float *const a, const int lda, 
         scale = power_of_two(e);
         unscale = power_of_two(-e);
     }
-    if (group == 1) {
+    if (group > 0) {
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) lds.sums[(tid >> 6) & 3][t][r][lane] = sums[t].sum(r);
+            for (int r = 0; r < 16; ++r) lds.sums[(tid >> 6) - 8 / G][t][r][lane] = sums[t].sum(r);
     }
     __syncthreads();
     if (group == 0) {
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[t][r] = (sums[t].sum(r) + lds.sums[tid >> 6][t][r][lane]) * unscale * inverse;
+            for (int r = 0; r < 16; ++r) {
+                float sum = sums[t].sum(r) + lds.sums[tid >> 6][t][r][lane];
+#pragma unroll
+                for (int g = 2; g < G; ++g) sum += lds.sums[(tid >> 6) + (g - 1) * (8 / G)][t][r][lane];
+                acc[t][r] = sum * unscale * inverse;
+            }
     }
 }
 
@@ -248,29 +254,31 @@ struct SplitWork {
 };
 
 // part[z][m][n]: the sums over split z's channels (splits == 1: the product).
-template <int MT, int TAPS>
+// A workgroup's columns: 32 for each of its 8 / G wavefronts of a group.
+template <int MT, int TAPS, int G>
 __global__ void __launch_bounds__(512) k_split_rows(const float *const a, const uint4 *const w, const int M, const int N, const int channels, const int mtiles,
                                                     const int ntiles, const int splits, float *const part) {
-    __shared__ SplitTile<MT, TAPS> lds;
+    __shared__ SplitTile<MT, TAPS, G> lds;
+    constexpr int kWide = 8 / G, kDeep = 16 * G;
     const SplitWork work((int)blockIdx.x, mtiles);
     if (work.nz >= ntiles * splits) return;
-    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
-    const int z = work.nz / ntiles, blocks = channels / 32 / splits;
-    const int col0 = (work.nz % ntiles) * 128 + wave * 32, m0 = work.m * 32 * MT;
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) % kWide;
+    const int z = work.nz / ntiles, share = channels / splits;
+    const int col0 = ((work.nz % ntiles) * kWide + wave) * 32, m0 = work.m * 32 * MT;
     f32x16 acc[MT];
     const SplitWeight weight(w, (size_t)N, (size_t)channels, TAPS);
-    const size_t step = ((size_t)(min(col0, N - 32) / 32) * (channels / 32) + z * blocks) * (2 * TAPS);   // the tile's first
+    const size_t step = ((size_t)(min(col0, N - 32) / 32) * (channels / 16) + z * (share / 16)) * TAPS;   // the tile's first
     const uint4 *tile = w + step * 128;
     const float inverse = weight.inverses()[min(col0, N - 32) + (lane & 31)];
-    split_tile<MT, TAPS>(a + z * blocks * 32, channels, m0, M, tile, inverse, blocks, lds, acc);
-    if (threadIdx.x >= 256 || col0 >= N) return;
-    split_store<MT, TAPS>(a + z * blocks * 32, channels, m0, M, weight.values() + step * 128, blocks, acc, part + (size_t)z * M * N + col0 + (lane & 31), N);
+    split_tile<MT, TAPS, G>(a + z * share, channels, m0, M, tile, inverse, share / kDeep, lds, acc);
+    if (threadIdx.x >= 64 * kWide || col0 >= N) return;
+    split_store<MT, TAPS>(a + z * share, channels, m0, M, weight.values() + step * 128, share / 32, acc, part + (size_t)z * M * N + col0 + (lane & 31), N);
 }
 
 // The K and V halves of every layer's kv_net on that layer's normalised memory, one launch: blockIdx.y names the layer.
 __global__ void __launch_bounds__(512) k_split_cross_kv(const float *const normed, const SplitLayers weights, const int M, const int width, const int xw,
                                                         const int mtiles, float *const k_out, float *const v_out) {
-    __shared__ SplitTile<2, 1> lds;
+    __shared__ SplitTile<2, 1, 2> lds;
     const int N = 2 * xw, ntiles = (N + 127) / 128;
     const SplitWork work((int)blockIdx.x, mtiles);
     if (work.nz >= ntiles) return;
@@ -281,7 +289,7 @@ __global__ void __launch_bounds__(512) k_split_cross_kv(const float *const norme
     const size_t step = (size_t)(min(col0, N - 32) / 32) * (width / 32) * 2;
     const uint4 *tile = weights.w[layer] + step * 128;
     const float inverse = weight.inverses()[min(col0, N - 32) + (lane & 31)];
-    split_tile<2, 1>(normed + (size_t)layer * M * width, width, m0, M, tile, inverse, width / 32, lds, acc);
+    split_tile<2, 1, 2>(normed + (size_t)layer * M * width, width, m0, M, tile, inverse, width / 32, lds, acc);
     if (threadIdx.x >= 256 || col0 >= N) return;
     float *const out = (col0 < xw ? k_out + col0 : v_out + col0 - xw) + (size_t)layer * M * xw + (lane & 31);
     split_store<2, 1>(normed + (size_t)layer * M * width, width, m0, M, weight.values() + step * 128, width / 32, acc, out, xw);
@@ -513,13 +521,19 @@ int launch_split_product(State *st, const float *in, const uint4 *w, size_t rows
         set_error(error, capacity, "f32 product: shape outside the matrix-core kernel's");
         return -1;
     }
-    const int mt = split_row_tiles(st, rows, n, splits > 1), mtiles = (int)((rows + 32 * mt - 1) / (32 * mt)), ntiles = (int)((n + 127) / 128);
+    const int mt = split_row_tiles(st, rows, n, splits > 1), mtiles = (int)((rows + 32 * mt - 1) / (32 * mt));
+    // An unsplit product of 32-row tiles, where that still gives every workgroup a CU of its own: 64 columns a workgroup and four groups of
+    // wavefronts over the channels, twice the workgroups with half the chain.  us a launch, 768 -> 2304 by 64 / 128 columns: 16 rows 8.8 / 11.7,
+    // 96 8.9 / 12.1, 192 10.1 / 13.7.  (Split ones fill the chip by their splits: 16 rows of 3072 -> 768 as twelve, 7.2 / 7.0.)
+    const bool deep = mt == 1 && taps == 1 && splits == 1 && channels % 128 == 0 && (n + 63) / 64 * mtiles <= (size_t)st->cu_count;
+    const int ntiles = (int)((n + (deep ? 63 : 127)) / (deep ? 64 : 128));
     const dim3 grid((unsigned)((ntiles * splits + 7) / 8 * 8 * mtiles)), block(512);
     const auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, block, 0, st->stream, in, w, (int)rows, (int)n, (int)channels, mtiles, ntiles, splits, part);
     };
-    if (taps == 1) mt == 1 ? launch(k_split_rows<1, 1>) : launch(k_split_rows<2, 1>);
-    else mt == 1 ? launch(k_split_rows<1, 3>) : launch(k_split_rows<2, 3>);
+    if (deep) launch(k_split_rows<1, 1, 4>);
+    else if (taps == 1) mt == 1 ? launch(k_split_rows<1, 1, 2>) : launch(k_split_rows<2, 1, 2>);
+    else mt == 1 ? launch(k_split_rows<1, 3, 2>) : launch(k_split_rows<2, 3, 2>);
     return hip_check(hipGetLastError(), "f32 product launch", error, capacity);
 }
 

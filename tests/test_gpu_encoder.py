@@ -206,6 +206,19 @@ def test_encoder_f32_operands_match_oracle(pkg, backend, orc, synth, nerr, causa
     assert nerr(half, got) < 2e-3
 
 
+@pytest.mark.parametrize("tokens,width", [(1, 128), (33, 128), (40, 192), (224, 768), (225, 768)])
+def test_encoder_f32_wide_and_deep_products(pkg, backend, orc, synth, nerr, tokens, width):
+    """The unsplit QKV product by 64 and by 128 columns a workgroup: widths that are and are not a multiple of 128, and the last padded
+    length of 768 whose tiles of 64 columns have a CU each and the first whose have not.  1e-5, the bar of an f32 operator."""
+    _announce("encoder f32 QKV tokens=%d width=%d" % (tokens, width))
+    cfg = dict(synth.encoder_config(layers=1, width=width, heads=width // 64, ffn=256, vocab=300, max_positions=256), causal=True, ffn_kernel=1)
+    w = synth.encoder_weights_f16(cfg, seed=75, kernel=1)
+    ids = np.random.default_rng(76).integers(0, cfg["vocab"], size=tokens).astype(np.int32)
+    got = _prefill_f32(pkg, backend, cfg, w, ids)
+    _, want = orc.encoder_prefill(cfg, _f16_bits(w), ids)
+    assert nerr(got, want) < 1e-5
+
+
 @pytest.mark.parametrize("kernel", [1, 3])
 def test_encoder_f32_operands_match_the_reference_fixture(pkg, backend, synth, nerr, kernel):
     """Against the committed outputs of the compiled reference's transformer_stack, both builds, at the f32 bar."""
