@@ -736,18 +736,24 @@ int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size
 // the f16 form's.  192 tokens, causal, three taps: 3.5 ms as the library's f32 operators one after the other (some forty launches
 // a layer, most of them a fraction of the chip).
 
+constexpr int kThreadsF32 = 512;
+// (what P V's partial sums take is the least)
+size_t attention_f32_lds_bytes(size_t tpad) { return std::max(attention_lds_bytes(tpad), (size_t)3 * 32 * 64 * sizeof(float)); }
+
 // One (32-query tile, head), f32 throughout: S = scale * Q K^T (in LDS) -> softmax numerators and 1 / sum -> P V.
-// Wavefront w scores key tiles w, w + 4, ..; for P V it takes columns 32 * (w % 2) .. over keys half w / 2.  A matrix instruction
-// (v_mfma_f32_32x32x2_f32) takes one value per lane and operand, of inner index l / 32: the scores give lanes below 32 columns 0..31
-// of the head and the rest 32..63, P V gives them keys 0..3 and 4..7 of eight, so that both come in 16-byte reads (any pairing of
-// inner indices is the same sum).  qkv rows are read as they lie: a lane's 128 bytes of its own row cost 64 line visits a
-// request, a quarter of the time the tile's matrix instructions take.
-__global__ void __launch_bounds__(kThreads) k_enc_attention_f32(const float *qkv, float *ctx, const EncParams *params, int tpad, int width, float scale,
+// Eight wavefronts:
+// the longest workgroup's chain bounds the launch (72 workgroups at 192 tokens x 12 heads, whose matrix instructions are 3 of its 11.5 us), and a second wavefront
+// on a SIMD hides a part of the requests.  Wavefront w scores key tiles w, w + 8, ..; for P V it takes columns 32 * (w % 2) .. over the sixteens of keys
+// w / 2, w / 2 + 4, ..  Causal, 192 tokens: 12.2 us by four wavefronts, 11.5 by eight; V requested before the scores as well: 12.0.
+// A matrix instruction (v_mfma_f32_32x32x2_f32) takes one value per lane and operand, of inner index l / 32: the scores give lanes
+// below 32 columns 0..3 of eight and the rest 4..7, P V the same of eight keys, so that both come in 16-byte reads (any pairing of
+// inner indices is the same sum).  qkv rows are read as they lie, 32 line visits a request (64 with columns 0..31 and 32..63: 0.3 us
+// a launch more).
+__global__ void __launch_bounds__(kThreadsF32) k_enc_attention_f32(const float *qkv, float *ctx, const EncParams *params, int tpad, int width, float scale,
                                                                 int causal) {
     const int tokens = params->tokens;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float s_inv[kQTile];
-    __shared__ __align__(16) float s_half[2][16][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hi = lane >> 5;
     const int q0 = blockIdx.x * kQTile, head = blockIdx.y;
     const int keys = causal ? q0 + kQTile : tpad;            // what lies behind is masked for every query here; a multiple of 32
@@ -759,12 +765,12 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention_f32(const float *qkv
     const auto fetch = [&](float (&f)[32], const float *row) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float4 v = *reinterpret_cast<const float4 *>(row + 32 * hi + 4 * i);
+            const float4 v = *reinterpret_cast<const float4 *>(row + 8 * i + 4 * hi);
             f[4 * i] = v.x; f[4 * i + 1] = v.y; f[4 * i + 2] = v.z; f[4 * i + 3] = v.w;
         }
     };
     fetch(fq, base + (size_t)(q0 + (lane & 31)) * stride);
-    for (int tile = wave; tile < keys / 32; tile += 4) {
+    for (int tile = wave; tile < keys / 32; tile += kThreadsF32 / 64) {
         fetch(fk, base + width + (size_t)(tile * 32 + (lane & 31)) * stride);
         floatx16 acc = {0};
 #pragma unroll
@@ -777,20 +783,21 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention_f32(const float *qkv
         }
     }
     __syncthreads();
-    {   // softmax_row_inplace (src/graph.c:245-257) of row tid / 8 by eight lanes; the division by the sum is left to the end
-        const int row = tid >> 3, part = tid & 7;
+    {   // softmax_row_inplace (src/graph.c:245-257) of row tid / 16 by sixteen lanes; the division by the sum is left to the end
+        const int row = tid >> 4, part = tid & 15;
         float4 *srow = reinterpret_cast<float4 *>(S + row * sstride);
         const int npieces = keys / 4;
         float m = -__builtin_inff();   // (every row sees a key: m is one of its scores in the end)
-        for (int c = part; c < npieces; c += 8) {
+        for (int c = part; c < npieces; c += 16) {
             const float4 v = srow[c];
             m = fmaxf(fmaxf(m, fmaxf(v.x, v.y)), fmaxf(v.z, v.w));
         }
         m = fmaxf(m, __shfl_xor(m, 1));
         m = fmaxf(m, __shfl_xor(m, 2));
         m = fmaxf(m, __shfl_xor(m, 4));
+        m = fmaxf(m, __shfl_xor(m, 8));
         float l = 0.0f;
-        for (int c = part; c < npieces; c += 8) {
+        for (int c = part; c < npieces; c += 16) {
             float4 v = srow[c];
             v.x = expf(v.x - m); v.y = expf(v.y - m); v.z = expf(v.z - m); v.w = expf(v.w - m);
             l += (v.x + v.y) + (v.z + v.w);
@@ -799,13 +806,14 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention_f32(const float *qkv
         l += __shfl_xor(l, 1);
         l += __shfl_xor(l, 2);
         l += __shfl_xor(l, 4);
+        l += __shfl_xor(l, 8);
         if (part == 0) s_inv[row] = 1.0f / l;
     }
     __syncthreads();
     {
-        const int wn = wave & 1, kh = wave >> 1, span = keys / 2;   // a multiple of 16
-        const float *prow = S + (lane & 31) * sstride + kh * span + 4 * hi;
-        const float *vcol = base + 2 * width + (size_t)(kh * span + 4 * hi) * stride + wn * 32 + (lane & 31);
+        const int wn = wave & 1, quarter = wave >> 1, last = keys - 16;
+        const float *prow = S + (lane & 31) * sstride + 4 * hi;
+        const float *vcol = base + 2 * width + (size_t)(4 * hi) * stride + wn * 32 + (lane & 31);
         floatx16 acc = {0};
         float fv[2][8];   // sixteen keys of this wavefront's columns, requested a step ahead
         const auto request = [&](float (&f)[8], int k) {
@@ -822,23 +830,26 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention_f32(const float *qkv
                 acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p.w, f[4 * j + 3], acc, 0, 0, 0);
             }
         };
-        request(fv[0], 0);
-        for (int k = 0; k < span; k += 32) {
-            request(fv[1], min(k + 16, span - 16));
+        request(fv[0], min(16 * quarter, last));
+        for (int k = 16 * quarter; k < keys; k += 128) {
+            request(fv[1], min(k + 64, last));
             multiply(fv[0], k);
-            request(fv[0], min(k + 32, span - 16));
-            if (k + 16 < span) multiply(fv[1], k + 16);
+            request(fv[0], min(k + 128, last));
+            if (k + 64 < keys) multiply(fv[1], k + 64);
         }
-        if (kh == 1) {
+        __syncthreads();   // (S is read: the quarters' sums go over it)
+        float *const sums = S + (wn * 16) * 64 + lane;
+        if (quarter > 0) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s_half[wn][r][lane] = acc[r];
+            for (int r = 0; r < 16; ++r) sums[((quarter - 1) * 32 + r) * 64] = acc[r];
         }
         __syncthreads();
-        if (kh == 0) {
+        if (quarter == 0) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int row = acc_row(r, lane);
-                ctx[(size_t)(q0 + row) * width + head * 64 + wn * 32 + (lane & 31)] = (acc[r] + s_half[wn][r][lane]) * s_inv[row];
+                const float sum = ((acc[r] + sums[r * 64]) + sums[(32 + r) * 64]) + sums[(64 + r) * 64];
+                ctx[(size_t)(q0 + row) * width + head * 64 + wn * 32 + (lane & 31)] = sum * s_inv[row];
             }
         }
     }
@@ -886,7 +897,7 @@ int enqueue_prefill_f32(State *st, mynah_hip_encoder *e, int tpad, char *error, 
         if (l > 0) launch_rows<ROWS_F32>(st, (int)w, e->x, pending, down_splits, rows * w, e->n1g[l], e->n1b[l], e->f_nrm, e->params, tpad);
         // (not split: the attention kernel reads every row several times and would add the planes up as often)
         if (launch_split_product(st, e->f_nrm, e->qkv32[l], rows, w, 1, 3 * w, 1, e->f_qkv, error, capacity) != 0) return -1;
-        hipLaunchKernelGGL(k_enc_attention_f32, dim3(tpad / kQTile, (unsigned)e->heads), dim3(kThreads), attention_lds_bytes(rows), st->stream, e->f_qkv, e->f_ctx,
+        hipLaunchKernelGGL(k_enc_attention_f32, dim3(tpad / kQTile, (unsigned)e->heads), dim3(kThreadsF32), attention_f32_lds_bytes(rows), st->stream, e->f_qkv, e->f_ctx,
                            e->params, tpad, (int)w, scale, e->causal);
         if (launch_split_product(st, e->f_ctx, e->o32[l], rows, w, 1, w, o_splits, e->part, error, capacity) != 0) return -1;
         launch_rows<ROWS_F32>(st, (int)w, e->x, e->part, o_splits, rows * w, e->n2g[l], e->n2b[l], e->f_nrm, e->params, tpad);

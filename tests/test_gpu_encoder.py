@@ -206,6 +206,19 @@ def test_encoder_f32_operands_match_oracle(pkg, backend, orc, synth, nerr, causa
     assert nerr(half, got) < 2e-3
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("tokens", [32, 33, 65, 129, 257, 1000])
+def test_encoder_f32_attention_key_counts(pkg, backend, orc, synth, nerr, tokens, causal):
+    """Key tiles and sixteens of keys that leave some of the eight wavefronts idle in their last turn, and the longest rows."""
+    _announce("encoder f32 attention tokens=%d causal=%s" % (tokens, causal))
+    cfg = dict(synth.encoder_config(layers=1, width=64, heads=1, ffn=128, vocab=300, max_positions=1024), causal=causal, ffn_kernel=1)
+    w = synth.encoder_weights_f16(cfg, seed=77, kernel=1)
+    ids = np.random.default_rng(78).integers(0, cfg["vocab"], size=tokens).astype(np.int32)
+    got = _prefill_f32(pkg, backend, cfg, w, ids)
+    _, want = orc.encoder_prefill(cfg, _f16_bits(w), ids)
+    assert nerr(got, want) < 1e-5
+
+
 @pytest.mark.parametrize("tokens,width", [(1, 128), (33, 128), (40, 192), (224, 768), (225, 768)])
 def test_encoder_f32_wide_and_deep_products(pkg, backend, orc, synth, nerr, tokens, width):
     """The unsplit QKV product by 64 and by 128 columns a workgroup: widths that are and are not a multiple of 128, and the last padded
