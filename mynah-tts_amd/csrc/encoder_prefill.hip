@@ -471,19 +471,24 @@ int launch_first(State *st, EncFirst &a, const int32_t *ids, char *error, size_t
     return hip_check(hipGetLastError(), "encoder embedding launch", error, capacity);
 }
 
+constexpr int kAttentionThreads = 512;
+
 // One (32-query tile, head): S = scale * Q K^T over all keys (f32, in LDS) -> row softmax numerators
 // (f16, written over the row's own storage) and denominators -> O = P V / denom.
-// Wavefront w takes key tiles w, w+4, ... for the scores and, for PV, output columns 32*(w & 1) .. +31
-// over the key half (w >> 1); the two halves meet in LDS.
-// kKeyTiles, kValueSteps: score tiles and PV steps of a wavefront whose fragments are requested up front; the launch
-// picks the smallest pair that covers the padded length (up to 4 and 16: 512 tokens), so that none is requested in vain.
-template <int kKeyTiles, int kValueSteps>
-__global__ void __launch_bounds__(kThreads) k_enc_attention(const _Float16 *qk, const _Float16 *vt, _Float16 *ctx, const EncParams *params,
+// Wavefront w takes key tiles w, w+8, ... for the scores and, for PV, output columns 32*(w & 1) .. +31
+// over the key quarter (w >> 1); the quarters meet in LDS.
+// Its chain bounds a launch (96 workgroups at 256 tokens x 12 heads): eight wavefronts, so that each has half the requests, tiles and steps of four, and
+// sixteen lanes a row with no more pieces than the length has.  us a launch, four wavefronts and 32 pieces a lane / this: 60 tokens 5.5 / 4.6,
+// 128 6.7 / 4.7, 192 7.4 / 5.3, 512 11.4 / 8.8; a prefill of 256 tokens 235 / 223.
+// kKeyTiles, kValueSteps: score tiles and PV steps of a wavefront whose fragments are requested up front; kPieces: float4 pieces of a
+// score row that a softmax lane may hold.  The launch picks the smallest set that covers the padded length (tiles and steps up to 512
+// tokens, pieces up to 1024), so that none is requested or stepped over in vain.
+template <int kKeyTiles, int kValueSteps, int kPieces>
+__global__ void __launch_bounds__(kAttentionThreads) k_enc_attention(const _Float16 *qk, const _Float16 *vt, _Float16 *ctx, const EncParams *params,
                                                             int tpad, int width, float scale, int causal) {
     const int tokens = params->tokens;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float s_inv[kQTile];
-    __shared__ __align__(16) float s_half[2][16][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q0 = blockIdx.x * kQTile, head = blockIdx.y;
     const int sstride = tpad + kScorePad;                    // floats per score row
@@ -497,19 +502,19 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention(const _Float16 *qk, 
     // how many may still be out, and behind a conditional request the compiler has to wait for everything.
     const int heads = width / 64;
     const int ntiles = tpad / 32;
-    const int wn = wave & 1, kh = wave >> 1;
-    const int kspan = tpad / 2;                              // keys per PV half, multiple of 32
+    const int wn = wave & 1, quarter = wave >> 1;
+    const int kspan = tpad / 4;                              // keys per PV quarter, multiple of 16
     // Every request is one operand of one matrix instruction for the whole wavefront, 1 KiB of consecutive bytes (see the
     // layout note at the top).
     const half8 *qblock = reinterpret_cast<const half8 *>(qk + ((size_t)head * ntiles + q0 / 32) * 2048) + lane;
     const half8 *kblocks = reinterpret_cast<const half8 *>(qk + (size_t)(heads + head) * ntiles * 2048) + lane;
-    const half8 *vblocks = reinterpret_cast<const half8 *>(vt + ((size_t)(head * 2 + wn) * (tpad / 16) + kh * (kspan / 16)) * 512) + lane;
+    const half8 *vblocks = reinterpret_cast<const half8 *>(vt + ((size_t)(head * 2 + wn) * (tpad / 16) + quarter * (kspan / 16)) * 512) + lane;
     half8 fq[4], fk[kKeyTiles][4], fv[kValueSteps];
 #pragma unroll
     for (int j = 0; j < 4; ++j) fq[j] = qblock[j * 64];
 #pragma unroll
     for (int t = 0; t < kKeyTiles; ++t) {
-        const int tile = min(wave + 4 * t, ntiles - 1);
+        const int tile = min(wave + 8 * t, ntiles - 1);
 #pragma unroll
         for (int j = 0; j < 4; ++j) fk[t][j] = kblocks[(size_t)tile * 256 + j * 64];
     }
@@ -532,8 +537,8 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention(const _Float16 *qk, 
         };
 #pragma unroll
         for (int t = 0; t < kKeyTiles; ++t)
-            if (wave + 4 * t < ntiles) score_tile(wave + 4 * t, fk[t]);
-        for (int tile = wave + 4 * kKeyTiles; tile < ntiles; tile += 4) {   // beyond the tiles requested up front (more than 512 tokens)
+            if (wave + 8 * t < ntiles) score_tile(wave + 8 * t, fk[t]);
+        for (int tile = wave + 8 * kKeyTiles; tile < ntiles; tile += 8) {   // beyond the tiles requested up front (more than 512 tokens)
             half8 k4[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) k4[j] = kblocks[(size_t)tile * 256 + j * 64];
@@ -542,13 +547,12 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention(const _Float16 *qk, 
     }
     __syncthreads();
 
-    // ---- softmax of row tid / 8 by eight adjacent lanes (softmax_row_inplace, src/graph.c:245-257).  A lane takes
-    // float4 pieces part, part + 8, ... of the row (up to kPieces of them in registers, i.e. 1024 keys), so the row is
-    // read from LDS once.  The numerators go back as f16 over the first half of the row's own bytes: the eight lanes
+    // ---- softmax of row tid / 16 by sixteen adjacent lanes (softmax_row_inplace, src/graph.c:245-257).  A lane takes
+    // float4 pieces part, part + 16, ... of the row (up to kPieces of them in registers), so the row is
+    // read from LDS once.  The numerators go back as f16 over the first half of the row's own bytes: the sixteen lanes
     // of a row belong to one wavefront and all of their reads are done before the first of these writes is issued.
     {
-        constexpr int kPieces = 32;
-        const int row = tid >> 3, part = tid & 7;
+        const int row = tid >> 4, part = tid & 15;
         const float4 *srow = reinterpret_cast<const float4 *>(S + row * sstride);
         half4 *prow = reinterpret_cast<half4 *>(S + row * sstride);
         const int npieces = tpad / 4;
@@ -556,7 +560,7 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention(const _Float16 *qk, 
         float m = -3.0e38f;
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
-            const int c = part + 8 * i;
+            const int c = part + 16 * i;
             if (c < npieces) {
                 v[i] = srow[c];
                 m = fmaxf(fmaxf(m, fmaxf(v[i].x, v[i].y)), fmaxf(v[i].z, v[i].w));
@@ -565,10 +569,11 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention(const _Float16 *qk, 
         m = fmaxf(m, __shfl_xor(m, 1));
         m = fmaxf(m, __shfl_xor(m, 2));
         m = fmaxf(m, __shfl_xor(m, 4));
+        m = fmaxf(m, __shfl_xor(m, 8));
         float l = 0.0f;
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
-            const int c = part + 8 * i;
+            const int c = part + 16 * i;
             if (c < npieces) {
                 // hardware exponential: the numerators are rounded to f16 anyway; masked keys hold -3e38 and give 0
                 const float e0 = __expf(v[i].x - m), e1 = __expf(v[i].y - m), e2 = __expf(v[i].z - m), e3 = __expf(v[i].w - m);
@@ -580,13 +585,14 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention(const _Float16 *qk, 
         l += __shfl_xor(l, 1);
         l += __shfl_xor(l, 2);
         l += __shfl_xor(l, 4);
+        l += __shfl_xor(l, 8);
         if (part == 0) s_inv[row] = 1.0f / l;
     }
     __syncthreads();
 
     // ---- P V
     {
-        const _Float16 *prow = reinterpret_cast<const _Float16 *>(S + (lane & 31) * sstride) + kh * kspan + 8 * (lane >> 5);
+        const _Float16 *prow = reinterpret_cast<const _Float16 *>(S + (lane & 31) * sstride) + quarter * kspan + 8 * (lane >> 5);
         floatx16 acc = {0};
 #pragma unroll
         for (int st = 0; st < kValueSteps; ++st) {
@@ -600,16 +606,18 @@ __global__ void __launch_bounds__(kThreads) k_enc_attention(const _Float16 *qk, 
             const half8 fvk = vblocks[(k / 16) * 64];
             acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fp, fvk, acc, 0, 0, 0);
         }
-        if (kh == 1) {
+        __syncthreads();   // (S is read: the quarters' sums go over it)
+        float *const sums = S + wn * 16 * 64 + lane;
+        if (quarter > 0) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s_half[wn][r][lane] = acc[r];
+            for (int r = 0; r < 16; ++r) sums[((quarter - 1) * 32 + r) * 64] = acc[r];
         }
         __syncthreads();
-        if (kh == 0) {
+        if (quarter == 0) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int row = acc_row(r, lane);
-                const float o = (acc[r] + s_half[wn][r][lane]) * s_inv[row];
+                const float o = (((acc[r] + sums[r * 64]) + sums[(32 + r) * 64]) + sums[(64 + r) * 64]) * s_inv[row];
                 ctx[(size_t)(q0 + row) * width + head * 64 + wn * 32 + (lane & 31)] = (_Float16)o;
             }
         }
@@ -669,7 +677,8 @@ int tap_major_f16(State *st, const float *host, size_t n, size_t cin, size_t tap
     return 0;
 }
 
-size_t attention_lds_bytes(size_t tpad) { return (size_t)kQTile * (tpad + kScorePad) * sizeof(float); }
+// The scores, and over them what P V's partial sums take.
+size_t attention_lds_bytes(size_t tpad) { return std::max((size_t)kQTile * (tpad + kScorePad), (size_t)3 * 32 * 64) * sizeof(float); }
 
 constexpr int kMaxSplits = 4;   // k_enc_rows reads exactly this many partial planes at most
 // Most splits that leave each workgroup at least three K steps, preferring a step count the products' pipeline takes
@@ -700,11 +709,11 @@ int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size
         g.out = e->qk; g.vt = e->vt; g.width = w;
         if (launch_gemm<ENC_QKV>(st, g, 1, error, capacity) != 0) return -1;
         {
-            // a wavefront scores every fourth 32-key tile and multiplies half of the keys in steps of 16
-            const dim3 agrid(tpad / kQTile, (unsigned)e->heads), ablock(kThreads);
-            if (tpad <= 128) hipLaunchKernelGGL((k_enc_attention<1, 4>), agrid, ablock, lds, st->stream, e->qk, e->vt, e->ctx, e->params, tpad, w, scale, e->causal);
-            else if (tpad <= 256) hipLaunchKernelGGL((k_enc_attention<2, 8>), agrid, ablock, lds, st->stream, e->qk, e->vt, e->ctx, e->params, tpad, w, scale, e->causal);
-            else hipLaunchKernelGGL((k_enc_attention<4, 16>), agrid, ablock, lds, st->stream, e->qk, e->vt, e->ctx, e->params, tpad, w, scale, e->causal);
+            // a wavefront scores every eighth 32-key tile and multiplies a quarter of the keys in steps of 16
+            const dim3 agrid(tpad / kQTile, (unsigned)e->heads), ablock(kAttentionThreads);
+            if (tpad <= 128) hipLaunchKernelGGL((k_enc_attention<1, 2, 2>), agrid, ablock, lds, st->stream, e->qk, e->vt, e->ctx, e->params, tpad, w, scale, e->causal);
+            else if (tpad <= 256) hipLaunchKernelGGL((k_enc_attention<1, 4, 4>), agrid, ablock, lds, st->stream, e->qk, e->vt, e->ctx, e->params, tpad, w, scale, e->causal);
+            else hipLaunchKernelGGL((k_enc_attention<2, 8, 16>), agrid, ablock, lds, st->stream, e->qk, e->vt, e->ctx, e->params, tpad, w, scale, e->causal);
         }
         g = GemmArgs{};
         g.a = e->ctx; g.w = static_cast<const _Float16 *>(e->o[l]->data); g.M = tpad; g.N = w; g.K = w; g.part = e->part;
@@ -736,10 +745,6 @@ int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size
 // the f16 form's.  192 tokens, causal, three taps: 3.5 ms as the library's f32 operators one after the other (some forty launches
 // a layer, most of them a fraction of the chip).
 
-constexpr int kThreadsF32 = 512;
-// (what P V's partial sums take is the least)
-size_t attention_f32_lds_bytes(size_t tpad) { return std::max(attention_lds_bytes(tpad), (size_t)3 * 32 * 64 * sizeof(float)); }
-
 // One (32-query tile, head), f32 throughout: S = scale * Q K^T (in LDS) -> softmax numerators and 1 / sum -> P V.
 // Eight wavefronts:
 // the longest workgroup's chain bounds the launch (72 workgroups at 192 tokens x 12 heads, whose matrix instructions are 3 of its 11.5 us), and a second wavefront
@@ -749,7 +754,7 @@ size_t attention_f32_lds_bytes(size_t tpad) { return std::max(attention_lds_byte
 // below 32 columns 0..3 of eight and the rest 4..7, P V the same of eight keys, so that both come in 16-byte reads (any pairing of
 // inner indices is the same sum).  qkv rows are read as they lie, 32 line visits a request (64 with columns 0..31 and 32..63: 0.3 us
 // a launch more).
-__global__ void __launch_bounds__(kThreadsF32) k_enc_attention_f32(const float *qkv, float *ctx, const EncParams *params, int tpad, int width, float scale,
+__global__ void __launch_bounds__(kAttentionThreads) k_enc_attention_f32(const float *qkv, float *ctx, const EncParams *params, int tpad, int width, float scale,
                                                                 int causal) {
     const int tokens = params->tokens;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -770,7 +775,7 @@ __global__ void __launch_bounds__(kThreadsF32) k_enc_attention_f32(const float *
         }
     };
     fetch(fq, base + (size_t)(q0 + (lane & 31)) * stride);
-    for (int tile = wave; tile < keys / 32; tile += kThreadsF32 / 64) {
+    for (int tile = wave; tile < keys / 32; tile += kAttentionThreads / 64) {
         fetch(fk, base + width + (size_t)(tile * 32 + (lane & 31)) * stride);
         floatx16 acc = {0};
 #pragma unroll
@@ -897,7 +902,7 @@ int enqueue_prefill_f32(State *st, mynah_hip_encoder *e, int tpad, char *error, 
         if (l > 0) launch_rows<ROWS_F32>(st, (int)w, e->x, pending, down_splits, rows * w, e->n1g[l], e->n1b[l], e->f_nrm, e->params, tpad);
         // (not split: the attention kernel reads every row several times and would add the planes up as often)
         if (launch_split_product(st, e->f_nrm, e->qkv32[l], rows, w, 1, 3 * w, 1, e->f_qkv, error, capacity) != 0) return -1;
-        hipLaunchKernelGGL(k_enc_attention_f32, dim3(tpad / kQTile, (unsigned)e->heads), dim3(kThreadsF32), attention_f32_lds_bytes(rows), st->stream, e->f_qkv, e->f_ctx,
+        hipLaunchKernelGGL(k_enc_attention_f32, dim3(tpad / kQTile, (unsigned)e->heads), dim3(kAttentionThreads), attention_lds_bytes(rows), st->stream, e->f_qkv, e->f_ctx,
                            e->params, tpad, (int)w, scale, e->causal);
         if (launch_split_product(st, e->f_ctx, e->o32[l], rows, w, 1, w, o_splits, e->part, error, capacity) != 0) return -1;
         launch_rows<ROWS_F32>(st, (int)w, e->x, e->part, o_splits, rows * w, e->n2g[l], e->n2b[l], e->f_nrm, e->params, tpad);
@@ -1040,9 +1045,9 @@ extern "C" int mynah_hip_encoder_create(void *state, const mynah_hip_encoder_des
     }
     if (attention_lds_bytes(e->tpad_max) > 48 * 1024) {
         const int bytes = (int)attention_lds_bytes(e->tpad_max);
-        if (hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<1, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
-            hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
-            hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<4, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
+        if (hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<1, 2, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
+            hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<1, 4, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
+            hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention<2, 8, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0 ||
             hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(k_enc_attention_f32), hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "encoder attention LDS size", error, capacity) != 0)
             return fail();
     }

@@ -207,6 +207,20 @@ def test_encoder_f32_operands_match_oracle(pkg, backend, orc, synth, nerr, causa
 
 
 @pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("tokens", [64, 65, 128, 129, 256, 257, 513, 1000])
+def test_encoder_f16_attention_key_counts(pkg, backend, orc, synth, nerr, tokens, causal):
+    """The padded lengths at which the attention's build changes, and key tiles and steps beyond those requested up front: the bar of the
+    f16 form."""
+    _announce("encoder f16 attention tokens=%d causal=%s" % (tokens, causal))
+    cfg = dict(synth.encoder_config(layers=1, width=64, heads=1, ffn=128, vocab=300, max_positions=1024), causal=causal, ffn_kernel=1)
+    w = synth.encoder_weights_f16(cfg, seed=79, kernel=1)
+    ids = np.random.default_rng(80).integers(0, cfg["vocab"], size=tokens).astype(np.int32)
+    got = _prefill(pkg, backend, cfg, w, ids)
+    _, want = orc.encoder_prefill(cfg, _f16_bits(w), ids)
+    assert nerr(got, want) < 2e-3
+
+
+@pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("tokens", [32, 33, 65, 129, 257, 1000])
 def test_encoder_f32_attention_key_counts(pkg, backend, orc, synth, nerr, tokens, causal):
     """Key tiles and sixteens of keys that leave some of the eight wavefronts idle in their last turn, and the longest rows."""
