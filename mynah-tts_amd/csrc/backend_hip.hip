@@ -277,8 +277,8 @@ int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch
     return 0;
 }
 
-int cached_split_weight(State *st, const float *host, size_t n, size_t channels, size_t taps, const uint4 **out, char *error, size_t capacity) {
-    if (host == nullptr || n == 0 || n % 32 != 0 || channels == 0 || channels % 64 != 0 || (taps != 1 && taps != 3) || n > SIZE_MAX / channels / taps / sizeof(float) / 4) {
+int cached_split_weight(State *st, const float *host, size_t n, size_t channels, size_t taps, const float4 **out, char *error, size_t capacity) {
+    if (host == nullptr || n == 0 || n % 32 != 0 || channels == 0 || channels % 64 != 0 || (taps != 1 && taps != 3) || n > SIZE_MAX / channels / taps / sizeof(float) / 2) {
         set_error(error, capacity, "invalid product weight");
         return -1;
     }
@@ -287,22 +287,22 @@ int cached_split_weight(State *st, const float *host, size_t n, size_t channels,
     std::lock_guard<std::mutex> lock(st->mu);
     auto it = st->weights.find(key);
     if (it != st->weights.end()) {
-        *out = static_cast<const uint4 *>(it->second.data);
+        *out = static_cast<const float4 *>(it->second.data);
         return 0;
     }
     if (stage_weight(st, host, count, error, capacity) != 0) return -1;
     CachedWeight cw;
     cw.n = n;
     cw.k = channels * taps;
-    cw.bytes = count * 8 + n * sizeof(float) + kSplitWeightOverrun;   // two pieces a value and the value, a scale an output
+    cw.bytes = count * sizeof(float) + kSplitWeightOverrun;
     MYNAH_TRY(hipMalloc(&cw.data, cw.bytes));
-    if (launch_split_pack(st, st->pack_staging, static_cast<uint4 *>(cw.data), n, channels, taps, error, capacity) != 0) {
+    if (launch_split_pack(st, st->pack_staging, static_cast<float4 *>(cw.data), n, channels, taps, error, capacity) != 0) {
         (void)hipFree(cw.data);
         return -1;
     }
     st->weight_bytes += cw.bytes;
     st->weights.emplace(key, cw);
-    *out = static_cast<const uint4 *>(cw.data);
+    *out = static_cast<const float4 *>(cw.data);
     return 0;
 }
 

@@ -1604,6 +1604,38 @@ int launch_conv_split_batch(State *st, ConvBatchArgs &b, int count, char *error,
 
 }  // namespace
 
+// A weight's rows get a scale each: the largest value under it lies in [2^13, 2^14), unless it is 2^20 times the row's usual size and
+// more -- then what is 2^20 times that lies there, and what does not fit above it is kept as its bits (half_product.h).  A workgroup a row, four
+// requests of a thread side by side (a wavefront a row and one request at a time: 39 us for 768 x 6912); rows past the last one get 1.
+__global__ void __launch_bounds__(256) k_half_row_scales(const float *src, float *inverses, int rows, size_t per_row) {
+    __shared__ float s4[4];
+    const int row = (int)blockIdx.x, tid = (int)threadIdx.x;
+    float sum = 0.0f, count = 0.0f, most = -127.0f;
+    if (row < rows)
+        for (size_t i0 = 0; i0 < per_row; i0 += 1024) {
+            float v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = src[(size_t)row * per_row + min(i0 + 256 * k + tid, per_row - 1)];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int e = exponent_of(v[k]);
+                const bool counts = i0 + 256 * k + tid < per_row && v[k] != 0.0f && e != 128;   // (else nothing, or no finite number)
+                sum += counts ? (float)e : 0.0f;
+                count += counts ? 1.0f : 0.0f;
+                most = counts ? fmaxf(most, (float)e) : most;
+            }
+        }
+    sum = block_sum(sum, s4);
+    count = block_sum(count, s4);
+    most = block_max(most, s4);
+    const int top = count == 0.0f ? 13 : (int)fminf(most, floorf(sum / count) + 20.0f);
+    if (tid == 0) inverses[row] = power_of_two(max(top - 13, -126));
+}
+int mynah::launch_half_row_scales(State *st, const float *src, float *inverses, size_t rows, size_t padded_rows, size_t per_row, char *error, size_t capacity) {
+    hipLaunchKernelGGL(k_half_row_scales, dim3((unsigned)padded_rows), dim3(256), 0, st->stream, src, inverses, (int)rows, per_row);
+    return hip_check(hipGetLastError(), "weight scale launch", error, capacity);
+}
+
 int mynah::launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_ch, size_t in_ch, size_t kernel, char *error, size_t capacity) {
     const size_t blocks = (in_ch + 15) / 16, count = (out_ch + 31) / 32 * blocks * kernel * 64;
     const size_t rows = (out_ch + 31) / 32 * 32;

@@ -243,7 +243,7 @@ struct ConvBlocks {
 int cached_snake_pairs(State *st, const float *host, size_t n, const float **dev, char *error, size_t capacity);
 int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch, size_t kernel, ConvBlocks *out, char *error, size_t capacity);
 // An f32 weight [n, channels, taps] in the order in which split_product.hip's kernels take it; n a multiple of 32, channels of 64.
-int cached_split_weight(State *st, const float *host, size_t n, size_t channels, size_t taps, const uint4 **out, char *error, size_t capacity);
+int cached_split_weight(State *st, const float *host, size_t n, size_t channels, size_t taps, const float4 **out, char *error, size_t capacity);
 int ensure_attention_workspace(State *st, size_t batch, size_t heads, size_t head_width, size_t max_valid,
                                char *error, size_t capacity, size_t chunk_rows = kAttnChunk);
 int ensure_pinned(State *st, size_t bytes, char *error, size_t capacity);

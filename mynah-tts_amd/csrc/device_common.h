@@ -118,7 +118,7 @@ __device__ __forceinline__ float block_max(float v, float *s4) {
 }
 
 // mynah_layernorm_f32 (src/kernels.c:186-244): mean, then the variance of (x - mean), eps inside the
-// square root, y = (x - mean) * scale * gain (+ bias).  One workgroup per row.  A null gain is ones (the row normalised and no more).
+// square root, y = (x - mean) * scale * gain (+ bias).  One workgroup per row.
 // Rows of up to 256 * NV values stay in registers: one round trip for the row, its gain and its bias (requested side by
 // side, none under a condition) instead of three passes over memory with a round trip per 256 values each.  A thread
 // adds its values in the order of the loop below, so the results are the same bits.
@@ -126,17 +126,13 @@ template <int NV>
 __device__ __forceinline__ void layernorm_row_in_registers(const float *x, float *y, const float *gain, const float *bias, int width,
                                                            float *s4) {
     float xv[NV], gv[NV], bv[NV];
-    const float *const gain_or_row = gain != nullptr ? gain : x, *const bias_or_gain = bias != nullptr ? bias : gain_or_row;
+    const float *bias_or_gain = bias != nullptr ? bias : gain;
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
         const int i = threadIdx.x + 256 * u, at = i < width ? i : width - 1;
         xv[u] = x[at];
-        gv[u] = gain_or_row[at];
+        gv[u] = gain[at];
         bv[u] = bias_or_gain[at];
-    }
-    if (gain == nullptr) {
-#pragma unroll
-        for (int u = 0; u < NV; ++u) gv[u] = 1.0f;
     }
     float s = 0.0f;
 #pragma unroll
@@ -173,17 +169,13 @@ __device__ __forceinline__ void layernorm_row_as_prologue(const float *x, float 
     const int nf4 = width >> 2;
     const int tid = threadIdx.x & 255;
     float4 xv[NV4], gv[NV4], bv[NV4];
-    const float *const gain_or_row = gain != nullptr ? gain : x, *const bias_or_gain = bias != nullptr ? bias : gain_or_row;
+    const float *bias_or_gain = bias != nullptr ? bias : gain;
 #pragma unroll
     for (int i = 0; i < NV4; ++i) {
         const int f = tid + 256 * i, at = f < nf4 ? f : nf4 - 1;
         xv[i] = reinterpret_cast<const float4 *>(x)[at];
-        gv[i] = reinterpret_cast<const float4 *>(gain_or_row)[at];
+        gv[i] = reinterpret_cast<const float4 *>(gain)[at];
         bv[i] = reinterpret_cast<const float4 *>(bias_or_gain)[at];
-    }
-    if (gain == nullptr) {
-#pragma unroll
-        for (int i = 0; i < NV4; ++i) gv[i] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
     }
     float s = 0.0f;
 #pragma unroll
@@ -238,7 +230,7 @@ __device__ __forceinline__ void layernorm_row(const float *x, float *y, const fl
     const float variance = block_sum(v, s4);
     const float scale = 1.0f / sqrtf(variance / (float)width + 1.0e-5f);
     for (int i = threadIdx.x; i < width; i += 256) {
-        float z = ((x[i] - mean) * scale) * (gain != nullptr ? gain[i] : 1.0f);
+        float z = ((x[i] - mean) * scale) * gain[i];
         if (bias != nullptr) z += bias[i];
         y[i] = z;
     }

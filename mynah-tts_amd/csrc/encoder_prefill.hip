@@ -67,7 +67,7 @@ struct mynah_hip_encoder {
     // order of split_product.hip, f32 rows padded like the f16 form's
     bool f32 = false;
     const CachedWeight *tok32 = nullptr, *pos32 = nullptr;
-    std::vector<const uint4 *> qkv32, o32, up32, down32;
+    std::vector<const float4 *> qkv32, o32, up32, down32;
     float *f_nrm = nullptr, *f_qkv = nullptr, *f_ctx = nullptr, *f_hid = nullptr;
     float *f_nrm_alloc = nullptr, *f_hid_alloc = nullptr;   // f_nrm and f_hid begin kLeadRows rows into these
 };
@@ -740,8 +740,8 @@ int enqueue_prefill(State *st, mynah_hip_encoder *e, int tpad, char *error, size
 // ---- f32 operands: the stack as the reference computes it ---------------------------------------------------------------
 // transformer_stack (src/graph.c:634-711) is LayerNorm -> QKV linear -> per head scaled Q K^T -> masked row softmax -> P V -> O linear
 // -> residual -> LayerNorm -> causal_conv_ffn -> residual, all f32.  This form keeps every value f32 -- only the order of additions
-// inside a product differs from the CPU: 1e-5 instead of the 2e-3 of f16 operands.  The products run on the f16 matrix cores in
-// two-piece form (half_product.h: f32 operands, f32 sums), scores and P V on the f32 ones, in eight kernels a layer, captured like
+// inside a product differs from the CPU: 1e-5 instead of the 2e-3 of f16 operands.  The products run on the bf16 matrix cores in
+// three-piece form (split_product.h: f32 operands, f32 sums), scores and P V on the f32 ones, in eight kernels a layer, captured like
 // the f16 form's.  192 tokens, causal, three taps: 3.5 ms as the library's f32 operators one after the other (some forty launches
 // a layer, most of them a fraction of the chip).
 
@@ -972,7 +972,7 @@ extern "C" int mynah_hip_encoder_create(void *state, const mynah_hip_encoder_des
             return fail();
         }
         if (e->f32) {
-            const uint4 *packed = nullptr;
+            const float4 *packed = nullptr;
             if (cached_split_weight(st, d->qkv_w[l], 3 * d->width, d->width, 1, &packed, error, capacity) != 0) return fail();
             e->qkv32.push_back(packed);
             if (cached_split_weight(st, d->o_w[l], d->width, d->width, 1, &packed, error, capacity) != 0) return fail();

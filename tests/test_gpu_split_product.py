@@ -1,4 +1,4 @@
-"""The f32 products on the f16 matrix cores (two f16 pieces per operand) through the entry points that use them, at the edges of
+"""The f32 products on the bf16 matrix cores (three bf16 pieces per operand) through the entry points that use them, at the edges of
 their tiles: rows around 32 / 64 / a second tile, output widths that end inside a 128-column tile, more layers than one launch
 takes, both FFN forms.  Against float64 (cross K/V, weights with all 24 bits and rows of very different size) and the oracle."""
 import numpy as np
@@ -87,7 +87,7 @@ def test_one_buffer_under_two_shapes(backend, pkg, orc):
 
 
 def test_cross_kv_extremes(backend, pkg, orc):
-    """Operands without two finite f16 pieces: infinities, NaN, values up to f32's largest.  What f32 multiply-adds give, and only in
+    """Operands without three finite bf16 pieces: infinities, NaN, values from 2^128 - 2^119 on.  What f32 multiply-adds give, and only in
     the outputs that they enter."""
     print("[gpu-case] cross K/V extremes", flush=True)
     rng = np.random.default_rng(8)
@@ -163,8 +163,8 @@ def test_encoder_f32_large_weights(backend, pkg, synth, nerr, taps):
 
 
 def test_cross_kv_tiny_weights(backend, pkg, orc):
-    """Rows of weights down to 2^-126, each under a scale of its own, which ends at 2^126: what is lost of a term is no more than half of
-    2^-133."""
+    """Below 2^-110 an operand keeps fewer than its 24 bits: its third piece ends at bf16's smallest subnormal, 2^-133, so that at most half
+    of that is lost."""
     print("[gpu-case] cross K/V, tiny weights", flush=True)
     rng = np.random.default_rng(9)
     backend.set_quant(pkg.F32)
@@ -219,8 +219,8 @@ def test_workspace_and_weight_memory(backend, pkg, synth):
 @pytest.mark.parametrize("bias", ["none", "all", "some"])
 @pytest.mark.parametrize("rows", [65, 128, 129, 193, 256, 257, 300])
 def test_cross_kv_wide_tiles(backend, pkg, orc, rows, bias):
-    """More rows than one 64-row tile, in workgroups of 64 to 256: the last row of a tile and the first of the next, widths that end inside a
-    128-column tile, with and without LayerNorm biases (and in only some of the layers: the narrow tiles), an infinity in one row."""
+    """More rows than one 64-row tile: the last row of a tile and the first of the next, widths that end inside a 128-column tile, with and
+    without LayerNorm biases (and in only some of the layers), an infinity in one row."""
     print("[gpu-case] cross K/V wide rows=%d bias=%s" % (rows, bias), flush=True)
     rng = np.random.default_rng(rows)
     backend.set_quant(pkg.F32)
@@ -242,6 +242,72 @@ def test_cross_kv_wide_tiles(backend, pkg, orc, rows, bias):
     for l in range(layers):
         normed = np.stack([orc.layernorm(r, gains[l], biases[l]) for r in memory[keep]]).astype(np.float64)
         want = normed @ kvw[l].astype(np.float64).T
-        assert np.linalg.norm(got[l][keep] - want) < 1e-6 * np.linalg.norm(want), l       # (22 bits an operand, f32 sums of 128 terms)
+        assert np.linalg.norm(got[l][keep] - want) < 1e-6 * np.linalg.norm(want), l       # (f32 sums of 128 terms)
     for d in (dmem, dk, dv):
         d.free()
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("rows", [40, 70, 150, 256, 300])
+def test_cross_kv_rows_of_different_size(backend, pkg, orc, rows, bias):
+    """Rows that lie beside much larger ones in a tile (the LayerNorm's eps leaves a row of 1e-9 at 3e-7), and channels of very different
+    gain under weights that make up for it: f32's accuracy in every row.  An infinity in one row changes no other, and a row's bits do not depend
+    on how many are beside it."""
+    print("[gpu-case] cross K/V rows of different size, %d, bias %s" % (rows, bias), flush=True)
+    rng = np.random.default_rng(rows)
+    backend.set_quant(pkg.F32)
+    width, xw = 128, 96
+    size = np.exp2(rng.choice([0, -6, -16, -24], size=(1, width))).astype(np.float32)
+    gain = backend.keep(((1.0 + 0.1 * rng.standard_normal((1, width))) * size).astype(np.float32)[0])
+    biases = [backend.keep((1e-8 * rng.standard_normal((1, width)) * size).astype(np.float32)[0])] if bias else None
+    kvw = backend.keep((rng.standard_normal((2 * xw, width)) / size).astype(np.float32))
+    memory = (rng.standard_normal((rows, width)) * 10.0 ** rng.choice([0, -5, -7, -9], size=(rows, 1))).astype(np.float32)
+    infinite = rows // 3
+    memory[infinite, 5] = np.inf
+    dmem = backend.alloc(rows * width).write(memory)
+    dk, dv = (backend.alloc(rows * xw) for _ in range(2))
+    backend.cross_kv_dev(dmem.ptr, rows, width, [gain], biases, [kvw], xw, dk.ptr, dv.ptr)
+    got = np.concatenate([dk.read().reshape(rows, xw), dv.read().reshape(rows, xw)], axis=1)
+    assert np.isnan(got[infinite]).all()
+    keep = np.arange(rows) != infinite
+    normed = np.stack([orc.layernorm(r, gain, biases[0] if bias else None) for r in memory[keep]]).astype(np.float64)
+    want = normed @ kvw.astype(np.float64).T
+    # operands in full, f32 sums of 128 terms, and the rounding of the row's mean (some 2^-24 of the row): the bar of test_cross_kv_tiles, row by row
+    err = np.linalg.norm(got[keep] - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert err.max() < 2e-6, float(err.max())
+    some = min(50, rows)                                     # (up to 16 rows go through the matvecs, which add in another order)
+    for first in {*range(0, rows - some, some), rows - some}:
+        backend.cross_kv_dev(dmem.ptr + 4 * first * width, some, width, [gain], biases, [kvw], xw, dk.ptr, dv.ptr)
+        part = np.concatenate([dk.read()[:some * xw].reshape(some, xw), dv.read()[:some * xw].reshape(some, xw)], axis=1)
+        assert np.array_equal(part, got[first:first + some], equal_nan=True), first
+    for d in (dmem, dk, dv):
+        d.free()
+
+
+@pytest.mark.parametrize("taps,tokens", [(1, 20), (1, 100), (3, 20), (3, 100)])
+def test_encoder_f32_channels_of_different_size(backend, pkg, synth, taps, tokens):
+    """LayerNorm gains of 2^-30 in some channels and 2^30 in the weights behind them: powers of two, so every product is the one of the even
+    stack and the output is the same bits."""
+    print("[gpu-case] encoder f32, channels of different size, taps=%d tokens=%d" % (taps, tokens), flush=True)
+    cfg = dict(synth.encoder_config(layers=2, width=128, heads=2, ffn=192, vocab=32, max_positions=128), causal=True, ffn_kernel=taps, operands_f32=True)
+    rng = np.random.default_rng(taps)
+    normal = lambda *shape: (0.02 * rng.standard_normal(shape)).astype(np.float32)
+    even = {"tok_table": normal(32, 128), "pos_table": normal(128, 128), "qkv": normal(2, 384, 128), "o": normal(2, 128, 128),
+            "up": normal(2, 192, 128 * taps), "down": normal(2, 128, 192 * taps), "norm_out_g": np.ones(128, np.float32), "norm_out_b": None}
+    for name in ("norm1", "norm2"):
+        even[name + "_g"], even[name + "_b"] = (1.0 + normal(2, 128)), None
+    uneven = {k: None if v is None else v.copy() for k, v in even.items()}
+    quiet = rng.random(128) < 0.5
+    for name, behind, each in (("norm1_g", "qkv", 1), ("norm2_g", "up", taps)):
+        uneven[name][:, quiet] *= np.float32(2.0 ** -30)
+        uneven[behind].reshape(2, -1, 128, each)[:, :, quiet] *= np.float32(2.0 ** 30)
+    ids = rng.integers(0, 32, size=tokens).astype(np.int32)
+    out = []
+    for w in (even, uneven):
+        enc = pkg.Encoder(backend, cfg, w)
+        dout = backend.alloc(tokens * 128)
+        enc.prefill(ids, 0, dout.ptr)
+        out.append(dout.read())
+        enc.destroy()
+        dout.free()
+    assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
