@@ -151,11 +151,9 @@ int mynah_hip_argmax_dev(void *state, const float *dev_logits, size_t vocab, siz
  * that registers attention is also given the codec (src/graph.c:2514-2518), which fails hard without these
  * (:2552-2555): with them MYNAH_METAL_CPU_CODEC is not needed.
  * conv1d: causal, dilated; weight [out, in, kernel]; bias may be NULL (conv1d_causal, src/graph.c:2010-2160); runs
- *   on the f16 matrix cores with f32 operands in two f16 pieces under power-of-two scales and f32 sums: closer to double precision than
- *   f32 multiply-adds where operands of a row and of a tile lie within 2^24 of each other; 22 bits of an operand count, of an input those down to 2^-37
- *   (2^-27 of the largest in a tile of smaller ones), of a weight down to 2^-50 of the largest of its output channel; infinite, NaN and operands from 2^24 on give what f32
- *   multiply-adds give, the sums that they enter one by one; kernel <= 16, (kernel - 1) * dilation <= 128.  The products of cross_kv_dev and of the f32 encoder
- *   keep their operands in full, in three bf16 pieces (below 2^-110 fewer than 24 bits: at most 2^-134 is lost).
+ *   on the bf16 matrix cores with f32 operands in three bf16 pieces and f32 sums (no less precise than f32 multiply-adds;
+ *   infinite, NaN and largest operands give what those give; below 2^-110 an operand keeps fewer than 24 bits, at most 2^-134 of it is
+ *   lost); kernel <= 16, (kernel - 1) * dilation <= 128.  The products of cross_kv_dev and of the f32 encoder are made the same way.
  * conv_transpose_dev: grouped, weight [in, out / groups, kernel], output trimmed to output_length; bit-identical to
  *   the reference's scalar loop (convt_channel, src/graph.c:2179-2198).
  * snake_dev: in place; rows below snake_channels get x + sin(a x)^2 / (a + 1e-9), the rest a leaky ReLU of slope 0.01

@@ -263,8 +263,7 @@ int cached_conv_blocks(State *st, const float *host, size_t out_ch, size_t in_ch
     CachedWeight cw;
     cw.n = out_ch;
     cw.k = in_ch * kernel;
-    // three pieces a value; behind them the rows' inverse scales, in room for the steps that the kernels request past the last
-    cw.bytes = tiles * blocks * kernel * 3072 + std::max<size_t>(kConvStepsAhead * 3072, tiles * 32 * sizeof(float));
+    cw.bytes = (tiles * blocks * kernel + kConvStepsAhead) * 3072;   // (the kernels request that many steps past the last)
     if (stage_weight(st, host, out_ch * in_ch * kernel, error, capacity) != 0) return -1;
     MYNAH_TRY(hipMalloc(&cw.data, cw.bytes));
     if (launch_conv_pack(st, st->pack_staging, static_cast<uint4 *>(cw.data), out_ch, in_ch, kernel, error, capacity) != 0) {

@@ -5,8 +5,8 @@
 //
 //   conv1d          out[o][t] = bias[o] + sum_i sum_k w[(o*in + i)*K + k] * in[i][t - (K-1-k)*dilation]   (conv1d_causal,
 //                   src/graph.c:2010-2160).  The reference builds an im2col matrix and calls sgemm; here the same GEMM
-//                   (M = out channels, N = length, inner = in channels x taps) runs on the f16 matrix cores, two pieces a
-//                   value (half_product.h: f32 operands, f32 accumulation, the accuracy of an f32 product) with the im2col
+//                   (M = out channels, N = length, inner = in channels x taps) runs on the bf16 matrix cores in three-piece
+//                   form (split_product.h: f32 operands, f32 accumulation, the accuracy of an f32 product) with the im2col
 //                   done by addressing: a workgroup stages the input rows of sixteen channels once, with a halo of
 //                   (K-1)*dilation positions, and every tap reads the same rows at its own offset.
 //   conv_transpose  grouped, trimmed to output_length (conv_transpose_causal / convt_channel, src/graph.c:2179-2231):
@@ -20,13 +20,28 @@
 #include <type_traits>
 #include <utility>
 
-#include "half_product.h"
+#include "split_product.h"
 
 using namespace mynah;
 
 namespace {
 
 typedef f32x16 floatx16;
+typedef unsigned short ushort8 __attribute__((ext_vector_type(8)));
+
+// A value at `bytes` behind an address that is the same for every lane: one instruction with the address in scalar registers, where
+// pointer arithmetic by lanes takes 64-bit addresses in vector registers.
+// (opaque: what stays the same from request to request is otherwise added up ahead of all loops, 64 bits a lane and request)
+template <class T>
+__device__ __forceinline__ T load_behind(const T *base, unsigned bytes) { return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes); }
+__device__ __forceinline__ unsigned opaque(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ int opaque_scalar(int v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
 
 constexpr int kConvMaxKernel = 16;
 constexpr int kConvMaxHalo = 128;     // (kernel - 1) * dilation
@@ -108,13 +123,9 @@ __device__ __forceinline__ void conv_emit(const ConvArgs &a, int m, size_t index
 }
 
 // The convolution's inner dimension goes in steps of one tap of sixteen input channels: one 16-deep matrix instruction per pair of
-// pieces.  Weights: taken apart once, when they are cached, in the order of the steps (ConvBlocks), so that a wavefront's two
-// pieces of a step are two requests of 1 KiB straight to its registers.  Inputs: a staged (position, eight channels) is 16 bytes
+// pieces.  Weights: taken apart once, when they are cached, in the order of the steps (ConvBlocks), so that a wavefront's three
+// pieces of a step are three requests of 1 KiB straight to its registers.  Inputs: a staged (position, eight channels) is 16 bytes
 // of LDS per piece, so a tap's operand is 512 consecutive bytes for 32 positions, whatever the tap's offset.
-// 108 channels x 16384, taps 3 / 7 / 11 in one launch, cycles of a workgroup (three to a CU, one of each): until its first product 5,000,
-// products 44,000 (its matrix instructions alone 28,000; without the weights' requests 31,500, without the LDS reads 38,000), residual
-// and stores 15,000, all workgroups at the same time.  As three bf16 pieces, with 64-bit addresses a lane and request that spilled, the
-// first product came after 35,000 and the launch took 55 us (now 41).
 struct ConvWeights {   // the weight pieces of one row tile, requested kAhead steps before they are multiplied
     static constexpr int kAhead = kConvStepsAhead;
     const uint4 *next;   // the same for every lane, like the inputs' rows below: an address is then a pair of scalar registers and the lane's offset, where
@@ -123,12 +134,12 @@ struct ConvWeights {   // the weight pieces of one row tile, requested kAhead st
     size_t skip;       // from the end of a block to the next one this wavefront multiplies
     int blocks;        // it multiplies
     int tap = 0;       // of the next request (a constant wherever the tap count is one)
-    uint4 ring[kAhead][2];
+    uint4 ring[kAhead][3];
     __device__ __forceinline__ void request(int slot, int taps) {
         bytes = opaque(bytes);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) ring[slot][q] = load_behind(next + 64 * q, bytes);
-        next += 128;
+        for (int q = 0; q < 3; ++q) ring[slot][q] = load_behind(next + 64 * q, bytes);
+        next += 192;
         if (++tap == taps) {
             tap = 0;
             if (--blocks > 0) next += skip;
@@ -138,15 +149,15 @@ struct ConvWeights {   // the weight pieces of one row tile, requested kAhead st
     template <int BY>
     __device__ __forceinline__ void turn() {
         if constexpr (BY != 0) {
-            uint4 was[kAhead][2];
+            uint4 was[kAhead][3];
 #pragma unroll
             for (int i = 0; i < kAhead; ++i)
 #pragma unroll
-                for (int q = 0; q < 2; ++q) was[i][q] = ring[i][q];
+                for (int q = 0; q < 3; ++q) was[i][q] = ring[i][q];
 #pragma unroll
             for (int i = 0; i < kAhead; ++i)
 #pragma unroll
-                for (int q = 0; q < 2; ++q) ring[i][q] = was[(i + BY) % kAhead][q];
+                for (int q = 0; q < 3; ++q) ring[i][q] = was[(i + BY) % kAhead][q];
         }
     }
     // (what runs past the last step is requested and not used: it is what follows the last block, and the cache pads its copies)
@@ -164,20 +175,20 @@ struct ConvWeights {   // the weight pieces of one row tile, requested kAhead st
 // SIMD, and a second set of fragment registers, read a step ahead, spilled: 1884 against 1754 us for a 64-frame decode.)
 template <int KF, int NT, int PIECE, bool AHEAD = false, class Stage>
 __device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, const int dilation, const int blocks, const Stage stage,
-                                              HalfSums (&acc)[NT]) {
-    half8_t x[AHEAD ? 2 : 1][NT][2];
+                                              floatx16 (&acc)[NT]) {
+    bf16x8 x[AHEAD ? 2 : 1][NT][3];
     const auto read = [&](int set, const uint4 *at) {
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) x[set][n][q] = __builtin_bit_cast(half8_t, at[q * PIECE + 32 * n]);
+            for (int q = 0; q < 3; ++q) x[set][n][q] = __builtin_bit_cast(bf16x8, at[q * PIECE + 32 * n]);
     };
     const auto multiply = [&](int set, int slot) {
-        half8_t fw[2];
+        bf16x8 fw[3];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) fw[q] = __builtin_bit_cast(half8_t, w.ring[slot][q]);
+        for (int q = 0; q < 3; ++q) fw[q] = __builtin_bit_cast(bf16x8, w.ring[slot][q]);
 #pragma unroll
-        for (int n = 0; n < NT; ++n) acc[n].multiply(fw, x[set][n]);
+        for (int n = 0; n < NT; ++n) acc[n] = split_multiply(fw, x[set][n], acc[n]);
     };
     if constexpr (KF != 0 && AHEAD) {
         // (the one-launch block: its few blocks run once, and code that is run once is waited for, instruction by instruction; so one copy of a
@@ -219,55 +230,44 @@ __device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, co
 #pragma unroll
                 for (int i = 0; i + 1 < ConvWeights::kAhead; ++i)
 #pragma unroll
-                    for (int q = 0; q < 2; ++q) w.ring[i][q] = w.ring[i + 1][q];
+                    for (int q = 0; q < 3; ++q) w.ring[i][q] = w.ring[i + 1][q];
                 w.request(ConvWeights::kAhead - 1, taps);
             }
         }
     }
 }
 
-// The rows' inverse scales, behind a packed weight's steps (see ConvBlocks).
-__device__ __forceinline__ const float *conv_inverses(const uint4 *data, size_t steps) { return reinterpret_cast<const float *>(data + steps * 192); }
-
-// What a sum of pieces that is no finite number stands for (half_product.h): the chain of f32 multiply-adds, from `s`, over the channels
-// (eight, then the taps, then the next eight) of every block that mine(block) names.  inside(tap): whether the tap's position lies in the
-// row; fetch(channel, tap, x): its eight inputs from that channel on.
-struct ConvRow {   // an output row's weights
-    const uint4 *pieces, *third;
-    float inverse;
-    __device__ __forceinline__ ConvRow(const uint4 *data, int tiles, int blocks, int taps, int row) {
-        const size_t tile = (size_t)blocks * taps, steps = tile * tiles;
-        pieces = data + (row >> 5) * tile * 128 + (row & 31);
-        third = data + steps * 128 + (row >> 5) * tile * 64 + (row & 31);
-        inverse = conv_inverses(data, steps)[row];
-    }
-};
+// What a sum of pieces that is no finite number stands for (split_product.h): the chain of f32 multiply-adds, from `s`, over the channels
+// (eight, then the taps, then the next eight) of every block that mine(block) names.  w: the output row's first piece of the first block and
+// tap; inside(tap): whether the tap's position lies in the row; fetch(channel, tap, x): its eight inputs from that channel on.
 template <class Mine, class Inside, class Fetch>
-__device__ __forceinline__ float conv_chain(const ConvRow w, const int channels, const int taps, const Mine mine, const Inside inside, const Fetch fetch, float s) {
+__device__ __forceinline__ float conv_chain(const uint4 *const w, const int channels, const int taps, const Mine mine, const Inside inside, const Fetch fetch, float s) {
 #pragma unroll 1
     for (int c = 0; c < channels && s == s; c += 8) {
         if (!mine(c >> 4)) continue;
 #pragma unroll 1
         for (int tap = 0; tap < taps; ++tap) {
             if (!inside(tap)) continue;
-            const size_t step = (size_t)((c >> 4) * taps + tap);
-            const uint4 *const at = w.pieces + step * 128 + ((c >> 3) & 1) * 32;
-            const ushort8_t h = __builtin_bit_cast(ushort8_t, at[0]), m = __builtin_bit_cast(ushort8_t, at[64]),
-                            l = __builtin_bit_cast(ushort8_t, w.third[step * 64 + ((c >> 3) & 1) * 32]);
+            const uint4 *const at = w + (size_t)((c >> 4) * taps + tap) * 192 + ((c >> 3) & 1) * 32;
+            const ushort8 h = __builtin_bit_cast(ushort8, at[0]), m = __builtin_bit_cast(ushort8, at[64]), l = __builtin_bit_cast(ushort8, at[128]);
             float x[8];
             fetch(c, tap, x);
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                if (c + e < channels) s = __builtin_fmaf(half_value(h[e], m[e], l[e], w.inverse), x[e], s);
+                if (c + e < channels) s = __builtin_fmaf(split_value(h[e], m[e], l[e]), x[e], s);
         }
     }
     return s;
+}
+// An output row's first piece of the first block and tap.
+__device__ __forceinline__ const uint4 *conv_row(const uint4 *data, const int blocks, const int taps, const int row) {
+    return data + (size_t)(row >> 5) * blocks * taps * 192 + (row & 31);
 }
 // ... of a convolution's own input rows, at output position t of row m.
 template <class Mine>
 __device__ __forceinline__ float conv_chain_rows(const ConvArgs &a, const int m, const int t, const Mine mine, const float s) {
     const int back = (a.kernel - 1) * a.dilation;
-    return conv_chain(ConvRow(a.weights, (a.out_ch + 31) / 32, (a.in_ch + 15) / 16, a.kernel, m), a.in_ch, a.kernel, mine, [&](int tap) { return t - back + tap * a.dilation >= 0; },
+    return conv_chain(conv_row(a.weights, (a.in_ch + 15) / 16, a.kernel, m), a.in_ch, a.kernel, mine, [&](int tap) { return t - back + tap * a.dilation >= 0; },
                       [&](int c, int tap, float (&x)[8]) {
 #pragma unroll
                           for (int e = 0; e < 8; ++e) x[e] = a.in[(size_t)min(c + e, a.in_ch - 1) * a.length + t - back + tap * a.dilation];
@@ -283,6 +283,12 @@ __device__ __forceinline__ void request_rows(float (&v)[8], const float *first, 
         row += channel + e + 1 < channels ? length : 0;
     }
 }
+__device__ __forceinline__ void store_pieces(const float (&v)[8], uint4 *at, int piece_stride) {
+    bf16x8 p[3];
+    split_eight(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]), p);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) at[q * piece_stride] = __builtin_bit_cast(uint4, p[q]);
+}
 // One (position, eight channels) on its way to LDS: eight requests, then the pieces of the eight values.
 struct ConvColumn {
     float v[8];
@@ -293,9 +299,11 @@ struct ConvColumn {
         channel = opaque_scalar(channel);
         request_rows(v, origin, channel, channels, length, bytes);
     }
-    __device__ __forceinline__ void store(uint4 *at, int piece_stride, bool inside, float scale, float &largest) const {
-        // (in front of the row: nothing, or no number where the row's first value is none -- then the sums are looked for as such)
-        half_eight(v, inside ? scale : 0.0f, largest, at[0], at[piece_stride]);
+    __device__ __forceinline__ void store(uint4 *at, int piece_stride, bool inside) const {
+        float u[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) u[e] = inside ? v[e] : 0.0f;   // (in front of the row)
+        store_pieces(u, at, piece_stride);
     }
 };
 
@@ -336,11 +344,11 @@ __device__ __forceinline__ void conv_split_rest(const ConvArgs *const args, floa
     }
 }
 
-// A tile's output rows: what their sums are multiplied by, and their biases; and the largest input that each wavefront has staged.
 constexpr int conv_pitch(int positions) { return positions + kConvMaxHalo; }
-struct ConvTileRows {
-    alignas(16) float inverse[64], bias[64];
-    float largest[4];
+// (channel-split tiles: 64 * parts positions hold the window)
+constexpr int conv_split_pitch(int nt, int parts) { return 64 * parts < conv_pitch(32 * nt) ? 64 * parts : conv_pitch(32 * nt); }
+struct ConvTileRows {   // of a tile's output rows
+    alignas(16) float bias[64];
     float alpha[32], inverse_alpha[32];   // (channel-split tiles) of the rows' half-snake, and 1 / (alpha + 1e-9)
 };
 
@@ -388,19 +396,15 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
         for (int x = 0; x < kColumns; ++x) column[x].request(a.in + first, 16 * block + 8 * group_of(x), a.in_ch, a.length, from[x]);
     };
     constexpr int kPitch = conv_pitch(TN);
-    uint4 *stage_now = lds, *stage_next = lds + 4 * kPitch;   // [piece][eight channels][position]
-    float scale = 1.0f, unscale = 1.0f, largest = 0.0f;
+    uint4 *stage_now = lds, *stage_next = lds + 6 * kPitch;   // [piece][eight channels][position]
     const auto publish = [&](uint4 *stage) {
 #pragma unroll
         for (int x = 0; x < kColumns; ++x)
-            if (place[x] >= 0) column[x].store(stage + group_of(x) * kPitch + place[x], 2 * kPitch, inside[x], scale, largest);
+            if (place[x] >= 0) column[x].store(stage + group_of(x) * kPitch + place[x], 2 * kPitch, inside[x]);
     };
     const int tile = min((int)blockIdx.y * WM + wm, w_arg.tiles - 1);
     // (requested here, beside the first block: at the end they would be a round trip in front of the stores)
-    if (tid < TM) {
-        s_rows.inverse[tid] = conv_inverses(w_arg.data, (size_t)w_arg.tiles * w_arg.blocks * a.kernel)[min(m0 + tid, 32 * w_arg.tiles - 1)];
-        s_rows.bias[tid] = a.bias != nullptr && m0 + tid < a.out_ch ? a.bias[m0 + tid] : 0.0f;
-    }
+    if (tid < TM) s_rows.bias[tid] = a.bias != nullptr && m0 + tid < a.out_ch ? a.bias[m0 + tid] : 0.0f;
     const auto stage = [&](int block) {
         __syncthreads();   // this block is stored, and nobody multiplies the one whose place the next one takes
         const uint4 *at = stage_now + half * kPitch + wn * 64 + col;
@@ -413,38 +417,25 @@ __device__ __forceinline__ void conv_tile(const ConvArgs &a_arg, const ConvBlock
         stage_next = t;
         return at;
     };
-    HalfSums sums[2];
-    for (bool once_more = false;; once_more = true) {
-        sums[0].clear();
-        sums[1].clear();
-        fetch(0);
-        ConvWeights w(w_arg.data + (size_t)tile * w_arg.blocks * a.kernel * 128, lane, 0, 1, a.kernel);
-        publish(stage_now);
-        fetch(min(1, w_arg.blocks - 1));
-        conv_products<KF, 2, 2 * kPitch>(w, a.kernel, a.dilation, w_arg.blocks, stage, sums);
-        largest = wave_max(largest);
-        if (lane == 0) s_rows.largest[wave] = largest;
-        __syncthreads();   // (and the epilogue's pieces of LDS overwrite the stages)
-        if (once_more) break;
-        const int e = __builtin_amdgcn_readfirstlane(half_rescale(fmaxf(fmaxf(s_rows.largest[0], s_rows.largest[1]), fmaxf(s_rows.largest[2], s_rows.largest[3]))));
-        if (__builtin_expect(e == 0, 1)) break;
-        scale = power_of_two(e);
-        unscale = power_of_two(-e);
-    }
+    // The sums start from the rows' biases, so a value is bias + products in the products' order.
+    floatx16 sums[2];
+    fetch(0);
+    ConvWeights w(w_arg.data + (size_t)tile * w_arg.blocks * a.kernel * 192, lane, 0, 1, a.kernel);
+    publish(stage_now);
+    fetch(min(1, w_arg.blocks - 1));
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sums[0][r] = s_rows.bias[wm * 32 + split_acc_row(r, lane)];
+    sums[1] = sums[0];
+    conv_products<KF, 2, 2 * kPitch>(w, a.kernel, a.dilation, w_arg.blocks, stage, sums);
+    __syncthreads();   // the epilogue's pieces of LDS overwrite the stages
     // What follows starts from the thread's number anew: what the compiler may take from above it forms ahead of the products and keeps in
     // scratch memory meanwhile (35 values of a thread, 27 MB a launch written before the first product and read behind the last).
     const int tid_after = (int)opaque(threadIdx.x), lane_after = tid_after & 63, wave_after = __builtin_amdgcn_readfirstlane(tid_after >> 6);
     const auto finish = [&](const int lane, const int wave) {
     const int wm = wave / WN, wn = wave % WN, half = lane >> 5, col = lane & 31;
-    floatx16 acc[2];
+    floatx16 (&acc)[2] = sums;
     floatx16 &acc0 = acc[0], &acc1 = acc[1];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = wm * 32 + split_acc_row(r, lane);
-        const float inverse = s_rows.inverse[row], bias = s_rows.bias[row];
-        acc0[r] = sums[0].sum(r) * unscale * inverse + bias;
-        acc1[r] = sums[1].sum(r) * unscale * inverse + bias;
-    }
     // The fused build's residual values, requested side by side; a residual may be the output itself -- every workgroup reads and
     // writes its own tile only.
     float res_first[FUSED ? 32 : 1], res_second[FUSED ? 32 : 1];
@@ -615,21 +606,19 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
     const int halo = (a.kernel - 1) * a.dilation;
     const int win = TN + halo;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    constexpr int kPitch = conv_pitch(TN);
-    uint4 *s_in = lds + wave * (4 * kPitch);   // [piece][eight channels][position] of this wavefront
+    constexpr int kPitch = conv_split_pitch(NT, PARTS);
+    uint4 *s_in = lds + wave * (6 * kPitch);   // [piece][eight channels][position] of this wavefront
     const int split = (int)blockIdx.x % a.splits, sharing = 4 * a.splits, rank = 4 * split + wave;   // this wavefront among those that share the channels
     const int m0 = blockIdx.y * TM, t0 = (int)blockIdx.x / a.splits * TN;
     const int half = lane >> 5, col = lane & 31;
 
-    HalfSums acc[NT];
+    floatx16 acc[NT];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) acc[n].clear();
-    float scale = 1.0f, unscale = 1.0f;   // (this wavefront's: its sums are its own)
+    for (int n = 0; n < NT; ++n) acc[n] = floatx16{0};
     // what the finished rows need (behind the products each request would be a round trip of its own)
     if (tid < TM) {
         const int m = m0 + tid;
         const float al = a.activate && m < a.snake_channels ? a.alpha[m] : 0.0f;
-        s_rows.inverse[tid] = conv_inverses(w_arg.data, (size_t)w_arg.tiles * w_arg.blocks * a.kernel)[m];
         s_rows.bias[tid] = a.bias != nullptr && m < a.out_ch ? a.bias[m] : 0.0f;
         s_rows.alpha[tid] = al;
         s_rows.inverse_alpha[tid] = 1.0f / (al + 1e-9f);
@@ -650,8 +639,7 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
                         column[g][x].request(a.in + first, 16 * (sharing * i + rank) + 8 * g, a.in_ch, a.length, from[x]);
                 }
         };
-        const size_t per_block = (size_t)a.kernel * 128;
-        float largest = 0.0f;
+        const size_t per_block = (size_t)a.kernel * 192;
         // (no workgroup barrier in the loop: a wavefront stages into its own part of LDS and reads nothing else, and its own
         // LDS accesses complete in the order it issued them -- the four wavefronts walk their channel blocks independently)
         const auto stage = [&](int i) {
@@ -661,24 +649,16 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
                 const int p = lane + 64 * x;
                 if (p < win) {
 #pragma unroll
-                    for (int g = 0; g < 2; ++g) column[g][x].store(s_in + g * kPitch + p, 2 * kPitch, t0 - halo + p >= 0, scale, largest);
+                    for (int g = 0; g < 2; ++g) column[g][x].store(s_in + g * kPitch + p, 2 * kPitch, t0 - halo + p >= 0);
                 }
             }
             fetch(min(i + 1, mine - 1));   // in flight during this block's products
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             return const_cast<const uint4 *>(s_in + half * kPitch + col);
         };
-        for (bool once_more = false;; once_more = true) {
-            fetch(0);
-            ConvWeights w(w_arg.data + ((size_t)blockIdx.y * w_arg.blocks + rank) * per_block, lane, (size_t)(sharing - 1) * per_block, mine, a.kernel);
-            conv_products<KF, NT, 2 * kPitch>(w, a.kernel, a.dilation, mine, stage, acc);
-            const int e = once_more ? 0 : half_rescale(wave_max(largest));
-            if (__builtin_expect(e == 0, 1)) break;
-            scale = power_of_two(e);
-            unscale = power_of_two(-e);
-#pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n].clear();
-        }
+        fetch(0);
+        ConvWeights w(w_arg.data + ((size_t)blockIdx.y * w_arg.blocks + rank) * per_block, lane, (size_t)(sharing - 1) * per_block, mine, a.kernel);
+        conv_products<KF, NT, 2 * kPitch>(w, a.kernel, a.dilation, mine, stage, acc);
     }
     // A thread finishes the tile's values at (row wave + 4 j, position lane): a store instruction then covers one row's 64
     // consecutive positions and whether the row exists is the same for all its lanes (in the accumulators' order an
@@ -703,7 +683,7 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s_part[(wave * 32 + 16 * n + r) * 64 + lane] = acc[n].sum(r) * unscale * s_rows.inverse[split_acc_row(r, lane)];
+        for (int r = 0; r < 16; ++r) s_part[(wave * 32 + 16 * n + r) * 64 + lane] = acc[n][r];
     __syncthreads();
     float sum[8], zero = 0.0f;
     const auto add_parts = [&]() {
@@ -878,19 +858,16 @@ struct ResMember {
     int kernel, dilation;
 };
 constexpr int kResMaxChannels = 128, kResMaxReach = 64;
-constexpr float kLargest = 0x1.ffp127f;   // no finite value of use in a sum is above it
 struct ResArgs {
     ResMember member[kConvBatchMax];
     int order[kConvBatchMax];
     int channels, length, snake_channels, blocks, tiles;
 };
 
-// The block's channels: (alpha, 1 / (alpha + 1e-9), a bound, -) of the inner rows' half-snake, (inverse scale, bias) of both convolutions;
-// and the largest input and inner value of each wavefront.
+// The block's channels: (alpha, 1 / (alpha + 1e-9), a bound, -) of the inner rows' half-snake, and the biases of both convolutions.
 struct ResRows {
     float4 pair[kResMaxChannels];
-    float2 in[kResMaxChannels], skip[kResMaxChannels];
-    float largest[8], largest_inner[8];
+    float in[kResMaxChannels], skip[kResMaxChannels];
 };
 
 template <int WM, int WN, int NT, bool SPLIT, int KF>
@@ -916,7 +893,6 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
         place[x] = p < win ? p : -1;
     }
     float column[kColumns][8];
-    float scale = 1.0f, unscale = 1.0f, largest = 0.0f;
     const auto fetch = [&](int block) {
 #pragma unroll
         for (int x = 0; x < kColumns; ++x) {
@@ -965,22 +941,22 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = first + place[x] < 0 ? 0.0f : v[e];   // in front of the rows
-            uint4 *const at = stage + group_of(x) * kPitch + place[x];
-            half_eight(v, scale, largest, at[0], at[2 * kPitch]);
+            store_pieces(v, stage + group_of(x) * kPitch + place[x], 2 * kPitch);
         }
     };
     // the inner rows' alphas, 1 / (alpha + 1e-9), and what a value is multiplied by to be told from those that need the long way: the
-    // library's sine, or (no finite number, or none to speak of) more than that.  (Requested here, looked at behind the first block's requests.)
+    // library's sine, or (no finite number, or none that three pieces add up to) more than that; an infinite 1 / (alpha + 1e-9) sends all that way.
+    // (Requested here, looked at behind the first block's requests.)
     constexpr int kRowsEach = (kResMaxChannels + T - 1) / T;
-    float2 row_pair[kRowsEach], row_in[kRowsEach], row_skip[kRowsEach];
+    float2 row_pair[kRowsEach];
+    float row_in[kRowsEach], row_skip[kRowsEach];
 #pragma unroll
     for (int i = 0; i < kRowsEach; ++i) {
         const int c = tid + T * i;
         const bool there = c < a.channels;   // (else zero: a wavefront without a row tile of its own multiplies the last one's weights)
-        const size_t steps = (size_t)a.tiles * a.blocks * KF;
         row_pair[i] = c < a.snake_channels ? m.snake_skip[c] : make_float2(0.0f, 0.0f);
-        row_in[i] = make_float2(there ? conv_inverses(m.w_in, steps)[c] : 0.0f, there && m.b_in != nullptr ? m.b_in[c] : 0.0f);
-        row_skip[i] = make_float2(there ? conv_inverses(m.w_skip, steps)[c] : 0.0f, there && m.b_skip != nullptr ? m.b_skip[c] : 0.0f);
+        row_in[i] = there && m.b_in != nullptr ? m.b_in[c] : 0.0f;
+        row_skip[i] = there && m.b_skip != nullptr ? m.b_skip[c] : 0.0f;
     }
     const auto keep_rows = [&]() {
 #pragma unroll
@@ -988,150 +964,120 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
             const int c = tid + T * i;
             if (c >= kResMaxChannels) break;
             const float2 pair = row_pair[i];
-            s_rows.pair[c] = make_float4(pair.x, pair.y, fmaxf(fabsf(pair.x), 1.01f * (kShortSineLimit / kLargest)), 0.0f);
+            const float bound = fmaxf(fabsf(pair.x), 1.01f * (kShortSineLimit / kSplitLimit));
+            s_rows.pair[c] = make_float4(pair.x, pair.y, split_finite(pair.y) ? bound : __builtin_inff(), 0.0f);
             s_rows.in[c] = row_in[i];
             s_rows.skip[c] = row_skip[i];
         }
     };
 
-    HalfSums sums[NT];
-    f32x16 acc[NT];   // (SPLIT: the blocks before, then) the finished sums
-    const auto start = [&]() {
+    f32x16 acc[NT], sum[SPLIT ? NT : 1];
+    const auto start = [&](const float (&bias)[kResMaxChannels]) {
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
-            sums[n].clear();
-            if constexpr (SPLIT) acc[n] = f32x16{0};
+            if constexpr (SPLIT) {
+                acc[n] = f32x16{0};
+                sum[n] = f32x16{0};
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[n][r] = bias[wm * 32 + split_acc_row(r, lane)];
+            }
         }
     };
-    // (SPLIT) a block's sums to those of the blocks before it
+    // (SPLIT) a block's sums to those of the blocks before it; in the end, the bias
     const auto add_block = [&]() {
         if constexpr (SPLIT) {
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[n][r] += sums[n].sum(r);
-                sums[n].clear();
+                sum[n] += acc[n];
+                acc[n] = f32x16{0};
             }
         }
     };
-    // the scales divided out, and the bias
-    const auto finish = [&](const float2 (&rows)[kResMaxChannels], float unscaled) {
+    const auto finish = [&](const float (&bias)[kResMaxChannels]) {
         add_block();
+        if constexpr (SPLIT) {
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
+            for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float2 row = rows[wm * 32 + split_acc_row(r, lane)];
-                acc[n][r] = (SPLIT ? acc[n][r] : sums[n].sum(r)) * unscaled * row.x + row.y;
-            }
+                for (int r = 0; r < 16; ++r) acc[n][r] = sum[n][r] + bias[wm * 32 + split_acc_row(r, lane)];
+        }
     };
-    const size_t w_at = (size_t)min(wm, a.tiles - 1) * a.blocks * KF * 128;
-    uint4 *stage_now = lds, *stage_next = lds + 4 * kPitch;
-    float inner_largest;
-    for (bool once_more = false;; once_more = true) {
-        fetch(0);
-        ConvWeights w(m.w_in + w_at, lane, 0, 1, KF);
-        start();
-        if (!once_more) keep_rows();
-        publish(0, stage_now);
-        fetch(min(1, a.blocks - 1));
-        conv_products<KF, NT, 2 * kPitch, true>(w, KF, m.dilation, a.blocks, [&](int block) {
-            if (block > 0) add_block();
-            __syncthreads();
-            const uint4 *at = stage_now + half * kPitch + wn * WP + col;
-            if (block + 1 < a.blocks) {
-                publish(block + 1, stage_next);
-                fetch(min(block + 2, a.blocks - 1));
-            }
-            uint4 *t = stage_now;
-            stage_now = stage_next;
-            stage_next = t;
-            return at;
-        }, sums);
-        finish(s_rows.in, unscale);
-        bool large = false;
-    #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float bound = s_rows.pair[wm * 32 + split_acc_row(r, lane)].z;
-    #pragma unroll
-            for (int n = 0; n < NT; ++n) large = large || !(fabsf(bound * acc[n][r]) < kShortSineLimit);
+    const size_t w_at = (size_t)min(wm, a.tiles - 1) * a.blocks * KF * 192;
+    uint4 *stage_now = lds, *stage_next = lds + 6 * kPitch;
+    fetch(0);
+    ConvWeights w(m.w_in + w_at, lane, 0, 1, KF);
+    keep_rows();
+    publish(0, stage_now);
+    fetch(min(1, a.blocks - 1));
+    __syncthreads();
+    start(s_rows.in);
+    conv_products<KF, NT, 2 * kPitch, true>(w, KF, m.dilation, a.blocks, [&](int block) {
+        if (block > 0) add_block();
+        __syncthreads();
+        const uint4 *at = stage_now + half * kPitch + wn * WP + col;
+        if (block + 1 < a.blocks) {
+            publish(block + 1, stage_next);
+            fetch(min(block + 2, a.blocks - 1));
         }
-        if (__builtin_expect(!__any(large), 1)) {
-    #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = wm * 32 + split_acc_row(r, lane);
-                const float4 pair = s_rows.pair[row];
-    #pragma unroll
-                for (int n = 0; n < NT; ++n) {
-                    const float v = acc[n][r];
-                    float y = v < 0.0f ? v * 0.01f : v;
-                    if (wm * 32 + 8 * (r >> 2) < a.snake_channels) {   // (else no lane's row of these registers is a snake row)
-                        const float sn = short_sine(pair.x * v);
-                        y = row < a.snake_channels ? v + sn * sn * pair.y : y;
-                    }
-                    acc[n][r] = y;
-                }
-            }
-        } else {
-    #pragma unroll 1
-            for (int r = 0; r < 16; ++r) {
-                const int row = wm * 32 + split_acc_row(r, lane);
-                const float4 pair = s_rows.pair[row];
-    #pragma unroll
-                for (int n = 0; n < NT; ++n) {
-                    const int t = t0 - (KF - 1) + wn * WP + 32 * n + col;
-                    float v = acc[n][r];
-                    if (row < a.channels && t >= 0 && t < a.length && !split_finite(v)) {
-                        const float bias = s_rows.in[row].y;
-                        v = conv_chain(ConvRow(m.w_in, a.tiles, a.blocks, KF, row), a.channels, KF, [](int) { return true; }, [&](int tap) { return t - halo + tap * m.dilation >= 0; },
-                                       [&](int c, int tap, float (&x)[8]) {
-    #pragma unroll 1
-                                           for (int e = 0; e < 8; ++e) {
-                                               const int channel = min(c + e, a.channels - 1);
-                                               const float2 in_pair = channel < a.snake_channels ? m.snake_in[channel] : make_float2(0.0f, 0.0f);
-                                               x[e] = half_snake(m.in[(size_t)channel * a.length + t - halo + tap * m.dilation], channel < a.snake_channels, in_pair.x, in_pair.y);
-                                           }
-                                       }, SPLIT ? 0.0f : bias);
-                        if (SPLIT) v = v + bias;
-                    }
-                    v = row < a.channels ? half_snake(v, row < a.snake_channels, pair.x, pair.y) : 0.0f;
-                    acc[n][r] = v;
-                }
-            }
-        }
-        // the largest values of the workgroup, for the scales under which they are taken apart
-        largest = wave_max(largest);
-        float largest_inner = 0.0f;
-    #pragma unroll
-        for (int n = 0; n < NT; ++n) {
-            const bool in_front = t0 - (KF - 1) + wn * WP + 32 * n + col < 0;
-    #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                if (in_front) acc[n][r] = 0.0f;
-                largest_inner = fmaxf(largest_inner, fabsf(acc[n][r]));
-            }
-        }
-        largest_inner = wave_max(largest_inner);
-        if (lane == 0) {
-            s_rows.largest[wave] = largest;
-            s_rows.largest_inner[wave] = largest_inner;
-        }
-        __syncthreads();   // (and the stages have been read)
-        const auto of_all = [&](const float (&each)[8]) {
-            float v = each[0];
-    #pragma unroll
-            for (int i = 1; i < WM * WN; ++i) v = fmaxf(v, each[i]);
-            return v;
-        };
-        const int e = once_more ? 0 : __builtin_amdgcn_readfirstlane(half_rescale(of_all(s_rows.largest)));
-        if (__builtin_expect(e == 0, 1)) {
-            inner_largest = of_all(s_rows.largest_inner);
-            break;
-        }
-        scale = power_of_two(e);
-        unscale = power_of_two(-e);
+        uint4 *t = stage_now;
+        stage_now = stage_next;
+        stage_next = t;
+        return at;
+    }, acc);
+    finish(s_rows.in);
+    bool large = false, kept = false;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const float bound = s_rows.pair[wm * 32 + split_acc_row(r, lane)].z;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) large = large || !(fabsf(bound * acc[n][r]) < kShortSineLimit);
     }
-
+    if (__builtin_expect(!__any(large), 1)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = wm * 32 + split_acc_row(r, lane);
+            const float4 pair = s_rows.pair[row];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const float v = acc[n][r];
+                float y = v < 0.0f ? v * 0.01f : v;
+                if (wm * 32 + 8 * (r >> 2) < a.snake_channels) {   // (else no lane's row of these registers is a snake row)
+                    const float sn = short_sine(pair.x * v);
+                    y = row < a.snake_channels ? v + sn * sn * pair.y : y;
+                }
+                acc[n][r] = y;
+            }
+        }
+    } else {
+#pragma unroll 1
+        for (int r = 0; r < 16; ++r) {
+            const int row = wm * 32 + split_acc_row(r, lane);
+            const float4 pair = s_rows.pair[row];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const int t = t0 - (KF - 1) + wn * WP + 32 * n + col;
+                float v = acc[n][r];
+                if (row < a.channels && t >= 0 && t < a.length && !split_finite(SPLIT ? sum[SPLIT ? n : 0][r] : v)) {
+                    const float bias = s_rows.in[row];
+                    v = conv_chain(conv_row(m.w_in, a.blocks, KF, row), a.channels, KF, [](int) { return true; }, [&](int tap) { return t - halo + tap * m.dilation >= 0; },
+                                   [&](int c, int tap, float (&x)[8]) {
+#pragma unroll 1
+                                       for (int e = 0; e < 8; ++e) {
+                                           const int channel = min(c + e, a.channels - 1);
+                                           const float2 in_pair = channel < a.snake_channels ? m.snake_in[channel] : make_float2(0.0f, 0.0f);
+                                           x[e] = half_snake(m.in[(size_t)channel * a.length + t - halo + tap * m.dilation], channel < a.snake_channels, in_pair.x, in_pair.y);
+                                       }
+                                   }, SPLIT ? 0.0f : bias);
+                    if (SPLIT) v = v + bias;
+                }
+                v = row < a.channels ? half_snake(v, row < a.snake_channels, pair.x, pair.y) : 0.0f;
+                kept = kept || !(fabsf(v) < kSplitLimit);
+                acc[n][r] = v;
+            }
+        }
+        kept = __any(kept);
+    }
     // the finished rows' residual (x itself), on its way during the rest: whole rows of consecutive positions, as it is stored
     const int rows = min(32, a.channels - wm * 32);
     constexpr int kRowsAtOnce = 64 / WP;                 // rows a wavefront stores with one instruction
@@ -1142,68 +1088,49 @@ __device__ __forceinline__ void res_block_tile(const ResArgs &a, const ResMember
     for (int i = 0; i < 32 / kRowsAtOnce; ++i) x[i] = m.in[at_out + (size_t)max(min(row0 + kRowsAtOnce * i, rows - 1), 0) * a.length];
     // the inner rows: activated, zero in front of the first position, in pieces to LDS where the second convolution reads them
     ConvWeights w2(m.w_skip + w_at, lane, 0, 1, KF);
-    const int inner_e = __builtin_amdgcn_readfirstlane(half_rescale(inner_largest));
-    scale = power_of_two(inner_e);
-    unscale = power_of_two(-inner_e);
-    const bool kept = !(__uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(inner_largest))) * scale < kHalfLimit);
+    __syncthreads();   // the stages have been read
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const int p = wn * WP + 32 * n + col;
+        const bool in_front = t0 - (KF - 1) + p < 0;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {   // rows 8 g + 4 half .. + 3 of the tile: half of the eight channels of one place
             const int block = wm * 2 + (g >> 1);
             if (block >= a.blocks) continue;
-            unsigned h[2], mid[2], low[2];
+            const float4 v = make_float4(acc[n][4 * g], acc[n][4 * g + 1], acc[n][4 * g + 2], acc[n][4 * g + 3]);
+            SplitFour s(in_front ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : v);
+            if (__builtin_expect(kept, 0) && !in_front) s.keep_bits(v);   // (the rows themselves are nowhere else)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                float rest[2];
-                half_pieces(acc[n][4 * g + 2 * i], acc[n][4 * g + 2 * i + 1], scale, h[i], mid[i], rest);
-                low[i] = half_third(mid[i], rest);
-            }
-            uint2 piece[3] = {make_uint2(h[0], h[1]), make_uint2(mid[0], mid[1]), make_uint2(low[0], low[1])};
-            if (__builtin_expect(kept, 0)) {   // (the rows themselves are nowhere else)
-                ushort4_t at[3];
-#pragma unroll
-                for (int q = 0; q < 3; ++q) at[q] = __builtin_bit_cast(ushort4_t, piece[q]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    unsigned short ph = at[0][i], pm = at[1][i], pl = at[2][i];
-                    half_keep_bits(acc[n][4 * g + i], scale, ph, pm, pl);
-                    at[0][i] = ph;
-                    at[1][i] = pm;
-                    at[2][i] = pl;
-                }
-#pragma unroll
-                for (int q = 0; q < 3; ++q) piece[q] = __builtin_bit_cast(uint2, at[q]);
-            }
-#pragma unroll
-            for (int q = 0; q < 3; ++q) reinterpret_cast<uint2 *>(&lds[(block * 6 + q * 2 + (g & 1)) * RN + p])[half] = piece[q];
+            for (int q = 0; q < 3; ++q) reinterpret_cast<uint2 *>(&lds[(block * 6 + q * 2 + (g & 1)) * RN + p])[half] = s.piece[q];
         }
     }
-    start();
+    start(s_rows.skip);
     __syncthreads();
     conv_products<KF, NT, 2 * RN, true>(w2, KF, 1, a.blocks, [&](int block) {
         if (block > 0) add_block();
         return const_cast<const uint4 *>(lds + (block * 6 + half) * RN + wn * WP + col);
-    }, sums);
-    finish(s_rows.skip, unscale);
-    if (__builtin_expect(!split_all_finite(acc), 0)) {
+    }, acc);
+    finish(s_rows.skip);
+    bool finite;
+    if constexpr (SPLIT) finite = split_all_finite(sum);
+    else finite = split_all_finite(acc);
+    if (__builtin_expect(!finite, 0)) {
 #pragma unroll 1
         for (int r = 0; r < 16; ++r) {
             const int row = wm * 32 + split_acc_row(r, lane);
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
                 const int p = wn * WP + 32 * n + col, t = t0 + p;
-                if (row >= a.channels || p >= TN || t >= a.length || split_finite(acc[n][r])) continue;
-                const float bias = s_rows.skip[row].y;
-                const float v = conv_chain(ConvRow(m.w_skip, a.tiles, a.blocks, KF, row), a.channels, KF, [](int) { return true; },
+                if (row >= a.channels || p >= TN || t >= a.length || split_finite(SPLIT ? sum[SPLIT ? n : 0][r] : acc[n][r])) continue;
+                const float bias = s_rows.skip[row];
+                const float v = conv_chain(conv_row(m.w_skip, a.blocks, KF, row), a.channels, KF, [](int) { return true; },
                                            [&](int tap) { return t - (KF - 1) + tap >= 0; },
                                            [&](int c, int tap, float (&x)[8]) {
                                                const uint4 *const at = lds + ((c >> 4) * 6 + ((c >> 3) & 1)) * RN + p + tap;
-                                               const ushort8_t xh = __builtin_bit_cast(ushort8_t, at[0]), xm = __builtin_bit_cast(ushort8_t, at[2 * RN]),
-                                                               xl = __builtin_bit_cast(ushort8_t, at[4 * RN]);
+                                               const ushort8 xh = __builtin_bit_cast(ushort8, at[0]), xm = __builtin_bit_cast(ushort8, at[2 * RN]),
+                                                             xl = __builtin_bit_cast(ushort8, at[4 * RN]);
 #pragma unroll
-                                               for (int e = 0; e < 8; ++e) x[e] = half_value(xh[e], xm[e], xl[e], unscale);
+                                               for (int e = 0; e < 8; ++e) x[e] = split_value(xh[e], xm[e], xl[e]);
                                            }, SPLIT ? 0.0f : bias);
                 acc[n][r] = SPLIT ? v + bias : v;
             }
@@ -1293,7 +1220,7 @@ int launch_res_block(State *st, ResArgs &a, int count, char *error, size_t capac
     constexpr int RN = 32 * NT * WN;
     int taps = 0;
     for (int i = 0; i < count; ++i) taps = a.member[i].kernel > taps ? a.member[i].kernel : taps;
-    size_t lds = (size_t)2 * 4 * (RN + kResMaxReach) * 16;                                   // two stages, or
+    size_t lds = (size_t)2 * 6 * (RN + kResMaxReach) * 16;                             // two stages, or
     const size_t inner = ((size_t)a.blocks * 6 * RN + 16) * 16;                        // the inner rows (a tap past the last place is read, not used), or
     const size_t tiles = (size_t)WM * WN * 32 * (32 * NT + 1) * sizeof(float);        // the finished tiles
     lds = inner > lds ? inner : lds;
@@ -1315,19 +1242,28 @@ __global__ void __launch_bounds__(256) k_conv_pack(const float *src, uint4 *dst,
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= count) return;
     const int lane = (int)(i & 63);
-    const size_t step = i >> 6, tile = step / ((size_t)blocks * kernel), steps = count >> 6;
+    const size_t step = i >> 6, tile = step / ((size_t)blocks * kernel);
     const int tap = (int)(step % (size_t)kernel), block = (int)(step / (size_t)kernel % (size_t)blocks);
     const size_t o = tile * 32 + (lane & 31);
     const int c0 = block * 16 + (lane >> 5) * 8;
-    const float scale = 1.0f / conv_inverses(dst, steps)[o];
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = o < (size_t)out_ch && c0 + e < in_ch ? src[(o * in_ch + c0 + e) * kernel + tap] : 0.0f;
-    uint4 piece[3];
-    half_keep_eight(v, scale, piece);   // (the kernels have no other copy of a weight)
-    dst[step * 128 + lane] = piece[0];
-    dst[step * 128 + 64 + lane] = piece[1];
-    dst[steps * 128 + step * 64 + lane] = piece[2];
+    bf16x8 p[3];
+    split_eight(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]), p);
+    ushort8 at[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) at[q] = __builtin_bit_cast(ushort8, p[q]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {   // (the kernels have no other copy of a weight)
+        unsigned short h = at[0][e], m = at[1][e], l = at[2][e];
+        split_keep_bits(v[e], h, m, l);
+        at[0][e] = h;
+        at[1][e] = m;
+        at[2][e] = l;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) dst[step * 192 + q * 64 + lane] = __builtin_bit_cast(uint4, at[q]);
 }
 
 struct ConvTransposeArgs {
@@ -1471,15 +1407,15 @@ __global__ void __launch_bounds__(256) k_rows_combine(const RowsCombineArgs a) {
 // LDS of a launch: two stages of one block of channels (the channel-split kernel: one per wavefront), or what the epilogue keeps there.
 template <int WM, int WN>
 constexpr size_t conv_lds() {
-    constexpr size_t stages = (size_t)2 * 4 * conv_pitch(64 * WN) * 16, epilogue = (4 * 32 * kTileStride + 4 * 64) * sizeof(float);
+    constexpr size_t stages = (size_t)2 * 6 * conv_pitch(64 * WN) * 16, epilogue = (4 * 32 * kTileStride + 4 * 64) * sizeof(float);
     return stages > epilogue ? stages : epilogue;
 }
-template <int NT>
+template <int NT, int PARTS>
 constexpr size_t conv_split_lds() {
-    constexpr size_t stages = (size_t)4 * 4 * conv_pitch(32 * NT) * 16, epilogue = 5 * 2048 * sizeof(float);
+    constexpr size_t stages = (size_t)4 * 6 * conv_split_pitch(NT, PARTS) * 16, epilogue = 5 * 2048 * sizeof(float);
     return stages > epilogue ? stages : epilogue;
 }
-constexpr int kConvMaxLds = 2 * 4 * (256 + kConvMaxHalo) * 16;   // the largest of them
+constexpr int kConvMaxLds = 2 * 6 * (256 + kConvMaxHalo) * 16;   // the largest of them
 
 template <int WM, int WN, int KF, bool FUSED>
 int launch_conv_f(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
@@ -1521,7 +1457,7 @@ int launch_conv_split_p(State *st, const ConvArgs &a, const ConvBlocks &weights,
         raised = true;
     }
     const dim3 grid((unsigned)((a.length + 32 * NT - 1) / (32 * NT) * a.splits), (unsigned)((a.out_ch + 31) / 32));
-    hipLaunchKernelGGL((k_conv1d_split<KF, NT, PARTS>), grid, dim3(256), conv_split_lds<NT>(), st->stream, a.in, a.out, weights.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel,
+    hipLaunchKernelGGL((k_conv1d_split<KF, NT, PARTS>), grid, dim3(256), (conv_split_lds<NT, PARTS>()), st->stream, a.in, a.out, weights.data, a.bias, a.in_ch, a.out_ch, a.length, a.kernel,
                        a.dilation, weights.tiles, a);
     return hip_check(hipGetLastError(), "conv1d launch", error, capacity);
 }
@@ -1582,7 +1518,7 @@ int launch_conv_batch(State *st, ConvBatchArgs &b, int count, char *error, size_
 
 template <int NT, int PARTS>
 int launch_conv_split_batch_p(State *st, ConvBatchArgs &b, int count, char *error, size_t capacity) {
-    constexpr size_t lds = conv_split_lds<NT>();
+    constexpr size_t lds = conv_split_lds<NT, PARTS>();
     static bool raised = false;
     if (!raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_split_batch<NT, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
@@ -1604,43 +1540,8 @@ int launch_conv_split_batch(State *st, ConvBatchArgs &b, int count, char *error,
 
 }  // namespace
 
-// A weight's rows get a scale each: the largest value under it lies in [2^13, 2^14), unless it is 2^20 times the row's usual size and
-// more -- then what is 2^20 times that lies there, and what does not fit above it is kept as its bits (half_product.h).  A workgroup a row, four
-// requests of a thread side by side (a wavefront a row and one request at a time: 39 us for 768 x 6912); rows past the last one get 1.
-__global__ void __launch_bounds__(256) k_half_row_scales(const float *src, float *inverses, int rows, size_t per_row) {
-    __shared__ float s4[4];
-    const int row = (int)blockIdx.x, tid = (int)threadIdx.x;
-    float sum = 0.0f, count = 0.0f, most = -127.0f;
-    if (row < rows)
-        for (size_t i0 = 0; i0 < per_row; i0 += 1024) {
-            float v[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = src[(size_t)row * per_row + min(i0 + 256 * k + tid, per_row - 1)];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int e = exponent_of(v[k]);
-                const bool counts = i0 + 256 * k + tid < per_row && v[k] != 0.0f && e != 128;   // (else nothing, or no finite number)
-                sum += counts ? (float)e : 0.0f;
-                count += counts ? 1.0f : 0.0f;
-                most = counts ? fmaxf(most, (float)e) : most;
-            }
-        }
-    sum = block_sum(sum, s4);
-    count = block_sum(count, s4);
-    most = block_max(most, s4);
-    const int top = count == 0.0f ? 13 : (int)fminf(most, floorf(sum / count) + 20.0f);
-    if (tid == 0) inverses[row] = power_of_two(max(top - 13, -126));
-}
-int mynah::launch_half_row_scales(State *st, const float *src, float *inverses, size_t rows, size_t padded_rows, size_t per_row, char *error, size_t capacity) {
-    hipLaunchKernelGGL(k_half_row_scales, dim3((unsigned)padded_rows), dim3(256), 0, st->stream, src, inverses, (int)rows, per_row);
-    return hip_check(hipGetLastError(), "weight scale launch", error, capacity);
-}
-
 int mynah::launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_ch, size_t in_ch, size_t kernel, char *error, size_t capacity) {
     const size_t blocks = (in_ch + 15) / 16, count = (out_ch + 31) / 32 * blocks * kernel * 64;
-    const size_t rows = (out_ch + 31) / 32 * 32;
-    float *const inverses = reinterpret_cast<float *>(dst + (count / 64) * 192);
-    if (launch_half_row_scales(st, src, inverses, out_ch, rows, in_ch * kernel, error, capacity) != 0) return -1;
     hipLaunchKernelGGL(k_conv_pack, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st->stream, src, dst, count, (int)out_ch, (int)in_ch, (int)kernel, (int)blocks);
     return hip_check(hipGetLastError(), "weight packing launch", error, capacity);
 }

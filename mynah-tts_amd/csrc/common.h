@@ -230,11 +230,9 @@ State *enter_state(void *opaque, bool enqueues = true);
 int cached_matrix(State *st, const float *host, size_t n, size_t k, int want_qtype, const CachedWeight **out,
                   char *error, size_t capacity);
 int cached_vector(State *st, const float *host, size_t n, const float **dev, char *error, size_t capacity);
-// A conv1d weight [out_ch, in_ch, kernel] in the form the convolution kernels multiply it (codec_ops.hip): three f16 pieces per value
-// under a scale for each output channel (half_product.h).  Per tile of 32 output channels, block of 16 input channels and tap (a step)
-// two runs of 64 uint4s, one per piece, lane l's being output channel l % 32, input channels 8 * (l / 32) .. + 7 of the block; zeros where
-// the tensor has no row or channel.  Behind all steps the third pieces, one run a step, which only sums that are no finite number need,
-// and behind those the output channels' inverse scales (floats, 32 * tiles).
+// A conv1d weight [out_ch, in_ch, kernel] in the form the convolution kernels multiply it (codec_ops.hip): three bf16 pieces per value
+// (split_product.h), per tile of 32 output channels, block of 16 input channels and tap three runs of 64 uint4s, one per piece, lane
+// l's being output channel l % 32, input channels 8 * (l / 32) .. + 7 of the block; zeros where the tensor has no row or channel.
 struct ConvBlocks {
     const uint4 *data = nullptr;
     int tiles = 0, blocks = 0;

@@ -52,7 +52,7 @@ int launch_sgemm(State *st, int ta, int tb, size_t m, size_t n, size_t k, float 
 // Many-row f32 products on the bf16 matrix cores (split_product.hip).  Weights packed by launch_split_pack (cached_split_weight);
 // n a multiple of 32, channels of 64; the rows may be read up to kSplitOverrun floats past their end.
 constexpr size_t kSplitOverrun = 256;
-constexpr int kConvStepsAhead = 3;   // steps of a packed convolution weight that are requested ahead of the one multiplied (4: 1250 us a 64-frame decode, 1227 with 3)
+constexpr int kConvStepsAhead = 3;   // steps (3 KiB) of a packed convolution weight that are requested ahead of the one multiplied
 constexpr size_t kSplitWeightOverrun = 64 * 1024;   // bytes behind a packed weight that may be requested (never used)
 constexpr size_t kSplitMaxLayers = 32;
 struct SplitLayers {
@@ -60,8 +60,6 @@ struct SplitLayers {
     const float *gain[kSplitMaxLayers], *bias[kSplitMaxLayers];   // bias entries may be null
 };
 int launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_ch, size_t in_ch, size_t kernel, char *error, size_t capacity);
-// One power of two a row, inverted, for its values to be taken apart under (half_product.h); 1 for rows there are not.
-int launch_half_row_scales(State *st, const float *src, float *inverses, size_t rows, size_t padded_rows, size_t per_row, char *error, size_t capacity);
 int launch_split_pack(State *st, const float *src, float4 *dst, size_t n, size_t channels, size_t taps, char *error, size_t capacity);
 int split_product_splits(const State *st, size_t rows, size_t channels, size_t n, size_t most);
 // part[z][rows][n] = split z's share of in[rows][channels] * W (taps == 3: causal convolution, two rows in front of `in` are zeros).

@@ -1,5 +1,5 @@
 """GPU parity of the codec operators (mynah_hip_conv1d / _conv_transpose_dev / _snake_dev) against the oracle, through the
-C ABI.  conv1d runs in two-piece form on the f16 matrix cores and adds in a different order than the CPU: 1e-5 normalised.  The transposed
+C ABI.  conv1d runs in three-piece form on the bf16 matrix cores and adds in a different order than the CPU: 1e-5 normalised.  The transposed
 conv adds in the reference's order: bit-exact.  snake: the device sine against libm's, 1e-6 normalised."""
 import numpy as np
 import pytest
@@ -567,26 +567,117 @@ def test_res_layer_extremes(pkg, backend, C, L, taps):
         d.free()
 
 
-def test_conv1d_input_sizes(backend):
-    """Inputs whose largest value lies on either side of the lines at which a tile is multiplied once more under a scale of its own (2^-10,
-    65520, 2^24), far from them, and rows of very different size side by side, in each kind of tile: f32's accuracy against float64."""
-    rng = np.random.default_rng(77)
-    for C, O, L, K, D in ((20, 70, 300, 7, 3), (27, 27, 500, 3, 1), (432, 64, 33, 3, 1), (216, 216, 320, 11, 1), (40, 48, 300, 5, 5)):
-        w = (rng.standard_normal((O, C, K)) / np.sqrt(C * K)).astype(np.float32)
-        w *= np.exp2(rng.integers(-60, 60, size=(O, 1, 1))).astype(np.float32)      # each output channel has a scale of its own
-        base = rng.uniform(-1, 1, size=(C, L)).astype(np.float32)
-        base[0, 0] = 1.0
-        for size in (2.0 ** -60, 2.0 ** -30, 2.0 ** -10 * (1 - 2.0 ** -20), 2.0 ** -10, 1.0, 65519.0, 65521.0, 2.0 ** 20, 2.0 ** 24 * (1 - 2.0 ** -20), 2.0 ** 24, 0.0):
-            _announce("conv1d input size %g, %d -> %d x %d, %d taps" % (size, C, O, L, K))
-            x = base * np.float32(size)
-            got = _run_conv1d(backend, x, w, np.zeros(O, np.float32), D).astype(np.float64)
-            want = np.zeros((O, L))
-            for k in range(K):
-                back = min((K - 1 - k) * D, L)
-                want[:, back:] += w[:, :, k].astype(np.float64) @ x[:, :L - back].astype(np.float64)
-            norm = np.linalg.norm(want, axis=1)
-            # every product's operands keep 22 bits, the sums f32's: 2^-22 a term and 2^-24 an addition of at most 150, of either sign
-            assert (np.linalg.norm(got - want, axis=1) <= 1e-6 * norm).all(), size
+# large tiles (two shapes), channels split over the wavefronts (both widths) and over workgroups, each with straight-line taps and any
+UNEVEN = [(20, 70, 300, 7, 3), (27, 27, 900, 3, 1), (27, 30, 90, 4, 2), (40, 48, 300, 5, 5), (216, 216, 320, 11, 1), (432, 64, 33, 3, 1), (432, 100, 130, 7, 3)]
+
+
+def _uneven_rows(rng, channels, length, sizes):
+    """Rows in stretches of 1 to 40 positions, each of one of the sizes."""
+    x = rng.uniform(-1, 1, size=(channels, length)).astype(np.float32)
+    size, t = np.empty(length, np.float32), 0
+    while t < length:
+        n = int(rng.integers(1, 41))
+        size[t:t + n] = rng.choice(sizes)
+        t += n
+    return x * size, size
+
+
+@pytest.mark.parametrize("C,O,L,K,D", UNEVEN)
+def test_conv1d_input_sizes(backend, C, O, L, K, D):
+    """Positions from 2^-40 to 2^24 beside each other in a tile, output channels from 2^-60 to 2^60, and input channels of 2^-20 under weights that
+    make up for it: f32's accuracy at every position."""
+    _announce("conv1d input sizes %d -> %d x %d, %d taps" % (C, O, L, K))
+    rng = np.random.default_rng(C + L)
+    x, size = _uneven_rows(rng, C, L, np.exp2([-40, -30, -24, -20, -12, -9, 0, 15, 17, 24]).astype(np.float32))
+    w = (rng.standard_normal((O, C, K)) / np.sqrt(C * K)).astype(np.float32)
+    quiet = np.exp2(-20 * rng.integers(0, 2, size=(C, 1))).astype(np.float32)
+    scale = np.exp2(rng.integers(-60, 60, size=(O, 1))).astype(np.float32)
+    got = _run_conv1d(backend, x * quiet, w / quiet.reshape(1, C, 1) * scale[:, :, None], None, D).astype(np.float64) / scale
+    want = np.zeros((O, L))
+    for k in range(K):
+        back = min((K - 1 - k) * D, L)
+        want[:, back:] += w[:, :, k].astype(np.float64) @ x[:, :L - back].astype(np.float64)
+    # operands in full; a term's products that are left out are 2^-26 of it in the mean, one of at most 900 additions in a row rounds 2^-25 of the running
+    # sum in the mean, all of either sign: some 30 * 2^-25 of the result
+    assert (np.linalg.norm(got - want, axis=0) <= 1e-6 * np.linalg.norm(want, axis=0)).all()
+
+
+@pytest.mark.parametrize("C,O,L,K,D", UNEVEN)
+def test_conv1d_neighbours_do_not_count(backend, C, O, L, K, D):
+    """A position's bits follow from the inputs it reads alone, whatever else its tile reads (nothing, ordinary values, 2^24, f32's largest, an
+    infinity, NaN), and a power of two in every input is one in every output."""
+    _announce("conv1d neighbours %d -> %d x %d, %d taps" % (C, O, L, K))
+    rng = np.random.default_rng(2 * C + L)
+    x, _ = _uneven_rows(rng, C, L, np.exp2([-30, -20, -13]).astype(np.float32))
+    w, b = (rng.standard_normal((O, C, K)) / np.sqrt(C * K)).astype(np.float32), np.zeros(O, np.float32)
+    loud = rng.choice(L, size=max(1, L // 60), replace=False)
+    free = np.ones(L, bool)
+    for t in loud:
+        for k in range(K):
+            if t + k * D < L:
+                free[t + k * D] = False
+    assert free.any()
+    want = _run_conv1d(backend, x, w, b, D)
+    for value in (0.0, 2.0 ** -9, 1.0, 65521.0, 2.0 ** 24, 3.4028235e38, np.inf, np.nan):
+        y = x.copy()
+        y[rng.integers(0, C, size=loud.size), loud] = value
+        assert np.array_equal(_run_conv1d(backend, y, w, b, D)[:, free].view(np.uint32), want[:, free].view(np.uint32)), value
+    for power in (-30, -9, 13, 40):
+        assert np.array_equal(_run_conv1d(backend, x * np.float32(2.0 ** power), w, b, D), want * np.float32(2.0 ** power)), power
+
+
+# every way in which a position is launched (test_res_layer_builds): tiles of all widths, shared channels, each one-launch block
+@pytest.mark.parametrize("C,L,taps", [(432, 40, (3, 7, 11)), (432, 300, (3, 7, 11)), (216, 320, (3, 7, 11)), (216, 1000, (3, 7)), (216, 4700, (3, 11)), (108, 1000, (3, 7, 11)),
+                                      (108, 6300, (11,)), (27, 1300, (3, 7, 11)), (27, 42000, (3, 7)), (54, 2000, (3, 7, 11)), (54, 8000, (3, 7, 11)), (54, 13000, (3, 7, 11)),
+                                      (64, 20700, (3, 7, 11))])
+def test_res_layer_uneven_rows(pkg, backend, C, L, taps):
+    """Rows with stretches and blocks of sixteen channels of 2^-24 to 2^17 beside each other and biases as small, so that tiles of every size
+    meet values on both sides of any line: all forms of the layer still give the operator sequence's bits."""
+    import importlib
+    codec = importlib.import_module(pkg.__name__ + ".codec")
+    _announce("residual layer uneven rows %d x %d taps %s" % (C, L, taps))
+    x, blocks = _res_layer_inputs(C, L, 500 + C, taps)
+    rng = np.random.default_rng(C + L)
+    x, _ = _uneven_rows(rng, C, L, np.exp2([-24, -13, -12, -11, -9, 0, 17]).astype(np.float32))
+    x *= np.repeat(np.exp2(-rng.integers(0, 14, size=(C + 15) // 16)), 16)[:C, None].astype(np.float32)
+    for branch in blocks:
+        for _, (_, b_in), _, (_, b_skip), _ in branch:
+            b_in *= np.float32(1e-4)
+            b_skip *= np.float32(1e-4)
+    n, b = C * L, len(taps)
+    din = backend.alloc(n).write(x)
+    bufs = [backend.alloc(n) for _ in range(2 + max(4, 3 * b))]
+    at = [d.ptr for d in bufs]
+    codec.res_layer(backend, blocks, din.ptr, at[0], C, L, *at[2:6])
+    want = bufs[0].read()
+    assert np.isfinite(want).all()
+    codec.res_layer_fused(backend, blocks, din.ptr, at[1], C, L, *at[2:5])
+    assert np.array_equal(want.view(np.uint32), bufs[1].read().view(np.uint32))
+    codec.res_layer_batched(backend, blocks, din.ptr, at[1], C, L, at[2:2 + b], at[2 + b:2 + 2 * b], at[2 + 2 * b:2 + 3 * b])
+    assert np.array_equal(want.view(np.uint32), bufs[1].read().view(np.uint32))
+    for d in bufs + [din]:
+        d.free()
+
+
+def test_conv_batch_members_uneven_rows(pkg, backend):
+    """One call alone and two to four side by side, whose tiles differ in width: the same bits where the second half of a tile is the larger one."""
+    _announce("conv1d_fused_batch members, uneven rows")
+    rng = np.random.default_rng(78)
+    for C, O, L in ((432, 432, 64), (432, 432, 256), (216, 216, 700), (40, 72, 210)):
+        x, _ = _uneven_rows(rng, C, L, np.exp2([-13.0]).astype(np.float32))
+        x[rng.integers(0, C, size=L // 32), np.arange(32, L + 32, 32)[:L // 32] % L] = 2.0 ** -9
+        ws = [(rng.standard_normal((O, C, k)) / np.sqrt(C * k)).astype(np.float32) for k in (3, 7, 11, 3)]
+        din, outs = backend.alloc(C * L).write(x), [backend.alloc(O * L) for _ in ws]
+        alone = []
+        for w in ws:
+            backend.conv1d(din.ptr, outs[0].ptr, C, O, L, w.shape[2], 1, w, None)
+            alone.append(outs[0].read().view(np.uint32))
+        for members in (2, 3, 4):
+            backend.conv1d_fused_batch([dict(din=din.ptr, dout=outs[i].ptr, kernel=ws[i].shape[2], dilation=1, weight=ws[i]) for i in range(members)], C, O, L)
+            for i in range(members):
+                assert np.array_equal(outs[i].read().view(np.uint32), alone[i]), (C, O, L, members, i)
+        for d in [din] + outs:
+            d.free()
 
 
 @pytest.mark.parametrize("stride,kernel", [(2, 4), (4, 8), (8, 16), (2, 2), (2, 3), (4, 5), (8, 11), (4, 9), (8, 5), (3, 6), (1, 2)])
