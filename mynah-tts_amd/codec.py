@@ -5,8 +5,8 @@ copy, snake, conv, snake, conv, residual add, then the branch added to the outpu
 three: a third) at the end.  `res_layer_fused` computes the same values, bit for bit, from a third of the launches: the element-wise operators
 travel in the epilogue of the convolution before them (mynah_hip_conv1d_fused), and only a branch's first activation is a
 pass of its own (snake_copy_dev).  `res_layer_batched` is the whole layer as one call (mynah_hip_res_layer_dev), the three branches
-side by side -- they do not depend on each other until their sum -- and a block of all branches in one launch up to 32 channels, and
-up to 64 for the middle range of lengths (three branches: 3393 to some 20500 positions).  Same values again, bit for bit.
+side by side -- they do not depend on each other until their sum -- and a block of all branches in one launch up to 32 channels,
+up to 64 from 4097 positions on (three branches), and up to 128 for some lengths of few branches.  Same values again, bit for bit.
 
 blocks[branch][block] = (alpha_in, (w_in, b_in), alpha_skip, (w_skip, b_skip), dilation); the branch's kernel size is the
 weights' last dimension.  Buffers are device allocations of channels * length floats.

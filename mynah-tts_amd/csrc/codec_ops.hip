@@ -192,7 +192,7 @@ __device__ __forceinline__ void conv_products(ConvWeights &w, const int taps, co
     };
     if constexpr (KF != 0 && AHEAD) {
         // (the one-launch block: its few blocks run once, and code that is run once is waited for, instruction by instruction; so one copy of a
-        // block's steps, the weights' registers turned back in place at its end -- three copies: 27 channels x 65536 144 us a layer, 140 with one; 54 x 32768 190, 186)
+        // block's steps, the weights' registers turned back in place at its end: as fast as three copies (54 channels x 13824 112.5 us a layer, 111.3 with one) in less code)
         for (int block = 0; block < blocks; ++block) {
             const uint4 *at = stage(block);
             read(0, at);
@@ -664,7 +664,7 @@ __device__ __forceinline__ void conv_split_tile(const ConvArgs &a_arg, const Con
     // consecutive positions and whether the row exists is the same for all its lanes (in the accumulators' order an
     // instruction covers halves of two rows, four apart).  e: where that value sits in a partial tile (element r of lane l).
     // Residuals are requested here, side by side, before the wavefronts meet, and the activation is straight-line code for all eight values: in
-    // a loop a value at a time, with the requests where they are used, the finish was 7,000 to 9,000 of 18,000 cycles (108 channels x 1280).
+    // a loop a value at a time, with the requests where they are used, the finish was 7,000 to 9,000 cycles (108 channels x 1280).
     const int pos = lane, t = t0 + pos;
     const bool t_ok = (NT > 1 || pos < 32) && t < a.length;
     float first[8], second[8];
@@ -1168,9 +1168,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_res_block(const ResArgs a) 
 // The order in which a launch's members start, `each` workgroups apiece.  Workgroups are dealt to the CUs in turn, so member p of the order
 // covers CUs p * each .. on, round and round: the order whose most loaded CU has the fewest taps, and of equal ones the one that starts the most
 // taps first (a long workgroup is not started last).  Taps 3 / 7 / 11, us a layer of three positions, most taps first / this order: 432
-// channels x 512 (112 workgroups each) 192 / 183, 216 x 3584 (112) 258 / 249, 216 x 4096 (128) 266 / 257; where nothing is gained it is the same
-// order, and another is slower: 108 x 12288 (192) 221 / 230, 432 x 320 (140) 144 / 151.  With one or two workgroups of each member for every CU, and
-// more members than two, the second one by its taps goes first: 216 x 3072 258 / 238, 108 x 5120 173 / 165, x 4096 128 / 124, x 16384 260 / 258.
+// channels x 512 (112 workgroups each) 240 / 225, 216 x 1024 (112) 140 / 129, 108 x 8192 (128) 237 / 216; where nothing is gained it is the same
+// order, and another is slower: 108 x 12288 (192) 318 / 325, 432 x 320 (140) 181 / 195.  With one or two workgroups of each member for every CU, and
+// more members than two, the second one by its taps goes first: 108 x 4096 (256) 154 / 136, 216 x 2560 (280) 265 / 260, x 4096 (448) 360 / 350.
 void order_members(const State *st, const int *taps, int count, long each, int *order) {
     int by_taps[kConvBatchMax], at[kConvBatchMax], best = INT_MAX;
     for (int i = 0; i < count; ++i) {
@@ -1550,10 +1550,11 @@ int mynah::launch_conv_pack(State *st, const float *src, uint4 *dst, size_t out_
 // wavefronts.  (Few output channels: the large tiles are one row of wavefronts, wider in time.)  The two add in different orders, so
 // the choice is the shape's alone, for single, batched and fused launches alike, and the line lies where a residual layer's
 // three members meet; one convolution alone would change over later.  us, small tiles / large:
-//   three members of taps 3, 7, 11, six launches:  216 channels x 3584 248 / 259, x 4096 274 / 272, x 4608 289 / 311, x 5120 334 / 327;
-//     160 x 4096 173 / 195, x 6144 232 / 246;  108 x 5120 141 / 157, x 6144 156 / 159, x 7168 180 / 165
-//   alone (as three bf16 pieces), 3 / 11 taps:  216 x 3072 18.7 33 / 26 54;  108 x 5120 12.2 19 / 17.8 29.5;  54 x 12000 9.9 (11.8 with 7 taps) / 13 17;
-//     64 -> 864 x 640 9.6 (13.4) / 13.3 17.8, x 1280 16.3 (19) / 14 17.5;  32 -> 864 x 5, 7 taps: 8.8 / 11.6, x 128 7.9 / 12
+//   three members of taps 3, 7, 11, six launches:  432 channels x 2048 600 / 601, x 2560 754 / 764, x 3072 (168 large tiles) 892 / 832;
+//     216 x 3584 340 / 346, x 4608 394 / 450, x 5120 (160) 446 / 458, x 6144 522 / 543;  160 x 4096 209 / 257, x 6144 302 / 343;
+//     108 x 5120 161 / 200, x 6144 200 / 202, x 7168 212 / 209, x 8192 231 / 217
+//   alone, 3 / 11 taps:  216 x 3072 14.0 27 / 21 44, x 4608 14.7 30 / 21 45;  108 x 5120 9.5 15.5 / 11.6 23;  54 x 12000 6.9 10.4 (8.4 with 7 taps) / 7.8 14;
+//     64 -> 864 x 640 6.8 (8.4) / 7.8 11, x 1280 10.5 (12.8) / 8.2 11.3;  32 -> 864 x 5, 7 taps: 5.2 / 6.6, x 128 5.1 / 6.7
 // A layer of at most 32 channels has two blocks at most and runs as one launch a block, in the large tiles' order.
 static bool conv_takes_split(const State *st, int in_channels, int out_channels, int length) {
     const long tiles = out_channels <= 32 ? (long)((length + 255) / 256) : (long)((out_channels + 63) / 64) * ((length + 127) / 128);
@@ -1565,8 +1566,8 @@ static bool conv_takes_split(const State *st, int in_channels, int out_channels,
 // weights of all channels through one CU (some 40 GB/s: 0.9 MB with 432 channels and eleven taps); so as many as bring a wavefront's
 // blocks of channels down while three members' workgroups are two to a CU at most.  The sums' order follows, so this is the shape's
 // alone, too.  k_conv_finish is 3.4 us of a launch, so a wavefront must be spared three blocks at least.  us a layer of three positions, taps 3 / 7 /
-// 11, unshared / shared by so many: 432 channels (27 blocks) x 40 121 / 72 by 7, x 128 125 / 89 by 4, x 320 167 / 141 by 2; 216 (14) x 320 88 / 79 by 4,
-// x 640 92 / 99 by 2, which spares two.
+// 11, unshared / shared by so many: 432 channels (27 blocks) x 40 131 / 79 by 7, x 128 145 / 102 by 4, x 320 219 / 181 by 2; 216 (14) x 320 101 / 90 by 4,
+// x 640 110 / 122 by 2, which spares two; 160 (10) x 160 76 / 73 by 3, x 320 79 / 80, x 640 79 / 95, which spares two as well.
 constexpr int kConvSharedTiles = 160;
 static int conv_splits(int in_channels, int out_channels, int length) {
     const long tiles = (long)((out_channels + 31) / 32) * ((length + 63) / 64), blocks = (in_channels + 15) / 16;
@@ -1811,16 +1812,16 @@ extern "C" int mynah_hip_rows_combine_dev(void *state, const float *const *dev_i
 
 // The one-launch build for a position of a layer, or none.  Which are there follows the order in which the layer's convolutions add
 // (conv_takes_split) and how many workgroups find a place at once: three to a CU with 32 positions to a wavefront (narrow), whose chain of
-// products is half as long, two with 64 (wide), one of 512 threads.  Narrow while all find a place; else wide while all of those do; else whichever
-// needs less time for its rounds.  Measured per layer of three positions, branches of 3 / 7 / 11 taps, us:
-//   27 channels: x 5120 47 narrow, 65 wide, 84 as two launches a position; x 28672 74, 84, 105; x 32768 (more than three to a CU) 98, 85, 111;
-//     x 40960 107, 89; x 43008 (more wide than two to a CU) 108, 129; x 65536 145, 150, 160
-//   54, split order: x 1024 57 narrow, 47 as two launches of split tiles; x 2560 66, 57; x 5120 70.5, 69; x 10240 86, 111
-//   54, large order: x 13824 92 narrow, 104 wide, 127 as two launches; x 16384 133, 113, 133; x 20480 141, 120, 154; x 22528 152, 164, 163; x 28672
-//     160, 179, 175; x 32768 193, 201, 202; x 40960 229, 200, 268
-//   108, large order, 3 and 11 taps: x 6144 173 narrow, 202; x 8192 186, 204; x 12288 (more than fit) 276, 240; three branches: x 6144 155, 160;
-//     x 7168 175, 165
-// (three branches of 65 to 128 channels are never in the large order and few enough)
+// products is half as long, two with 64 (wide), one of 512 threads.  Narrow while all find a place; else, up to 32 channels, wide while all of those do and
+// then narrow again, and up to 64 wide.  Measured per layer of three positions, branches of 3 / 7 / 11 taps (or those named), us:
+//   27 channels: x 5120 47 narrow, 70 wide, 101 as two launches a position; x 28672 73, 80, 123; x 32768 (more than three to a CU) 94, 97, 127;
+//     11 taps x 98304 120, 112; 3 and 11 x 49152 98, 94; x 43008 (more wide than two to a CU) 106, 128, 156; x 65536 151, 158, 216
+//   54, split order: x 1024 69 narrow, 50 as two launches of split tiles; x 2560 73, 63; x 4096 (192 tiles of 64 positions) 73, 68; x 4224 73, 79;
+//     x 8192 90, 100; x 10240 102, 113
+//   54, large order: x 13824 110 narrow, 111 wide, 154 as two launches; x 16384 142, 143, 157; x 20480 167, 151, 207; x 24576 180, 177, 239; x 28672
+//     216, 186, 249; x 32768 247, 234, 259; x 40960 297, 266, 334; 11 taps x 40960 154, 164, 201; 11 taps x 65536 240, 244, 234
+//   108, large order: 11 taps x 6144 146, 186 as two launches; x 12288 161, 190; x 16384 (more than one to a CU) 271, 203.  (Where no CU gets the
+//     member with the most taps twice, more than one to a CU is faster as well: 3 and 11 x 12288 202, 237; three branches x 6144 160, 203, but x 7168 223, 209.)
 enum ResBuild { RES_NONE, RES_32_NARROW, RES_32_WIDE, RES_64_SPLIT, RES_64_NARROW, RES_64_WIDE, RES_128 };
 static ResBuild res_build(const State *st, const mynah_hip_res_block *blocks, size_t branches, size_t stride, size_t channels, size_t length) {
     if (channels > (size_t)kResMaxChannels) return RES_NONE;
@@ -1836,8 +1837,8 @@ static ResBuild res_build(const State *st, const mynah_hip_res_block *blocks, si
     if (channels <= 32) return fit(128, 3) || !fit(256, 2) ? RES_32_NARROW : RES_32_WIDE;
     const bool split = conv_takes_split(st, (int)channels, (int)channels, (int)length);
     if (channels > 64) return !split && fit(64, 1) ? RES_128 : RES_NONE;
-    if (split) return 2 * (long)((length + 63) / 64) * (long)branches < 2 * (long)st->cu_count ? RES_NONE : RES_64_SPLIT;
-    return fit(64, 3) || (!fit(128, 2) && fit(64, 7)) ? RES_64_NARROW : RES_64_WIDE;
+    if (split) return 4 * (long)((length + 63) / 64) * (long)branches <= 3 * (long)st->cu_count ? RES_NONE : RES_64_SPLIT;
+    return fit(64, 3) ? RES_64_NARROW : RES_64_WIDE;
 }
 
 // One position (block) of every branch in one launch, where there is a build for it; *done tells.

@@ -951,7 +951,7 @@ extern "C" int mynah_hip_encoder_create(void *state, const mynah_hip_encoder_des
     if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, 0) != hipSuccess || lds <= 0) lds = 65536;
     e->max_lds = (size_t)lds;
     auto fail = [&](void) { mynah_hip_encoder_destroy(state, e); return -1; };
-    if (e->tpad_max > 1024 || attention_lds_bytes(e->tpad_max) + 10 * 1024 > e->max_lds) {   // 1024: a softmax lane keeps 32 float4 pieces of its row
+    if (e->tpad_max > 1024 || attention_lds_bytes(e->tpad_max) + 10 * 1024 > e->max_lds) {   // 1024: sixteen softmax lanes keep a row, sixteen float4 pieces each
         set_error(error, capacity, "encoder_create: max_positions beyond 1024, or more LDS per workgroup than this device has");
         return fail();
     }

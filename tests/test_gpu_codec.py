@@ -200,7 +200,7 @@ def test_res_layer_call(pkg, backend, orc, nerr, C, L):
 
 
 # (branches by their taps) each build of the one-launch block and the edges between it and its neighbours, on 256 CUs: at most 32 channels
-# narrow and wide; to 64 two launches / split order / wide in the large order / two launches; to 128 (fewer branches) split tiles / one launch
+# narrow and wide; to 64 two launches / split order / narrow and wide in the large order; to 128 (fewer branches) split tiles / one launch
 @pytest.mark.parametrize("C,L,taps", [(27, 20780, (3, 7, 11)), (27, 20786, (3, 7, 11)), (32, 30300, (3, 11)), (64, 3392, (3, 7, 11)), (64, 3393, (3, 7, 11)),
                                       (33, 4609, (3, 7, 11)), (50, 8193, (7,)), (50, 10300, (7,)), (54, 12160, (11, 3, 3, 7)), (54, 12161, (3, 7, 11)), (64, 20741, (3, 7, 11)),
                                       (54, 20800, (3, 7, 11)), (108, 6016, (11,)), (108, 6017, (11,)), (65, 6017, (3, 11)), (128, 6090, (7, 3)),
@@ -715,8 +715,8 @@ def test_conv_transpose_forms(backend, stride, kernel):
 
 
 # (branches of 3, 7 and 11 taps, 256 CUs) the last and the first length of each one-launch build: at most 32 channels narrow / wide / narrow again; to 64
-# two launches / one, the two orders, narrow / wide / narrow / wide; more channels: split and large tiles
-@pytest.mark.parametrize("C,L", [(27, 31152), (27, 31153), (27, 42558), (27, 42559), (40, 1), (50, 5440), (50, 5441), (54, 12160), (54, 12161), (54, 14790), (54, 14791), (64, 20768), (64, 20769),
+# two launches / one, the two orders, narrow / wide; more channels: split and large tiles
+@pytest.mark.parametrize("C,L", [(27, 31152), (27, 31153), (27, 42558), (27, 42559), (40, 1), (50, 4096), (50, 4097), (50, 5440), (50, 5441), (54, 12160), (54, 12161), (54, 14790), (54, 14791), (64, 20768), (64, 20769),
                                  (33, 34510), (33, 34511), (216, 4608), (216, 4609)])
 def test_res_layer_build_lines(pkg, backend, C, L):
     test_res_layer_builds(pkg, backend, C, L, (3, 7, 11))
