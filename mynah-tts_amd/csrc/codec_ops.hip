@@ -1225,7 +1225,7 @@ int launch_res_block(State *st, ResArgs &a, int count, char *error, size_t capac
     const size_t tiles = (size_t)WM * WN * 32 * (32 * NT + 1) * sizeof(float);        // the finished tiles
     lds = inner > lds ? inner : lds;
     lds = tiles > lds ? tiles : lds;
-    static bool raised = false;
+    static std::atomic<bool> raised{false};   // per instantiation; states on separate threads meet here
     if (!raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_res_block<WM, WN, NT, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, 112 * 1024));
         raised = true;
@@ -1420,7 +1420,7 @@ constexpr int kConvMaxLds = 2 * 6 * (256 + kConvMaxHalo) * 16;   // the largest 
 template <int WM, int WN, int KF, bool FUSED>
 int launch_conv_f(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
     constexpr int TM = 32 * WM, TN = 64 * WN;
-    static bool raised = false;   // per instantiation
+    static std::atomic<bool> raised{false};   // per instantiation; states on separate threads meet here
     if (!raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d<WM, WN, KF, FUSED>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
         raised = true;
@@ -1451,7 +1451,7 @@ inline int conv_split_parts(const ConvArgs &a, int tn) { return tn + (a.kernel -
 
 template <int KF, int NT, int PARTS>
 int launch_conv_split_p(State *st, const ConvArgs &a, const ConvBlocks &weights, char *error, size_t capacity) {
-    static bool raised = false;
+    static std::atomic<bool> raised{false};   // per instantiation; states on separate threads meet here
     if (!raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_split<KF, NT, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
         raised = true;
@@ -1504,7 +1504,7 @@ template <int WM, int WN>
 int launch_conv_batch(State *st, ConvBatchArgs &b, int count, char *error, size_t capacity) {
     constexpr int TM = 32 * WM, TN = 64 * WN;
     constexpr size_t lds = conv_lds<WM, WN>();
-    static bool raised = false;   // per instantiation
+    static std::atomic<bool> raised{false};   // per instantiation; states on separate threads meet here
     if (!raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_batch<WM, WN>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
         raised = true;
@@ -1519,7 +1519,7 @@ int launch_conv_batch(State *st, ConvBatchArgs &b, int count, char *error, size_
 template <int NT, int PARTS>
 int launch_conv_split_batch_p(State *st, ConvBatchArgs &b, int count, char *error, size_t capacity) {
     constexpr size_t lds = conv_split_lds<NT, PARTS>();
-    static bool raised = false;
+    static std::atomic<bool> raised{false};   // per instantiation; states on separate threads meet here
     if (!raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv1d_split_batch<NT, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize, kConvMaxLds));
         raised = true;

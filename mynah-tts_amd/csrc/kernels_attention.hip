@@ -623,7 +623,7 @@ int launch_attention(State *st, const AttnArgs &a, char *error, size_t capacity)
     const size_t hw = (size_t)a.head_width;
     const size_t lds = ((fast ? 0 : hw) + kAttnChunk + (size_t)kPosPerPass * hw + 2 * (size_t)a.max_chunks + kThreads) * sizeof(float);
     const dim3 grid((unsigned)a.max_chunks, (unsigned)a.heads, (unsigned)a.batch);
-    static bool raised[2] = {false, false};
+    static std::atomic<bool> raised[2] = {};   // states on separate threads meet here
     if (lds > 48 * 1024 && !fast && !raised[vec ? 1 : 0]) {
         const void *fn = vec ? reinterpret_cast<const void *>(&k_attention_any<true>) : reinterpret_cast<const void *>(&k_attention_any<false>);
         MYNAH_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));

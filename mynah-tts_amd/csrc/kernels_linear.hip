@@ -622,7 +622,7 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
     const int rows_per_wg = rows_per_wg_pass * passes;
     const int grid = (a.n + rows_per_wg - 1) / rows_per_wg;
     const size_t lds = (size_t)BT * a.k * (kQuantised<QT> ? 1 : 4);
-    static bool raised = false;   // per instantiation
+    static std::atomic<bool> raised{false};   // per instantiation; states on separate threads meet here
     if (lds > 48 * 1024 && !raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_linear<QT, BT, NVT, KFIX, SPEC>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));

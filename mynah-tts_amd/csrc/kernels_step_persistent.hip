@@ -802,7 +802,7 @@ static int launch_pt(State *st, const PersistArgs &a, int grid, char *error, siz
         set_error(error, capacity, "persistent step: the attention partials of these lengths exceed the workgroup's LDS");
         return -1;
     }
-    static bool raised = false;   // per instantiation
+    static std::atomic<bool> raised{false};   // per instantiation; states on separate threads meet here
     if (!raised) {
         MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_step_persistent<QT, BT>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       120 * 1024));

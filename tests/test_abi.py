@@ -127,3 +127,17 @@ def test_entry_points_refuse_a_null_state(pkg):
         rc = getattr(lib, name)(*args, err, C.c_size_t(len(err)))
         assert rc == -1, name
         assert b"state is null" in err.value, (name, err.value)
+
+
+def test_no_plain_variable_is_shared_between_states(pkg):
+    """Separate states may be used from separate threads: a variable of static duration in the host code is constant, atomic or made under the
+    language's own lock (a constant's initialiser); `static __device__` memory is the one exception, named in the header."""
+    root = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "mynah-tts_amd", "csrc")
+    shared = []
+    for name in sorted(os.listdir(root)):
+        for number, line in enumerate(open(os.path.join(root, name)), 1):
+            code = line.split("//")[0]
+            variable = re.match(r"\s*(?:static|thread_local)\s+(?!inline\b|constexpr\b|const\b|__device__|std::atomic\b)[\w:<>, *&]*?\w+\s*(?:\[\w*\]\s*)?(?:=|\{|;)", code)
+            if variable and "(" not in variable.group(0):
+                shared.append("%s:%d: %s" % (name, number, line.strip()))
+    assert not shared, shared
