@@ -184,7 +184,7 @@ def time_codec(pkg, backend, frames=64, runs=4, warmup=2):
     on synthetic weights: 32 -> 864 pre-conv, five stages of half-snake, grouped transposed conv (rates 8 8 4 2 2, channels
     halving) and a residual layer of 3 branches x 3 x (snake, conv k, snake, conv k) with k = 3 / 7 / 11 and dilations
     1 / 3 / 5, then snake, the 1-channel post-conv and the clip.  f32 operands and sums throughout; the convolutions run
-    on the f16 matrix cores in two-piece form.  Timed with HIP events on the backend's stream over whole decodes of `frames` raw frames."""
+    on the bf16 matrix cores in three-piece form.  Timed with HIP events on the backend's stream over whole decodes of `frames` raw frames."""
     rng = np.random.default_rng(11)
 
     def conv_w(out_ch, in_ch, k):
@@ -281,11 +281,11 @@ STAGES = [("self-attention", "k_step_attention<self>", "LayerNorm + int8 act-qua
 # then WRITE_SIZE), each scaled by what the same counter reads for the library's plain 256 MiB read+write kernel.  A figure
 # belongs to the kernel sources it was measured on: it is reported only while their hash is the one recorded here.
 MEASURED_TRAFFIC = {
-    1: {"kernel": "k_linear<k=768, residual>", "bytes": 937930, "profile": "profiles/decode_step_int8_hbm_counters.md",
-        "sources": ("kernels_linear.hip", "device_common.h", "kernels.h", "common.h"), "csrc_sha256": "f22a1da788ba942c"},
-    8: {"kernel": "k_step_attention<self>", "bytes": 54459630, "profile": "profiles/decode_step_int8_hbm_counters.md",
+    1: {"kernel": "k_linear<k=768, residual>", "bytes": 937921, "profile": "profiles/decode_step_int8_hbm_counters.md",
+        "sources": ("kernels_linear.hip", "device_common.h", "kernels.h", "common.h"), "csrc_sha256": "aefd793795f67117"},
+    8: {"kernel": "k_step_attention<self>", "bytes": 54459728, "profile": "profiles/decode_step_int8_hbm_counters.md",
         "sources": ("kernels_step_attention.hip", "step_attention_core.h", "step_items.h", "tagged_exchange.h", "device_common.h",
-                    "kernels.h", "common.h"), "csrc_sha256": "b5fa90ca42b21f2b"},
+                    "kernels.h", "common.h"), "csrc_sha256": "ce4c11fffeb0abb1"},
 }
 
 
@@ -502,10 +502,10 @@ def main():
                                        "frac": round(r["gbps"] / PEAK_GBPS, 4)} for r in local]}
     if codec is not None:
         result["codec"] = {"workload": "NanoCodec decode operator sequence, %d raw frames -> %d samples, f32: causal conv1d (kernels 3/7/11, "
-                                       "dilations 1/3/5, 864..27 channels) as products of two f16 pieces a value, grouped transposed conv, half-snake"
+                                       "dilations 1/3/5, 864..27 channels) as three-piece bf16 products, grouped transposed conv, half-snake"
                                        % (codec["frames"], codec["samples"]),
                            "ms": round(codec["ms"], 3), "flops": codec["flops"], "tflops": round(codec["tflops"], 2), "bound": "mfma",
-                           "peak_tflops": 833.3, "frac": round(codec["tflops"] / 833.3, 4),   # three f16 piece products per f32 one: a third of 2500
+                           "peak_tflops": 416.7, "frac": round(codec["tflops"] / 416.7, 4),   # six bf16 piece products per f32 one: a sixth of 2500
                            "form": "a residual layer as one call (mynah_hip_res_layer_dev): element-wise operators in the convolutions' epilogues, the three "
                                    "branches side by side, one launch per block and position at 27 and 54 channels and two elsewhere; samples bit-identical "
                                    "to the seam's operator sequence",

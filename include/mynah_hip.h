@@ -242,8 +242,8 @@ int mynah_hip_rows_combine_dev(void *state, const float *const *dev_inputs, size
  * and alphas are host pointers, cached like every weight.  dev_work: 3 * branches row sets [channels, length] of the caller's,
  * overwritten, none of them another one or dev_input (a single branch's first may be dev_input); dev_output may be dev_input or
  * any of them.  The values are those of the operator sequence above, bit for bit.  With 3, 7 or 11 taps in all of
- * a position's convolutions the position is one launch up to 32 channels, and above (to 128) where few enough workgroups take it; else
- * two, the branches side by side.  No counterpart in the reference's seam. */
+ * a position's convolutions the position is one launch up to 32 channels, up to 64 where the rows are long enough and up to 128 for some lengths of
+ * few branches; else two, the branches side by side.  No counterpart in the reference's seam. */
 typedef struct mynah_hip_res_block {
     const float *alpha_in, *weight_in, *bias_in;
     const float *alpha_skip, *weight_skip, *bias_skip;
