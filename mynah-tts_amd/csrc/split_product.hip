@@ -231,15 +231,18 @@ __global__ void __launch_bounds__(512) k_split_rows(const float *const a, const 
     split_store<MT, TAPS>(a + z * share, channels, m0, M, tile, share / 32, acc, part + (size_t)z * M * N + col0 + (lane & 31), N);
 }
 
-// The K and V halves of every layer's kv_net on that layer's normalised memory, one launch: blockIdx.y names the layer.
+// The K and V halves of every layer's kv_net on that layer's normalised memory, one launch.  The column tiles of all layers make one
+// list, of which an XCD takes every eighth: layer by layer the twelve of a 768-wide one would give XCDs 0 to 3 two each and the others one, and the
+// launch waits for the fullest.  Twelve layers, us a call, a grid of tiles a layer / one list: 100 rows 40.8 / 38.7, 180 58.3 / 47.5, 256 65.6 / 61.5.
+// (Two workgroups to a CU at 180 rows, some 23 ns a matrix instruction with its 6.4 vector instructions; a pass over the weight to have it in L2 first: 52.)
 __global__ void __launch_bounds__(512) k_split_cross_kv(const float *const normed, const SplitLayers weights, const int M, const int width, const int xw,
-                                                        const int mtiles, float *const k_out, float *const v_out) {
+                                                        const int mtiles, const int layers, float *const k_out, float *const v_out) {
     __shared__ SplitTile<2, 1, 2> lds;
     const int N = 2 * xw, ntiles = (N + 127) / 128;
     const SplitWork work((int)blockIdx.x, mtiles);
-    if (work.nz >= ntiles) return;
-    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3, layer = (int)blockIdx.y;
-    const int col0 = work.nz * 128 + wave * 32, m0 = work.m * 64;
+    if (work.nz >= ntiles * layers) return;
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3, layer = work.nz / ntiles;
+    const int col0 = (work.nz - layer * ntiles) * 128 + wave * 32, m0 = work.m * 64;
     f32x16 acc[2] = {f32x16{0}, f32x16{0}};
     const float4 *tile = weights.w[layer] + (size_t)(min(col0, N - 32) / 32) * (width / 32) * 256;
     split_tile<2, 1, 2>(normed + (size_t)layer * M * width, width, m0, M, tile, width / 32, lds, acc);
@@ -306,8 +309,8 @@ int launch_split_cross_kv(State *st, const float *memory, size_t rows, size_t wi
                           float *k_out, float *v_out, char *error, size_t capacity) {
     hipLaunchKernelGGL(k_layernorm_layers, dim3((unsigned)rows, (unsigned)count), dim3(256), 0, st->stream, memory, normed, layers, (int)rows, (int)width);
     const int mtiles = (int)((rows + 63) / 64), ntiles = (int)((2 * xw + 127) / 128);
-    hipLaunchKernelGGL(k_split_cross_kv, dim3((unsigned)((ntiles + 7) / 8 * 8 * mtiles), (unsigned)count), dim3(512), 0, st->stream, normed, layers, (int)rows,
-                       (int)width, (int)xw, mtiles, k_out, v_out);
+    hipLaunchKernelGGL(k_split_cross_kv, dim3((unsigned)((ntiles * (int)count + 7) / 8 * 8 * mtiles)), dim3(512), 0, st->stream, normed, layers,
+                       (int)rows, (int)width, (int)xw, mtiles, (int)count, k_out, v_out);
     return hip_check(hipGetLastError(), "cross K/V launch", error, capacity);
 }
 

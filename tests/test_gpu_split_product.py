@@ -32,6 +32,27 @@ def test_cross_kv_tiles(backend, pkg, orc, rows, width, xw, layers):
         d.free()
 
 
+@pytest.mark.parametrize("rows,xw,layers", [(5, 32, 9), (64, 224, 5), (130, 96, 3)])
+def test_cross_kv_layers_together(backend, pkg, rows, xw, layers):
+    """The layers' column tiles share one list: counts that no multiple of eight divides, a last tile that is not full, and every layer's
+    values are those of a call for that layer alone, bit for bit."""
+    print("[gpu-case] cross K/V together rows=%d xw=%d layers=%d" % (rows, xw, layers), flush=True)
+    rng, width = np.random.default_rng(rows + layers), 128
+    backend.set_quant(pkg.F32)
+    gains = [backend.keep((1.0 + 0.1 * rng.standard_normal(width)).astype(np.float32)) for _ in range(layers)]
+    kvw = [backend.keep(rng.standard_normal((2 * xw, width)).astype(np.float32)) for _ in range(layers)]
+    dmem = backend.alloc(rows * width).write(rng.standard_normal((rows, width)).astype(np.float32))
+    dk, dv = (backend.alloc(layers * rows * xw) for _ in range(2))
+    one_k, one_v = (backend.alloc(rows * xw) for _ in range(2))
+    backend.cross_kv_dev(dmem.ptr, rows, width, gains, None, kvw, xw, dk.ptr, dv.ptr)
+    k, v = dk.read().reshape(layers, -1), dv.read().reshape(layers, -1)
+    for l in range(layers):
+        backend.cross_kv_dev(dmem.ptr, rows, width, [gains[l]], None, [kvw[l]], xw, one_k.ptr, one_v.ptr)
+        assert np.array_equal(one_k.read(), k[l]) and np.array_equal(one_v.read(), v[l]), l
+    for d in (dmem, dk, dv, one_k, one_v):
+        d.free()
+
+
 @pytest.mark.parametrize("kernel", [1, 3])
 @pytest.mark.parametrize("tokens", [31, 32, 33, 64, 65, 97])
 def test_encoder_f32_tiles(backend, pkg, orc, synth, nerr, kernel, tokens):
