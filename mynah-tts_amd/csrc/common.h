@@ -24,10 +24,9 @@ constexpr size_t kQuantMaxK = 8192;  // QMAT_K_MAX, src/qmat.c:33
 constexpr int kWideRows = 16;        // the same for their wide-head form (one wavefront per row)
 constexpr int kAttnChunk = 64;       // cache positions handled by one workgroup of the stand-alone attention kernels
 constexpr int kStepUnitRows = 128;   // cache rows per attention unit (workgroup) of the fused resident step
-// Up to this many streams the resident step is laid out for latency: the output projection folds the attention
-// partials itself and attention workgroups request their weights before looking at the slot table.  Above it a
-// separate fold kernel runs once (every workgroup folding every stream would outweigh one extra launch) and
-// workgroups of units a stream does not have leave before requesting anything.
+// Up to this many streams the resident step is laid out for latency: attention workgroups find their work from their index and request
+// their weights before looking at the slot table, and the output projection folds their partials.  Above it they find it in a
+// work table written at the step's start; who folds is folds_behind's choice (decoder_step.hip).
 constexpr int kConsumerFoldMaxBatch = 2;
 constexpr int kMaxLanes = 3;         // groups of a batch's streams that step side by side, each on a stream of its own (a process has four
                                      // hardware queues here: with a fourth stream in use two of them share one, and chains that share a queue run one after the other)

@@ -61,15 +61,22 @@ struct mynah_hip_decoder {
     float *probe_sx = nullptr;
     int max_units = 0;
     bool fused_attention = false;
+    bool long_caches = false, long_memories = false;   // of the streams stepped now (caches_long; they choose among captured graphs)
+    bool no_tables = false;     // the work tables are not written for the launches now enqueued
+    bool beside = false;        // the step now enqueued runs in more than one lane
     // [with the end kernel or without it][stream count]: this lane's layer kernels as one chain of kernel nodes (without the
     // end kernel: the step whose final LayerNorm the output head's product does, mynah_hip_decoder_step_head)
     // forms: 0 the layers and the end kernel, 1 the layers alone, 2 the layers and the output head of HeadCall (its pointers are
     // part of the captured nodes: head_signature says whose they are, and the graph is captured again when they change)
-    hipGraphExec_t graphs[3][mynah::kMaxBatch + 1] = {};
-    int eager_steps[3][mynah::kMaxBatch + 1] = {};   // a stream count runs eagerly once before it is captured
-    unsigned long long head_signature[mynah::kMaxBatch + 1] = {};
+    struct Graphs {
+        hipGraphExec_t graphs[3][mynah::kMaxBatch + 1] = {};
+        int eager_steps[3][mynah::kMaxBatch + 1] = {};   // a stream count runs eagerly once before it is captured
+        unsigned long long head_signature[mynah::kMaxBatch + 1] = {};
+        hipGraphExec_t stage_graphs[MYNAH_HIP_STAGE_COUNT][mynah::kMaxBatch + 1] = {};   // single-stage graphs (measurement only)
+    };
+    Graphs forms[8];   // what a captured step depends on beside its stream count
+    Graphs &form() { return forms[(long_caches ? 1 : 0) + (long_memories ? 2 : 0) + (beside ? 4 : 0)]; }
     int head_recaptures = 0;
-    hipGraphExec_t stage_graphs[MYNAH_HIP_STAGE_COUNT][mynah::kMaxBatch + 1] = {};   // single-stage graphs (measurement only)
     int arith = 0;
     // Lanes: a batch above two streams is cut into groups that step side by side, each on a stream of its own with
     // workspaces, slot table and work tables of its own (a sibling decoder that shares this one's weights).  A stream's
@@ -86,6 +93,31 @@ struct mynah_hip_decoder {
 };
 
 namespace mynah {
+
+// Whether the product behind an attention launch folds the launch's partials (stream by stream, in its prologue: launch_linear_b), or
+// the launch folds its own.  A fold inside the launch is a hand-over between workgroups of 2 to 2.5 us at its end; behind it every
+// workgroup of the product repeats the fold for its stream, which grows with the streams and their lengths.  us a step, inside / behind: int8 three
+// streams (611, 1339 and 87 rows) 371 / 349, four 371 / 339, five (7000 rows together) 460 / 443; six of 1060 rows 376 / 353, of 4500 412 / 413,
+// of 6000 436 / 445; eight of 1000 371 / 359, of 3000 401 / 395, of 5000 418 / 415, of 7600 469 / 477.  Cross-attention memories are short: eight streams
+// 479 / 472 (f16 16 streams as two lanes 796 / 785 with both behind).  Either way gives the same bits (fold_partials' arithmetic).
+// What a prologue does not request at once (kFoldAhead + kFoldMore partials) it takes one after the other: longer streams fold inside.
+constexpr int kFoldBehindStreams = 5, kFoldBehindUnits = 40, kFoldBehindRows = (kFoldAhead + kFoldMore - 1) * kStepUnitRows;
+static bool folds_behind(const mynah_hip_decoder *d, int is_self, int batch) {
+    if (batch <= kConsumerFoldMaxBatch) return true;
+    if (batch > kBatchTile || d->width != 768 || !linear_folds_streams((int)d->width, (int)(is_self ? d->width : d->xw), (int)(is_self ? d->heads : d->cross_heads), d->max_units))
+        return false;
+    return !(is_self ? d->long_caches : d->long_memories);
+}
+// ... and what the caches of the streams stepped next (`rows` of them each) have to do with it.
+static bool caches_long(const int *rows, int batch, int most_units) {
+    int units = 0;
+    bool any = false;
+    for (int b = 0; b < batch; ++b) {
+        units += (rows[b] + kStepUnitRows - 1) / kStepUnitRows;
+        any = any || rows[b] > kFoldBehindRows;
+    }
+    return batch > kConsumerFoldMaxBatch && (any || (batch > kFoldBehindStreams && units > most_units));
+}
 
 // fold: 0 = plain input rows, 1 = fold of the self-attention partials, 2 = fold of the cross-attention partials
 static int enqueue_linear(State *st, const mynah_hip_decoder *d, const CachedWeight *w, const float *in, size_t in_stride,
@@ -122,6 +154,7 @@ static int enqueue_linear(State *st, const mynah_hip_decoder *d, const CachedWei
         a.ln_bias = ln_bias;
         a.epilogue = epilogue;
         a.arith = d->arith;
+        a.beside = d->beside ? 1 : 0;
         if (launch_linear(st, a, error, capacity) != 0) return -1;
     }
     return 0;
@@ -188,12 +221,13 @@ static int enqueue_step_attention(State *st, const mynah_hip_decoder *d, int is_
     a.scale = 1.0f / sqrtf((float)a.head_width);
     a.partial = d->partial;
     a.partial_ml = d->partial_ml;
-    a.records = batch > kConsumerFoldMaxBatch ? (is_self ? d->self_records : d->cross_records) : nullptr;
+    a.records = !folds_behind(d, is_self, batch) ? (is_self ? d->self_records : d->cross_records) : nullptr;
     a.fold_out = is_self ? d->attn : d->ctx;
     a.spin_limit = st->persist_spin_limit;
     a.abort_word = st->persist_abort_dev;
+    a.plain_table = batch > kConsumerFoldMaxBatch && folds_behind(d, is_self, batch) && !d->no_tables;
     if (launch_step_attention(st, a, error, capacity) != 0) return -1;
-    if (batch > kConsumerFoldMaxBatch && a.records == nullptr) return launch_step_fold(st, a, a.fold_out, error, capacity);
+    if (!folds_behind(d, is_self, batch) && a.records == nullptr) return launch_step_fold(st, a, a.fold_out, error, capacity);
     return 0;
 }
 
@@ -211,15 +245,14 @@ static int enqueue_layers(State *st, const mynah_hip_decoder *d, int batch, char
             const LayerWeights &lw = d->lw[l];
             if (on(MYNAH_HIP_STAGE_SELF_ATTENTION) &&
                 enqueue_step_attention(st, d, 1, l, batch, lw.qkv, lw.norm_self, lw.norm_self_b, error, capacity) != 0) return -1;
-            const bool consumer_fold = batch <= kConsumerFoldMaxBatch;
             const int slot0 = (int)l * 6;
             if (on(MYNAH_HIP_STAGE_SELF_OUT) &&
-                enqueue_linear(st, d, lw.o_self, d->attn, w, d->x, w, batch, nullptr, nullptr, EPI_RESIDUAL, error, capacity, consumer_fold ? 1 : 0, slot0 + 1) != 0) return -1;
+                enqueue_linear(st, d, lw.o_self, d->attn, w, d->x, w, batch, nullptr, nullptr, EPI_RESIDUAL, error, capacity, folds_behind(d, 1, batch) ? 1 : 0, slot0 + 1) != 0) return -1;
             if (d->xw != 0) {
                 if (on(MYNAH_HIP_STAGE_CROSS_ATTENTION) &&
                     enqueue_step_attention(st, d, 0, l, batch, lw.q_cross, lw.norm_cross, lw.norm_cross_b, error, capacity) != 0) return -1;
                 if (on(MYNAH_HIP_STAGE_CROSS_OUT) &&
-                    enqueue_linear(st, d, lw.o_cross, d->ctx, d->xw, d->x, w, batch, nullptr, nullptr, EPI_RESIDUAL, error, capacity, consumer_fold ? 2 : 0, slot0 + 3) != 0) return -1;
+                    enqueue_linear(st, d, lw.o_cross, d->ctx, d->xw, d->x, w, batch, nullptr, nullptr, EPI_RESIDUAL, error, capacity, folds_behind(d, 0, batch) ? 2 : 0, slot0 + 3) != 0) return -1;
             }
             if (on(MYNAH_HIP_STAGE_FFN_UP) &&
                 enqueue_linear(st, d, lw.up, d->x, w, d->hidden, d->ffn, batch, lw.norm_ff, lw.norm_ff_b, EPI_GELU, error, capacity, 0, slot0 + 4) != 0) return -1;
@@ -250,7 +283,8 @@ DecoderRows decoder_rows(mynah_hip_decoder *d) { return DecoderRows{d->x, d->dev
 
 StepItemTables decoder_item_tables(mynah_hip_decoder *d, int batch) {
     if (!d->fused_attention || batch <= kConsumerFoldMaxBatch) return StepItemTables{};
-    return step_item_tables(batch, (int)d->heads, (int)d->cross_heads, d->max_units, d->self_items, d->cross_items, d->self_records != nullptr,
+    return step_item_tables(batch, (int)d->heads, (int)d->cross_heads, d->max_units, d->self_items, d->cross_items,
+                            d->self_records != nullptr && !folds_behind(d, 1, batch), d->self_records != nullptr && !folds_behind(d, 0, batch),
                             d->self_slots, d->cross_slots);
 }
 
@@ -353,12 +387,14 @@ extern "C" void mynah_hip_decoder_destroy(void *opaque, mynah_hip_decoder *d) {
         mynah_hip_decoder_destroy(opaque, d->lanes[i]);
     }
     d->lanes.clear();
-    for (auto &form : d->graphs)
-        for (auto &g : form)
-            if (g != nullptr) (void)hipGraphExecDestroy(g);
-    for (auto &row : d->stage_graphs)
-        for (auto &g : row)
-            if (g != nullptr) (void)hipGraphExecDestroy(g);
+    for (auto &f : d->forms) {
+        for (auto &form : f.graphs)
+            for (auto &g : form)
+                if (g != nullptr) (void)hipGraphExecDestroy(g);
+        for (auto &row : f.stage_graphs)
+            for (auto &g : row)
+                if (g != nullptr) (void)hipGraphExecDestroy(g);
+    }
     float *bufs[] = {d->x, d->qkv, d->attn, d->qx, d->ctx, d->hidden, d->partial, d->partial_ml, d->seam_partial};
     for (float *p : bufs)
         if (p != nullptr) (void)hipFree(p);
@@ -680,6 +716,7 @@ static int run_lane(State *st, mynah_hip_decoder *lane, int count, hipStream_t s
     hipStream_t main_stream = st->stream;
     st->stream = stream;   // the launch wrappers enqueue on the state's stream
     int rc = 0;
+    mynah_hip_decoder::Graphs &captured = lane->form();
     const int form = head != nullptr ? 2 : with_end ? 0 : 1;
     const auto enqueue = [&]() {
         int r = enqueue_layers(st, lane, count, error, capacity, kAllStages, with_end);
@@ -690,21 +727,21 @@ static int run_lane(State *st, mynah_hip_decoder *lane, int count, hipStream_t s
         // another head, or other rows for its results, than this stream count's last step had: captured again, behind one
         // eager step (a weight seen for the first time is converted and uploaded there: no part of a capture)
         const unsigned long long signature = head_signature_of(st, *head, count);
-        if (lane->head_signature[count] != signature) {
-            if (lane->graphs[2][count] != nullptr) {
-                (void)hipGraphExecDestroy(lane->graphs[2][count]);
-                lane->graphs[2][count] = nullptr;
+        if (captured.head_signature[count] != signature) {
+            if (captured.graphs[2][count] != nullptr) {
+                (void)hipGraphExecDestroy(captured.graphs[2][count]);
+                captured.graphs[2][count] = nullptr;
             }
-            if (lane->head_signature[count] != 0) ++lane->head_recaptures;
-            lane->eager_steps[2][count] = 0;
-            lane->head_signature[count] = signature;
+            if (captured.head_signature[count] != 0) ++lane->head_recaptures;
+            captured.eager_steps[2][count] = 0;
+            captured.head_signature[count] = signature;
         }
     }
-    if (st->graph_mode == 0 || lane->eager_steps[form][count] == 0) {
-        lane->eager_steps[form][count] = 1;
+    if (st->graph_mode == 0 || captured.eager_steps[form][count] == 0) {
+        captured.eager_steps[form][count] = 1;
         rc = enqueue();
     } else {
-        hipGraphExec_t &exec = lane->graphs[form][count];
+        hipGraphExec_t &exec = captured.graphs[form][count];
         if (exec == nullptr) {
             hipGraph_t graph = nullptr;
             rc = hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "begin capture", error, capacity);
@@ -827,6 +864,9 @@ static int decoder_step(State *st, mynah_hip_decoder *d, const mynah_hip_decoder
         StepSlots ls = lanes == 1 ? s : lane_slots(s, plan, i);
         if (decoder_next_epochs(st, lane, 1, &ls.epoch, error, capacity) != 0) return -1;
         lane->last_slots = ls;
+        lane->long_caches = caches_long(ls.length, plan.count[i], kFoldBehindUnits);
+        lane->long_memories = caches_long(ls.memory_length, plan.count[i], kFoldBehindUnits);
+        lane->beside = lanes > 1;
         if (launch_step_begin(st, ls, lane->dev_slots, plan.count[i], d->width, d->position, lane->x, d->width, decoder_item_tables(lane, plan.count[i]), error,
                               capacity) != 0)
             return -1;
@@ -887,10 +927,12 @@ int mynah::rerun_last_step_without_waits(State *st, char *error, size_t capacity
     // another workgroup.  The arithmetic is the one of every other form, so these are the bits the step would have given.
     unsigned long long *const self_records = d->self_records, *const cross_records = d->cross_records;
     d->self_records = d->cross_records = nullptr;
+    d->no_tables = true;
     int rc = launch_step_begin(st, s, d->dev_slots, B, d->width, d->position, d->x, d->width, StepItemTables{}, error, capacity);
     if (rc == 0) rc = enqueue_layers(st, d, B, error, capacity);
     d->self_records = self_records;
     d->cross_records = cross_records;
+    d->no_tables = false;
     d->last_batch_slots = s;
     d->last_lanes = 1;
     d->last_batch = B;
@@ -957,7 +999,7 @@ extern "C" int mynah_hip_decoder_stage_enqueue(void *opaque, mynah_hip_decoder *
         set_error(error, capacity, "decoder has no cross-attention sublayer");
         return -1;
     }
-    hipGraphExec_t &exec = d->stage_graphs[stage][batch];
+    hipGraphExec_t &exec = d->form().stage_graphs[stage][batch];
     // The stage runs in one lane whatever the step does: when the last step ran in several, the owner's slot table holds one
     // lane's streams only and is rewritten for the whole batch first.  A fresh step counter, as every real step has one, for the
     // attention launches that fold their own partials: the workgroups that wait for tagged values then really wait.

@@ -38,11 +38,14 @@ struct LinearArgs {
     const StepSlots *ln_out_slots;
     float *aux_out;
     float *act_out;         // the input row as the prologue formed it (the fold of attention partials), before any LayerNorm
+    int beside;             // resident step: another lane's launches run beside this one
 };
 
 // True when the fused matvec kernel supports this shape/storage; otherwise use linear_generic.
 bool linear_fast_supported(int qtype, size_t n, size_t k);
 int launch_linear(State *st, const LinearArgs &args, char *error, size_t capacity);
+// Whether launch_linear takes such a product with the fold for more than two streams (rows one behind the other, residual epilogue).
+bool linear_folds_streams(int n, int k, int heads, int max_units);
 // Any shape, f32 weights: out[r,n] = in[r,k] W[n,k]^T + bias (rows may be large).
 int launch_gemm_f32(State *st, const float *in, float *out, size_t rows, size_t k, size_t n, const float *w,
                     const float *bias, char *error, size_t capacity);
@@ -118,7 +121,7 @@ struct StepItem {
 };
 struct StepAttnArgs {
     const StepSlots *slots;
-    const StepItem *items;    // batch > kConsumerFoldMaxBatch: one entry per workgroup of this launch's grid
+    const StepItem *items;    // batch > kConsumerFoldMaxBatch: one entry per workgroup of this launch's grid (read if records or plain_table say so)
     const float *x;           // [batch, width] residual stream
     int batch, width;
     const float *ln_gain, *ln_bias;
@@ -132,6 +135,7 @@ struct StepAttnArgs {
     float scale;
     float *partial;           // partial outputs [batch, heads, max_units, head_width]
     float *partial_ml;        // chunk maxima and sums [batch, heads, 2, max_units]
+    int plain_table;          // more than two streams, the partials left to the product behind (width 768): work from the table, no records
     // many streams, fold inside the launch: the partials as tagged records [batch, heads, max_units, kStepRecord] (non-null
     // selects this form), the folded rows [batch, heads * head_width], and the bound of the fold workgroups' wait
     unsigned long long *records;
@@ -152,10 +156,10 @@ struct StepItemTables {
     StepItem *self_items, *cross_items;
     int self_entries, cross_entries;
     int batch, heads, cross_heads;
-    int with_fold, self_budget, cross_budget;
+    int self_fold, cross_fold, self_budget, cross_budget;
 };
-StepItemTables step_item_tables(int batch, int heads, int cross_heads, int max_units, StepItem *self_items, StepItem *cross_items, bool with_fold,
-                                int self_slots, int cross_slots);
+StepItemTables step_item_tables(int batch, int heads, int cross_heads, int max_units, StepItem *self_items, StepItem *cross_items, bool self_fold,
+                                bool cross_fold, int self_slots, int cross_slots);
 inline unsigned step_item_workgroups(const StepItemTables &t) { return (unsigned)((t.self_entries + t.cross_entries + 255) / 256); }
 // Workgroups of the many-stream attention kernel for this weight storage and shape that the device holds at once.
 int step_attention_slots(int qtype, int width, int max_units, int is_self, bool with_fold);

@@ -51,7 +51,9 @@ __device__ __forceinline__ float *stream_out(const LinearArgs &a, int b) {
 // decided at run time).  SPEC_RESIDUAL: no LayerNorm, no bias, no probes, residual epilogue (the step's output and
 // FFN-down projections; the fold source stays a run-time choice).  SPEC_UP: LayerNorm, no fold, no bias, no probes,
 // GELU epilogue (the step's FFN-up projection).
-enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2 };
+// SPEC_SIDE (with one of the two, one stream to a workgroup): the launch takes several streams side by side, one to each row of the grid
+// (launch_linear_b); a build of its own, so that a lone stream does not wait for the arithmetic that finds a row.
+enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2, SPEC_SIDE = 4 };
 
 // More than two streams: one wavefront stages one stream (load_stream_row / finish_stream_row,
 // device_common.h) -- staging every stream's activations is what such a launch spends most of its time on, every workgroup
@@ -66,9 +68,10 @@ constexpr bool kWaveStaging = BT > kConsumerFoldMaxBatch;
 template <int BT>
 constexpr int kLinearThreads = kWaveStaging<BT> ? 64 * (BT > 4 ? BT : 4) : kThreads;
 
-// The builds whose leading arguments are repacked (see the kernel): specialised ones, one or two streams.
+// The builds whose leading arguments are repacked (see the kernel): specialised ones of one stream, which also take several streams side
+// by side, one to each row of the grid (launch_linear_b).
 template <int BT, int SPEC>
-constexpr bool kPackedLead = BT <= 2 && SPEC != SPEC_ANY;
+constexpr bool kPackedLead = BT == 1 && SPEC != SPEC_ANY;
 // The same for more streams, when the rows of a launch lie at a fixed stride (the step's workspaces do): the specialised
 // builds that stage a stream per wavefront take two row pointers and two strides instead of sixteen row pointers.
 template <int BT, int SPEC>
@@ -105,6 +108,12 @@ inline bool rows_strided(const LinearArgs &a, size_t *in_stride, size_t *out_str
     return true;
 }
 
+// Rows of a launch one behind the other: what the one-stream builds need to take several streams side by side.
+inline bool dense_rows(const LinearArgs &a) {
+    size_t si, so;
+    return a.batch < 2 || (rows_strided(a, &si, &so) && so == (size_t)a.n && (a.fold_partial != nullptr || si == (size_t)a.k));
+}
+
 // The small numbers such a launch needs before its first request, in the 64 bits of one pointer argument.
 struct LeadShape {
     int n, rows_per_wg, batch, folding, is_self, stream0, heads, max_units, head_width;
@@ -126,7 +135,7 @@ __device__ __forceinline__ LeadShape unpack_lead(const unsigned long long v) {
     return s;
 }
 
-template <int QT, int BT, int NVT, int KFIX, int SPEC>
+template <int QT, int BT, int NVT, int KFIX, int BUILD>
 __global__ void __launch_bounds__(kLinearThreads<BT>)
 k_linear(const float *const in0, const float *const fold_partial, const float *const fold_partial_ml, const StepSlots *const fold_slots,
          const void *const w, const float *const scales, float *const out0, const int n, const int batch, const LinearArgs a_arg,
@@ -136,6 +145,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
     // these are what the first requests are formed from.
     // (Only for one or two streams: with more, the rows of a.in and a.out are picked by a run-time index, and a structure that
     // has been written to is then kept in scratch memory -- the eight-stream matvecs took 20 us instead of 4.5.)
+    constexpr int SPEC = BUILD & ~SPEC_SIDE;
     static_assert(64 + sizeof(LinearArgs) > 0x100 + 4, "the warmed lines lie inside the kernel arguments");
     constexpr bool kStrided = kStridedLead<BT, SPEC>;
     WarmArguments warm{0u, 0u, 0u, 0u};
@@ -167,8 +177,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
     }
     if constexpr (kPackedLead<BT, SPEC>) {
         // Fourteen dwords of arguments -- the seven pointers -- are in registers at wavefront start; n, batch, the structure and
-        // rows_per_wg_arg come out of memory, a round trip that stood in front of the first request.  The specialised builds for
-        // one or two streams never use all seven pointers at once, so the launch (pack_lead) passes in the free places what
+        // rows_per_wg_arg come out of memory, a round trip that stood in front of the first request.  These builds never use all seven pointers at once, so the launch (pack_lead) passes in the free places what
         // the first requests are formed from: LayerNorm vectors where nothing is folded, the slot table's address in the place
         // of the unused input row where something is, and every small number in the place of the slot table's pointer.
         const LeadShape shape = unpack_lead(reinterpret_cast<unsigned long long>(fold_slots));
@@ -185,6 +194,12 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
             if (shape.folding) {
                 a.fold_partial = fold_partial; a.fold_partial_ml = fold_partial_ml; a.fold_slots = reinterpret_cast<const StepSlots *>(in0);
             }
+        }
+        if constexpr ((BUILD & SPEC_SIDE) != 0) {
+            const size_t y = blockIdx.y;   // the workgroup's stream (dense_rows)
+            a.out[0] += y * (size_t)a.n;
+            if (SPEC == SPEC_UP || !shape.folding) a.in[0] += y * (size_t)KFIX;
+            a.fold_stream0 += (int)y;
         }
     } else if constexpr (BT <= 2) {
         a.in[0] = in0; a.fold_partial = fold_partial; a.fold_partial_ml = fold_partial_ml; a.fold_slots = fold_slots;
@@ -606,8 +621,9 @@ static bool stream_groups_enabled() {
     return on;
 }
 
-template <int QT, int BT, int NVT, int KFIX, int SPEC>
+template <int QT, int BT, int NVT, int KFIX, int BUILD>
 int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity) {
+    constexpr int SPEC = BUILD & ~SPEC_SIDE;
     constexpr int epc = Chunk<QT>::n;
     const int chunks = a.k / epc;
     const int lg = lane_group_log2(chunks);
@@ -615,16 +631,22 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
     const int target_wgs = st->cu_count * 3;
     int passes = (a.n + rows_per_wg_pass * target_wgs - 1) / (rows_per_wg_pass * target_wgs);
     if (passes < 1) passes = 1;
-    // strided builds take more streams than their tile holds as groups of BT side by side (the grid's second dimension);
-    // with twice the rows per workgroup when the groups together would otherwise be more workgroups than the chip has CUs
-    const int groups = kStridedLead<BT, SPEC> ? (a.batch + BT - 1) / BT : 1;
-    if (groups > 1 && (long)((a.n + rows_per_wg_pass * passes - 1) / (rows_per_wg_pass * passes)) * groups > st->cu_count) passes *= 2;
+    // Builds that take more streams than their tile holds: groups of BT side by side (the grid's second dimension).
+    const int groups = kStridedLead<BT, SPEC> || (BUILD & SPEC_SIDE) != 0 ? (a.batch + BT - 1) / BT : 1;
+    const auto workgroups = [&]() { return (long)((a.n + rows_per_wg_pass * passes - 1) / (rows_per_wg_pass * passes)) * groups; };
+    // four streams to a group: twice the rows per workgroup when the groups together would otherwise be more workgroups than the chip has CUs
+    if (kStridedLead<BT, SPEC> && groups > 1 && workgroups() > st->cu_count) passes *= 2;
+    // One stream to a group, attention folded in the prologue: twice the rows from three workgroups a CU on, where folds repeated cost more than
+    // the second pass (eight f32 streams, 1536 / 768 workgroups: 614 / 582 us a step; f16, 768 / 384: 459 / 469), and from two a CU on beside
+    // another lane (sixteen f16 streams 818 / 785, f32 839 / 829).
+    if ((BUILD & SPEC_SIDE) != 0 && groups > 2 && a.fold_partial != nullptr)
+        while (workgroups() > (a.beside ? 2 : 3) * st->cu_count) passes *= 2;
     const int rows_per_wg = rows_per_wg_pass * passes;
     const int grid = (a.n + rows_per_wg - 1) / rows_per_wg;
     const size_t lds = (size_t)BT * a.k * (kQuantised<QT> ? 1 : 4);
     static std::atomic<bool> raised{false};   // per instantiation; states on separate threads meet here
     if (lds > 48 * 1024 && !raised) {
-        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_linear<QT, BT, NVT, KFIX, SPEC>),
+        MYNAH_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_linear<QT, BT, NVT, KFIX, BUILD>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));
         raised = true;
     }
@@ -636,13 +658,13 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
             return -1;
         }
         const StepSlots *const packed = reinterpret_cast<const StepSlots *>(pack_strided(shape));
-        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, SPEC>), dim3(grid, groups), dim3(kLinearThreads<BT>), lds, st->stream, a.in[0],
+        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, BUILD>), dim3(grid, groups), dim3(kLinearThreads<BT>), lds, st->stream, a.in[0],
                            SPEC == SPEC_UP ? a.ln_gain : nullptr, SPEC == SPEC_UP ? a.ln_bias : nullptr, packed, a.w, a.scales, a.out[0], a.n, a.batch, a,
                            rows_per_wg, lg);
     } else if constexpr (kPackedLead<BT, SPEC>) {
         // the launch's small numbers in the slot table pointer's place, and what the free pointer places carry (see the kernel)
         LeadShape shape{};
-        shape.n = a.n; shape.rows_per_wg = rows_per_wg; shape.batch = a.batch;
+        shape.n = a.n; shape.rows_per_wg = rows_per_wg; shape.batch = groups > 1 ? 1 : a.batch;
         const bool folding = SPEC == SPEC_RESIDUAL && a.fold_partial != nullptr;
         if (folding) {
             shape.folding = 1; shape.is_self = a.fold_is_self; shape.stream0 = a.fold_stream0; shape.heads = a.fold_heads;
@@ -656,10 +678,10 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
         const float *lead0 = a.in[0], *lead1 = nullptr, *lead2 = nullptr;
         if (SPEC == SPEC_UP) { lead1 = a.ln_gain; lead2 = a.ln_bias; }
         else if (folding) { lead0 = reinterpret_cast<const float *>(a.fold_slots); lead1 = a.fold_partial; lead2 = a.fold_partial_ml; }
-        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, SPEC>), dim3(grid), dim3(kLinearThreads<BT>), lds, st->stream, lead0, lead1, lead2, packed,
+        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, BUILD>), dim3(grid, groups), dim3(kLinearThreads<BT>), lds, st->stream, lead0, lead1, lead2, packed,
                            a.w, a.scales, a.out[0], a.n, a.batch, a, rows_per_wg, lg);
     } else {
-        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, SPEC>), dim3(grid), dim3(kLinearThreads<BT>), lds, st->stream, a.in[0], a.fold_partial,
+        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, BUILD>), dim3(grid), dim3(kLinearThreads<BT>), lds, st->stream, a.in[0], a.fold_partial,
                            a.fold_partial_ml, a.fold_slots, a.w, a.scales, a.out[0], a.n, a.batch, a, rows_per_wg, lg);
     }
     return hip_check(hipGetLastError(), "linear launch", error, capacity);
@@ -667,8 +689,22 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
 
 template <int QT, int NVT, int KFIX, int SPEC>
 int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity) {
-    if (a.batch <= 1) return launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
-    if (a.batch == 2) return launch_linear_t<QT, 2, NVT, KFIX, SPEC>(st, a, error, capacity);
+    if constexpr (SPEC != SPEC_ANY) {
+        // Streams side by side in ONE launch of the one-stream build: a workgroup stages one stream's row, and folds one stream's attention, whatever
+        // else is stepped, for a weight that is read once a stream (from L2 after the first).  us a step, as tiles / side by side: output projections
+        // with the fold, int8 two streams (600 and 900 rows) 360 / 326; FFN up two streams 326 / 318 (three int8 360 / 363, four f32 491 / 510: not from three on);
+        // FFN down two streams 318 / 314, three int4 382 / 368, f16 422 / 407, four int8 371 / 370.
+        if (a.batch <= 1) return launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
+        const int most = a.fold_partial != nullptr ? kBatchTile : SPEC == SPEC_UP || KFIX == 768 ? 2 : 4;
+        if (a.batch <= most && dense_rows(a)) return launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE>(st, a, error, capacity);
+        if (a.batch <= 2) {   // (launch_linear_q sends such launches to the general build; this is the backstop)
+            set_error(error, capacity, "linear: rows do not lie one behind the other");
+            return -1;
+        }
+    } else {
+        if (a.batch <= 1) return launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
+        if (a.batch == 2) return launch_linear_t<QT, 2, NVT, KFIX, SPEC>(st, a, error, capacity);
+    }
     if (a.batch <= 4) return launch_linear_t<QT, 4, NVT, KFIX, SPEC>(st, a, error, capacity);
     // five to eight streams, rows at a fixed stride, residual epilogue (the output projections and the
     // FFN-down product): two groups of four in one launch -- what a workgroup stages, every stream of its tile, halves, and a
@@ -685,15 +721,15 @@ int launch_linear_q(State *st, const LinearArgs &a, char *error, size_t capacity
     // what the arguments rule out decides the build (see SPEC above)
     const bool plain = a.bias == nullptr && a.probe_qx == nullptr && a.probe_sx == nullptr && a.probe_acc == nullptr &&
                        a.ln_out == nullptr && a.ln_out_slots == nullptr && a.aux_out == nullptr && a.act_out == nullptr;
-    // (the specialised builds for one or two streams take their small numbers packed into one argument: when one of them
+    // (the specialised builds of one stream take their small numbers packed into one argument: when one of them
     // does not fit its bit field the launch takes the general build, with the same arithmetic)
     LeadShape fit{};
     fit.n = a.n; fit.batch = a.batch; fit.rows_per_wg = 2048;   // above what launch_linear_t chooses for any n that fits (256 rows per 196,608 of n)
     if (a.fold_partial != nullptr) {
         fit.is_self = a.fold_is_self; fit.stream0 = a.fold_stream0; fit.heads = a.fold_heads; fit.max_units = a.fold_max_units; fit.head_width = a.fold_head_width;
     }
-    bool packs = lead_fits(fit);
-    if (a.batch > 2) {   // more streams: the specialised builds take rows at a fixed stride
+    bool packs = lead_fits(fit) && (a.batch > 2 || dense_rows(a));
+    if (a.batch > 2 && a.fold_partial == nullptr) {   // more streams: the specialised builds take rows at a fixed stride
         StridedShape strided{};
         strided.n = a.n; strided.batch = a.batch; strided.rows_per_wg = 2048;
         packs = rows_strided(a, &strided.in_stride, &strided.out_stride) && strided_fits(strided);
@@ -721,14 +757,21 @@ bool linear_fast_supported(int qtype, size_t n, size_t k) {
     return qtype == MYNAH_HIP_F32 || qtype == MYNAH_HIP_F16 || qtype == MYNAH_HIP_INT8 || qtype == MYNAH_HIP_INT4;
 }
 
+bool linear_folds_streams(int n, int k, int heads, int max_units) {
+    LeadShape fit{};
+    fit.n = n; fit.rows_per_wg = 2048; fit.batch = 1; fit.folding = 1; fit.heads = heads; fit.max_units = max_units;
+    return k == 768 && lead_fits(fit);
+}
+
 int launch_linear(State *st, const LinearArgs &a, char *error, size_t capacity) {
     if (a.batch < 1 || a.batch > kBatchTile) {
         set_error(error, capacity, "linear: batch tile out of range");
         return -1;
     }
-    if (a.fold_partial != nullptr && (a.batch > kConsumerFoldMaxBatch || a.k != a.fold_heads * a.fold_head_width || a.fold_slots == nullptr ||
+    if (a.fold_partial != nullptr && ((a.batch > kConsumerFoldMaxBatch && !(dense_rows(a) && linear_folds_streams(a.n, a.k, a.fold_heads, a.fold_max_units) &&
+                                                                             a.epilogue == EPI_RESIDUAL)) || a.k != a.fold_heads * a.fold_head_width || a.fold_slots == nullptr ||
                                       a.fold_partial_ml == nullptr)) {
-        set_error(error, capacity, "linear: the fold source takes at most two streams and rows of heads x head width");
+        set_error(error, capacity, "linear: more than two streams to fold for, or rows that are not heads x head width");
         return -1;
     }
     if (!linear_fast_supported(a.qtype, (size_t)a.n, (size_t)a.k)) {

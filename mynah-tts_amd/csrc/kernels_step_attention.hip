@@ -186,7 +186,7 @@ k_step_attention(const StepSlots *const slots_arg, const float *const x_arg, con
     }
     const bool role_qk = is_self && unit == 0;
     const bool role_v = is_self && unit == 1;
-    const int chunk = (PACKED == 1 ? item_group : CP) * (is_self ? unit - 2 : unit);   // first cache chunk of this workgroup (chunk roles only)
+    const int chunk = (PACKED != 0 ? item_group : CP) * (is_self ? unit - 2 : unit);   // first cache chunk of this workgroup (chunk roles only)
     const int pidx = is_self ? chunk + 1 : chunk;         // partial slot of that chunk (slot 0 of self-attention = the new row)
 
     const int chunks = a.width / kEpc;
@@ -256,7 +256,7 @@ k_step_attention(const StepSlots *const slots_arg, const float *const x_arg, con
     // ---- many streams, cache chunks: the whole of this role here, ahead of the new row's roles.  Kept apart from the code
     // below so that nothing of those roles (their second weight bank, parked in registers) is alive while this one runs:
     // the chunk loop then fits the registers that one chunk needs.
-    if constexpr (PACKED == 1) {
+    if constexpr (PACKED != 0) {
         if (!new_row) {
             static_assert(CP == 1, "the chunk loop keeps one chunk's rows in registers");
             const bool have_rows = count[0] > 0;   // an empty memory has none (its pointers may be null): read the activation buffer
@@ -274,13 +274,20 @@ k_step_attention(const StepSlots *const slots_arg, const float *const x_arg, con
             if constexpr (PF != kPrefetchLatency) load_activations<1, NVT>(pro, act, whole_workgroup(), xr, gv, bv);
             finish_activations<QT, 1, NVT>(pro, whole_workgroup(), xr, gv, bv, smem, s_sx, s_scratch);
             const size_t sh = (size_t)b * a.heads + head;
-            u64 *const rec0 = a.records + sh * a.max_units * kStepRecord;   // the partials leave as tagged records (see the fold role)
+            // the partials leave as tagged records (see the fold role), or as plain rows for the next product to fold
+            u64 *const rec0 = PACKED == 1 ? a.records + sh * a.max_units * kStepRecord : nullptr;
             const unsigned tag = (item_epoch << 8) | (unsigned)(a.layer + 1);
+            float *const plain_o = a.partial + (sh * a.max_units + pidx) * kHw, *const plain_m = a.partial_ml + sh * 2 * a.max_units + pidx;
             project_rows<QT, PF>(a, pre, PF, 0, kHw, head, lg, chunks, smem, s_sx[0], s_proj);
             __syncthreads();
             if (!have_rows) {   // empty memory (cross only): the context stays zero (src/graph.c:3242)
-                if (tid < kHw) put(rec0 + (size_t)pidx * kStepRecord + tid, tag, 0.0f);
-                if (tid == 0) put_ml(rec0 + (size_t)pidx * kStepRecord, tag, 0.0f, 1.0f);
+                if constexpr (PACKED == 1) {
+                    if (tid < kHw) put(rec0 + (size_t)pidx * kStepRecord + tid, tag, 0.0f);
+                    if (tid == 0) put_ml(rec0 + (size_t)pidx * kStepRecord, tag, 0.0f, 1.0f);
+                } else {
+                    if (tid < kHw) plain_o[tid] = 0.0f;
+                    if (tid == 0) { plain_m[0] = 0.0f; plain_m[a.max_units] = 1.0f; }
+                }
                 return;
             }
             const float4 qv = *reinterpret_cast<const float4 *>(s_proj + 4 * j);
@@ -289,6 +296,11 @@ k_step_attention(const StepSlots *const slots_arg, const float *const x_arg, con
                     float4 o;
                     float M, L;
                     merge_chunk(tid, s_red[0], s_wave_ml[0], o, M, L);
+                    if constexpr (PACKED != 1) {
+                        *reinterpret_cast<float4 *>(plain_o + (size_t)cc * kHw + 4 * tid) = o;
+                        if (tid == 0) { plain_m[cc] = M; plain_m[cc + a.max_units] = L; }
+                        return;
+                    }
                     u64 *rec = rec0 + (size_t)(pidx + cc) * kStepRecord;
                     put(rec + 4 * tid, tag, o.x); put(rec + 4 * tid + 1, tag, o.y); put(rec + 4 * tid + 2, tag, o.z); put(rec + 4 * tid + 3, tag, o.w);
                     if (tid == 0) put_ml(rec, tag, M, L);
@@ -439,7 +451,7 @@ k_step_attention(const StepSlots *const slots_arg, const float *const x_arg, con
         return;
     }
 
-    if constexpr (PACKED == 1) return;   // the chunk role of the many-stream build is complete further up
+    if constexpr (PACKED != 0) return;   // the chunk role of the many-stream build is complete further up
 
     // ---- cache chunk: this head's q, then the chunk's scores
     project_rows<QT, PF>(a, pre, PF, 0, kHw, head, lg, chunks, smem, s_sx[0], s_proj);
@@ -494,7 +506,8 @@ using StepAttnKernel = void (*)(const StepSlots *, const float *, const void *, 
 // streams (work found from the workgroup index; it also serves more streams when the launch cannot fold its own partials),
 // else the many-stream build (work table, partials as tagged records, fold inside the launch).
 template <int QT>
-StepAttnKernel kernel_for(int width, bool is_self, bool latency) {
+StepAttnKernel kernel_for(int width, bool is_self, bool latency, bool plain = false) {
+    if (plain) return is_self ? k_step_attention<QT, 1, kPrefetchLatency, 768, 1, 2> : k_step_attention<QT, 1, kPrefetchLatency, 768, 0, 2>;
     if (width == 768) {
         // the fixed-shape build needs few enough registers (154 for int8) to hold three workgroups per CU with four-pass banks
         if (is_self && latency) return k_step_attention<QT, 1, kPrefetchLatency, 768, 1, 0>;
@@ -524,11 +537,10 @@ template <int QT>
 int launch_t(State *st, const StepAttnArgs &a, char *error, size_t capacity) {
     const int chunks = a.width / Chunk<QT>::n;
     const int lg = lane_group_log2(chunks);
-    const bool packed_grid = a.records != nullptr;
-    const int grid = step_attention_grid(a.heads, a.batch, a.max_units, a.is_self, packed_grid);
+    const bool packed = a.records != nullptr || a.plain_table != 0;
+    const int grid = step_attention_grid(a.heads, a.batch, a.max_units, a.is_self, packed);
     const int per_xcd = grid / 8;
-    const bool packed = a.records != nullptr;
-    const size_t lds = lds_for<QT>(a.width, a.max_units, packed);
+    const size_t lds = lds_for<QT>(a.width, a.max_units, a.records != nullptr);
     // the builds without a work table take the grid's shape in the table pointer's place (see the kernel): 16 bits each for the
     // workgroups per XCD and the units per stream, 8 each for streams and heads
     const StepItem *items_or_shape = a.items;
@@ -541,7 +553,7 @@ int launch_t(State *st, const StepAttnArgs &a, char *error, size_t capacity) {
                                          ((unsigned long long)a.heads << 40);
         items_or_shape = reinterpret_cast<const StepItem *>(shape);
     }
-    hipLaunchKernelGGL(kernel_for<QT>(a.width, a.is_self != 0, !packed), dim3(grid), dim3(kThreads), lds, st->stream, a.slots, a.x, a.w, a.scales, a.ln_gain,
+    hipLaunchKernelGGL(kernel_for<QT>(a.width, a.is_self != 0, !packed, a.plain_table != 0), dim3(grid), dim3(kThreads), lds, st->stream, a.slots, a.x, a.w, a.scales, a.ln_gain,
                        a.ln_bias, items_or_shape, per_xcd, lg, a);
     return hip_check(hipGetLastError(), "step attention launch", error, capacity);
 }
@@ -596,8 +608,8 @@ int step_attention_grid(int heads, int batch, int max_units, int is_self, bool p
     return 8 * ((items + 7) / 8);
 }
 
-StepItemTables step_item_tables(int batch, int heads, int cross_heads, int max_units, StepItem *self_items, StepItem *cross_items, bool with_fold,
-                                int self_slots, int cross_slots) {
+StepItemTables step_item_tables(int batch, int heads, int cross_heads, int max_units, StepItem *self_items, StepItem *cross_items, bool self_fold,
+                                bool cross_fold, int self_slots, int cross_slots) {
     StepItemTables t{};
     if (batch < 1 || batch > kMaxBatch || heads < 1 || heads > 255 || cross_heads < 0 || cross_heads > 255 || max_units < 1 || max_units > 32000 ||
         self_items == nullptr || (cross_heads > 0 && cross_items == nullptr))
@@ -609,9 +621,10 @@ StepItemTables step_item_tables(int batch, int heads, int cross_heads, int max_u
     t.batch = batch;
     t.heads = heads;
     t.cross_heads = cross_heads;
-    t.with_fold = with_fold ? 1 : 0;
-    t.self_budget = self_slots - 8 * ((2 * batch * heads + 7) / 8) - (with_fold ? heads * batch : 0);
-    t.cross_budget = cross_slots - (with_fold ? cross_heads * batch : 0);
+    t.self_fold = self_fold ? 1 : 0;
+    t.cross_fold = cross_fold ? 1 : 0;
+    t.self_budget = self_slots - 8 * ((2 * batch * heads + 7) / 8) - (self_fold ? heads * batch : 0);
+    t.cross_budget = cross_slots - (cross_fold ? cross_heads * batch : 0);
     return t;
 }
 
@@ -619,6 +632,7 @@ int launch_step_attention(State *st, const StepAttnArgs &a, char *error, size_t 
     if (a.batch < 1 || a.batch > kMaxBatch || a.max_units < 1 || a.partial == nullptr || a.partial_ml == nullptr || a.slots == nullptr ||
         (a.records != nullptr && (a.batch <= kConsumerFoldMaxBatch || a.items == nullptr || a.layer >= 255 || a.abort_word == nullptr ||
                                   a.fold_out == nullptr)) ||
+        (a.plain_table != 0 && (a.records != nullptr || a.width != 768 || a.items == nullptr)) ||
         !step_attention_supported(a.qtype, (size_t)a.width, (size_t)a.heads, (size_t)a.head_width)) {
         set_error(error, capacity, "step attention: invalid or unsupported shape");
         return -1;

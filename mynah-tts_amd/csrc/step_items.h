@@ -92,10 +92,10 @@ __device__ inline StepItem make_item(const StepSlots &slots, int uniform_length,
 // Entry i of the two tables laid end to end (self first); callers run it for i = 0 .. self_entries + cross_entries - 1.
 __device__ inline void write_step_item(const StepItemTables &t, const StepSlots &slots, int uniform_length, int epoch, int i) {
     if (i < t.self_entries)
-        t.self_items[i] = make_item(slots, uniform_length, t.batch, t.heads, true, i, epoch, t.with_fold != 0, t.self_budget);
+        t.self_items[i] = make_item(slots, uniform_length, t.batch, t.heads, true, i, epoch, t.self_fold != 0, t.self_budget);
     else if (i - t.self_entries < t.cross_entries)
         t.cross_items[i - t.self_entries] =
-            make_item(slots, uniform_length, t.batch, t.cross_heads, false, i - t.self_entries, epoch, t.with_fold != 0, t.cross_budget);
+            make_item(slots, uniform_length, t.batch, t.cross_heads, false, i - t.self_entries, epoch, t.cross_fold != 0, t.cross_budget);
 }
 
 }  // namespace mynah

@@ -691,6 +691,64 @@ def test_many_stream_forms_agree(pkg, backend, synth, qtype_name):
         backend.set_quant(0)
 
 
+@pytest.mark.parametrize("qtype_name,batch", [("int8", 6), ("int4", 3), ("f16", 8), ("f32", 5), ("int8", 2)])
+def test_who_folds_keeps_every_bit(pkg, backend, synth, qtype_name, batch):
+    """The same streams with caches on either side of the lines between folding in the attention launch and in the product behind it (one stream
+    beyond 2,176 rows; more than forty units between more than five streams), in turns on one decoder, and beyond the lines also with the
+    fold kernel and with grouped chunks: every stream's rows and appended cache rows are those of the stream alone.  Stream 0's units go past what the
+    prologue requests at once, and past the second batch."""
+    import os
+    _announce("who folds, %s batch %d" % (qtype_name, batch))
+    longs = [2320, 900, 1290, 1153, 1300, 600, 128, 129][:batch]
+    shorts = [1153, 0, 129, 1152, 127, 1, 300, 128][:batch]
+    mems = [40, 0, 130, 7, 129, 64, 3, 200][:batch]
+    cfg = synth.decoder_config(layers=2, capacity=2400)
+    weights = synth.decoder_weights(cfg, seed=0)
+    long_streams = synth.decoder_streams(cfg, longs, mems, seed=3)
+    streams = [dict(s, length=n) for s, n in zip(long_streams, shorts)]
+    backend.set_quant(QT[qtype_name])
+
+    def rows(h, b, n):
+        k, v = h.cache_rows(b)
+        return k[:, n].copy(), v[:, n].copy()
+
+    try:
+        h = Harness(pkg, backend, cfg, weights, long_streams)
+        alone = {}
+        for lengths, which in ((longs, long_streams), (shorts, streams)):
+            h.streams = which
+            for b in range(batch):
+                out = h.step([b])[0]
+                alone[id(which), b] = (out,) + rows(h, b, lengths[b])
+                h.reset_cache(b)
+        for turn in range(4):                                   # eager, capture and two replays of either form
+            for lengths, which in ((longs, long_streams), (shorts, streams)):
+                h.streams = which
+                outs = h.step()
+                for b in range(batch):
+                    want = alone[id(which), b]
+                    got = (outs[b],) + rows(h, b, lengths[b])
+                    assert all(np.array_equal(g.view(np.uint32), w.view(np.uint32)) for g, w in zip(got, want)), "turn %d, %s stream %d" % (turn, lengths, b)
+                    h.reset_cache(b)
+        h.close()
+        for env in ({"MYNAH_HIP_FOLD_IN_LAUNCH": "0"}, {"MYNAH_HIP_ATTN_SLOTS": "100"}):
+            os.environ.update(env)
+            try:
+                h = Harness(pkg, backend, cfg, weights, long_streams)
+            finally:
+                for k in env:
+                    del os.environ[k]
+            for lengths, which in ((longs, long_streams), (shorts, streams)):
+                h.streams = which
+                outs = h.step()
+                for b in range(batch):
+                    assert np.array_equal(outs[b].view(np.uint32), alone[id(which), b][0].view(np.uint32)), "%s %s stream %d" % (env, lengths, b)
+                    h.reset_cache(b)
+            h.close()
+    finally:
+        backend.set_quant(0)
+
+
 def test_long_cache_takes_the_fold_kernel(pkg, backend, orc, synth, nerr):
     """A capacity whose per-(stream, head) partial records exceed the LDS a launch may use without asking (more than
     about 19,000 rows): the many-stream step then folds in a kernel of its own.  Three streams, one of them 20,000 rows
