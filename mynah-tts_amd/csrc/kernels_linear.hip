@@ -636,10 +636,10 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
     const auto workgroups = [&]() { return (long)((a.n + rows_per_wg_pass * passes - 1) / (rows_per_wg_pass * passes)) * groups; };
     // four streams to a group: twice the rows per workgroup when the groups together would otherwise be more workgroups than the chip has CUs
     if (kStridedLead<BT, SPEC> && groups > 1 && workgroups() > st->cu_count) passes *= 2;
-    // One stream to a group, attention folded in the prologue: twice the rows from three workgroups a CU on, where folds repeated cost more than
-    // the second pass (eight f32 streams, 1536 / 768 workgroups: 614 / 582 us a step; f16, 768 / 384: 459 / 469), and from two a CU on beside
-    // another lane (sixteen f16 streams 818 / 785, f32 839 / 829).
-    if ((BUILD & SPEC_SIDE) != 0 && groups > 2 && a.fold_partial != nullptr)
+    // One stream to a group: twice the rows from three workgroups a CU on, where prologues repeated cost more than the second pass (output
+    // projections with the fold, eight f32 streams, 1536 / 768 workgroups: 614 / 582 us a step; f16, 768 / 384: 459 / 469), and from two a CU
+    // on beside another lane (sixteen f16 streams 818 / 785, f32 839 / 829).
+    if ((BUILD & SPEC_SIDE) != 0 && groups > 2)
         while (workgroups() > (a.beside ? 2 : 3) * st->cu_count) passes *= 2;
     const int rows_per_wg = rows_per_wg_pass * passes;
     const int grid = (a.n + rows_per_wg - 1) / rows_per_wg;
@@ -692,10 +692,13 @@ int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity
     if constexpr (SPEC != SPEC_ANY) {
         // Streams side by side in ONE launch of the one-stream build: a workgroup stages one stream's row, and folds one stream's attention, whatever
         // else is stepped, for a weight that is read once a stream (from L2 after the first).  us a step, as tiles / side by side: output projections
-        // with the fold, int8 two streams (600 and 900 rows) 360 / 326; FFN up two streams 326 / 318 (three int8 360 / 363, four f32 491 / 510: not from three on);
-        // FFN down two streams 318 / 314, three int4 382 / 368, f16 422 / 407, four int8 371 / 370.
+        // with the fold, int8 two streams (600 and 900 rows) 360 / 326; FFN up two streams 326 / 318; FFN down 318 / 314, three int4 382 / 368, f16 422 / 407,
+        // four int8 371 / 370.  Of more streams only where staging a tile of them costs more than their own workgroups do -- int4 and f16 rows
+        // beside their products' instructions, f32 rows of 3072 -- and with no lane beside: FFN down, five f16 441 / 426, eight 517 / 503, f32 610 / 599 (int8 466 /
+        // 472, sixteen f16 in two lanes 791 / 831); FFN up, five f16 425 / 418, six int4 358 / 350 (three int8 360 / 363, eight f32 599 / 614).
         if (a.batch <= 1) return launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
-        const int most = a.fold_partial != nullptr ? kBatchTile : SPEC == SPEC_UP || KFIX == 768 ? 2 : 4;
+        const bool all = a.beside == 0 && (SPEC == SPEC_UP ? QT == MYNAH_HIP_INT4 || QT == MYNAH_HIP_F16 : KFIX == 3072 && QT != MYNAH_HIP_INT8);
+        const int most = a.fold_partial != nullptr || all ? kBatchTile : SPEC == SPEC_RESIDUAL && KFIX == 3072 ? 4 : 2;
         if (a.batch <= most && dense_rows(a)) return launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE>(st, a, error, capacity);
         if (a.batch <= 2) {   // (launch_linear_q sends such launches to the general build; this is the backstop)
             set_error(error, capacity, "linear: rows do not lie one behind the other");

@@ -691,7 +691,7 @@ def test_many_stream_forms_agree(pkg, backend, synth, qtype_name):
         backend.set_quant(0)
 
 
-@pytest.mark.parametrize("qtype_name,batch", [("int8", 6), ("int4", 3), ("f16", 8), ("f32", 5), ("int8", 2)])
+@pytest.mark.parametrize("qtype_name,batch", [("int8", 6), ("int4", 3), ("f16", 8), ("f32", 5), ("int8", 2), ("int4", 7)])
 def test_who_folds_keeps_every_bit(pkg, backend, synth, qtype_name, batch):
     """The same streams with caches on either side of the lines between folding in the attention launch and in the product behind it (one stream
     beyond 2,176 rows; more than forty units between more than five streams), in turns on one decoder, and beyond the lines also with the
