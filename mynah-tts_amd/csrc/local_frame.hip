@@ -53,16 +53,10 @@ struct LocalFrameDev {
 };
 
 struct SampleArgs {
-    LocalFrameDev *frame;
-    const float *logits;          // [batch, vocab]
-    const float *audio_table;     // [vocab, width] of this position
-    const float *next_position;   // position row of the next step, or null
-    float *x;                     // [batch, width]: residual rows of the stack = its next input
     StepSlots *slots;             // cache lengths advance here
     unsigned *values, *stored;    // [batch, streams]
-    int stream, streams, vocab, codebook_size, eos_id, codebook_count, width;
-    int batch;                    // workgroups behind the items' fill `tables` for the next pass through the stack
-    StepItemTables tables;
+    int stream, streams, codebook_count, width;
+    StepItemTables tables;        // for the next pass through the stack, filled by the workgroups behind the items'
 };
 
 // Monotone map float -> unsigned: a > b  <=>  key(a) > key(b)  (no NaNs among logits that matter), and back.
@@ -93,36 +87,30 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
     return max(max(r0, r1), max(r2, r3));
 }
 
-// How many of list[0, n) are above `mine` (pairs of entries per LDS read; the list is 16-byte aligned), counted by four
-// adjacent threads: thread `part` of the four looks at pairs part, part + 4, ... and the four sums meet by shuffles.  Every
-// lane of the wavefront must call it.
-__device__ __forceinline__ int count_above_by_four(const unsigned long long *list, int n, unsigned long long mine, int part) {
-    const ulonglong2 *pairs = reinterpret_cast<const ulonglong2 *>(list);
-    int above = 0;
+// How many of the collected candidates come before candidate (key, index) in the list, in full: the larger key first, among equal keys the
+// smaller index.
+__device__ __forceinline__ int count_before(const unsigned *keys, const int *ids, int n, unsigned key, int id, int from, int step) {
+    int before = 0;
 #pragma unroll 4
-    for (int j = part; j < n / 2; j += 4) {
-        const ulonglong2 p = pairs[j];
-        above += (p.x > mine ? 1 : 0) + (p.y > mine ? 1 : 0);
-    }
-    if ((n & 1) && part == 0) above += list[n - 1] > mine ? 1 : 0;
-    above += dpp_i<kDppXor1>(above);
-    above += dpp_i<kDppXor2>(above);
-    return above;
+    for (int j = from; j < n; j += step) before += keys[j] > key || (keys[j] == key && ids[j] < id) ? 1 : 0;
+    return before;
 }
-
-// The same for a list of at most 64 entries followed by zeros up to 64 (no candidate is zero): every thread's eight reads
-// are requested at once.
-__device__ __forceinline__ int count_above_in_64(const unsigned long long *list, unsigned long long mine, int part) {
-    const ulonglong2 *pairs = reinterpret_cast<const ulonglong2 *>(list);
-    ulonglong2 p[8];
+// The same by the keys alone, counted by LANES adjacent threads: thread `part` compares the quads of keys part, part + LANES, ..., sixteen reads
+// together; the keys behind the list are zero (no candidate's is).  Every lane of the wavefront must call it.
+template <int LANES>
+__device__ __forceinline__ int count_larger(const unsigned *keys, int n, unsigned key, int part) {
+    const uint4 *const quads = reinterpret_cast<const uint4 *>(keys) + part;
+    int larger = 0;
+#pragma unroll 1
+    for (int q0 = 0; 4 * q0 < n; q0 += 16 * LANES) {
+        uint4 k[16];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) p[j] = pairs[part + 4 * j];
-    int above = 0;
+        for (int i = 0; i < 16; ++i) k[i] = quads[q0 + i * LANES];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) above += (p[j].x > mine ? 1 : 0) + (p[j].y > mine ? 1 : 0);
-    above += dpp_i<kDppXor1>(above);
-    above += dpp_i<kDppXor2>(above);
-    return above;
+        for (int i = 0; i < 16; ++i) larger += (k[i].x > key ? 1 : 0) + (k[i].y > key ? 1 : 0) + (k[i].z > key ? 1 : 0) + (k[i].w > key ? 1 : 0);
+    }
+    if (LANES == 2) larger += dpp_i<kDppXor1>(larger);
+    return larger;
 }
 
 // Frame start: the slot table (caches of this object, every length 0), x[b] = decoder_last[b] + position[0]
@@ -152,95 +140,115 @@ __global__ void __launch_bounds__(256) k_local_begin(LocalFrameDev *frame, const
 // Sampling needs the top_count largest candidates in list order.  Common case: every thread keeps the best of its own
 // (strided) candidates; each wavefront finds the ceil(top_count / 4)-th best among its 64 (bit by bit, with ballots),
 // and the smallest of the four is a lower bound of the wanted threshold with at least top_count candidates at or above
-// it, and usually not many more (some 60 for top-50 of 2048 logits).  Those are collected and ranked against each other,
-// all pairs.  When more than kFastCandidates qualify (large top-k, many equal logits) the
+// it, and usually not many more (some 60 for top-50 of 2048 logits, 115 to 130 for top-80).  Those are collected and ranked against each
+// other, all pairs.  When more than kFastCandidates qualify (large top-k, many equal logits) the
 // threshold is found exactly by radix selection instead and exactly top_count candidates are collected.  Both ways end in
 // the same list, ranked the same way.
+//
+// A launch is one workgroup's chain.  Cycles by clock stamps for top-80 of 2048 (115 candidates), before / now: arguments 900 / 640, logits, mask,
+// bests and bound 3850 / 2650, collection 2050 / 1590, ranking and numerators 4600 / 2030, running sums, draw and pick 2200 / 2360, next row
+// 1900 / 1800.  What changed: leading arguments in registers; nothing written to LDS that only the radix selection reads; candidates not taken
+// stored where nobody looks, without a branch; the ranking by the keys' 32 bits, two threads a candidate (list places that two equal keys
+// leave empty are seen afterwards and filled in full); and behind the ranking the first wavefront alone, so that nothing waits at a barrier.
+// Measured and not kept: the rows of the first 8 or 32 list positions fetched by the other wavefronts meanwhile (no change).
+// A frame of 16 positions, us, int8: one stream top-80 402 -> 380, three top-100 461 -> 439, eight top-50 494 -> 472.
 constexpr int kFastCandidates = 512;
+constexpr int kRankByKeys = 256;     // candidates ranked by their keys alone
+constexpr int kEmptyPlace = 0x7fffffff;
 
-__global__ void __launch_bounds__(256) k_local_sample(const SampleArgs a) {
+__global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame, const float *const logits, const float *const audio_table,
+                                                      const float *const next_position, float *const x, const int V, const int batch, const int codebook_size,
+                                                      const int eos_id, const SampleArgs a) {
+    // (the fourteen dwords in front are in registers when a wavefront starts; the rest comes out of memory)
     extern __shared__ __align__(16) unsigned char smem[];
-    unsigned *s_key = reinterpret_cast<unsigned *>(smem);          // [vocab] order keys of the masked logits
+    unsigned *s_key = reinterpret_cast<unsigned *>(smem);          // [vocab] order keys of the masked logits (where registers do not hold them, and for the radix selection)
     __shared__ unsigned long long s_head[4];                       // every wavefront's best candidate
     __shared__ unsigned s_bound[4];
-    __shared__ __align__(16) unsigned long long s_cand[kFastCandidates];
+    __shared__ __align__(16) unsigned s_cand_key[kFastCandidates + 1];
+    __shared__ int s_cand_id[kFastCandidates + 1];
     __shared__ unsigned s_hist[4][256];
     __shared__ __align__(16) float s_top_val[kMaxTopK + 32];
     __shared__ int s_top_idx[kMaxTopK];
     __shared__ unsigned s_wave_total[4];
     __shared__ unsigned s_prefix, s_count;
-    __shared__ int s_remaining, s_pick;
-    __shared__ float s_draw;
+    __shared__ int s_remaining;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b = blockIdx.x;
-    if (b >= a.batch) {
+    if (b >= batch) {
         // the next pass's caches hold stream + 1 rows each whatever is chosen here; the slot table's pointers are the frame's
         if (a.stream + 1 < a.streams)
-            write_step_item(a.tables, *a.slots, a.stream + 1, (int)((a.frame->epoch_base + (unsigned)a.stream + 1u) & 0xffffffu), (b - a.batch) * 256 + tid);
+            write_step_item(a.tables, *a.slots, a.stream + 1, (int)((frame->epoch_base + (unsigned)a.stream + 1u) & 0xffffffu), (b - batch) * 256 + tid);
         return;
     }
-    LocalItemDev &item = a.frame->items[b];
-    const int V = a.vocab;
-    const float *lg = a.logits + (size_t)b * V;
+    LocalItemDev &item = frame->items[b];
+    const float *lg = logits + (size_t)b * V;
     // Everything the kernel takes from memory before the choice is requested here, side by side and under no condition
     // (ids past the vocabulary repeat its last one): one round trip.  Requested where they are used, the item's fields, the
     // frame's pointer and the logits were three round trips one after the other, and the generator state a fourth.
-    float first_logits[8];
+    constexpr int kKeysInRegisters = 8;              // a vocabulary of up to 8 * 256 ids: a thread's keys stay in registers
+    float first_logits[kKeysInRegisters];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) first_logits[i] = lg[min(tid + 256 * i, V - 1)];
+    for (int i = 0; i < kKeysInRegisters; ++i) first_logits[i] = lg[min(tid + 256 * i, V - 1)];
     const int forbid_eos = item.forbid_eos;
     const float temperature = item.temperature;
     const unsigned topk = item.topk;
-    const unsigned long long rng_before = item.rng_state;
-    float *logits_copy = a.frame->logits_copy;
+    unsigned long long bits = item.rng_state;
+    float *logits_copy = frame->logits_copy;
+    if (tid < kRankByKeys) s_cand_key[tid] = 0u;   // (256 threads: all of them; behind a list its keys are zero, see count_larger)
+    if (tid == 0) s_count = 0u;
 
     // ---- constraint mask (src/graph.c:1556-1563); eight candidates per thread at a time, the first eight already requested
-    unsigned long long mine = 0ull;
-    constexpr int kKeysInRegisters = 8;              // a vocabulary of up to 8 * 256 ids: a thread's keys stay in registers for the collection below
     const bool keys_in_registers = V <= kKeysInRegisters * 256;
-    unsigned own_key[kKeysInRegisters];
-    const auto mask_eight = [&](const int c0, const float (&v)[8], const bool keep) {
+    unsigned own_key[kKeysInRegisters], best_key = 0u;
+    int best_id = 0;
+    const auto masked_key = [&](const int c, const float v) -> unsigned {
+        const float masked = c < codebook_size || (c == eos_id && !forbid_eos) ? v : -FLT_MAX;
+        const unsigned key = c < V ? order_key(masked) : 0u;
+        if (key > best_key) { best_key = key; best_id = c; }   // (a thread's ids ascend: the first of equal ones stays)
+        return key;
+    };
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int c = c0 + 256 * i;
-            const bool allowed = c < a.codebook_size || (c == a.eos_id && !forbid_eos);
-            const float masked = allowed ? v[i] : -FLT_MAX;
-            const unsigned key = order_key(masked);
-            if (keep) own_key[i] = c < V ? key : 0u;
-            if (c < V) {
-                s_key[c] = key;
-                if (logits_copy != nullptr) logits_copy[((size_t)b * a.streams + a.stream) * V + c] = masked;
-                const unsigned long long cand = candidate(key, c);
-                mine = cand > mine ? cand : mine;
+    for (int i = 0; i < kKeysInRegisters; ++i) own_key[i] = masked_key(tid + 256 * i, first_logits[i]);
+    if (!keys_in_registers) {
+#pragma unroll
+        for (int i = 0; i < kKeysInRegisters; ++i) s_key[tid + 256 * i] = own_key[i];
+        for (int c0 = tid + 8 * 256; c0 < V; c0 += 8 * 256) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = c0 + 256 * i < V ? lg[c0 + 256 * i] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const unsigned key = masked_key(c0 + 256 * i, v[i]);
+                if (c0 + 256 * i < V) s_key[c0 + 256 * i] = key;
             }
         }
-    };
-    mask_eight(tid, first_logits, true);
-    for (int c0 = tid + 8 * 256; c0 < V; c0 += 8 * 256) {
-        float v[8];
+    }
+    if (logits_copy != nullptr) {
+        float *const copy = logits_copy + ((size_t)b * a.streams + a.stream) * V;
+        if (keys_in_registers) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = c0 + 256 * i < V ? lg[c0 + 256 * i] : 0.0f;
-        mask_eight(c0, v, false);
+            for (int i = 0; i < kKeysInRegisters; ++i)
+                if (tid + 256 * i < V) copy[tid + 256 * i] = key_value(own_key[i]);
+        } else {
+            for (int c = tid; c < V; c += 256) copy[c] = key_value(s_key[c]);   // (a thread's own)
+        }
     }
     const int top_count = min((int)min(topk, (unsigned)V), kMaxTopK);
     const bool sampling = temperature > 0.0f && topk > 1u;
-    for (int p = 0; p < 4; ++p) s_hist[p][tid] = 0u;
-    if (tid < 64) s_cand[tid] = 0ull;   // a list of up to 64 candidates is followed by zeros (see count_above_in_64)
-    if (tid == 0) { s_prefix = 0u; s_remaining = top_count; s_count = 0u; s_pick = top_count - 1; }
     // ---- the head of the list: the largest candidate of the wavefront (the largest key, and among the lanes that hold it the
     // largest low word = the smallest id), then of the four
-    const unsigned head_key = wave_max_u32(candidate_key(mine));
-    const unsigned head_low = wave_max_u32(candidate_key(mine) == head_key ? (unsigned)(mine & 0xffffffffull) : 0u);
+    const unsigned head_key = wave_max_u32(best_key);
+    const unsigned head_low = wave_max_u32(best_key == head_key ? 0xffffffffu - (unsigned)best_id : 0u);
     unsigned long long head = ((unsigned long long)head_key << 32) | (unsigned long long)head_low;
     // (sampling) the largest key with its low half clear that at least `want` of the wavefront's 64 bests reach: sixteen
     // ballots; the keys between this bound and the exact one (1/128 of the logit's magnitude) add a candidate or two
     unsigned bound = 0u;
     if (sampling) {
         const int want = (top_count + 3) / 4;
-        const unsigned own = candidate_key(mine);
+#pragma unroll
         for (int bit = 31; bit >= 16; --bit) {
             const unsigned trial = bound | (1u << bit);
-            if ((int)__popcll(__ballot(own >= trial)) >= want) bound = trial;
+            if ((int)__popcll(__ballot(best_key >= trial)) >= want) bound = trial;
         }
     }
     if (lane == 0) { s_head[wave] = head; s_bound[wave] = bound; }
@@ -257,12 +265,13 @@ __global__ void __launch_bounds__(256) k_local_sample(const SampleArgs a) {
     if (sampling) {
         // ---- collect the candidates at or above the bound: one LDS counter update per wavefront, places by ballot
         if (keys_in_registers) {
-            // from the keys the thread kept (ids tid + 256 i): eight ballots, no LDS read
+            // from the keys the thread kept (ids tid + 256 i): eight ballots, no LDS read; what is not taken goes to a place nobody reads
             unsigned long long masks[kKeysInRegisters];
             unsigned in_wave = 0u;
+            const unsigned least = max(bound, 1u);   // (ids past the vocabulary have key zero)
 #pragma unroll
             for (int i = 0; i < kKeysInRegisters; ++i) {
-                masks[i] = __ballot(tid + 256 * i < V && own_key[i] >= bound);
+                masks[i] = __ballot(own_key[i] >= least);
                 in_wave += (unsigned)__popcll(masks[i]);
             }
             unsigned next_slot = 0u;
@@ -270,9 +279,10 @@ __global__ void __launch_bounds__(256) k_local_sample(const SampleArgs a) {
             next_slot = (unsigned)__builtin_amdgcn_readfirstlane((int)next_slot);
 #pragma unroll
             for (int i = 0; i < kKeysInRegisters; ++i) {
-                const bool take = (masks[i] >> lane) & 1ull;
-                const unsigned slot = next_slot + (unsigned)__popcll(masks[i] & ((1ull << lane) - 1ull));
-                if (take && slot < (unsigned)kFastCandidates) s_cand[slot] = candidate(own_key[i], tid + 256 * i);
+                const unsigned ahead = __builtin_amdgcn_mbcnt_hi((unsigned)(masks[i] >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)masks[i], next_slot));
+                const unsigned slot = own_key[i] >= least ? min(ahead, (unsigned)kFastCandidates) : (unsigned)kFastCandidates;
+                s_cand_key[slot] = own_key[i];
+                s_cand_id[slot] = tid + 256 * i;
                 next_slot += (unsigned)__popcll(masks[i]);
             }
         } else {
@@ -290,16 +300,26 @@ __global__ void __launch_bounds__(256) k_local_sample(const SampleArgs a) {
                 const bool take = c < V && key >= bound;
                 const unsigned long long mask = __ballot(take);
                 const unsigned slot = next_slot + (unsigned)__popcll(mask & ((1ull << lane) - 1ull));
-                if (take && slot < (unsigned)kFastCandidates) s_cand[slot] = candidate(key, c);
+                if (take && slot < (unsigned)kFastCandidates) { s_cand_key[slot] = key; s_cand_id[slot] = c; }
                 next_slot += (unsigned)__popcll(mask);
             }
         }
+        if (tid < top_count) s_top_idx[tid] = kEmptyPlace;
+        if (tid < 32) s_top_val[top_count + tid] = 0.0f;   // lets the running sum below go in whole groups of 32
         __syncthreads();
         int listed = (int)s_count;
         if (listed > kFastCandidates) {
             // ---- the top_count-th largest key by radix selection: four 8-bit digits, most significant first.  Per digit
             // one LDS histogram of the candidates that share the digits chosen so far; the first wavefront then finds the
             // bin in which the wanted rank falls (four bins per lane, suffix sums across lanes by shuffles).
+            if (keys_in_registers) {
+#pragma unroll
+                for (int i = 0; i < kKeysInRegisters; ++i)
+                    if (tid + 256 * i < V) s_key[tid + 256 * i] = own_key[i];
+            }
+            for (int p = 0; p < 4; ++p) s_hist[p][tid] = 0u;
+            if (tid == 0) { s_prefix = 0u; s_remaining = top_count; }
+            __syncthreads();
             for (int p = 0; p < 4; ++p) {
                 const int shift = 24 - 8 * p;
                 const unsigned prefix = s_prefix;
@@ -358,94 +378,145 @@ __global__ void __launch_bounds__(256) k_local_sample(const SampleArgs a) {
             for (int c = c0; c < c1; ++c) {
                 const unsigned key = s_key[c];
                 if (key > threshold) {
-                    s_cand[pos_gt++] = candidate(key, c);
+                    s_cand_key[pos_gt] = key;
+                    s_cand_id[pos_gt++] = c;
                 } else if (key == threshold) {
-                    if (pos_eq < take_equal) s_cand[total_gt + pos_eq] = candidate(key, c);
+                    if (pos_eq < take_equal) { s_cand_key[total_gt + pos_eq] = key; s_cand_id[total_gt + pos_eq] = c; }
                     ++pos_eq;
                 }
             }
             listed = top_count;
-            if (tid >= top_count && tid < 64) s_cand[tid] = 0ull;   // behind a short list: zeros again (count_above_in_64)
+            if (tid >= top_count) s_cand_key[tid] = 0u;   // behind the list: zeros again (at most 256 places: top_count <= kMaxTopK)
             __syncthreads();
         }
         // ---- list position = how many collected candidates come before; numerators expf((l - max) / T) (src/graph.c:1599-1604)
-        for (int q0 = 0; q0 < listed; q0 += 64) {   // four adjacent threads per candidate; every lane takes part in the exchanges
-            const int q = q0 + (tid >> 2);
-            const unsigned long long own = s_cand[q < listed ? q : listed - 1];
-            const int place = listed <= 64 ? count_above_in_64(s_cand, own, tid & 3) : count_above_by_four(s_cand, listed, own, tid & 3);
-            if (q < listed && (tid & 3) == 0 && place < top_count) {
-                s_top_idx[place] = candidate_index(own);
-                s_top_val[place] = expf((key_value(candidate_key(own)) - maximum) / temperature);
+        // (equal keys ranked by their keys alone share a place: the smallest id stays there, and the places behind it stay empty)
+        const auto put_in_place = [&](const int place, const unsigned key, const int id) {
+            atomicMin(&s_top_idx[place], id);
+            s_top_val[place] = expf((key_value(key) - maximum) / temperature);
+        };
+        static_assert(kMaxTopK == 256 && kRankByKeys == 256, "a thread for every candidate ranked by its key");
+        if (listed <= kRankByKeys / 2) {
+            const unsigned key = s_cand_key[tid >> 1];
+            const int id = s_cand_id[min(tid >> 1, listed - 1)], place = count_larger<2>(s_cand_key, listed, key, tid & 1);
+            if ((tid >> 1) < listed && (tid & 1) == 0 && place < top_count) put_in_place(place, key, id);
+        } else if (listed <= kRankByKeys) {
+            const unsigned key = s_cand_key[tid];
+            const int id = s_cand_id[min(tid, listed - 1)], place = count_larger<1>(s_cand_key, listed, key, 0);
+            if (tid < listed && place < top_count) put_in_place(place, key, id);
+        } else {
+            for (int q0 = 0; q0 < listed; q0 += 64) {   // four adjacent threads per candidate; every lane takes part in the exchanges
+                const int q = min(q0 + (tid >> 2), listed - 1), id = s_cand_id[q];
+                const unsigned key = s_cand_key[q];
+                int place = count_before(s_cand_key, s_cand_id, listed, key, id, tid & 3, 4);
+                place += dpp_i<kDppXor1>(place);
+                place += dpp_i<kDppXor2>(place);
+                if (q0 + (tid >> 2) < listed && (tid & 3) == 0 && place < top_count) put_in_place(place, key, id);
             }
         }
-        if (tid < 32) s_top_val[top_count + tid] = 0.0f;   // lets the running sum below go in whole groups of 32
         __syncthreads();
-        // ---- running sums in list order by one thread, kept in place (src/graph.c:1605-1616): float32 sums depend on
-        // the order, and the last running sum is the reference's total
-        if (tid == 0) {
-            float running = 0.0f;
-            for (int q0 = 0; q0 < top_count; q0 += 32) {   // a group's reads are requested together, its sums stay in registers
-                float4 part[8];
+        if (wave > 0) return;
+        int ids[4];   // of list positions lane, lane + 64, ...
+        bool empty = false;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) part[i] = *reinterpret_cast<const float4 *>(&s_top_val[q0 + 4 * i]);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    running += part[i].x; part[i].x = running;
-                    running += part[i].y; part[i].y = running;
-                    running += part[i].z; part[i].z = running;
-                    running += part[i].w; part[i].w = running;
-                }
-#pragma unroll
-                for (int i = 0; i < 8; ++i) *reinterpret_cast<float4 *>(&s_top_val[q0 + 4 * i]) = part[i];
-            }
-            unsigned long long bits = rng_before;
-            bits ^= bits << 13;
-            bits ^= bits >> 7;
-            bits ^= bits << 17;
-            bits = bits == 0ull ? 0x9e3779b97f4a7c15ull : bits;
-            item.rng_state = bits;
-            s_draw = ((float)((bits >> 40) & 0xffffffull) / 16777216.0f) * running;
+        for (int r = 0; r < 4; ++r) {
+            ids[r] = 64 * r + lane < top_count ? s_top_idx[64 * r + lane] : 0;
+            empty = empty || ids[r] == kEmptyPlace;
         }
-        __syncthreads();
+        if (__builtin_expect(__any(empty), 0)) {   // equal keys: their order is their ids'
+            for (int q = lane; q < listed; q += 64) {
+                const int place = count_before(s_cand_key, s_cand_id, listed, s_cand_key[q], s_cand_id[q], 0, 1);
+                if (place < top_count) put_in_place(place, s_cand_key[q], s_cand_id[q]);   // (a shared place already holds its own: the smallest id)
+            }
+            __builtin_amdgcn_wave_barrier();
+            __threadfence_block();
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ids[r] = 64 * r + lane < top_count ? s_top_idx[64 * r + lane] : 0;
+        }
+        // ---- running sums in list order (src/graph.c:1605-1616), kept in place: float32 sums depend on the order, and the last running
+        // sum is the reference's total.  Every lane forms all of them, then takes the ones of its own list positions.
+        float running = 0.0f;
+        const auto request_group = [&](float4 (&g)[8], const int q0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) g[i] = *reinterpret_cast<const float4 *>(&s_top_val[min(q0, kMaxTopK) + 4 * i]);
+        };
+        const auto sum_group = [&](float4 (&g)[8], const int q0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                running += g[i].x; g[i].x = running;
+                running += g[i].y; g[i].y = running;
+                running += g[i].z; g[i].z = running;
+                running += g[i].w; g[i].w = running;
+            }
+            if (lane == 0) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) *reinterpret_cast<float4 *>(&s_top_val[q0 + 4 * i]) = g[i];
+            }
+        };
+        float4 even[8], odd[8];   // groups of 32, a group's reads requested before the sums of the one in front
+        request_group(even, 0);
+        for (int q0 = 0; q0 < top_count; q0 += 64) {
+            request_group(odd, q0 + 32);
+            sum_group(even, q0);
+            if (q0 + 32 >= top_count) break;
+            request_group(even, q0 + 64);
+            sum_group(odd, q0 + 32);
+        }
+        float reached[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) reached[r] = s_top_val[64 * r + lane];
+        bits ^= bits << 13;
+        bits ^= bits >> 7;
+        bits ^= bits << 17;
+        bits = bits == 0ull ? 0x9e3779b97f4a7c15ull : bits;
+        const float draw = ((float)((bits >> 40) & 0xffffffull) / 16777216.0f) * running;
         // the first list position whose running sum reaches the draw; the last one if rounding leaves none
-        const float draw = s_draw;
-        for (int q = tid; q < top_count; q += 256)
-            if (draw <= s_top_val[q] && !(q > 0 && draw <= s_top_val[q - 1])) s_pick = q;
-        __syncthreads();
-        value = (unsigned)s_top_idx[s_pick];
-    }
-    // ---- EOS in either the greedy or the chosen token (src/graph.c:1572-1574,1617-1622), codes, next input row
-    if (tid == 0) {
-        if (argmax == (unsigned)a.eos_id || value == (unsigned)a.eos_id) {
-            item.saw_eos = 1;
-            const unsigned long long frame = (unsigned long long)(a.stream / a.codebook_count);
-            if (frame < item.eos_frame) item.eos_frame = frame;
+        int pick = top_count - 1;
+#pragma unroll
+        for (int r = 3; r >= 0; --r) {
+            const unsigned long long there = __ballot(64 * r + lane < top_count && draw <= reached[r]);
+            if (there != 0ull) pick = 64 * r + __builtin_ctzll(there);
         }
-        a.values[(size_t)b * a.streams + a.stream] = value;
-        a.stored[(size_t)b * a.streams + a.stream] = value < (unsigned)a.codebook_size ? value : 0u;   // :1627
-        a.slots->length[b] = a.stream + 1;
+        int id = ids[0];
+#pragma unroll
+        for (int r = 1; r < 4; ++r) id = pick / 64 == r ? ids[r] : id;
+        value = (unsigned)__builtin_amdgcn_readlane(id, pick & 63);
     }
+    if (wave > 0) return;   // (greedy: the first wavefront goes on alone from here)
+    // ---- EOS in either the greedy or the chosen token (src/graph.c:1572-1574,1617-1622), codes, next input row
     if (a.stream + 1 < a.streams) {
         const unsigned emit = value < (unsigned)V ? value : 0u;                                          // :1626
-        const float *row = a.audio_table + (size_t)emit * a.width;                                      // :1651
-        const float *pe = a.next_position;                                                             // :1262-1264
-        if (a.width <= 1024) {   // one round trip: every request before the first sum
-            float rv[4], pv[4];
-            const float *second = pe != nullptr ? pe : row;
+        const float *row = audio_table + (size_t)emit * a.width;                                        // :1651
+        const float *pe = next_position;                                                                // :1262-1264
+        float *const to = x + (size_t)b * a.width;
+        // one round trip per 1024 floats: every request before the first sum (widths are multiples of four, rows whole aligned float4s)
+        const float *second = pe != nullptr ? pe : row;
+        const int n4 = a.width / 4;
+        for (int u0 = lane; u0 - lane < n4; u0 += 256) {
+            float4 rv[4], pv[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int d = tid + 256 * u, at = d < a.width ? d : a.width - 1;
-                rv[u] = row[at];
-                pv[u] = second[at];
+                const int at = min(u0 + 64 * u, n4 - 1);
+                rv[u] = reinterpret_cast<const float4 *>(row)[at];
+                pv[u] = reinterpret_cast<const float4 *>(second)[at];
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int d = tid + 256 * u;
-                if (d < a.width) a.x[(size_t)b * a.width + d] = pe != nullptr ? rv[u] + pv[u] : rv[u];
-            }
-        } else {
-            for (int d = tid; d < a.width; d += 256) a.x[(size_t)b * a.width + d] = pe != nullptr ? row[d] + pe[d] : row[d];
+            for (int u = 0; u < 4; ++u)
+                if (u0 + 64 * u < n4)
+                    reinterpret_cast<float4 *>(to)[u0 + 64 * u] =
+                        pe != nullptr ? make_float4(rv[u].x + pv[u].x, rv[u].y + pv[u].y, rv[u].z + pv[u].z, rv[u].w + pv[u].w) : rv[u];
         }
+    }
+    if (lane == 0) {
+        if (sampling) item.rng_state = bits;   // (stored behind the row's arrival: a wait for loads waits for the stores in front of them)
+        if (argmax == (unsigned)eos_id || value == (unsigned)eos_id) {
+            item.saw_eos = 1;
+            const unsigned long long at = (unsigned long long)(a.stream / a.codebook_count);
+            if (at < item.eos_frame) item.eos_frame = at;
+        }
+        a.values[(size_t)b * a.streams + a.stream] = value;
+        a.stored[(size_t)b * a.streams + a.stream] = value < (unsigned)codebook_size ? value : 0u;   // :1627
+        a.slots->length[b] = a.stream + 1;
     }
 }
 
@@ -506,13 +577,12 @@ static int enqueue_frame(State *st, mynah_hip_local *l, int B, char *error, size
             if (launch_linear(st, p, error, capacity) != 0) return -1;
         }
         SampleArgs a{};
-        a.frame = l->frame; a.logits = l->logits; a.audio_table = l->audio_table[stream];
-        a.next_position = rows.position != nullptr ? rows.position + (stream + 1) * l->width : nullptr;
-        a.x = rows.x; a.slots = rows.slots; a.values = l->values; a.stored = l->values + (size_t)kMaxBatch * l->streams;
-        a.stream = (int)stream; a.streams = (int)l->streams; a.vocab = (int)l->vocab; a.codebook_size = (int)l->codebook_size;
-        a.eos_id = (int)l->eos_id; a.codebook_count = (int)l->codebook_count; a.width = width;
-        a.batch = B; a.tables = tables;
-        hipLaunchKernelGGL(k_local_sample, dim3(B + (stream + 1 < l->streams ? table_workgroups : 0u)), dim3(256), l->vocab * sizeof(float), st->stream, a);
+        a.slots = rows.slots; a.values = l->values; a.stored = l->values + (size_t)kMaxBatch * l->streams;
+        a.stream = (int)stream; a.streams = (int)l->streams; a.codebook_count = (int)l->codebook_count; a.width = width;
+        a.tables = tables;
+        const float *const next_position = rows.position != nullptr ? rows.position + (stream + 1) * l->width : nullptr;
+        hipLaunchKernelGGL(k_local_sample, dim3(B + (stream + 1 < l->streams ? table_workgroups : 0u)), dim3(256), l->vocab * sizeof(float), st->stream,
+                           l->frame, l->logits, l->audio_table[stream], next_position, rows.x, (int)l->vocab, B, (int)l->codebook_size, (int)l->eos_id, a);
         MYNAH_TRY(hipGetLastError());
     }
     return 0;

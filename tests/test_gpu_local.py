@@ -218,6 +218,37 @@ def test_frame_many_tied_candidates(pkg, backend, orc, synth, nerr):
     backend.set_quant(0)
 
 
+@pytest.mark.parametrize("V,copies", [(96, 2), (2048, 3), (2049, 2), (4096, 7)])
+def test_frame_equal_logits_within_the_list(pkg, backend, orc, synth, V, copies):
+    """Every logit comes two, three or seven times over, so equal keys share list places all along the list and across its end, for lists of
+    2 to 256 entries in vocabularies on either side of what the sampler keeps in registers: every choice replayed from the device's own logits."""
+    _announce("local frame, equal logits, vocab %d x %d" % (V, copies))
+    S, codebook, eos, cbc = 4, V - 2, V - 1, 4
+    cfg, w, proj, bias, tables, rng = _setup(synth, 1, S, V, seed=V)
+    groups = (V + copies - 1) // copies
+    for s in range(S):
+        for c in range(1, copies):
+            n = len(proj[s][c * groups:(c + 1) * groups])
+            proj[s][c * groups:(c + 1) * groups] = proj[s][:n]
+            bias[s][c * groups:(c + 1) * groups] = bias[s][:n]
+    items = [{"temperature": 2.0 + 0.3 * i, "topk": k, "rng_state": 77 + 1234567 * i, "forbid_eos": True}
+             for i, k in enumerate((2, 3, 5, 16, 51, 64, 80, 97, 100, 127, 128, 160, 201, 255, 256, 90))]
+    backend.set_quant(QT["f32"])
+    loc = pkg.Local(backend, cfg, w, proj, bias, tables, codebook, eos, cbc)
+    drows = [backend.alloc(cfg["width"]).write(rng.standard_normal(cfg["width"]).astype(np.float32)) for _ in items]
+    dlogits = backend.alloc(len(items) * S * V)
+    for attempt in range(4):     # eager, captured and replays, each from the generator states the frame before left
+        got = loc.frame([dict(it, row=d.ptr) for it, d in zip(items, drows)], dlogits.ptr)
+        logits = dlogits.read().reshape(len(items), S, V)
+        assert np.array_equal(logits[:, :, :2], logits[:, :, groups:groups + 2])
+        _replay_choices(orc, logits, items, got, codebook, eos, cbc)
+        items = [dict(it, rng_state=r) for it, r in zip(items, got["rng_state"])]
+    loc.destroy()
+    for d in drows + [dlogits]:
+        d.free()
+    backend.set_quant(0)
+
+
 def test_frame_eos_outside_vocabulary(pkg, backend, orc, synth, nerr):
     """An end-of-sequence id that is no id of the vocabulary (here one whose low 32 bits are 5, a real id) matches
     nothing, as in the reference's full-width comparison (src/graph.c:1563-1574): only codebook ids are ever allowed,
