@@ -104,7 +104,7 @@ namespace mynah {
 constexpr int kFoldBehindStreams = 5, kFoldBehindUnits = 40, kFoldBehindRows = (kFoldAhead + kFoldMore - 1) * kStepUnitRows;
 static bool folds_behind(const mynah_hip_decoder *d, int is_self, int batch) {
     if (batch <= kConsumerFoldMaxBatch) return true;
-    if (batch > kBatchTile || d->width != 768 || !linear_folds_streams((int)d->width, (int)(is_self ? d->width : d->xw), (int)(is_self ? d->heads : d->cross_heads), d->max_units))
+    if (d->width != 768 || !linear_folds_streams((int)d->width, (int)(is_self ? d->width : d->xw), (int)(is_self ? d->heads : d->cross_heads), d->max_units))
         return false;
     return !(is_self ? d->long_caches : d->long_memories);
 }
@@ -123,7 +123,8 @@ static bool caches_long(const int *rows, int batch, int most_units) {
 static int enqueue_linear(State *st, const mynah_hip_decoder *d, const CachedWeight *w, const float *in, size_t in_stride,
                           float *out, size_t out_stride, int batch, const float *ln_gain, const float *ln_bias, int epilogue,
                           char *error, size_t capacity, int fold = 0, int probe_slot = -1) {
-    for (int b0 = 0; b0 < batch; b0 += kBatchTile) {
+    const int tile = linear_takes_all((int)w->n, (int)w->k, epilogue, ln_gain != nullptr, in_stride, out_stride) ? kMaxBatch : kBatchTile;
+    for (int b0 = 0; b0 < batch; b0 += tile) {
         LinearArgs a{};
         if (d->probe_qx != nullptr && probe_slot >= 0 && b0 == 0) {
             a.probe_qx = d->probe_qx + (size_t)probe_slot * d->ffn;
@@ -145,8 +146,8 @@ static int enqueue_linear(State *st, const mynah_hip_decoder *d, const CachedWei
         a.qtype = w->qtype;
         a.n = (int)w->n;
         a.k = (int)w->k;
-        a.batch = batch - b0 < kBatchTile ? batch - b0 : kBatchTile;
-        for (int b = 0; b < a.batch; ++b) {
+        a.batch = batch - b0 < tile ? batch - b0 : tile;
+        for (int b = 0; b < a.batch && b < kBatchTile; ++b) {
             a.in[b] = in + (size_t)(b0 + b) * in_stride;
             a.out[b] = out + (size_t)(b0 + b) * out_stride;
         }

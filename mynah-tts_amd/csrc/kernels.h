@@ -14,7 +14,8 @@ struct LinearArgs {
     const float *bias;      // [n] or null
     int qtype;
     int n, k;
-    int batch;              // streams in this pass (<= kBatchTile)
+    int batch;              // streams in this pass: up to kBatchTile, or, where linear_takes_all says so, up to kMaxBatch -- in and out then hold the
+                            // first kBatchTile rows, which lie at one stride, and the others lie on at it
     const float *in[kBatchTile];
     float *out[kBatchTile];
     const float *ln_gain;   // non-null: LayerNorm prologue (eps 1e-5)
@@ -44,6 +45,8 @@ struct LinearArgs {
 // True when the fused matvec kernel supports this shape/storage; otherwise use linear_generic.
 bool linear_fast_supported(int qtype, size_t n, size_t k);
 int launch_linear(State *st, const LinearArgs &args, char *error, size_t capacity);
+// Whether launch_linear takes more than kBatchTile streams of such a product in one launch (no probes, no bias).
+bool linear_takes_all(int n, int k, int epilogue, bool layernorm, size_t in_stride, size_t out_stride);   // strides in floats
 // Whether launch_linear takes such a product with the fold for more than two streams (rows one behind the other, residual epilogue).
 bool linear_folds_streams(int n, int k, int heads, int max_units);
 // Any shape, f32 weights: out[r,n] = in[r,k] W[n,k]^T + bias (rows may be large).

@@ -50,10 +50,10 @@ __device__ __forceinline__ float *stream_out(const LinearArgs &a, int b) {
 // SPEC: what the launch is known not to use, so that the corresponding code is not there at all (0 = everything
 // decided at run time).  SPEC_RESIDUAL: no LayerNorm, no bias, no probes, residual epilogue (the step's output and
 // FFN-down projections; the fold source stays a run-time choice).  SPEC_UP: LayerNorm, no fold, no bias, no probes,
-// GELU epilogue (the step's FFN-up projection).
+// GELU epilogue (the step's FFN-up projection).  SPEC_PLAIN: the product alone (the local frame's vocabulary projections).
 // SPEC_SIDE (with one of the two, one stream to a workgroup): the launch takes several streams side by side, one to each row of the grid
 // (launch_linear_b); a build of its own, so that a lone stream does not wait for the arithmetic that finds a row.
-enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2, SPEC_SIDE = 4 };
+enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2, SPEC_PLAIN = 3, SPEC_SIDE = 4 };
 
 // More than two streams: one wavefront stages one stream (load_stream_row / finish_stream_row,
 // device_common.h) -- staging every stream's activations is what such a launch spends most of its time on, every workgroup
@@ -77,32 +77,33 @@ constexpr bool kPackedLead = BT == 1 && SPEC != SPEC_ANY;
 template <int BT, int SPEC>
 constexpr bool kStridedLead = kWaveStaging<BT> && SPEC != SPEC_ANY;
 
-// n:20 | rows per workgroup:12 | streams:4 | input stride / 4:14 | output stride / 4:14 (strides in floats)
+// n:20 | rows per workgroup:12 | streams:5 | input stride / 4:13 | output stride / 4:14 (strides in floats)
 struct StridedShape {
     int n, rows_per_wg, batch;
     size_t in_stride, out_stride;
 };
 __host__ __device__ inline bool strided_fits(const StridedShape &s) {
-    return s.n >= 0 && s.n < (1 << 20) && s.rows_per_wg >= 0 && s.rows_per_wg < (1 << 12) && s.batch >= 0 && s.batch < 16 && s.in_stride % 4 == 0 &&
-           s.in_stride / 4 < (1u << 14) && s.out_stride % 4 == 0 && s.out_stride / 4 < (1u << 14);
+    return s.n >= 0 && s.n < (1 << 20) && s.rows_per_wg >= 0 && s.rows_per_wg < (1 << 12) && s.batch >= 0 && s.batch <= kMaxBatch && s.in_stride % 4 == 0 &&
+           s.in_stride / 4 < (1u << 13) && s.out_stride % 4 == 0 && s.out_stride / 4 < (1u << 14);
 }
 __host__ __device__ inline unsigned long long pack_strided(const StridedShape &s) {
     return (unsigned long long)s.n | ((unsigned long long)s.rows_per_wg << 20) | ((unsigned long long)s.batch << 32) |
-           ((unsigned long long)(s.in_stride / 4) << 36) | ((unsigned long long)(s.out_stride / 4) << 50);
+           ((unsigned long long)(s.in_stride / 4) << 37) | ((unsigned long long)(s.out_stride / 4) << 50);
 }
 __device__ __forceinline__ StridedShape unpack_strided(const unsigned long long v) {
     StridedShape s;
-    s.n = (int)(v & 0xfffffu); s.rows_per_wg = (int)((v >> 20) & 0xfffu); s.batch = (int)((v >> 32) & 0xfu);
-    s.in_stride = (size_t)((v >> 36) & 0x3fffu) * 4; s.out_stride = (size_t)((v >> 50) & 0x3fffu) * 4;
+    s.n = (int)(v & 0xfffffu); s.rows_per_wg = (int)((v >> 20) & 0xfffu); s.batch = (int)((v >> 32) & 0x1fu);
+    s.in_stride = (size_t)((v >> 37) & 0x1fffu) * 4; s.out_stride = (size_t)((v >> 50) & 0x3fffu) * 4;
     return s;
 }
+static_assert(kMaxBatch < 32, "the streams' five bits");
 // rows of a launch at one stride (floats) from the first, or no stride at all
 inline bool rows_strided(const LinearArgs &a, size_t *in_stride, size_t *out_stride) {
     *in_stride = *out_stride = 0;
     if (a.batch < 2) return true;
     if (a.in[1] < a.in[0] || a.out[1] < a.out[0]) return false;
     const size_t si = (size_t)(a.in[1] - a.in[0]), so = (size_t)(a.out[1] - a.out[0]);
-    for (int b = 2; b < a.batch; ++b)
+    for (int b = 2; b < a.batch && b < kBatchTile; ++b)
         if (a.in[b] != a.in[0] + (size_t)b * si || a.out[b] != a.out[0] + (size_t)b * so) return false;
     *in_stride = si; *out_stride = so;
     return true;
@@ -190,7 +191,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
         a.fold_is_self = shape.is_self; a.fold_stream0 = shape.stream0;
         if constexpr (SPEC == SPEC_UP) {
             a.ln_gain = fold_partial; a.ln_bias = fold_partial_ml;
-        } else {
+        } else if constexpr (SPEC == SPEC_RESIDUAL) {
             if (shape.folding) {
                 a.fold_partial = fold_partial; a.fold_partial_ml = fold_partial_ml; a.fold_slots = reinterpret_cast<const StepSlots *>(in0);
             }
@@ -198,7 +199,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
         if constexpr ((BUILD & SPEC_SIDE) != 0) {
             const size_t y = blockIdx.y;   // the workgroup's stream (dense_rows)
             a.out[0] += y * (size_t)a.n;
-            if (SPEC == SPEC_UP || !shape.folding) a.in[0] += y * (size_t)KFIX;
+            if (SPEC != SPEC_RESIDUAL || !shape.folding) a.in[0] += y * (size_t)KFIX;
             a.fold_stream0 += (int)y;
         }
     } else if constexpr (BT <= 2) {
@@ -233,10 +234,10 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
     float *const arg_probe_sx = SPEC != SPEC_ANY ? nullptr : a.probe_sx;
     int32_t *const arg_probe_acc = SPEC != SPEC_ANY ? nullptr : a.probe_acc;
     float *const arg_aux_out = SPEC != SPEC_ANY ? nullptr : a.aux_out;
-    const int arg_epilogue = SPEC == SPEC_UP ? EPI_GELU : SPEC == SPEC_RESIDUAL ? EPI_RESIDUAL : a.epilogue;
-    const float *const arg_ln_gain = SPEC == SPEC_RESIDUAL ? nullptr : a.ln_gain;
-    const float *const arg_ln_bias = SPEC == SPEC_RESIDUAL ? nullptr : a.ln_bias;
-    const float *const arg_fold_partial = (SPEC == SPEC_UP || BT > kConsumerFoldMaxBatch) ? nullptr : a.fold_partial;   // larger batches fold in a kernel of their own
+    const int arg_epilogue = SPEC == SPEC_UP ? EPI_GELU : SPEC == SPEC_RESIDUAL ? EPI_RESIDUAL : SPEC == SPEC_PLAIN ? EPI_NONE : a.epilogue;
+    const float *const arg_ln_gain = SPEC == SPEC_RESIDUAL || SPEC == SPEC_PLAIN ? nullptr : a.ln_gain;
+    const float *const arg_ln_bias = SPEC == SPEC_RESIDUAL || SPEC == SPEC_PLAIN ? nullptr : a.ln_bias;
+    const float *const arg_fold_partial = (SPEC == SPEC_UP || SPEC == SPEC_PLAIN || BT > kConsumerFoldMaxBatch) ? nullptr : a.fold_partial;   // larger batches fold in a kernel of their own
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float s_sx[BT];
     __shared__ float s_scratch[kPrologueScratch * BT];
@@ -698,7 +699,7 @@ int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity
         // 472, sixteen f16 in two lanes 791 / 831); FFN up, five f16 425 / 418, six int4 358 / 350 (three int8 360 / 363, eight f32 599 / 614).
         if (a.batch <= 1) return launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
         const bool all = a.beside == 0 && (SPEC == SPEC_UP ? QT == MYNAH_HIP_INT4 || QT == MYNAH_HIP_F16 : KFIX == 3072 && QT != MYNAH_HIP_INT8);
-        const int most = a.fold_partial != nullptr || all ? kBatchTile : SPEC == SPEC_RESIDUAL && KFIX == 3072 ? 4 : 2;
+        const int most = a.fold_partial != nullptr ? kMaxBatch : all ? 8 : SPEC == SPEC_RESIDUAL && KFIX == 3072 ? 4 : 2;
         if (a.batch <= most && dense_rows(a)) return launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE>(st, a, error, capacity);
         if (a.batch <= 2) {   // (launch_linear_q sends such launches to the general build; this is the backstop)
             set_error(error, capacity, "linear: rows do not lie one behind the other");
@@ -715,6 +716,8 @@ int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity
     // product the same way, whose LayerNorm prologue each group then runs for its four rows, 497 us with twice the rows per
     // workgroup and 486 us with twice the workgroups; with the second pass's operands requested ahead as below, 476 against 477 us:
     // it keeps the tile of eight.)
+    // Nine to sixteen streams (rows at a stride, linear_takes_all): as many groups, four of four or two of eight, in the one launch -- a
+    // local frame as two launches a product / one, us: int8 ten streams 676 / 482, sixteen 748 / 533, f16 twelve 752 / 598.
     if (kStridedLead<4, SPEC> && SPEC == SPEC_RESIDUAL && stream_groups_enabled()) return launch_linear_t<QT, 4, NVT, KFIX, SPEC>(st, a, error, capacity);
     return launch_linear_t<QT, 8, NVT, KFIX, SPEC>(st, a, error, capacity);
 }
@@ -727,7 +730,7 @@ int launch_linear_q(State *st, const LinearArgs &a, char *error, size_t capacity
     // (the specialised builds of one stream take their small numbers packed into one argument: when one of them
     // does not fit its bit field the launch takes the general build, with the same arithmetic)
     LeadShape fit{};
-    fit.n = a.n; fit.batch = a.batch; fit.rows_per_wg = 2048;   // above what launch_linear_t chooses for any n that fits (256 rows per 196,608 of n)
+    fit.n = a.n; fit.batch = 1; fit.rows_per_wg = 2048;   // above what launch_linear_t chooses for any n that fits (256 rows per 196,608 of n)
     if (a.fold_partial != nullptr) {
         fit.is_self = a.fold_is_self; fit.stream0 = a.fold_stream0; fit.heads = a.fold_heads; fit.max_units = a.fold_max_units; fit.head_width = a.fold_head_width;
     }
@@ -739,9 +742,11 @@ int launch_linear_q(State *st, const LinearArgs &a, char *error, size_t capacity
     }
     const bool residual = plain && packs && a.epilogue == EPI_RESIDUAL && a.ln_gain == nullptr;
     const bool up = plain && packs && a.epilogue == EPI_GELU && a.ln_gain != nullptr && a.fold_partial == nullptr;
+    const bool alone = plain && packs && a.epilogue == EPI_NONE && a.ln_gain == nullptr && a.fold_partial == nullptr;
     if (a.k == 768) {
         if (residual) return launch_linear_b<QT, 1, 768, SPEC_RESIDUAL>(st, a, error, capacity);
         if (up) return launch_linear_b<QT, 1, 768, SPEC_UP>(st, a, error, capacity);
+        if (alone) return launch_linear_b<QT, 1, 768, SPEC_PLAIN>(st, a, error, capacity);
         return launch_linear_b<QT, 1, 768, SPEC_ANY>(st, a, error, capacity);
     }
     if (a.k == 3072) {
@@ -766,8 +771,21 @@ bool linear_folds_streams(int n, int k, int heads, int max_units) {
     return k == 768 && lead_fits(fit);
 }
 
+bool linear_takes_all(int n, int k, int epilogue, bool layernorm, size_t in_stride, size_t out_stride) {
+    StridedShape s{};
+    s.n = n; s.rows_per_wg = 2048; s.batch = kMaxBatch; s.in_stride = in_stride; s.out_stride = out_stride;
+    if (!strided_fits(s) || out_stride == 0) return false;
+    if (epilogue == EPI_RESIDUAL) return !layernorm && (k == 768 || k == 3072);
+    return k == 768 && epilogue == (layernorm ? EPI_GELU : EPI_NONE);
+}
+
 int launch_linear(State *st, const LinearArgs &a, char *error, size_t capacity) {
-    if (a.batch < 1 || a.batch > kBatchTile) {
+    const bool probed = a.probe_qx != nullptr || a.probe_sx != nullptr || a.probe_acc != nullptr || a.ln_out != nullptr || a.ln_out_slots != nullptr ||
+                        a.aux_out != nullptr || a.act_out != nullptr;
+    size_t in_stride = 0, out_stride = 0;
+    if (a.batch < 1 || a.batch > kMaxBatch ||
+        (a.batch > kBatchTile && (a.bias != nullptr || probed || !rows_strided(a, &in_stride, &out_stride) ||
+                                  !linear_takes_all(a.n, a.k, a.epilogue, a.ln_gain != nullptr, in_stride, out_stride)))) {
         set_error(error, capacity, "linear: batch tile out of range");
         return -1;
     }

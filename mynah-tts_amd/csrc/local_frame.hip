@@ -559,7 +559,8 @@ static int enqueue_frame(State *st, mynah_hip_local *l, int B, char *error, size
     for (size_t stream = 0; stream < l->streams; ++stream) {
         if (decoder_enqueue_layers(st, l->stack, B, error, capacity) != 0) return -1;
         const CachedWeight *cw = l->projection[stream];
-        for (int b0 = 0; b0 < B; b0 += kBatchTile) {
+        const int tile = l->projection_bias[stream] == nullptr && linear_takes_all((int)l->vocab, width, EPI_NONE, false, l->width, l->vocab) ? kMaxBatch : kBatchTile;
+        for (int b0 = 0; b0 < B; b0 += tile) {
             LinearArgs p{};
             p.w = cw->data;
             p.scales = cw->scales;
@@ -567,8 +568,8 @@ static int enqueue_frame(State *st, mynah_hip_local *l, int B, char *error, size
             p.qtype = cw->qtype;
             p.n = (int)l->vocab;
             p.k = width;
-            p.batch = B - b0 < kBatchTile ? B - b0 : kBatchTile;
-            for (int b = 0; b < p.batch; ++b) {
+            p.batch = B - b0 < tile ? B - b0 : tile;
+            for (int b = 0; b < p.batch && b < kBatchTile; ++b) {
                 p.in[b] = rows.x + (size_t)(b0 + b) * width;
                 p.out[b] = l->logits + (size_t)(b0 + b) * l->vocab;
             }

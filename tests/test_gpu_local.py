@@ -218,6 +218,31 @@ def test_frame_many_tied_candidates(pkg, backend, orc, synth, nerr):
     backend.set_quant(0)
 
 
+@pytest.mark.parametrize("qtype_name,batch", [("int8", 9), ("int4", 13), ("f16", 16), ("f32", 10), ("int8", 2), ("f16", 5)])
+def test_frame_batches_keep_every_bit(pkg, backend, synth, qtype_name, batch):
+    """Every item of a frame of two to sixteen has the tokens, generator states and masked logits of a frame of its own: the products of all
+    streams are one launch each whatever their number."""
+    _announce("local frame batch %d %s against single frames" % (batch, qtype_name))
+    S, V, codebook, eos, cbc = 5, 544, 530, 531, 4
+    cfg, w, proj, _, tables, rng = _setup(synth, 2, S, V, seed=batch)
+    backend.set_quant(QT[qtype_name])
+    loc = pkg.Local(backend, cfg, w, proj, None, tables, codebook, eos, cbc)
+    items = [dict(ITEMS[i % len(ITEMS)], rng_state=ITEMS[i % len(ITEMS)]["rng_state"] + 31 * i) for i in range(batch)]
+    drows = [backend.alloc(cfg["width"]).write(rng.standard_normal(cfg["width"]).astype(np.float32)) for _ in range(batch)]
+    dlogits = backend.alloc(batch * S * V)
+    for attempt in range(3):     # eager, captured, replayed
+        got = loc.frame([dict(it, row=d.ptr) for it, d in zip(items, drows)], dlogits.ptr)
+        logits = dlogits.read().reshape(batch, S, V).copy()
+        for b in range(batch):
+            one = loc.frame([dict(items[b], row=drows[b].ptr)], dlogits.ptr)
+            assert np.array_equal(dlogits.read(S * V).view(np.uint32), logits[b].reshape(-1).view(np.uint32)), "item %d" % b
+            assert np.array_equal(one["values"][0], got["values"][b]) and one["rng_state"][0] == got["rng_state"][b], "item %d" % b
+    loc.destroy()
+    for d in drows + [dlogits]:
+        d.free()
+    backend.set_quant(0)
+
+
 @pytest.mark.parametrize("V,copies", [(96, 2), (2048, 3), (2049, 2), (4096, 7)])
 def test_frame_equal_logits_within_the_list(pkg, backend, orc, synth, V, copies):
     """Every logit comes two, three or seven times over, so equal keys share list places all along the list and across its end, for lists of
