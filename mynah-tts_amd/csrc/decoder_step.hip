@@ -100,8 +100,10 @@ namespace mynah {
 // streams (611, 1339 and 87 rows) 371 / 349, four 371 / 339, five (7000 rows together) 460 / 443; six of 1060 rows 376 / 353, of 4500 412 / 413,
 // of 6000 436 / 445; eight of 1000 371 / 359, of 3000 401 / 395, of 5000 418 / 415, of 7600 469 / 477.  Cross-attention memories are short: eight streams
 // 479 / 472 (f16 16 streams as two lanes 796 / 785 with both behind).  Either way gives the same bits (fold_partials' arithmetic).
+// Beside another lane the line lies higher (sixteen streams of 12000 rows in two lanes, int8 593 / 579, f16 739 / 725).
 // What a prologue does not request at once (kFoldAhead + kFoldMore partials) it takes one after the other: longer streams fold inside.
-constexpr int kFoldBehindStreams = 5, kFoldBehindUnits = 40, kFoldBehindRows = (kFoldAhead + kFoldMore - 1) * kStepUnitRows;
+constexpr int kFoldBehindStreams = 5, kFoldBehindUnits = 40, kFoldBehindUnitsBeside = 80,
+              kFoldBehindRows = (kFoldAhead + kFoldMore - 1) * kStepUnitRows;
 static bool folds_behind(const mynah_hip_decoder *d, int is_self, int batch) {
     if (batch <= kConsumerFoldMaxBatch) return true;
     if (d->width != 768 || !linear_folds_streams((int)d->width, (int)(is_self ? d->width : d->xw), (int)(is_self ? d->heads : d->cross_heads), d->max_units))
@@ -865,9 +867,9 @@ static int decoder_step(State *st, mynah_hip_decoder *d, const mynah_hip_decoder
         StepSlots ls = lanes == 1 ? s : lane_slots(s, plan, i);
         if (decoder_next_epochs(st, lane, 1, &ls.epoch, error, capacity) != 0) return -1;
         lane->last_slots = ls;
-        lane->long_caches = caches_long(ls.length, plan.count[i], kFoldBehindUnits);
-        lane->long_memories = caches_long(ls.memory_length, plan.count[i], kFoldBehindUnits);
         lane->beside = lanes > 1;
+        lane->long_caches = caches_long(ls.length, plan.count[i], lane->beside ? kFoldBehindUnitsBeside : kFoldBehindUnits);
+        lane->long_memories = caches_long(ls.memory_length, plan.count[i], lane->beside ? kFoldBehindUnitsBeside : kFoldBehindUnits);
         if (launch_step_begin(st, ls, lane->dev_slots, plan.count[i], d->width, d->position, lane->x, d->width, decoder_item_tables(lane, plan.count[i]), error,
                               capacity) != 0)
             return -1;
