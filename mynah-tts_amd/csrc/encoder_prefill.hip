@@ -79,11 +79,10 @@ typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTile = 64;            // workgroup tile of the products: 64 x 64, K step 64
-constexpr int kLdsStride = 72;       // halfs per staged row: 64 + 8 keeps 16-byte reads of 32 rows off each other's banks
+constexpr int kTile = 64;            // widths and padded lengths are multiples of this; the products' largest tile is 64 x 64
+constexpr int kStep = 64;            // K step of the products
 constexpr int kQTile = 32;           // queries per attention workgroup
 constexpr int kScorePad = 8;         // floats appended to a score row (bank spread for the row-wise softmax)
-constexpr int kGemmDepth = 4;        // K steps of operand tiles in flight in the products (see k_enc_gemm)
 constexpr int kLeadRows = 2;         // zero rows in front of the conv FFN's activations (kernel size 3 looks two rows back)
 
 enum { ENC_QKV = 0, ENC_PARTIAL = 1, ENC_GELU = 2 };
@@ -111,139 +110,11 @@ __device__ __forceinline__ float gelu_tanh_for_f16(float x) {
 // Row of C held in accumulator register r of lane l for a 32x32 MFMA tile; the column is l % 32.
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
-// One K step of both operand tiles on its way from global memory to LDS (four 16-byte pieces per thread).
-struct StagedTiles {
-    u32x4 a0 = {0, 0, 0, 0}, a1 = {0, 0, 0, 0}, w0 = {0, 0, 0, 0}, w1 = {0, 0, 0, 0};
-    __device__ __forceinline__ void load(const u32x4 *ga0, const u32x4 *ga1, const u32x4 *gw0, const u32x4 *gw1, int a_chunk, int w_chunk) {
-        a0 = ga0[a_chunk]; a1 = ga1[a_chunk]; w0 = gw0[w_chunk]; w1 = gw1[w_chunk];
-    }
-    __device__ __forceinline__ void store(_Float16 *sa, _Float16 *sw, int off0, int off1) const {
-        *reinterpret_cast<u32x4 *>(sa + off0) = a0;
-        *reinterpret_cast<u32x4 *>(sa + off1) = a1;
-        *reinterpret_cast<u32x4 *>(sw + off0) = w0;
-        *reinterpret_cast<u32x4 *>(sw + off1) = w1;
-    }
-};
-
-// The fragments of one 64-deep K step of a wavefront's 32 x 32 tile (four 32x32x16 MFMAs), read from LDS into registers
-// a step ahead of their use, so that the reads' round trip runs beside the previous step's matrix instructions.
-struct StepFragments {
-    half8 a[kTile / 16], w[kTile / 16];
-    __device__ __forceinline__ void read(const _Float16 *pa, const _Float16 *pw) {
-#pragma unroll
-        for (int j = 0; j < kTile / 16; ++j) {
-            a[j] = *reinterpret_cast<const half8 *>(pa + 16 * j);
-            w[j] = *reinterpret_cast<const half8 *>(pw + 16 * j);
-        }
-    }
-    __device__ __forceinline__ void multiply(floatx16 &acc) const {
-#pragma unroll
-        for (int j = 0; j < kTile / 16; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[j], w[j], acc, 0, 0, 0);
-    }
-};
-
-// D: K steps whose operand tiles are on their way from global memory at any time (even, so that a step's LDS buffer
-// is the parity of its register stage; 16 registers per step).
-// EXACT: the number of K steps is a multiple of D, and the loop body has no branch at all: every iteration stores,
-// requests, reads and multiplies, the requests past the last step repeating the last step's (never used).  This is what
-// makes the depth real.  Loads return in order and a wait names how many may still be out, so when a request is issued
-// under a condition the compiler must assume it was not, and the wait before storing the oldest block then drains every
-// younger one as well: with `if (kt + D < nk)` around the requests the pipeline was one step deep whatever D said.
-// Without EXACT (an odd number of steps) the guarded form is used, with that cost.
-// CONV: the A operand of K step s is the 64 channels (s % (cin / 64)) * 64 .. of row m - (taps - 1) + s / (cin / 64).
-// The fields of GemmArgs as scalar arguments, in the order in which the kernel needs them: the first sixteen dwords of
-// scalar kernel arguments are in registers when a wavefront starts (the build asks for that), a structure passed by value
-// is fetched from memory.
-template <int EPI, int D, bool EXACT, bool CONV>
-__global__ void __launch_bounds__(kThreads)
-k_enc_gemm(const _Float16 *const a_arg, const _Float16 *const w_arg, const int M, const int N, const int K, const int taps, const int cin,
-           const int splits, float *const part, _Float16 *const out, _Float16 *const vt, const int width) {
-    GemmArgs g;
-    g.a = a_arg; g.w = w_arg; g.M = M; g.N = N; g.K = K; g.part = part; g.out = out; g.vt = vt; g.width = width;
-    g.taps = taps; g.cin = cin;
-    static_assert(D >= 2 && D % 2 == 0, "stage parity must equal step parity");
-    __shared__ __align__(16) _Float16 s_a[2][kTile * kLdsStride];
-    __shared__ __align__(16) _Float16 s_w[2][kTile * kLdsStride];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int m0 = blockIdx.y * kTile, n0 = blockIdx.x * kTile;
-    // staging: thread -> (row tid / 8 and + 32, 16-byte chunk tid % 8) of both tiles
-    const int srow = tid >> 3, schunk = tid & 7;
-    const int lda = CONV ? g.cin : g.K;
-    const u32x4 *ga0 = reinterpret_cast<const u32x4 *>(g.a + (ptrdiff_t)(m0 + srow) * lda) + schunk;
-    const u32x4 *ga1 = reinterpret_cast<const u32x4 *>(g.a + (ptrdiff_t)(m0 + srow + 32) * lda) + schunk;
-    const u32x4 *gw0 = reinterpret_cast<const u32x4 *>(g.w + (size_t)(n0 + srow) * g.K) + schunk;
-    const u32x4 *gw1 = reinterpret_cast<const u32x4 *>(g.w + (size_t)(n0 + srow + 32) * g.K) + schunk;
-    const int soff0 = srow * kLdsStride + schunk * 8, soff1 = (srow + 32) * kLdsStride + schunk * 8;
-
-    // K range of this workgroup (blockIdx.z splits K; only ENC_PARTIAL launches more than one split)
-    // (the K split is an argument among the first fourteen dwords, which are in registers at wavefront start; the grid's own
-    // dimensions would come out of memory, a round trip in front of the first request)
-    const int nk = g.K / kTile / splits;
-    const int kbase = (int)blockIdx.z * nk * (kTile / 8);   // in 16-byte chunks
-    gw0 += kbase; gw1 += kbase;
-    if constexpr (!CONV) { ga0 += kbase; ga1 += kbase; }
-    const int first_step = (int)blockIdx.z * nk;
-    const int steps_per_tap = CONV ? g.cin / kTile : 1;
-    const int row_chunks = lda / 8;   // 16-byte chunks per row of A
-
-    // Global -> register -> LDS -> register pipeline.  Step kt waits in register stage kt % D, is stored to LDS buffer
-    // kt % 2 one iteration before its products, and after that iteration's barrier its fragments are read into registers
-    // while the matrix instructions of step kt - 1 run from the other fragment set; the same stage then requests step
-    // kt + D.  A buffer is overwritten two steps after it was read: every wavefront has passed a barrier in between, which
-    // it reaches only with its LDS reads complete.  The products are issued in ascending K order.
-    StagedTiles st[D];
-    const int last = nk - 1;
-    const auto chunk_of = [&](int step) { return (step < last ? step : last) * (kTile / 8); };   // past the end: the last step again
-    // chunk offset of a step's A operand from ga0 / ga1: along the row, or (conv form) to an earlier row as well
-    const auto a_chunk_of = [&](int step) {
-        if constexpr (!CONV) return chunk_of(step);
-        else {
-            const int s = first_step + (step < last ? step : last);
-            const int tap = (s >= steps_per_tap ? 1 : 0) + (s >= 2 * steps_per_tap ? 1 : 0);   // taps <= 3
-            return (tap - (g.taps - 1)) * row_chunks + (s - tap * steps_per_tap) * (kTile / 8);
-        }
-    };
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-        if (EXACT || d < nk) st[d].load(ga0, ga1, gw0, gw1, a_chunk_of(d), chunk_of(d));
-
-    floatx16 acc = {0};
-    const int frag = (lane & 31) * kLdsStride + 8 * (lane >> 5);
-    const int fa_off = wm * 32 * kLdsStride + frag, fw_off = wn * 32 * kLdsStride + frag;
-    StepFragments fr[2];   // fragments of step kt in fr[kt % 2]
-    st[0].store(&s_a[0][0], &s_w[0][0], soff0, soff1);
-    if (EXACT || D < nk) st[0].load(ga0, ga1, gw0, gw1, a_chunk_of(D), chunk_of(D));
-    __syncthreads();
-    fr[0].read(&s_a[0][fa_off], &s_w[0][fw_off]);
-    // iteration kt: stage step kt + 1, barrier, read its fragments, multiply step kt
-    for (int base = 0; base < nk; base += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const int kt = base + d;
-            const int dn = (d + 1) % D;   // register stage of step kt + 1 (a constant after unrolling)
-            if constexpr (EXACT) {
-                st[dn].store(&s_a[(d + 1) & 1][0], &s_w[(d + 1) & 1][0], soff0, soff1);
-                st[dn].load(ga0, ga1, gw0, gw1, a_chunk_of(kt + 1 + D), chunk_of(kt + 1 + D));
-                __syncthreads();
-                fr[(d + 1) & 1].read(&s_a[(d + 1) & 1][fa_off], &s_w[(d + 1) & 1][fw_off]);
-                fr[d & 1].multiply(acc);
-            } else if (kt < nk) {   // the same for every thread of the grid
-                if (kt + 1 < nk) {
-                    st[dn].store(&s_a[(d + 1) & 1][0], &s_w[(d + 1) & 1][0], soff0, soff1);
-                    if (kt + 1 + D < nk) st[dn].load(ga0, ga1, gw0, gw1, a_chunk_of(kt + 1 + D), chunk_of(kt + 1 + D));
-                }
-                __syncthreads();
-                if (kt + 1 < nk) fr[(d + 1) & 1].read(&s_a[(d + 1) & 1][fa_off], &s_w[(d + 1) & 1][fw_off]);
-                fr[d & 1].multiply(acc);
-            }
-        }
-    }
-
-    const int n = n0 + wn * 32 + (lane & 31);
-    const int mbase = m0 + wm * 32;
+// What becomes of a wavefront's finished 32 x 32 piece (registers as acc_row has them): rows from mbase, this lane's column n.
+template <int EPI>
+__device__ __forceinline__ void finish_piece(const GemmArgs &g, const floatx16 &acc, int mbase, int n, int lane, int split) {
     if constexpr (EPI == ENC_PARTIAL) {
-        float *part = g.part + (size_t)blockIdx.z * g.M * g.N;
+        float *part = g.part + (size_t)split * g.M * g.N;
 #pragma unroll
         for (int r = 0; r < 16; ++r) part[(size_t)(mbase + acc_row(r, lane)) * g.N + n] = acc[r];
     } else if constexpr (EPI == ENC_GELU) {
@@ -268,6 +139,119 @@ k_enc_gemm(const _Float16 *const a_arg, const _Float16 *const w_arg, const int M
             }
         }
     }
+}
+
+// 64 lanes' 16 bytes from base + lane_bytes to consecutive LDS bytes from `lds` on (base and lds the same for the whole wavefront).
+__device__ __forceinline__ void global_to_lds(const void *base, unsigned lane_bytes, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(lane_bytes), "s"(base) : "memory", "m0");
+}
+
+// Waits until at most PER requests for each of the `left` steps behind this one (MOST at most) are out and this wavefront's LDS
+// reads are done, then (MEET) for the workgroup's other wavefronts.
+template <int PER, int MOST, bool MEET>
+__device__ __forceinline__ void step_arrived(int left) {
+    if (left >= MOST) {
+        if constexpr (MEET) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PER * MOST) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER * MOST) : "memory");
+    } else if constexpr (MOST > 0) {
+        step_arrived<PER, MOST - 1, MEET>(left);
+    }
+}
+
+// C tile of 32 * WM rows and 32 * WN columns, a wavefront 32 x 32 of it, K in steps of 64 through a ring of D stages in LDS.
+// The operands go from global memory straight to LDS, D - 2 steps ahead of their use: no registers, no LDS stores, one wait and one
+// barrier (none where a tile is one wavefront's) a step.  What bounds a launch at these sizes is how fast one CU gets its tile's rows
+// (some 64 KB in flight, a round trip for each such piece) and the step's own chain; through registers that was store, request,
+// barrier, read, multiply, on 64 x 64 tiles always.  us a prefill then / now, tokens: 20 211 / 176, 100 216 / 191, 192 223 / 208, 256 227 / 221,
+// 384 276 / 260, 512 315 / 287; three taps: 60 297 / 247, 128 294 / 255, 256 305 / 299, 400 414 / 392.
+// Iteration kt: wait for step kt, meet, request step kt + D - 2 (over step kt - 2, whose reads every wavefront has finished), read kt's
+// fragments, multiply step kt - 1 meanwhile.  A value's additions run over k in ascending order whatever the tile.
+// CONV: the A operand of K step s is the 64 channels (s % (cin / 64)) * 64 .. of row m - (taps - 1) + s / (cin / 64).
+// The fields of GemmArgs as scalar arguments, in the order in which the kernel needs them: the first fourteen dwords of
+// scalar kernel arguments are in registers when a wavefront starts (the build asks for that), a structure passed by value
+// is fetched from memory.
+template <int EPI, int WM, int WN, int D, bool CONV>
+__global__ void __launch_bounds__(64 * WM * WN)
+k_enc_gemm(const _Float16 *const a_arg, const _Float16 *const w_arg, const int M, const int N, const int K, const int steps, const int cin, const int taps,
+           float *const part, _Float16 *const out, _Float16 *const vt, const int width) {
+    GemmArgs g;
+    g.a = a_arg; g.w = w_arg; g.M = M; g.N = N; g.K = K; g.part = part; g.out = out; g.vt = vt; g.width = width;
+    g.taps = taps; g.cin = cin;
+    constexpr int kWaves = WM * WN, kRowBytes = kStep * 2, kTileA = 32 * WM * kRowBytes, kStage = kTileA + 32 * WN * kRowBytes;
+    constexpr int kAskA = 4 * WM / kWaves, kAskW = 4 * WN / kWaves;   // a wavefront's requests a step: eight rows of 128 bytes each
+    static_assert(D >= 4 && (kAskA + kAskW) * (D - 3) < 64, "the wait's counter ends at 63");
+    __shared__ __align__(16) unsigned char stages[D * kStage];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int wm = wave % WM, wn = wave / WM;
+    const int m0 = blockIdx.y * 32 * WM, n0 = blockIdx.x * 32 * WN, first = (int)blockIdx.z * steps;   // (blockIdx.z: the K split)
+    const int lda = CONV ? g.cin : g.K;
+    // LDS piece s of row r holds the row's 16-byte piece s ^ (r % 8): a request writes consecutive bytes, eight rows without padding,
+    // and the fragment reads of eight rows still lie on different banks.
+    const unsigned piece = (unsigned)((lane & 7) ^ (lane >> 3)) * 16;
+    const unsigned lane_a = (unsigned)(wave * kAskA * 8 + (lane >> 3)) * (unsigned)lda * 2 + piece;
+    const unsigned lane_w = (unsigned)(wave * kAskW * 8 + (lane >> 3)) * (unsigned)g.K * 2 + piece;
+    const unsigned char *const abase = reinterpret_cast<const unsigned char *>(g.a + (ptrdiff_t)m0 * lda);
+    const unsigned char *const wbase = reinterpret_cast<const unsigned char *>(g.w + (size_t)n0 * g.K) + (ptrdiff_t)first * kRowBytes;
+    const int steps_per_tap = CONV ? g.cin / kStep : 1;
+    const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)stages;
+    const auto request = [&](int step, int slot) {
+        const unsigned char *a;
+        if constexpr (!CONV) a = abase + (ptrdiff_t)(first + step) * kRowBytes;
+        else {
+            const int s = first + step, tap = (s >= steps_per_tap ? 1 : 0) + (s >= 2 * steps_per_tap ? 1 : 0);   // taps <= 3
+            a = abase + ((ptrdiff_t)(tap - (g.taps - 1)) * lda + (ptrdiff_t)(s - tap * steps_per_tap) * kStep) * 2;
+        }
+        const unsigned char *const w = wbase + (ptrdiff_t)step * kRowBytes;
+        const unsigned to_a = lds0 + slot * kStage + wave * kAskA * 1024, to_w = lds0 + slot * kStage + kTileA + wave * kAskW * 1024;
+#pragma unroll
+        for (int i = 0; i < kAskA; ++i) global_to_lds(a, lane_a + (unsigned)(i * 16 * lda), to_a + i * 1024);
+#pragma unroll
+        for (int i = 0; i < kAskW; ++i) global_to_lds(w, lane_w + (unsigned)(i * 16 * g.K), to_w + i * 1024);
+    };
+#pragma unroll
+    for (int d = 0; d < D - 2; ++d)
+        if (d < steps) request(d, d);
+
+    floatx16 acc = {0};
+    half8 fa[2][kStep / 16], fw[2][kStep / 16];   // fragments of step kt in set kt % 2
+    const int row = lane & 31, high = lane >> 5;
+    int slot = 0, next = D - 2;
+    const auto iteration = [&](int kt, int set) {
+        const int left = steps - 1 - kt;
+        step_arrived<kAskA + kAskW, D - 3, (kWaves > 1)>(left);
+        if (left >= D - 2) {
+            request(kt + D - 2, next);
+            next = next + 1 == D ? 0 : next + 1;
+        }
+        const unsigned char *const sa = stages + slot * kStage + (wm * 32 + row) * kRowBytes, *const sw = stages + slot * kStage + kTileA + (wn * 32 + row) * kRowBytes;
+        slot = slot + 1 == D ? 0 : slot + 1;
+#pragma unroll
+        for (int j = 0; j < kStep / 16; ++j) {
+            const int at = ((2 * j + high) ^ (row & 7)) * 16;
+            fa[set][j] = *reinterpret_cast<const half8 *>(sa + at);
+            fw[set][j] = *reinterpret_cast<const half8 *>(sw + at);
+        }
+        if (kt > 0) {
+#pragma unroll
+            for (int j = 0; j < kStep / 16; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[set ^ 1][j], fw[set ^ 1][j], acc, 0, 0, 0);
+        }
+    };
+    const auto last = [&](int set) {
+#pragma unroll
+        for (int j = 0; j < kStep / 16; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[set][j], fw[set][j], acc, 0, 0, 0);
+    };
+    int kt = 0;
+    for (; kt + 1 < steps; kt += 2) {
+        iteration(kt, 0);
+        iteration(kt + 1, 1);
+    }
+    if (kt < steps) {
+        iteration(kt, 0);
+        last(0);
+    } else {
+        last(1);
+    }
+    finish_piece<EPI>(g, acc, m0 + wm * 32, n0 + wn * 32 + (lane & 31), lane, (int)blockIdx.z);
 }
 
 // A lane's part of a row pass from here on: the LayerNorm of the row it holds in v (pieces past the row are zero), written as f16
@@ -624,6 +608,12 @@ __global__ void __launch_bounds__(kAttentionThreads) k_enc_attention(const _Floa
     }
 }
 
+template <int EPI, int WM, int WN, int D, bool CONV>
+void launch_gemm_tiles(State *st, const GemmArgs &g, int splits) {
+    hipLaunchKernelGGL((k_enc_gemm<EPI, WM, WN, D, CONV>), dim3(g.N / (32 * WN), g.M / (32 * WM), splits), dim3(64 * WM * WN), 0, st->stream, g.a, g.w, g.M, g.N,
+                       g.K, g.K / kStep / splits, g.cin, g.taps, g.part, g.out, g.vt, g.width);
+}
+
 template <int EPI, bool CONV = false>
 int launch_gemm(State *st, const GemmArgs &g, int splits, char *error, size_t capacity) {
     if (g.M % kTile != 0 || g.N % kTile != 0 || g.M <= 0 || g.N <= 0 || g.K <= 0 || splits < 1 || g.K % (kTile * splits) != 0 ||
@@ -632,15 +622,15 @@ int launch_gemm(State *st, const GemmArgs &g, int splits, char *error, size_t ca
         set_error(error, capacity, "encoder product: shape is not a multiple of the 64 x 64 x 64 tile");
         return -1;
     }
-    const int steps = g.K / kTile / splits;
-    const dim3 grid(g.N / kTile, g.M / kTile, splits), block(kThreads);
-    if (steps % kGemmDepth == 0)
-        hipLaunchKernelGGL((k_enc_gemm<EPI, kGemmDepth, true, CONV>), grid, block, 0, st->stream, g.a, g.w, g.M, g.N, g.K, g.taps, g.cin, splits, g.part, g.out,
-                           g.vt, g.width);
-    else if (steps % 2 == 0)
-        hipLaunchKernelGGL((k_enc_gemm<EPI, 2, true, CONV>), grid, block, 0, st->stream, g.a, g.w, g.M, g.N, g.K, g.taps, g.cin, splits, g.part, g.out, g.vt, g.width);
-    else
-        hipLaunchKernelGGL((k_enc_gemm<EPI, 2, false, CONV>), grid, block, 0, st->stream, g.a, g.w, g.M, g.N, g.K, g.taps, g.cin, splits, g.part, g.out, g.vt, g.width);
+    // The smallest tile that still puts no more than about a workgroup on a CU: fewer rows to fetch for each (98, 147 or 196 KB at
+    // twelve steps), while a second round costs more than that.  us a launch (12 steps, weights no cache holds) with 32 x 32 / 64 x 32 /
+    // 64 x 64 tiles, in brackets their workgroups: FFN up, 64 rows 5.1 (192) / 5.5 / 6.6; 128 5.8 (384) / 5.7 (192) / 6.4; 192 10.0
+    // / 6.4 (288) / 6.5 (144); 256 - / 6.7 (384) / 6.4 (192).  Deeper rings than these leave a CU one workgroup where two are wanted (64 x 64 with
+    // six stages at 512 rows: 11.0 against 8.4), shallower ones wait for weights (FFN up, 64 x 64 with four stages: 7.2 against 6.4).
+    const int small = g.M / 32 * (g.N / 32) * splits, middle = g.M / 64 * (g.N / 32) * splits, most = st->cu_count + st->cu_count / 4;
+    if (small <= most) launch_gemm_tiles<EPI, 1, 1, 7, CONV>(st, g, splits);
+    else if (middle <= most) launch_gemm_tiles<EPI, 2, 1, 6, CONV>(st, g, splits);
+    else launch_gemm_tiles<EPI, 2, 2, 5, CONV>(st, g, splits);
     return hip_check(hipGetLastError(), "encoder product launch", error, capacity);
 }
 
@@ -681,10 +671,9 @@ int tap_major_f16(State *st, const float *host, size_t n, size_t cin, size_t tap
 size_t attention_lds_bytes(size_t tpad) { return std::max((size_t)kQTile * (tpad + kScorePad), (size_t)3 * 32 * 64) * sizeof(float); }
 
 constexpr int kMaxSplits = 4;   // k_enc_rows reads exactly this many partial planes at most
-// Most splits that leave each workgroup at least three K steps, preferring a step count the products' pipeline takes
-// without guards: a multiple of its depth, else an even one.
+// Most splits that leave each workgroup at least three K steps, preferring a step count that is a multiple of four, else an even one.
 int pick_splits(int k) {
-    for (const int multiple : {kGemmDepth, 2, 1})
+    for (const int multiple : {4, 2, 1})
         for (int s = kMaxSplits; s > 1; --s)
             if (k % (kTile * s) == 0 && k / (kTile * s) >= 3 && (k / (kTile * s)) % multiple == 0) return s;
     return 1;

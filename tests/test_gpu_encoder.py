@@ -206,6 +206,20 @@ def test_encoder_f32_operands_match_oracle(pkg, backend, orc, synth, nerr, causa
     assert nerr(half, got) < 2e-3
 
 
+@pytest.mark.parametrize("tokens,width,ffn,kernel", [(64, 768, 3072, 1), (192, 768, 3072, 3), (448, 768, 3072, 1), (512, 768, 3072, 3), (64, 192, 192, 3),
+                                                     (129, 192, 320, 1), (512, 320, 704, 3), (320, 1152, 576, 1)])
+def test_encoder_f16_product_tiles(pkg, backend, orc, synth, nerr, tokens, width, ffn, kernel):
+    """The products' tiles follow from how many workgroups each makes: lengths and widths on both sides of the lines, K loops of 1 to 36 steps, odd
+    ones among them, rings longer than the loop.  One layer: the bound of this file, 2e-3."""
+    _announce("encoder product tiles tokens=%d width=%d ffn=%d kernel=%d" % (tokens, width, ffn, kernel))
+    cfg = dict(synth.encoder_config(layers=1, width=width, heads=width // 64, ffn=ffn, vocab=300, max_positions=512), causal=True, ffn_kernel=kernel)
+    w = synth.encoder_weights_f16(cfg, seed=71, kernel=kernel, biases=True)
+    ids = np.random.default_rng(72).integers(0, cfg["vocab"], size=tokens).astype(np.int32)
+    got = _prefill(pkg, backend, cfg, w, ids)
+    _, want = orc.encoder_prefill(cfg, _f16_bits(w), ids)
+    assert nerr(got, want) < 2e-3
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("tokens", [64, 65, 128, 129, 256, 257, 513, 1000])
 def test_encoder_f16_attention_key_counts(pkg, backend, orc, synth, nerr, tokens, causal):
