@@ -1245,11 +1245,17 @@ extern "C" int mynah_hip_cross_kv_dev(void *opaque, const float *dev_memory, siz
     // product.  One layer's product is 36 tiles of work on 256 CUs and its LayerNorm a launch as long: 12 layers of 180 rows
     // took 36 launches and 630 us one after the other.
     const bool grouped = memory_length > kQuantMaxRows && width % 64 == 0 && xattn_width % 32 == 0 && memory_length <= 0x10000 && width <= 0x10000 && xattn_width <= 0x10000;
-    const size_t group = grouped ? (layers < kSplitMaxLayers ? layers : kSplitMaxLayers) : 1;
+    // Up to kQuantMaxRows rows take the current storage's matvecs; where one launch takes a list of them, every layer in two launches as
+    // well (twelve f32 layers, us a call, a LayerNorm and two products a layer one by one / this: 8 rows 150 / 27, 12 245 / 29, 16 249 / 31; the same bits).
+    const bool listed = !grouped && memory_length <= kQuantMaxRows && width <= 0x10000 && xattn_width <= 0x10000 &&
+                        linear_takes_list(st->qtype, (int)xattn_width, (int)width, (int)memory_length, width, xattn_width);
+    const size_t group = grouped || listed ? (layers < kSplitMaxLayers ? layers : kSplitMaxLayers) : 1;
     // The normalised rows live in a buffer the backend keeps and grows: one allocation per call would add up between
     // synchronisations when a caller prepares many utterances in a row.  An outgrown buffer may still be read by earlier
     // launches: it waits in the list that the next idle stream frees (bounded like mynah_hip_dev_free's).
-    const size_t norm_floats = group * memory_length * width + kSplitOverrun;
+    constexpr size_t kListFloats = sizeof(CrossProducts) / sizeof(float);   // the table of a list of products lies in front of the rows
+    static_assert(kListFloats % 64 == 0, "the rows keep the allocation's alignment");
+    const size_t norm_floats = kListFloats + group * memory_length * width + kSplitOverrun;
     if (st->cross_norm_floats < norm_floats) {
         if (st->cross_norm != nullptr) {
             st->pending_free.push_back(st->cross_norm);
@@ -1260,7 +1266,8 @@ extern "C" int mynah_hip_cross_kv_dev(void *opaque, const float *dev_memory, siz
         MYNAH_TRY(hipMalloc(reinterpret_cast<void **>(&st->cross_norm), norm_floats * sizeof(float)));
         st->cross_norm_floats = norm_floats;
     }
-    float *const normed = st->cross_norm;
+    LinearProduct *const list = reinterpret_cast<LinearProduct *>(st->cross_norm);
+    float *const normed = st->cross_norm + kListFloats;
     const size_t per_layer = memory_length * xattn_width;
     for (size_t l0 = 0; l0 < layers; l0 += group) {
         const size_t count = layers - l0 < group ? layers - l0 : group;
@@ -1275,6 +1282,34 @@ extern "C" int mynah_hip_cross_kv_dev(void *opaque, const float *dev_memory, siz
                                       dev_cross_v + l0 * per_layer, error, capacity) != 0)
                 return -1;
             continue;
+        }
+        if (listed) {
+            LinearArgs first{};
+            CrossProducts products{};
+            bool alike = true;
+            for (size_t p = 0; p < 2 * count && alike; ++p) {   // layer p / 2: its K half, its V half
+                const size_t layer = l0 + p / 2;
+                const CachedWeight *cw = nullptr;
+                if (cached_matrix(st, kv_w[layer] + (p % 2) * xattn_width * width, xattn_width, width, st->qtype, &cw, error, capacity) != 0) return -1;
+                const float *const in = normed + p / 2 * memory_length * width;
+                float *const out = (p % 2 != 0 ? dev_cross_v : dev_cross_k) + layer * per_layer;
+                if (p == 0) {
+                    first.w = cw->data; first.scales = cw->scales; first.qtype = cw->qtype; first.arith = st->arith; first.epilogue = EPI_NONE;
+                    first.n = (int)xattn_width; first.k = (int)width; first.batch = (int)memory_length;
+                    for (size_t b = 0; b < memory_length && b < (size_t)kBatchTile; ++b) { first.in[b] = in + b * width; first.out[b] = out + b * xattn_width; }
+                }
+                alike = cw->qtype == first.qtype;   // (a matrix that the storage cannot hold is kept as f32)
+                products.of[p] = LinearProduct{static_cast<const char *>(cw->data) - static_cast<const char *>(first.w), cw->scales - first.scales,
+                                               in - first.in[0], out - first.out[0]};
+            }
+            if (alike) {
+                if (launch_cross_norms(st, dev_memory, memory_length, width, table, count, normed, &products, list, error, capacity) != 0 ||
+                    launch_linear_products(st, first, list, (int)(2 * count), error, capacity) != 0)
+                    return -1;
+                continue;
+            }
+            set_error(error, capacity, "cross K/V: weights of one shape in different storages");
+            return -1;
         }
         if (launch_layernorm(st, dev_memory, normed, table.gain[0], table.bias[0], memory_length, width, error, capacity) != 0) return -1;
         if (matmul_device(st, normed, dev_cross_k + l0 * per_layer, memory_length, width, xattn_width, kv_w[l0], nullptr, error, capacity) != 0) return -1;

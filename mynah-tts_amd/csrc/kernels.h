@@ -49,6 +49,13 @@ int launch_linear(State *st, const LinearArgs &args, char *error, size_t capacit
 bool linear_takes_all(int n, int k, int epilogue, bool layernorm, size_t in_stride, size_t out_stride);   // strides in floats
 // Whether launch_linear takes such a product with the fold for more than two streams (rows one behind the other, residual epilogue).
 bool linear_folds_streams(int n, int k, int heads, int max_units);
+// Products of one shape and storage in one launch: product i's weight, scales, first input and output row lie at these distances from
+// the ones in `first` (bytes of packed weight, floats).  list: device memory, `products` entries.  The rows as linear_takes_list asks.
+struct LinearProduct {
+    ptrdiff_t w, scales, in, out;
+};
+bool linear_takes_list(int qtype, int n, int k, int rows, size_t in_stride, size_t out_stride);
+int launch_linear_products(State *st, const LinearArgs &first, const LinearProduct *list, int products, char *error, size_t capacity);
 // Any shape, f32 weights: out[r,n] = in[r,k] W[n,k]^T + bias (rows may be large).
 int launch_gemm_f32(State *st, const float *in, float *out, size_t rows, size_t k, size_t n, const float *w,
                     const float *bias, char *error, size_t capacity);
@@ -71,6 +78,13 @@ int split_product_splits(const State *st, size_t rows, size_t channels, size_t n
 // part[z][rows][n] = split z's share of in[rows][channels] * W (taps == 3: causal convolution, two rows in front of `in` are zeros).
 int launch_split_product(State *st, const float *in, const float4 *w, size_t rows, size_t channels, size_t taps, size_t n, int splits, float *part,
                          char *error, size_t capacity);
+// The first launch of either form of the cross K/V: every layer's LayerNorm of the rows to normed[layer][row].  list (may be null): the
+// table of the products behind it, 2 * count entries, leaves with the launch.
+struct CrossProducts {
+    LinearProduct of[2 * kSplitMaxLayers];
+};
+int launch_cross_norms(State *st, const float *memory, size_t rows, size_t width, const SplitLayers &layers, size_t count, float *normed,
+                       const CrossProducts *products, LinearProduct *list, char *error, size_t capacity);
 // normed: [count][rows][width] floats (+ kSplitOverrun); k_out / v_out: [count][rows][xw].
 int launch_split_cross_kv(State *st, const float *memory, size_t rows, size_t width, const SplitLayers &layers, size_t count, size_t xw, float *normed,
                           float *k_out, float *v_out, char *error, size_t capacity);

@@ -53,7 +53,9 @@ __device__ __forceinline__ float *stream_out(const LinearArgs &a, int b) {
 // GELU epilogue (the step's FFN-up projection).  SPEC_PLAIN: the product alone (the local frame's vocabulary projections).
 // SPEC_SIDE (with one of the two, one stream to a workgroup): the launch takes several streams side by side, one to each row of the grid
 // (launch_linear_b); a build of its own, so that a lone stream does not wait for the arithmetic that finds a row.
-enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2, SPEC_PLAIN = 3, SPEC_SIDE = 4 };
+// SPEC_LIST (with SPEC_PLAIN, more than two rows): several products of one shape in one launch, the grid's third dimension naming them
+// (launch_linear_products).
+enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2, SPEC_PLAIN = 3, SPEC_SIDE = 4, SPEC_LIST = 8 };
 
 // More than two streams: one wavefront stages one stream (load_stream_row / finish_stream_row,
 // device_common.h) -- staging every stream's activations is what such a launch spends most of its time on, every workgroup
@@ -146,7 +148,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
     // these are what the first requests are formed from.
     // (Only for one or two streams: with more, the rows of a.in and a.out are picked by a run-time index, and a structure that
     // has been written to is then kept in scratch memory -- the eight-stream matvecs took 20 us instead of 4.5.)
-    constexpr int SPEC = BUILD & ~SPEC_SIDE;
+    constexpr int SPEC = BUILD & 3;
     static_assert(64 + sizeof(LinearArgs) > 0x100 + 4, "the warmed lines lie inside the kernel arguments");
     constexpr bool kStrided = kStridedLead<BT, SPEC>;
     WarmArguments warm{0u, 0u, 0u, 0u};
@@ -174,6 +176,14 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
         a.fold_heads = 0; a.fold_head_width = 0; a.fold_max_units = 0; a.fold_is_self = 0; a.fold_stream0 = 0;
         if constexpr (SPEC == SPEC_UP) {
             a.ln_gain = fold_partial; a.ln_bias = fold_partial_ml;
+        }
+        if constexpr ((BUILD & SPEC_LIST) != 0) {
+            // (distances from the first product's places, so that every address stays one of a kernel argument's)
+            const LinearProduct at = reinterpret_cast<const LinearProduct *>(fold_partial)[blockIdx.z];
+            a.w = static_cast<const unsigned char *>(w) + at.w;
+            a.scales = scales + at.scales;
+            in_base += at.in;
+            out_base += at.out;
         }
     }
     if constexpr (kPackedLead<BT, SPEC>) {
@@ -623,14 +633,14 @@ static bool stream_groups_enabled() {
 }
 
 template <int QT, int BT, int NVT, int KFIX, int BUILD>
-int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity) {
-    constexpr int SPEC = BUILD & ~SPEC_SIDE;
+int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity, const LinearProduct *list = nullptr, int products = 1) {
+    constexpr int SPEC = BUILD & 3;
     constexpr int epc = Chunk<QT>::n;
     const int chunks = a.k / epc;
     const int lg = lane_group_log2(chunks);
     const int rows_per_wg_pass = 4 * (64 >> lg);
     const int target_wgs = st->cu_count * 3;
-    int passes = (a.n + rows_per_wg_pass * target_wgs - 1) / (rows_per_wg_pass * target_wgs);
+    int passes = (int)(((long)a.n * products + rows_per_wg_pass * target_wgs - 1) / (rows_per_wg_pass * target_wgs));
     if (passes < 1) passes = 1;
     // Builds that take more streams than their tile holds: groups of BT side by side (the grid's second dimension).
     const int groups = kStridedLead<BT, SPEC> || (BUILD & SPEC_SIDE) != 0 ? (a.batch + BT - 1) / BT : 1;
@@ -659,8 +669,8 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
             return -1;
         }
         const StepSlots *const packed = reinterpret_cast<const StepSlots *>(pack_strided(shape));
-        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, BUILD>), dim3(grid, groups), dim3(kLinearThreads<BT>), lds, st->stream, a.in[0],
-                           SPEC == SPEC_UP ? a.ln_gain : nullptr, SPEC == SPEC_UP ? a.ln_bias : nullptr, packed, a.w, a.scales, a.out[0], a.n, a.batch, a,
+        hipLaunchKernelGGL((k_linear<QT, BT, NVT, KFIX, BUILD>), dim3(grid, groups, products), dim3(kLinearThreads<BT>), lds, st->stream, a.in[0],
+                           SPEC == SPEC_UP ? a.ln_gain : reinterpret_cast<const float *>(list), SPEC == SPEC_UP ? a.ln_bias : nullptr, packed, a.w, a.scales, a.out[0], a.n, a.batch, a,
                            rows_per_wg, lg);
     } else if constexpr (kPackedLead<BT, SPEC>) {
         // the launch's small numbers in the slot table pointer's place, and what the free pointer places carry (see the kernel)
@@ -757,6 +767,12 @@ int launch_linear_q(State *st, const LinearArgs &a, char *error, size_t capacity
     return launch_linear_b<QT, 3, 0, SPEC_ANY>(st, a, error, capacity);
 }
 
+template <int QT>
+int launch_linear_list(State *st, const LinearArgs &a, const LinearProduct *list, int products, char *error, size_t capacity) {
+    if (a.batch <= 4) return launch_linear_t<QT, 4, 1, 768, SPEC_PLAIN | SPEC_LIST>(st, a, error, capacity, list, products);
+    return launch_linear_t<QT, 8, 1, 768, SPEC_PLAIN | SPEC_LIST>(st, a, error, capacity, list, products);
+}
+
 }  // namespace
 
 bool linear_fast_supported(int qtype, size_t n, size_t k) {
@@ -777,6 +793,26 @@ bool linear_takes_all(int n, int k, int epilogue, bool layernorm, size_t in_stri
     if (!strided_fits(s) || out_stride == 0) return false;
     if (epilogue == EPI_RESIDUAL) return !layernorm && (k == 768 || k == 3072);
     return k == 768 && epilogue == (layernorm ? EPI_GELU : EPI_NONE);
+}
+
+bool linear_takes_list(int qtype, int n, int k, int rows, size_t in_stride, size_t out_stride) {
+    return rows > kConsumerFoldMaxBatch && rows <= kMaxBatch && linear_fast_supported(qtype, (size_t)n, (size_t)k) &&
+           linear_takes_all(n, k, EPI_NONE, false, in_stride, out_stride);
+}
+
+int launch_linear_products(State *st, const LinearArgs &a, const LinearProduct *list, int products, char *error, size_t capacity) {
+    size_t in_stride = 0, out_stride = 0;
+    if (products < 1 || products > 65535 || list == nullptr || a.bias != nullptr || a.ln_gain != nullptr || a.epilogue != EPI_NONE ||
+        !rows_strided(a, &in_stride, &out_stride) || !linear_takes_list(a.qtype, a.n, a.k, a.batch, in_stride, out_stride)) {
+        set_error(error, capacity, "linear: products that do not go in one launch");
+        return -1;
+    }
+    switch (a.qtype) {
+        case MYNAH_HIP_F32: return launch_linear_list<MYNAH_HIP_F32>(st, a, list, products, error, capacity);
+        case MYNAH_HIP_F16: return launch_linear_list<MYNAH_HIP_F16>(st, a, list, products, error, capacity);
+        case MYNAH_HIP_INT8: return launch_linear_list<MYNAH_HIP_INT8>(st, a, list, products, error, capacity);
+        default: return launch_linear_list<MYNAH_HIP_INT4>(st, a, list, products, error, capacity);
+    }
 }
 
 int launch_linear(State *st, const LinearArgs &a, char *error, size_t capacity) {

@@ -258,7 +258,28 @@ __global__ void __launch_bounds__(256) k_layernorm_layers(const float *in, float
     layernorm_row(in + (size_t)row * width, normed + ((size_t)layer * rows + row) * width, layers.gain[layer], layers.bias[layer], width, s4);
 }
 
+// The same, and the table of the products that follow, which the first workgroup leaves in device memory: what changes from call to call
+// arrives as arguments, and nothing is copied.
+__global__ void __launch_bounds__(256) k_layernorm_products(const float *in, float *normed, const SplitLayers layers, int rows, int width,
+                                                            LinearProduct *list, const CrossProducts products, int count) {
+    __shared__ float s4[4];
+    const int row = (int)blockIdx.x, layer = (int)blockIdx.y;
+    if (row == 0 && layer == 0 && (int)threadIdx.x < count) list[threadIdx.x] = products.of[threadIdx.x];
+    layernorm_row(in + (size_t)row * width, normed + ((size_t)layer * rows + row) * width, layers.gain[layer], layers.bias[layer], width, s4);
+}
+
 }  // namespace
+
+int launch_cross_norms(State *st, const float *memory, size_t rows, size_t width, const SplitLayers &layers, size_t count, float *normed,
+                       const CrossProducts *products, LinearProduct *list, char *error, size_t capacity) {
+    static_assert(2 * kSplitMaxLayers <= 256, "a thread an entry of the table");
+    const dim3 grid((unsigned)rows, (unsigned)count);
+    if (list != nullptr)
+        hipLaunchKernelGGL(k_layernorm_products, grid, dim3(256), 0, st->stream, memory, normed, layers, (int)rows, (int)width, list, *products, (int)(2 * count));
+    else
+        hipLaunchKernelGGL(k_layernorm_layers, grid, dim3(256), 0, st->stream, memory, normed, layers, (int)rows, (int)width);
+    return hip_check(hipGetLastError(), "cross K/V LayerNorm launch", error, capacity);
+}
 
 int launch_split_pack(State *st, const float *src, float4 *dst, size_t n, size_t channels, size_t taps, char *error, size_t capacity) {
     const size_t pieces = n * channels * taps / 4;
@@ -307,7 +328,7 @@ int launch_split_product(State *st, const float *in, const float4 *w, size_t row
 
 int launch_split_cross_kv(State *st, const float *memory, size_t rows, size_t width, const SplitLayers &layers, size_t count, size_t xw, float *normed,
                           float *k_out, float *v_out, char *error, size_t capacity) {
-    hipLaunchKernelGGL(k_layernorm_layers, dim3((unsigned)rows, (unsigned)count), dim3(256), 0, st->stream, memory, normed, layers, (int)rows, (int)width);
+    if (launch_cross_norms(st, memory, rows, width, layers, count, normed, nullptr, nullptr, error, capacity) != 0) return -1;
     const int mtiles = (int)((rows + 63) / 64), ntiles = (int)((2 * xw + 127) / 128);
     hipLaunchKernelGGL(k_split_cross_kv, dim3((unsigned)((ntiles * (int)count + 7) / 8 * 8 * mtiles)), dim3(512), 0, st->stream, normed, layers,
                        (int)rows, (int)width, (int)xw, mtiles, (int)count, k_out, v_out);

@@ -53,6 +53,37 @@ def test_cross_kv_layers_together(backend, pkg, rows, xw, layers):
         d.free()
 
 
+@pytest.mark.parametrize("storage", ["F32", "F16", "INT8", "INT4"])
+@pytest.mark.parametrize("rows,xw,layers", [(3, 768, 2), (4, 36, 1), (5, 96, 34), (8, 768, 1), (9, 768, 3), (16, 160, 2)])
+def test_cross_kv_few_rows_as_a_list(backend, pkg, storage, rows, xw, layers):
+    """Three to sixteen rows of width 768: every layer's products in one launch (more than 32 layers: two).  A row's values are those of a call
+    for that row and layer alone, which takes the matvecs one by one, bit for bit."""
+    print("[gpu-case] cross K/V list %s rows=%d xw=%d layers=%d" % (storage, rows, xw, layers), flush=True)
+    rng, width = np.random.default_rng(rows + layers), 768
+    backend.set_quant(getattr(pkg, storage))
+    try:
+        gains = [backend.keep((1.0 + 0.1 * rng.standard_normal(width)).astype(np.float32)) for _ in range(layers)]
+        biases = [backend.keep((0.02 * rng.standard_normal(width)).astype(np.float32)) for _ in range(layers)] if rows % 2 else None
+        kvw = [backend.keep(rng.standard_normal((2 * xw, width)).astype(np.float32)) for _ in range(layers)]
+        dmem = backend.alloc(rows * width).write(rng.standard_normal((rows, width)).astype(np.float32))
+        guard = np.full(xw, 7.0, np.float32)
+        dk, dv = (backend.alloc(layers * rows * xw + xw).write(guard, layers * rows * xw) for _ in range(2))
+        one_k, one_v = (backend.alloc(xw) for _ in range(2))
+        for _ in range(2):
+            backend.cross_kv_dev(dmem.ptr, rows, width, gains, biases, kvw, xw, dk.ptr, dv.ptr)
+        k, v = dk.read(), dv.read()
+        assert np.array_equal(k[-xw:], guard) and np.array_equal(v[-xw:], guard)
+        k, v = k[:-xw].reshape(layers, rows, xw), v[:-xw].reshape(layers, rows, xw)
+        for l in sorted({0, layers // 2, layers - 1}):
+            for r in range(rows):
+                backend.cross_kv_dev(dmem.ptr + 4 * r * width, 1, width, [gains[l]], [biases[l]] if biases else None, [kvw[l]], xw, one_k.ptr, one_v.ptr)
+                assert np.array_equal(one_k.read(), k[l, r]) and np.array_equal(one_v.read(), v[l, r]), (l, r)
+        for d in (dmem, dk, dv, one_k, one_v):
+            d.free()
+    finally:
+        backend.set_quant(pkg.F32)
+
+
 @pytest.mark.parametrize("kernel", [1, 3])
 @pytest.mark.parametrize("tokens", [31, 32, 33, 64, 65, 97])
 def test_encoder_f32_tiles(backend, pkg, orc, synth, nerr, kernel, tokens):
