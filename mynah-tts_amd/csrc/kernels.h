@@ -64,9 +64,9 @@ int launch_sgemm(State *st, int ta, int tb, size_t m, size_t n, size_t k, float 
 
 // Many-row f32 products on the bf16 matrix cores (split_product.hip).  Weights packed by launch_split_pack (cached_split_weight);
 // n a multiple of 32, channels of 64; the rows may be read up to kSplitOverrun floats past their end.
-constexpr size_t kSplitOverrun = 256;
+constexpr size_t kSplitOverrun = 384;   // three blocks of 16 channels for each of eight groups
 constexpr int kConvStepsAhead = 3;   // steps (3 KiB) of a packed convolution weight that are requested ahead of the one multiplied
-constexpr size_t kSplitWeightOverrun = 64 * 1024;   // bytes behind a packed weight that may be requested (never used)
+constexpr size_t kSplitWeightOverrun = 64 * 1024;   // bytes behind a packed weight that may be requested (never used): 48 KiB with eight groups, three taps
 constexpr size_t kSplitMaxLayers = 32;
 struct SplitLayers {
     const float4 *w[kSplitMaxLayers];

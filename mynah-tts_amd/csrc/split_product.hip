@@ -34,7 +34,7 @@ __global__ void __launch_bounds__(256) k_split_pack(const float *src, float4 *ds
 template <int MT, int TAPS, int G>
 struct SplitTile {
     static constexpr int kRows = 32 * MT + (TAPS - 1), kPitch = (kRows + 11) / 16 * 16 + 4;
-    static_assert(kPitch >= kRows && kPitch % 16 == 4 && (G == 2 || G == 4), "bank layout");
+    static_assert(kPitch >= kRows && kPitch % 16 == 4 && (G == 2 || G == 4 || G == 8), "bank layout");
     union {
         uint4 a[3][G][3][2][kPitch];
         float sums[8 - 8 / G][MT][16][64];
@@ -303,6 +303,19 @@ int split_product_splits(const State *st, size_t rows, size_t channels, size_t n
     return (int)best;
 }
 
+// Groups of wavefronts over the channels: the most, and so the narrowest tile (256 / groups columns), that still give every workgroup a CU of
+// its own.  What bounds these launches is how fast a CU gets its piece of the weight, and few rows make few workgroups: with four groups a
+// workgroup has half the piece, with eight (tiles of 32 rows) a quarter.  us a prefill of six layers with two groups (four in the unsplit
+// QKV product) / this, one tap: 20 rows 292 / 274, 60 325 / 308, 96 344 / 332; three taps: 20 350 / 318, 60 386 / 351, 96 410 / 398.  A quarter more
+// workgroups than CUs instead: 303, 325, 353 and 341, 380, 448.
+// A sum is then more and shorter chains of additions: the prefill's error against double precision (2-norm) 4.5e-7 / 3.7e-7 at 20 rows, 4.5e-7 /
+// 3.9e-7 at 50 with one tap, 6.3e-7 / 5.4e-7 and 6.6e-7 / 5.6e-7 with three.
+static int split_groups(const State *st, size_t mt, size_t mtiles, size_t channels, size_t n, size_t splits) {
+    for (size_t groups = mt == 1 ? 8 : 4; groups > 2; groups /= 2)
+        if (channels % (16 * groups * kBlocksAhead * splits) == 0 && (n * groups + 255) / 256 * mtiles * splits <= (size_t)st->cu_count) return (int)groups;
+    return 2;
+}
+
 int launch_split_product(State *st, const float *in, const float4 *w, size_t rows, size_t channels, size_t taps, size_t n, int splits, float *part,
                          char *error, size_t capacity) {
     if (rows == 0 || n == 0 || n % 32 != 0 || channels == 0 || splits < 1 || channels % (32 * kBlocksAhead * (size_t)splits) != 0 || (taps != 1 && taps != 3) ||
@@ -311,18 +324,19 @@ int launch_split_product(State *st, const float *in, const float4 *w, size_t row
         return -1;
     }
     const int mt = split_row_tiles(st, rows, n, splits > 1), mtiles = (int)((rows + 32 * mt - 1) / (32 * mt));
-    // An unsplit product of 32-row tiles, where that still gives every workgroup a CU of its own: 64 columns a workgroup and four groups of
-    // wavefronts over the channels, twice the workgroups with half the chain.  us a launch, 768 -> 2304 by 64 / 128 columns: 16 rows 9.8 / 14.2,
-    // 96 9.8 / 14.1, 192 10.4 / 14.1, 224 13.8 / 14.1.
-    const bool deep = mt == 1 && taps == 1 && splits == 1 && channels % 128 == 0 && (n + 63) / 64 * mtiles <= (size_t)st->cu_count;
-    const int ntiles = (int)((n + (deep ? 63 : 127)) / (deep ? 64 : 128));
+    const int groups = split_groups(st, (size_t)mt, (size_t)mtiles, channels, n, (size_t)splits);
+    const int wide = 256 / groups, ntiles = (int)((n + wide - 1) / wide);
     const dim3 grid((unsigned)((ntiles * splits + 7) / 8 * 8 * mtiles)), block(512);
     const auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, block, 0, st->stream, in, w, (int)rows, (int)n, (int)channels, mtiles, ntiles, splits, part);
     };
-    if (deep) launch(k_split_rows<1, 1, 4>);
-    else if (taps == 1) mt == 1 ? launch(k_split_rows<1, 1, 2>) : launch(k_split_rows<2, 1, 2>);
-    else mt == 1 ? launch(k_split_rows<1, 3, 2>) : launch(k_split_rows<2, 3, 2>);
+    if (taps == 1) {
+        if (mt == 1) groups == 8 ? launch(k_split_rows<1, 1, 8>) : groups == 4 ? launch(k_split_rows<1, 1, 4>) : launch(k_split_rows<1, 1, 2>);
+        else groups == 4 ? launch(k_split_rows<2, 1, 4>) : launch(k_split_rows<2, 1, 2>);
+    } else {
+        if (mt == 1) groups == 8 ? launch(k_split_rows<1, 3, 8>) : groups == 4 ? launch(k_split_rows<1, 3, 4>) : launch(k_split_rows<1, 3, 2>);
+        else groups == 4 ? launch(k_split_rows<2, 3, 4>) : launch(k_split_rows<2, 3, 2>);
+    }
     return hip_check(hipGetLastError(), "f32 product launch", error, capacity);
 }
 

@@ -261,6 +261,19 @@ def test_encoder_f32_wide_and_deep_products(pkg, backend, orc, synth, nerr, toke
 
 
 @pytest.mark.parametrize("kernel", [1, 3])
+@pytest.mark.parametrize("tokens,width,ffn", [(1, 256, 512), (32, 256, 256), (20, 768, 3072), (33, 768, 3072), (64, 768, 1536), (65, 512, 1024), (100, 768, 768)])
+def test_encoder_f32_channel_groups(pkg, backend, orc, synth, nerr, tokens, width, ffn, kernel):
+    """Few rows: the products' wavefronts in two, four or eight groups over the channels (tiles of 128, 64 or 32 columns), split and not."""
+    _announce("encoder f32 channel groups tokens=%d width=%d ffn=%d kernel=%d" % (tokens, width, ffn, kernel))
+    cfg = dict(synth.encoder_config(layers=1, width=width, heads=width // 64, ffn=ffn, vocab=300, max_positions=128), causal=True, ffn_kernel=kernel)
+    w = synth.encoder_weights_f16(cfg, seed=81, kernel=kernel, biases=True)
+    ids = np.random.default_rng(82).integers(0, cfg["vocab"], size=tokens).astype(np.int32)
+    got = _prefill_f32(pkg, backend, cfg, w, ids)
+    _, want = orc.encoder_prefill(cfg, _f16_bits(w), ids)
+    assert nerr(got, want) < 1e-5
+
+
+@pytest.mark.parametrize("kernel", [1, 3])
 def test_encoder_f32_operands_match_the_reference_fixture(pkg, backend, synth, nerr, kernel):
     """Against the committed outputs of the compiled reference's transformer_stack, both builds, at the f32 bar."""
     from tests.golden import make_golden as mg
