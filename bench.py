@@ -270,10 +270,10 @@ def time_codec(pkg, backend, frames=64, runs=4, warmup=2):
 # (with one or two streams the attention partials are folded by the output projection that follows; with more, by
 # workgroups of the attention launch itself, and the stage timing of those launches includes, per twelve launches, the two
 # small launches that give the step its counter)
-STAGES = [("self-attention", "k_step_attention<self>", "LayerNorm + int8 act-quant + per-head Q/K/V rows + KV append + attention over the self cache (+ fold of the partials when more than two streams)"),
-          ("self-out", "k_linear<k=768, residual>", "(fold of attention partials, up to two streams) + act-quant + O matvec + residual"),
-          ("cross-attention", "k_step_attention<cross>", "LayerNorm + act-quant + per-head Q rows + attention over the cross cache (+ fold when more than two streams)"),
-          ("cross-out", "k_linear<k=768, residual>", "(fold, up to two streams) + act-quant + O matvec + residual"),
+STAGES = [("self-attention", "k_step_attention<self>", "LayerNorm + int8 act-quant + per-head Q/K/V rows + KV append + attention over the self cache (+ fold of the partials where the projection does not do it)"),
+          ("self-out", "k_linear<k=768, residual>", "(fold of attention partials: two streams, or short caches) + act-quant + O matvec + residual"),
+          ("cross-attention", "k_step_attention<cross>", "LayerNorm + act-quant + per-head Q rows + attention over the cross cache (+ fold where the projection does not do it)"),
+          ("cross-out", "k_linear<k=768, residual>", "(fold: two streams, or short memories) + act-quant + O matvec + residual"),
           ("ffn-up", "k_linear<k=768, LayerNorm, GELU>", "LayerNorm + act-quant + up matvec + GELU"),
           ("ffn-down", "k_linear<k=3072, residual>", "act-quant + down matvec + residual")]
 
@@ -281,11 +281,11 @@ STAGES = [("self-attention", "k_step_attention<self>", "LayerNorm + int8 act-qua
 # then WRITE_SIZE), each scaled by what the same counter reads for the library's plain 256 MiB read+write kernel.  A figure
 # belongs to the kernel sources it was measured on: it is reported only while their hash is the one recorded here.
 MEASURED_TRAFFIC = {
-    1: {"kernel": "k_linear<k=768, residual>", "bytes": 937921, "profile": "profiles/decode_step_int8_hbm_counters.md",
-        "sources": ("kernels_linear.hip", "device_common.h", "kernels.h", "common.h"), "csrc_sha256": "aefd793795f67117"},
-    8: {"kernel": "k_step_attention<self>", "bytes": 54459728, "profile": "profiles/decode_step_int8_hbm_counters.md",
+    1: {"kernel": "k_linear<k=768, residual>", "bytes": 955833, "profile": "profiles/decode_step_int8_hbm_counters.md",
+        "sources": ("kernels_linear.hip", "device_common.h", "kernels.h", "common.h"), "csrc_sha256": "35a62c05e339ea94"},
+    8: {"kernel": "k_step_attention<self>", "bytes": 54473543, "profile": "profiles/decode_step_int8_hbm_counters.md",
         "sources": ("kernels_step_attention.hip", "step_attention_core.h", "step_items.h", "tagged_exchange.h", "device_common.h",
-                    "kernels.h", "common.h"), "csrc_sha256": "ce4c11fffeb0abb1"},
+                    "kernels.h", "common.h"), "csrc_sha256": "5b706ec975938d8d"},
 }
 
 
