@@ -96,7 +96,7 @@ __device__ __forceinline__ int count_before(const unsigned *keys, const int *ids
     return before;
 }
 // The same by the keys alone, counted by LANES adjacent threads: thread `part` compares the quads of keys part, part + LANES, ..., sixteen reads
-// together; the keys behind the list are zero (no candidate's is).  Every lane of the wavefront must call it.
+// together; the keys behind the list are zero, which is larger than none.  Every lane of the wavefront must call it.
 template <int LANES>
 __device__ __forceinline__ int count_larger(const unsigned *keys, int n, unsigned key, int part) {
     const uint4 *const quads = reinterpret_cast<const uint4 *>(keys) + part;
@@ -266,25 +266,31 @@ __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame
         // ---- collect the candidates at or above the bound: one LDS counter update per wavefront, places by ballot
         if (keys_in_registers) {
             // from the keys the thread kept (ids tid + 256 i): eight ballots, no LDS read; what is not taken goes to a place nobody reads
-            unsigned long long masks[kKeysInRegisters];
-            unsigned in_wave = 0u;
-            const unsigned least = max(bound, 1u);   // (ids past the vocabulary have key zero)
+            const auto collect = [&](const auto taken) {
+                unsigned long long masks[kKeysInRegisters];
+                unsigned in_wave = 0u;
 #pragma unroll
-            for (int i = 0; i < kKeysInRegisters; ++i) {
-                masks[i] = __ballot(own_key[i] >= least);
-                in_wave += (unsigned)__popcll(masks[i]);
-            }
-            unsigned next_slot = 0u;
-            if (lane == 0) next_slot = atomicAdd(&s_count, in_wave);
-            next_slot = (unsigned)__builtin_amdgcn_readfirstlane((int)next_slot);
+                for (int i = 0; i < kKeysInRegisters; ++i) {
+                    masks[i] = __ballot(taken(i));
+                    in_wave += (unsigned)__popcll(masks[i]);
+                }
+                unsigned next_slot = 0u;
+                if (lane == 0) next_slot = atomicAdd(&s_count, in_wave);
+                next_slot = (unsigned)__builtin_amdgcn_readfirstlane((int)next_slot);
 #pragma unroll
-            for (int i = 0; i < kKeysInRegisters; ++i) {
-                const unsigned ahead = __builtin_amdgcn_mbcnt_hi((unsigned)(masks[i] >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)masks[i], next_slot));
-                const unsigned slot = own_key[i] >= least ? min(ahead, (unsigned)kFastCandidates) : (unsigned)kFastCandidates;
-                s_cand_key[slot] = own_key[i];
-                s_cand_id[slot] = tid + 256 * i;
-                next_slot += (unsigned)__popcll(masks[i]);
-            }
+                for (int i = 0; i < kKeysInRegisters; ++i) {
+                    const unsigned ahead = __builtin_amdgcn_mbcnt_hi((unsigned)(masks[i] >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)masks[i], next_slot));
+                    const unsigned slot = taken(i) ? min(ahead, (unsigned)kFastCandidates) : (unsigned)kFastCandidates;
+                    s_cand_key[slot] = own_key[i];
+                    s_cand_id[slot] = tid + 256 * i;
+                    next_slot += (unsigned)__popcll(masks[i]);
+                }
+            };
+            // (ids past the vocabulary have key zero.  So has the NaN of all ones, and the bound is zero where too few of a wavefront's bests are above
+            // such keys, or where a wavefront has too few ids: only then does the id have to be looked at.)
+            const unsigned least = (unsigned)__builtin_amdgcn_readfirstlane((int)bound);
+            if (__builtin_expect(least != 0u, 1)) collect([&](const int i) { return own_key[i] >= least; });
+            else collect([&](const int i) { return tid + 256 * i < V; });
         } else {
             unsigned in_wave = 0u;
             for (int base = wave * 64; base < V; base += 256) {

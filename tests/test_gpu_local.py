@@ -274,6 +274,49 @@ def test_frame_equal_logits_within_the_list(pkg, backend, orc, synth, V, copies)
     backend.set_quant(0)
 
 
+@pytest.mark.parametrize("finite", [0, 3, 40])
+@pytest.mark.parametrize("V", [96, 200, 300, 544, 2048])
+def test_frame_nan_logits(pkg, backend, orc, synth, V, finite):
+    """Logits that are the NaN of all ones, whose order key is zero: all of the codebook's or all but `finite` of it.  The list is what it is for any
+    keys, larger ones first and smaller ids first among equal ones, masked ids (the lowest finite value) in front of such NaNs; a list that
+    holds a NaN has a NaN total, which no running sum reaches, and its last place is taken; a list without one is chosen from as ever."""
+    _announce("local frame, NaN logits, vocab %d, %d finite" % (V, finite))
+    S, codebook, eos, cbc = 3, V - 2, V - 1, 4
+    cfg, w, proj, bias, tables, rng = _setup(synth, 1, S, V, seed=V + finite)
+    nan = np.array([0xFFFFFFFF], np.uint32).view(np.float32)[0]
+    kept = rng.permutation(codebook)[:finite]
+    for s in range(S):
+        values = bias[s][kept].copy()
+        bias[s][:] = nan
+        bias[s][kept] = values
+    items = [{"temperature": 0.9, "topk": k, "rng_state": 1000 + 37 * i, "forbid_eos": True} for i, k in enumerate((2, 3, 7, 50, 80, 129, 256))]
+    backend.set_quant(QT["f32"])
+    loc = pkg.Local(backend, cfg, w, proj, bias, tables, codebook, eos, cbc)
+    drows = [backend.alloc(cfg["width"]).write(rng.standard_normal(cfg["width"]).astype(np.float32)) for _ in items]
+    dlogits = backend.alloc(len(items) * S * V)
+    for attempt in range(3):     # eager, captured, replayed
+        got = loc.frame([dict(it, row=d.ptr) for it, d in zip(items, drows)], dlogits.ptr)
+        logits = dlogits.read().reshape(len(items), S, V)
+        for b, it in enumerate(items):
+            state = it["rng_state"]
+            for s in range(S):
+                bits = logits[b, s].view(np.uint32)
+                assert np.all(np.delete(bits[:codebook], kept) == 0xFFFFFFFF) and np.all(logits[b, s, codebook:] == -np.finfo(np.float32).max)
+                keys = np.where(bits >> 31, ~bits, bits | np.uint32(0x80000000)).astype(np.uint64)
+                order = np.argsort(((np.uint64(0xFFFFFFFF) - keys) << np.uint64(32)) | np.arange(V, dtype=np.uint64), kind="stable")
+                top = min(it["topk"], V)
+                plain = np.where(np.isnan(logits[b, s]), np.float32(-np.inf), logits[b, s])   # behind everything, as such NaNs are
+                value, _, state, _ = orc.local_choose(plain, codebook, eos, it["temperature"], it["topk"], state, True)
+                if np.isnan(logits[b, s][order[:top]]).any():
+                    value = order[top - 1]
+                assert got["values"][b, s] == value, "topk %d position %d" % (it["topk"], s)
+                assert got["stored"][b, s] == (value if value < codebook else 0)
+            assert got["rng_state"][b] == state
+    loc.destroy()
+    for d in drows + [dlogits]:
+        d.free()
+
+
 def test_frame_eos_outside_vocabulary(pkg, backend, orc, synth, nerr):
     """An end-of-sequence id that is no id of the vocabulary (here one whose low 32 bits are 5, a real id) matches
     nothing, as in the reference's full-width comparison (src/graph.c:1563-1574): only codebook ids are ever allowed,
