@@ -25,9 +25,9 @@
 // are live, so a stream inside a batch is bit-identical to the same stream run alone
 // (the contract of src/qmat.c:1107-1179).
 #include <stdlib.h>
-
-#include <stdlib.h>
 #include <string.h>
+
+#include <algorithm>
 
 #include "device_common.h"
 
@@ -79,6 +79,8 @@ constexpr bool kPackedLead = BT == 1 && SPEC != SPEC_ANY;
 template <int BT, int SPEC>
 constexpr bool kStridedLead = kWaveStaging<BT> && SPEC != SPEC_ANY;
 
+// Rows a workgroup of either such build takes at most (launch_linear_t), below what twelve bits hold and a multiple of every pass.
+constexpr int kMostPackedRows = 2048;
 // n:20 | rows per workgroup:12 | streams:5 | input stride / 4:13 | output stride / 4:14 (strides in floats)
 struct StridedShape {
     int n, rows_per_wg, batch;
@@ -652,6 +654,8 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
     // on beside another lane (sixteen f16 streams 818 / 785, f32 839 / 829).
     if ((BUILD & SPEC_SIDE) != 0 && groups > 2)
         while (workgroups() > (a.beside ? 2 : 3) * st->cu_count) passes *= 2;
+    // (many products, or many groups of wide ones, would choose more than the packed arguments hold: more workgroups instead)
+    if (kPackedLead<BT, SPEC> || kStridedLead<BT, SPEC>) passes = std::min(passes, kMostPackedRows / rows_per_wg_pass);
     const int rows_per_wg = rows_per_wg_pass * passes;
     const int grid = (a.n + rows_per_wg - 1) / rows_per_wg;
     const size_t lds = (size_t)BT * a.k * (kQuantised<QT> ? 1 : 4);
@@ -740,14 +744,14 @@ int launch_linear_q(State *st, const LinearArgs &a, char *error, size_t capacity
     // (the specialised builds of one stream take their small numbers packed into one argument: when one of them
     // does not fit its bit field the launch takes the general build, with the same arithmetic)
     LeadShape fit{};
-    fit.n = a.n; fit.batch = 1; fit.rows_per_wg = 2048;   // above what launch_linear_t chooses for any n that fits (256 rows per 196,608 of n)
+    fit.n = a.n; fit.batch = 1; fit.rows_per_wg = kMostPackedRows;
     if (a.fold_partial != nullptr) {
         fit.is_self = a.fold_is_self; fit.stream0 = a.fold_stream0; fit.heads = a.fold_heads; fit.max_units = a.fold_max_units; fit.head_width = a.fold_head_width;
     }
     bool packs = lead_fits(fit) && (a.batch > 2 || dense_rows(a));
     if (a.batch > 2 && a.fold_partial == nullptr) {   // more streams: the specialised builds take rows at a fixed stride
         StridedShape strided{};
-        strided.n = a.n; strided.batch = a.batch; strided.rows_per_wg = 2048;
+        strided.n = a.n; strided.batch = a.batch; strided.rows_per_wg = kMostPackedRows;
         packs = rows_strided(a, &strided.in_stride, &strided.out_stride) && strided_fits(strided);
     }
     const bool residual = plain && packs && a.epilogue == EPI_RESIDUAL && a.ln_gain == nullptr;
@@ -783,13 +787,13 @@ bool linear_fast_supported(int qtype, size_t n, size_t k) {
 
 bool linear_folds_streams(int n, int k, int heads, int max_units) {
     LeadShape fit{};
-    fit.n = n; fit.rows_per_wg = 2048; fit.batch = 1; fit.folding = 1; fit.heads = heads; fit.max_units = max_units;
+    fit.n = n; fit.rows_per_wg = kMostPackedRows; fit.batch = 1; fit.folding = 1; fit.heads = heads; fit.max_units = max_units;
     return k == 768 && lead_fits(fit);
 }
 
 bool linear_takes_all(int n, int k, int epilogue, bool layernorm, size_t in_stride, size_t out_stride) {
     StridedShape s{};
-    s.n = n; s.rows_per_wg = 2048; s.batch = kMaxBatch; s.in_stride = in_stride; s.out_stride = out_stride;
+    s.n = n; s.rows_per_wg = kMostPackedRows; s.batch = kMaxBatch; s.in_stride = in_stride; s.out_stride = out_stride;
     if (!strided_fits(s) || out_stride == 0) return false;
     if (epilogue == EPI_RESIDUAL) return !layernorm && (k == 768 || k == 3072);
     return k == 768 && epilogue == (layernorm ? EPI_GELU : EPI_NONE);

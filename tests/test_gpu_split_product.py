@@ -84,6 +84,27 @@ def test_cross_kv_few_rows_as_a_list(backend, pkg, storage, rows, xw, layers):
         backend.set_quant(pkg.F32)
 
 
+def test_cross_kv_few_rows_of_many_wide_layers(backend, pkg):
+    """A list of products so long and wide that its rows per workgroup reach what a launch's packed arguments hold: taken like any other, every
+    layer's values those of a call for that layer alone."""
+    rows, width, xw, layers = 3, 768, 49152, 32
+    print("[gpu-case] cross K/V list of %d layers of %d" % (layers, xw), flush=True)
+    rng = np.random.default_rng(5)
+    backend.set_quant(pkg.F32)
+    gains = [backend.keep((1.0 + 0.1 * rng.standard_normal(width)).astype(np.float32)) for _ in range(layers)]
+    kvw = backend.keep(rng.standard_normal((2 * xw, width), dtype=np.float32))     # one tensor for all: their normalised rows differ
+    dmem = backend.alloc(rows * width).write(rng.standard_normal((rows, width)).astype(np.float32))
+    dk, dv = (backend.alloc(layers * rows * xw) for _ in range(2))
+    one_k, one_v = (backend.alloc(rows * xw) for _ in range(2))
+    backend.cross_kv_dev(dmem.ptr, rows, width, gains, None, [kvw] * layers, xw, dk.ptr, dv.ptr)
+    k, v = dk.read().reshape(layers, -1), dv.read().reshape(layers, -1)
+    for l in (0, 1, 17, layers - 1):
+        backend.cross_kv_dev(dmem.ptr, rows, width, [gains[l]], None, [kvw], xw, one_k.ptr, one_v.ptr)
+        assert np.array_equal(one_k.read(), k[l]) and np.array_equal(one_v.read(), v[l]), l
+    for d in (dmem, dk, dv, one_k, one_v):
+        d.free()
+
+
 @pytest.mark.parametrize("kernel", [1, 3])
 @pytest.mark.parametrize("tokens", [31, 32, 33, 64, 65, 97])
 def test_encoder_f32_tiles(backend, pkg, orc, synth, nerr, kernel, tokens):
