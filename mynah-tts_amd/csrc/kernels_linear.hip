@@ -736,11 +736,16 @@ int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity
     return launch_linear_t<QT, 8, NVT, KFIX, SPEC>(st, a, error, capacity);
 }
 
+// Neither bias nor probes nor a further output: what the specialised builds have no code for.
+bool no_extras(const LinearArgs &a) {
+    return a.bias == nullptr && a.probe_qx == nullptr && a.probe_sx == nullptr && a.probe_acc == nullptr && a.ln_out == nullptr &&
+           a.ln_out_slots == nullptr && a.aux_out == nullptr && a.act_out == nullptr;
+}
+
 template <int QT>
 int launch_linear_q(State *st, const LinearArgs &a, char *error, size_t capacity) {
     // what the arguments rule out decides the build (see SPEC above)
-    const bool plain = a.bias == nullptr && a.probe_qx == nullptr && a.probe_sx == nullptr && a.probe_acc == nullptr &&
-                       a.ln_out == nullptr && a.ln_out_slots == nullptr && a.aux_out == nullptr && a.act_out == nullptr;
+    const bool plain = no_extras(a);
     // (the specialised builds of one stream take their small numbers packed into one argument: when one of them
     // does not fit its bit field the launch takes the general build, with the same arithmetic)
     LeadShape fit{};
@@ -820,18 +825,19 @@ int launch_linear_products(State *st, const LinearArgs &a, const LinearProduct *
 }
 
 int launch_linear(State *st, const LinearArgs &a, char *error, size_t capacity) {
-    const bool probed = a.probe_qx != nullptr || a.probe_sx != nullptr || a.probe_acc != nullptr || a.ln_out != nullptr || a.ln_out_slots != nullptr ||
-                        a.aux_out != nullptr || a.act_out != nullptr;
+    const bool plain = no_extras(a);
     size_t in_stride = 0, out_stride = 0;
     if (a.batch < 1 || a.batch > kMaxBatch ||
-        (a.batch > kBatchTile && (a.bias != nullptr || probed || !rows_strided(a, &in_stride, &out_stride) ||
+        (a.batch > kBatchTile && (!plain || !rows_strided(a, &in_stride, &out_stride) ||
                                   !linear_takes_all(a.n, a.k, a.epilogue, a.ln_gain != nullptr, in_stride, out_stride)))) {
         set_error(error, capacity, "linear: batch tile out of range");
         return -1;
     }
-    if (a.fold_partial != nullptr && ((a.batch > kConsumerFoldMaxBatch && !(dense_rows(a) && linear_folds_streams(a.n, a.k, a.fold_heads, a.fold_max_units) &&
-                                                                             a.epilogue == EPI_RESIDUAL)) || a.k != a.fold_heads * a.fold_head_width || a.fold_slots == nullptr ||
-                                      a.fold_partial_ml == nullptr)) {
+    // (for more than two streams only the residual build of one stream a workgroup folds: what would take another build is refused)
+    const bool folds_many = plain && a.ln_gain == nullptr && a.epilogue == EPI_RESIDUAL && dense_rows(a) &&
+                            linear_folds_streams(a.n, a.k, a.fold_heads, a.fold_max_units);
+    if (a.fold_partial != nullptr && ((a.batch > kConsumerFoldMaxBatch && !folds_many) || a.k != a.fold_heads * a.fold_head_width ||
+                                      a.fold_slots == nullptr || a.fold_partial_ml == nullptr)) {
         set_error(error, capacity, "linear: more than two streams to fold for, or rows that are not heads x head width");
         return -1;
     }

@@ -39,3 +39,38 @@ def test_list_of_products_that_the_rule_takes_is_launched(pkg, tmp_path):
     assert len(lines) == 28
     for line in lines:
         assert ": 1 -1 " in line and "no ROCm-capable device" in line, line
+
+
+def test_fold_of_many_streams_is_refused_where_the_build_cannot(pkg, tmp_path):
+    """Only the side-by-side residual build folds for more than two streams: with a bias, a LayerNorm, a probe or a further output the general
+    build would run, which multiplies the rows as they are -- such a launch is refused."""
+    lines = _run(pkg, tmp_path, """
+    static StepSlots slots;
+    static float at[4];
+    for (int what = 0; what < 10; ++what)
+        for (const int batch : {2, 3, 8}) {
+            State st;
+            LinearArgs a{};
+            a.w = at; a.scales = at; a.qtype = MYNAH_HIP_INT8; a.n = a.k = 768; a.batch = batch; a.epilogue = EPI_RESIDUAL;
+            for (int b = 0; b < a.batch && b < kBatchTile; ++b) { a.in[b] = at + (size_t)b * a.k; a.out[b] = at + (size_t)b * a.n; }
+            a.fold_partial = a.fold_partial_ml = at; a.fold_slots = &slots;
+            a.fold_heads = 12; a.fold_head_width = 64; a.fold_max_units = 17; a.fold_is_self = 1;
+            switch (what) {
+                case 1: a.bias = at; break;
+                case 2: a.ln_gain = at; break;
+                case 3: a.probe_qx = reinterpret_cast<int8_t *>(at); break;
+                case 4: a.probe_sx = at; break;
+                case 5: a.probe_acc = reinterpret_cast<int32_t *>(at); break;
+                case 6: a.ln_out = at; break;
+                case 7: a.ln_out_slots = &slots; break;
+                case 8: a.aux_out = at; break;
+                case 9: a.act_out = at; break;
+            }
+            const int rc = launch_linear(&st, a, e, sizeof e);
+            printf("%d %d %d %s\\n", what, batch, rc, e);
+        }""")
+    assert len(lines) == 30
+    for line in lines:
+        what, batch = map(int, line.split()[:2])
+        refused = batch > 2 and what != 0
+        assert ("streams to fold for" if refused else "no ROCm-capable device") in line, line
