@@ -21,6 +21,7 @@
 #include <new>
 
 #include "device_common.h"
+#include "head_rows.h"
 
 namespace mynah {
 
@@ -76,7 +77,7 @@ struct mynah_hip_decoder {
     };
     Graphs forms[8];   // what a captured step depends on beside its stream count
     Graphs &form() { return forms[(long_caches ? 1 : 0) + (long_memories ? 2 : 0) + (beside ? 4 : 0)]; }
-    int head_recaptures = 0;
+    HeadRows head_rows;   // of the calls with a head, whichever form they step in
     int arith = 0;
     // Lanes: a batch above two streams is cut into groups that step side by side, each on a stream of its own with
     // workspaces, slot table and work tables of its own (a sibling decoder that shares this one's weights).  A stream's
@@ -727,15 +728,15 @@ static int run_lane(State *st, mynah_hip_decoder *lane, int count, hipStream_t s
         return r;
     };
     if (head != nullptr) {
-        // another head, or other rows for its results, than this stream count's last step had: captured again, behind one
+        // another head, or other rows for its results, than this form's last step of this stream count had: captured again, behind one
         // eager step (a weight seen for the first time is converted and uploaded there: no part of a capture)
         const unsigned long long signature = head_signature_of(st, *head, count);
+        lane->head_rows.step(count, signature);
         if (captured.head_signature[count] != signature) {
             if (captured.graphs[2][count] != nullptr) {
                 (void)hipGraphExecDestroy(captured.graphs[2][count]);
                 captured.graphs[2][count] = nullptr;
             }
-            if (captured.head_signature[count] != 0) ++lane->head_recaptures;
             captured.eager_steps[2][count] = 0;
             captured.head_signature[count] = signature;
         }
@@ -854,9 +855,8 @@ static int decoder_step(State *st, mynah_hip_decoder *d, const mynah_hip_decoder
     if (ensure_lanes(st, d, lanes, error, capacity) != 0) return -1;
     const bool with_end = want_end || lanes != 1 || !d->fused_attention;
     *ended = with_end;
-    // (a caller that hands over other rows for the results at every step would have the graph captured at every step)
     static const bool head_in_graph = !(getenv("MYNAH_HIP_HEAD_IN_GRAPH") != nullptr && strcmp(getenv("MYNAH_HIP_HEAD_IN_GRAPH"), "0") == 0);
-    const bool head_along = head_in_graph && head != nullptr && !with_end && head_done != nullptr && d->head_recaptures < 8;
+    const bool head_along = head_in_graph && head != nullptr && !with_end && head_done != nullptr && d->head_rows.in_graph();
     if (head_along) *head_done = true;
     const LanePlan plan = plan_lanes(s, B, lanes);
     d->last_batch_slots = s;

@@ -12,7 +12,7 @@ def _run(pkg, tmp_path, body):
     """The lines a program prints whose main() has `body`."""
     lib = pkg.load_library()._name
     source, program = tmp_path / "rules.cpp", tmp_path / "rules"
-    source.write_text("#include \"kernels.h\"\n#include <cstdio>\nusing namespace mynah;\nint main() {\n    char e[256] = \"\";\n%s\n}\n" % body)
+    source.write_text("#include \"kernels.h\"\n#include \"head_rows.h\"\n#include <cstdio>\nusing namespace mynah;\nint main() {\n    char e[256] = \"\";\n%s\n}\n" % body)
     subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"), "-I", os.path.join(ROOT, "include"), "-I",
                     os.path.join(ROOT, "mynah-tts_amd", "csrc"), str(source), lib, "-L", os.path.join(ROCM, "lib"), "-lamdhip64",
                     "-Wl,-rpath," + os.path.dirname(lib), "-Wl,-rpath," + os.path.join(ROCM, "lib"), "-o", str(program)], check=True)
@@ -74,3 +74,20 @@ def test_fold_of_many_streams_is_refused_where_the_build_cannot(pkg, tmp_path):
         what, batch = map(int, line.split()[:2])
         refused = batch > 2 and what != 0
         assert ("streams to fold for" if refused else "no ROCm-capable device") in line, line
+
+
+def test_head_leaves_the_graph_by_the_callers_changes(pkg, tmp_path):
+    """Other rows for the head's results count once, however many forms of the step (short and long caches or memories) are captured again for
+    them; a caller that changes them at every step has the head run behind the graph after eight."""
+    lines = _run(pkg, tmp_path, """
+    HeadRows running;                       // three stream counts, four forms each, the caller's rows changed twice
+    for (unsigned long long rows = 1; rows <= 3; ++rows)
+        for (int turn = 0; turn < 2; ++turn)
+            for (int form = 0; form < 4; ++form)
+                for (int count = 3; count <= 5; ++count) running.step(count, 100 * rows + count);
+    printf("%d %d\\n", running.changes, running.in_graph());
+    HeadRows restless;
+    int taken = 0;
+    for (unsigned long long rows = 1; rows <= 20 && restless.in_graph(); ++rows, ++taken) restless.step(1, rows);
+    printf("%d %d\\n", taken, restless.in_graph());""")
+    assert lines == ["6 1", "9 0"]
