@@ -77,7 +77,7 @@ struct mynah_hip_decoder {
     };
     Graphs forms[8];   // what a captured step depends on beside its stream count
     Graphs &form() { return forms[(long_caches ? 1 : 0) + (long_memories ? 2 : 0) + (beside ? 4 : 0)]; }
-    HeadRows head_rows;   // of the calls with a head, whichever form they step in
+    mynah::HeadRows head_rows;   // of the calls with a head, whichever form they step in
     int arith = 0;
     // Lanes: a batch above two streams is cut into groups that step side by side, each on a stream of its own with
     // workspaces, slot table and work tables of its own (a sibling decoder that shares this one's weights).  A stream's
