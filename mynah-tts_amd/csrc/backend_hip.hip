@@ -1286,8 +1286,7 @@ extern "C" int mynah_hip_cross_kv_dev(void *opaque, const float *dev_memory, siz
         if (listed) {
             LinearArgs first{};
             CrossProducts products{};
-            bool alike = true;
-            for (size_t p = 0; p < 2 * count && alike; ++p) {   // layer p / 2: its K half, its V half
+            for (size_t p = 0; p < 2 * count; ++p) {   // layer p / 2: its K half, its V half (all of one storage: it follows from their one shape)
                 const size_t layer = l0 + p / 2;
                 const CachedWeight *cw = nullptr;
                 if (cached_matrix(st, kv_w[layer] + (p % 2) * xattn_width * width, xattn_width, width, st->qtype, &cw, error, capacity) != 0) return -1;
@@ -1298,18 +1297,13 @@ extern "C" int mynah_hip_cross_kv_dev(void *opaque, const float *dev_memory, siz
                     first.n = (int)xattn_width; first.k = (int)width; first.batch = (int)memory_length;
                     for (size_t b = 0; b < memory_length && b < (size_t)kBatchTile; ++b) { first.in[b] = in + b * width; first.out[b] = out + b * xattn_width; }
                 }
-                alike = cw->qtype == first.qtype;   // (a matrix that the storage cannot hold is kept as f32)
                 products.of[p] = LinearProduct{static_cast<const char *>(cw->data) - static_cast<const char *>(first.w), cw->scales - first.scales,
                                                in - first.in[0], out - first.out[0]};
             }
-            if (alike) {
-                if (launch_cross_norms(st, dev_memory, memory_length, width, table, count, normed, &products, list, error, capacity) != 0 ||
-                    launch_linear_products(st, first, list, (int)(2 * count), error, capacity) != 0)
-                    return -1;
-                continue;
-            }
-            set_error(error, capacity, "cross K/V: weights of one shape in different storages");
-            return -1;
+            if (launch_cross_norms(st, dev_memory, memory_length, width, table, count, normed, &products, list, error, capacity) != 0 ||
+                launch_linear_products(st, first, list, (int)(2 * count), error, capacity) != 0)
+                return -1;
+            continue;
         }
         if (launch_layernorm(st, dev_memory, normed, table.gain[0], table.bias[0], memory_length, width, error, capacity) != 0) return -1;
         if (matmul_device(st, normed, dev_cross_k + l0 * per_layer, memory_length, width, xattn_width, kv_w[l0], nullptr, error, capacity) != 0) return -1;
