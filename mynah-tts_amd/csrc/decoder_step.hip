@@ -50,7 +50,9 @@ struct mynah_hip_decoder {
     // [kMaxBatch, heads, max_units, kStepRecord] (one area per attention kind); null: a fold kernel follows each launch
     unsigned long long *self_records = nullptr, *cross_records = nullptr;
     size_t records_bytes = 0;
-    int self_slots = 0, cross_slots = 0;   // workgroups of the many-stream attention kernels that the device holds at once
+    // workgroups that the device holds at once of the many-stream attention kernels: [0] of those that fold their own partials, [1] of
+    // those that leave them to the product behind
+    int self_slots[2] = {}, cross_slots[2] = {};
     unsigned item_epoch = 0;                    // next step counter for the tables (24 bits, never 0)
     mynah::StepSlots last_slots;                // of the last step of this lane
     mynah::StepSlots last_batch_slots;          // of the last step, every stream of it (the single-stage measurement graphs rebuild the tables from it)
@@ -289,7 +291,7 @@ StepItemTables decoder_item_tables(mynah_hip_decoder *d, int batch) {
     if (!d->fused_attention || batch <= kConsumerFoldMaxBatch) return StepItemTables{};
     return step_item_tables(batch, (int)d->heads, (int)d->cross_heads, d->max_units, d->self_items, d->cross_items,
                             d->self_records != nullptr && !folds_behind(d, 1, batch), d->self_records != nullptr && !folds_behind(d, 0, batch),
-                            d->self_slots, d->cross_slots);
+                            d->self_slots[folds_behind(d, 1, batch) ? 1 : 0], d->cross_slots[folds_behind(d, 0, batch) ? 1 : 0]);
 }
 
 int decoder_enqueue_layers(State *st, mynah_hip_decoder *d, int batch, char *error, size_t capacity) {
@@ -353,13 +355,13 @@ static int allocate_workspaces(State *st, mynah_hip_decoder *d, char *error, siz
                 // ("device": what the device holds of this kernel at once).  Measured with eight ragged streams, same box, twice
                 // each: grouped to fit the device (pairs of chunks, one round of workgroups instead of two) 654 us per step,
                 // one chunk per workgroup 649 us -- the second chunk of a pair waits for its rows a full round trip after the first.
-                d->self_slots = d->cross_slots = 1 << 30;
                 const char *slots_env = getenv("MYNAH_HIP_ATTN_SLOTS");
-                if (slots_env != nullptr && strcmp(slots_env, "device") == 0) {
-                    d->self_slots = step_attention_slots(l0.qkv->qtype, (int)w, d->max_units, 1, d->self_records != nullptr);
-                    d->cross_slots = xw != 0 ? step_attention_slots(l0.q_cross->qtype, (int)w, d->max_units, 0, d->cross_records != nullptr) : 0;
-                } else if (slots_env != nullptr && atoi(slots_env) > 0) {
-                    d->self_slots = d->cross_slots = atoi(slots_env);
+                const bool device = slots_env != nullptr && strcmp(slots_env, "device") == 0;
+                const int named = slots_env != nullptr && atoi(slots_env) > 0 ? atoi(slots_env) : 1 << 30;
+                for (int plain = 0; plain < 2; ++plain) {
+                    const bool records = d->self_records != nullptr && plain == 0;
+                    d->self_slots[plain] = device ? step_attention_slots(l0.qkv->qtype, (int)w, d->max_units, 1, records, plain != 0) : named;
+                    d->cross_slots[plain] = !device ? named : xw != 0 ? step_attention_slots(l0.q_cross->qtype, (int)w, d->max_units, 0, records, plain != 0) : 0;
                 }
             }
             if (rc == 0 && xw != 0)

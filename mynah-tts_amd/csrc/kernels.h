@@ -178,8 +178,9 @@ struct StepItemTables {
 StepItemTables step_item_tables(int batch, int heads, int cross_heads, int max_units, StepItem *self_items, StepItem *cross_items, bool self_fold,
                                 bool cross_fold, int self_slots, int cross_slots);
 inline unsigned step_item_workgroups(const StepItemTables &t) { return (unsigned)((t.self_entries + t.cross_entries + 255) / 256); }
-// Workgroups of the many-stream attention kernel for this weight storage and shape that the device holds at once.
-int step_attention_slots(int qtype, int width, int max_units, int is_self, bool with_fold);
+// Workgroups of the many-stream attention kernel for this weight storage and shape that the device holds at once.  plain: of the
+// build that leaves its partials to the product behind it (width 768), else of the one that folds its own.
+int step_attention_slots(int qtype, int width, int max_units, int is_self, bool with_fold, bool plain);
 // LDS a fold workgroup needs: the launch's dynamic LDS is at least this when it folds its own partials.
 size_t step_fold_lds_bytes(int max_units);
 // Folds the partials of the same arguments into out[batch][heads * head_width] (large batches only).

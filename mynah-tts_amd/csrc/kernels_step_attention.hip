@@ -559,9 +559,9 @@ int launch_t(State *st, const StepAttnArgs &a, char *error, size_t capacity) {
 }
 
 template <int QT>
-int slots_t(int width, int max_units, bool is_self, bool with_fold) {
+int slots_t(int width, int max_units, bool is_self, bool with_fold, bool plain) {
     int per_cu = 0, device = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kernel_for<QT>(width, is_self, false)), kThreads,
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kernel_for<QT>(width, is_self, false, plain)), kThreads,
                                                      lds_for<QT>(width, max_units, with_fold)) != hipSuccess ||
         hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return 0;
@@ -579,12 +579,12 @@ bool step_attention_supported(int qtype, size_t width, size_t heads, size_t head
     return (chunks + group - 1) / group <= 4;   // one register group of four chunks per lane and pass
 }
 
-int step_attention_slots(int qtype, int width, int max_units, int is_self, bool with_fold) {
+int step_attention_slots(int qtype, int width, int max_units, int is_self, bool with_fold, bool plain) {
     switch (qtype) {
-        case MYNAH_HIP_F32: return slots_t<MYNAH_HIP_F32>(width, max_units, is_self != 0, with_fold);
-        case MYNAH_HIP_F16: return slots_t<MYNAH_HIP_F16>(width, max_units, is_self != 0, with_fold);
-        case MYNAH_HIP_INT8: return slots_t<MYNAH_HIP_INT8>(width, max_units, is_self != 0, with_fold);
-        default: return slots_t<MYNAH_HIP_INT4>(width, max_units, is_self != 0, with_fold);
+        case MYNAH_HIP_F32: return slots_t<MYNAH_HIP_F32>(width, max_units, is_self != 0, with_fold, plain);
+        case MYNAH_HIP_F16: return slots_t<MYNAH_HIP_F16>(width, max_units, is_self != 0, with_fold, plain);
+        case MYNAH_HIP_INT8: return slots_t<MYNAH_HIP_INT8>(width, max_units, is_self != 0, with_fold, plain);
+        default: return slots_t<MYNAH_HIP_INT4>(width, max_units, is_self != 0, with_fold, plain);
     }
 }
 
