@@ -650,9 +650,9 @@ def test_captured_step_survives_a_growing_backend_workspace(pkg, backend, synth)
 
 @pytest.mark.parametrize("qtype_name", ["int8", "f32", "int4"])
 def test_many_stream_forms_agree(pkg, backend, synth, qtype_name):
-    """Five ragged streams (one with an empty cache, one without encoder memory) stepped by the many-stream attention launches
-    in each of their forms -- partials folded inside the launch (the default), by a fold kernel behind it, and with two or
-    more cache chunks per workgroup -- give the same bits, outputs and appended cache rows, eagerly and as a captured graph."""
+    """Five ragged streams (one with an empty cache, one without encoder memory), short enough that the products behind the attention launches
+    fold their partials, with every switch that many-stream attention has (the fold kernel's does nothing here: nothing folds inside), one or
+    more cache chunks per workgroup: the same bits, outputs and appended cache rows, eagerly and as a captured graph."""
     import os
     _announce("many-stream forms agree, %s" % qtype_name)
     lengths, mems = [700, 0, 129, 383, 512], [40, 7, 0, 130, 129]
@@ -687,6 +687,49 @@ def test_many_stream_forms_agree(pkg, backend, synth, qtype_name):
             for b in range(len(lengths)):
                 assert np.array_equal(out[b].view(np.uint32), ref_out[b].view(np.uint32)), "%s differs from the default, stream %d" % (name, b)
                 assert np.array_equal(rows[b][0], ref_rows[b][0]) and np.array_equal(rows[b][1], ref_rows[b][1]), "%s: appended rows differ" % name
+    finally:
+        backend.set_quant(0)
+
+
+@pytest.mark.parametrize("qtype_name,batch", [("int8", 3), ("f32", 6), ("int8", 10), ("int4", 9), ("f16", 11), ("f32", 16)])
+def test_forms_agree_beyond_the_lines(pkg, backend, synth, qtype_name, batch):
+    """Streams with caches and memories beyond what the products behind the attention launches fold, in one lane and in two (each of which has such
+    a stream): folded inside the launches, by the fold kernel, and with several chunks per workgroup, outputs and appended rows are those of
+    each stream alone, eagerly and as a captured graph."""
+    import os
+    _announce("forms agree beyond the lines, %s batch %d" % (qtype_name, batch))
+    lengths = [2300, 129, 2250, 0, 383, 512, 700, 100, 1, 640, 127, 128, 1153, 5, 64, 300][:batch]
+    mems = [2250, 40, 2300, 7, 0, 130, 129, 300, 64, 256, 1, 128, 33, 200, 0, 90][:batch]     # the two longest streams lead the lanes
+    cfg = synth.decoder_config(layers=2, capacity=2400)
+    weights = synth.decoder_weights(cfg, seed=0)
+    streams = synth.decoder_streams(cfg, lengths, mems, seed=5)
+    backend.set_quant(QT[qtype_name])
+
+    def appended(h):
+        return [tuple(a[:, n].copy() for a in h.cache_rows(b)) for b, n in enumerate(lengths)]
+
+    try:
+        alone = None
+        for env in ({}, {"MYNAH_HIP_FOLD_IN_LAUNCH": "0"}, {"MYNAH_HIP_ATTN_SLOTS": "device"}, {"MYNAH_HIP_ATTN_SLOTS": "100"}):
+            os.environ.update(env)                              # read when a decoder, or a lane of it at its first step, is made
+            try:
+                h = Harness(pkg, backend, cfg, weights, streams)
+                if alone is None:
+                    outs = [h.step([b])[0] for b in range(batch)]
+                    alone = outs, appended(h)
+                for turn in range(3):                           # eager, capture, replay
+                    for b in range(batch):
+                        h.reset_cache(b)
+                    outs = h.step()
+                    for b in range(batch):
+                        assert np.isfinite(outs[b]).all()
+                        assert np.array_equal(outs[b].view(np.uint32), alone[0][b].view(np.uint32)), "%s turn %d stream %d" % (env, turn, b)
+                for b, rows in enumerate(appended(h)):
+                    assert all(np.array_equal(g, w) for g, w in zip(rows, alone[1][b])), "%s: appended rows of stream %d" % (env, b)
+                h.close()
+            finally:
+                for k in env:
+                    del os.environ[k]
     finally:
         backend.set_quant(0)
 
