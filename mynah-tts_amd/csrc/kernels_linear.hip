@@ -55,7 +55,8 @@ __device__ __forceinline__ float *stream_out(const LinearArgs &a, int b) {
 // (launch_linear_b); a build of its own, so that a lone stream does not wait for the arithmetic that finds a row.
 // SPEC_LIST (with SPEC_PLAIN, more than two rows): several products of one shape in one launch, the grid's third dimension naming them
 // (launch_linear_products).
-enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2, SPEC_PLAIN = 3, SPEC_SIDE = 4, SPEC_LIST = 8 };
+// SPEC_ROWS (with SPEC_RESIDUAL, one stream to a workgroup, k = 3072): the rows are there, nothing is folded (launch_linear_b).
+enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2, SPEC_PLAIN = 3, SPEC_SIDE = 4, SPEC_LIST = 8, SPEC_ROWS = 16 };
 
 // More than two streams: one wavefront stages one stream (load_stream_row / finish_stream_row,
 // device_common.h) -- staging every stream's activations is what such a launch spends most of its time on, every workgroup
@@ -203,7 +204,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
         a.fold_is_self = shape.is_self; a.fold_stream0 = shape.stream0;
         if constexpr (SPEC == SPEC_UP) {
             a.ln_gain = fold_partial; a.ln_bias = fold_partial_ml;
-        } else if constexpr (SPEC == SPEC_RESIDUAL) {
+        } else if constexpr (SPEC == SPEC_RESIDUAL && (BUILD & SPEC_ROWS) == 0) {
             if (shape.folding) {
                 a.fold_partial = fold_partial; a.fold_partial_ml = fold_partial_ml; a.fold_slots = reinterpret_cast<const StepSlots *>(in0);
             }
@@ -211,7 +212,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
         if constexpr ((BUILD & SPEC_SIDE) != 0) {
             const size_t y = blockIdx.y;   // the workgroup's stream (dense_rows)
             a.out[0] += y * (size_t)a.n;
-            if (SPEC != SPEC_RESIDUAL || !shape.folding) a.in[0] += y * (size_t)KFIX;
+            if (SPEC != SPEC_RESIDUAL || (BUILD & SPEC_ROWS) != 0 || !shape.folding) a.in[0] += y * (size_t)KFIX;
             a.fold_stream0 += (int)y;
         }
     } else if constexpr (BT <= 2) {
@@ -249,7 +250,7 @@ k_linear(const float *const in0, const float *const fold_partial, const float *c
     const int arg_epilogue = SPEC == SPEC_UP ? EPI_GELU : SPEC == SPEC_RESIDUAL ? EPI_RESIDUAL : SPEC == SPEC_PLAIN ? EPI_NONE : a.epilogue;
     const float *const arg_ln_gain = SPEC == SPEC_RESIDUAL || SPEC == SPEC_PLAIN ? nullptr : a.ln_gain;
     const float *const arg_ln_bias = SPEC == SPEC_RESIDUAL || SPEC == SPEC_PLAIN ? nullptr : a.ln_bias;
-    const float *const arg_fold_partial = (SPEC == SPEC_UP || SPEC == SPEC_PLAIN || BT > kConsumerFoldMaxBatch) ? nullptr : a.fold_partial;   // larger batches fold in a kernel of their own
+    const float *const arg_fold_partial = (SPEC == SPEC_UP || SPEC == SPEC_PLAIN || (BUILD & SPEC_ROWS) != 0 || BT > kConsumerFoldMaxBatch) ? nullptr : a.fold_partial;   // (a tile of streams takes its rows as they are)
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float s_sx[BT];
     __shared__ float s_scratch[kPrologueScratch * BT];
@@ -711,10 +712,17 @@ int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity
         // four int8 371 / 370.  Of more streams only where staging a tile of them costs more than their own workgroups do -- int4 and f16 rows
         // beside their products' instructions, f32 rows of 3072 -- and with no lane beside: FFN down, five f16 441 / 426, eight 517 / 503, f32 610 / 599 (int8 466 /
         // 472, sixteen f16 in two lanes 791 / 831); FFN up, five f16 425 / 418, six int4 358 / 350 (three int8 360 / 363, eight f32 599 / 614).
-        if (a.batch <= 1) return launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
+        // The FFN-down product folds nothing: a build without that code, three copies of it (one a piece of a thread's row), 22 of its 24 KB.  us a step, one
+        // stream of 300 rows, with / without it: f32 422.9 / 419.6, f16, int8 and int4 the same; four f32 streams 457.9 / 452.8.
+        constexpr int kRows = SPEC == SPEC_RESIDUAL && KFIX == 3072 ? SPEC_ROWS : 0;
+        const bool rows = kRows != 0 && a.fold_partial == nullptr;
+        if (a.batch <= 1)
+            return rows ? launch_linear_t<QT, 1, NVT, KFIX, SPEC | kRows>(st, a, error, capacity) : launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
         const bool all = a.beside == 0 && (SPEC == SPEC_UP ? QT == MYNAH_HIP_INT4 || QT == MYNAH_HIP_F16 : KFIX == 3072 && QT != MYNAH_HIP_INT8);
         const int most = a.fold_partial != nullptr ? kMaxBatch : all ? 8 : SPEC == SPEC_RESIDUAL && KFIX == 3072 ? 4 : 2;
-        if (a.batch <= most && dense_rows(a)) return launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE>(st, a, error, capacity);
+        if (a.batch <= most && dense_rows(a))
+            return rows ? launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE | kRows>(st, a, error, capacity)
+                        : launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE>(st, a, error, capacity);
         if (a.batch <= 2) {   // (launch_linear_q sends such launches to the general build; this is the backstop)
             set_error(error, capacity, "linear: rows do not lie one behind the other");
             return -1;

@@ -792,6 +792,35 @@ def test_who_folds_keeps_every_bit(pkg, backend, synth, qtype_name, batch):
         backend.set_quant(0)
 
 
+@pytest.mark.parametrize("qtype_name", ["int8", "int4"])
+def test_widest_decoder_folds_and_does_not(pkg, backend, orc, synth, nerr, qtype_name):
+    """The widest decoder: its output projections fold attention partials into rows of 3072 (more of them than are requested at once for the first
+    stream), where a 768-wide one's FFN-down product takes rows of that length as they are.  Against the oracle, two streams and each alone."""
+    _announce("widest decoder, %s" % qtype_name)
+    lengths, mems = [1400, 37], [200, 5]
+    cfg = synth.decoder_config(layers=1, width=3072, heads=48, ffn=768, cross_heads=48, capacity=1450)
+    weights = synth.decoder_weights(cfg, seed=0)
+    streams = synth.decoder_streams(cfg, lengths, mems, seed=1)
+    backend.set_quant(QT[qtype_name])
+    try:
+        h = Harness(pkg, backend, cfg, weights, streams)
+        want, _, _ = _oracle_step(orc, cfg, weights, streams, QT[qtype_name])
+        first = h.step()
+        quantised_errors_ok([nerr(first[b], want[b]) for b in range(2)], 2, "widest decoder " + qtype_name)
+        for turn in range(3):
+            for b in range(2):
+                h.reset_cache(b)
+            again = h.step()
+            for b in range(2):
+                assert np.array_equal(again[b].view(np.uint32), first[b].view(np.uint32)), "turn %d stream %d" % (turn, b)
+        for b in range(2):
+            h.reset_cache(b)
+            assert np.array_equal(h.step([b])[0].view(np.uint32), first[b].view(np.uint32)), "stream %d alone" % b
+        h.close()
+    finally:
+        backend.set_quant(0)
+
+
 def test_long_cache_takes_the_fold_kernel(pkg, backend, orc, synth, nerr):
     """A capacity whose per-(stream, head) partial records exceed the LDS a launch may use without asking (more than
     about 19,000 rows): the many-stream step then folds in a kernel of its own.  Three streams, one of them 20,000 rows
