@@ -28,6 +28,7 @@ struct LinearArgs {
     const float *fold_partial_ml;
     const StepSlots *fold_slots;
     int fold_heads, fold_head_width, fold_max_units, fold_is_self, fold_stream0;
+    int beside;             // resident step: another lane's launches run beside this one (host only; here it takes no further place of the arguments)
     int8_t *probe_qx;       // parity probes (null in production)
     float *probe_sx;
     int32_t *probe_acc;
@@ -39,7 +40,6 @@ struct LinearArgs {
     const StepSlots *ln_out_slots;
     float *aux_out;
     float *act_out;         // the input row as the prologue formed it (the fold of attention partials), before any LayerNorm
-    int beside;             // resident step: another lane's launches run beside this one
 };
 
 // True when the fused matvec kernel supports this shape/storage; otherwise use linear_generic.

@@ -55,7 +55,8 @@ __device__ __forceinline__ float *stream_out(const LinearArgs &a, int b) {
 // (launch_linear_b); a build of its own, so that a lone stream does not wait for the arithmetic that finds a row.
 // SPEC_LIST (with SPEC_PLAIN, more than two rows): several products of one shape in one launch, the grid's third dimension naming them
 // (launch_linear_products).
-// SPEC_ROWS (with SPEC_RESIDUAL, one stream to a workgroup, k = 3072): the rows are there, nothing is folded (launch_linear_b).
+// SPEC_ROWS (one or two streams to a workgroup, with SPEC_ANY or, rows of 3072, SPEC_RESIDUAL): the rows are there, and the fold's code is not
+// (launch_linear_b).
 enum { SPEC_ANY = 0, SPEC_RESIDUAL = 1, SPEC_UP = 2, SPEC_PLAIN = 3, SPEC_SIDE = 4, SPEC_LIST = 8, SPEC_ROWS = 16 };
 
 // More than two streams: one wavefront stages one stream (load_stream_row / finish_stream_row,
@@ -712,8 +713,9 @@ int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity
         // four int8 371 / 370.  Of more streams only where staging a tile of them costs more than their own workgroups do -- int4 and f16 rows
         // beside their products' instructions, f32 rows of 3072 -- and with no lane beside: FFN down, five f16 441 / 426, eight 517 / 503, f32 610 / 599 (int8 466 /
         // 472, sixteen f16 in two lanes 791 / 831); FFN up, five f16 425 / 418, six int4 358 / 350 (three int8 360 / 363, eight f32 599 / 614).
-        // The FFN-down product folds nothing: a build without that code, three copies of it (one a piece of a thread's row), 22 of its 24 KB.  us a step, one
-        // stream of 300 rows, with / without it: f32 422.9 / 419.6, f16, int8 and int4 the same; four f32 streams 457.9 / 452.8.
+        // Rows that are there have builds without the fold's code, of which the FFN-down product has three copies (one a piece of a thread's row), 22 of its 24
+        // KB.  us a step, one stream of 300 rows, with / without it: f32 422.9 / 419.6, f16, int8 and int4 the same; four f32 streams 457.9 / 452.8.  General builds
+        // (a seam product of one f32 row, 3072 x 3072, us a launch): 6.5 / 6.2.
         constexpr int kRows = SPEC == SPEC_RESIDUAL && KFIX == 3072 ? SPEC_ROWS : 0;
         const bool rows = kRows != 0 && a.fold_partial == nullptr;
         if (a.batch <= 1)
@@ -723,13 +725,12 @@ int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity
         if (a.batch <= most && dense_rows(a))
             return rows ? launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE | kRows>(st, a, error, capacity)
                         : launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE>(st, a, error, capacity);
-        if (a.batch <= 2) {   // (launch_linear_q sends such launches to the general build; this is the backstop)
-            set_error(error, capacity, "linear: rows do not lie one behind the other");
-            return -1;
-        }
-    } else {
-        if (a.batch <= 1) return launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
-        if (a.batch == 2) return launch_linear_t<QT, 2, NVT, KFIX, SPEC>(st, a, error, capacity);
+        if (a.batch <= 2) return launch_linear_b<QT, NVT, KFIX, SPEC_ANY>(st, a, error, capacity);
+    } else if (a.batch <= 2) {
+        if (a.fold_partial == nullptr)
+            return a.batch <= 1 ? launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_ROWS>(st, a, error, capacity)
+                                : launch_linear_t<QT, 2, NVT, KFIX, SPEC | SPEC_ROWS>(st, a, error, capacity);
+        return a.batch <= 1 ? launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity) : launch_linear_t<QT, 2, NVT, KFIX, SPEC>(st, a, error, capacity);
     }
     if (a.batch <= 4) return launch_linear_t<QT, 4, NVT, KFIX, SPEC>(st, a, error, capacity);
     // five to eight streams, rows at a fixed stride, residual epilogue (the output projections and the
