@@ -73,9 +73,9 @@ template <int BT>
 constexpr int kLinearThreads = kWaveStaging<BT> ? 64 * (BT > 4 ? BT : 4) : kThreads;
 
 // The builds whose leading arguments are repacked (see the kernel): specialised ones of one stream, which also take several streams side
-// by side, one to each row of the grid (launch_linear_b).
+// by side, one to each row of the grid, and of two (launch_linear_b).
 template <int BT, int SPEC>
-constexpr bool kPackedLead = BT == 1 && SPEC != SPEC_ANY;
+constexpr bool kPackedLead = BT <= 2 && SPEC != SPEC_ANY;
 // The same for more streams, when the rows of a launch lie at a fixed stride (the step's workspaces do): the specialised
 // builds that stage a stream per wavefront take two row pointers and two strides instead of sixteen row pointers.
 template <int BT, int SPEC>
@@ -659,7 +659,10 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
     // (many products, or many groups of wide ones, would choose more than the packed arguments hold: more workgroups instead)
     if (kPackedLead<BT, SPEC> || kStridedLead<BT, SPEC>) passes = std::min(passes, kMostPackedRows / rows_per_wg_pass);
     const int rows_per_wg = rows_per_wg_pass * passes;
-    const int grid = (a.n + rows_per_wg - 1) / rows_per_wg;
+    int grid = (a.n + rows_per_wg - 1) / rows_per_wg;
+    // Streams side by side: the same rows on the same XCD for every stream (workgroup i runs on XCD i % 8), whose L2 has them from the first.  With 683 row
+    // blocks two f32 streams' 8192 rows of 768 took 8.7 us, 6.1 as a tile, 5.8 with 688 (weights in turn).  Blocks past the rows ask for the last one's and end.
+    if ((BUILD & SPEC_SIDE) != 0) grid = (grid + 7) / 8 * 8;
     const size_t lds = (size_t)BT * a.k * (kQuantised<QT> ? 1 : 4);
     static std::atomic<bool> raised{false};   // per instantiation; states on separate threads meet here
     if (lds > 48 * 1024 && !raised) {
@@ -704,6 +707,21 @@ int launch_linear_t(State *st, const LinearArgs &a, char *error, size_t capacity
     return hip_check(hipGetLastError(), "linear launch", error, capacity);
 }
 
+// Whether a weight is too large to be read once a stream (rows that are there; streams side by side of launch_linear_b).  Of what all eight L2s
+// hold (32 MiB) every stream's workgroups want their XCD's eighth, which the launch's grid sees to; beyond that two streams of a product of
+// 768-wide rows take turns at the weight again (f32, us a launch as a tile / side by side, weights in turn: 8192 rows 6.0 / 5.8, 12288 8.5 / 8.6, 16384 10.8 / 11.4).
+// Rows of 3072 are for a 768-wide decoder's 768 outputs; with wider decoders a tile's workgroups have fewer prologues to a weight as large.
+// us a step of three layers, width 3072, as tiles / side by side: f32 two streams 280 / 298, four 389 / 405, eight 545 / 614; f16 two 231 / 228, four 350 / 364, eight
+// 517 / 566; int8 two 306 / 303, three 292 / 294, four 335 / 337; int4 three 219 / 211, eight the same.  Width 1536: f32 two 202 / 207, eight 461 / 467;
+// f16 four 247 / 242, int8 three 186 / 182.
+template <int QT, int KFIX>
+bool too_heavy_side_by_side(const LinearArgs &a) {
+    const size_t values = (size_t)a.n * a.k;
+    const size_t bytes = QT == MYNAH_HIP_F32 ? 4 * values : QT == MYNAH_HIP_F16 ? 2 * values : QT == MYNAH_HIP_INT8 ? values : values / 2 + values / 8;
+    if (KFIX != 3072) return bytes > (32u << 20);
+    return bytes > (QT == MYNAH_HIP_INT8 ? 8u << 20 : 12u << 20) * (QT != MYNAH_HIP_F32 && a.batch == 2 ? 2u : 1u);
+}
+
 template <int QT, int NVT, int KFIX, int SPEC>
 int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity) {
     if constexpr (SPEC != SPEC_ANY) {
@@ -720,12 +738,16 @@ int launch_linear_b(State *st, const LinearArgs &a, char *error, size_t capacity
         const bool rows = kRows != 0 && a.fold_partial == nullptr;
         if (a.batch <= 1)
             return rows ? launch_linear_t<QT, 1, NVT, KFIX, SPEC | kRows>(st, a, error, capacity) : launch_linear_t<QT, 1, NVT, KFIX, SPEC>(st, a, error, capacity);
+        const bool heavy = too_heavy_side_by_side<QT, KFIX>(a);
         const bool all = a.beside == 0 && (SPEC == SPEC_UP ? QT == MYNAH_HIP_INT4 || QT == MYNAH_HIP_F16 : KFIX == 3072 && QT != MYNAH_HIP_INT8);
-        const int most = a.fold_partial != nullptr ? kMaxBatch : all ? 8 : SPEC == SPEC_RESIDUAL && KFIX == 3072 ? 4 : 2;
+        const int most = a.fold_partial != nullptr ? kMaxBatch : heavy ? 1 : all ? 8 : SPEC == SPEC_RESIDUAL && KFIX == 3072 ? 4 : 2;
         if (a.batch <= most && dense_rows(a))
             return rows ? launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE | kRows>(st, a, error, capacity)
                         : launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_SIDE>(st, a, error, capacity);
-        if (a.batch <= 2) return launch_linear_b<QT, NVT, KFIX, SPEC_ANY>(st, a, error, capacity);
+        if (a.batch <= 2) {
+            if (rows && dense_rows(a)) return launch_linear_t<QT, 2, NVT, KFIX, SPEC | kRows>(st, a, error, capacity);
+            return launch_linear_b<QT, NVT, KFIX, SPEC_ANY>(st, a, error, capacity);
+        }
     } else if (a.batch <= 2) {
         if (a.fold_partial == nullptr)
             return a.batch <= 1 ? launch_linear_t<QT, 1, NVT, KFIX, SPEC | SPEC_ROWS>(st, a, error, capacity)

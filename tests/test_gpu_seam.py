@@ -153,6 +153,31 @@ def test_batched_matvec_bit_identical_to_solo(backend, pkg, qtype_name):
     backend.set_quant(pkg.F32)
 
 
+@pytest.mark.parametrize("qtype_name,n", [("f32", 770), ("f32", 8190), ("f32", 10922), ("f32", 10923), ("int8", 8190), ("f16", 8190), ("f16", 21846), ("int4", 8190)])
+def test_two_rows_of_a_large_weight(backend, pkg, nerr, qtype_name, n):
+    """Two rows one behind the other with row counts that leave the last XCDs' workgroups without rows, and weights on either side of what goes side by side
+    (32 MiB): each row's bits those of the row alone, nothing written behind them, and f32 against float64."""
+    k = 768
+    _announce("two rows of a large weight %s n=%d" % (qtype_name, n))
+    rng = np.random.default_rng(n)
+    w = backend.keep(rng.standard_normal((n, k), dtype=np.float32))
+    x = rng.standard_normal((2, k)).astype(np.float32)
+    backend.set_quant({"int8": pkg.INT8, "int4": pkg.INT4, "f16": pkg.F16, "f32": pkg.F32}[qtype_name])
+    guard = np.full(64, 7.0, np.float32)
+    din, dout, one = backend.alloc(2 * k).write(x), backend.alloc(2 * n + 64).write(guard, 2 * n), backend.alloc(n)
+    backend.matmul_d2d(din.ptr, dout.ptr, 2, k, n, w)
+    got = dout.read()
+    assert np.array_equal(got[2 * n:], guard)
+    for r in range(2):
+        backend.matmul_d2d(din.ptr + 4 * r * k, one.ptr, 1, k, n, w)
+        assert np.array_equal(one.read().view(np.uint32), got[r * n:(r + 1) * n].view(np.uint32)), r
+    if qtype_name == "f32":
+        assert nerr(got[:2 * n].reshape(2, n), x.astype(np.float64) @ w.T.astype(np.float64)) < 1e-5
+    for d in (din, dout, one):
+        d.free()
+    backend.set_quant(pkg.F32)
+
+
 def test_matmul_rows_and_generic_shapes(backend, pkg, orc, nerr):
     """rows > 1 through matmul_d2d (prefill-like), shapes the fused matvec does not take, host-pointer matmul."""
     _announce("generic matmul shapes")

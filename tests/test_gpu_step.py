@@ -792,12 +792,13 @@ def test_who_folds_keeps_every_bit(pkg, backend, synth, qtype_name, batch):
         backend.set_quant(0)
 
 
-@pytest.mark.parametrize("qtype_name", ["int8", "int4"])
-def test_widest_decoder_folds_and_does_not(pkg, backend, orc, synth, nerr, qtype_name):
-    """The widest decoder: its output projections fold attention partials into rows of 3072 (more of them than are requested at once for the first
-    stream), where a 768-wide one's FFN-down product takes rows of that length as they are.  Against the oracle, two streams and each alone."""
+@pytest.mark.parametrize("qtype_name", ["int8", "int4", "f16", "f32"])
+def test_widest_decoder(pkg, backend, orc, synth, nerr, qtype_name):
+    """The widest decoder, whose weights are four times a 768-wide one's: its output projections fold attention partials into rows of 3072 (int8 and int4; more
+    of them than are requested at once for the first stream) or take rows of that length as they are, and which products go side by side
+    depends on the weight's size.  Two and three streams against the oracle, and every stream's bits those of the stream alone."""
     _announce("widest decoder, %s" % qtype_name)
-    lengths, mems = [1400, 37], [200, 5]
+    lengths, mems = [1400, 37, 130], [200, 5, 64]
     cfg = synth.decoder_config(layers=1, width=3072, heads=48, ffn=768, cross_heads=48, capacity=1450)
     weights = synth.decoder_weights(cfg, seed=0)
     streams = synth.decoder_streams(cfg, lengths, mems, seed=1)
@@ -806,16 +807,18 @@ def test_widest_decoder_folds_and_does_not(pkg, backend, orc, synth, nerr, qtype
         h = Harness(pkg, backend, cfg, weights, streams)
         want, _, _ = _oracle_step(orc, cfg, weights, streams, QT[qtype_name])
         first = h.step()
-        quantised_errors_ok([nerr(first[b], want[b]) for b in range(2)], 2, "widest decoder " + qtype_name)
-        for turn in range(3):
-            for b in range(2):
-                h.reset_cache(b)
-            again = h.step()
-            for b in range(2):
-                assert np.array_equal(again[b].view(np.uint32), first[b].view(np.uint32)), "turn %d stream %d" % (turn, b)
-        for b in range(2):
-            h.reset_cache(b)
-            assert np.array_equal(h.step([b])[0].view(np.uint32), first[b].view(np.uint32)), "stream %d alone" % b
+        errors = [nerr(first[b], want[b]) for b in range(3)]
+        if qtype_name in ("int8", "int4"):
+            quantised_errors_ok(errors, 3, "widest decoder " + qtype_name)
+        else:
+            assert max(errors) < TOL[qtype_name], errors
+        for which in ([0, 1, 2], [0, 1], [1, 0], [0], [1], [2]):
+            for turn in range(3 if len(which) > 1 else 1):          # eager, captured, replayed
+                for b in which:
+                    h.reset_cache(b)
+                outs = h.step(which)
+                for out, b in zip(outs, which):
+                    assert np.array_equal(out.view(np.uint32), first[b].view(np.uint32)), "%s turn %d stream %d" % (which, turn, b)
         h.close()
     finally:
         backend.set_quant(0)
