@@ -232,17 +232,18 @@ __global__ void __launch_bounds__(512) k_split_rows(const float *const a, const 
 }
 
 // The K and V halves of every layer's kv_net on that layer's normalised memory, one launch.  The column tiles of all layers make one
-// list, of which an XCD takes every eighth: layer by layer the twelve of a 768-wide one would give XCDs 0 to 3 two each and the others one, and the
-// launch waits for the fullest.  Twelve layers, us a call, a grid of tiles a layer / one list: 100 rows 40.8 / 38.7, 180 58.3 / 47.5, 256 65.6 / 61.5.
-// (Two workgroups to a CU at 180 rows, some 23 ns a matrix instruction with its 6.4 vector instructions; a pass over the weight to have it in L2 first: 52.)
+// list, of which an XCD takes every eighth: layer by layer the twelve of a 768-wide one give XCDs 0 to 3 two each and the others one, and the
+// launch waits for the fullest.  `places` of the list are a layer's: its tiles, or (launch_split_cross_kv) the next multiple of eight.
+// (Two workgroups to a CU at 180 rows, some 23 ns a matrix instruction with its 6.4 vector instructions; a pass over the weight to have it in L2 first: slower.)
 __global__ void __launch_bounds__(512) k_split_cross_kv(const float *const normed, const SplitLayers weights, const int M, const int width, const int xw,
-                                                        const int mtiles, const int layers, float *const k_out, float *const v_out) {
+                                                        const int mtiles, const int layers, const int places, float *const k_out, float *const v_out) {
     __shared__ SplitTile<2, 1, 2> lds;
     const int N = 2 * xw, ntiles = (N + 127) / 128;
     const SplitWork work((int)blockIdx.x, mtiles);
-    if (work.nz >= ntiles * layers) return;
-    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3, layer = work.nz / ntiles;
-    const int col0 = (work.nz - layer * ntiles) * 128 + wave * 32, m0 = work.m * 64;
+    const int layer = work.nz / places, ntile = work.nz - layer * places;
+    if (layer >= layers || ntile >= ntiles) return;
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
+    const int col0 = ntile * 128 + wave * 32, m0 = work.m * 64;
     f32x16 acc[2] = {f32x16{0}, f32x16{0}};
     const float4 *tile = weights.w[layer] + (size_t)(min(col0, N - 32) / 32) * (width / 32) * 256;
     split_tile<2, 1, 2>(normed + (size_t)layer * M * width, width, m0, M, tile, width / 32, lds, acc);
@@ -344,8 +345,16 @@ int launch_split_cross_kv(State *st, const float *memory, size_t rows, size_t wi
                           float *k_out, float *v_out, char *error, size_t capacity) {
     if (launch_cross_norms(st, memory, rows, width, layers, count, normed, nullptr, nullptr, error, capacity) != 0) return -1;
     const int mtiles = (int)((rows + 63) / 64), ntiles = (int)((2 * xw + 127) / 128);
-    hipLaunchKernelGGL(k_split_cross_kv, dim3((unsigned)((ntiles * (int)count + 7) / 8 * 8 * mtiles)), dim3(512), 0, st->stream, normed, layers,
-                       (int)rows, (int)width, (int)xw, mtiles, (int)count, k_out, v_out);
+    // Layers one behind the other in the list, or each from a multiple of eight on (its first tile on XCD 0), by what the fullest XCD has to do.  The list is the
+    // shorter, but where either way some CUs have two workgroups and the list gives them to only a few of each XCD, layer by layer
+    // is faster.  us a call, layers of 768, layer by layer / list (workgroups of the fullest XCD, 32 CUs): twelve layers, 64 rows 23.4 / 23.5 (24 / 18), 100 35.8 /
+    // 37.0 (48 / 36), 180 53.9 / 42.8 (72 / 54), 256 61.6 / 59.4 (96 / 72), 320 78.5 / 63.6; 128 rows, nine layers 34.7 / 25.8 (36 / 28), eleven 35.6 / 37.2 (44 / 34),
+    // fourteen 39.1 / 39.5 (56 / 42), sixteen 42.6 / 42.2 (64 / 48); 192 rows, ten layers 41.1 / 40.8 (60 / 45); six layers of 256 rows 36.6 / 38.0 (48 / 36).
+    const int cus = st->cu_count / 8, apart = (ntiles + 7) / 8 * (int)count * mtiles, together = (ntiles * (int)count + 7) / 8 * mtiles;
+    const bool by_layer = together > cus && together <= cus + 3 * cus / 8 && apart <= 2 * cus;
+    const int places = by_layer ? (ntiles + 7) / 8 * 8 : ntiles;
+    hipLaunchKernelGGL(k_split_cross_kv, dim3((unsigned)((places * (int)count + 7) / 8 * 8 * mtiles)), dim3(512), 0, st->stream, normed, layers,
+                       (int)rows, (int)width, (int)xw, mtiles, (int)count, places, k_out, v_out);
     return hip_check(hipGetLastError(), "cross K/V launch", error, capacity);
 }
 

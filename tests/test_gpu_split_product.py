@@ -32,11 +32,11 @@ def test_cross_kv_tiles(backend, pkg, orc, rows, width, xw, layers):
         d.free()
 
 
-@pytest.mark.parametrize("rows,xw,layers", [(5, 32, 9), (17, 32, 9), (64, 224, 5), (130, 96, 3)])
+@pytest.mark.parametrize("rows,xw,layers", [(5, 32, 9), (17, 32, 9), (64, 224, 5), (130, 96, 3), (100, 768, 12), (130, 448, 12), (65, 768, 33)])
 def test_cross_kv_layers_together(backend, pkg, rows, xw, layers):
     """The layers' column tiles share one list: counts that no multiple of eight divides, a last tile that is not full (17 rows of 32 columns:
     nine tiles, each half empty), and every layer's values are those of a call for that layer alone, bit for bit.  (Five rows of this width
-    go layer by layer.)"""
+    go layer by layer; of twelve layers, 100 rows by 768 and 130 by 448, each starts at a place of its own in the list.)"""
     print("[gpu-case] cross K/V together rows=%d xw=%d layers=%d" % (rows, xw, layers), flush=True)
     rng, width = np.random.default_rng(rows + layers), 128
     backend.set_quant(pkg.F32)
