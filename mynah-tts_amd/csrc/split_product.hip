@@ -311,9 +311,13 @@ int split_product_splits(const State *st, size_t rows, size_t channels, size_t n
 // workgroups than CUs instead: 303, 325, 353 and 341, 380, 448.
 // A sum is then more and shorter chains of additions: the prefill's error against double precision (2-norm) 4.5e-7 / 3.7e-7 at 20 rows, 4.5e-7 /
 // 3.9e-7 at 50 with one tap, 6.3e-7 / 5.4e-7 and 6.6e-7 / 5.6e-7 with three.
-static int split_groups(const State *st, size_t mt, size_t mtiles, size_t channels, size_t n, size_t splits) {
+// A group of 32 channels, one round of the loop, pays for one more share of the sums to add where its weights are three taps or the row tiles are two at most:
+// four layers of width 256, one tap, us with groups of 64 at least / of 32: 16 rows 149.2 / 147.8, 64 167.7 / 165.7, 129 189.6 / 191.6, 160 189.6 / 191.9, 256 211.2 / 212.9;
+// three taps 16 rows 166.0 / 159.8, 256 235.9 / 229.1.
+static int split_groups(const State *st, size_t mt, size_t mtiles, size_t channels, size_t taps, size_t n, size_t splits) {
+    const size_t least = taps == 3 || mtiles <= 2 ? 32 : 64;
     for (size_t groups = mt == 1 ? 8 : 4; groups > 2; groups /= 2)
-        if (channels % (16 * groups * kBlocksAhead * splits) == 0 && (n * groups + 255) / 256 * mtiles * splits <= (size_t)st->cu_count) return (int)groups;
+        if (channels >= least * groups * splits && channels % (16 * groups * kBlocksAhead * splits) == 0 && (n * groups + 255) / 256 * mtiles * splits <= (size_t)st->cu_count) return (int)groups;
     return 2;
 }
 
@@ -325,7 +329,7 @@ int launch_split_product(State *st, const float *in, const float4 *w, size_t row
         return -1;
     }
     const int mt = split_row_tiles(st, rows, n, splits > 1), mtiles = (int)((rows + 32 * mt - 1) / (32 * mt));
-    const int groups = split_groups(st, (size_t)mt, (size_t)mtiles, channels, n, (size_t)splits);
+    const int groups = split_groups(st, (size_t)mt, (size_t)mtiles, channels, taps, n, (size_t)splits);
     const int wide = 256 / groups, ntiles = (int)((n + wide - 1) / wide);
     const dim3 grid((unsigned)((ntiles * splits + 7) / 8 * 8 * mtiles)), block(512);
     const auto launch = [&](auto kernel) {

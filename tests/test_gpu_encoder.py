@@ -261,9 +261,10 @@ def test_encoder_f32_wide_and_deep_products(pkg, backend, orc, synth, nerr, toke
 
 
 @pytest.mark.parametrize("kernel", [1, 3])
-@pytest.mark.parametrize("tokens,width,ffn", [(1, 256, 512), (32, 256, 256), (20, 768, 3072), (33, 768, 3072), (64, 768, 1536), (65, 512, 1024), (100, 768, 768)])
+@pytest.mark.parametrize("tokens,width,ffn", [(1, 256, 512), (32, 256, 256), (20, 768, 3072), (33, 768, 3072), (64, 768, 1536), (65, 512, 1024), (100, 768, 768), (128, 256, 1024)])
 def test_encoder_f32_channel_groups(pkg, backend, orc, synth, nerr, tokens, width, ffn, kernel):
-    """Few rows: the products' wavefronts in two, four or eight groups over the channels (tiles of 128, 64 or 32 columns), split and not."""
+    """Few rows: the products' wavefronts in two, four or eight groups over the channels (tiles of 128, 64 or 32 columns), split and not,
+    of 32 channels at least (few rows, three taps) or of 64."""
     _announce("encoder f32 channel groups tokens=%d width=%d ffn=%d kernel=%d" % (tokens, width, ffn, kernel))
     cfg = dict(synth.encoder_config(layers=1, width=width, heads=width // 64, ffn=ffn, vocab=300, max_positions=128), causal=True, ffn_kernel=kernel)
     w = synth.encoder_weights_f16(cfg, seed=81, kernel=kernel, biases=True)
