@@ -87,30 +87,45 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
     return max(max(r0, r1), max(r2, r3));
 }
 
-// How many of the collected candidates come before candidate (key, index) in the list, in full: the larger key first, among equal keys the
-// smaller index.
-__device__ __forceinline__ int count_before(const unsigned *keys, const int *ids, int n, unsigned key, int id, int from, int step) {
-    int before = 0;
-#pragma unroll 4
-    for (int j = from; j < n; j += step) before += keys[j] > key || (keys[j] == key && ids[j] < id) ? 1 : 0;
-    return before;
-}
-// The same by the keys alone, counted by LANES adjacent threads: thread `part` compares the quads of keys part, part + LANES, ..., sixteen reads
-// together; the keys behind the list are zero, which is larger than none.  Every lane of the wavefront must call it.
-template <int LANES>
-__device__ __forceinline__ int count_larger(const unsigned *keys, int n, unsigned key, int part) {
+// How many of the collected candidates have a larger key than each of KEYS own ones, counted by LANES adjacent threads: thread `part` compares the quads of
+// keys part, part + LANES, ..., sixteen reads together; the keys behind the list are zero, which is larger than none.  Every lane of the wavefront
+// must call it.
+template <int LANES, int KEYS>
+__device__ __forceinline__ void count_larger(const unsigned *keys, int n, const unsigned (&own)[KEYS], int part, int (&larger)[KEYS]) {
     const uint4 *const quads = reinterpret_cast<const uint4 *>(keys) + part;
-    int larger = 0;
+#pragma unroll
+    for (int j = 0; j < KEYS; ++j) larger[j] = 0;
 #pragma unroll 1
     for (int q0 = 0; 4 * q0 < n; q0 += 16 * LANES) {
         uint4 k[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) k[i] = quads[q0 + i * LANES];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) larger += (k[i].x > key ? 1 : 0) + (k[i].y > key ? 1 : 0) + (k[i].z > key ? 1 : 0) + (k[i].w > key ? 1 : 0);
+        for (int j = 0; j < KEYS; ++j)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                larger[j] += (k[i].x > own[j] ? 1 : 0) + (k[i].y > own[j] ? 1 : 0) + (k[i].z > own[j] ? 1 : 0) + (k[i].w > own[j] ? 1 : 0);
     }
-    if (LANES == 2) larger += dpp_i<kDppXor1>(larger);
-    return larger;
+    if (LANES == 2) {
+#pragma unroll
+        for (int j = 0; j < KEYS; ++j) larger[j] += dpp_i<kDppXor1>(larger[j]);
+    }
+}
+// How many have the same key and a smaller index.  Keys and indexes are read whatever the keys are (an index read only behind an equal key
+// was a round trip of its own: 16 us a choice from 96 with two equal ones); the indexes behind the list are larger than any.
+template <int LANES>
+__device__ __forceinline__ int count_equal_before(const unsigned *keys, const int *ids, int n, unsigned key, int id, int part) {
+    const uint4 *const key_quads = reinterpret_cast<const uint4 *>(keys);
+    const int4 *const id_quads = reinterpret_cast<const int4 *>(ids);
+    int before = 0;
+#pragma unroll 4
+    for (int q = part; 4 * q < n; q += LANES) {
+        const uint4 k = key_quads[q];
+        const int4 i = id_quads[q];
+        before += ((k.x == key) & (i.x < id)) + ((k.y == key) & (i.y < id)) + ((k.z == key) & (i.z < id)) + ((k.w == key) & (i.w < id));
+    }
+    if (LANES == 2) before += dpp_i<kDppXor1>(before);
+    return before;
 }
 
 // Frame start: the slot table (caches of this object, every length 0), x[b] = decoder_last[b] + position[0]
@@ -148,12 +163,12 @@ __global__ void __launch_bounds__(256) k_local_begin(LocalFrameDev *frame, const
 // A launch is one workgroup's chain.  Cycles by clock stamps for top-80 of 2048 (115 candidates), before / now: arguments 900 / 640, logits, mask,
 // bests and bound 3850 / 2650, collection 2050 / 1590, ranking and numerators 4600 / 2030, running sums, draw and pick 2200 / 2360, next row
 // 1900 / 1800.  What changed: leading arguments in registers; nothing written to LDS that only the radix selection reads; candidates not taken
-// stored where nobody looks, without a branch; the ranking by the keys' 32 bits, two threads a candidate (list places that two equal keys
-// leave empty are seen afterwards and filled in full); and behind the ranking the first wavefront alone, so that nothing waits at a barrier.
+// stored where nobody looks, without a branch; the ranking by the keys' 32 bits, two threads a candidate up to 128, one or two candidates a thread
+// beyond (list places that equal keys leave empty are seen afterwards and filled by the ids of the equal ones); and behind the ranking the first wavefront alone, so that nothing waits at a barrier.
 // Measured and not kept: the rows of the first 8 or 32 list positions fetched by the other wavefronts meanwhile (no change).
-// A frame of 16 positions, us, int8: one stream top-80 402 -> 380, three top-100 461 -> 439, eight top-50 494 -> 472.
+// A frame of 16 positions, us, int8: one stream top-80 402 -> 380, three top-100 461 -> 439, eight top-50 494 -> 472; of 8 positions, one stream: top-160 252 -> 221,
+// top-200 302 -> 234, top-256 300 -> 279; top-100 of 96 ids, two of them masked and so equal, 206 -> 212.
 constexpr int kFastCandidates = 512;
-constexpr int kRankByKeys = 256;     // candidates ranked by their keys alone
 constexpr int kEmptyPlace = 0x7fffffff;
 
 __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame, const float *const logits, const float *const audio_table,
@@ -165,7 +180,7 @@ __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame
     __shared__ unsigned long long s_head[4];                       // every wavefront's best candidate
     __shared__ unsigned s_bound[4];
     __shared__ __align__(16) unsigned s_cand_key[kFastCandidates + 1];
-    __shared__ int s_cand_id[kFastCandidates + 1];
+    __shared__ __align__(16) int s_cand_id[kFastCandidates + 1];
     __shared__ unsigned s_hist[4][256];
     __shared__ __align__(16) float s_top_val[kMaxTopK + 32];
     __shared__ int s_top_idx[kMaxTopK];
@@ -194,7 +209,7 @@ __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame
     const unsigned topk = item.topk;
     unsigned long long bits = item.rng_state;
     float *logits_copy = frame->logits_copy;
-    if (tid < kRankByKeys) s_cand_key[tid] = 0u;   // (256 threads: all of them; behind a list its keys are zero, see count_larger)
+    s_cand_key[tid] = s_cand_key[256 + tid] = 0u;   // behind a list the keys are zero (count_larger)
     if (tid == 0) s_count = 0u;
 
     // ---- constraint mask (src/graph.c:1556-1563); eight candidates per thread at a time, the first eight already requested
@@ -401,27 +416,25 @@ __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame
             atomicMin(&s_top_idx[place], id);
             s_top_val[place] = expf((key_value(key) - maximum) / temperature);
         };
-        static_assert(kMaxTopK == 256 && kRankByKeys == 256, "a thread for every candidate ranked by its key");
-        if (listed <= kRankByKeys / 2) {
-            const unsigned key = s_cand_key[tid >> 1];
-            const int id = s_cand_id[min(tid >> 1, listed - 1)], place = count_larger<2>(s_cand_key, listed, key, tid & 1);
-            if ((tid >> 1) < listed && (tid & 1) == 0 && place < top_count) put_in_place(place, key, id);
-        } else if (listed <= kRankByKeys) {
-            const unsigned key = s_cand_key[tid];
-            const int id = s_cand_id[min(tid, listed - 1)], place = count_larger<1>(s_cand_key, listed, key, 0);
-            if (tid < listed && place < top_count) put_in_place(place, key, id);
+        static_assert(kMaxTopK == 256 && kFastCandidates == 512, "two candidates a thread at most");
+        const bool paired = listed <= 128;   // two threads a candidate
+        const int first = paired ? tid >> 1 : tid;
+        const unsigned own_keys[2] = {s_cand_key[first], s_cand_key[256 + tid]};
+        const int own_ids[2] = {s_cand_id[min(first, listed - 1)], s_cand_id[min(256 + tid, listed - 1)]};
+        int place[2] = {0, 0};
+        if (paired) {
+            count_larger<2>(s_cand_key, listed, {own_keys[0]}, tid & 1, reinterpret_cast<int (&)[1]>(place));
+        } else if (listed <= 256) {
+            count_larger<1>(s_cand_key, listed, {own_keys[0]}, 0, reinterpret_cast<int (&)[1]>(place));
         } else {
-            for (int q0 = 0; q0 < listed; q0 += 64) {   // four adjacent threads per candidate; every lane takes part in the exchanges
-                const int q = min(q0 + (tid >> 2), listed - 1), id = s_cand_id[q];
-                const unsigned key = s_cand_key[q];
-                int place = count_before(s_cand_key, s_cand_id, listed, key, id, tid & 3, 4);
-                place += dpp_i<kDppXor1>(place);
-                place += dpp_i<kDppXor2>(place);
-                if (q0 + (tid >> 2) < listed && (tid & 3) == 0 && place < top_count) put_in_place(place, key, id);
-            }
+            count_larger<1>(s_cand_key, listed, own_keys, 0, place);
         }
+        const auto put_own = [&]() {
+            if (first < listed && (!paired || (tid & 1) == 0) && place[0] < top_count) put_in_place(place[0], own_keys[0], own_ids[0]);
+            if (256 + tid < listed && place[1] < top_count) put_in_place(place[1], own_keys[1], own_ids[1]);
+        };
+        put_own();
         __syncthreads();
-        if (wave > 0) return;
         int ids[4];   // of list positions lane, lane + 64, ...
         bool empty = false;
 #pragma unroll
@@ -429,16 +442,22 @@ __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame
             ids[r] = 64 * r + lane < top_count ? s_top_idx[64 * r + lane] : 0;
             empty = empty || ids[r] == kEmptyPlace;
         }
-        if (__builtin_expect(__any(empty), 0)) {   // equal keys: their order is their ids'
-            for (int q = lane; q < listed; q += 64) {
-                const int place = count_before(s_cand_key, s_cand_id, listed, s_cand_key[q], s_cand_id[q], 0, 1);
-                if (place < top_count) put_in_place(place, s_cand_key[q], s_cand_id[q]);   // (a shared place already holds its own: the smallest id)
+        // Equal keys: their order is their ids'.  Every wavefront sees the same places, and none is filled before all have looked.
+        if (__builtin_expect(__any(empty), 0)) {
+            if (tid < 4) s_cand_id[min(listed + tid, kFastCandidates)] = kEmptyPlace;   // (what a last quad reads behind the list)
+            __syncthreads();
+            if (paired) {
+                place[0] += count_equal_before<2>(s_cand_key, s_cand_id, listed, own_keys[0], own_ids[0], tid & 1);
+            } else {
+                place[0] += count_equal_before<1>(s_cand_key, s_cand_id, listed, own_keys[0], own_ids[0], 0);
+                if (listed > 256) place[1] += count_equal_before<1>(s_cand_key, s_cand_id, listed, own_keys[1], own_ids[1], 0);
             }
-            __builtin_amdgcn_wave_barrier();
-            __threadfence_block();
+            put_own();   // (a shared place already holds its own: the smallest id)
+            __syncthreads();
 #pragma unroll
             for (int r = 0; r < 4; ++r) ids[r] = 64 * r + lane < top_count ? s_top_idx[64 * r + lane] : 0;
         }
+        if (wave > 0) return;
         // ---- running sums in list order (src/graph.c:1605-1616), kept in place: float32 sums depend on the order, and the last running
         // sum is the reference's total.  Every lane forms all of them, then takes the ones of its own list positions.
         float running = 0.0f;
