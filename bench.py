@@ -267,13 +267,13 @@ def time_codec(pkg, backend, frames=64, runs=4, warmup=2):
             "ms_seam_operator_sequence": timings[False], "ms_one_launch_per_convolution": timings[True]}
 
 
-# (with one or two streams the attention partials are folded by the output projection that follows; with more, by
-# workgroups of the attention launch itself, and the stage timing of those launches includes, per twelve launches, the two
-# small launches that give the step its counter)
+# (the attention partials are folded by the output projection that follows, or, with more than five streams of more than 40 units of 128 rows together
+# or a stream of more than 2176 rows, by workgroups of the attention launch itself; with more than two streams the stage timing of
+# those launches includes, per twelve launches, the two small launches that give the step its counter)
 STAGES = [("self-attention", "k_step_attention<self>", "LayerNorm + int8 act-quant + per-head Q/K/V rows + KV append + attention over the self cache (+ fold of the partials where the projection does not do it)"),
-          ("self-out", "k_linear<k=768, residual>", "(fold of attention partials: two streams, or short caches) + act-quant + O matvec + residual"),
+          ("self-out", "k_linear<k=768, residual>", "(fold of attention partials where the attention launch does not) + act-quant + O matvec + residual"),
           ("cross-attention", "k_step_attention<cross>", "LayerNorm + act-quant + per-head Q rows + attention over the cross cache (+ fold where the projection does not do it)"),
-          ("cross-out", "k_linear<k=768, residual>", "(fold: two streams, or short memories) + act-quant + O matvec + residual"),
+          ("cross-out", "k_linear<k=768, residual>", "(fold where the attention launch does not) + act-quant + O matvec + residual"),
           ("ffn-up", "k_linear<k=768, LayerNorm, GELU>", "LayerNorm + act-quant + up matvec + GELU"),
           ("ffn-down", "k_linear<k=3072, residual>", "act-quant + down matvec + residual")]
 

@@ -18,7 +18,7 @@ namespace mynah {
 
 constexpr int kWave = 64;            // CDNA wavefront
 constexpr int kMaxBatch = MYNAH_HIP_MAX_BATCH;
-constexpr int kBatchTile = 8;        // streams served by one pass over a weight tile
+constexpr int kBatchTile = 8;        // streams served by one pass over a weight tile (a launch may hold two such groups, or streams side by side)
 constexpr size_t kQuantMaxRows = 16; // QMAT_SMALL_COUNT, src/qmat.c:32
 constexpr size_t kQuantMaxK = 8192;  // QMAT_K_MAX, src/qmat.c:33
 constexpr int kWideRows = 16;        // the same for their wide-head form (one wavefront per row)
@@ -30,7 +30,7 @@ constexpr int kStepUnitRows = 128;   // cache rows per attention unit (workgroup
 constexpr int kConsumerFoldMaxBatch = 2;
 constexpr int kMaxLanes = 3;         // groups of a batch's streams that step side by side, each on a stream of its own (a process has four
                                      // hardware queues here: with a fourth stream in use two of them share one, and chains that share a queue run one after the other)
-constexpr int kLaneStreams = 8;      // streams per lane when the caller names no lane count: one weight pass serves eight, so nine to sixteen streams step
+constexpr int kLaneStreams = 8;      // streams per lane when the caller names no lane count: a tile serves eight, and nine to sixteen streams step
                                      // as two lanes (measured, sixteen uniform streams: 1048 us in one lane, 856 us in two, 942 us in three; eight ragged
                                      // streams: 602 / 596 / 633 us -- a lane of four takes 480 us alone, and two chains side by side 1.24 times one)
 constexpr int kStepRecord = 68;      // 64-bit slots of one attention partial of the persistent step: out[64] | max | sum | two unused

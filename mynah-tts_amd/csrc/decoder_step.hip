@@ -99,12 +99,21 @@ namespace mynah {
 
 // Whether the product behind an attention launch folds the launch's partials (stream by stream, in its prologue: launch_linear_b), or
 // the launch folds its own.  A fold inside the launch is a hand-over between workgroups of 2 to 2.5 us at its end; behind it every
-// workgroup of the product repeats the fold for its stream, which grows with the streams and their lengths.  us a step, inside / behind: int8 three
-// streams (611, 1339 and 87 rows) 371 / 349, four 371 / 339, five (7000 rows together) 460 / 443; six of 1060 rows 376 / 353, of 4500 412 / 413,
-// of 6000 436 / 445; eight of 1000 371 / 359, of 3000 401 / 395, of 5000 418 / 415, of 7600 469 / 477.  Cross-attention memories are short: eight streams
-// 479 / 472 (f16 16 streams as two lanes 796 / 785 with both behind).  Either way gives the same bits (fold_partials' arithmetic).
-// Beside another lane the line lies higher (sixteen streams of 12000 rows in two lanes, int8 593 / 579, f16 739 / 725).
-// What a prologue does not request at once (kFoldAhead + kFoldMore partials) it takes one after the other: longer streams fold inside.
+// workgroup of the product repeats the fold for its stream, which grows with the streams and their lengths.  Either way gives the same bits
+// (fold_partials' arithmetic).  us a step, inside / behind, streams of equal length (units: 128 rows, of all streams of a lane):
+//   int8  three streams 12 units 313 / 293, 36 380 / 362, 48 407 / 413; five 40 402 / 393, 85 488 / 482; six 36 412 / 396, 42 411 / 404, 48 423 / 426, 96 512 / 517;
+//         eight 32 403 / 392, 40 413 / 403, 48 427 / 429, 64 456 / 450, 96 520 / 524, 128 573 / 574
+//   f16   three 36 431 / 418, 51 482 / 475; six 42 506 / 500, 48 528 / 531; eight 32 508 / 496, 40 523 / 528, 48 556 / 544, 96 647 / 637
+//   int4  three 51 434 / 408; eight 40 430 / 392, 96 537 / 510, 136 606 / 573
+//   f32   three 24 477 / 472, 36 487 / 492; eight 40 639 / 604, 96 773 / 740, 136 863 / 832
+//   two lanes, units a lane: int8 sixteen 64 627 / 613, 80 673 / 672, 96 721 / 728, 128 833 / 829; f16 64 785 / 775, 80 842 / 836, 128 1017 / 1005;
+//         int4 80 678 / 657, 128 826 / 797; f32 80 1027 / 1006, 128 1224 / 1213
+//   one long stream beside 87 and 300 rows: int8 2170 rows 341 / 334, 2300 347 / 347, 3072 362 / 372; f16 2300 411 / 407, 2560 417 / 421; int4 2560 361 / 360,
+//         3072 369 / 373; f32 2170 472 / 471, 3072 475 / 494
+//   cross-attention, eight streams of 256 encoder states: int8 369 / 356, f32 546 / 521; of 1280: int8 503 / 485, f32 709 / 678
+// The lines are where int8 stops gaining; int4 and f32 would still gain beyond them.  What a prologue does not request at once (kFoldAhead +
+// kFoldMore partials) it takes one after the other: longer streams fold inside.  A batch that comes to a line steps with other graphs from there on
+// (Graphs): the first step of a stream count is eager, the second is captured (int8 eight streams 426 and 840 us, then 433; f16 sixteen 907 and 1348, then 770).
 constexpr int kFoldBehindStreams = 5, kFoldBehindUnits = 40, kFoldBehindUnitsBeside = 80,
               kFoldBehindRows = (kFoldAhead + kFoldMore - 1) * kStepUnitRows;
 static bool folds_behind(const mynah_hip_decoder *d, int is_self, int batch) {
@@ -928,8 +937,8 @@ int mynah::rerun_last_step_without_waits(State *st, char *error, size_t capacity
     StepSlots s = st->last_step_slots;
     s.epoch = 1;
     // One lane, every kernel a launch of its own, and no record areas: the attention launches then take the build that
-    // finds its work from the workgroup index and a fold kernel follows each of them -- nothing in this form waits for
-    // another workgroup.  The arithmetic is the one of every other form, so these are the bits the step would have given.
+    // finds its work from the workgroup index, and the product behind folds or, long caches, a fold kernel in between --
+    // nothing in this form waits for another workgroup.  The arithmetic is the one of every other form, so these are the bits the step would have given.
     unsigned long long *const self_records = d->self_records, *const cross_records = d->cross_records;
     d->self_records = d->cross_records = nullptr;
     d->no_tables = true;

@@ -671,7 +671,9 @@ int tap_major_f16(State *st, const float *host, size_t n, size_t cin, size_t tap
 size_t attention_lds_bytes(size_t tpad) { return std::max((size_t)kQTile * (tpad + kScorePad), (size_t)3 * 32 * 64) * sizeof(float); }
 
 constexpr int kMaxSplits = 4;   // k_enc_rows reads exactly this many partial planes at most
-// Most splits that leave each workgroup at least three K steps, preferring a step count that is a multiple of four, else an even one.
+// Most splits that leave each workgroup at least three K steps, preferring a step count that is a multiple of four, else an even one: fewer planes
+// for the row pass to add where the steps are few.  The O product (twelve steps) in three splits / in four, us a prefill, tokens: one tap, 64 169.8 / 169.9,
+// 192 205.4 / 207.9, 256 212.0 / 215.2, 384 251.2 / 256.4, 512 282.3 / 283.6; three taps, 100 248.6 / 255.3, 512 392.1 / 391.8.
 int pick_splits(int k) {
     for (const int multiple : {4, 2, 1})
         for (int s = kMaxSplits; s > 1; --s)

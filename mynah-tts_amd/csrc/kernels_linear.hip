@@ -1,13 +1,13 @@
 // Weight-stationary decode matvec for gfx950, fused with its neighbours.
 //
-// One launch computes, for up to 8 concurrent streams b,
+// One launch computes, for up to 16 concurrent streams b (in groups of up to 8, or side by side one to a workgroup),
 //     out[b] = epilogue( W . prologue(in[b]) )
 // prologue : the activation row (a device vector, or the fold of the split-L attention partials written
 //            by the preceding attention kernel), optional LayerNorm (two-pass mean / variance, eps 1e-5,
 //            gain and optional bias), then for int8/int4 weights the per-vector absmax int8 activation
 //            quantisation (quantize_act_int8, src/qmat.c:94-113) -- each workgroup recomputes it from the
 //            3-12 KB input vector instead of paying a grid-wide dependency for it;
-// body     : every 16-byte weight chunk is fetched from HBM exactly once per launch (128-bit loads,
+// body     : every 16-byte weight chunk is fetched from HBM once per launch (by each group from L2; 128-bit loads,
 //            a row's chunks spread over a lane group of G lanes so a group reads 16*G contiguous
 //            bytes) and dotted against all streams' activations held in LDS: v_dot4_i32_i8 for
 //            int8/int4 (dot_q8/dot_q4, src/qmat.c:136-185), f32 FMA of exactly widened halves for f16

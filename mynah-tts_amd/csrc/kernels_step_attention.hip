@@ -12,7 +12,8 @@
 // anything else has arrived: workgroup 0 computes this head's Q and K rows, appends K
 // (src/graph.c:3180-3181) and contributes the new row's own score; workgroup 1 computes the V row,
 // appends it and contributes it as that partial's output.  The next kernel (the output projection) folds
-// the partials in its prologue, so no fence, atomic or second pass is needed here.  How a stream is cut
+// the partials in its prologue, so no fence, atomic or second pass is needed here (many long streams: workgroups of this
+// launch fold them, see the fold role).  How a stream is cut
 // into units depends on its own length only, and a unit's arithmetic on nothing but its own inputs, so a
 // stream in a batch is bit-identical to the same stream alone.
 //
@@ -69,10 +70,11 @@ __device__ __forceinline__ float4 fold_records(const float *rec, const float *we
 // per bank become constants and the per-chunk range checks fold away.  The decoder stack's width (768) gets such a build.
 // SELF: 1 / 0 = self / cross attention known at compile time (the cross build has no new-row roles at all), -1 = from the arguments.
 // PACKED: how a workgroup finds its work.  0: from its index alone (one or two streams: nearly every unit of the grid
-// exists, and the weight rows can be requested before the slot table has arrived).  1: from its index and the slot
-// table (more streams, ragged lengths: most of a grid sized for the longest possible stream would belong to units that
+// exists, and the weight rows can be requested before the slot table has arrived).  1 and 2: from its entry of a work table
+// (more streams, ragged lengths: most of a grid sized for the longest possible stream would belong to units that
 // short streams do not have; here the workgroups are numbered over the units that exist, so those with nothing to do
-// are the last ones of the grid and leave after one read instead of holding places among the working ones).
+// are the last ones of the grid and leave after one read instead of holding places among the working ones); with 1 the
+// partials leave as tagged records that fold workgroups of the launch wait for, with 2 as plain rows for the product behind.
 template <int QT, int NVT, int PF, int WFIX, int SELF, int PACKED>
 __global__ void __launch_bounds__(kThreads)
 k_step_attention(const StepSlots *const slots_arg, const float *const x_arg, const void *const w_arg, const float *const scales_arg,
@@ -485,9 +487,8 @@ k_step_attention(const StepSlots *const slots_arg, const float *const x_arg, con
     }
 }
 
-// Stand-alone fold of the partials into out[stream][heads * 64]: used instead of the consumer-side fold when
-// the batch is large enough that every workgroup of the output projection folding every stream would cost more
-// than one extra launch.  Same arithmetic (fold_partials), so the result does not depend on which path ran.
+// Stand-alone fold of the partials into out[stream][heads * 64], for streams that fold inside the launch where that is switched off, cannot
+// be waited for or has no room for the records, and for the step repeated without waits.  Same arithmetic (fold_partials), so the result does not depend on which path ran.
 __global__ void __launch_bounds__(kThreads) k_step_fold(const float *partial, const float *partial_ml, const StepSlots *slots, int heads,
                                                         int max_units, int is_self, float *out) {
     const int stream = blockIdx.y;
@@ -503,8 +504,9 @@ using StepAttnKernel = void (*)(const StepSlots *, const float *, const void *, 
                                 const int, const StepAttnArgs);
 
 // The build that runs a shape: fixed-width builds for the decoder stack's width; `latency`: the build for one or two
-// streams (work found from the workgroup index; it also serves more streams when the launch cannot fold its own partials),
-// else the many-stream build (work table, partials as tagged records, fold inside the launch).
+// streams (work found from the workgroup index; it also serves more streams when the launch cannot fold its own partials); else
+// the many-stream build: work table, partials as tagged records, fold inside the launch, or (`plain`, width 768) work table and
+// partials as rows that the product behind folds.
 template <int QT>
 StepAttnKernel kernel_for(int width, bool is_self, bool latency, bool plain = false) {
     if (plain) return is_self ? k_step_attention<QT, 1, kPrefetchLatency, 768, 1, 2> : k_step_attention<QT, 1, kPrefetchLatency, 768, 0, 2>;

@@ -67,11 +67,8 @@ __device__ __forceinline__ unsigned order_key(float v) {
 __device__ __forceinline__ float key_value(unsigned key) {
     return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
 }
-// (key, index) in one integer whose order is the order of the reference's candidate list: larger logit first, among
-// equal logits the smaller index first.  No two candidates share one, and every one is above zero.
-__device__ __forceinline__ unsigned long long candidate(unsigned key, int index) {
-    return ((unsigned long long)key << 32) | (unsigned long long)(0xffffffffu - (unsigned)index);
-}
+// (key, ~index) in one integer whose order is the order of the reference's candidate list: larger logit first, among
+// equal logits the smaller index first.
 __device__ __forceinline__ int candidate_index(unsigned long long c) { return (int)(0xffffffffu - (unsigned)(c & 0xffffffffull)); }
 __device__ __forceinline__ unsigned candidate_key(unsigned long long c) { return (unsigned)(c >> 32); }
 
@@ -725,8 +722,9 @@ extern "C" int mynah_hip_local_frame(void *state, mynah_hip_local *l, mynah_hip_
     const int B = (int)batch;
     MYNAH_TRY(hipStreamSynchronize(st->stream));   // the staging buffers of the previous frame may still be in flight
     l->frame_host->logits_copy = dev_logits_copy;
-    // a frame's many-stream attention launches wait like a decode step's, but a frame cannot be repeated from here (its
-    // generator states have moved on): a wait given up inside it is reported as the error it is, never taken for a decode step's
+    // a frame's attention launches of more than two streams wait like a decode step's where the stack is not 768 wide (there the products
+    // behind fold), but a frame cannot be repeated from here (its generator states have moved on): a wait given up inside it is
+    // reported as the error it is, never taken for a decode step's
     st->last_step_decoder = nullptr;
     st->steps_since_sync += 2;
     if (decoder_next_epochs(st, l->stack, (unsigned)l->streams, &l->frame_host->epoch_base, error, capacity) != 0) return -1;

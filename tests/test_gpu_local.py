@@ -164,7 +164,7 @@ def test_frame_model_shape_batch8(pkg, backend, orc, synth, nerr, qtype_name):
 
 
 def test_frame_batch16_two_tiles(pkg, backend, orc, synth, nerr):
-    """Sixteen items (two passes of eight through every matvec, the many-stream attention layout), alternating greedy and
+    """Sixteen items (two groups of eight or four of four in every product's launch, the many-stream attention layout), alternating greedy and
     sampling, f32: tokens and generator states equal to the oracle's frame."""
     _announce("local frame batch 16 f32")
     S, V, codebook, eos, cbc = 16, 512, 480, 481, 8
