@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(256) k_local_begin(LocalFrameDev *frame, const
 // beyond (list places that equal keys leave empty are seen afterwards and filled by the ids of the equal ones); and behind the ranking the first wavefront alone, so that nothing waits at a barrier.
 // Measured and not kept: the rows of the first 8 or 32 list positions fetched by the other wavefronts meanwhile (no change).
 // A frame of 16 positions, us, int8: one stream top-80 402 -> 380, three top-100 461 -> 439, eight top-50 494 -> 472; of 8 positions, one stream: top-160 252 -> 221,
-// top-200 302 -> 234, top-256 300 -> 279; top-100 of 96 ids, two of them masked and so equal, 206 -> 212.
+// top-200 302 -> 233, top-256 300 -> 276; top-100 of 96 ids, two of them masked and so equal, 206 -> 215.
 constexpr int kFastCandidates = 512;
 constexpr int kEmptyPlace = 0x7fffffff;
 
@@ -413,24 +413,34 @@ __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame
             atomicMin(&s_top_idx[place], id);
             s_top_val[place] = expf((key_value(key) - maximum) / temperature);
         };
-        static_assert(kMaxTopK == 256 && kFastCandidates == 512, "two candidates a thread at most");
-        const bool paired = listed <= 128;   // two threads a candidate
-        const int first = paired ? tid >> 1 : tid;
-        const unsigned own_keys[2] = {s_cand_key[first], s_cand_key[256 + tid]};
-        const int own_ids[2] = {s_cand_id[min(first, listed - 1)], s_cand_id[min(256 + tid, listed - 1)]};
-        int place[2] = {0, 0};
-        if (paired) {
-            count_larger<2>(s_cand_key, listed, {own_keys[0]}, tid & 1, reinterpret_cast<int (&)[1]>(place));
-        } else if (listed <= 256) {
-            count_larger<1>(s_cand_key, listed, {own_keys[0]}, 0, reinterpret_cast<int (&)[1]>(place));
-        } else {
-            count_larger<1>(s_cand_key, listed, own_keys, 0, place);
-        }
-        const auto put_own = [&]() {
-            if (first < listed && (!paired || (tid & 1) == 0) && place[0] < top_count) put_in_place(place[0], own_keys[0], own_ids[0]);
-            if (256 + tid < listed && place[1] < top_count) put_in_place(place[1], own_keys[1], own_ids[1]);
+        // (more than 128 candidates: one or two a thread; `by_id`: among equal keys by their ids, a shared place already holds its own, the smallest)
+        const auto rank_long = [&](const bool by_id) {
+            const unsigned own_keys[2] = {s_cand_key[tid], s_cand_key[256 + tid]};
+            int place[2] = {0, 0};
+            if (listed <= 256) count_larger<1>(s_cand_key, listed, {own_keys[0]}, 0, reinterpret_cast<int (&)[1]>(place));
+            else count_larger<1>(s_cand_key, listed, own_keys, 0, place);
+#pragma unroll 1
+            for (int j = 0; j < 2; ++j) {
+                const int q = 256 * j + tid;
+                if (q < listed) {
+                    const int id = s_cand_id[q];
+                    int at = j == 0 ? place[0] : place[1];
+                    const unsigned key = j == 0 ? own_keys[0] : own_keys[1];
+                    if (by_id) at += count_equal_before<1>(s_cand_key, s_cand_id, listed, key, id, 0);
+                    if (at < top_count) put_in_place(at, key, id);
+                }
+            }
         };
-        put_own();
+        static_assert(kMaxTopK == 256 && kFastCandidates == 512, "two candidates a thread at most");
+        if (listed <= 128) {   // two threads a candidate
+            const unsigned key[1] = {s_cand_key[tid >> 1]};
+            const int id = s_cand_id[min(tid >> 1, listed - 1)];
+            int place[1];
+            count_larger<2>(s_cand_key, listed, key, tid & 1, place);
+            if ((tid >> 1) < listed && (tid & 1) == 0 && place[0] < top_count) put_in_place(place[0], key[0], id);
+        } else {
+            rank_long(false);
+        }
         __syncthreads();
         int ids[4];   // of list positions lane, lane + 64, ...
         bool empty = false;
@@ -443,13 +453,16 @@ __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame
         if (__builtin_expect(__any(empty), 0)) {
             if (tid < 4) s_cand_id[min(listed + tid, kFastCandidates)] = kEmptyPlace;   // (what a last quad reads behind the list)
             __syncthreads();
-            if (paired) {
-                place[0] += count_equal_before<2>(s_cand_key, s_cand_id, listed, own_keys[0], own_ids[0], tid & 1);
+            if (listed <= 128) {
+                const unsigned key[1] = {s_cand_key[tid >> 1]};
+                const int id = s_cand_id[min(tid >> 1, listed - 1)];
+                int place[1];
+                count_larger<2>(s_cand_key, listed, key, tid & 1, place);
+                place[0] += count_equal_before<2>(s_cand_key, s_cand_id, listed, key[0], id, tid & 1);
+                if ((tid >> 1) < listed && (tid & 1) == 0 && place[0] < top_count) put_in_place(place[0], key[0], id);
             } else {
-                place[0] += count_equal_before<1>(s_cand_key, s_cand_id, listed, own_keys[0], own_ids[0], 0);
-                if (listed > 256) place[1] += count_equal_before<1>(s_cand_key, s_cand_id, listed, own_keys[1], own_ids[1], 0);
+                rank_long(true);
             }
-            put_own();   // (a shared place already holds its own: the smallest id)
             __syncthreads();
 #pragma unroll
             for (int r = 0; r < 4; ++r) ids[r] = 64 * r + lane < top_count ? s_top_idx[64 * r + lane] : 0;
