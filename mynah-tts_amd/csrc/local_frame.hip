@@ -84,30 +84,24 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
     return max(max(r0, r1), max(r2, r3));
 }
 
-// How many of the collected candidates have a larger key than each of KEYS own ones, counted by LANES adjacent threads: thread `part` compares the quads of
-// keys part, part + LANES, ..., sixteen reads together; the keys behind the list are zero, which is larger than none.  Every lane of the wavefront
-// must call it.
-template <int LANES, int KEYS>
-__device__ __forceinline__ void count_larger(const unsigned *keys, int n, const unsigned (&own)[KEYS], int part, int (&larger)[KEYS]) {
+// How many of the collected candidates have a larger key, counted by LANES adjacent threads: thread `part` compares the quads of keys part, part + LANES, ..., sixteen reads
+// together; the keys behind the list are zero, which is larger than none.  Every lane of the wavefront must call it.
+template <int LANES>
+__device__ __forceinline__ int count_larger(const unsigned *keys, int n, unsigned key, int part) {
     const uint4 *const quads = reinterpret_cast<const uint4 *>(keys) + part;
-#pragma unroll
-    for (int j = 0; j < KEYS; ++j) larger[j] = 0;
+    int larger = 0;
 #pragma unroll 1
     for (int q0 = 0; 4 * q0 < n; q0 += 16 * LANES) {
         uint4 k[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) k[i] = quads[q0 + i * LANES];
 #pragma unroll
-        for (int j = 0; j < KEYS; ++j)
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                larger[j] += (k[i].x > own[j] ? 1 : 0) + (k[i].y > own[j] ? 1 : 0) + (k[i].z > own[j] ? 1 : 0) + (k[i].w > own[j] ? 1 : 0);
+        for (int i = 0; i < 16; ++i) larger += (k[i].x > key ? 1 : 0) + (k[i].y > key ? 1 : 0) + (k[i].z > key ? 1 : 0) + (k[i].w > key ? 1 : 0);
     }
-    if (LANES == 2) {
-#pragma unroll
-        for (int j = 0; j < KEYS; ++j) larger[j] += dpp_i<kDppXor1>(larger[j]);
-    }
+    if (LANES == 2) larger += dpp_i<kDppXor1>(larger);
+    return larger;
 }
+
 // How many have the same key and a smaller index.  Keys and indexes are read whatever the keys are (an index read only behind an equal key
 // was a round trip of its own: 16 us a choice from 96 with two equal ones); the indexes behind the list are larger than any.
 template <int LANES>
@@ -163,8 +157,8 @@ __global__ void __launch_bounds__(256) k_local_begin(LocalFrameDev *frame, const
 // stored where nobody looks, without a branch; the ranking by the keys' 32 bits, two threads a candidate up to 128, one or two candidates a thread
 // beyond (list places that equal keys leave empty are seen afterwards and filled by the ids of the equal ones); and behind the ranking the first wavefront alone, so that nothing waits at a barrier.
 // Measured and not kept: the rows of the first 8 or 32 list positions fetched by the other wavefronts meanwhile (no change).
-// A frame of 16 positions, us, int8: one stream top-80 402 -> 380, three top-100 461 -> 439, eight top-50 494 -> 472; of 8 positions, one stream: top-160 252 -> 221,
-// top-200 302 -> 233, top-256 300 -> 276; top-100 of 96 ids, two of them masked and so equal, 206 -> 215.
+// A frame of 16 positions, us, int8: one stream top-80 402 -> 380, three top-100 461 -> 439, eight top-50 494 -> 472; of 8 positions, one stream: top-160 254 -> 225,
+// top-200 304 -> 242, top-256 301 -> 274; top-100 of 96 ids, two of them masked and so equal, 207 -> 214.
 constexpr int kFastCandidates = 512;
 constexpr int kEmptyPlace = 0x7fffffff;
 
@@ -413,33 +407,22 @@ __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame
             atomicMin(&s_top_idx[place], id);
             s_top_val[place] = expf((key_value(key) - maximum) / temperature);
         };
-        // (more than 128 candidates: one or two a thread; `by_id`: among equal keys by their ids, a shared place already holds its own, the smallest)
-        const auto rank_long = [&](const bool by_id) {
-            const unsigned own_keys[2] = {s_cand_key[tid], s_cand_key[256 + tid]};
-            int place[2] = {0, 0};
-            if (listed <= 256) count_larger<1>(s_cand_key, listed, {own_keys[0]}, 0, reinterpret_cast<int (&)[1]>(place));
-            else count_larger<1>(s_cand_key, listed, own_keys, 0, place);
-#pragma unroll 1
-            for (int j = 0; j < 2; ++j) {
-                const int q = 256 * j + tid;
-                if (q < listed) {
-                    const int id = s_cand_id[q];
-                    int at = j == 0 ? place[0] : place[1];
-                    const unsigned key = j == 0 ? own_keys[0] : own_keys[1];
-                    if (by_id) at += count_equal_before<1>(s_cand_key, s_cand_id, listed, key, id, 0);
-                    if (at < top_count) put_in_place(at, key, id);
-                }
-            }
-        };
         static_assert(kMaxTopK == 256 && kFastCandidates == 512, "two candidates a thread at most");
-        if (listed <= 128) {   // two threads a candidate
-            const unsigned key[1] = {s_cand_key[tid >> 1]};
-            const int id = s_cand_id[min(tid >> 1, listed - 1)];
-            int place[1];
-            count_larger<2>(s_cand_key, listed, key, tid & 1, place);
-            if ((tid >> 1) < listed && (tid & 1) == 0 && place[0] < top_count) put_in_place(place[0], key[0], id);
+        if (listed <= 128) {
+            const unsigned key = s_cand_key[tid >> 1];
+            const int id = s_cand_id[min(tid >> 1, listed - 1)], place = count_larger<2>(s_cand_key, listed, key, tid & 1);
+            if ((tid >> 1) < listed && (tid & 1) == 0 && place < top_count) put_in_place(place, key, id);
+        } else if (listed <= 256) {
+            const unsigned key = s_cand_key[tid];
+            const int id = s_cand_id[min(tid, listed - 1)], place = count_larger<1>(s_cand_key, listed, key, 0);
+            if (tid < listed && place < top_count) put_in_place(place, key, id);
         } else {
-            rank_long(false);
+#pragma unroll 1
+            for (int q0 = 0; q0 < listed; q0 += 256) {
+                const unsigned key = s_cand_key[q0 + tid];
+                const int id = s_cand_id[min(q0 + tid, listed - 1)], place = count_larger<1>(s_cand_key, listed, key, 0);
+                if (q0 + tid < listed && place < top_count) put_in_place(place, key, id);
+            }
         }
         __syncthreads();
         int ids[4];   // of list positions lane, lane + 64, ...
@@ -453,15 +436,20 @@ __global__ void __launch_bounds__(256) k_local_sample(LocalFrameDev *const frame
         if (__builtin_expect(__any(empty), 0)) {
             if (tid < 4) s_cand_id[min(listed + tid, kFastCandidates)] = kEmptyPlace;   // (what a last quad reads behind the list)
             __syncthreads();
+            // (a shared place already holds its own: the smallest id)
             if (listed <= 128) {
-                const unsigned key[1] = {s_cand_key[tid >> 1]};
+                const unsigned key = s_cand_key[tid >> 1];
                 const int id = s_cand_id[min(tid >> 1, listed - 1)];
-                int place[1];
-                count_larger<2>(s_cand_key, listed, key, tid & 1, place);
-                place[0] += count_equal_before<2>(s_cand_key, s_cand_id, listed, key[0], id, tid & 1);
-                if ((tid >> 1) < listed && (tid & 1) == 0 && place[0] < top_count) put_in_place(place[0], key[0], id);
+                const int place = count_larger<2>(s_cand_key, listed, key, tid & 1) + count_equal_before<2>(s_cand_key, s_cand_id, listed, key, id, tid & 1);
+                if ((tid >> 1) < listed && (tid & 1) == 0 && place < top_count) put_in_place(place, key, id);
             } else {
-                rank_long(true);
+#pragma unroll 1
+                for (int q0 = 0; q0 < listed; q0 += 256) {
+                    const unsigned key = s_cand_key[q0 + tid];
+                    const int id = s_cand_id[min(q0 + tid, listed - 1)];
+                    const int place = count_larger<1>(s_cand_key, listed, key, 0) + count_equal_before<1>(s_cand_key, s_cand_id, listed, key, id, 0);
+                    if (q0 + tid < listed && place < top_count) put_in_place(place, key, id);
+                }
             }
             __syncthreads();
 #pragma unroll
