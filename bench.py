@@ -281,11 +281,11 @@ STAGES = [("self-attention", "k_step_attention<self>", "LayerNorm + int8 act-qua
 # then WRITE_SIZE), each scaled by what the same counter reads for the library's plain 256 MiB read+write kernel.  A figure
 # belongs to the kernel sources it was measured on: it is reported only while their hash is the one recorded here.
 MEASURED_TRAFFIC = {
-    1: {"kernel": "k_linear<k=768, residual>", "bytes": 955833, "profile": "profiles/decode_step_int8_hbm_counters.md",
-        "sources": ("kernels_linear.hip", "device_common.h", "kernels.h", "common.h"), "csrc_sha256": "35a62c05e339ea94"},
-    8: {"kernel": "k_step_attention<self>", "bytes": 54473543, "profile": "profiles/decode_step_int8_hbm_counters.md",
+    1: {"kernel": "k_linear<k=768, residual>", "bytes": 950201, "profile": "profiles/decode_step_int8_hbm_counters.md",
+        "sources": ("kernels_linear.hip", "device_common.h", "kernels.h", "common.h"), "csrc_sha256": "a85c87c9e05e5a65"},
+    8: {"kernel": "k_step_attention<self>", "bytes": 54473038, "profile": "profiles/decode_step_int8_hbm_counters.md",
         "sources": ("kernels_step_attention.hip", "step_attention_core.h", "step_items.h", "tagged_exchange.h", "device_common.h",
-                    "kernels.h", "common.h"), "csrc_sha256": "5b706ec975938d8d"},
+                    "kernels.h", "common.h"), "csrc_sha256": "b10e83c81ad358f1"},
 }
 
 
